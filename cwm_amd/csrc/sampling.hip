@@ -17,12 +17,15 @@
 // f(t) = sum of e_i > t, the kept set is {e_i >= t*} for the smallest float t*
 // with f(t*) <= top_p * sum(e); t* is found by cutting the interval of bit patterns.
 // Entries exactly equal to the threshold are all kept.  Without a nucleus (top_p = 1)
-// nothing is stored: the draw recomputes e_i where it walks.  A row of 128k logits
-// takes about 22 us greedy, 44 us at a temperature and 170 us with a nucleus.
+// nothing is stored: the draw recomputes e_i where it walks.  A row of 128k logits done so
+// takes about 22 us greedy, 44 us at a temperature and 170 us with a nucleus; rows of more than
+// 8,192 entries are cut into segments instead (below): 16, 21 and 27 us, 49 us with a nucleus of
+// thousands of entries, launches included; 743 such rows 200 us instead of 1,220.
 #include "common.h"
 #include "no_alloc.h"
 
 #include <mutex>
+#include <type_traits>
 
 CWM_DEFINE_ERROR_API
 
@@ -62,18 +65,25 @@ __device__ __forceinline__ void each_strided(const float* x, int n, int tid, F&&
 #define SEARCH_WAYS 2  // thresholds tried in one pass over the row (measured at 128k entries: 2 169 us, 3 187, 4 196, 8 242)
 #endif
 
-template <bool VEC>
-__global__ void __launch_bounds__(SAMPLE_THREADS)
-sample_kernel(const float* __restrict__ logits, long row_stride, int vocab, const float* __restrict__ temperature,
-              const float* __restrict__ top_p, const float* __restrict__ uniform, float* __restrict__ workspace,
-              int* __restrict__ token_out, float* __restrict__ logprob_out, float* __restrict__ sample_logprob_out) {
-  __shared__ float scratch[16];
-  __shared__ float mv[SAMPLE_THREADS / CWM_WAVE];
-  __shared__ int mi[SAMPLE_THREADS / CWM_WAVE];
-  __shared__ float seg_sum[2 * SAMPLE_THREADS / CWM_WAVE];  // masses of the 16 regions, then of the chosen region's 16 parts
-  __shared__ float above_part[SAMPLE_THREADS / CWM_WAVE][SEARCH_WAYS];
+struct WholeRowShared {
+  float scratch[16];
+  float mv[SAMPLE_THREADS / CWM_WAVE];
+  int mi[SAMPLE_THREADS / CWM_WAVE];
+  float seg_sum[2 * SAMPLE_THREADS / CWM_WAVE];  // masses of the 16 regions, then of the chosen region's 16 parts
+  float above_part[SAMPLE_THREADS / CWM_WAVE][SEARCH_WAYS];
+};
 
-  const int row = blockIdx.x;
+// One block does a whole row by itself.
+template <bool VEC>
+__device__ __forceinline__ void sample_whole_row(WholeRowShared& sh, const int row, const float* __restrict__ logits, long row_stride, int vocab,
+                                 const float* __restrict__ temperature, const float* __restrict__ top_p, const float* __restrict__ uniform,
+                                 float* __restrict__ workspace, int* __restrict__ token_out, float* __restrict__ logprob_out,
+                                 float* __restrict__ sample_logprob_out) {
+  float* scratch = sh.scratch;
+  float* mv = sh.mv;
+  int* mi = sh.mi;
+  float* seg_sum = sh.seg_sum;
+  auto& above_part = sh.above_part;
   const int tid = threadIdx.x;
   const float* x = logits + (size_t)row * row_stride;
   float* e = workspace + (size_t)row * vocab;
@@ -311,11 +321,494 @@ sample_kernel(const float* __restrict__ logits, long row_stride, int vocab, cons
   }
 }
 
+template <bool VEC>
+__global__ void __launch_bounds__(SAMPLE_THREADS)
+sample_kernel(const float* __restrict__ logits, long row_stride, int vocab, const float* __restrict__ temperature,
+              const float* __restrict__ top_p, const float* __restrict__ uniform, float* __restrict__ workspace,
+              int* __restrict__ token_out, float* __restrict__ logprob_out, float* __restrict__ sample_logprob_out) {
+  __shared__ WholeRowShared sh;
+  sample_whole_row<VEC>(sh, blockIdx.x, logits, row_stride, vocab, temperature, top_p, uniform, workspace, token_out, logprob_out,
+                        sample_logprob_out);
+}
+
+// ---- rows cut into segments ----------------------------------------------------------- //
+// One compute unit reads a row of 128k logits at a hundredth of the memory's rate and needs 8 us for as many exponentials,
+// so a row is cut into segments of at most 2,048 entries, a block each, read once; a second kernel of one block a row puts
+// the segments' records together.  The nucleus is found through a histogram of mass instead of passes over the row: a bin
+// is floor(x * 8 / (T ln 2)), an eighth of an octave of e^(x/T), the same bin in every segment whatever its maximum, and the
+// bin in which the mass from the top passes top_p * z is the only one whose entries have to be looked at.  Masses that
+// several threads add to one place are integers (units of 2^-40 of the largest entry), so their order does not matter and
+// a row's result is the same every time.
+#define SEG_THREADS 256
+#define SEG_PER_THREAD 8
+#define SEG_ENTRIES (SEG_THREADS * SEG_PER_THREAD)
+#define SEG_MOST 256     // segments of a row
+#define SEG_BINS 256     // the last one holds everything 32 octaves and more below the segment's maximum
+#define SEGMENTS_FROM 8192  // longer rows are cut: the second launch costs 4 us, and a nucleus in a row of 8,192 takes 37 us as a whole, 20 to 28 in segments
+#define SEG_LIST 4096    // entries of the decisive bin that are kept in LDS
+#define SEG_SORT 1024    // and those of its decisive part that are put in order
+#define SEG_FIXED 1099511627776.0f  // 2^40
+
+struct SegRecord {
+  float max;
+  int argmax;
+  float sum;   // of exp(x - max)
+  float mass;  // of exp((x - max) / T)
+};
+
+// Where the records and histograms of a row lie in its part of the workspace (vocab floats).
+__host__ __device__ __forceinline__ int seg_length(int vocab) {
+  const int n = (vocab + SEG_ENTRIES - 1) / SEG_ENTRIES;
+  return (((vocab + n - 1) / n) + 63) / 64 * 64;
+}
+__device__ __forceinline__ SegRecord* seg_records(float* row_workspace) {
+  return (SegRecord*)(((uintptr_t)row_workspace + 15) & ~(uintptr_t)15);
+}
+__device__ __forceinline__ float* seg_histogram(float* row_workspace, int n_segs, int seg) {
+  return (float*)(seg_records(row_workspace) + n_segs) + (size_t)seg * SEG_BINS;
+}
+
+// the bin of x counted downwards from the one of `top` (both times 8 / (T ln 2))
+__device__ __forceinline__ int bins_below(float top_floor, float scaled) { return (int)fminf(top_floor - floorf(scaled), (float)(SEG_BINS - 1)); }
+
+template <bool VEC>
+__global__ void __launch_bounds__(SEG_THREADS)
+sample_segment_kernel(const float* __restrict__ logits, long row_stride, int vocab, int seg_len, const float* __restrict__ temperature,
+                      const float* __restrict__ top_p, float* __restrict__ workspace) {
+  __shared__ float wv[SEG_THREADS / CWM_WAVE];
+  __shared__ int wi[SEG_THREADS / CWM_WAVE];
+  __shared__ float ws[SEG_THREADS / CWM_WAVE], wz[SEG_THREADS / CWM_WAVE], wt[SEG_THREADS / CWM_WAVE];
+  __shared__ unsigned long long bins[SEG_BINS];
+  const int seg = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid & (CWM_WAVE - 1), wave = tid / CWM_WAVE;
+  const int begin = seg * seg_len, end = min(vocab, begin + seg_len);
+  const float* x = logits + (size_t)row * row_stride;
+  bins[tid] = 0;
+  float v[SEG_PER_THREAD];
+  int at[SEG_PER_THREAD / 4];  // first entry of every four
+#pragma unroll
+  for (int q = 0; q < SEG_PER_THREAD / 4; ++q) {
+    at[q] = begin + 4 * (q * SEG_THREADS + tid);
+    if (VEC) {  // begin, end: multiples of 4
+      const float4 f = at[q] < end ? *(const float4*)(x + at[q]) : make_float4(-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff());
+      v[4 * q] = f.x, v[4 * q + 1] = f.y, v[4 * q + 2] = f.z, v[4 * q + 3] = f.w;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[4 * q + j] = at[q] + j < end ? x[at[q] + j] : -__builtin_inff();
+    }
+  }
+  MaxIdx best = {-__builtin_inff(), 0x7fffffff};
+#pragma unroll
+  for (int j = 0; j < SEG_PER_THREAD; ++j)
+    if (v[j] > best.v) best.v = v[j], best.i = at[j / 4] + j % 4;
+#pragma unroll
+  for (int off = CWM_WAVE / 2; off > 0; off >>= 1) best = better(best, MaxIdx{__shfl_xor(best.v, off, CWM_WAVE), __shfl_xor(best.i, off, CWM_WAVE)});
+  if (lane == 0) wv[wave] = best.v, wi[wave] = best.i;
+  __syncthreads();
+  best = MaxIdx{wv[0], wi[0]};
+#pragma unroll
+  for (int w = 1; w < SEG_THREADS / CWM_WAVE; ++w) best = better(best, MaxIdx{wv[w], wi[w]});
+
+  const float temp = temperature[row];
+  const bool draw = temp > 0.f, nucleus = draw && top_p[row] < 1.0f;
+  const float inv_t = draw ? 1.0f / temp : 0.f, inv_w = inv_t * 11.541560327f;  // 8 / ln 2
+  const float top_floor = floorf(best.v * inv_w);
+  float s = 0.f, z = 0.f, tail = 0.f;
+#pragma unroll
+  for (int j = 0; j < SEG_PER_THREAD; ++j) {
+    const float d = v[j] == -__builtin_inff() ? v[j] : v[j] - best.v;  // (a segment may hold nothing else; a NaN stays one)
+    s += expf(d);
+    if (draw) {
+      const float e = expf(d * inv_t);
+      z += e;
+      if (nucleus) {
+        const int k = bins_below(top_floor, v[j] * inv_w);
+        if (k < SEG_BINS - 1 && e > 0.f) atomicAdd(&bins[k], (unsigned long long)(e * SEG_FIXED));
+        else tail += e;
+      }
+    }
+  }
+  s = wave_sum(s), z = wave_sum(z), tail = wave_sum(tail);
+  if (lane == 0) ws[wave] = s, wz[wave] = z, wt[wave] = tail;
+  __syncthreads();
+  float* row_workspace = workspace + (size_t)row * vocab;
+  if (nucleus) {
+    float* out = seg_histogram(row_workspace, gridDim.x, seg);
+    out[tid] = tid < SEG_BINS - 1 ? (float)bins[tid] * (1.0f / SEG_FIXED) : wt[0] + wt[1] + wt[2] + wt[3];
+  }
+  if (tid == 0) seg_records(row_workspace)[seg] = SegRecord{best.v, best.i, ws[0] + ws[1] + ws[2] + ws[3], wz[0] + wz[1] + wz[2] + wz[3]};
+}
+
+// Inclusive sums over the block's threads in a fixed order; `scratch` holds 16 floats.
+__device__ __forceinline__ float block_scan(float v, float* scratch) {
+  const int lane = threadIdx.x & (CWM_WAVE - 1), wave = threadIdx.x / CWM_WAVE;
+#pragma unroll
+  for (int off = 1; off < CWM_WAVE; off <<= 1) {
+    const float o = __shfl_up(v, off, CWM_WAVE);
+    if (lane >= off) v += o;
+  }
+  __syncthreads();
+  if (lane == CWM_WAVE - 1) scratch[wave] = v;
+  __syncthreads();
+  float before = 0.f;
+  for (int w = 0; w < wave; ++w) before += scratch[w];
+  return before + v;
+}
+
+struct JoinShared {
+  float scratch[16];
+  int first, last, count, smallest;
+  int argmax[SEG_MOST];
+  float max[SEG_MOST], scale[SEG_MOST], mass[SEG_MOST];
+  int below[SEG_MOST];  // bins from the row's top bin down to the segment's
+  unsigned long long kept[SEG_MOST];
+  union {
+    float part[4][SEG_BINS];
+    float sorted[SEG_SORT];
+  };
+  unsigned long long sub[SEG_BINS];
+  float list_x[SEG_LIST];
+  int list_i[SEG_LIST];
+  float before;
+};
+
+// The index of the first thread, in order, whose inclusive sum `cum` passes `target` while it has mass; the last one with
+// mass if none does.  `before` receives the sum before it.  All threads call it and get the same answer.
+__device__ __forceinline__ int first_past(JoinShared& sh, float mass, float cum, float target, float& before) {
+  if (threadIdx.x == 0) sh.first = 0x7fffffff, sh.last = -1;
+  __syncthreads();
+  if (mass > 0.f) {
+    if (cum > target) atomicMin(&sh.first, (int)threadIdx.x);
+    atomicMax(&sh.last, (int)threadIdx.x);
+  }
+  __syncthreads();
+  const int pick = sh.first != 0x7fffffff ? sh.first : sh.last;
+  if ((int)threadIdx.x == pick) sh.before = cum - mass;
+  __syncthreads();
+  before = pick >= 0 ? sh.before : 0.f;
+  return pick;
+}
+
+// False where the row has to be done by `sample_whole_row`; the block's threads agree.
+template <bool VEC>
+__device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, const float* __restrict__ logits, long row_stride, int vocab, int seg_len, int n_segs, const float* __restrict__ temperature,
+                   const float* __restrict__ top_p, const float* __restrict__ uniform, float* __restrict__ workspace,
+                   int* __restrict__ token_out, float* __restrict__ logprob_out, float* __restrict__ sample_logprob_out) {
+  const int tid = threadIdx.x, lane = tid & (CWM_WAVE - 1), wave = tid / CWM_WAVE;
+  const float* x = logits + (size_t)row * row_stride;
+  float* row_workspace = workspace + (size_t)row * vocab;
+  const float temp = temperature[row], row_top_p = top_p[row], u = uniform[row];
+
+  // 1. the row's maximum, its first index and the log of the sum at temperature 1
+  SegRecord rec = {-__builtin_inff(), 0x7fffffff, 0.f, 0.f};
+  if (tid < n_segs) rec = seg_records(row_workspace)[tid];
+  MaxIdx best = {rec.max, rec.argmax};
+#pragma unroll
+  for (int off = CWM_WAVE / 2; off > 0; off >>= 1) best = better(best, MaxIdx{__shfl_xor(best.v, off, CWM_WAVE), __shfl_xor(best.i, off, CWM_WAVE)});
+  if (lane == 0 && wave < SEG_MOST / CWM_WAVE) sh.max[wave] = best.v, sh.argmax[wave] = best.i;
+  __syncthreads();
+  best = MaxIdx{sh.max[0], sh.argmax[0]};
+#pragma unroll
+  for (int w = 1; w < SEG_MOST / CWM_WAVE; ++w) best = better(best, MaxIdx{sh.max[w], sh.argmax[w]});
+  const float xmax = best.v;
+  const float sum = block_sum(tid < n_segs ? (rec.max == -__builtin_inff() ? rec.sum : rec.sum * expf(rec.max - xmax)) : 0.f, sh.scratch);
+  const float lse = xmax + logf(sum);
+  // NaN among the logits, infinities, temperatures at which a bin's number would not be exact: one block, pass by pass
+  const float inv_t = 1.0f / temp, inv_w = inv_t * 11.541560327f;
+  if (!(sum > 0.f) || !(fabsf(xmax) < __builtin_inff()) || (temp > 0.f && !(fabsf(xmax) * inv_w < 1e6f && inv_w < 1e6f))) {
+    return false;
+  }
+  if (!(temp > 0.f)) {  // greedy
+    if (tid == 0) {
+      token_out[row] = best.i;
+      logprob_out[row] = xmax - lse;
+      sample_logprob_out[row] = 0.f;
+    }
+    return true;
+  }
+
+  // 2. every segment's mass over the row's maximum
+  const float top_floor = floorf(xmax * inv_w);
+  __syncthreads();  // (sh.max, sh.argmax have been read)
+  float seg_mass = 0.f;
+  if (tid < SEG_MOST) {
+    const float scale = tid < n_segs && rec.max > -__builtin_inff() ? expf((rec.max - xmax) * inv_t) : 0.f;
+    seg_mass = scale > 0.f ? rec.mass * scale : 0.f;
+    sh.scale[tid] = scale;
+    sh.below[tid] = scale > 0.f ? bins_below(top_floor, rec.max * inv_w) : SEG_BINS;
+    sh.kept[tid] = 0;
+  }
+  const float z = block_sum(seg_mass, sh.scratch);
+  const bool nucleus = row_top_p < 1.0f;
+  int bin = SEG_BINS, sub = SEG_BINS;  // kept whole: the bins before `bin`, and of that one the parts before `sub`
+  float least = 0.f;                   // kept of part `sub` (of the whole bin if it is not divided): the entries from here on
+  auto e_of = [&](float v) { return expf((v - xmax) * inv_t); };
+  auto bin_of = [&](float scaled) { return bins_below(top_floor, scaled); };
+  auto sub_of = [&](float scaled) { return SEG_BINS - 1 - min(SEG_BINS - 1, (int)((scaled - floorf(scaled)) * SEG_BINS)); };
+  auto kept = [&](float v) {
+    if (!nucleus) return v > -__builtin_inff() ? e_of(v) : 0.f;
+    const float scaled = v * inv_w;
+    const int k = v > -__builtin_inff() ? bin_of(scaled) : SEG_BINS;
+    if (k != bin) return k < bin ? e_of(v) : 0.f;
+    if (sub < SEG_BINS) {
+      const int j = sub_of(scaled);
+      if (j != sub) return j < sub ? e_of(v) : 0.f;
+    }
+    const float e = e_of(v);
+    return e >= least ? e : 0.f;
+  };
+
+  if (nucleus) {
+    // 3. the bin in which the mass from the top passes top_p * z
+    const float target = row_top_p * z;
+    const int g = tid & (SEG_BINS - 1);
+    float m = 0.f;
+    for (int s = tid / SEG_BINS; s < n_segs; s += SAMPLE_THREADS / SEG_BINS) {
+      const int k = g - sh.below[s];
+      if (k >= 0 && k < SEG_BINS - 1) m += seg_histogram(row_workspace, n_segs, s)[k] * sh.scale[s];
+    }
+    sh.part[tid / SEG_BINS][g] = m;
+    __syncthreads();
+    m = tid < SEG_BINS - 1 ? sh.part[0][tid] + sh.part[1][tid] + sh.part[2][tid] + sh.part[3][tid] : 0.f;
+    const float cum = block_scan(m, sh.scratch);
+    if (tid == 0) sh.first = SEG_BINS, sh.count = 0, sh.smallest = 0x7f800000;
+    __syncthreads();
+    if (m > 0.f && cum > target) atomicMin(&sh.first, tid);
+    __syncthreads();
+    bin = sh.first;
+    if (bin >= SEG_BINS - 1) {  // the passing point lies below 32 octaves
+      return false;
+    }
+    if (tid == bin) sh.before = cum - m;
+    if (tid < SEG_BINS) sh.sub[tid] = 0;
+    __syncthreads();
+    float above = sh.before;
+
+    // 4. that bin's entries, a segment a wavefront, where the segment has mass in it: take(segment, its first entry,
+    //    the lane's entries that lie in the bin)
+    const float edge = top_floor - bin;  // x lies in the bin if edge <= x * inv_w < edge + 1
+    auto scan_bin = [&](auto&& take) {
+      for (int s = wave; s < n_segs; s += SAMPLE_THREADS / CWM_WAVE) {
+        const int k = bin - sh.below[s];
+        if (k < 0 || !(seg_histogram(row_workspace, n_segs, s)[min(k, SEG_BINS - 1)] > 0.f)) continue;
+        const int begin = s * seg_len, end = min(vocab, begin + seg_len);
+        constexpr int LOADS = SEG_ENTRIES / (4 * CWM_WAVE);
+        uint32_t marked = 0;
+#pragma unroll 1
+        for (int h = 0; h < LOADS; h += LOADS / 2) {
+          float4 f[LOADS / 2];  // in flight at once
+#pragma unroll
+          for (int q = 0; q < LOADS / 2; ++q) {
+            const int i = begin + 4 * ((h + q) * CWM_WAVE + lane);
+            f[q] = make_float4(-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff());
+            if (VEC) {
+              if (i < end) f[q] = *(const float4*)(x + i);
+            } else {
+              if (i < end) f[q].x = x[i];
+              if (i + 1 < end) f[q].y = x[i + 1];
+              if (i + 2 < end) f[q].z = x[i + 2];
+              if (i + 3 < end) f[q].w = x[i + 3];
+            }
+          }
+          auto in_bin = [&](float v) { return v * inv_w >= edge && v * inv_w < edge + 1.0f; };
+#pragma unroll
+          for (int q = 0; q < LOADS / 2; ++q) {
+            const uint32_t four = (in_bin(f[q].x) ? 1u : 0u) | (in_bin(f[q].y) ? 2u : 0u) | (in_bin(f[q].z) ? 4u : 0u) | (in_bin(f[q].w) ? 8u : 0u);
+            marked |= four << (4 * (h + q));
+          }
+        }
+        take(s, begin, marked);
+      }
+      __syncthreads();
+    };
+    auto entry_at = [&](int begin, int j) { return begin + 4 * ((j / 4) * CWM_WAVE + lane) + j % 4; };
+    // the marked entries go to the list; a wavefront takes its places there with one addition
+    auto list = [&](int begin, uint32_t marked) {
+      const int mine = __popc(marked);
+      int through = mine;
+#pragma unroll
+      for (int off = 1; off < CWM_WAVE; off <<= 1) {
+        const int o = __shfl_up(through, off, CWM_WAVE);
+        if (lane >= off) through += o;
+      }
+      int place = 0;
+      if (lane == CWM_WAVE - 1 && through > 0) place = atomicAdd(&sh.count, through);
+      place = __shfl(place, CWM_WAVE - 1, CWM_WAVE) + through - mine;
+      for (; marked; marked &= marked - 1, ++place) {
+        const int i = entry_at(begin, __ffs(marked) - 1);
+        if (place < SEG_LIST) sh.list_x[place] = x[i], sh.list_i[place] = i;
+      }
+    };
+    scan_bin([&](int, int begin, uint32_t marked) { list(begin, marked); });
+    int n = sh.count;
+    const bool all_listed = n <= SEG_LIST;
+    if (n > SEG_SORT) {
+      // 5. too many to put in order: the bin's 256 parts by their masses, and the entries of the part in which the point lies
+      auto add = [&](float v) { atomicAdd(&sh.sub[sub_of(v * inv_w)], (unsigned long long)(e_of(v) * SEG_FIXED)); };
+      if (all_listed) {
+        for (int j = tid; j < n; j += SAMPLE_THREADS) add(sh.list_x[j]);
+        __syncthreads();
+      } else {
+        scan_bin([&](int, int begin, uint32_t marked) {
+          for (; marked; marked &= marked - 1) add(x[entry_at(begin, __ffs(marked) - 1)]);
+        });
+      }
+      const float part = tid < SEG_BINS ? (float)sh.sub[tid] * (1.0f / SEG_FIXED) : 0.f;
+      const float run = block_scan(part, sh.scratch);
+      float before;
+      sub = first_past(sh, part, run, target - above, before);
+      above += before;
+      if (tid == 0) sh.count = 0;
+      __syncthreads();
+      if (all_listed) {
+        // the list's entries before the part are kept; the part's go to the list's front, once everything has been read
+        float v[SEG_LIST / SAMPLE_THREADS];
+        int at[SEG_LIST / SAMPLE_THREADS];
+#pragma unroll
+        for (int q = 0; q < SEG_LIST / SAMPLE_THREADS; ++q) {
+          const int j = q * SAMPLE_THREADS + tid;
+          v[q] = j < n ? sh.list_x[j] : 0.f;
+          at[q] = j < n ? sh.list_i[j] : -1;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < SEG_LIST / SAMPLE_THREADS; ++q) {
+          if (at[q] < 0) continue;
+          const int p = sub_of(v[q] * inv_w);
+          if (p < sub) atomicAdd(&sh.kept[at[q] / seg_len], (unsigned long long)(e_of(v[q]) * SEG_FIXED));
+          if (p == sub) {
+            const int place = atomicAdd(&sh.count, 1);
+            sh.list_x[place] = v[q], sh.list_i[place] = at[q];
+          }
+        }
+        __syncthreads();
+      } else {
+        scan_bin([&](int s, int begin, uint32_t marked) {
+          float whole = 0.f;
+          uint32_t in_part = 0;
+          for (; marked; marked &= marked - 1) {
+            const int j = __ffs(marked) - 1;
+            const float v = x[entry_at(begin, j)];
+            const int p = sub_of(v * inv_w);
+            if (p < sub) whole += e_of(v);
+            if (p == sub) in_part |= 1u << j;
+          }
+          whole = wave_sum(whole);
+          if (lane == 0) sh.kept[s] = (unsigned long long)(whole * SEG_FIXED);
+          list(begin, in_part);
+        });
+      }
+      n = sh.count;
+      if (n > SEG_SORT) {  // over a thousand entries within a 2,048th of an octave
+        return false;
+      }
+    }
+    // 6. an entry is kept if the mass of the larger ones does not pass the target: the listed ones in descending order
+    const float own = tid < n ? e_of(sh.list_x[tid]) : 0.f;
+    const int owner = tid < n ? sh.list_i[tid] / seg_len : 0;
+    float key = own;
+    int size = CWM_WAVE;
+    while (size < n) size <<= 1;
+    for (int k = 2; k <= size; k <<= 1)
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        float other;
+        if (j < CWM_WAVE) {
+          other = __shfl_xor(key, j, CWM_WAVE);
+        } else {
+          __syncthreads();
+          sh.sorted[tid] = key;
+          __syncthreads();
+          other = sh.sorted[tid ^ j];
+        }
+        key = ((tid & k) == 0) == ((tid & j) == 0) ? fmaxf(key, other) : fminf(key, other);
+      }
+    const float through = block_scan(key, sh.scratch);
+    if (tid < n && above + (through - key) <= target) atomicMin(&sh.smallest, __float_as_int(key));
+    __syncthreads();
+    least = __int_as_float(sh.smallest);
+    if (tid < n && own >= least) atomicAdd(&sh.kept[owner], (unsigned long long)(own * SEG_FIXED));
+    __syncthreads();
+    // the kept mass of every segment: its bins before `bin`, a wavefront a segment, and what the list gave
+    seg_mass = 0.f;
+    for (int s = wave; s < n_segs; s += SAMPLE_THREADS / CWM_WAVE) {
+      const float* hist = seg_histogram(row_workspace, n_segs, s);
+      float h = 0.f;
+#pragma unroll
+      for (int q = 0; q < SEG_BINS / CWM_WAVE; ++q) {
+        const int k = q * CWM_WAVE + lane;
+        if (k < SEG_BINS - 1 && k + sh.below[s] < bin) h += hist[k];
+      }
+      h = wave_sum(h);
+      if (lane == 0) sh.mass[s] = h * sh.scale[s] + (float)sh.kept[s] * (1.0f / SEG_FIXED);
+    }
+    __syncthreads();
+    seg_mass = tid < n_segs ? sh.mass[tid] : 0.f;
+  }
+
+  // 7. inverse CDF: the segment in which the running mass passes u * (kept mass), then the entry.  The two levels' sums are
+  //    rounded differently, so a level may find the point beyond its last mass: it then takes its last entry with mass.
+  const float run = block_scan(seg_mass, sh.scratch);
+  const float total = block_sum(seg_mass, sh.scratch);
+  const float target = u * total;
+  float before;
+  const int seg = first_past(sh, seg_mass, run, target, before);
+  if (seg < 0) {
+    return false;
+  }
+  const int begin = seg * seg_len, end = min(vocab, begin + seg_len);
+  const int i = begin + 2 * tid;  // two adjacent entries a thread
+  const float e0 = i < end ? kept(x[i]) : 0.f, e1 = i + 1 < end ? kept(x[i + 1]) : 0.f;
+  const float cum = block_scan(e0 + e1, sh.scratch);
+  float entry_before;
+  const int pick = first_past(sh, e0 + e1, cum, target - before, entry_before);
+  if (pick < 0) {
+    if (tid == 0) token_out[row] = best.i, logprob_out[row] = xmax - lse, sample_logprob_out[row] = logf(1.0f / total);
+    return true;
+  }
+  if (tid == pick) {
+    const bool second = !(e0 > 0.f) || (e1 > 0.f && entry_before + e0 <= target - before);
+    token_out[row] = second ? i + 1 : i;
+    logprob_out[row] = x[second ? i + 1 : i] - lse;
+    sample_logprob_out[row] = logf((second ? e1 : e0) / total);
+  }
+  return true;
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(SAMPLE_THREADS, 8)
+sample_join_kernel(const float* __restrict__ logits, long row_stride, int vocab, int seg_len, int n_segs, const float* __restrict__ temperature,
+                   const float* __restrict__ top_p, const float* __restrict__ uniform, float* __restrict__ workspace,
+                   int* __restrict__ token_out, float* __restrict__ logprob_out, float* __restrict__ sample_logprob_out) {
+  __shared__ union {
+    JoinShared join;
+    WholeRowShared whole;
+  } shared;
+  if (join_segments<VEC>(shared.join, blockIdx.x, logits, row_stride, vocab, seg_len, n_segs, temperature, top_p, uniform, workspace, token_out,
+                         logprob_out, sample_logprob_out))
+    return;
+  __syncthreads();
+  sample_whole_row<VEC>(shared.whole, blockIdx.x, logits, row_stride, vocab, temperature, top_p, uniform, workspace, token_out, logprob_out,
+                        sample_logprob_out);
+}
+
 static void launch_sample(const float* logits, long row_stride, int n_rows, int vocab, const float* temperature, const float* top_p,
                           const float* uniform, float* workspace, int* token_out, float* logprob_out, float* sample_logprob_out,
                           hipStream_t stream) {
   // four entries a load where every row of the logits and of the workspace starts at a multiple of 16 bytes
   const bool vec = vocab % 4 == 0 && row_stride % 4 == 0 && (uintptr_t)logits % 16 == 0 && (uintptr_t)workspace % 16 == 0;
+  // in segments where the row is long enough and their number fits the second kernel's lists; the records and histograms
+  // (1,040 bytes for every 1,024 entries or more) fit the row's part of the workspace
+  const int seg_len = seg_length(vocab), n_segs = (vocab + seg_len - 1) / seg_len;
+  if (vocab > SEGMENTS_FROM && n_segs <= SEG_MOST && n_rows <= 65535) {
+    auto launch = [&](auto v) {
+      hipLaunchKernelGGL(sample_segment_kernel<decltype(v)::value>, dim3(n_segs, n_rows), dim3(SEG_THREADS), 0, stream, logits, row_stride, vocab,
+                         seg_len, temperature, top_p, workspace);
+      hipLaunchKernelGGL(sample_join_kernel<decltype(v)::value>, dim3(n_rows), dim3(SAMPLE_THREADS), 0, stream, logits, row_stride, vocab, seg_len,
+                         n_segs, temperature, top_p, uniform, workspace, token_out, logprob_out, sample_logprob_out);
+    };
+    if (vec) launch(std::true_type());
+    else launch(std::false_type());
+    return;
+  }
   if (vec)
     hipLaunchKernelGGL(sample_kernel<true>, dim3(n_rows), dim3(SAMPLE_THREADS), 0, stream, logits, row_stride, vocab, temperature,
                        top_p, uniform, workspace, token_out, logprob_out, sample_logprob_out);

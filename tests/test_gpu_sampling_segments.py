@@ -1,0 +1,106 @@
+"""Sampling of rows that are cut into segments: vocabularies at the edges of segments and of 16-byte loads, distributions
+whose nucleus ends in a bin of few entries, of thousands and of equal ones, masked logits, extreme temperatures, and rows
+that one block does alone."""
+
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from plain import llama3_plain as plain
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _rows(vocab, g):
+    """Rows of logits by kind."""
+    normal = lambda std: torch.randn(vocab, generator=g) * std  # noqa: E731
+    peaked = normal(0.3)
+    peaked[vocab // 3] += 14.0
+    masked = torch.full((vocab,), -math.inf)
+    masked[vocab // 2 : vocab // 2 + 40] = normal(2.0)[:40]  # whole segments without an entry
+    far = normal(1.0) + 3000.0
+    few = torch.round(normal(2.0))  # many equal ones in every bin
+    return {"normal": normal(3.0), "flat": normal(0.02), "peaked": peaked, "masked": masked, "far": far, "equal": torch.zeros(vocab), "few": few}
+
+
+@pytest.mark.parametrize("vocab", [8192, 8193, 8256, 10243, 32768, 100003, 131072])
+def test_draws_follow_the_inverse_cdf_of_the_nucleus(vocab):
+    from cwm_amd import ops
+
+    g = torch.Generator().manual_seed(vocab)
+    rows, temps, tops, kinds = [], [], [], []
+    for kind, row in _rows(vocab, g).items():
+        for temp, top_p in ((0.0, 0.9), (0.7, 0.95), (1.0, 0.5), (1.3, 1.0), (0.9, 1e-6), (0.05, 0.9), (50.0, 0.8), (1.0, 0.9999)):
+            rows.append(row), temps.append(temp), tops.append(top_p), kinds.append(kind)
+    logits = torch.stack(rows)
+    n = len(rows)
+    us = torch.rand(n, generator=g)
+    us[::7], us[3::11] = 0.0, 1.0 - 2.0 ** -24
+    args = [t.to(DEV) for t in (logits, torch.tensor(temps), torch.tensor(tops), us)]
+    packed = ops.sample_packed(*args)
+    assert torch.equal(packed, ops.sample_packed(*args))  # the same bits every time
+    toks, lp, slp = (t.cpu() for t in ops.unpack_sampled(packed))
+    logp = torch.log_softmax(logits.double(), -1)
+    for r in range(n):
+        tok, where = int(toks[r]), f"vocabulary {vocab}, {kinds[r]}, temperature {temps[r]}, top_p {tops[r]}"
+        assert 0 <= tok < vocab, where
+        # 2^-24 of the logit itself (the far ones) beside the sum's rounding
+        np.testing.assert_allclose(float(lp[r]), float(logp[r, tok]), rtol=1e-4, atol=5e-4 if kinds[r] == "far" else 1e-4, err_msg=where)
+        if temps[r] <= 0:
+            assert tok == plain.greedy(logits[r]), where
+            continue
+        probs = torch.softmax(logits[r].double() / temps[r], -1)
+        values = torch.sort(probs, descending=True).values
+        above = torch.cumsum(values, 0) - values
+        # entries that are kept for certain and those that may be: equal ones are all kept, and a sum of float32 values is
+        # off by up to 1e-5 of the mass; float32 exponents of (x - max) / T are off by 1e-6 and, far from 0, by x's own rounding
+        off = 2e-5 if kinds[r] != "far" else 1e-3
+        least = float(values[above <= tops[r] + off][-1]) * (1 - 1e-4)
+        assert float(probs[tok]) >= least, where
+        kept = torch.where(probs >= float(values[above <= tops[r]][-1]) * (1 - 1e-6), probs, torch.zeros_like(probs))
+        total = float(kept.sum())
+        np.testing.assert_allclose(float(slp[r]), math.log(float(probs[tok]) / total), rtol=2e-3, atol=2e-3 if kinds[r] != "far" else 2e-2, err_msg=where)
+        cdf = torch.cumsum(kept / total, 0)
+        slack = 2e-3 if kinds[r] == "far" else 1e-4
+        assert float(cdf[tok] - kept[tok] / total) <= float(us[r]) + slack and float(cdf[tok]) >= float(us[r]) - slack, where
+
+
+def test_rows_that_one_block_does_alone():
+    """NaN, infinities and temperatures beyond the bins' range give what they gave in a row of one segment."""
+    from cwm_amd import ops
+
+    short = 2000
+    g = torch.Generator().manual_seed(5)
+    base = torch.randn(short, generator=g)
+    rows = []
+    for kind in range(6):
+        row = base.clone()
+        if kind == 0:
+            row[700] = math.nan
+        elif kind == 1:
+            row[:] = -math.inf
+        elif kind == 2:
+            row[[300, 900]] = math.inf
+        elif kind == 3:
+            row[:] = math.nan
+        elif kind == 4:
+            row *= 1e30
+        rows.append(row)
+    rows = torch.stack(rows).repeat_interleave(4, 0)
+    n = rows.shape[0]
+    temps = torch.tensor([0.0, 0.8, 0.8, 1e-9]).repeat(n // 4)
+    tops = torch.tensor([1.0, 0.9, 1.0, 0.9]).repeat(n // 4)
+    us = torch.full((n,), 0.4)
+    want = ops.sample(*(t.to(DEV) for t in (rows, temps, tops, us)))
+    # the same rows with entries behind them that nothing chooses
+    longer = torch.full((n, 9001), -math.inf)
+    longer[:, :short] = rows
+    got = ops.sample(*(t.to(DEV) for t in (longer, temps, tops, us)))
+    assert torch.equal(got[0], want[0])
+    for a, b in zip(got[1:], want[1:]):
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5, equal_nan=True)
