@@ -6,8 +6,9 @@
 //                    equal groups of neighbours, of which only those with the best members stay open to the choice.
 //   group_by_expert  the step's (token, choice) pairs grouped by expert, each group padded to whole tiles of 16
 //                    rows: row_token[row] (-1 in the padding), pair_row[pair], tile_expert[tile] (-1 beyond the
-//                    last tile).  One block; no count leaves the device.  The order of a group's rows is whatever
-//                    the block's atomic counters give: a row's result does not depend on its place.
+//                    last tile), and behind the last tile the number of tiles in use.  One block; no count leaves the
+//                    device.  The order of a group's rows is whatever the block's atomic counters give: a row's
+//                    result does not depend on its place.
 //   grouped product  out[row] = W[e(row)] a[row] on the matrix cores, e from tile_expert (16 rows a tile share it)
 //                    or, for a batch of independent products (one weight per head, say), from the block's z.
 //                    bfloat16 operands on v_mfma_f32_16x16x32_bf16, float32 operands on v_mfma_f32_16x16x4_f32
@@ -206,26 +207,64 @@ __device__ __forceinline__ void group_pairs(const int* chosen, int n_pairs, int 
                                             int tile_align, int* count, int* start) {
   for (int e = threadIdx.x; e < n_experts; e += blockDim.x) count[e] = 0;
   for (int i = threadIdx.x; i < n_tiles * TILE_ROWS; i += blockDim.x) row_token[i] = -1;
-  for (int i = threadIdx.x; i < n_tiles; i += blockDim.x) tile_expert[i] = -1;
   __syncthreads();
-  for (int i = threadIdx.x; i < n_pairs; i += blockDim.x) {
-    const int e = chosen[i];
-    if (e >= 0 && e < n_experts) atomicAdd(&count[e], 1);
+  constexpr int HELD = 8;  // a thread's first choices stay in registers
+  int held[HELD];
+#pragma unroll
+  for (int q = 0; q < HELD; ++q) {
+    const int i = threadIdx.x + q * blockDim.x;
+    held[q] = i < n_pairs ? chosen[i] : -1;
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int tile = 0;
-    for (int e = 0; e < n_experts; ++e) {
-      start[e] = tile * TILE_ROWS;
-      const int tiles = (count[e] + TILE_ROWS - 1) / TILE_ROWS;
-      for (int k = 0; k < tiles && tile + k < n_tiles; ++k) tile_expert[tile + k] = e;
-      tile += (tiles + tile_align - 1) / tile_align * tile_align;  // an expert's tiles start at a multiple of tile_align
-      count[e] = 0;
+  auto each_pair = [&](auto&& f) {
+#pragma unroll
+    for (int q = 0; q < HELD; ++q) {
+      const int i = threadIdx.x + q * blockDim.x;
+      if (i < n_pairs) f(i, held[q]);
     }
+    for (int i = threadIdx.x + HELD * blockDim.x; i < n_pairs; i += blockDim.x) f(i, chosen[i]);
+  };
+  each_pair([&](int, int e) {
+    if (e >= 0 && e < n_experts) atomicAdd(&count[e], 1);
+  });
+  __syncthreads();
+  if (threadIdx.x < CWM_WAVE) {
+    // four neighbouring experts a lane: an expert's tiles start at a multiple of tile_align behind the ones before
+    const int lane = threadIdx.x;
+    int tiles[4], sum = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int e = 4 * lane + q;
+      tiles[q] = e < n_experts ? ((count[e] + TILE_ROWS - 1) / TILE_ROWS + tile_align - 1) / tile_align * tile_align : 0;
+      sum += tiles[q];
+    }
+    int through = sum;
+#pragma unroll
+    for (int off = 1; off < CWM_WAVE; off <<= 1) {
+      const int o = __shfl_up(through, off, CWM_WAVE);
+      if (lane >= off) through += o;
+    }
+    int tile = through - sum;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (4 * lane + q < n_experts) start[4 * lane + q] = tile * TILE_ROWS;
+      tile += tiles[q];
+    }
+    if (lane == CWM_WAVE - 1) tile_expert[n_tiles] = min(through, n_tiles);
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < n_pairs; i += blockDim.x) {
-    const int e = chosen[i];
+  // tile by tile: the last expert that starts at it or before (those without rows start where the next one does)
+  for (int i = threadIdx.x; i < n_tiles; i += blockDim.x) {
+    int low = 0, high = n_experts - 1;
+    while (low < high) {
+      const int mid = (low + high + 1) >> 1;
+      if (start[mid] <= i * TILE_ROWS) low = mid; else high = mid - 1;
+    }
+    tile_expert[i] = i * TILE_ROWS < start[low] + count[low] ? low : -1;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n_experts; e += blockDim.x) count[e] = 0;
+  __syncthreads();
+  each_pair([&](int i, int e) {
     int row = -1;
     if (e >= 0 && e < n_experts) {
       row = start[e] + atomicAdd(&count[e], 1);
@@ -235,7 +274,7 @@ __device__ __forceinline__ void group_pairs(const int* chosen, int n_pairs, int 
         row = -1;
     }
     pair_row[i] = row;
-  }
+  });
 }
 
 __global__ void __launch_bounds__(1024) group_by_expert_kernel(const int* __restrict__ chosen, int n_pairs, int n_experts,
@@ -246,7 +285,7 @@ __global__ void __launch_bounds__(1024) group_by_expert_kernel(const int* __rest
   group_pairs(chosen, n_pairs, n_experts, row_token, pair_row, tile_expert, n_tiles, top, tile_align, count, start);
 }
 
-// tile_align: an expert's first tile lies at a multiple of so many tiles (the tiles that one block of the product takes).
+// tile_expert: n_tiles + 1 entries.  tile_align: an expert's first tile lies at a multiple of so many tiles (the tiles that one block of the product takes).
 extern "C" int cwm_group_by_expert(const int* chosen, int n_tokens, int top, int n_experts, int* row_token, int* pair_row,
                                    int* tile_expert, int n_tiles, int tile_align, hipStream_t stream) {
   CWM_REQUIRE(chosen && row_token && pair_row && tile_expert, "group_by_expert: arguments missing");
@@ -450,14 +489,19 @@ template <typename T, bool GATED>
 __global__ void __launch_bounds__(256) grouped_stream_kernel(const T* __restrict__ a, long a_ld, long a_batch, const int* __restrict__ row_token,
                                                              const T* __restrict__ w0, const T* __restrict__ w1, long w_stride,
                                                              const int* __restrict__ tile_expert, int n_tiles, void* __restrict__ out,
-                                                             int out_dtype, long out_ld, long out_batch, int n_rows, int N, int K, GateAct act) {
+                                                             int out_dtype, long out_ld, long out_batch, int n_rows, int N, int K, GateAct act,
+                                                             int tile_align) {
   __shared__ float sums[4][GATED ? 2 : 1][64][4];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int r = lane & 15, j = lane >> 4;
-  const int tile = blockIdx.x;
+  int tile = blockIdx.x;
   int expert;
   if (tile_expert) {
+    // the first tiles of the list's multiples, then the second ones, ...: few experts have a second tile, and blocks without
+    // work in regular places would leave whole XCDs without (they are dealt to the XCDs in turn; 22 and 35 us)
+    const int multiples = n_tiles / tile_align;
+    if (tile < multiples * tile_align) tile = tile % multiples * tile_align + tile / multiples;
     expert = tile < n_tiles ? tile_expert[tile] : -1;
     if (expert < 0) return;
   } else {
@@ -531,154 +575,149 @@ __global__ void __launch_bounds__(256) grouped_stream_kernel(const T* __restrict
   }
 }
 
-// Many rows an expert, bfloat16, K a multiple of 64: a block of four wavefronts (2 x 2) takes 8 row tiles of one expert
-// and 128 rows of weights (128 columns of the result; with two weights 64 columns of each), 64 values of k a step.
-// The step's 16 KB of rows and 16 KB of weights go from global memory to registers while the step before is
-// multiplied, then into the other of two LDS buffers (16-byte pieces, a row's pieces XOR-swizzled by the row so that
-// the lanes of a matrix operand read different banks); every wavefront multiplies 64 rows by 64 weight rows from there.
-template <bool GATED>
-__global__ void __launch_bounds__(256) grouped_tiled_kernel(const bf16_t* __restrict__ a, long a_ld, long a_batch, const int* __restrict__ row_token,
-                                                            const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, long w_stride,
-                                                            const int* __restrict__ tile_expert, int n_tiles, void* __restrict__ out,
-                                                            int out_dtype, long out_ld, long out_batch, int n_rows, int N, int K, GateAct act) {
-  extern __shared__ uint4 tiled_lds[];  // [2 buffers][rows: 128 x 8 pieces | weights: 128 x 8 pieces]
+// Many rows an expert, bfloat16, K a multiple of 64: a block of four wavefronts takes RT row tiles of one expert and 64 CT
+// rows of weights, 64 values of k a step.  Every wavefront multiplies all of the block's rows by CT weight tiles of its own
+// (with two weights half of them of each), so a piece of a weight tile is needed by one wavefront alone: it goes straight
+// to registers, half a step ahead of its use, and only the rows go through LDS (two buffers; 16-byte pieces, a row's pieces
+// XOR-swizzled by the row so that the lanes of a matrix operand read different banks).  That leaves LDS, which bounds a
+// block whose wavefronts share both operands, 40% busy beside the matrix cores.
+// With a list the blocks are numbered so that an XCD gets a run of neighbours in the order (group of WIDE_GROUP row blocks,
+// columns, row block): the row blocks of an expert then share its weights in one L2, where dealing them to the XCDs in turn
+// has every XCD read every expert's weights.  The list says how many tiles it holds, so the runs are equally long.
+// 16 experts of 2,048 x 1,024, four a token, gate and up / down: 2,048 tokens 128 / 71 us (535 / 484 TFLOP/s; blocks that
+// staged both operands through LDS: 204 / 135 us), 4,096 tokens 215 / 117 us (370 / 240 us), 300 tokens 51 / 30 us (117 / 79
+// us straight from memory); the last round of blocks is nearly empty at some sizes, which costs up to a quarter.
+#define WIDE_GROUP 4
+
+template <int RT, int CT, bool GATED>
+__global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __restrict__ a, long a_ld, long a_batch, const int* __restrict__ row_token,
+                                                              const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, long w_stride,
+                                                              const int* __restrict__ tile_expert, int n_tiles, int row_blocks, int col_blocks,
+                                                              void* __restrict__ out, int out_dtype, long out_ld, long out_batch, int vec_out,
+                                                              int n_rows, int N, int K, GateAct act) {
+  constexpr int ROWS = RT * TILE_ROWS, FETCH = ROWS * 8 / 256;  // 16-byte pieces of the rows that a thread fetches a step
+  constexpr int WT = GATED ? CT / 2 : CT;                       // column tiles of the result a wavefront makes
+  __shared__ uint4 lds_rows[2][ROWS * 8];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int wr = wave >> 1, wc = wave & 1;
   const int r = lane & 15, j = lane >> 4;
-  const int block_tile0 = blockIdx.x * 8;
-  int expert;
+  int bx, by, expert;
   if (tile_expert) {
-    expert = block_tile0 < n_tiles ? tile_expert[block_tile0] : -1;
+    const int live = (tile_expert[n_tiles] + RT - 1) / RT, total = live * col_blocks;
+    const int run = (total + 7) >> 3, at = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= run || at >= total) return;
+    const int first = at / (WIDE_GROUP * col_blocks) * WIDE_GROUP, rest = at - first * col_blocks;
+    const int together = min(WIDE_GROUP, live - first);
+    bx = first + rest % together;
+    by = rest / together;
+    expert = tile_expert[bx * RT];
     if (expert < 0) return;
   } else {
+    bx = blockIdx.x % row_blocks;
+    by = blockIdx.x / row_blocks;
     expert = blockIdx.z;
   }
-  constexpr int OUT_COLS = GATED ? 64 : 128;  // columns of the result a block makes
-  const int n0 = blockIdx.y * OUT_COLS;
-  // what this thread fetches every step: pieces id = threadIdx.x + 256 i, i < 4, of the rows and of the weights
-  const bf16_t* src_a[4];
-  const bf16_t* src_w[4];
+  const int tile0 = bx * RT;
+  const int n0 = by * (64 * WT) + wave * (16 * WT);
+  // rows that do not exist, and those of tiles that are another expert's, are read from a row that does; nothing uses the results
+  const bf16_t* src_a[FETCH];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < FETCH; ++i) {
     const int id = threadIdx.x + 256 * i;
-    const int row = id >> 3, piece = id & 7;
-    const int tile = block_tile0 + (row >> 4);
-    const bool live = tile_expert ? (tile < n_tiles && tile_expert[tile] == expert) : tile * TILE_ROWS < n_rows;
-    const int list_row = tile * TILE_ROWS + (row & 15);
-    long src = -1;
-    if (live) src = row_token ? row_token[list_row] : (list_row < n_rows ? list_row : -1);
-    src_a[i] = src >= 0 ? a + (size_t)blockIdx.z * a_batch + (size_t)src * a_ld + piece * 8 : nullptr;
-    int col;  // the weight row: with two weights rows 0..63 are the first one's, 64..127 the second one's
-    const bf16_t* w = w0;
-    if (GATED) {
-      col = n0 + (row & 63);
-      if (row >= 64) w = w1;
-    } else {
-      col = n0 + row;
-    }
-    src_w[i] = w + (size_t)expert * w_stride + (size_t)(col < N ? col : N - 1) * K + piece * 8;
+    const int list_row = tile0 * TILE_ROWS + (id >> 3);
+    long src;
+    if (tile_expert)
+      src = list_row < n_tiles * TILE_ROWS ? max(row_token[list_row], 0) : 0;
+    else
+      src = min(list_row, n_rows - 1);
+    src_a[i] = a + (size_t)blockIdx.z * a_batch + (size_t)src * a_ld + (id & 7) * 8;
   }
-  // three steps of operands on their way: what is fetched at the start of step k is put into LDS at the end of step k + 2
-  uint4 ra[3][4], rw[3][4];
-  auto fetch = [&](uint4 (&fa)[4], uint4 (&fw)[4], int k0) {
+  const bf16_t* we0 = w0 + (size_t)expert * w_stride;
+  const bf16_t* we1 = GATED ? w1 + (size_t)expert * w_stride : nullptr;
+  uint32_t src_w[CT];  // N * K < 2^31
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const bool inside = k0 < K;
-      fa[i] = (inside && src_a[i]) ? *(const uint4*)(src_a[i] + k0) : make_uint4(0, 0, 0, 0);
-      fw[i] = inside ? *(const uint4*)(src_w[i] + k0) : make_uint4(0, 0, 0, 0);
-    }
+  for (int ct = 0; ct < CT; ++ct) src_w[ct] = (uint32_t)min(n0 + (ct % WT) * 16 + r, N - 1) * (uint32_t)K + j * 8;
+  typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
+  Words4 ra[FETCH];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < FETCH; ++i) ra[i] = *(const Words4*)(src_a[i] + k0);
   };
-  auto stage = [&](const uint4 (&fa)[4], const uint4 (&fw)[4], int buf) {
-    uint4* rows = tiled_lds + buf * 2048;
-    uint4* weights = rows + 1024;
+  auto stage = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < FETCH; ++i) {
       const int id = threadIdx.x + 256 * i;
       const int row = id >> 3, piece = id & 7;
-      rows[row * 8 + (piece ^ (row & 7))] = fa[i];
-      weights[row * 8 + (piece ^ (row & 7))] = fw[i];
+      *(Words4*)&lds_rows[buf][row * 8 + (piece ^ (row & 7))] = ra[i];
     }
   };
-  float4v acc0[4][GATED ? 2 : 4], acc1[4][GATED ? 2 : 1];
+  Frag8 fw[2][CT];
+  auto load_weights = [&](int half, int k0) {
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt) {
+    for (int ct = 0; ct < CT; ++ct) fw[half][ct].u = *(const uint4*)((ct < WT ? we0 : we1) + (src_w[ct] + (uint32_t)(k0 + 32 * half)));
+  };
+  float4v acc[RT][CT];
 #pragma unroll
-    for (int ct = 0; ct < (GATED ? 2 : 4); ++ct) acc0[rt][ct] = (float4v){0.f, 0.f, 0.f, 0.f};
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int ct = 0; ct < (GATED ? 2 : 1); ++ct) acc1[rt][ct] = (float4v){0.f, 0.f, 0.f, 0.f};
-  }
-  auto multiply = [&](int buf) {
-    const uint4* rows = tiled_lds + buf * 2048;
-    const uint4* weights = rows + 1024;
+    for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = (float4v){0.f, 0.f, 0.f, 0.f};
+  const int steps = K / 64;
+  fetch(0);
+  load_weights(0, 0);
+  load_weights(1, 0);
+  stage(0);
+  fetch(min(1, steps - 1) * 64);
+  __syncthreads();
+  // No branch in the loop (the last steps load again what they have): with one around a load the compiler waits for the
+  // load where the paths meet.  The scheduling barriers keep the loads where they are, ahead of the other half's products.
+  for (int step = 0; step < steps; ++step) {
+    const uint4* rows = lds_rows[step & 1];
+    const int next = min(step + 1, steps - 1) * 64;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int piece = half * 4 + j;
-      Frag8 fa[4], fw[4];
+      Frag8 fa[RT];
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        const int row = wr * 64 + rt * 16 + r;
-        fa[rt].u = rows[row * 8 + (piece ^ (row & 7))];
-      }
+      for (int rt = 0; rt < RT; ++rt) fa[rt].u = rows[(rt * 16 + r) * 8 + (piece ^ (r & 7))];
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) {
-        // weight rows of this wavefront: 64 in a row, or (two weights) 32 of each
-        const int row = GATED ? (ct < 2 ? wc * 32 + ct * 16 + r : 64 + wc * 32 + (ct - 2) * 16 + r) : wc * 64 + ct * 16 + r;
-        fw[ct].u = weights[row * 8 + (piece ^ (row & 7))];
-      }
+      for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        if (GATED) {
-#pragma unroll
-          for (int ct = 0; ct < 2; ++ct) {
-            acc0[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[ct].v, fa[rt].v, acc0[rt][ct], 0, 0, 0);
-            acc1[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[2 + ct].v, fa[rt].v, acc1[rt][ct], 0, 0, 0);
-          }
-        } else {
-#pragma unroll
-          for (int ct = 0; ct < 4; ++ct) acc0[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[ct].v, fa[rt].v, acc0[rt][ct], 0, 0, 0);
-        }
-      }
+        for (int rt = 0; rt < RT; ++rt) acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[half][ct].v, fa[rt].v, acc[rt][ct], 0, 0, 0);
+      load_weights(half, next);
+      __builtin_amdgcn_sched_barrier(0);
     }
-  };
-  const int steps = K / 64;
-  fetch(ra[0], rw[0], 0);
-  stage(ra[0], rw[0], 0);
-  fetch(ra[1], rw[1], 64);
-  fetch(ra[2], rw[2], 128);
-  __syncthreads();
-  for (int base = 0; base < steps; base += 6) {  // six steps a turn: register set step % 3 and buffer step % 2 keep their names
-#pragma unroll
-    for (int u = 0; u < 6; ++u) {
-      const int step = base + u;
-      if (step >= steps) break;
-      fetch(ra[u % 3], rw[u % 3], (step + 3) * 64);  // this set's step went into LDS a step ago
-      multiply(u % 2);
-      stage(ra[(u + 1) % 3], rw[(u + 1) % 3], (u + 1) % 2);
-      __syncthreads();
-    }
+    stage((step + 1) & 1);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(min(step + 2, steps - 1) * 64);
+    __syncthreads();
   }
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt) {
-    const int tile = block_tile0 + wr * 4 + rt;
-    const bool live = tile_expert ? (tile < n_tiles && tile_expert[tile] == expert) : tile * TILE_ROWS < n_rows;
-    if (!live) continue;
-    const int row = tile * TILE_ROWS + r;
-    if (!tile_expert && row >= n_rows) continue;
+  for (int rt = 0; rt < RT; ++rt) {
+    const int tile = tile0 + rt, row = tile * TILE_ROWS + r;
+    if (tile_expert ? !(tile < n_tiles && tile_expert[tile] == expert) : row >= n_rows) continue;
     const size_t base = (size_t)blockIdx.z * out_batch + (size_t)row * out_ld;
 #pragma unroll
-    for (int ct = 0; ct < (GATED ? 2 : 4); ++ct)
+    for (int ct = 0; ct < WT; ++ct) {
+      const int c = n0 + ct * 16 + 4 * j;  // four adjacent columns
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = GATED ? gated_value(acc[rt][ct][i], acc[rt][ct + (GATED ? WT : 0)][i], act) : acc[rt][ct][i];
+      if (vec_out && c + 3 < N) {
+        if (out_dtype == CWM_F32)
+          *(float4*)((float*)out + base + c) = make_float4(v[0], v[1], v[2], v[3]);
+        else
+          *(uint2*)((bf16_t*)out + base + c) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+        continue;
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int c = n0 + (GATED ? wc * 32 : wc * 64) + ct * 16 + 4 * j + i;
-        if (c >= N) continue;
-        float v = acc0[rt][ct][i];
-        if (GATED) v = gated_value(v, acc1[rt][ct][i], act);
+        if (c + i >= N) continue;
         if (out_dtype == CWM_F32)
-          ((float*)out)[base + c] = v;
+          ((float*)out)[base + c + i] = v[i];
         else
-          ((bf16_t*)out)[base + c] = f32_to_bf16(v);
+          ((bf16_t*)out)[base + c + i] = f32_to_bf16(v[i]);
       }
+    }
   }
 }
 
@@ -699,13 +738,13 @@ static void launch_grouped(bool vec, int tiles, int n_batch, hipStream_t stream,
 // a: rows of K values, `a_ld` apart (row `row_token[row]` for list row `row` if a list is given; batch z starts
 // `a_batch` further).  w0 (and w1 for the gated form): [experts or batches][N][K], `w_stride` apart.  With
 // `tile_expert` the rows are the list's n_tiles * 16 and out is [rows][out_ld]; without, every batch z < n_batch
-// multiplies the same n_rows rows by its own weight into out + z * out_batch.  tiles_a_block: 1, 4 or 8 row tiles
-// a block (with a list, an expert's tiles start at a multiple of it).  act_kind, act_alpha, act_limit: the gated
+// multiplies the same n_rows rows by its own weight into out + z * out_batch.  tiles_a_block: 1, 2, 4 or 8 row tiles
+// a block; with a list, an expert's tiles start at a multiple of `tile_align`, itself a multiple of tiles_a_block.  act_kind, act_alpha, act_limit: the gated
 // form's activation (`GateAct`).
 extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int dtype, const int* row_token, const void* w0, const void* w1,
                                    long w_stride, const int* tile_expert, int n_tiles, int n_batch, void* out, int out_dtype, long out_ld,
-                                   long out_batch, int n_rows, int N, int K, int tiles_a_block, int act_kind, float act_alpha,
-                                   float act_limit, hipStream_t stream) {
+                                   long out_batch, int n_rows, int N, int K, int tiles_a_block, int tile_align, int act_kind,
+                                   float act_alpha, float act_limit, hipStream_t stream) {
   CWM_REQUIRE(a && w0 && out, "grouped_product: arguments missing");
   CWM_REQUIRE(act_kind >= 0 && act_kind <= 2, "grouped_product: unknown gated activation %d", act_kind);
   const GateAct act = {act_kind, act_alpha, act_limit};
@@ -717,7 +756,9 @@ extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int d
   const int piece = dtype == CWM_BF16 ? 8 : 4;
   const bool vec = K % piece == 0 && (a_ld * esize) % 16 == 0 && (a_batch * esize) % 16 == 0 && (w_stride * esize) % 16 == 0 &&
                    ((uintptr_t)a % 16) == 0 && ((uintptr_t)w0 % 16) == 0 && (!w1 || ((uintptr_t)w1 % 16) == 0);
-  CWM_REQUIRE(tiles_a_block == 1 || tiles_a_block == 4 || tiles_a_block == 8, "grouped_product: a block takes 1, 4 or 8 row tiles");
+  CWM_REQUIRE(tiles_a_block == 1 || tiles_a_block == 2 || tiles_a_block == 4 || tiles_a_block == 8, "grouped_product: a block takes 1, 2, 4 or 8 row tiles");
+  CWM_REQUIRE(!tile_expert || (tile_align >= 1 && tile_align % tiles_a_block == 0), "grouped_product: the list's tiles start at multiples of %d, a block takes %d",
+              tile_align, tiles_a_block);
   CWM_REQUIRE((N + 15) / 16 <= 65535, "grouped_product: too many columns");
   const int nb = tile_expert ? 1 : n_batch;
 #define CWM_GROUPED(T, RT, CT, WR, GATED)                                                                                                 \
@@ -735,30 +776,57 @@ extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int d
       else CWM_GROUPED(T, 1, 1, 1, false);                                      \
     }                                                                           \
   } while (0)
-  if (tiles_a_block == 1 && vec && (dtype == CWM_BF16 || dtype == CWM_F32)) {
+  if (tiles_a_block > 1 && vec && dtype == CWM_BF16 && K % 64 == 0 && (long)N * K < (1l << 31)) {
+    // the shape whose rows go through LDS
+    const int osize = out_dtype == CWM_F32 ? 4 : 2;
+    const int vec_out = (out_ld * osize) % (4 * osize) == 0 && (out_batch * osize) % (4 * osize) == 0 && ((uintptr_t)out % (4 * osize)) == 0;
+    const int row_blocks = (tiles + tiles_a_block - 1) / tiles_a_block;
+#define CWM_WIDE(RT, CT, GATED)                                                                                                            \
+  do {                                                                                                                                     \
+    const int cols = (GATED ? 32 : 64) * CT, col_blocks = (N + cols - 1) / cols;                                                           \
+    dim3 grid((row_blocks * col_blocks + 7) / 8 * 8, 1, nb);                                                                               \
+    if (!tile_expert) grid.x = row_blocks * col_blocks;                                                                                    \
+    hipLaunchKernelGGL((grouped_wide_kernel<RT, CT, GATED>), grid, dim3(256), 0, stream, (const bf16_t*)a, a_ld, a_batch, row_token,        \
+                       (const bf16_t*)w0, (const bf16_t*)w1, w_stride, tile_expert, n_tiles, row_blocks, col_blocks, out, out_dtype,       \
+                       out_ld, out_batch, vec_out, n_rows, N, K, act);                                                                     \
+  } while (0)
+    // Four weight tiles a wavefront where that still makes about two blocks a compute unit, else two, which makes twice as
+    // many blocks (measured with 16 experts of 2,048 x 1,024, gate and up: 200 rows an expert 96 and 81 us, 1,024 rows 214 and
+    // 220 us; 32 of 3,072 x 1,536: 256 rows 320 and 363 us).  Blocks of two row tiles stream the weights: always two.
+    const int blocks4 = row_blocks * ((N + (w1 ? 127 : 255)) / (w1 ? 128 : 256));
+    const bool many = tiles_a_block == 8 ? blocks4 >= 500 : tiles_a_block == 4 && blocks4 >= 560;
+#define CWM_WIDE_COLS(RT, GATED)   \
+  do {                             \
+    if (many)                      \
+      CWM_WIDE(RT, 4, GATED);      \
+    else                           \
+      CWM_WIDE(RT, 2, GATED);      \
+  } while (0)
+    if (w1) {
+      if (tiles_a_block == 8) CWM_WIDE_COLS(8, true);
+      else if (tiles_a_block == 4) CWM_WIDE_COLS(4, true);
+      else CWM_WIDE(2, 2, true);
+    } else {
+      if (tiles_a_block == 8) CWM_WIDE_COLS(8, false);
+      else if (tiles_a_block == 4) CWM_WIDE_COLS(4, false);
+      else CWM_WIDE(2, 2, false);
+    }
+#undef CWM_WIDE_COLS
+#undef CWM_WIDE
+    return cwm_launch_status("grouped_product");
+  }
+  if (tiles_a_block <= 2 && vec && (dtype == CWM_BF16 || dtype == CWM_F32)) {
     // the weight-streaming shape
     dim3 grid(tiles, (N + 15) / 16, nb);
 #define CWM_STREAMED(T, GATED)                                                                                                             \
   hipLaunchKernelGGL((grouped_stream_kernel<T, GATED>), grid, dim3(256), 0, stream, (const T*)a, a_ld, a_batch, row_token, (const T*)w0,     \
-                     (const T*)w1, w_stride, tile_expert, n_tiles, out, out_dtype, out_ld, out_batch, n_rows, N, K, act)
+                     (const T*)w1, w_stride, tile_expert, n_tiles, out, out_dtype, out_ld, out_batch, n_rows, N, K, act, tile_align)
     if (dtype == CWM_BF16) {
       if (w1) CWM_STREAMED(bf16_t, true); else CWM_STREAMED(bf16_t, false);
     } else {
       if (w1) CWM_STREAMED(float, true); else CWM_STREAMED(float, false);
     }
 #undef CWM_STREAMED
-    return cwm_launch_status("grouped_product");
-  }
-  if (tiles_a_block == 8 && vec && dtype == CWM_BF16 && K % 64 == 0) {
-    // the shape that goes through LDS
-    const size_t lds_bytes = 2 * 2048 * sizeof(uint4);
-    dim3 grid((tiles + 7) / 8, w1 ? (N + 63) / 64 : (N + 127) / 128, nb);
-    if (w1)
-      hipLaunchKernelGGL(grouped_tiled_kernel<true>, grid, dim3(256), lds_bytes, stream, (const bf16_t*)a, a_ld, a_batch, row_token,
-                         (const bf16_t*)w0, (const bf16_t*)w1, w_stride, tile_expert, n_tiles, out, out_dtype, out_ld, out_batch, n_rows, N, K, act);
-    else
-      hipLaunchKernelGGL(grouped_tiled_kernel<false>, grid, dim3(256), lds_bytes, stream, (const bf16_t*)a, a_ld, a_batch, row_token,
-                         (const bf16_t*)w0, (const bf16_t*)w1, w_stride, tile_expert, n_tiles, out, out_dtype, out_ld, out_batch, n_rows, N, K, act);
     return cwm_launch_status("grouped_product");
   }
   if (dtype == CWM_BF16)

@@ -14,8 +14,13 @@ from . import build as _build
 MAX_ROUTE_TOP = 16  # csrc/routed.hip: ROUTE_MAX_TOP
 MAX_EXPERTS = 256  # csrc/routed.hip: ROUTE_MAX_EXPERTS
 TILE_ROWS = 16  # rows of a tile of the grouped product
-MEDIUM_ROWS = 64  # from so many rows an expert (on average) a block of the grouped product takes 4 row tiles,
-WIDE_ROWS = 256  # and from so many, 8
+# From MEDIUM_ROWS rows an expert (on average) a block of the grouped product takes 4 row tiles instead of 2, and from
+# WIDE_ROWS, 8: at 16 experts of 2,048 x 1,024 gate, up and down together take 49 us with 2 and 4 tiles at 16 rows, 71 and
+# 50 us at 24; 76 us with 4 and 57 us with 8 at 48, where the busier experts have more than 64.
+MEDIUM_ROWS = 16
+WIDE_ROWS = 48
+STREAM_ROWS = 3  # up to so many rows an expert, gate and up go to the kernel that splits K: 28 instead of 30 us at 2 rows (weights
+# of 2,048 x 1,024), 102 instead of 115 us (3,072 x 1,536, 32 experts); at 4 rows 35 and 33 us, 134 and 124 us
 
 
 def _base():
@@ -71,14 +76,21 @@ class ExpertGroups:
 
     row_token: torch.Tensor  # int32 [tiles * 16]: the token of each row, -1 in the padding
     pair_row: torch.Tensor  # int32 [T * top]: the row of each pair
-    tile_expert: torch.Tensor  # int32 [tiles]: the expert of each tile, -1 for tiles not in use
+    tile_expert: torch.Tensor  # int32 [tiles]: the expert of each tile, -1 for tiles not in use (in memory, their number follows)
     n_tiles: int
-    tiles_a_block: int  # row tiles that one block of the grouped product takes (an expert's tiles start at a multiple)
+    tiles_a_block: int  # an expert's tiles start at a multiple of so many: the most row tiles that a block of the grouped product takes
     top: int
 
 
 def _tiles_a_block(rows: float) -> int:
-    return 8 if rows >= WIDE_ROWS else 4 if rows >= MEDIUM_ROWS else 1
+    return 8 if rows >= WIDE_ROWS else 4 if rows >= MEDIUM_ROWS else 2
+
+
+def _product_tiles(dtype: torch.dtype, k: int, rows: float, gated: bool) -> int:
+    """Row tiles that a block of the product takes: a divisor of the list's own multiple (`_tiles_a_block`)."""
+    if dtype != torch.bfloat16 or k % 64 != 0:  # the kernels whose operands do not go through LDS
+        return 8 if rows >= 256 else 4 if rows >= 64 else 1
+    return 1 if gated and rows < STREAM_ROWS else _tiles_a_block(rows)
 
 
 def group_by_expert(chosen: torch.Tensor, n_experts: int) -> ExpertGroups:
@@ -95,9 +107,9 @@ def group_by_expert(chosen: torch.Tensor, n_experts: int) -> ExpertGroups:
     pairs = n * top
     align = _tiles_a_block(pairs / n_experts)
     n_tiles = -(-pairs // TILE_ROWS) + n_experts * align
-    lists = torch.empty(n_tiles * TILE_ROWS + pairs + n_tiles, dtype=torch.int32, device=chosen.device)
+    lists = torch.empty(n_tiles * TILE_ROWS + pairs + n_tiles + 1, dtype=torch.int32, device=chosen.device)
     a, b = n_tiles * TILE_ROWS, n_tiles * TILE_ROWS + pairs
-    groups = ExpertGroups(lists[:a], lists[a:b], lists[b:], n_tiles, align, top)
+    groups = ExpertGroups(lists[:a], lists[a:b], lists[b:-1], n_tiles, align, top)
     lib = _build.load("routed")
     _check(
         lib,
@@ -111,14 +123,18 @@ def group_by_expert(chosen: torch.Tensor, n_experts: int) -> ExpertGroups:
 
 def _grouped(
     a: torch.Tensor, a_ld: int, a_batch: int, groups: Optional[ExpertGroups], w0: torch.Tensor, w1: Optional[torch.Tensor],
-    out: torch.Tensor, out_ld: int, out_batch: int, n_rows: int, n_batch: int, tiles_a_block: int,
+    out: torch.Tensor, out_ld: int, out_batch: int, n_rows: int, n_batch: int,
     activation: Optional["GatedActivation"] = None,
 ) -> None:
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
     _need_gpu(a, w0, w1, out)
     if w0.dim() != 3 or not w0.is_contiguous() or w0.dtype != a.dtype or (w1 is not None and (w1.shape != w0.shape or not w1.is_contiguous() or w1.dtype != a.dtype)):
         raise KernelError("grouped weights must be contiguous [experts, N, K] tensors of the rows' type")
-    _, n, k = w0.shape
+    e, n, k = w0.shape
+    if groups is not None:
+        tiles_a_block = min(groups.tiles_a_block, _product_tiles(a.dtype, k, groups.pair_row.numel() / e, w1 is not None))
+    else:  # a product a head: few rows go through the weights' stream
+        tiles_a_block = _product_tiles(a.dtype, k, n_rows, False) if n_rows >= MEDIUM_ROWS else 1
     lib = _build.load("routed")
     _check(
         lib,
@@ -128,6 +144,7 @@ def _grouped(
             _ptr(groups.tile_expert if groups is not None else None), ctypes.c_int(groups.n_tiles if groups is not None else 0),
             ctypes.c_int(n_batch), _ptr(out), ctypes.c_int(_code(out.dtype)), ctypes.c_long(out_ld), ctypes.c_long(out_batch),
             ctypes.c_int(n_rows), ctypes.c_int(n), ctypes.c_int(k), ctypes.c_int(tiles_a_block),
+            ctypes.c_int(groups.tiles_a_block if groups is not None else 1),
             ctypes.c_int(activation.code() if activation is not None else 0), ctypes.c_float(activation.alpha if activation is not None else 1.0),
             ctypes.c_float(activation.limit if activation is not None else 0.0), _stream(),
         ),
@@ -162,7 +179,7 @@ def grouped_gate_up(
     if x.dim() != 2 or not x.is_contiguous() or gate.shape[2] != x.shape[1]:
         raise KernelError("x must be a contiguous [T, D] tensor that fits the experts' weights")
     out = torch.empty((groups.n_tiles * TILE_ROWS, gate.shape[1]), dtype=x.dtype, device=x.device)
-    _grouped(x, x.shape[1], 0, groups, gate, up, out, gate.shape[1], 0, groups.n_tiles * TILE_ROWS, 1, groups.tiles_a_block, activation)
+    _grouped(x, x.shape[1], 0, groups, gate, up, out, gate.shape[1], 0, groups.n_tiles * TILE_ROWS, 1, activation)
     return out
 
 
@@ -174,7 +191,7 @@ def grouped_linear(rows: torch.Tensor, groups: ExpertGroups, weight: torch.Tenso
         raise KernelError("the rows do not fit the list or the experts' weights")
     out = torch.empty((rows.shape[0], weight.shape[1]), dtype=torch.float32, device=rows.device)
     identity = ExpertGroups(_identity_rows(rows.shape[0], rows.device), groups.pair_row, groups.tile_expert, groups.n_tiles, groups.tiles_a_block, groups.top)
-    _grouped(rows, rows.shape[1], 0, identity, weight, None, out, weight.shape[1], 0, rows.shape[0], 1, groups.tiles_a_block)
+    _grouped(rows, rows.shape[1], 0, identity, weight, None, out, weight.shape[1], 0, rows.shape[0], 1)
     return out
 
 
@@ -220,8 +237,7 @@ def absorb_queries(rest: torch.Tensor, ask: torch.Tensor, lead: int, weight: tor
     if rest.dim() != 3 or tuple(rest.shape) != (n_tokens, heads, weight.shape[2]) or rest.stride(2) != 1:
         raise KernelError(f"unrotated parts {tuple(rest.shape)} do not fit the heads' weights {tuple(weight.shape)}")
     if n_tokens:
-        tiles = _tiles_a_block(n_tokens)
-        _grouped(rest, max(rest.stride(0), heads * rest.shape[2]), rest.stride(1), None, weight, None, ask.view(-1)[lead:], heads * width, width, n_tokens, heads, tiles)
+        _grouped(rest, max(rest.stride(0), heads * rest.shape[2]), rest.stride(1), None, weight, None, ask.view(-1)[lead:], heads * width, width, n_tokens, heads)
     return ask
 
 
@@ -235,6 +251,5 @@ def expand_values(mixed: torch.Tensor, lead: int, weight: torch.Tensor) -> torch
     v = weight.shape[1]
     out = torch.empty((n_tokens, heads * v), dtype=mixed.dtype, device=mixed.device)
     if n_tokens:
-        tiles = _tiles_a_block(n_tokens)
-        _grouped(mixed.view(-1)[lead:], heads * width, width, None, weight, None, out, heads * v, v, n_tokens, heads, tiles)
+        _grouped(mixed.view(-1)[lead:], heads * width, width, None, weight, None, out, heads * v, v, n_tokens, heads)
     return out
