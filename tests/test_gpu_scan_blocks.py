@@ -1,0 +1,71 @@
+"""The selective scan of long bfloat16 portions, 64 tokens at a time on the matrix cores, against the recurrence in float64:
+portions that end inside a block of tokens, at its edge and one past it, states whose rows fill no tile of 16, columns that
+fill no block of 64, decays that forget within a token and ones that keep a state for thousands."""
+
+from __future__ import annotations
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _batch(q_lens, slots):
+    cu = torch.tensor([0] + q_lens).cumsum(0).int()
+    seq = torch.repeat_interleave(torch.arange(len(q_lens)), torch.tensor(q_lens)).int()
+    return SimpleNamespace(
+        n_tokens=sum(q_lens), n_seqs=len(q_lens), q_lens=list(q_lens), cu_q=cu.to(DEV), seq_of_token=seq.to(DEV),
+        state_slots=torch.tensor(slots, dtype=torch.int32, device=DEV), scratch={},
+    )
+
+
+def _exact(xbc, dt, bias, a_log, d_skip, state, q_lens, slots, heads, width, rows, groups):
+    """float64 on the CPU; `state` [slots, heads, rows, width] is updated."""
+    inner = heads * width
+    xs = xbc[:, :inner].reshape(-1, heads, width)
+    b, c = (t.reshape(-1, groups, rows).repeat_interleave(heads // groups, 1) for t in (xbc[:, inner : inner + groups * rows], xbc[:, inner + groups * rows :]))
+    dt = torch.nn.functional.softplus(dt + bias, threshold=100.0)
+    keep = torch.exp(-torch.exp(a_log) * dt)
+    y, at = torch.zeros_like(xs), 0
+    for q, slot in zip(q_lens, slots):
+        S = state[slot]
+        for t in range(at, at + q):
+            S = keep[t][:, None, None] * S + (dt[t][:, None] * b[t])[:, :, None] * xs[t][:, None, :]
+            y[t] = (S * c[t][:, :, None]).sum(1) + d_skip[:, None] * xs[t]
+        state[slot] = S
+        at += q
+    return y.reshape(-1, inner)
+
+
+@pytest.mark.parametrize("heads,width,rows,groups", [(4, 64, 128, 2), (2, 16, 8, 1), (3, 48, 72, 3), (2, 80, 64, 1), (1, 128, 24, 1)])
+@pytest.mark.parametrize("q_lens", [[257], [320, 1, 64], [5, 511, 768], [1025, 256]])
+def test_long_portions_against_float64(heads, width, rows, groups, q_lens):
+    from cwm_amd import ops
+
+    g = torch.Generator().manual_seed(sum(q_lens) + rows)
+    normal = lambda *shape: torch.randn(shape, generator=g)  # noqa: E731
+    slots = [2, 0, 1][: len(q_lens)]
+    total = heads * width + 2 * groups * rows
+    bias, d_skip = normal(heads) * 0.5, normal(heads)
+    a_log = torch.linspace(-7.0, 2.5, heads) if heads > 1 else torch.tensor([-2.0])
+    state = normal(3, heads, rows, width) * 0.3
+    packed = torch.stack([ops.scan_state_pack(s) for s in state]).to(DEV)
+    exact_state = state.double()
+    for _ in range(2):  # the second step goes on from the first one's states
+        n = sum(q_lens)
+        xbc, dt = normal(n, total).bfloat16(), (normal(n, heads) - 1).bfloat16()
+        dt[::97] += 24.0  # steps beyond the softplus' linear part
+        wide = torch.zeros((n, total + 24), dtype=torch.bfloat16, device=DEV)  # rows that lie apart
+        wide[:, :total] = xbc.to(DEV)
+        got = ops.selective_scan(wide[:, :total], dt.to(DEV), bias.to(DEV), a_log.to(DEV), d_skip.to(DEV), packed, _batch(q_lens, slots), heads, width, rows, groups)
+        want = _exact(xbc.double(), dt.double(), bias.double(), a_log.double(), d_skip.double(), exact_state, q_lens, slots, heads, width, rows, groups)
+        # float32 sums of at most some thousand terms: 64 roundings of 2^-24 of the values' size
+        scale = want.reshape(n, heads, width).abs().amax((0, 2)).clamp(min=1.0)
+        assert bool(((got.double().cpu() - want).reshape(n, heads, width).abs().amax((0, 2)) <= 4e-6 * scale).all())
+        for slot in range(3):
+            mine = ops.scan_state_unpack(packed[slot].cpu(), heads, width, rows).double()
+            size = exact_state[slot].abs().amax((1, 2)).clamp(min=1.0)
+            assert bool(((mine.reshape(heads, rows, width) - exact_state[slot]).abs().amax((1, 2)) <= 4e-6 * size).all())
