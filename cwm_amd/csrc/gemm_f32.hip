@@ -1,5 +1,6 @@
 // C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in true float32 on the matrix cores
-// (v_mfma_f32_32x32x2_f32: float32 operands, exact products, float32 sums): the matrix
+// (v_mfma_f32_32x32x2_f32: float32 operands, exact products, float32 sums; float32 operands with
+// K a multiple of 32 in exact bfloat16 parts instead, see below): the matrix
 // product of the 32-bit path.  Operands may be stored as float32 or bfloat16 (converted
 // exactly on load); nothing is rounded below float32 before the final store.  Every output
 // element is the sum over k = 0, 1, ... in one fixed grouping (eight values at a time, as the
@@ -43,21 +44,18 @@ __device__ __forceinline__ void load4(const T* row, int k, int K, bool vec, floa
 }
 
 // WAVES_M x WAVES_N wavefronts, each with TM x TN matrix-instruction tiles of 32 x 32; BK: a multiple of 8
+// One block's tile of the result, from row m0 and column n0 on; As, Ws: BM and BN rows of BK + 4 floats of LDS
 template <typename TA, typename TW, typename TC, int WAVES_M, int WAVES_N, int TM, int TN, int BK>
-__global__ void __launch_bounds__(64 * WAVES_M * WAVES_N)
-gemm_f32_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw, TC* __restrict__ C,
-                long ldc, const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int vec_a, int vec_w) {
+__device__ __forceinline__ void gemm_f32_tile(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw, TC* __restrict__ C, long ldc,
+                                              const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int vec_a, int vec_w, const int m0,
+                                              const int n0, float* As, float* Ws) {
   constexpr int BM = 32 * TM * WAVES_M, BN = 32 * TN * WAVES_N, THREADS = 64 * WAVES_M * WAVES_N;
   constexpr int BKP = BK + 4, Q = BK / 4;  // Q: 16-byte pieces in a row of a step
   constexpr int A_LOADS = (BM * Q + THREADS - 1) / THREADS, W_LOADS = (BN * Q + THREADS - 1) / THREADS;
-  __shared__ __attribute__((aligned(16))) float As[BM * BKP];
-  __shared__ __attribute__((aligned(16))) float Ws[BN * BKP];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  const int m0 = blockIdx.y * BM;
-  const int n0 = blockIdx.x * BN;
   const int r32 = lane & 31;  // the lane's row of a 32 x 32 operand
   const int kh = lane >> 5;   // and its half of the k values
 
@@ -146,12 +144,171 @@ gemm_f32_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lo
   }
 }
 
+template <typename TA, typename TW, typename TC, int WAVES_M, int WAVES_N, int TM, int TN, int BK>
+__global__ void __launch_bounds__(64 * WAVES_M * WAVES_N)
+gemm_f32_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw, TC* __restrict__ C,
+                long ldc, const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int vec_a, int vec_w) {
+  constexpr int BM = 32 * TM * WAVES_M, BN = 32 * TN * WAVES_N;
+  __shared__ __attribute__((aligned(16))) float As[BM * (BK + 4)];
+  __shared__ __attribute__((aligned(16))) float Ws[BN * (BK + 4)];
+  gemm_f32_tile<TA, TW, TC, WAVES_M, WAVES_N, TM, TN, BK>(A, lda, W, ldw, C, ldc, bias, bias_dtype, M, N, K, vec_a, vec_w, blockIdx.y * BM, blockIdx.x * BN,
+                                                          As, Ws);
+}
+
+// ---- float32 operands in three parts of eight bits ------------------------------------------------------------------ //
+// a = a1 + a2 + a3 exactly, each part a bfloat16: a1 = a rounded, a2 = a - a1 rounded (the difference is exact and has at
+// most 16 bits), a3 what is left (at most 8 bits).  a * w is then the sum of nine products of parts, exact in float32, of which
+// the six largest are added up on the bfloat16 matrix instruction (v_mfma_f32_16x16x32_bf16, float32 sums), 16 times the
+// rate of the float32 one: the three left out are below 2^-24 of the product together, and a sum takes 6 K / 32 roundings
+// instead of K / 2.  Against float64 (normal operands, K = 512, 4,096 and 14,336) a result is 3.4e-7, 1.0e-6 and 1.9e-6 off,
+// 4.1e-7, 1.15e-6 and 2.15e-6 with float32 operands; with positive operands 2.4e-7, 6.2e-7 and 1.2e-6 against 3.1e-7, 9.9e-7
+// and 1.8e-6.  Bound by the matrix cores and the vector instructions that make the parts (times that add).  743 rows, float32
+// operands and parts: 28,672 x 4,096 1,847 and 1,045 us (167 TFLOP/s of float32 products), 2,048 x 2,048 191 and 82 us; 64 rows
+// 6,144 x 4,096 361 and 144 us; 32 rows 168 and 94 us.
+// The parts are made on the way into LDS, so memory holds float32 as before.  The order of k and of the parts is the same for
+// every element of the result, whatever tile it lies in.  Values that round to infinity have no such parts: a block that
+// meets one (its largest magnitude says so) does its tile once more with float32 operands.
+#define SPLIT_STEP 32
+#define SPLIT_LD (SPLIT_STEP + 8)      // a row of a part in LDS: 80 bytes, so that 16 rows' pieces lie in different banks
+#define SPLIT_LIMIT 3.3895313e38f      // from here on bfloat16 rounds to infinity
+
+// WAVES_M x WAVES_N wavefronts, each with TM x TN tiles of 16 x 16
+template <typename TC, int WAVES_M, int WAVES_N, int TM, int TN>
+__global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, TM * TN <= 8 ? 3 : 2)
+gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, TC* __restrict__ C, long ldc,
+                      const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int row_blocks, int total) {
+  constexpr int BM = 16 * TM * WAVES_M, BN = 16 * TN * WAVES_N, THREADS = 64 * WAVES_M * WAVES_N;
+  constexpr int A_LOADS = BM * (SPLIT_STEP / 4) / THREADS, W_LOADS = BN * (SPLIT_STEP / 4) / THREADS;
+  constexpr int PARTS_BYTES = 3 * (BM + BN) * SPLIT_LD * 2, WHOLE_BYTES = (BM + BN) * (16 + 4) * 4;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[PARTS_BYTES > WHOLE_BYTES ? PARTS_BYTES : WHOLE_BYTES];
+  bf16_t* a_parts = (bf16_t*)lds;                  // [3][BM][SPLIT_LD]
+  bf16_t* w_parts = a_parts + 3 * BM * SPLIT_LD;   // [3][BN][SPLIT_LD]
+  // an XCD gets a run of neighbours, the row blocks of a panel of W one after the other: its L2 reads the panel once
+  const int run = (total + 7) >> 3, at = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= run || at >= total) return;
+  const int m0 = at % row_blocks * BM, n0 = at / row_blocks * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, j = lane >> 4;
+  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  // piece f of a step: row f / 8, values 4 (f % 8) .. + 3; rows past the last are read from the last, their results not written
+  const float* src_a[A_LOADS];
+  const float* src_w[W_LOADS];
+#pragma unroll
+  for (int i = 0; i < A_LOADS; ++i) src_a[i] = A + (size_t)min(m0 + (tid + i * THREADS) / 8, M - 1) * lda + 4 * (tid & 7);
+#pragma unroll
+  for (int i = 0; i < W_LOADS; ++i) src_w[i] = W + (size_t)min(n0 + (tid + i * THREADS) / 8, N - 1) * ldw + 4 * (tid & 7);
+  // two steps of operands on their way: what is fetched while step k is multiplied goes into LDS before step k + 2
+  float4v ra[2][A_LOADS], rw[2][W_LOADS];
+  auto fetch = [&](int set, int k) {
+    const int k0 = min(k, K - SPLIT_STEP);
+#pragma unroll
+    for (int i = 0; i < A_LOADS; ++i) ra[set][i] = *(const float4v*)(src_a[i] + k0);
+#pragma unroll
+    for (int i = 0; i < W_LOADS; ++i) rw[set][i] = *(const float4v*)(src_w[i] + k0);
+  };
+  float largest = 0.f;
+  auto stage = [&](float4v v, bf16_t* parts, int plane, int f) {
+    largest = fmaxf(largest, fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+    bf16_t* to = parts + (f / 8) * SPLIT_LD + 4 * (f % 8);
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+      const uint32_t lo = pack2_bf16(v[0], v[1]), hi = pack2_bf16(v[2], v[3]);
+      *(uint2*)(to + part * plane) = make_uint2(lo, hi);
+      v[0] -= __uint_as_float(lo << 16), v[1] -= __uint_as_float(lo & 0xffff0000u);
+      v[2] -= __uint_as_float(hi << 16), v[3] -= __uint_as_float(hi & 0xffff0000u);
+    }
+  };
+  float4v acc[TM][TN];
+#pragma unroll
+  for (int a = 0; a < TM; ++a)
+#pragma unroll
+    for (int b = 0; b < TN; ++b) acc[a][b] = (float4v){0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int set, int next) {
+#pragma unroll
+    for (int i = 0; i < A_LOADS; ++i) stage(ra[set][i], a_parts, BM * SPLIT_LD, tid + i * THREADS);
+#pragma unroll
+    for (int i = 0; i < W_LOADS; ++i) stage(rw[set][i], w_parts, BN * SPLIT_LD, tid + i * THREADS);
+    __syncthreads();
+    fetch(set, next);
+    Frag8 fa[3][TM];
+#pragma unroll
+    for (int part = 0; part < 3; ++part)
+#pragma unroll
+      for (int a = 0; a < TM; ++a) fa[part][a].u = *(const uint4*)(a_parts + (part * BM + (wm * TM + a) * 16 + r) * SPLIT_LD + 8 * j);
+#pragma unroll
+    for (int b = 0; b < TN; ++b) {
+      Frag8 fw[3];
+#pragma unroll
+      for (int part = 0; part < 3; ++part) fw[part].u = *(const uint4*)(w_parts + (part * BN + (wn * TN + b) * 16 + r) * SPLIT_LD + 8 * j);
+      constexpr int PART_A[6] = {2, 0, 1, 1, 0, 0}, PART_W[6] = {0, 2, 1, 0, 1, 0};  // the smaller products first
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int a = 0; a < TM; ++a) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[PART_W[q]].v, fa[PART_A[q]][a].v, acc[a][b], 0, 0, 0);
+    }
+    __syncthreads();
+  };
+  fetch(0, 0);
+  fetch(1, SPLIT_STEP);
+  int k0 = 0;
+  for (; k0 + 2 * SPLIT_STEP <= K; k0 += 2 * SPLIT_STEP) {
+    step(0, k0 + 2 * SPLIT_STEP);
+    step(1, k0 + 3 * SPLIT_STEP);
+  }
+  if (k0 < K) step(0, K);
+  if (__syncthreads_or(!(largest < SPLIT_LIMIT))) {
+    constexpr int WHOLE_M = BM / 32, WHOLE_N = BN / 32;
+    gemm_f32_tile<float, float, TC, WAVES_M, WAVES_N, WHOLE_M / WAVES_M, WHOLE_N / WAVES_N, 16>(A, lda, W, ldw, C, ldc, bias, bias_dtype, M, N, K, 1, 1, m0, n0,
+                                                                                                 (float*)lds, (float*)lds + BM * 20);
+    return;
+  }
+  // lane 16 j + r of a tile holds row r, columns 4 j + i
+#pragma unroll
+  for (int b = 0; b < TN; ++b)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int n = n0 + (wn * TN + b) * 16 + 4 * j + i;
+      if (n >= N) continue;
+      float add = 0.f;
+      if (bias) add = bias_dtype == CWM_BF16 ? bf16_to_f32(((const bf16_t*)bias)[n]) : ((const float*)bias)[n];
+#pragma unroll
+      for (int a = 0; a < TM; ++a) {
+        const int m = m0 + (wm * TM + a) * 16 + r;
+        if (m < M) Elem<TC>::store(C + (size_t)m * ldc + n, acc[a][b][i] + add);
+      }
+    }
+}
+
+template <typename TC>
+static void launch_split(const float* A, long lda, const float* W, long ldw, TC* C, long ldc, const void* bias, int bias_dtype, int M, int N, int K,
+                         hipStream_t stream) {
+#define CWM_SPLIT(WAVES_M, WAVES_N, TM, TN)                                                                                                \
+  do {                                                                                                                                     \
+    const int row_blocks = (M + 16 * TM * WAVES_M - 1) / (16 * TM * WAVES_M), total = row_blocks * ((N + 16 * TN * WAVES_N - 1) / (16 * TN * WAVES_N)); \
+    hipLaunchKernelGGL((gemm_f32_split_kernel<TC, WAVES_M, WAVES_N, TM, TN>), dim3((total + 7) / 8 * 8), dim3(64 * WAVES_M * WAVES_N), 0, stream, A,   \
+                       lda, W, ldw, C, ldc, bias, bias_dtype, M, N, K, row_blocks, total);                                                \
+  } while (0)
+  const long wide = (long)((M + 127) / 128) * ((N + 127) / 128);
+  if (M <= 32)
+    CWM_SPLIT(1, 2, 2, 2);
+  else if (M <= 64 || wide < 512)  // too few blocks of 128 x 128 for two a compute unit
+    CWM_SPLIT(2, 2, 2, 4);
+  else
+    CWM_SPLIT(2, 2, 4, 4);
+#undef CWM_SPLIT
+}
+
 template <typename TA, typename TW, typename TC>
 static void launch(const void* A, long lda, const void* W, long ldw, void* C, long ldc, const void* bias,
                    int bias_dtype, int M, int N, int K, hipStream_t stream) {
   // 16-byte loads of four values where every row allows them
   const int vec_a = lda % 4 == 0 && ((uintptr_t)A % 16) == 0;
   const int vec_w = ldw % 4 == 0 && ((uintptr_t)W % 16) == 0;
+  if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4) {
+    if (vec_a && vec_w && K % SPLIT_STEP == 0) {  // whatever M is: a row's result does not depend on the others
+      launch_split<TC>((const float*)A, lda, (const float*)W, ldw, (TC*)C, ldc, bias, bias_dtype, M, N, K, stream);
+      return;
+    }
+  }
   if (M > 32) {
     dim3 grid((N + 127) / 128, (M + 127) / 128);
     hipLaunchKernelGGL((gemm_f32_kernel<TA, TW, TC, 2, 2, 2, 2, 16>), grid, dim3(256), 0, stream, (const TA*)A, lda, (const TW*)W,

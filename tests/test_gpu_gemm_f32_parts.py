@@ -1,0 +1,70 @@
+"""The float32 product whose operands go to the matrix cores in three bfloat16 parts: sizes at the edges of its tiles and steps,
+values that need all 24 bits, of very different sizes, and ones that round to infinity in bfloat16."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _normal(shape, seed):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(DEV)
+
+
+@pytest.mark.parametrize("m", [1, 17, 32, 33, 64, 65, 130, 300])
+@pytest.mark.parametrize("n,k", [(1, 32), (63, 64), (129, 96), (520, 1056)])
+@pytest.mark.parametrize("c_dtype", [torch.float32, torch.bfloat16])
+def test_against_float64(m, n, k, c_dtype):
+    from cwm_amd import ops
+
+    a, w, b = _normal((m, k), m), _normal((n, k), n), _normal((n,), k)
+    got = ops.gemm_f32(a, w, b, out_dtype=c_dtype).double()
+    want = a.double() @ w.double().T + b.double()
+    # each of the k products is off by less than 2^-23 of itself, each of the 6 k / 32 sums by 2^-24 of the running sum
+    bound = (a.double().abs() @ w.double().abs().T) * 2.0 ** -23 + (0.2 * k + 2) * 2.0 ** -24 * (k ** 0.5 + 4)
+    if c_dtype == torch.bfloat16:
+        bound = bound + want.abs() * 2.0 ** -8
+    assert bool(((got - want).abs() <= bound).all())
+    # a row's bits do not depend on the others
+    for rows in (slice(0, 1), slice(m // 2, m)):
+        assert torch.equal(ops.gemm_f32(a[rows].contiguous(), w, b, out_dtype=c_dtype).double(), got[rows])
+
+
+def test_rows_that_lie_apart_and_values_of_all_sizes():
+    from cwm_amd import ops
+
+    m, n, k = 70, 200, 128
+    scale = 10.0 ** torch.linspace(-18, 18, k, device=DEV)  # the products are of order one, their parts from 1e-22 to 1e22
+    wide = _normal((m, k + 36), 1)
+    a = wide[:, 4 : 4 + k]
+    a *= scale
+    w = _normal((n, k), 2) / scale
+    got, want = ops.gemm_f32(a, w).double(), a.double() @ w.double().T
+    assert bool(((got - want).abs() <= (a.double().abs() @ w.double().abs().T) * 2.0 ** -21).all())
+    # numbers with all 24 bits set: a part less would show
+    a, w = torch.full((40, 32), 1.0 + 2.0 ** -23, device=DEV), torch.full((40, 32), 1.0 - 2.0 ** -24, device=DEV)
+    exact = 32.0 * (1.0 + 2.0 ** -23) * (1.0 - 2.0 ** -24)
+    assert float((ops.gemm_f32(a, w).double() - exact).abs().max()) <= 32 * 2.0 ** -23
+
+
+def test_values_beyond_the_parts():
+    """Infinities, NaN and the largest float32 values give what float32 gives."""
+    from cwm_amd import ops
+
+    m, n, k = 140, 150, 64
+    a, w = _normal((m, k), 3), _normal((n, k), 4)
+    a[5, 7], a[20, 1], a[139, 60] = math.inf, -math.inf, math.nan
+    a[60] = 0.0
+    a[60, 3] = 3.4e38
+    w[8, 3], w[9, 3] = 1.0, 0.5
+    w[100, 7] = 0.0
+    got, want = ops.gemm_f32(a, w), (a.double() @ w.double().T).float()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    fine = torch.isfinite(want)
+    torch.testing.assert_close(got[fine], want[fine], rtol=1e-5, atol=2e-5)
+    assert bool((got[~fine & ~torch.isnan(want)] == want[~fine & ~torch.isnan(want)]).all())
