@@ -972,13 +972,13 @@ class StaticPlans:
         self.homes: dict = {}  # (group, key/value heads, window, chunk) -> (capacity, device vector, uploaded plan)
 
     def _padded(self, batch, group: int, n_kv: int, window: Optional[int], capacity, chunk: Optional[int] = None):
-        from .attention_plan import build_plan, capacity_until, pad_plan
+        from .attention_plan import FEW_HEADS, build_plan, capacity_until, pad_plan
 
         wide_cut_below = -(-2 * _compute_units(self.device) // n_kv)
         if capacity is None:
-            plan, capacity = capacity_until(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, self.max_keys, chunk)
+            plan, capacity = capacity_until(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, self.max_keys, chunk, n_kv <= FEW_HEADS)
         else:
-            plan = build_plan(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, chunk)
+            plan = build_plan(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, chunk, n_kv <= FEW_HEADS)
         flat = pad_plan(plan, capacity)
         return plan, capacity, flat
 
@@ -1011,7 +1011,7 @@ class StaticPlans:
 
 def _attention_plan(batch, group: int, n_kv: int, window: Optional[int], device: torch.device, chunk: Optional[int] = None) -> _UploadedPlan:
     """The step's work list for this (group size, key/value heads, window or block of keys), uploaded once per step."""
-    from .attention_plan import build_plan
+    from .attention_plan import FEW_HEADS, build_plan
 
     static = getattr(batch, "static", None)
     if static is not None:
@@ -1021,7 +1021,7 @@ def _attention_plan(batch, group: int, n_kv: int, window: Optional[int], device:
     if cached is None:
         # a sequence whose blocks of 128 rows, over all key/value heads, would not give every compute unit two
         wide_cut_below = -(-2 * _compute_units(device) // n_kv) if device.type == "cuda" else 0
-        plan = build_plan(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, chunk)
+        plan = build_plan(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, chunk, n_kv <= FEW_HEADS)
         flat = np.concatenate([plan.work.reshape(-1), plan.work_wide.reshape(-1), plan.merge.reshape(-1)]).astype(np.int32)
         host = torch.from_numpy(flat)
         if device.type == "cuda":

@@ -22,18 +22,24 @@ WIDE_CHUNK = 8192  # keys after which such a block's range is cut (at fixed abso
 WIDE_CHUNK_FINE = 2048  # the same for a sequence with very few such blocks
 
 
-def chunk_keys(n_keys):
+def chunk_keys(n_keys, few_heads: bool = False):
     """Keys per chunk (a multiple of 128: four wavefronts take a chunk's tiles of 32 keys in turn) for a row tile
     that reads `n_keys` keys (a number or an array of them).  Up to 2,048 keys are not cut: a block of four
     wavefronts reads them and leaves no partial result (64 sequences of 1,024 keys: 45 us a layer of the 32B
     shape against 59 us in two chunks with their merge; a lone sequence of 1,024 keys pays 15 us against 10 us
     in chunks of 256).  Longer ranges are cut so that a few sequences still spread over the chip: 512 keys up
     to 8,192 (eight sequences in a window of 8,192 keys: 54 us against 58 us in chunks of 1,024), 1,024 up to
-    65,536, then 2,048 (eight sequences of 131,072 keys: 647 us against 665 us in chunks of 4,096)."""
+    65,536, then 2,048 (eight sequences of 131,072 keys: 647 us against 665 us in chunks of 4,096).
+    `few_heads` (see FEW_HEADS): chunks of 256 keys, of 512 beyond 8,192 and 1,024 beyond 65,536 keys.  With one key/value
+    head of 256 (attention through a latent) the chunks above leave most of the chip idle: eight sequences of 65 to
+    4,096 keys 45 us a layer and 19 us in chunks of 256, 48 of up to 2,048 keys 61 and 21 us, one of 4,096 20 and 17 us."""
     n = np.asarray(n_keys)
+    if few_heads:
+        return np.where(n <= 8192, 256, np.where(n <= 65536, 512, 1024))
     return np.where(n <= 2048, 2048, np.where(n <= 8192, 512, np.where(n <= 65536, 1024, 2048)))
 
 
+FEW_HEADS = 2  # key/value heads up to which a row tile's blocks are so few that its keys are cut finer
 MERGE_MID_MAX = 32  # partials up to which an item is merged by 4 wavefronts instead of 16
 WORK_INTS = 6
 PARTIAL_PAD = 4
@@ -62,12 +68,12 @@ def first_keys(last_key, window: Optional[int], chunk: Optional[int]):
 
 def build_plan(
     q_lens: Sequence[int], kv_lens: Sequence[int], group: int, window: Optional[int], wide_cut_below: int = 0,
-    chunk: Optional[int] = None,
+    chunk: Optional[int] = None, few_heads: bool = False,
 ) -> AttentionPlan:
     """`window` or `chunk` (at most one): which keys a query reads, see `first_keys`.  `wide_cut_below`: a sequence with fewer wide items than this has their keys cut at multiples of
     WIDE_CHUNK (its blocks alone would leave compute units idle), with fewer than an eighth of it at
     multiples of WIDE_CHUNK_FINE; the caller derives the number from the model's heads and the chip,
-    so that it is the same whatever else the batch holds."""
+    so that it is the same whatever else the batch holds.  `few_heads`: see `chunk_keys`."""
     q = np.asarray(q_lens, dtype=np.int64)
     kv = np.asarray(kv_lens, dtype=np.int64)
     n_rows = q * group
@@ -100,7 +106,7 @@ def build_plan(
     last_tok = np.minimum(row0 + ROWS_PER_TILE - 1, n_rows[seq] - 1) // group
     hi = n_old + last_tok + 1  # exclusive
     lo = first_keys(n_old + first_tok, window, chunk)
-    cut = chunk_keys(hi - lo)
+    cut = chunk_keys(hi - lo, few_heads)
     c0 = lo // cut
     n_chunks = (hi - 1) // cut - c0 + 1
     split = n_chunks > 1
@@ -231,17 +237,17 @@ CHUNK_RULE_ENDS = (2048, 8192, 65536)
 
 def capacity_until(
     q_lens: Sequence[int], kv_lens: Sequence[int], group: int, window: Optional[int], wide_cut_below: int, max_keys: int,
-    chunk: Optional[int] = None,
+    chunk: Optional[int] = None, few_heads: bool = False,
 ) -> "tuple[AttentionPlan, PlanCapacity]":
     """The step's plan, and the sizes of its lists for as long as no sequence holds more than `max_keys` keys
     (every sequence growing by a token a step): the sequences as they are, all of them grown to `max_keys`, and
     grown to each length in between at which the rule for cutting the keys changes."""
-    plan = build_plan(q_lens, kv_lens, group, window, wide_cut_below, chunk)
+    plan = build_plan(q_lens, kv_lens, group, window, wide_cut_below, chunk, few_heads)
     plans = [plan]
     for length in sorted({max_keys, *(n + d for n in CHUNK_RULE_ENDS for d in (0, 1) if n + d < max_keys)}):
         grown = [min(max(kv, length), max(kv, max_keys)) for kv in kv_lens]
         if grown != list(kv_lens):
-            plans.append(build_plan(q_lens, grown, group, window, wide_cut_below, chunk))
+            plans.append(build_plan(q_lens, grown, group, window, wide_cut_below, chunk, few_heads))
     capacity = PlanCapacity.covering(plans)
     span = window if chunk is None else chunk
     if span is not None and max(max(kv_lens), max_keys) > span:

@@ -1,0 +1,31 @@
+"""The work lists of attention with one or two key/value heads, whose keys are cut finer (host arithmetic only)."""
+
+import numpy as np
+import pytest
+
+from cwm_amd.ops.attention_plan import NULL_ROW, build_plan, capacity_until, pad_plan
+
+
+@pytest.mark.parametrize("window", [None, 100, 8192])
+@pytest.mark.parametrize("kv", [[1], [256], [257, 3], [8192, 8193, 40], [65536, 65537], [70000, 511, 513]])
+def test_keys_are_covered_once_at_every_length_of_the_rule(kv, window):
+    q = [1] * len(kv)
+    plan = build_plan(q, kv, 16, window, few_heads=True)
+    for b, n in enumerate(kv):
+        items = sorted(w[2:5] for w in plan.work.tolist() if w[0] == b)
+        lo = 0 if window is None else max(0, n - window)
+        cut = 256 if n - lo <= 8192 else 512 if n - lo <= 65536 else 1024
+        assert items[0][0] == lo and items[-1][1] == n and all(a[1] == c[0] for a, c in zip(items, items[1:]))
+        assert all(end - first <= cut and (first % cut == 0 or first == lo) for first, end, _ in items)
+        assert (len(items) == 1) == (items[0][2] == -1)
+
+
+@pytest.mark.parametrize("window", [None, 300])
+def test_captured_lists_hold_every_later_step(window):
+    q, kv, most = [1, 1, 1], [8000, 200, 255], 9000
+    plan, capacity = capacity_until(q, kv, 16, window, 0, most, few_heads=True)
+    for t in [0, 1, 2, 56, 57, 191, 192, 193, 194, 500, most - 8000]:
+        flat = pad_plan(build_plan(q, [n + t for n in kv], 16, window, few_heads=True), capacity)
+        assert flat is not None and flat.size == capacity.ints
+        work = flat[: capacity.work * 6].reshape(-1, 6)
+        assert np.all((work[:, 1] == NULL_ROW) | (work[:, 3] > work[:, 2]))
