@@ -182,13 +182,141 @@ token_side_kernel(float* __restrict__ h, const int* __restrict__ tokens, const T
   }
 }
 
+// The same for bfloat16 weights whose inputs are rounded, on the matrix cores: TOK tokens a block of sixteen wavefronts.  The
+// gate's product (16 tokens x side_dim, K = dim) is split over the wavefronts by columns and K, whose parts meet in LDS; the
+// projection's (16 x dim, K = side_dim) by columns.  Both weights are read as they lie, 16 bytes a lane, once a block: w_proj
+// is [dim, side_dim] here.  A lane's results are four adjacent elements of one token's row.  The kernel above is bound by its
+// multiply-adds and by LDS (every product's x and gated value is a read of its own): of width 2,048 with 64 side values and two
+// addends, 1,500 tokens take it 88 us and 4,096 169; here 37 and 54, bound by the latency of a block's three stages.  All of a
+// row's loads in flight at once (24 more registers a load stage) measured slower, 38 to 68 us: they spill.
+// dim: a multiple of 64 and at most 256 MAXT; side_dim: a multiple of 32, at most SIDE_TILE_MAX; rows of h, the addends and the
+// norm's weight start at multiples of 16 bytes (bfloat16 addends: of 8).
+#define SIDE_TILE_MAX 128
+
+template <int TOK, int MAXT>
+__global__ void __launch_bounds__(SIDE_THREADS)
+token_side_tile_kernel(float* __restrict__ h, const int* __restrict__ tokens, const bf16_t* __restrict__ table, long table_ld, int column0,
+                       const bf16_t* __restrict__ w_gate, const bf16_t* __restrict__ w_proj, const float* __restrict__ weight, int n_tokens,
+                       int dim, int side_dim, int vocab, float eps, SideAddends addends) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
+  constexpr int WAVES = SIDE_THREADS / CWM_WAVE, A_TOKEN = WAVES / TOK;  // wavefronts that load a token's row
+  const int x_ld = dim + 8;
+  bf16_t* xs = (bf16_t*)tile_lds;                                // [TOK][x_ld]
+  float* parts = (float*)(xs + (size_t)TOK * x_ld);              // [WAVES][16 side values][TOK]
+  bf16_t* gated = (bf16_t*)(parts + WAVES * 16 * TOK);           // [TOK][SIDE_TILE_MAX + 8]
+  float* squares = (float*)(gated + TOK * (SIDE_TILE_MAX + 8));  // [WAVES][TOK]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, j = lane >> 4;
+  const int t0 = blockIdx.x * TOK;
+  // 1. the rows: pending addends into the residual, bfloat16 into LDS
+  {
+    const int tok = wave / A_TOKEN, t = t0 + tok;
+    for (int e = 4 * ((wave % A_TOKEN) * CWM_WAVE + lane); e < dim; e += 4 * CWM_WAVE * A_TOKEN) {
+      float4v x = {0.f, 0.f, 0.f, 0.f};
+      if (t < n_tokens) {
+        x = *(const float4v*)(h + (size_t)t * dim + e);
+        for (int a = 0; a < addends.n; ++a) {
+          const SideAddend& ad = addends.a[a];
+          float4v y = {0.f, 0.f, 0.f, 0.f};
+          for (int p = 0; p < ad.n_partials; ++p) {
+            const size_t at = (size_t)p * ad.partial_stride + (size_t)t * ad.ld + e;
+            if (ad.dtype == CWM_F32) {
+              y += *(const float4v*)((const float*)ad.ptr + at);
+            } else {
+              const uint2 w = *(const uint2*)((const bf16_t*)ad.ptr + at);
+              y += (float4v){__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u)};
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[i] = fmaf(ad.scale, y[i], x[i]);
+        }
+        if (addends.n > 0) *(float4v*)(h + (size_t)t * dim + e) = x;  // read again at the end, after the block's barriers
+      }
+      *(uint2*)(xs + (size_t)tok * x_ld + e) = make_uint2(pack2_bf16(x[0], x[1]), pack2_bf16(x[2], x[3]));
+    }
+  }
+  __syncthreads();
+  // 2. the gate's product: wavefront w has the side values 16 (w % columns) .. + 15 and every k_parts-th step of K from w / columns on
+  const int columns = side_dim / 16, k_parts = WAVES / columns;
+  {
+    const int c = wave % columns, first = wave / columns;
+    float4v acc = {0.f, 0.f, 0.f, 0.f};
+    if (first < k_parts) {
+      const bf16_t* w = w_gate + (size_t)(16 * c + r) * dim + 8 * j;
+      const bf16_t* x = xs + (size_t)min(r, TOK - 1) * x_ld + 8 * j;
+#pragma unroll 4
+      for (int step = first; step < dim / 32; step += k_parts) {
+        Frag8 fw, fx;
+        fw.u = *(const uint4*)(w + 32 * step);
+        fx.u = *(const uint4*)(x + 32 * step);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw.v, fx.v, acc, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (r < TOK) parts[(wave * 16 + 4 * j + i) * TOK + r] = acc[i];
+  }
+  __syncthreads();
+  for (int id = threadIdx.x; id < TOK * side_dim; id += SIDE_THREADS) {
+    const int tok = id % TOK, k = id / TOK, t = t0 + tok;
+    float sum = 0.f;
+    for (int part = 0; part < k_parts; ++part) sum += parts[((part * columns + k / 16) * 16 + k % 16) * TOK + tok];
+    const float z = side_round(sum, true);
+    const float gelu = 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+    const int token = t < n_tokens ? tokens[t] : 0;
+    const bool known = token >= 0 && token < vocab;
+    const float e_k = known ? bf16_to_f32(table[(size_t)token * table_ld + column0 + k]) : __uint_as_float(0x7fc00000u);
+    gated[tok * (SIDE_TILE_MAX + 8) + k] = f32_to_bf16(gelu * e_k);
+  }
+  __syncthreads();
+  // 3. the projection: wavefront w has the tiles w, w + 16, ... of 16 elements; its squares; the scaled row into the residual
+  float4v y[MAXT];
+  float sq = 0.f;
+#pragma unroll
+  for (int q = 0; q < MAXT; ++q) {
+    y[q] = (float4v){0.f, 0.f, 0.f, 0.f};
+    const int e = 16 * (q * WAVES + wave);
+    if (e < dim) {
+      for (int k = 0; k < side_dim; k += 32) {
+        Frag8 fw, fg;
+        fw.u = *(const uint4*)(w_proj + (size_t)(e + r) * side_dim + k + 8 * j);
+        fg.u = *(const uint4*)(gated + min(r, TOK - 1) * (SIDE_TILE_MAX + 8) + k + 8 * j);
+        y[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw.v, fg.v, y[q], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sq = fmaf(y[q][i], y[q][i], sq);
+  }
+  sq += __shfl_xor(sq, 16, CWM_WAVE);
+  sq += __shfl_xor(sq, 32, CWM_WAVE);
+  if (j == 0 && r < TOK) squares[wave * TOK + r] = sq;
+  __syncthreads();
+  if (r >= TOK || t0 + r >= n_tokens) return;
+  float total = 0.f;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) total += squares[w * TOK + r];
+  const float rstd = 1.0f / sqrtf(total / (float)dim + eps);
+  float* row = h + (size_t)(t0 + r) * dim;
+#pragma unroll
+  for (int q = 0; q < MAXT; ++q) {
+    const int e = 16 * (q * WAVES + wave) + 4 * j;
+    if (e < dim) {
+      const float4v n = *(const float4v*)(weight + e);
+      float4v x = *(const float4v*)(row + e);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] += y[q][i] * rstd * n[i];
+      *(float4v*)(row + e) = x;
+    }
+  }
+}
+
 // h: float32 [T, dim], changed in place.  Addend a (n_addends of them, or none): ptrs[a] of dtypes[a], rows lds[a]
 // elements apart, n_partials[a] slabs partial_strides[a] elements apart, times scales[a]; they are added to h first.
 // tokens: int32 [T].  table: [vocab, >= column0 + side_dim] of `w_dtype`, rows
 // table_ld apart; w_gate [side_dim, dim] and w_proj_t [side_dim, dim] (the projection transposed) of `w_dtype`, contiguous;
+// w_proj: the projection as [dim, side_dim], or null (then the matrix cores are not used);
 // weight: float32 [dim].
 extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, long table_ld, int column0, const void* w_gate,
-                              const void* w_proj_t, int w_dtype, const float* weight, int n_tokens, int dim, int side_dim, int vocab,
+                              const void* w_proj_t, const void* w_proj, int w_dtype, const float* weight, int n_tokens, int dim, int side_dim, int vocab,
                               float eps, int round_inputs, int n_addends, const void* const* ptrs, const int* dtypes,
                               const long* lds_, const int* n_partials, const long* partial_strides, const float* scales,
                               hipStream_t stream) {
@@ -205,6 +333,31 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
     CWM_REQUIRE(ptrs[a] && n_partials[a] >= 1, "token_side: addend %d is empty", a);
     CWM_REQUIRE(n_partials[a] == 1 || dtypes[a] == CWM_F32, "token_side: partial sums must be float32");
     ad.a[a] = SideAddend{ptrs[a], lds_[a], partial_strides[a], n_partials[a], dtypes[a], scales[a]};
+  }
+  // from 256 tokens on (32 blocks of eight): with fewer the other kernel's blocks of one or two tokens spread over more of the chip
+  // (8 to 48 tokens of width 2,048: 19 us against 30; 300 tokens 44 against 31)
+  bool tiled = n_tokens >= 256 && w_proj && w_dtype == CWM_BF16 && round_inputs && dim % 64 == 0 && dim <= 4096 && side_dim % 32 == 0 && side_dim <= SIDE_TILE_MAX &&
+               (((uintptr_t)h | (uintptr_t)w_gate | (uintptr_t)w_proj | (uintptr_t)weight) % 16) == 0;
+  for (int a = 0; a < n_addends; ++a)
+    tiled = tiled && lds_[a] % 4 == 0 && partial_strides[a] % 4 == 0 && ((uintptr_t)ptrs[a] % (dtypes[a] == CWM_F32 ? 16 : 8)) == 0;
+  if (tiled) {
+    // sixteen tokens a block where that leaves no compute unit without one, else eight
+    const int tok = n_tokens >= 16 * 256 ? 16 : 8;
+    const size_t lds = (size_t)tok * (dim + 8) * 2 + 16 * 16 * tok * sizeof(float) + (size_t)tok * (SIDE_TILE_MAX + 8) * 2 + 16 * tok * sizeof(float);
+#define CWM_SIDE_TILE(TOK, MAXT)                                                                                                           \
+  do {                                                                                                                                     \
+    if (lds > 65536) (void)hipFuncSetAttribute((const void*)token_side_tile_kernel<TOK, MAXT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+    hipLaunchKernelGGL((token_side_tile_kernel<TOK, MAXT>), dim3((n_tokens + TOK - 1) / TOK), dim3(SIDE_THREADS), lds, stream, h, tokens,   \
+                       (const bf16_t*)table, table_ld, column0, (const bf16_t*)w_gate, (const bf16_t*)w_proj, weight, n_tokens, dim,        \
+                       side_dim, vocab, eps, ad);                                                                                          \
+  } while (0)
+    if (tok == 16) {
+      if (dim <= 2048) CWM_SIDE_TILE(16, 8); else CWM_SIDE_TILE(16, 16);
+    } else {
+      if (dim <= 2048) CWM_SIDE_TILE(8, 8); else CWM_SIDE_TILE(8, 16);
+    }
+#undef CWM_SIDE_TILE
+    return cwm_launch_status("token_side");
   }
   // tokens a block: as many (4, 2, 1) as fit the LDS and still leave the chip a block a few tokens
   int tok = 4;

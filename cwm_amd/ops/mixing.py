@@ -381,14 +381,16 @@ def short_conv(
 
 def token_side(
     h: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor, column0: int, w_gate: torch.Tensor, w_proj_t: torch.Tensor,
-    weight: torch.Tensor, eps: float, round_inputs: bool, pending: Any = None,
+    weight: torch.Tensor, eps: float, round_inputs: bool, pending: Any = None, w_proj: Optional[torch.Tensor] = None,
 ) -> None:
     """h (float32 [T, D]) += rms(y) * weight with y = w_proj (gelu_tanh(w_gate h) * e), e the columns column0 ..
     column0 + side_dim of the token's row of `table` ([vocab, n]); w_gate [side_dim, D], `w_proj_t` [side_dim, D] (the
     projection [D, side_dim] transposed, which the kernel reads along D) and the table have one type; `weight` float32 [D].  `round_inputs`: h and the gated values are rounded to bfloat16 where
-    they enter the two products.  float32 sums, activation and norm."""
+    they enter the two products.  float32 sums, activation and norm.  `w_proj`: the projection as it is, contiguous [D, side_dim];
+    with it bfloat16 weights and rounded inputs run on the matrix cores from 256
+    tokens on where the sizes allow."""
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
-    _need_gpu(h, tokens, table, w_gate, w_proj_t, weight)
+    _need_gpu(h, tokens, table, w_gate, w_proj_t, weight, w_proj)
     if h.dtype != torch.float32 or h.dim() != 2 or not h.is_contiguous():
         raise KernelError("the residual stream must be a contiguous float32 [T, D] tensor")
     n_tokens, dim = h.shape
@@ -400,6 +402,8 @@ def token_side(
     side_dim = w_gate.shape[0]
     if tuple(w_proj_t.shape) != (side_dim, dim) or not w_proj_t.is_contiguous():
         raise KernelError(f"the projection's weight must be handed over transposed, a contiguous [{side_dim}, {dim}] tensor")
+    if w_proj is not None and (tuple(w_proj.shape) != (dim, side_dim) or not w_proj.is_contiguous() or w_proj.dtype != w_proj_t.dtype):
+        raise KernelError(f"the projection's weight must be a contiguous [{dim}, {side_dim}] tensor of the other weights' type")
     if table.dim() != 2 or table.stride(1) != 1 or column0 < 0 or column0 + side_dim > table.shape[1]:
         raise KernelError(f"the table {tuple(table.shape)} has no columns {column0}..{column0 + side_dim - 1}")
     if not (table.dtype == w_gate.dtype == w_proj_t.dtype):
@@ -432,7 +436,7 @@ def token_side(
         lib,
         lib.cwm_token_side(
             _ptr(h), _ptr(tokens), _ptr(table), ctypes.c_long(table.stride(0)), ctypes.c_int(column0), _ptr(w_gate), _ptr(w_proj_t),
-            ctypes.c_int(_code(table.dtype)), _ptr(weight), ctypes.c_int(n_tokens), ctypes.c_int(dim), ctypes.c_int(side_dim),
+            _ptr(w_proj), ctypes.c_int(_code(table.dtype)), _ptr(weight), ctypes.c_int(n_tokens), ctypes.c_int(dim), ctypes.c_int(side_dim),
             ctypes.c_int(table.shape[0]), ctypes.c_float(eps), ctypes.c_int(int(round_inputs)), ctypes.c_int(len(terms)), ptrs, dtypes, lds,
             partials, strides, scales, _stream(),
         ),
