@@ -853,10 +853,38 @@ __global__ void __launch_bounds__(256) combine_routed_kernel(const float* __rest
   }
 }
 
+// The same sums, four adjacent elements a lane, four rows under way at a time (a choice without a row reads row 0 and
+// is left out): 2,296 tokens of 4 choices of 2,048 take 14.9 us where one element a load took 21.7, 300 tokens 2.4 of
+// 4.7 and one 1.9 of 3.9.  dim: a multiple of 4; rows at multiples of 16 bytes.
+__global__ void __launch_bounds__(256) combine_four_kernel(const float* __restrict__ rows, long rows_ld, const int* __restrict__ pair_row,
+                                                           const float* __restrict__ weights, float* __restrict__ out, int top, int dim) {
+  const size_t t = blockIdx.x;
+  for (int i = 4 * (blockIdx.y * blockDim.x + threadIdx.x); i < dim; i += 4 * gridDim.y * blockDim.x) {
+    float4v acc = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < top; k0 += 4) {
+      float4v x[4];
+      int row[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        row[u] = k0 + u < top ? pair_row[t * top + k0 + u] : -1;
+        x[u] = *(const float4v*)(rows + (size_t)(row[u] < 0 ? 0 : row[u]) * rows_ld + i);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (row[u] >= 0) acc += weights[t * top + k0 + u] * x[u];
+    }
+    *(float4v*)(out + t * dim + i) = acc;
+  }
+}
+
 extern "C" int cwm_combine_routed(const float* rows, long rows_ld, const int* pair_row, const float* weights, float* out, int n_tokens,
                                   int top, int dim, hipStream_t stream) {
   CWM_REQUIRE(rows && pair_row && weights && out && top >= 1 && dim > 0, "combine_routed: bad arguments");
   if (n_tokens <= 0) return 0;
+  if (dim % 4 == 0 && rows_ld % 4 == 0 && (((uintptr_t)rows | (uintptr_t)out) % 16) == 0) {
+    hipLaunchKernelGGL(combine_four_kernel, dim3(n_tokens, (dim + 1023) / 1024), dim3(256), 0, stream, rows, rows_ld, pair_row, weights, out, top, dim);
+    return cwm_launch_status("combine_routed");
+  }
   hipLaunchKernelGGL(combine_routed_kernel, dim3(n_tokens, (dim + 1023) / 1024), dim3(256), 0, stream, rows, rows_ld, pair_row, weights, out, top, dim);
   return cwm_launch_status("combine_routed");
 }
