@@ -13,8 +13,8 @@
 // of the step reads):
 //   1. `talk_scores_kernel`: a block a (row, key/value head, range of TALK_SPLIT columns) stages tiles of keys in LDS
 //      and leaves the scaled scores of the head's query heads;
-//   2. `talk_stats_kernel` (a block a (row, head): maximum and normaliser with the sink, over the columns the row
-//      may read) and `talk_mix_kernel` (a thread a column: every head's normalised weight, then the mixed weights,
+//   2. `talk_stats_kernel` (a wavefront a (row, head): maximum and normaliser with the sink, over the columns the row
+//      may read) and `talk_mix_kernel` (a thread a few columns: every head's normalised weight, then the mixed weights,
 //      written in the activation type; zero for a column the row does not read);
 //   3. `talk_values_kernel`: a block a (row, key/value head, range of columns) adds weight times value and leaves a
 //      partial sum a range, which the caller adds in their order (the weights are final, so the partial sums are plain).
@@ -32,7 +32,7 @@ CWM_DEFINE_ERROR_API
 #define TALK_SPLIT 128    // columns of a block's range (a multiple of the tile)
 #define TALK_MAX_HEADS 64
 #define TALK_MAX_HEAD_DIM 256
-#define TALK_MIX_COLUMNS 256  // columns of a block of the mixing kernel
+#define TALK_MIX_COLUMNS 256  // columns of a block of the mixing kernel for many heads
 
 extern "C" int cwm_talking_attention_split() { return TALK_SPLIT; }
 extern "C" int cwm_talking_attention_max_heads() { return TALK_MAX_HEADS; }
@@ -193,34 +193,166 @@ talk_scores_kernel(const T* __restrict__ q, long q_stride, const T* __restrict__
 }
 
 // ---- stage 2 -------------------------------------------------------------------------------------------------------- //
-// stats: [rows][heads][2]: the maximum (the sink included) and the inverse of the normaliser.  A block of four
-// wavefronts a (row, head), whatever the number of columns: the order of the sums hangs on the row alone.
+// stats: [rows][heads][2]: the maximum (the sink included) and the inverse of the normaliser.  A wavefront a (row, head): its
+// scores stay in registers between the maximum and the sum, so they are read once.  A row that reads more than they hold
+// (TALK_STATS_KEPT keys) has a block a head and is read twice: the order of the sums
+// hangs on the row alone.  A block a (row, head) that read each score twice, four bytes a load
+// took the two kernels of 16 heads, 1,024 rows of 1,024 columns, 76 us (8 heads: 38); with these two it is 40 (21).
+// V: columns of a load, at most those of the table; rows of scores start anywhere.
 #define TALK_STATS_THREADS 256
+#define TALK_STATS_KEPT 2048
+template <int V>
 __global__ void __launch_bounds__(TALK_STATS_THREADS)
 talk_stats_kernel(const float* __restrict__ scores, float* __restrict__ stats, const float* __restrict__ sink, TalkRows R,
                   TalkLayout L, int n_q_heads, int per, float score_scale) {
+  typedef float Part __attribute__((ext_vector_type(V), aligned(4)));
+  constexpr int WAVES = TALK_STATS_THREADS / CWM_WAVE, PARTS = TALK_STATS_KEPT / (CWM_WAVE * V);
   __shared__ float scratch[16];
-  const int r = blockIdx.x, g = blockIdx.y;
+  const int r = blockIdx.x, wave = threadIdx.x / CWM_WAVE, lane = threadIdx.x % CWM_WAVE;
   const TalkRow row = talk_row(R, r);
-  const float* s = scores + (size_t)(g / per) * L.stride_c + (size_t)r * L.stride_r + (size_t)(g % per) * L.stride_g - row.base;
-  float m = -__builtin_inff();
-  for (int j = row.first + threadIdx.x; j <= row.p; j += TALK_STATS_THREADS) m = fmaxf(m, s[j] * score_scale);
-  m = block_max(m, scratch);
-  if (sink) m = fmaxf(m, sink[g]);
-  float l = 0.f;
-  for (int j = row.first + threadIdx.x; j <= row.p; j += TALK_STATS_THREADS) l += __expf(s[j] * score_scale - m);  // a NaN among the scores stays
-  l = block_sum(l, scratch);
-  if (sink) l += __expf(sink[g] - m);
-  if (threadIdx.x == 0) {
+  // the columns the row reads, and where the load that holds the first of them starts
+  const int c0 = row.first - row.base, c1 = row.p - row.base, start = c0 - c0 % V;
+  const float none = -__builtin_inff();
+  // a load that would pass the table's last column starts earlier; the columns before its own place do not count
+  auto counts = [&](int c, int e) {
+    const int col = max(0, min(c, L.columns - V)) + e;
+    return col >= max(c, c0) && col <= c1;
+  };
+  auto part = [&](const float* s, int c) {
+    Part x = *(const Part*)(s + max(0, min(c, L.columns - V)));
+#pragma unroll
+    for (int e = 0; e < V; ++e) x[e] = counts(c, e) ? x[e] * score_scale : none;
+    return x;
+  };
+  auto largest = [&](const Part& x, float m) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) m = fmaxf(m, x[e]);
+    return m;
+  };
+  auto weights = [&](const Part& x, int c, float m, float l) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) l += counts(c, e) ? __expf(x[e] - m) : 0.f;  // a NaN among the scores stays
+    return l;
+  };
+  auto leave = [&](int g, float m, float l) {
+    if (sink) l += __expf(sink[g] - m);
     stats[((size_t)r * n_q_heads + g) * 2] = m;
     stats[((size_t)r * n_q_heads + g) * 2 + 1] = 1.0f / l;
+  };
+  auto scores_of = [&](int g) { return scores + (size_t)(g / per) * L.stride_c + (size_t)r * L.stride_r + (size_t)(g % per) * L.stride_g; };
+  if (c1 - start < TALK_STATS_KEPT) {
+    const int g = blockIdx.y * WAVES + wave;
+    if (g >= n_q_heads) return;  // and where the grid has a block a head, the blocks beyond the heads / WAVES
+    const float* s = scores_of(g);
+    Part x[PARTS];
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) {
+      const int at = start + CWM_WAVE * V * i;
+      if (at <= c1) x[i] = part(s, at + V * lane);
+    }
+    float m = none, l = 0.f;
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i)
+      if (start + CWM_WAVE * V * i <= c1) m = largest(x[i], m);
+    m = wave_max(m);
+    if (sink) m = fmaxf(m, sink[g]);
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) {
+      const int at = start + CWM_WAVE * V * i;
+      if (at <= c1) l = weights(x[i], at + V * lane, m, l);
+    }
+    l = wave_sum(l);
+    if (lane == 0) leave(g, m, l);
+    return;
+  }
+  const int g = blockIdx.y;
+  const float* s = scores_of(g);
+  float m = none, l = 0.f;
+#pragma unroll 4
+  for (int c = start + V * threadIdx.x; c <= c1; c += V * TALK_STATS_THREADS) m = largest(part(s, c), m);
+  m = block_max(m, scratch);
+  if (sink) m = fmaxf(m, sink[g]);
+#pragma unroll 4
+  for (int c = start + V * threadIdx.x; c <= c1; c += V * TALK_STATS_THREADS) l = weights(part(s, c), c, m, l);
+  l = block_sum(l, scratch);
+  if (threadIdx.x == 0) leave(g, m, l);
+}
+
+// weights: the layout of the scores, of TW; zero in the columns (below L.columns) that a row does not read.  A thread has V
+// adjacent columns and holds every head's weights of them (at most HEADS) in registers; the coefficients are the same for the
+// whole block and come as scalars; through LDS they and the weights were two LDS reads a multiply-add.  Bound by the latency of a
+// wavefront's loads (100 MB, 2.5 TB/s with the statistics): two columns a thread measured slower (52 us).
+// V <= L.columns; rows start anywhere.
+template <typename TW, int HEADS, int V>
+__global__ void __launch_bounds__(CWM_WAVE)
+talk_mix_kernel(const float* __restrict__ scores, const float* __restrict__ stats, const float* __restrict__ talk,
+                TW* __restrict__ weights, TalkRows R, TalkLayout L, int n_q_heads, int per, float score_scale) {
+  typedef float Part __attribute__((ext_vector_type(V), aligned(4)));
+  typedef uint32_t Packed __attribute__((ext_vector_type(2), aligned(2)));
+  // the thread that would pass the last column takes columns of its neighbour again and writes the same there
+  const int r = blockIdx.x, place = V * (blockIdx.y * CWM_WAVE + threadIdx.x), col = min(place, L.columns - V);
+  const TalkRow row = talk_row(R, r);
+  const int c0 = row.first - row.base, c1 = row.p - row.base;
+  const size_t at = (size_t)r * L.stride_r + col;
+  auto leave = [&](int h, Part w) {
+    if (place >= L.columns) return;
+#pragma unroll
+    for (int e = 0; e < V; ++e) w[e] = col + e >= c0 && col + e <= c1 ? w[e] : 0.f;
+    TW* to = weights + (size_t)(h / per) * L.stride_c + (size_t)(h % per) * L.stride_g + at;
+    if constexpr (V == 1)
+      Elem<TW>::store(to, w[0]);
+    else if constexpr (sizeof(TW) == 2)
+      *(Packed*)to = (Packed){pack2_bf16(w[0], w[1]), pack2_bf16(w[2], w[3])};
+    else
+      *(Part*)to = w;
+  };
+  const int block0 = V * blockIdx.y * CWM_WAVE;
+  if (block0 > c1 || block0 + V * CWM_WAVE <= c0) {  // the row reads none of the block's columns
+    Part zero;
+#pragma unroll
+    for (int e = 0; e < V; ++e) zero[e] = 0.f;
+    for (int h = 0; h < n_q_heads; ++h) leave(h, zero);
+    return;
+  }
+  Part p[HEADS];
+#pragma unroll
+  for (int g = 0; g < HEADS; ++g) {
+    const int head = min(g, n_q_heads - 1);
+    p[g] = *(const Part*)(scores + (size_t)(head / per) * L.stride_c + (size_t)(head % per) * L.stride_g + at);
+  }
+#pragma unroll
+  for (int g = 0; g < HEADS; ++g) {
+    const int head = min(g, n_q_heads - 1);
+    const float m = stats[((size_t)r * n_q_heads + head) * 2], inverse = stats[((size_t)r * n_q_heads + head) * 2 + 1];
+#pragma unroll
+    for (int e = 0; e < V; ++e) p[g][e] = g < n_q_heads ? __expf(p[g][e] * score_scale - m) * inverse : 0.f;
+  }
+  if (!talk) {
+#pragma unroll
+    for (int h = 0; h < HEADS; ++h)
+      if (h < n_q_heads) leave(h, p[h]);
+    return;
+  }
+  for (int h = 0; h < n_q_heads; ++h) {
+    const float* trow = talk + (size_t)h * n_q_heads;
+    Part w;
+#pragma unroll
+    for (int e = 0; e < V; ++e) w[e] = 0.f;
+#pragma unroll
+    for (int g = 0; g < HEADS; ++g) {
+      const float t = g < n_q_heads ? trow[min(g, n_q_heads - 1)] : 0.f;
+#pragma unroll
+      for (int e = 0; e < V; ++e) w[e] = fmaf(t, p[g][e], w[e]);
+    }
+    leave(h, w);
   }
 }
 
-// weights: the layout of the scores, of TW; zero in the columns (below L.columns) that a row does not read
+// The same for more than sixteen heads, whose weights go through LDS: in registers they leave too few wavefronts (32 heads, 1,024
+// rows of 1,024 columns: 196 us with the statistics against 149; 64 heads 632 against 593).
 template <typename TW>
 __global__ void __launch_bounds__(TALK_MIX_COLUMNS)
-talk_mix_kernel(const float* __restrict__ scores, const float* __restrict__ stats, const float* __restrict__ talk,
+talk_mix_many_kernel(const float* __restrict__ scores, const float* __restrict__ stats, const float* __restrict__ talk,
                 TW* __restrict__ weights, TalkRows R, TalkLayout L, int n_q_heads, int per, float score_scale) {
   extern __shared__ __attribute__((aligned(16))) float probs[];  // [heads][TALK_MIX_COLUMNS]
   const int r = blockIdx.x;
@@ -249,6 +381,33 @@ talk_mix_kernel(const float* __restrict__ scores, const float* __restrict__ stat
     }
     Elem<TW>::store(weights + (size_t)(h / per) * L.stride_c + (size_t)(h % per) * L.stride_g + at, reads ? w : 0.f);
   }
+}
+
+// Stage 2 on n_rows rows.
+template <typename TW>
+static void talk_normalise(const float* scores, float* stats, const float* sink, const float* talk, TW* weights, const TalkRows& R, const TalkLayout& L,
+                           int n_rows, int n_q_heads, int per, float scale, hipStream_t stream) {
+  const int waves = TALK_STATS_THREADS / CWM_WAVE;
+  const dim3 heads(n_rows, L.columns < TALK_STATS_KEPT ? (n_q_heads + waves - 1) / waves : n_q_heads);  // a block a head where a row may need it
+  if (L.columns >= 4)
+    hipLaunchKernelGGL(talk_stats_kernel<4>, heads, dim3(TALK_STATS_THREADS), 0, stream, scores, stats, sink, R, L, n_q_heads, per, scale);
+  else
+    hipLaunchKernelGGL(talk_stats_kernel<1>, heads, dim3(TALK_STATS_THREADS), 0, stream, scores, stats, sink, R, L, n_q_heads, per, scale);
+#define CWM_TALK_MIX(HEADS, V)                                                                                                        \
+  hipLaunchKernelGGL((talk_mix_kernel<TW, HEADS, V>), dim3(n_rows, (L.columns + V * CWM_WAVE - 1) / (V * CWM_WAVE)), dim3(CWM_WAVE), 0, \
+                     stream, scores, stats, talk, weights, R, L, n_q_heads, per, scale)
+  // four columns a thread where that leaves every SIMD a wavefront (eight rows of 1,152 columns, 16 heads: 15 us with four, 12.6 with one)
+  const bool four = L.columns >= 4 && (long)n_rows * L.columns >= 1 << 18;
+  if (n_q_heads <= 8 && four) CWM_TALK_MIX(8, 4);
+  else if (n_q_heads <= 8) CWM_TALK_MIX(8, 1);
+  else if (n_q_heads <= 16 && four) CWM_TALK_MIX(16, 4);
+  else if (n_q_heads <= 16) CWM_TALK_MIX(16, 1);
+  else {
+    const size_t lds = sizeof(float) * (size_t)n_q_heads * TALK_MIX_COLUMNS;
+    hipLaunchKernelGGL((talk_mix_many_kernel<TW>), dim3(n_rows, (L.columns + TALK_MIX_COLUMNS - 1) / TALK_MIX_COLUMNS), dim3(TALK_MIX_COLUMNS), lds, stream,
+                       scores, stats, talk, weights, R, L, n_q_heads, per, scale);
+  }
+#undef CWM_TALK_MIX
 }
 
 // ---- stage 3 -------------------------------------------------------------------------------------------------------- //
@@ -414,8 +573,6 @@ extern "C" int cwm_talking_attention(const void* q, long q_stride, int dtype, co
   const TalkCache ch{n_kv_heads, head_dim, page_size, num_pages, table_width};
   const int ranges = columns / TALK_SPLIT;
   const dim3 grid(n_rows, n_kv_heads, ranges);
-  const size_t lds2 = sizeof(float) * (size_t)n_q_heads * TALK_MIX_COLUMNS;
-  const dim3 grid_mix(n_rows, (columns + TALK_MIX_COLUMNS - 1) / TALK_MIX_COLUMNS);
 #define CWM_TALK_VALUES(T, NACC)                                                                                          \
   hipLaunchKernelGGL((talk_values_kernel<T, T, NACC>), grid, dim3(TALK_THREADS), lds3, stream, (const T*)weights,          \
                      (const T*)cache, block_table, partial, R, L, ch, n_q_heads, n_rows)
@@ -423,10 +580,7 @@ extern "C" int cwm_talking_attention(const void* q, long q_stride, int dtype, co
   do {                                                                                                                    \
     hipLaunchKernelGGL((talk_scores_kernel<T>), grid, dim3(TALK_THREADS), lds1, stream, (const T*)q, q_stride,             \
                        (const T*)cache, block_table, scores, R, L, ch, n_q_heads, scale);                                  \
-    hipLaunchKernelGGL(talk_stats_kernel, dim3(n_rows, n_q_heads), dim3(TALK_STATS_THREADS), 0, stream, scores, stats, sink, R, L,   \
-                       n_q_heads, per, 1.0f);                                                                              \
-    hipLaunchKernelGGL((talk_mix_kernel<T>), grid_mix, dim3(TALK_MIX_COLUMNS), lds2, stream, scores, stats, talk,          \
-                       (T*)weights, R, L, n_q_heads, per, 1.0f);                                                           \
+    talk_normalise<T>(scores, stats, sink, talk, (T*)weights, R, L, n_rows, n_q_heads, per, 1.0f, stream);                 \
     if (per * head_dim <= TALK_THREADS) CWM_TALK_VALUES(T, 1);                                                             \
     else if (per * head_dim <= 4 * TALK_THREADS) CWM_TALK_VALUES(T, 4);                                                    \
     else CWM_TALK_VALUES(T, 16);                                                                                           \
@@ -454,13 +608,10 @@ extern "C" int cwm_talking_mix(const float* scores, void* weights, int w_dtype, 
   const int per = n_q_heads / n_kv_heads;
   const TalkRows R{nullptr, nullptr, nullptr, nullptr, nullptr, pos0, base, window_left};
   const TalkLayout L{(long)n_rows * per * columns, (long)per * columns, (long)columns, columns};
-  const size_t lds2 = sizeof(float) * (size_t)n_q_heads * TALK_MIX_COLUMNS;
-  const dim3 grid_mix(n_rows, (columns + TALK_MIX_COLUMNS - 1) / TALK_MIX_COLUMNS);
-  hipLaunchKernelGGL(talk_stats_kernel, dim3(n_rows, n_q_heads), dim3(TALK_STATS_THREADS), 0, stream, scores, stats, sink, R, L, n_q_heads, per, scale);
   if (w_dtype == CWM_F32)
-    hipLaunchKernelGGL((talk_mix_kernel<float>), grid_mix, dim3(TALK_MIX_COLUMNS), lds2, stream, scores, stats, talk, (float*)weights, R, L, n_q_heads, per, scale);
+    talk_normalise<float>(scores, stats, sink, talk, (float*)weights, R, L, n_rows, n_q_heads, per, scale, stream);
   else if (w_dtype == CWM_BF16)
-    hipLaunchKernelGGL((talk_mix_kernel<bf16_t>), grid_mix, dim3(TALK_MIX_COLUMNS), lds2, stream, scores, stats, talk, (bf16_t*)weights, R, L, n_q_heads, per, scale);
+    talk_normalise<bf16_t>(scores, stats, sink, talk, (bf16_t*)weights, R, L, n_rows, n_q_heads, per, scale, stream);
   else
     return cwm_fail("talking_mix: unknown element type %d", w_dtype);
   return cwm_launch_status("talking_mix");
