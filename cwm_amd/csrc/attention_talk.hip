@@ -306,8 +306,9 @@ talk_mix_kernel(const float* __restrict__ scores, const float* __restrict__ stat
     else
       *(Part*)to = w;
   };
+  // the row reads none of the columns that the block's threads write, which in the last block may start before its own place
   const int block0 = V * blockIdx.y * CWM_WAVE;
-  if (block0 > c1 || block0 + V * CWM_WAVE <= c0) {  // the row reads none of the block's columns
+  if (min(block0, L.columns - V) > c1 || block0 + V * CWM_WAVE <= c0) {
     Part zero;
 #pragma unroll
     for (int e = 0; e < V; ++e) zero[e] = 0.f;

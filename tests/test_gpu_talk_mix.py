@@ -1,5 +1,5 @@
 """Normalising and mixing a table of scores: tables narrower than a load, odd widths, rows that read a part of them and rows beyond
-what a wavefront keeps, few and many heads."""
+what a wavefront keeps, few and many heads, and widths whose last block has only threads that start in the block before."""
 
 from __future__ import annotations
 
@@ -13,7 +13,11 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("n_q,n_kv", [(4, 2), (7, 7), (16, 4), (20, 5)])
-@pytest.mark.parametrize("rows,columns,base,window", [(1, 1, 0, None), (2, 3, 5, 1), (4, 4, 0, None), (37, 130, 9, 60), (300, 1001, 11, 500), (260, 1024, 0, None), (9, 4099, 3, None), (5, 2052, 0, 2049)])
+@pytest.mark.parametrize(
+    "rows,columns,base,window",
+    [(1, 1, 0, None), (2, 3, 5, 1), (4, 4, 0, None), (37, 130, 9, 60), (300, 1001, 11, 500), (260, 1024, 0, None), (9, 4099, 3, None), (5, 2052, 0, 2049),
+     (513, 513, 0, None), (514, 514, 0, None), (515, 515, 0, None), (769, 769, 0, None), (400, 770, 0, 300)],
+)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_against_float64(n_q, n_kv, rows, columns, base, window, dtype):
     from cwm_amd.ops import _check, _code, _ptr, _stream
