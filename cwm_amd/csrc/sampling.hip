@@ -371,6 +371,14 @@ __device__ __forceinline__ float* seg_histogram(float* row_workspace, int n_segs
 // the bin of x counted downwards from the one of `top` (both times 8 / (T ln 2))
 __device__ __forceinline__ int bins_below(float top_floor, float scaled) { return (int)fminf(top_floor - floorf(scaled), (float)(SEG_BINS - 1)); }
 
+// The part of its bin in which `scaled` (x * 8 / (T ln 2), rounded) lies, counted downwards.  The fraction comes from the same rounded
+// number as the bin: contracted with the multiplication before it, it may be negative and the part lie outside the bin.
+__device__ __forceinline__ int part_of_bin(float scaled) {
+#pragma clang fp contract(off)
+  const float fraction = scaled - floorf(scaled);
+  return SEG_BINS - 1 - max(0, min(SEG_BINS - 1, (int)(fraction * SEG_BINS)));
+}
+
 template <bool VEC>
 __global__ void __launch_bounds__(SEG_THREADS)
 sample_segment_kernel(const float* __restrict__ logits, long row_stride, int vocab, int seg_len, const float* __restrict__ temperature,
@@ -543,14 +551,13 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
   float least = 0.f;                   // kept of part `sub` (of the whole bin if it is not divided): the entries from here on
   auto e_of = [&](float v) { return expf((v - xmax) * inv_t); };
   auto bin_of = [&](float scaled) { return bins_below(top_floor, scaled); };
-  auto sub_of = [&](float scaled) { return SEG_BINS - 1 - min(SEG_BINS - 1, (int)((scaled - floorf(scaled)) * SEG_BINS)); };
   auto kept = [&](float v) {
     if (!nucleus) return v > -__builtin_inff() ? e_of(v) : 0.f;
     const float scaled = v * inv_w;
     const int k = v > -__builtin_inff() ? bin_of(scaled) : SEG_BINS;
     if (k != bin) return k < bin ? e_of(v) : 0.f;
     if (sub < SEG_BINS) {
-      const int j = sub_of(scaled);
+      const int j = part_of_bin(scaled);
       if (j != sub) return j < sub ? e_of(v) : 0.f;
     }
     const float e = e_of(v);
@@ -643,7 +650,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
     const bool all_listed = n <= SEG_LIST;
     if (n > SEG_SORT) {
       // 5. too many to put in order: the bin's 256 parts by their masses, and the entries of the part in which the point lies
-      auto add = [&](float v) { atomicAdd(&sh.sub[sub_of(v * inv_w)], (unsigned long long)(e_of(v) * SEG_FIXED)); };
+      auto add = [&](float v) { atomicAdd(&sh.sub[part_of_bin(v * inv_w)], (unsigned long long)(e_of(v) * SEG_FIXED)); };
       if (all_listed) {
         for (int j = tid; j < n; j += SAMPLE_THREADS) add(sh.list_x[j]);
         __syncthreads();
@@ -656,6 +663,9 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
       const float run = block_scan(part, sh.scratch);
       float before;
       sub = first_past(sh, part, run, target - above, before);
+      if (sub < 0) {  // no part with mass
+        return false;
+      }
       above += before;
       if (tid == 0) sh.count = 0;
       __syncthreads();
@@ -673,7 +683,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
 #pragma unroll
         for (int q = 0; q < SEG_LIST / SAMPLE_THREADS; ++q) {
           if (at[q] < 0) continue;
-          const int p = sub_of(v[q] * inv_w);
+          const int p = part_of_bin(v[q] * inv_w);
           if (p < sub) atomicAdd(&sh.kept[at[q] / seg_len], (unsigned long long)(e_of(v[q]) * SEG_FIXED));
           if (p == sub) {
             const int place = atomicAdd(&sh.count, 1);
@@ -688,7 +698,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
           for (; marked; marked &= marked - 1) {
             const int j = __ffs(marked) - 1;
             const float v = x[entry_at(begin, j)];
-            const int p = sub_of(v * inv_w);
+            const int p = part_of_bin(v * inv_w);
             if (p < sub) whole += e_of(v);
             if (p == sub) in_part |= 1u << j;
           }

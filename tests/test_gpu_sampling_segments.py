@@ -104,3 +104,37 @@ def test_rows_that_one_block_does_alone():
     assert torch.equal(got[0], want[0])
     for a, b in zip(got[1:], want[1:]):
         torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("value,temp", [(25.0, 0.001), (650.25, 0.05), (-25.0, 0.001), (650.25, 0.01), (3.1, 1.0)])
+@pytest.mark.parametrize("ties", [600, 1025, 1500, 4096, 6000])
+def test_ties_that_a_rounded_product_leaves_at_a_bins_edge(value, temp, ties):
+    """More entries of the decisive bin than are put in order, far from 0, where x / T lies a rounding above a bin's edge."""
+    from cwm_amd import ops
+
+    vocab = 20000
+    g = torch.Generator().manual_seed(ties)
+    base = torch.tensor(value)
+    step = base.abs() * 2.0 ** -22  # a few units of the last place
+    row = torch.full((vocab,), value - 60 * temp)
+    order = torch.randperm(vocab, generator=g)
+    row[order[:ties]] = base
+    row[order[ties : 2 * ties]] = base + step  # in the same bin, in another part or the same
+    row[order[2 * ties]] = value + 2 * temp
+    n = 24
+    us, tops = torch.rand(n, generator=g), torch.tensor([0.2, 0.5, 0.999]).repeat(n // 3)
+    temps = torch.full((n,), temp)
+    toks, lp, slp = (t.cpu() for t in ops.sample(row.repeat(n, 1).to(DEV), temps.to(DEV), tops.to(DEV), us.to(DEV)))
+    x = (row.double() - row.double().max()) * float(1.0 / torch.tensor(temp))
+    probs = torch.softmax(x, -1)
+    values = torch.sort(probs, descending=True).values
+    above = torch.cumsum(values, 0) - values
+    for r in range(n):
+        least = float(values[above <= float(tops[r])][-1])
+        kept = torch.where(probs >= least * (1 - 1e-9), probs, torch.zeros_like(probs))
+        cdf = torch.cumsum(kept / kept.sum(), 0)
+        tok = int(toks[r])
+        # the weights' exponents are float32 numbers of at most 60, and sums of thousands of equal weights are off by 1e-6
+        assert kept[tok] > 0, (r, tok)
+        assert float(cdf[tok] - kept[tok] / kept.sum()) <= float(us[r]) + 2e-5 and float(cdf[tok]) >= float(us[r]) - 2e-5, (r, tok)
+        np.testing.assert_allclose(float(slp[r]), math.log(float(kept[tok] / kept.sum())), atol=2e-5)
