@@ -337,8 +337,10 @@ sample_kernel(const float* __restrict__ logits, long row_stride, int vocab, cons
 // the segments' records together.  The nucleus is found through a histogram of mass instead of passes over the row: a bin
 // is floor(x * 8 / (T ln 2)), an eighth of an octave of e^(x/T), the same bin in every segment whatever its maximum, and the
 // bin in which the mass from the top passes top_p * z is the only one whose entries have to be looked at.  Masses that
-// several threads add to one place are integers (units of 2^-40 of the largest entry), so their order does not matter and
-// a row's result is the same every time.
+// several threads add to one place are integers, so their order does not matter and a row's result is the same every time: units
+// of 2^-52 of a segment's largest entry (the 2,048 entries of a segment fit 64 bits), of 2^-44 of the row's where all of its entries may
+// meet.  Entries of up to 29 octaves below the segment's largest are exact in them; what the smaller ones are rounded by is below
+// 2^-25 of the kept mass together (at most 2^19 entries, half a unit each), less than the rounding of a float32 sum.
 #define SEG_THREADS 256
 #define SEG_PER_THREAD 8
 #define SEG_ENTRIES (SEG_THREADS * SEG_PER_THREAD)
@@ -347,7 +349,8 @@ sample_kernel(const float* __restrict__ logits, long row_stride, int vocab, cons
 #define SEGMENTS_FROM 8192  // longer rows are cut: the second launch costs 4 us, and a nucleus in a row of 8,192 takes 37 us as a whole, 20 to 28 in segments
 #define SEG_LIST 4096    // entries of the decisive bin that are kept in LDS
 #define SEG_SORT 1024    // and those of its decisive part that are put in order
-#define SEG_FIXED 1099511627776.0f  // 2^40
+#define SEG_FIXED 4503599627370496.0f  // 2^52
+#define ROW_FIXED 17592186044416.0f    // 2^44
 
 struct SegRecord {
   float max;
@@ -430,7 +433,7 @@ sample_segment_kernel(const float* __restrict__ logits, long row_stride, int voc
       z += e;
       if (nucleus) {
         const int k = bins_below(top_floor, v[j] * inv_w);
-        if (k < SEG_BINS - 1 && e > 0.f) atomicAdd(&bins[k], (unsigned long long)(e * SEG_FIXED));
+        if (k < SEG_BINS - 1 && e > 0.f) atomicAdd(&bins[k], __float2ull_rn(e * SEG_FIXED));
         else tail += e;
       }
     }
@@ -650,7 +653,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
     const bool all_listed = n <= SEG_LIST;
     if (n > SEG_SORT) {
       // 5. too many to put in order: the bin's 256 parts by their masses, and the entries of the part in which the point lies
-      auto add = [&](float v) { atomicAdd(&sh.sub[part_of_bin(v * inv_w)], (unsigned long long)(e_of(v) * SEG_FIXED)); };
+      auto add = [&](float v) { atomicAdd(&sh.sub[part_of_bin(v * inv_w)], __float2ull_rn(e_of(v) * ROW_FIXED)); };
       if (all_listed) {
         for (int j = tid; j < n; j += SAMPLE_THREADS) add(sh.list_x[j]);
         __syncthreads();
@@ -659,7 +662,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
           for (; marked; marked &= marked - 1) add(x[entry_at(begin, __ffs(marked) - 1)]);
         });
       }
-      const float part = tid < SEG_BINS ? (float)sh.sub[tid] * (1.0f / SEG_FIXED) : 0.f;
+      const float part = tid < SEG_BINS ? (float)sh.sub[tid] * (1.0f / ROW_FIXED) : 0.f;
       const float run = block_scan(part, sh.scratch);
       float before;
       sub = first_past(sh, part, run, target - above, before);
@@ -684,7 +687,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
         for (int q = 0; q < SEG_LIST / SAMPLE_THREADS; ++q) {
           if (at[q] < 0) continue;
           const int p = part_of_bin(v[q] * inv_w);
-          if (p < sub) atomicAdd(&sh.kept[at[q] / seg_len], (unsigned long long)(e_of(v[q]) * SEG_FIXED));
+          if (p < sub) atomicAdd(&sh.kept[at[q] / seg_len], __float2ull_rn(e_of(v[q]) * ROW_FIXED));
           if (p == sub) {
             const int place = atomicAdd(&sh.count, 1);
             sh.list_x[place] = v[q], sh.list_i[place] = at[q];
@@ -703,7 +706,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
             if (p == sub) in_part |= 1u << j;
           }
           whole = wave_sum(whole);
-          if (lane == 0) sh.kept[s] = (unsigned long long)(whole * SEG_FIXED);
+          if (lane == 0) sh.kept[s] = __float2ull_rn(whole * ROW_FIXED);
           list(begin, in_part);
         });
       }
@@ -735,7 +738,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
     if (tid < n && above + (through - key) <= target) atomicMin(&sh.smallest, __float_as_int(key));
     __syncthreads();
     least = __int_as_float(sh.smallest);
-    if (tid < n && own >= least) atomicAdd(&sh.kept[owner], (unsigned long long)(own * SEG_FIXED));
+    if (tid < n && own >= least) atomicAdd(&sh.kept[owner], __float2ull_rn(own * ROW_FIXED));
     __syncthreads();
     // the kept mass of every segment: its bins before `bin`, a wavefront a segment, and what the list gave
     seg_mass = 0.f;
@@ -748,7 +751,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
         if (k < SEG_BINS - 1 && k + sh.below[s] < bin) h += hist[k];
       }
       h = wave_sum(h);
-      if (lane == 0) sh.mass[s] = h * sh.scale[s] + (float)sh.kept[s] * (1.0f / SEG_FIXED);
+      if (lane == 0) sh.mass[s] = h * sh.scale[s] + (float)sh.kept[s] * (1.0f / ROW_FIXED);
     }
     __syncthreads();
     seg_mass = tid < n_segs ? sh.mass[tid] : 0.f;
