@@ -254,8 +254,15 @@ def capacity_until(
         # a window's range moves over the fixed positions of the cuts: at some steps it straddles one cut more than at
         # others, whatever its length (a window shorter than a chunk is cut in two now and then).  While no sequence
         # is longer than the window every range starts at key 0, as without a window.  A block of positions moves likewise.
+        # Where a range of the window's length may be cut into more than MERGE_MID_MAX parts, one cut more or less moves a tile
+        # from one list of merges to the other (a window of 8,192 keys in chunks of 256: 32 parts from an aligned start, else 33).
         tiles = int((plan.work[:, 4] < 0).sum()) + plan.merge.shape[0]
-        capacity = PlanCapacity(work=capacity.work + tiles, merge_many=capacity.merge_many, merge_mid=max(capacity.merge_mid, tiles))
+        most_parts = (span - 2) // int(chunk_keys(span, few_heads)) + 2
+        capacity = PlanCapacity(
+            work=capacity.work + tiles,
+            merge_many=max(capacity.merge_many, tiles if most_parts > MERGE_MID_MAX else 0),
+            merge_mid=max(capacity.merge_mid, tiles),
+        )
     return plan, capacity
 
 

@@ -29,3 +29,19 @@ def test_captured_lists_hold_every_later_step(window):
         assert flat is not None and flat.size == capacity.ints
         work = flat[: capacity.work * 6].reshape(-1, 6)
         assert np.all((work[:, 1] == NULL_ROW) | (work[:, 3] > work[:, 2]))
+
+
+@pytest.mark.parametrize("few_heads,window,chunk", [(True, 8192, None), (True, 16384, None), (True, 16500, None), (False, 32768, None), (True, None, 8320), (True, 7936, None), (True, 8191, None)])
+@pytest.mark.parametrize("past", [0, 1, 255, 256, 512, 700])
+def test_captured_lists_hold_a_window_at_every_place(few_heads, window, chunk, past):
+    """A window's chunks are counted differently from step to step, also across the border between the two lists of merges."""
+    span = window if chunk is None else chunk
+    q, kv, most = [1, 1], [span + past, span + past + 256], 2 * span + 4096
+    _, capacity = capacity_until(q, kv, 16, window, 0, most, chunk, few_heads)
+    for t in [*range(0, 1100, 3), most - max(kv)]:
+        assert pad_plan(build_plan(q, [n + t for n in kv], 16, window, 0, chunk, few_heads), capacity) is not None, t
+
+
+def test_short_windows_leave_no_room_for_many_partials():
+    _, capacity = capacity_until([1], [9000], 16, 4096, 0, 16384, few_heads=True)
+    assert capacity.merge_many == 0 and capacity.merge_mid == 1
