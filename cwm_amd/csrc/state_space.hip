@@ -180,7 +180,8 @@ extern "C" int cwm_conv_silu(const void* in, long in_ld, int dtype, const float*
 // tokens from a zero state and leaves that state and the product of its decays in entry 1 + j; the last segment's
 // block copies the sequence's state into entry 0.  PHASE 2: segment j starts from entry 0 carried through the
 // entries 1 .. j (S <- decay_i S + state_i), walks its tokens and writes y; the last one leaves the sequence's state.
-// No block reads a state that another block of the same launch writes.
+// No block reads a state that another block of the same launch writes.  PHASE 3: the portions of one segment alone, walked as in
+// PHASE 0.
 template <typename T, int THREADS, int TC, bool VEC, int PHASE>
 __global__ void __launch_bounds__(THREADS) selective_scan_kernel(const T* __restrict__ xbc, long xbc_ld, const T* __restrict__ dt_raw,
                                                                  long dt_ld, const float* __restrict__ dt_bias,
@@ -198,6 +199,7 @@ __global__ void __launch_bounds__(THREADS) selective_scan_kernel(const T* __rest
     const int* entry = segments + 6 * blockIdx.z;
     b = entry[0], t0 = entry[1], t1 = entry[2], seg = entry[3], seg_base = entry[4], n_segs = entry[5];
   }
+  if (PHASE == 3 && n_segs > 1) return;
   const int cols = THREADS / split;
   const int s = threadIdx.x % split;
   const int col = threadIdx.x / split;
@@ -232,7 +234,7 @@ __global__ void __launch_bounds__(THREADS) selective_scan_kernel(const T* __rest
     }
   };
   auto entry_state = [&](int k) { return seg_state + ((size_t)(seg_base + k) * heads + h) * head_elems; };
-  if (PHASE == 0) {
+  if (PHASE == 0 || PHASE == 3) {
     load_state(st);
   } else if (PHASE == 1) {
     if (seg == n_segs - 1) {  // the whole block: the sequence's state as it is, for the segments of the next launch
@@ -414,7 +416,7 @@ __global__ void __launch_bounds__(THREADS) selective_scan_kernel(const T* __rest
       __syncthreads();
     }
   }
-  if (PHASE == 0) {
+  if (PHASE == 0 || PHASE == 3) {
     store_state(st);
   } else if (PHASE == 1) {
     store_state(entry_state(1 + seg));
@@ -492,6 +494,8 @@ __global__ void __launch_bounds__(256) selective_scan_single_kernel(const T* __r
 // C needs; a score's lane (query r, keys 4 j + i) is likewise the operand that x needs.
 // MODE 1 leaves the state that every segment but a sequence's last makes from zero, and the segment's decay; then
 // `scan_carry_kernel` turns those into the states at the segments' starts; MODE 2 walks every segment from there and writes y.
+// Portions of one segment, decoded tokens among them, are left to the walk: their bits and their cost are what they are without a
+// long portion beside them (in blocks a decoded token pays for 64).
 // Bound by the float32 matrix instructions (110k of a compute unit's cycles at 2,048 tokens of 64 heads, 64 columns, 128 rows)
 // and by the waits between a block's stages, two blocks a compute unit; the walk was bound by its reads of B and C from LDS.
 #define BLOCK_TOKENS 64
@@ -514,6 +518,7 @@ __global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restric
   __shared__ __attribute__((aligned(16))) float step_size[BLOCK_TOKENS], from_start[BLOCK_TOKENS], to_end[BLOCK_TOKENS];
   const int* entry = segments + 6 * blockIdx.z;
   const int t0 = entry[1], t1 = entry[2], seg = entry[3], seg_base = entry[4], n_segs = entry[5];
+  if (n_segs == 1) return;                     // a short portion is walked
   if (MODE == 1 && seg == n_segs - 1) return;  // nothing follows it
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, j = lane >> 4;
   const int h = blockIdx.y, g = h / (heads / groups), inner = heads * P;
@@ -694,7 +699,7 @@ __global__ void __launch_bounds__(256) scan_carry_kernel(const int* __restrict__
                                                          const int* __restrict__ slots, int n_slots, int heads, long head_elems,
                                                          float* __restrict__ seg_state, const float* __restrict__ seg_decay) {
   const int* entry = segments + 6 * blockIdx.y;
-  if (entry[3] != 0) return;  // the sequence's first segment stands for all of them
+  if (entry[3] != 0 || entry[5] == 1) return;  // the sequence's first segment stands for all of them; a short portion is walked
   const long i = (long)blockIdx.x * 256 + threadIdx.x, elems = heads * head_elems;
   if (i >= elems) return;
   const int h = (int)(i / head_elems), slot = slots[entry[0]], first = entry[4], count = entry[5];
@@ -703,8 +708,8 @@ __global__ void __launch_bounds__(256) scan_carry_kernel(const int* __restrict__
     float add[8], keep[8];
 #pragma unroll
     for (int a = 0; a < 8; ++a) {  // the last segment has neither: what lies past the others is not used
-      const size_t at = first + min(s + a, max(count - 2, 0));
-      add[a] = count > 1 ? seg_state[at * elems + i] : 0.f, keep[a] = count > 1 ? seg_decay[at * heads + h] : 0.f;
+      const size_t at = first + min(s + a, count - 2);
+      add[a] = seg_state[at * elems + i], keep[a] = seg_decay[at * heads + h];
     }
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
@@ -714,7 +719,8 @@ __global__ void __launch_bounds__(256) scan_carry_kernel(const int* __restrict__
   }
 }
 
-template <typename T, bool VEC>
+// ONLY: the one phase to launch, or -1: the walk, or with a list of segments both phases.
+template <typename T, bool VEC, int ONLY = -1>
 static void launch_scan(dim3 grid, int split, hipStream_t stream, const void* xbc, long xbc_ld, const void* dt_raw, long dt_ld,
                         const float* dt_bias, const float* a_log, const float* d_skip, float* state, long state_ld, const int* slots,
                         const int* cu_q, float* y, int heads, int P, int N, int groups, int n_slots, const int* segments, float* seg_state,
@@ -726,7 +732,9 @@ static void launch_scan(dim3 grid, int split, hipStream_t stream, const void* xb
   hipLaunchKernelGGL((selective_scan_kernel<T, THREADS, TC, VEC, PHASE>), grid, dim3(THREADS), lds_bytes, stream, (const T*)xbc, xbc_ld,     \
                      (const T*)dt_raw, dt_ld, dt_bias, a_log, d_skip, state, state_ld, slots, cu_q, y, heads, P, N, groups, split, n_slots, \
                      segments, seg_state, seg_decay)
-  if (!segments) {
+  if constexpr (ONLY >= 0) {
+    CWM_SCAN_PHASE(ONLY);
+  } else if (!segments) {
     CWM_SCAN_PHASE(0);
   } else {
     CWM_SCAN_PHASE(1);
@@ -738,7 +746,7 @@ static void launch_scan(dim3 grid, int split, hipStream_t stream, const void* xb
 extern "C" int cwm_selective_scan(const void* xbc, long xbc_ld, const void* dt_raw, long dt_ld, int dtype, const float* dt_bias,
                                   const float* a_log, const float* d_skip, float* state, long state_ld, const int* slots,
                                   const int* cu_q, float* y, int n_tokens, int n_seqs, int heads, int P, int N, int groups, int n_slots,
-                                  const int* segments, int n_segments, float* seg_state, float* seg_decay, hipStream_t stream) {
+                                  const int* segments, int n_segments, int n_short, float* seg_state, float* seg_decay, hipStream_t stream) {
   CWM_REQUIRE(xbc && dt_raw && dt_bias && a_log && d_skip && state && slots && cu_q && y, "selective_scan: arguments missing");
   CWM_REQUIRE(heads > 0 && P > 0 && N > 0 && groups > 0 && heads % groups == 0, "selective_scan: bad sizes");
   CWM_REQUIRE(N <= SCAN_ROWS * 16, "selective_scan: a state of %d rows, the kernel takes up to %d", N, SCAN_ROWS * 16);
@@ -751,7 +759,8 @@ extern "C" int cwm_selective_scan(const void* xbc, long xbc_ld, const void* dt_r
   const int cols = 256 / split;
   const int row = 2 * SCAN_ROWS * split + cols;
   CWM_REQUIRE(16 * row <= SCAN_PF * 256, "selective_scan: a chunk of tokens does not fit the threads' registers");
-  // with a list of segments (6 numbers each; its scratch lists have an entry for every segment) the blocks' z counts those
+  // with a list of segments (6 numbers each; its scratch lists have an entry for every segment) the blocks' z counts those;
+  // n_short of the portions are one segment each
   CWM_REQUIRE(!segments || (n_segments > 0 && n_segments <= 65535 && seg_state && seg_decay && ((uintptr_t)seg_state % 16) == 0),
               "selective_scan: a list of segments needs its scratch lists and at most 65535 entries");
   dim3 grid((P + cols - 1) / cols, heads, segments ? n_segments : n_seqs);
@@ -783,6 +792,9 @@ extern "C" int cwm_selective_scan(const void* xbc, long xbc_ld, const void* dt_r
                        slots, n_slots, heads, head_elems, seg_state, seg_decay);
     if (N <= 64) CWM_SCAN_BLOCK(4, 2); else CWM_SCAN_BLOCK(8, 2);
 #undef CWM_SCAN_BLOCK
+    if (n_short > 0)
+      launch_scan<bf16_t, true, 3>(grid, split, stream, xbc, xbc_ld, dt_raw, dt_ld, dt_bias, a_log, d_skip, state, state_ld, slots, cu_q, y, heads, P, N,
+                                   groups, n_slots, segments, seg_state, seg_decay);
     return cwm_launch_status("selective_scan");
   }
 #define CWM_SCAN(T, VEC) \

@@ -277,8 +277,8 @@ def selective_scan(
     first, `scan_state_elems` values in the kernel's own order, see `scan_state_pack`).  `xbc` [T, heads * head_dim + 2 * groups * n_state] = [x | B | C]; `dt` [T, heads] before
     bias and softplus (rows may lie apart); `dt_bias`, `a_log`, `d_skip` float32 [heads].  Returns y float32
     [T, heads * head_dim].  Portions of up to `SCAN_SEGMENT` tokens are walked token by token, which gives the same
-    bits however a sequence is cut; a step with a longer portion (`batch.q_lens`) cuts its portions into segments that
-    run side by side and carries the state across them, which differs from the walk by rounding (bfloat16 rows, states of up
+    bits however a sequence is cut and whatever else the step holds; a longer portion (`batch.q_lens`) is cut into segments that
+    run side by side, and the state is carried across them, which differs from the walk by rounding (bfloat16 rows, states of up
     to 128 rows and heads of whole tiles of 16 columns: 64 tokens at a time on the matrix cores, in float32)."""
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
     _need_gpu(xbc, dt, dt_bias, a_log, d_skip, state)
@@ -317,7 +317,8 @@ def selective_scan(
             ctypes.c_int(_code(xbc.dtype)), _ptr(dt_bias), _ptr(a_log), _ptr(d_skip), _ptr(state), ctypes.c_long(state.shape[1]),
             _ptr(batch.state_slots), _ptr(batch.cu_q), _ptr(y), ctypes.c_int(n_tokens), ctypes.c_int(batch.n_seqs), ctypes.c_int(heads),
             ctypes.c_int(head_dim), ctypes.c_int(n_state), ctypes.c_int(groups), ctypes.c_int(state.shape[0]),
-            _ptr(segments), ctypes.c_int(segments.shape[0] if segments is not None else 0), _ptr(seg_state), _ptr(seg_decay), _stream(),
+            _ptr(segments), ctypes.c_int(segments.shape[0] if segments is not None else 0),
+            ctypes.c_int(sum(q <= SCAN_SEGMENT for q in batch.q_lens) if segments is not None else 0), _ptr(seg_state), _ptr(seg_decay), _stream(),
         ),
     )
     return y

@@ -69,3 +69,25 @@ def test_long_portions_against_float64(heads, width, rows, groups, q_lens):
             mine = ops.scan_state_unpack(packed[slot].cpu(), heads, width, rows).double()
             size = exact_state[slot].abs().amax((1, 2)).clamp(min=1.0)
             assert bool(((mine.reshape(heads, rows, width) - exact_state[slot]).abs().amax((1, 2)) <= 4e-6 * size).all())
+
+
+@pytest.mark.parametrize("heads,width,rows,groups", [(4, 64, 128, 2), (3, 48, 72, 3)])
+@pytest.mark.parametrize("q_lens", [[320, 1, 64], [1, 256, 257], [1, 1, 600]])
+def test_short_portions_beside_a_long_one_keep_their_bits(heads, width, rows, groups, q_lens):
+    from cwm_amd import ops
+
+    g = torch.Generator().manual_seed(sum(q_lens))
+    normal = lambda *shape: torch.randn(shape, generator=g)  # noqa: E731
+    n = sum(q_lens)
+    xbc, dt = normal(n, heads * width + 2 * groups * rows).bfloat16().to(DEV), (normal(n, heads) - 1).bfloat16().to(DEV)
+    bias, d_skip, a_log = (normal(heads).to(DEV) for _ in range(3))
+    state = torch.stack([ops.scan_state_pack(normal(heads, rows, width) * 0.3) for _ in range(3)]).to(DEV)
+    slots, beside = [1, 2, 0], state.clone()
+    together = ops.selective_scan(xbc, dt, bias, a_log, d_skip, beside, _batch(q_lens, slots), heads, width, rows, groups)
+    at = 0
+    for q, slot in zip(q_lens, slots):
+        if q <= 256:
+            alone = state.clone()
+            y = ops.selective_scan(xbc[at : at + q], dt[at : at + q], bias, a_log, d_skip, alone, _batch([q], [slot]), heads, width, rows, groups)
+            assert torch.equal(y, together[at : at + q]) and torch.equal(alone[slot], beside[slot])
+        at += q
