@@ -579,8 +579,13 @@ __global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restric
       for (int e = 0; e < 8; ++e) b_cols[n + e][lane] = (bf16_t)(rb[k][e >> 1] >> (16 * (e & 1)));
     }
     float x[16];
+    uint32_t largest = 0;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) x[k] = __uint_as_float(k & 1 ? rx[k >> 1] & 0xffff0000u : rx[k >> 1] << 16);
+    for (int k = 0; k < 16; ++k) {
+      x[k] = __uint_as_float(k & 1 ? rx[k >> 1] & 0xffff0000u : rx[k >> 1] << 16);
+      largest = max(largest, __float_as_uint(x[k]) & 0x7fffffffu);
+    }
+    const bool all_finite = __ballot(largest >= 0x7f800000u) == 0;  // of the wavefront's columns
     if (wave == 0) {
       const bool inside = c0 + lane < t1;
       const float zt = r_dt + bias, dt = inside ? (zt > 20.f ? zt : log1pf(expf(zt))) : 0.f;
@@ -645,10 +650,25 @@ __global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restric
         for (int b = 0; b < 4; ++b)
 #pragma unroll
           for (int a = b; a < 4; ++a) {
+            if (a == b && !all_finite) continue;
             const float4v m = *(const float4v*)&scores[16 * a + r][16 * b + 4 * j];
 #pragma unroll
             for (int i = 0; i < 4; ++i) out[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[i], x[4 * b + i], out[a], 0, 0, 0);
           }
+        if (!all_finite) {
+          // a later key's score of 0 does not leave an infinity or a NaN out: the tiles on the diagonal key by key
+#pragma unroll
+          for (int k = 0; k < 16; ++k) {
+            const int b = k >> 2;
+            for (int from = 0; from < 4; ++from) {
+              const int key = 4 * from + (k & 3);
+              const float value = __shfl(x[k], 16 * from + r, CWM_WAVE);
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                if (4 * j + i >= key) out[b][i] = fmaf(scores[16 * b + 4 * j + i][16 * b + key], value, out[b][i]);
+            }
+          }
+        }
 #pragma unroll
         for (int a = 0; a < 4; ++a)
 #pragma unroll

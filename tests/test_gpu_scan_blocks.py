@@ -91,3 +91,30 @@ def test_short_portions_beside_a_long_one_keep_their_bits(heads, width, rows, gr
             y = ops.selective_scan(xbc[at : at + q], dt[at : at + q], bias, a_log, d_skip, alone, _batch([q], [slot]), heads, width, rows, groups)
             assert torch.equal(y, together[at : at + q]) and torch.equal(alone[slot], beside[slot])
         at += q
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("at", [1, 14, 64 + 37, 256 + 63, 300])
+def test_a_value_that_is_not_finite_reaches_no_earlier_token(bad, at):
+    from cwm_amd import ops
+
+    heads, width, rows, groups, n = 2, 48, 40, 1, 350
+    g = torch.Generator().manual_seed(at)
+    normal = lambda *shape: torch.randn(shape, generator=g)  # noqa: E731
+    xbc, dt = normal(n, heads * width + 2 * groups * rows).bfloat16().to(DEV), (normal(n, heads) - 1).bfloat16().to(DEV)
+    bias, d_skip, a_log = (normal(heads).to(DEV) for _ in range(3))
+    spoilt = xbc.clone()
+    spoilt[at, 5] = bad  # x of the first head
+    start = torch.stack([ops.scan_state_pack(normal(heads, rows, width) * 0.3)]).to(DEV)
+    fine, poisoned = start.clone(), start.clone()
+    want = ops.selective_scan(xbc, dt, bias, a_log, d_skip, fine, _batch([n], [0]), heads, width, rows, groups)
+    got = ops.selective_scan(spoilt, dt, bias, a_log, d_skip, poisoned, _batch([n], [0]), heads, width, rows, groups)
+    others = torch.arange(heads * width, device=DEV) != 5
+    assert torch.equal(got[:, others], want[:, others]) or bool(((got - want)[:, others].abs() <= 4e-6 * want.abs().amax()).all())
+    # the tokens before it, whose sums may come in another order
+    assert bool(((got - want)[:at].abs() <= 4e-6 * want.abs().amax()).all())
+    assert not bool(torch.isfinite(got[at, 5]))
+    # and as the walk leaves it: the same tokens in portions of one segment
+    walked = start.clone()
+    y = torch.cat([ops.selective_scan(spoilt[a:b], dt[a:b], bias, a_log, d_skip, walked, _batch([b - a], [0]), heads, width, rows, groups) for a, b in ((0, 200), (200, n))])
+    assert torch.equal(torch.isfinite(y), torch.isfinite(got))
