@@ -589,7 +589,9 @@ __global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restric
     if (wave == 0) {
       const bool inside = c0 + lane < t1;
       const float zt = r_dt + bias, dt = inside ? (zt > 20.f ? zt : log1pf(expf(zt))) : 0.f;
-      double through = (double)(rate * dt);
+      // e^-128 is 0 in float32, as the decays of more are; bounded, they leave differences of sums finite and exact
+      const float log_decay = inside ? rate * dt : 0.f;
+      double through = (double)(log_decay < -128.f ? -128.f : log_decay);
 #pragma unroll
       for (int off = 1; off < CWM_WAVE; off <<= 1) {
         const double o = __shfl_up(through, off, CWM_WAVE);

@@ -118,3 +118,23 @@ def test_a_value_that_is_not_finite_reaches_no_earlier_token(bad, at):
     walked = start.clone()
     y = torch.cat([ops.selective_scan(spoilt[a:b], dt[a:b], bias, a_log, d_skip, walked, _batch([b - a], [0]), heads, width, rows, groups) for a, b in ((0, 200), (200, n))])
     assert torch.equal(torch.isfinite(y), torch.isfinite(got))
+
+
+def test_decays_of_nothing_left():
+    """Rates whose logarithms are huge or infinite: the walk's decay is 0, and so is the blocks'."""
+    from cwm_amd import ops
+
+    heads, width, rows, groups, n = 4, 16, 24, 1, 400
+    g = torch.Generator().manual_seed(7)
+    normal = lambda *shape: torch.randn(shape, generator=g)  # noqa: E731
+    xbc, dt = normal(n, heads * width + 2 * groups * rows).bfloat16().to(DEV), normal(n, heads).bfloat16()
+    dt[100] = -60.0  # a step of e^-60: nothing added, and at the lesser rates nothing forgotten
+    a_log = torch.tensor([100.0, 88.0, 30.0, 5.0], device=DEV)
+    bias, d_skip, dt = normal(heads).to(DEV), normal(heads).to(DEV), dt.to(DEV)
+    start = torch.stack([ops.scan_state_pack(normal(heads, rows, width))]).to(DEV)
+    whole, walked = start.clone(), start.clone()
+    got = ops.selective_scan(xbc, dt, bias, a_log, d_skip, whole, _batch([n], [0]), heads, width, rows, groups)
+    want = torch.cat([ops.selective_scan(xbc[a:b], dt[a:b], bias, a_log, d_skip, walked, _batch([b - a], [0]), heads, width, rows, groups) for a, b in ((0, 256), (256, n))])
+    assert bool(torch.isfinite(want).all())
+    assert bool(((got - want).abs() <= 4e-6 * want.abs().amax()).all())
+    assert bool(((whole - walked).abs() <= 4e-6 * walked.abs().amax().clamp(min=1.0)).all())
