@@ -37,6 +37,22 @@ struct SideAddends {
   int n;
 };
 
+// Which tokens a launch serves, where a step holds portions of both kinds: those of portions of at least SIDE_TILE_FROM tokens
+// go to the matrix cores, the others to the kernel without them, so that a token's bits do not depend on the rest of the step.
+#define SIDE_TILE_FROM 256
+struct SidePortions {
+  const int* seq_of_token;  // null: every token of the step is served
+  const int* cu_q;
+  __device__ __forceinline__ bool serves(int t, int n_tokens, bool tiles) const {
+    if (t >= n_tokens) return false;
+    if (!seq_of_token) return true;
+    const int b = seq_of_token[t];
+    return (cu_q[b + 1] - cu_q[b] >= SIDE_TILE_FROM) == tiles;
+  }
+};
+
+extern "C" int cwm_token_side_tile_from() { return SIDE_TILE_FROM; }
+
 extern "C" int cwm_token_side_max_addends() { return SIDE_MAX_ADDENDS; }
 
 extern "C" int cwm_token_side_max_dim() { return SIDE_MAX_DIM; }
@@ -69,16 +85,23 @@ template <typename TW, int TOK>
 __global__ void __launch_bounds__(SIDE_THREADS)
 token_side_kernel(float* __restrict__ h, const int* __restrict__ tokens, const TW* __restrict__ table, long table_ld,
                   int column0, const TW* __restrict__ w_gate, const TW* __restrict__ w_proj_t, const float* __restrict__ weight,
-                  int n_tokens, int dim, int side_dim, int vocab, float eps, bool round_inputs, SideAddends addends) {
+                  int n_tokens, int dim, int side_dim, int vocab, float eps, bool round_inputs, SideAddends addends, SidePortions portions) {
   extern __shared__ __attribute__((aligned(16))) float rows[];  // [TOK][dim], then the gated values [TOK][side_dim]
   __shared__ float scratch[16];
   float* gated = rows + (size_t)TOK * dim;
   const int t0 = blockIdx.x * TOK;
+  bool mine[TOK], any = false;
+#pragma unroll
+  for (int tok = 0; tok < TOK; ++tok) any |= mine[tok] = portions.serves(t0 + tok, n_tokens, false);
+  if (!any) return;
   for (int e = threadIdx.x; e < TOK * dim; e += SIDE_THREADS) {
     const int tok = e / dim, el = e - tok * dim;
     const size_t t = (size_t)t0 + tok;
     float x = 0.f;
-    if (t < (size_t)n_tokens) {
+    bool serve = false;
+#pragma unroll
+    for (int i = 0; i < TOK; ++i) serve = tok == i ? mine[i] : serve;
+    if (serve) {
       x = h[t * dim + el];
       for (int a = 0; a < addends.n; ++a) {
         const SideAddend& ad = addends.a[a];
@@ -134,7 +157,7 @@ token_side_kernel(float* __restrict__ h, const int* __restrict__ tokens, const T
 #pragma unroll
       for (int tok = 0; tok < TOK; ++tok) {
         const float sum = wave_sum(a[kk][tok]);
-        if (lane == 0 && k < side_dim && t0 + tok < n_tokens) {
+        if (lane == 0 && k < side_dim && mine[tok]) {
           const float z = side_round(sum, round_inputs);
           const float gelu = 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
           const int token = tokens[t0 + tok];
@@ -171,7 +194,7 @@ token_side_kernel(float* __restrict__ h, const int* __restrict__ tokens, const T
 #pragma unroll
   for (int tok = 0; tok < TOK; ++tok) {
     const float rstd = 1.0f / sqrtf(block_sum(sq[tok], scratch) / (float)dim + eps);
-    if (t0 + tok < n_tokens) {
+    if (mine[tok]) {
       float* hrow = h + (size_t)(t0 + tok) * dim;
 #pragma unroll
       for (int i = 0; i < MAXE; ++i) {
@@ -197,7 +220,7 @@ template <int TOK, int MAXT>
 __global__ void __launch_bounds__(SIDE_THREADS)
 token_side_tile_kernel(float* __restrict__ h, const int* __restrict__ tokens, const bf16_t* __restrict__ table, long table_ld, int column0,
                        const bf16_t* __restrict__ w_gate, const bf16_t* __restrict__ w_proj, const float* __restrict__ weight, int n_tokens,
-                       int dim, int side_dim, int vocab, float eps, SideAddends addends) {
+                       int dim, int side_dim, int vocab, float eps, SideAddends addends, SidePortions portions) {
   extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
   constexpr int WAVES = SIDE_THREADS / CWM_WAVE, A_TOKEN = WAVES / TOK;  // wavefronts that load a token's row
   const int x_ld = dim + 8;
@@ -207,12 +230,17 @@ token_side_tile_kernel(float* __restrict__ h, const int* __restrict__ tokens, co
   float* squares = (float*)(gated + TOK * (SIDE_TILE_MAX + 8));  // [WAVES][TOK]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, j = lane >> 4;
   const int t0 = blockIdx.x * TOK;
+  bool any = false;
+#pragma unroll
+  for (int tok = 0; tok < TOK; ++tok) any |= portions.serves(t0 + tok, n_tokens, true);
+  if (!any) return;
   // 1. the rows: pending addends into the residual, bfloat16 into LDS
   {
     const int tok = wave / A_TOKEN, t = t0 + tok;
+    const bool serve = portions.serves(t, n_tokens, true);
     for (int e = 4 * ((wave % A_TOKEN) * CWM_WAVE + lane); e < dim; e += 4 * CWM_WAVE * A_TOKEN) {
       float4v x = {0.f, 0.f, 0.f, 0.f};
-      if (t < n_tokens) {
+      if (serve) {
         x = *(const float4v*)(h + (size_t)t * dim + e);
         for (int a = 0; a < addends.n; ++a) {
           const SideAddend& ad = addends.a[a];
@@ -290,7 +318,7 @@ token_side_tile_kernel(float* __restrict__ h, const int* __restrict__ tokens, co
   sq += __shfl_xor(sq, 32, CWM_WAVE);
   if (j == 0 && r < TOK) squares[wave * TOK + r] = sq;
   __syncthreads();
-  if (r >= TOK || t0 + r >= n_tokens) return;
+  if (r >= TOK || !portions.serves(t0 + r, n_tokens, true)) return;
   float total = 0.f;
 #pragma unroll
   for (int w = 0; w < WAVES; ++w) total += squares[w * TOK + r];
@@ -314,17 +342,19 @@ token_side_tile_kernel(float* __restrict__ h, const int* __restrict__ tokens, co
 // tokens: int32 [T].  table: [vocab, >= column0 + side_dim] of `w_dtype`, rows
 // table_ld apart; w_gate [side_dim, dim] and w_proj_t [side_dim, dim] (the projection transposed) of `w_dtype`, contiguous;
 // w_proj: the projection as [dim, side_dim], or null (then the matrix cores are not used);
-// weight: float32 [dim].
+// weight: float32 [dim].  seq_of_token, cu_q: the step's portions where some have SIDE_TILE_FROM tokens and more and some fewer,
+// null where all tokens are one kind (then n_tokens stands for the portion).
 extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, long table_ld, int column0, const void* w_gate,
                               const void* w_proj_t, const void* w_proj, int w_dtype, const float* weight, int n_tokens, int dim, int side_dim, int vocab,
                               float eps, int round_inputs, int n_addends, const void* const* ptrs, const int* dtypes,
                               const long* lds_, const int* n_partials, const long* partial_strides, const float* scales,
-                              hipStream_t stream) {
+                              const int* seq_of_token, const int* cu_q, hipStream_t stream) {
   CWM_REQUIRE(n_tokens >= 0 && vocab >= 1 && column0 >= 0, "token_side: bad sizes");
   CWM_REQUIRE(dim >= 1 && dim <= SIDE_MAX_WIDTH, "token_side: rows of %d elements are outside 1..%d", dim, SIDE_MAX_WIDTH);
   CWM_REQUIRE(side_dim >= 1 && side_dim <= SIDE_MAX_DIM, "token_side: %d side values are outside 1..%d", side_dim, SIDE_MAX_DIM);
   CWM_REQUIRE(h && tokens && table && w_gate && w_proj_t && weight, "token_side: arguments missing");
   CWM_REQUIRE(eps > 0.f, "token_side: eps must be positive");
+  CWM_REQUIRE(!seq_of_token == !cu_q, "token_side: the portions need both their lists");
   CWM_REQUIRE(n_addends >= 0 && n_addends <= SIDE_MAX_ADDENDS, "token_side: %d addends, at most %d are taken", n_addends, SIDE_MAX_ADDENDS);
   if (n_tokens == 0) return 0;
   SideAddends ad;
@@ -334,12 +364,13 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
     CWM_REQUIRE(n_partials[a] == 1 || dtypes[a] == CWM_F32, "token_side: partial sums must be float32");
     ad.a[a] = SideAddend{ptrs[a], lds_[a], partial_strides[a], n_partials[a], dtypes[a], scales[a]};
   }
-  // from 256 tokens on (32 blocks of eight): with fewer the other kernel's blocks of one or two tokens spread over more of the chip
+  // portions from SIDE_TILE_FROM tokens on (32 blocks of eight): with fewer the other kernel's blocks of one or two tokens spread over more of the chip
   // (8 to 48 tokens of width 2,048: 19 us against 30; 300 tokens 44 against 31)
-  bool tiled = n_tokens >= 256 && w_proj && w_dtype == CWM_BF16 && round_inputs && dim % 64 == 0 && dim <= 4096 && side_dim % 32 == 0 && side_dim <= SIDE_TILE_MAX &&
+  bool tiled = n_tokens >= SIDE_TILE_FROM && w_proj && w_dtype == CWM_BF16 && round_inputs && dim % 64 == 0 && dim <= 4096 && side_dim % 32 == 0 && side_dim <= SIDE_TILE_MAX &&
                (((uintptr_t)h | (uintptr_t)w_gate | (uintptr_t)w_proj | (uintptr_t)weight) % 16) == 0;
   for (int a = 0; a < n_addends; ++a)
     tiled = tiled && lds_[a] % 4 == 0 && partial_strides[a] % 4 == 0 && ((uintptr_t)ptrs[a] % (dtypes[a] == CWM_F32 ? 16 : 8)) == 0;
+  const SidePortions portions = {tiled ? seq_of_token : nullptr, cu_q};
   if (tiled) {
     // sixteen tokens a block where that leaves no compute unit without one, else eight
     const int tok = n_tokens >= 16 * 256 ? 16 : 8;
@@ -349,7 +380,7 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
     if (lds > 65536) (void)hipFuncSetAttribute((const void*)token_side_tile_kernel<TOK, MAXT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
     hipLaunchKernelGGL((token_side_tile_kernel<TOK, MAXT>), dim3((n_tokens + TOK - 1) / TOK), dim3(SIDE_THREADS), lds, stream, h, tokens,   \
                        (const bf16_t*)table, table_ld, column0, (const bf16_t*)w_gate, (const bf16_t*)w_proj, weight, n_tokens, dim,        \
-                       side_dim, vocab, eps, ad);                                                                                          \
+                       side_dim, vocab, eps, ad, portions);                                                                                \
   } while (0)
     if (tok == 16) {
       if (dim <= 2048) CWM_SIDE_TILE(16, 8); else CWM_SIDE_TILE(16, 16);
@@ -357,7 +388,7 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
       if (dim <= 2048) CWM_SIDE_TILE(8, 8); else CWM_SIDE_TILE(8, 16);
     }
 #undef CWM_SIDE_TILE
-    return cwm_launch_status("token_side");
+    if (!seq_of_token) return cwm_launch_status("token_side");
   }
   // tokens a block: as many (4, 2, 1) as fit the LDS and still leave the chip a block a few tokens
   int tok = 4;
@@ -367,7 +398,7 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
   const int blocks = (n_tokens + tok - 1) / tok;
 #define CWM_SIDE_TOK(TW, TOK)                                                                                            \
   hipLaunchKernelGGL((token_side_kernel<TW, TOK>), dim3(blocks), dim3(SIDE_THREADS), lds, stream, h, tokens, (const TW*)table, \
-                     table_ld, column0, (const TW*)w_gate, (const TW*)w_proj_t, weight, n_tokens, dim, side_dim, vocab, eps, round_inputs != 0, ad)
+                     table_ld, column0, (const TW*)w_gate, (const TW*)w_proj_t, weight, n_tokens, dim, side_dim, vocab, eps, round_inputs != 0, ad, portions)
 #define CWM_SIDE(TW)                            \
   do {                                          \
     if (tok == 4) CWM_SIDE_TOK(TW, 4);          \

@@ -19,6 +19,7 @@ MAX_SHORT_CONV_TAPS = 16  # csrc/short_conv.hip: SCONV_MAX_TAPS
 MAX_GLA_DIM = 256  # csrc/linear_attention.hip: GLA_MAX_DIM
 MAX_SIDE_DIM = 256  # csrc/token_side.hip: SIDE_MAX_DIM
 MAX_SIDE_ADDENDS = 4  # csrc/token_side.hip: SIDE_MAX_ADDENDS
+SIDE_TILE_FROM = 256  # csrc/token_side.hip: SIDE_TILE_FROM
 
 
 def _base():
@@ -381,14 +382,15 @@ def short_conv(
 
 def token_side(
     h: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor, column0: int, w_gate: torch.Tensor, w_proj_t: torch.Tensor,
-    weight: torch.Tensor, eps: float, round_inputs: bool, pending: Any = None, w_proj: Optional[torch.Tensor] = None,
+    weight: torch.Tensor, eps: float, round_inputs: bool, pending: Any = None, w_proj: Optional[torch.Tensor] = None, batch: Any = None,
 ) -> None:
     """h (float32 [T, D]) += rms(y) * weight with y = w_proj (gelu_tanh(w_gate h) * e), e the columns column0 ..
     column0 + side_dim of the token's row of `table` ([vocab, n]); w_gate [side_dim, D], `w_proj_t` [side_dim, D] (the
     projection [D, side_dim] transposed, which the kernel reads along D) and the table have one type; `weight` float32 [D].  `round_inputs`: h and the gated values are rounded to bfloat16 where
     they enter the two products.  float32 sums, activation and norm.  `w_proj`: the projection as it is, contiguous [D, side_dim];
-    with it bfloat16 weights and rounded inputs run on the matrix cores from 256
-    tokens on where the sizes allow."""
+    with it bfloat16 weights and rounded inputs run on the matrix cores where the sizes allow, in portions of at least SIDE_TILE_FROM
+    tokens.  `batch`: the step (`q_lens`, `seq_of_token`, `cu_q`), so that a token's bits depend on its own portion alone; without
+    it the tokens are one portion."""
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
     _need_gpu(h, tokens, table, w_gate, w_proj_t, weight, w_proj)
     if h.dtype != torch.float32 or h.dim() != 2 or not h.is_contiguous():
@@ -431,6 +433,16 @@ def token_side(
                 raise KernelError(f"an addend {tuple(t.shape)} does not match the residual stream {tuple(h.shape)}")
             partials[i], strides[i], lds[i] = 1, 0, (t.stride(0) if n_tokens > 1 else dim)
         ptrs[i], dtypes[i], scales[i] = t.data_ptr(), _code(t.dtype), c
+    seq_of_token = cu_q = None
+    if w_proj is not None and batch is not None:
+        if max(batch.q_lens, default=0) < SIDE_TILE_FROM:
+            w_proj = None
+        elif any(0 < q < SIDE_TILE_FROM for q in batch.q_lens):  # both kinds
+            seq_of_token, cu_q = batch.seq_of_token, batch.cu_q
+            _i32(seq_of_token, "seq_of_token")
+            _i32(cu_q, "cu_q")
+            if seq_of_token.numel() != n_tokens:
+                raise KernelError("the step's tokens do not match the residual stream")
     lib = _build.load("token_side")
     _check(
         lib,
@@ -438,7 +450,7 @@ def token_side(
             _ptr(h), _ptr(tokens), _ptr(table), ctypes.c_long(table.stride(0)), ctypes.c_int(column0), _ptr(w_gate), _ptr(w_proj_t),
             _ptr(w_proj), ctypes.c_int(_code(table.dtype)), _ptr(weight), ctypes.c_int(n_tokens), ctypes.c_int(dim), ctypes.c_int(side_dim),
             ctypes.c_int(table.shape[0]), ctypes.c_float(eps), ctypes.c_int(int(round_inputs)), ctypes.c_int(len(terms)), ptrs, dtypes, lds,
-            partials, strides, scales, _stream(),
+            partials, strides, scales, _ptr(seq_of_token), _ptr(cu_q), _stream(),
         ),
     )
 

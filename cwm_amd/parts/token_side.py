@@ -53,10 +53,9 @@ class GatedTokenSide(TokenInput):
         self.weight = tensors[self.norm_name].float().contiguous()
 
     def forward(self, h: torch.Tensor, batch: Any, pending: Any = None) -> None:
-        on_device = {"w_proj": self.w_proj} if h.is_cuda else {}  # what the matrix cores read
         ops.token_side(
             h, batch.tokens, self.table, self.index * self.side_dim, self.w_gate, self.w_proj_t, self.weight, self.eps,
-            round_inputs=self.runtime.act_dtype == torch.bfloat16, pending=pending, **on_device,
+            round_inputs=self.runtime.act_dtype == torch.bfloat16, pending=pending, w_proj=self.w_proj, batch=batch,
         )
 
 

@@ -479,7 +479,7 @@ def _as(t, dtype):
     return t.to(dtype).float()
 
 
-def token_side(h, tokens, table, column0, w_gate, w_proj_t, weight, eps, round_inputs, pending=None):
+def token_side(h, tokens, table, column0, w_gate, w_proj_t, weight, eps, round_inputs, pending=None, w_proj=None, batch=None):
     if pending is not None:
         h += _total(pending)
     side_dim = w_gate.shape[0]

@@ -3,6 +3,8 @@ and not, widths of few and many tiles, pending addends of either type."""
 
 from __future__ import annotations
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
@@ -40,3 +42,32 @@ def test_against_float64(n_tokens, dim, side):
         off = (result.double() - want).abs()
         assert bool((off <= bound).all())
         assert float(off.square().mean().sqrt()) <= 2e-3
+
+
+@pytest.mark.parametrize("q_lens", [[3, 300, 1], [1] * 260 + [256], [257, 255], [1] * 300, [400, 260], [17, 4100, 0, 2]])
+def test_a_portions_bits_do_not_depend_on_the_step(q_lens):
+    from cwm_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(sum(q_lens))
+    normal = lambda *shape: torch.randn(shape, generator=g, device=DEV)  # noqa: E731
+    dim, side, vocab, n = 192, 64, 61, sum(q_lens)
+    h, tokens = normal(n, dim), torch.randint(vocab, (n,), generator=g, device=DEV, dtype=torch.int32)
+    gate, proj, table = normal(side, dim).mul(dim ** -0.5).bfloat16(), normal(dim, side).bfloat16(), normal(vocab, side).bfloat16()
+    args = (table, 0, gate, proj.t().contiguous(), normal(dim).abs() + 0.3, 1e-6, True)
+    parts = normal(2, n, dim)
+
+    def step(lens, first, last):
+        lengths = torch.tensor(lens)
+        batch = SimpleNamespace(
+            q_lens=list(lens), cu_q=torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)]).int().to(DEV),
+            seq_of_token=torch.repeat_interleave(torch.arange(len(lens)), lengths).int().to(DEV),
+        )
+        out = h[first:last].clone()
+        ops.token_side(out, tokens[first:last], *args, pending=parts[:, first:last].contiguous(), w_proj=proj, batch=batch)
+        return out
+
+    together, first = step(q_lens, 0, n), 0
+    for b, q in enumerate(q_lens):
+        if q and (b < 6 or b >= len(q_lens) - 2):
+            assert torch.equal(together[first : first + q], step([q], first, first + q)), b
+        first += q
