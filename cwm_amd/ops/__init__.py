@@ -1327,7 +1327,7 @@ from .streams import (  # noqa: E402
 )
 from .mixing import (  # noqa: E402
     MAX_GLA_DIM, MAX_SHORT_CONV_TAPS, MAX_SIDE_ADDENDS, MAX_SIDE_DIM, MAX_TALK_HEADS, gated_act_rows, gated_linear_attention, gla_state_elems,
-    gla_state_unpack, short_conv, talking_attention, token_side, wkv, wkv_token,
+    gla_state_unpack, short_conv, side_tiles_take, talking_attention, token_side, wkv, wkv_token,
 )
 from .recurrence import (  # noqa: E402
     MAX_NORMED_ADDENDS, MAX_TOKEN_MIXES, NormedSum, add_normed_rmsnorm, embedding_sinusoid, min_gru, token_mixes,

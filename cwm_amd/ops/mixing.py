@@ -380,6 +380,11 @@ def short_conv(
     return outs
 
 
+def side_tiles_take(dim: int, side_dim: int, dtype: torch.dtype, round_inputs: bool) -> bool:
+    """Whether `token_side` has a form on the matrix cores for these sizes and types (and so a use for `w_proj`)."""
+    return dtype == torch.bfloat16 and round_inputs and dim % 64 == 0 and dim <= 4096 and side_dim % 32 == 0 and side_dim <= 128
+
+
 def token_side(
     h: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor, column0: int, w_gate: torch.Tensor, w_proj_t: torch.Tensor,
     weight: torch.Tensor, eps: float, round_inputs: bool, pending: Any = None, w_proj: Optional[torch.Tensor] = None, batch: Any = None,

@@ -48,8 +48,10 @@ class GatedTokenSide(TokenInput):
         super().bind(tensors, runtime)
         self.table = tensors[self.table_name]
         self.w_gate = tensors[self.gate_name].contiguous()
-        self.w_proj = tensors[self.proj_name].contiguous()
-        self.w_proj_t = self.w_proj.t().contiguous()  # a row a side value: what the kernel without matrix cores reads along the width
+        proj = tensors[self.proj_name]
+        self.w_proj_t = proj.t().contiguous()  # a row a side value: what the kernel without matrix cores reads along the width
+        tiles = ops.side_tiles_take(self.dim, self.side_dim, proj.dtype, runtime.act_dtype == torch.bfloat16)
+        self.w_proj = proj.contiguous() if tiles else None  # what the matrix cores read
         self.weight = tensors[self.norm_name].float().contiguous()
 
     def forward(self, h: torch.Tensor, batch: Any, pending: Any = None) -> None:

@@ -271,3 +271,14 @@ def test_regimes_against_plain(tmp_path, monkeypatch, name, regime):
         np.testing.assert_allclose(got[rid], want[rid].exact, rtol=2e-3, atol=2e-4 * float(np.abs(want[rid].exact).max()), err_msg=f"{name} {regime} {rid}")
     assert rep.manager.live_requests() == []
     assert all(f == g.pool.num_pages for f, g in zip(rep.manager.free_pages(), rep.manager.groups))
+
+
+@pytest.mark.parametrize("dim,side,dtype,kept", [(128, 64, torch.bfloat16, True), (128, 64, torch.float32, False), (96, 64, torch.bfloat16, False), (128, 24, torch.bfloat16, False), (128, 160, torch.bfloat16, False), (4160, 32, torch.bfloat16, False)])
+def test_a_token_inputs_projection_is_held_twice_only_where_both_kernels_run(dim, side, dtype, kept):
+    from cwm_amd.parts import GatedTokenSide
+    from cwm_amd.parts.base import Runtime
+
+    part = GatedTokenSide(11, dim, side, 0, 1, 1e-6)
+    tensors = {name: torch.zeros(spec.shape, dtype=dtype) for name, spec in part.tensor_specs().items()}
+    part.bind(tensors, Runtime(torch.device("cpu"), dtype))
+    assert (part.w_proj is not None) == kept and part.w_proj_t.shape == (side, dim)
