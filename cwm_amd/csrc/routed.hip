@@ -6,7 +6,7 @@
 //                    equal groups of neighbours, of which only those with the best members stay open to the choice.
 //   group_by_expert  the step's (token, choice) pairs grouped by expert, each group padded to whole tiles of 16
 //                    rows: row_token[row] (-1 in the padding), pair_row[pair], tile_expert[tile] (-1 beyond the
-//                    last tile), and behind the last tile the number of tiles in use.  One block; no count leaves the
+//                    last tile), and in a place of its own the number of tiles up to the last.  One block; no count leaves the
 //                    device.  The order of a group's rows is whatever the block's atomic counters give: a row's
 //                    result does not depend on its place.
 //   grouped product  out[row] = W[e(row)] a[row] on the matrix cores, e from tile_expert (16 rows a tile share it)
@@ -268,8 +268,8 @@ extern "C" int cwm_route_top(const float* logits, int* chosen, float* weights, i
 
 // The grouping, by one block; `chosen` may lie in global memory or in LDS.
 __device__ __forceinline__ void group_pairs(const int* chosen, int n_pairs, int n_experts, int* __restrict__ row_token,
-                                            int* __restrict__ pair_row, int* __restrict__ tile_expert, int n_tiles, int top,
-                                            int tile_align, int* count, int* start) {
+                                            int* __restrict__ pair_row, int* __restrict__ tile_expert, int* __restrict__ used, int n_tiles,
+                                            int top, int tile_align, int* count, int* start) {
   for (int e = threadIdx.x; e < n_experts; e += blockDim.x) count[e] = 0;
   for (int i = threadIdx.x; i < n_tiles * TILE_ROWS; i += blockDim.x) row_token[i] = -1;
   __syncthreads();
@@ -314,7 +314,7 @@ __device__ __forceinline__ void group_pairs(const int* chosen, int n_pairs, int 
       if (4 * lane + q < n_experts) start[4 * lane + q] = tile * TILE_ROWS;
       tile += tiles[q];
     }
-    if (lane == CWM_WAVE - 1) tile_expert[n_tiles] = min(through, n_tiles);
+    if (lane == CWM_WAVE - 1) *used = min(through, n_tiles);
   }
   __syncthreads();
   // tile by tile: the last expert that starts at it or before (those without rows start where the next one does)
@@ -344,16 +344,16 @@ __device__ __forceinline__ void group_pairs(const int* chosen, int n_pairs, int 
 
 __global__ void __launch_bounds__(1024) group_by_expert_kernel(const int* __restrict__ chosen, int n_pairs, int n_experts,
                                                                int* __restrict__ row_token, int* __restrict__ pair_row,
-                                                               int* __restrict__ tile_expert, int n_tiles, int top, int tile_align) {
+                                                               int* __restrict__ tile_expert, int* __restrict__ used, int n_tiles, int top, int tile_align) {
   __shared__ int count[ROUTE_MAX_EXPERTS];
   __shared__ int start[ROUTE_MAX_EXPERTS];
-  group_pairs(chosen, n_pairs, n_experts, row_token, pair_row, tile_expert, n_tiles, top, tile_align, count, start);
+  group_pairs(chosen, n_pairs, n_experts, row_token, pair_row, tile_expert, used, n_tiles, top, tile_align, count, start);
 }
 
-// tile_expert: n_tiles + 1 entries.  tile_align: an expert's first tile lies at a multiple of so many tiles (the tiles that one block of the product takes).
+// used: one number, the tiles up to the last one that has rows, rounded up to tile_align.  tile_align: an expert's first tile lies at a multiple of so many tiles (the tiles that one block of the product takes).
 extern "C" int cwm_group_by_expert(const int* chosen, int n_tokens, int top, int n_experts, int* row_token, int* pair_row,
-                                   int* tile_expert, int n_tiles, int tile_align, hipStream_t stream) {
-  CWM_REQUIRE(chosen && row_token && pair_row && tile_expert, "group_by_expert: arguments missing");
+                                   int* tile_expert, int* used, int n_tiles, int tile_align, hipStream_t stream) {
+  CWM_REQUIRE(chosen && row_token && pair_row && tile_expert && used, "group_by_expert: arguments missing");
   CWM_REQUIRE(n_experts >= 1 && n_experts <= ROUTE_MAX_EXPERTS && top >= 1, "group_by_expert: %d experts, the kernel takes up to %d", n_experts,
               ROUTE_MAX_EXPERTS);
   const long n_pairs = (long)n_tokens * top;
@@ -361,7 +361,7 @@ extern "C" int cwm_group_by_expert(const int* chosen, int n_tokens, int top, int
               "group_by_expert: %d tiles do not hold %ld pairs of %d experts", n_tiles, n_pairs, n_experts);
   if (n_tokens <= 0) return 0;
   hipLaunchKernelGGL(group_by_expert_kernel, dim3(1), dim3(1024), 0, stream, chosen, (int)n_pairs, n_experts, row_token, pair_row, tile_expert,
-                     n_tiles, top, tile_align);
+                     used, n_tiles, top, tile_align);
   return cwm_launch_status("group_by_expert");
 }
 
@@ -648,7 +648,7 @@ __global__ void __launch_bounds__(256) grouped_stream_kernel(const T* __restrict
 // block whose wavefronts share both operands, 40% busy beside the matrix cores.
 // With a list the blocks are numbered so that an XCD gets a run of neighbours in the order (group of WIDE_GROUP row blocks,
 // columns, row block): the row blocks of an expert then share its weights in one L2, where dealing them to the XCDs in turn
-// has every XCD read every expert's weights.  The list says how many tiles it holds, so the runs are equally long.
+// has every XCD read every expert's weights.  `used` says how many tiles of the list are in use, so the runs are equally long.
 // 16 experts of 2,048 x 1,024, four a token, gate and up / down: 2,048 tokens 128 / 71 us (535 / 484 TFLOP/s; blocks that
 // staged both operands through LDS: 204 / 135 us), 4,096 tokens 215 / 117 us (370 / 240 us), 300 tokens 51 / 30 us (117 / 79
 // us straight from memory); the last round of blocks is nearly empty at some sizes, which costs up to a quarter.
@@ -657,7 +657,8 @@ __global__ void __launch_bounds__(256) grouped_stream_kernel(const T* __restrict
 template <int RT, int CT, bool GATED>
 __global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __restrict__ a, long a_ld, long a_batch, const int* __restrict__ row_token,
                                                               const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, long w_stride,
-                                                              const int* __restrict__ tile_expert, int n_tiles, int row_blocks, int col_blocks,
+                                                              const int* __restrict__ tile_expert, const int* __restrict__ used, int n_tiles,
+                                                              int row_blocks, int col_blocks,
                                                               void* __restrict__ out, int out_dtype, long out_ld, long out_batch, int vec_out,
                                                               int n_rows, int N, int K, GateAct act) {
   constexpr int ROWS = RT * TILE_ROWS, FETCH = ROWS * 8 / 256;  // 16-byte pieces of the rows that a thread fetches a step
@@ -668,7 +669,7 @@ __global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __re
   const int r = lane & 15, j = lane >> 4;
   int bx, by, expert;
   if (tile_expert) {
-    const int live = (tile_expert[n_tiles] + RT - 1) / RT, total = live * col_blocks;
+    const int live = ((used ? min(*used, n_tiles) : n_tiles) + RT - 1) / RT, total = live * col_blocks;
     const int run = (total + 7) >> 3, at = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= run || at >= total) return;
     const int first = at / (WIDE_GROUP * col_blocks) * WIDE_GROUP, rest = at - first * col_blocks;
@@ -804,10 +805,11 @@ static void launch_grouped(bool vec, int tiles, int n_batch, hipStream_t stream,
 // `a_batch` further).  w0 (and w1 for the gated form): [experts or batches][N][K], `w_stride` apart.  With
 // `tile_expert` the rows are the list's n_tiles * 16 and out is [rows][out_ld]; without, every batch z < n_batch
 // multiplies the same n_rows rows by its own weight into out + z * out_batch.  tiles_a_block: 1, 2, 4 or 8 row tiles
-// a block; with a list, an expert's tiles start at a multiple of `tile_align`, itself a multiple of tiles_a_block.  act_kind, act_alpha, act_limit: the gated
+// a block; with a list, an expert's tiles start at a multiple of `tile_align`, itself a multiple of tiles_a_block.  used: how many
+// of the list's tiles may have rows (`cwm_group_by_expert` leaves the number), or null: any of them.  act_kind, act_alpha, act_limit: the gated
 // form's activation (`GateAct`).
 extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int dtype, const int* row_token, const void* w0, const void* w1,
-                                   long w_stride, const int* tile_expert, int n_tiles, int n_batch, void* out, int out_dtype, long out_ld,
+                                   long w_stride, const int* tile_expert, const int* used, int n_tiles, int n_batch, void* out, int out_dtype, long out_ld,
                                    long out_batch, int n_rows, int N, int K, int tiles_a_block, int tile_align, int act_kind,
                                    float act_alpha, float act_limit, hipStream_t stream) {
   CWM_REQUIRE(a && w0 && out, "grouped_product: arguments missing");
@@ -852,7 +854,7 @@ extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int d
     dim3 grid((row_blocks * col_blocks + 7) / 8 * 8, 1, nb);                                                                               \
     if (!tile_expert) grid.x = row_blocks * col_blocks;                                                                                    \
     hipLaunchKernelGGL((grouped_wide_kernel<RT, CT, GATED>), grid, dim3(256), 0, stream, (const bf16_t*)a, a_ld, a_batch, row_token,        \
-                       (const bf16_t*)w0, (const bf16_t*)w1, w_stride, tile_expert, n_tiles, row_blocks, col_blocks, out, out_dtype,       \
+                       (const bf16_t*)w0, (const bf16_t*)w1, w_stride, tile_expert, used, n_tiles, row_blocks, col_blocks, out, out_dtype,       \
                        out_ld, out_batch, vec_out, n_rows, N, K, act);                                                                     \
   } while (0)
     // Four weight tiles a wavefront where that still makes about two blocks a compute unit, else two, which makes twice as

@@ -76,10 +76,11 @@ class ExpertGroups:
 
     row_token: torch.Tensor  # int32 [tiles * 16]: the token of each row, -1 in the padding
     pair_row: torch.Tensor  # int32 [T * top]: the row of each pair
-    tile_expert: torch.Tensor  # int32 [tiles]: the expert of each tile, -1 for tiles not in use (in memory, their number follows)
+    tile_expert: torch.Tensor  # int32 [tiles]: the expert of each tile, -1 for tiles not in use
     n_tiles: int
     tiles_a_block: int  # an expert's tiles start at a multiple of so many: the most row tiles that a block of the grouped product takes
     top: int
+    used: Optional[torch.Tensor] = None  # int32 [1]: the tiles up to the last one in use, where they have been counted
 
 
 def _tiles_a_block(rows: float) -> int:
@@ -108,14 +109,14 @@ def group_by_expert(chosen: torch.Tensor, n_experts: int) -> ExpertGroups:
     align = _tiles_a_block(pairs / n_experts)
     n_tiles = -(-pairs // TILE_ROWS) + n_experts * align
     lists = torch.empty(n_tiles * TILE_ROWS + pairs + n_tiles + 1, dtype=torch.int32, device=chosen.device)
-    a, b = n_tiles * TILE_ROWS, n_tiles * TILE_ROWS + pairs
-    groups = ExpertGroups(lists[:a], lists[a:b], lists[b:-1], n_tiles, align, top)
+    row_token, pair_row, tile_expert, used = lists.split_with_sizes((n_tiles * TILE_ROWS, pairs, n_tiles, 1))
+    groups = ExpertGroups(row_token, pair_row, tile_expert, n_tiles, align, top, used)
     lib = _build.load("routed")
     _check(
         lib,
         lib.cwm_group_by_expert(
             _ptr(chosen), ctypes.c_int(n), ctypes.c_int(top), ctypes.c_int(n_experts), _ptr(groups.row_token), _ptr(groups.pair_row),
-            _ptr(groups.tile_expert), ctypes.c_int(n_tiles), ctypes.c_int(align), _stream(),
+            _ptr(groups.tile_expert), _ptr(groups.used), ctypes.c_int(n_tiles), ctypes.c_int(align), _stream(),
         ),
     )
     return groups
@@ -132,6 +133,8 @@ def _grouped(
         raise KernelError("grouped weights must be contiguous [experts, N, K] tensors of the rows' type")
     e, n, k = w0.shape
     if groups is not None:
+        if groups.tile_expert.numel() < groups.n_tiles or groups.row_token.numel() < groups.n_tiles * TILE_ROWS:
+            raise KernelError(f"lists of {groups.tile_expert.numel()} tiles and {groups.row_token.numel()} rows do not hold {groups.n_tiles} tiles")
         tiles_a_block = min(groups.tiles_a_block, _product_tiles(a.dtype, k, groups.pair_row.numel() / e, w1 is not None))
     else:  # a product a head: few rows go through the weights' stream
         tiles_a_block = _product_tiles(a.dtype, k, n_rows, False) if n_rows >= MEDIUM_ROWS else 1
@@ -141,7 +144,7 @@ def _grouped(
         lib.cwm_grouped_product(
             _ptr(a), ctypes.c_long(a_ld), ctypes.c_long(a_batch), ctypes.c_int(_code(a.dtype)),
             _ptr(groups.row_token if groups is not None else None), _ptr(w0), _ptr(w1), ctypes.c_long(n * k),
-            _ptr(groups.tile_expert if groups is not None else None), ctypes.c_int(groups.n_tiles if groups is not None else 0),
+            _ptr(groups.tile_expert if groups is not None else None), _ptr(groups.used if groups is not None else None), ctypes.c_int(groups.n_tiles if groups is not None else 0),
             ctypes.c_int(n_batch), _ptr(out), ctypes.c_int(_code(out.dtype)), ctypes.c_long(out_ld), ctypes.c_long(out_batch),
             ctypes.c_int(n_rows), ctypes.c_int(n), ctypes.c_int(k), ctypes.c_int(tiles_a_block),
             ctypes.c_int(groups.tiles_a_block if groups is not None else 1),
@@ -190,7 +193,7 @@ def grouped_linear(rows: torch.Tensor, groups: ExpertGroups, weight: torch.Tenso
     if rows.dim() != 2 or not rows.is_contiguous() or weight.shape[2] != rows.shape[1] or rows.shape[0] != groups.n_tiles * TILE_ROWS:
         raise KernelError("the rows do not fit the list or the experts' weights")
     out = torch.empty((rows.shape[0], weight.shape[1]), dtype=torch.float32, device=rows.device)
-    identity = ExpertGroups(_identity_rows(rows.shape[0], rows.device), groups.pair_row, groups.tile_expert, groups.n_tiles, groups.tiles_a_block, groups.top)
+    identity = ExpertGroups(_identity_rows(rows.shape[0], rows.device), groups.pair_row, groups.tile_expert, groups.n_tiles, groups.tiles_a_block, groups.top, groups.used)
     _grouped(rows, rows.shape[1], 0, identity, weight, None, out, weight.shape[1], 0, rows.shape[0], 1)
     return out
 

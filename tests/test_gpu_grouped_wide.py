@@ -3,6 +3,8 @@ wavefront), results' columns that no block divides, experts without tokens and o
 
 from __future__ import annotations
 
+import dataclasses
+
 import pytest
 import torch
 
@@ -64,3 +66,21 @@ def test_rows_of_heads(n_tokens, heads, lead, d, n):
     assert torch.equal(ask[..., :lead], before[..., :lead])
     want = torch.einsum("thd,hnd->thn", rest.double().cpu(), weight.double().cpu()).to(DEV)
     assert bool(((ask[..., lead:].double() - want).abs() <= want.abs() * 2.0 ** -8 + 2e-5).all())
+
+
+@pytest.mark.parametrize("n_tokens", [30, 96, 600])
+def test_lists_that_lie_elsewhere(n_tokens):
+    """Copies of a step's lists, and lists without the number of tiles in use: what is read lies inside what is handed over."""
+    from cwm_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(n_tokens)
+    normal = lambda *shape: torch.randn(shape, generator=g, device=DEV)  # noqa: E731
+    x, (gate, up) = normal(n_tokens, 128).bfloat16(), (normal(8, 192, 128).bfloat16() for _ in range(2))
+    groups = ops.group_by_expert(normal(n_tokens, 8).topk(4).indices.int().contiguous(), 8)
+    want = ops.grouped_gate_up(x, groups, gate, up)[groups.pair_row.long()]
+    copies = dataclasses.replace(groups, row_token=groups.row_token.clone(), tile_expert=groups.tile_expert.clone(), used=groups.used.clone())
+    for lists in (copies, dataclasses.replace(copies, used=None)):
+        assert lists.tile_expert.numel() == lists.n_tiles
+        assert torch.equal(ops.grouped_gate_up(x, lists, gate, up)[groups.pair_row.long()], want)
+    with pytest.raises(ops.KernelError):
+        ops.grouped_gate_up(x, dataclasses.replace(groups, tile_expert=groups.tile_expert[:-1]), gate, up)
