@@ -1,11 +1,11 @@
-// C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in true float32 on the matrix cores
+// C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in float32 on the matrix cores
 // (v_mfma_f32_32x32x2_f32: float32 operands, exact products, float32 sums; float32 operands with
-// K a multiple of 32 in exact bfloat16 parts instead, see below): the matrix
+// K a multiple of 32 and up to 65,536 in exact bfloat16 parts instead, see below): the matrix
 // product of the 32-bit path.  Operands may be stored as float32 or bfloat16 (converted
-// exactly on load); nothing is rounded below float32 before the final store.  Every output
+// exactly on load).  Every output
 // element is the sum over k = 0, 1, ... in one fixed grouping (eight values at a time, as the
-// pairs (j, j + 4), j = 0..3), whatever tile of the result it lies in, so
-// a row's result does not depend on how many other rows the call has.  Any M, N, K.
+// pairs (j, j + 4), j = 0..3; 32 at a time in parts), whatever tile of the result it lies in, so
+// a row's result does not depend on the other rows of the call.  Any M, N, K.
 //
 // A block takes a BM x BN tile of C (128 x 128 with 4 wavefronts; 32 x 32 with one for at most 32
 // rows); tiles of A and W of BK values of k go through LDS, the next ones waiting in registers.
@@ -44,11 +44,13 @@ __device__ __forceinline__ void load4(const T* row, int k, int K, bool vec, floa
 }
 
 // WAVES_M x WAVES_N wavefronts, each with TM x TN matrix-instruction tiles of 32 x 32; BK: a multiple of 8
-// One block's tile of the result, from row m0 and column n0 on; As, Ws: BM and BN rows of BK + 4 floats of LDS
-template <typename TA, typename TW, typename TC, int WAVES_M, int WAVES_N, int TM, int TN, int BK>
+// One block's tile of the result, from row m0 and column n0 on; As, Ws: BM and BN rows of BK + 4 floats of LDS.  MARKED: only the
+// elements of the tile's rows and columns with a mark are stored.
+template <typename TA, typename TW, typename TC, int WAVES_M, int WAVES_N, int TM, int TN, int BK, bool MARKED = false>
 __device__ __forceinline__ void gemm_f32_tile(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw, TC* __restrict__ C, long ldc,
                                               const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int vec_a, int vec_w, const int m0,
-                                              const int n0, float* As, float* Ws) {
+                                              const int n0, float* As, float* Ws, const unsigned char* marked_rows = nullptr,
+                                              const unsigned char* marked_columns = nullptr) {
   constexpr int BM = 32 * TM * WAVES_M, BN = 32 * TN * WAVES_N, THREADS = 64 * WAVES_M * WAVES_N;
   constexpr int BKP = BK + 4, Q = BK / 4;  // Q: 16-byte pieces in a row of a step
   constexpr int A_LOADS = (BM * Q + THREADS - 1) / THREADS, W_LOADS = (BN * Q + THREADS - 1) / THREADS;
@@ -139,6 +141,7 @@ __device__ __forceinline__ void gemm_f32_tile(const TA* __restrict__ A, long lda
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int m = m0 + (wm * TM + i) * 32 + 8 * (e >> 2) + 4 * kh + (e & 3);
+        if (MARKED && !(marked_rows[m - m0] | marked_columns[n - n0])) continue;
         if (m < M) Elem<TC>::store(C + (size_t)m * ldc + n, acc[i][j][e] + b);
       }
   }
@@ -163,14 +166,25 @@ gemm_f32_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lo
 // instead of K / 2.  Against float64 (normal operands, K = 512, 4,096 and 14,336) a result is 3.4e-7, 1.0e-6 and 1.9e-6 off,
 // 4.1e-7, 1.15e-6 and 2.15e-6 with float32 operands; with positive operands 2.4e-7, 6.2e-7 and 1.2e-6 against 3.1e-7, 9.9e-7
 // and 1.8e-6.  Bound by the matrix cores and the vector instructions that make the parts (times that add).  743 rows, float32
-// operands and parts: 28,672 x 4,096 1,847 and 1,045 us (167 TFLOP/s of float32 products), 2,048 x 2,048 191 and 82 us; 64 rows
-// 6,144 x 4,096 361 and 144 us; 32 rows 168 and 94 us.
-// The parts are made on the way into LDS, so memory holds float32 as before.  The order of k and of the parts is the same for
-// every element of the result, whatever tile it lies in.  Values that round to infinity have no such parts: a block that
-// meets one (its largest magnitude says so) does its tile once more with float32 operands.
+// operands and parts: 28,672 x 4,096 1,847 and 1,030 us (169 TFLOP/s of float32 products), 2,048 x 2,048 191 and 78 us; 64 rows
+// 6,144 x 4,096 361 and 139 us; 32 rows 168 and 91 us.
+// The parts are made on the way into LDS, so memory holds float32 as before.  Both operands are multiplied by 2^23 first, and
+// the sums by 2^-46 at the end, which rounds nothing: the last bit of the smallest float32 is then a normal bfloat16, so that the parts
+// of small values are exact too (without it the third part is lost below 2^-110 and the second below 2^-118).  Rows of A and W with a
+// value of 2^32 or more, or an infinity, are left to float32 operands, element by element of the result: with smaller ones the sums of
+// up to 65,536 scaled products stay below 2^126.  So an element's order of k and of the parts depends on its own row and column alone.
 #define SPLIT_STEP 32
 #define SPLIT_LD (SPLIT_STEP + 8)      // a row of a part in LDS: 80 bytes, so that 16 rows' pieces lie in different banks
-#define SPLIT_LIMIT 3.3895313e38f      // from here on bfloat16 rounds to infinity
+#define SPLIT_MOST_K 65536
+#define SPLIT_SCALE 8388608.0f               // 2^23
+#define SPLIT_UNSCALE 1.4210854715202004e-14f  // 2^-46
+#define SPLIT_LIMIT 3.602879701896397e16f    // 2^55: 2^32 once scaled
+
+typedef __bf16 bf16_pair __attribute__((ext_vector_type(2)));
+// c plus the product of two pairs of bfloat16 values (v_dot2_f32_bf16); with (-1, 0) or (0, -1) for `by`: c less one of the pair
+__device__ __forceinline__ float plus_pairs(uint32_t pair, uint32_t by, float c) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16_pair, pair), __builtin_bit_cast(bf16_pair, by), c, false);
+}
 
 // WAVES_M x WAVES_N wavefronts, each with TM x TN tiles of 16 x 16
 template <typename TC, int WAVES_M, int WAVES_N, int TM, int TN>
@@ -181,6 +195,7 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
   constexpr int A_LOADS = BM * (SPLIT_STEP / 4) / THREADS, W_LOADS = BN * (SPLIT_STEP / 4) / THREADS;
   constexpr int PARTS_BYTES = 3 * (BM + BN) * SPLIT_LD * 2, WHOLE_BYTES = (BM + BN) * (16 + 4) * 4;
   __shared__ __attribute__((aligned(16))) unsigned char lds[PARTS_BYTES > WHOLE_BYTES ? PARTS_BYTES : WHOLE_BYTES];
+  __shared__ unsigned char marked_rows[BM], marked_columns[BN];
   bf16_t* a_parts = (bf16_t*)lds;                  // [3][BM][SPLIT_LD]
   bf16_t* w_parts = a_parts + 3 * BM * SPLIT_LD;   // [3][BN][SPLIT_LD]
   // an XCD gets a run of neighbours, the row blocks of a panel of W one after the other: its L2 reads the panel once
@@ -205,16 +220,26 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
 #pragma unroll
     for (int i = 0; i < W_LOADS; ++i) rw[set][i] = *(const float4v*)(src_w[i] + k0);
   };
-  float largest = 0.f;
-  auto stage = [&](float4v v, bf16_t* parts, int plane, int f) {
+  // (-1, 0) and (0, -1), in registers: as an inline constant the instruction reads -1.0 as something else
+  uint32_t less_first = 0x0000bf80u, less_second = 0xbf800000u;
+  asm("" : "+v"(less_first), "+v"(less_second));
+  float largest_a[A_LOADS] = {}, largest_w[W_LOADS] = {};  // of a thread's pieces, which are the same rows' in every step
+  auto stage = [&](float4v v, bf16_t* parts, int plane, int f, float& largest) {
+    v *= SPLIT_SCALE;
     largest = fmaxf(largest, fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
     bf16_t* to = parts + (f / 8) * SPLIT_LD + 4 * (f % 8);
 #pragma unroll
     for (int part = 0; part < 3; ++part) {
       const uint32_t lo = pack2_bf16(v[0], v[1]), hi = pack2_bf16(v[2], v[3]);
       *(uint2*)(to + part * plane) = make_uint2(lo, hi);
-      v[0] -= __uint_as_float(lo << 16), v[1] -= __uint_as_float(lo & 0xffff0000u);
-      v[2] -= __uint_as_float(hi << 16), v[3] -= __uint_as_float(hi & 0xffff0000u);
+      // what is left, exactly
+      if constexpr (TM * TN <= 8) {  // one instruction an element; beside 96 matrix instructions a step it is the slower one (1,024 rows, 4,096 x 14,336: 899 and 864 us)
+        v[0] = plus_pairs(lo, less_first, v[0]), v[1] = plus_pairs(lo, less_second, v[1]);
+        v[2] = plus_pairs(hi, less_first, v[2]), v[3] = plus_pairs(hi, less_second, v[3]);
+      } else {
+        v[0] -= __uint_as_float(lo << 16), v[1] -= __uint_as_float(lo & 0xffff0000u);
+        v[2] -= __uint_as_float(hi << 16), v[3] -= __uint_as_float(hi & 0xffff0000u);
+      }
     }
   };
   float4v acc[TM][TN];
@@ -224,9 +249,9 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
     for (int b = 0; b < TN; ++b) acc[a][b] = (float4v){0.f, 0.f, 0.f, 0.f};
   auto step = [&](int set, int next) {
 #pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) stage(ra[set][i], a_parts, BM * SPLIT_LD, tid + i * THREADS);
+    for (int i = 0; i < A_LOADS; ++i) stage(ra[set][i], a_parts, BM * SPLIT_LD, tid + i * THREADS, largest_a[i]);
 #pragma unroll
-    for (int i = 0; i < W_LOADS; ++i) stage(rw[set][i], w_parts, BN * SPLIT_LD, tid + i * THREADS);
+    for (int i = 0; i < W_LOADS; ++i) stage(rw[set][i], w_parts, BN * SPLIT_LD, tid + i * THREADS, largest_w[i]);
     __syncthreads();
     fetch(set, next);
     Frag8 fa[3][TM];
@@ -255,12 +280,20 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
     step(1, k0 + 3 * SPLIT_STEP);
   }
   if (k0 < K) step(0, K);
-  if (__syncthreads_or(!(largest < SPLIT_LIMIT))) {
-    constexpr int WHOLE_M = BM / 32, WHOLE_N = BN / 32;
-    gemm_f32_tile<float, float, TC, WAVES_M, WAVES_N, WHOLE_M / WAVES_M, WHOLE_N / WAVES_N, 16>(A, lda, W, ldw, C, ldc, bias, bias_dtype, M, N, K, 1, 1, m0, n0,
-                                                                                                 (float*)lds, (float*)lds + BM * 20);
-    return;
-  }
+  // eight neighbouring threads have a row's pieces
+  bool any = false;
+  auto mark = [&](float largest, unsigned char* marks, int f) {
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) largest = fmaxf(largest, __shfl_xor(largest, off, CWM_WAVE));
+    const bool beyond = !(largest < SPLIT_LIMIT);
+    any |= beyond;
+    if ((f & 7) == 0) marks[f / 8] = beyond;
+  };
+#pragma unroll
+  for (int i = 0; i < A_LOADS; ++i) mark(largest_a[i], marked_rows, tid + i * THREADS);
+#pragma unroll
+  for (int i = 0; i < W_LOADS; ++i) mark(largest_w[i], marked_columns, tid + i * THREADS);
+  any = __syncthreads_or(any);
   // lane 16 j + r of a tile holds row r, columns 4 j + i
 #pragma unroll
   for (int b = 0; b < TN; ++b)
@@ -273,9 +306,15 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
 #pragma unroll
       for (int a = 0; a < TM; ++a) {
         const int m = m0 + (wm * TM + a) * 16 + r;
-        if (m < M) Elem<TC>::store(C + (size_t)m * ldc + n, acc[a][b][i] + add);
+        if (any && (marked_rows[m - m0] | marked_columns[n - n0])) continue;
+        if (m < M) Elem<TC>::store(C + (size_t)m * ldc + n, acc[a][b][i] * SPLIT_UNSCALE + add);
       }
     }
+  if (any) {
+    constexpr int WHOLE_M = BM / 32, WHOLE_N = BN / 32;
+    gemm_f32_tile<float, float, TC, WAVES_M, WAVES_N, WHOLE_M / WAVES_M, WHOLE_N / WAVES_N, 16, true>(
+        A, lda, W, ldw, C, ldc, bias, bias_dtype, M, N, K, 1, 1, m0, n0, (float*)lds, (float*)lds + BM * 20, marked_rows, marked_columns);
+  }
 }
 
 template <typename TC>
@@ -304,7 +343,7 @@ static void launch(const void* A, long lda, const void* W, long ldw, void* C, lo
   const int vec_a = lda % 4 == 0 && ((uintptr_t)A % 16) == 0;
   const int vec_w = ldw % 4 == 0 && ((uintptr_t)W % 16) == 0;
   if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4) {
-    if (vec_a && vec_w && K % SPLIT_STEP == 0) {  // whatever M is: a row's result does not depend on the others
+    if (vec_a && vec_w && K % SPLIT_STEP == 0 && K <= SPLIT_MOST_K) {  // whatever M is: a row's result does not depend on the others
       launch_split<TC>((const float*)A, lda, (const float*)W, ldw, (TC*)C, ldc, bias, bias_dtype, M, N, K, stream);
       return;
     }

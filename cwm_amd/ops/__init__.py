@@ -207,7 +207,8 @@ def gemm_f32(
     bias: Optional[torch.Tensor] = None,
     out_dtype: Optional[torch.dtype] = None,
 ) -> torch.Tensor:
-    """x [M, K] @ weight[N, K]^T (+ bias) with float32 multiply-add (no matrix cores)."""
+    """x [M, K] @ weight[N, K]^T (+ bias) in float32: float32 sums of products that are exact, or (float32
+    operands, K a multiple of 32) exact to 2^-24 of themselves, on the matrix cores; see csrc/gemm_f32.hip."""
     _need_gpu(x, weight, bias)
     if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
         raise KernelError(f"gemm: x {tuple(x.shape)} and weight {tuple(weight.shape)} do not fit")
@@ -308,7 +309,7 @@ def linear(
 ) -> torch.Tensor:
     """y = x W^T (+ b).  cwm/fastgen/forward.py:593-606.
 
-    float32 activations or float32 weights: the float32 kernels (exact products; up to 16
+    float32 activations or float32 weights: the float32 kernels (`gemm_f32`; up to 16
     rows of float32 on the weight-streaming one, whose sums differ from the other's by rounding).
     bfloat16 activations and weights: matrix cores with float32 accumulation, the
     library product for many rows.  With `partials_ok` the result may be float32

@@ -68,3 +68,36 @@ def test_values_beyond_the_parts():
     fine = torch.isfinite(want)
     torch.testing.assert_close(got[fine], want[fine], rtol=1e-5, atol=2e-5)
     assert bool((got[~fine & ~torch.isnan(want)] == want[~fine & ~torch.isnan(want)]).all())
+
+
+@pytest.mark.parametrize("m", [17, 40, 300])
+@pytest.mark.parametrize("a_size,w_size", [(1e-30, 1e3), (1e-36, 1e4), (1e-38, 1e9), (3e-43, 1e9), (1e-19, 1e-18), (1e-25, 1e-9), (1e9, 1e-36), (4e9, 4e9)])
+def test_sizes_at_the_ends_of_float32(m, a_size, w_size):
+    """Operands and products down to the smallest normal numbers and below, where a part more than the last bit would be lost."""
+    from cwm_amd import ops
+
+    n, k = 130, 96
+    a, w = _normal((m, k), 5) * a_size, _normal((n, k), 6).clamp(-1, 1) * w_size
+    a[:, ::7] = 0.0
+    got, want = ops.gemm_f32(a, w).double(), a.double() @ w.double().T
+    # as in the first test, and half of the smallest float32 number for a result below the normal ones
+    bound = (a.double().abs() @ w.double().abs().T) * (2.0 ** -23 + 0.2 * k * 2.0 ** -24) + 2.0 ** -150
+    assert bool(((got - want).abs() <= bound).all())
+
+
+def test_a_value_beyond_the_parts_changes_no_other_row():
+    from cwm_amd import ops
+
+    m, n, k = 140, 150, 64
+    a, w, b = _normal((m, k), 3), _normal((n, k), 4), _normal((n,), 5)
+    fine = ops.gemm_f32(a, w, b)
+    odd, odd_w = a.clone(), w.clone()
+    odd[5, 7], odd[20, 1], odd[139, 60], odd[60, 3], odd[61, 3] = math.inf, -math.inf, math.nan, 3.4e38, 2.0 ** 32
+    odd_w[8, 3], odd_w[149, 0] = 1e30, math.inf
+    got = ops.gemm_f32(odd, odd_w, b)
+    rows = [i for i in range(m) if i not in (5, 20, 139, 60, 61)]
+    columns = [i for i in range(n) if i not in (8, 149)]
+    assert torch.equal(got[rows][:, columns], fine[rows][:, columns])
+    # and the odd rows and columns are the same in any company
+    assert torch.equal(ops.gemm_f32(odd[60:62].contiguous(), odd_w, b), got[60:62])
+    assert torch.equal(ops.gemm_f32(odd, odd_w[8:9].contiguous(), b[8:9].contiguous())[:, 0][rows], got[:, 8][rows])
