@@ -970,24 +970,24 @@ class StaticPlans:
     def __init__(self, device: torch.device, max_keys: int) -> None:
         self.device = device
         self.max_keys = max_keys  # the most keys a sequence may hold while the capture is in use
-        self.homes: dict = {}  # (group, key/value heads, window, chunk) -> (capacity, device vector, uploaded plan)
+        self.homes: dict = {}  # (group, key/value heads, window, chunk, whether keys are cut finer) -> (capacity, device vector, uploaded plan)
 
-    def _padded(self, batch, group: int, n_kv: int, window: Optional[int], capacity, chunk: Optional[int] = None):
-        from .attention_plan import FEW_HEADS, build_plan, capacity_until, pad_plan
+    def _padded(self, batch, group: int, n_kv: int, window: Optional[int], capacity, chunk: Optional[int], finer: bool):
+        from .attention_plan import build_plan, capacity_until, pad_plan
 
         wide_cut_below = -(-2 * _compute_units(self.device) // n_kv)
         if capacity is None:
-            plan, capacity = capacity_until(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, self.max_keys, chunk, n_kv <= FEW_HEADS)
+            plan, capacity = capacity_until(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, self.max_keys, chunk, finer)
         else:
-            plan = build_plan(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, chunk, n_kv <= FEW_HEADS)
+            plan = build_plan(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, chunk, finer)
         flat = pad_plan(plan, capacity)
         return plan, capacity, flat
 
-    def plan(self, batch, group: int, n_kv: int, window: Optional[int], chunk: Optional[int] = None) -> "_UploadedPlan":
-        key = (group, n_kv, window, chunk)
+    def plan(self, batch, group: int, n_kv: int, window: Optional[int], chunk: Optional[int], finer: bool) -> "_UploadedPlan":
+        key = (group, n_kv, window, chunk, finer)
         home = self.homes.get(key)
         if home is None:
-            plan, capacity, flat = self._padded(batch, group, n_kv, window, None, chunk)
+            plan, capacity, flat = self._padded(batch, group, n_kv, window, None, chunk, finer)
             if flat is None:
                 raise KernelError("this step's attention work has items that a captured step does not take")
             dev = torch.from_numpy(flat).pin_memory().to(self.device, non_blocking=True)
@@ -1002,27 +1002,28 @@ class StaticPlans:
 
     def refresh(self, batch) -> bool:
         """Fill every home with the lists of `batch`; False if one of them has outgrown its home."""
-        for (group, n_kv, window, chunk), (capacity, dev, _) in self.homes.items():
-            _, _, flat = self._padded(batch, group, n_kv, window, capacity, chunk)
+        for (group, n_kv, window, chunk, finer), (capacity, dev, _) in self.homes.items():
+            _, _, flat = self._padded(batch, group, n_kv, window, capacity, chunk, finer)
             if flat is None:
                 return False
             dev.copy_(torch.from_numpy(flat).pin_memory(), non_blocking=True)
         return True
 
 
-def _attention_plan(batch, group: int, n_kv: int, window: Optional[int], device: torch.device, chunk: Optional[int] = None) -> _UploadedPlan:
-    """The step's work list for this (group size, key/value heads, window or block of keys), uploaded once per step."""
-    from .attention_plan import FEW_HEADS, build_plan
+def _attention_plan(batch, group: int, n_kv: int, head_dim: int, window: Optional[int], device: torch.device, chunk: Optional[int] = None) -> _UploadedPlan:
+    """The step's work list for this (group size, key/value heads and their size, window or block of keys), uploaded once per step."""
+    from .attention_plan import build_plan, cuts_finer
 
+    finer = cuts_finer(n_kv, head_dim)
     static = getattr(batch, "static", None)
     if static is not None:
-        return static.plan(batch, group, n_kv, window, chunk)
-    key = ("attention_plan", group, n_kv, window, chunk)
+        return static.plan(batch, group, n_kv, window, chunk, finer)
+    key = ("attention_plan", group, n_kv, window, chunk, finer)
     cached = batch.scratch.get(key)
     if cached is None:
         # a sequence whose blocks of 128 rows, over all key/value heads, would not give every compute unit two
         wide_cut_below = -(-2 * _compute_units(device) // n_kv) if device.type == "cuda" else 0
-        plan = build_plan(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, chunk, n_kv <= FEW_HEADS)
+        plan = build_plan(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, chunk, finer)
         flat = np.concatenate([plan.work.reshape(-1), plan.work_wide.reshape(-1), plan.merge.reshape(-1)]).astype(np.int32)
         host = torch.from_numpy(flat)
         if device.type == "cuda":
@@ -1108,7 +1109,7 @@ def paged_attention_mfma(
     _i32(block_table, "block_table")
     if block_table.dim() != 2 or block_table.shape[0] != batch.n_seqs or n_tokens != batch.n_tokens:
         raise KernelError("block_table must be [B, W] for the batch's sequences, q [T, ...] for its tokens")
-    plan = _attention_plan(batch, n_q // n_kv, n_kv, window, q.device, chunk)
+    plan = _attention_plan(batch, n_q // n_kv, n_kv, hd, window, q.device, chunk)
     out = torch.empty((n_tokens, n_q * hd), dtype=q.dtype, device=q.device)
     partial = None
     if plan.n_partials:

@@ -30,16 +30,24 @@ def chunk_keys(n_keys, few_heads: bool = False):
     in chunks of 256).  Longer ranges are cut so that a few sequences still spread over the chip: 512 keys up
     to 8,192 (eight sequences in a window of 8,192 keys: 54 us against 58 us in chunks of 1,024), 1,024 up to
     65,536, then 2,048 (eight sequences of 131,072 keys: 647 us against 665 us in chunks of 4,096).
-    `few_heads` (see FEW_HEADS): chunks of 256 keys, of 512 beyond 8,192 and 1,024 beyond 65,536 keys.  With one key/value
-    head of 256 (attention through a latent) the chunks above leave most of the chip idle: eight sequences of 65 to
-    4,096 keys 45 us a layer and 19 us in chunks of 256, 48 of up to 2,048 keys 61 and 21 us, one of 4,096 20 and 17 us."""
+    `few_heads` (see `cuts_finer`): chunks of 256 keys, of 512 beyond 8,192 and 1,024 beyond 65,536 keys."""
     n = np.asarray(n_keys)
     if few_heads:
         return np.where(n <= 8192, 256, np.where(n <= 65536, 512, 1024))
     return np.where(n <= 2048, 2048, np.where(n <= 8192, 512, np.where(n <= 65536, 1024, 2048)))
 
 
-FEW_HEADS = 2  # key/value heads up to which a row tile's blocks are so few that its keys are cut finer
+def cuts_finer(n_kv: int, head_dim: int) -> bool:
+    """Whether a model's row tiles are so few, and each so much work, that their keys are cut finer (`chunk_keys`): one
+    key/value head of more than 128, which is attention through a latent.  The longer chunks leave most of the chip idle up to some
+    64 sequences: one head of 256, eight sequences of 16 to 4,096 keys 44 us a layer and 18 in chunks of 256, one of 2,000
+    59 and 16, 24 of up to 2,048 59 and 20, 64 of 1,100 40 and 30.  Below 512 keys and in large batches the merge costs more
+    than the cut gives: eight of 300 keys 14 and 16 us, 128 of 1,100 42 and 52, 256 of 1,100 57 and 81.  One or two heads of 128
+    gain less and lose sooner (two heads, eight sequences of 2,000 keys 24 and 12 us, but 64 of 1,100 18 and 21, 128 of 2,000 44 and
+    50, 256 of 300 19 and 28): they keep the longer chunks.  The rule cannot look at the batch, or a token's bits would."""
+    return n_kv == 1 and head_dim > 128
+
+
 MERGE_MID_MAX = 32  # partials up to which an item is merged by 4 wavefronts instead of 16
 WORK_INTS = 6
 PARTIAL_PAD = 4

@@ -1,8 +1,12 @@
-"""The work lists of attention with one or two key/value heads, whose keys are cut finer (host arithmetic only)."""
+"""The work lists of attention with one large key/value head, whose keys are cut finer (host arithmetic only)."""
+
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
+import torch
 
+from cwm_amd import ops
 from cwm_amd.ops.attention_plan import NULL_ROW, build_plan, capacity_until, pad_plan
 
 
@@ -45,3 +49,13 @@ def test_captured_lists_hold_a_window_at_every_place(few_heads, window, chunk, p
 def test_short_windows_leave_no_room_for_many_partials():
     _, capacity = capacity_until([1], [9000], 16, 4096, 0, 16384, few_heads=True)
     assert capacity.merge_many == 0 and capacity.merge_mid == 1
+
+
+@pytest.mark.parametrize("n_kv,head_dim,finer", [(1, 256, True), (1, 192, True), (1, 128, False), (2, 128, False), (2, 256, False), (8, 128, False)])
+def test_keys_are_cut_finer_for_one_large_head_alone(n_kv, head_dim, finer):
+    batch = SimpleNamespace(q_lens=[1, 1], kv_lens=[2000, 700], scratch={}, static=None)
+    plan = ops._attention_plan(batch, 16, n_kv, head_dim, None, torch.device("cpu"))
+    assert plan.n_work == (11 if finer else 2)
+    # lists of other sizes of head are others, in a captured step as well
+    other = ops._attention_plan(batch, 16, n_kv, 64, None, torch.device("cpu"))
+    assert other.n_work == 2 and (other is plan) == (not finer)
