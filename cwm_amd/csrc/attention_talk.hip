@@ -210,8 +210,8 @@ talk_stats_kernel(const float* __restrict__ scores, float* __restrict__ stats, c
   __shared__ float scratch[16];
   const int r = blockIdx.x, wave = threadIdx.x / CWM_WAVE, lane = threadIdx.x % CWM_WAVE;
   const TalkRow row = talk_row(R, r);
-  // the columns the row reads, and where the load that holds the first of them starts
-  const int c0 = row.first - row.base, c1 = row.p - row.base, start = c0 - c0 % V;
+  // the columns the row reads (keys before the table's first are not there), and where the load that holds the first of them starts
+  const int c0 = max(0, row.first - row.base), c1 = row.p - row.base, start = c0 - c0 % V;
   const float none = -__builtin_inff();
   // a load that would pass the table's last column starts earlier; the columns before its own place do not count
   auto counts = [&](int c, int e) {
