@@ -186,8 +186,10 @@ __device__ __forceinline__ float plus_pairs(uint32_t pair, uint32_t by, float c)
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16_pair, pair), __builtin_bit_cast(bf16_pair, by), c, false);
 }
 
-// WAVES_M x WAVES_N wavefronts, each with TM x TN tiles of 16 x 16
-template <typename TC, int WAVES_M, int WAVES_N, int TM, int TN>
+// WAVES_M x WAVES_N wavefronts, each with TM x TN tiles of 16 x 16.  PAIRS: a value less its part in one instruction instead of two.
+// It has the shorter chain and the lower rate, so it pays where blocks wait for themselves: with 64 x 128 blocks and 300 rows of 4,096 x
+// 14,336 (160 blocks) 487 us and 504, 743 rows of 2,048 x 2,048 (192) 76 and 87, but 743 rows of 6,144 x 4,096 (576) 306 and 295.
+template <typename TC, int WAVES_M, int WAVES_N, int TM, int TN, bool PAIRS>
 __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, TM * TN <= 8 ? 3 : 2)
 gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, TC* __restrict__ C, long ldc,
                       const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int row_blocks, int total) {
@@ -226,14 +228,17 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
   float largest_a[A_LOADS] = {}, largest_w[W_LOADS] = {};  // of a thread's pieces, which are the same rows' in every step
   auto stage = [&](float4v v, bf16_t* parts, int plane, int f, float& largest) {
     v *= SPLIT_SCALE;
-    largest = fmaxf(largest, fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+    if constexpr (TM * TN > 8)  // two instructions, or three in a shorter chain
+      largest = fmaxf(fmaxf(fmaxf(fmaxf(largest, fabsf(v[0])), fabsf(v[1])), fabsf(v[2])), fabsf(v[3]));
+    else
+      largest = fmaxf(largest, fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
     bf16_t* to = parts + (f / 8) * SPLIT_LD + 4 * (f % 8);
 #pragma unroll
     for (int part = 0; part < 3; ++part) {
       const uint32_t lo = pack2_bf16(v[0], v[1]), hi = pack2_bf16(v[2], v[3]);
       *(uint2*)(to + part * plane) = make_uint2(lo, hi);
       // what is left, exactly
-      if constexpr (TM * TN <= 8) {  // one instruction an element; beside 96 matrix instructions a step it is the slower one (1,024 rows, 4,096 x 14,336: 899 and 864 us)
+      if constexpr (PAIRS) {
         v[0] = plus_pairs(lo, less_first, v[0]), v[1] = plus_pairs(lo, less_second, v[1]);
         v[2] = plus_pairs(hi, less_first, v[2]), v[3] = plus_pairs(hi, less_second, v[3]);
       } else {
@@ -320,19 +325,19 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
 template <typename TC>
 static void launch_split(const float* A, long lda, const float* W, long ldw, TC* C, long ldc, const void* bias, int bias_dtype, int M, int N, int K,
                          hipStream_t stream) {
-#define CWM_SPLIT(WAVES_M, WAVES_N, TM, TN)                                                                                                \
+#define CWM_SPLIT(WAVES_M, WAVES_N, TM, TN, PAIRS)                                                                                          \
   do {                                                                                                                                     \
     const int row_blocks = (M + 16 * TM * WAVES_M - 1) / (16 * TM * WAVES_M), total = row_blocks * ((N + 16 * TN * WAVES_N - 1) / (16 * TN * WAVES_N)); \
-    hipLaunchKernelGGL((gemm_f32_split_kernel<TC, WAVES_M, WAVES_N, TM, TN>), dim3((total + 7) / 8 * 8), dim3(64 * WAVES_M * WAVES_N), 0, stream, A,   \
+    hipLaunchKernelGGL((gemm_f32_split_kernel<TC, WAVES_M, WAVES_N, TM, TN, PAIRS>), dim3((total + 7) / 8 * 8), dim3(64 * WAVES_M * WAVES_N), 0, stream, A,   \
                        lda, W, ldw, C, ldc, bias, bias_dtype, M, N, K, row_blocks, total);                                                \
   } while (0)
   const long wide = (long)((M + 127) / 128) * ((N + 127) / 128);
   if (M <= 32)
-    CWM_SPLIT(1, 2, 2, 2);
+    CWM_SPLIT(1, 2, 2, 2, true);
   else if (M <= 64 || wide < 512)  // too few blocks of 128 x 128 for two a compute unit
-    CWM_SPLIT(2, 2, 2, 4);
+    if ((long)((M + 63) / 64) * ((N + 127) / 128) <= 256) CWM_SPLIT(2, 2, 2, 4, true); else CWM_SPLIT(2, 2, 2, 4, false);
   else
-    CWM_SPLIT(2, 2, 4, 4);
+    CWM_SPLIT(2, 2, 4, 4, false);
 #undef CWM_SPLIT
 }
 
