@@ -12,7 +12,8 @@
 //   grouped product  out[row] = W[e(row)] a[row] on the matrix cores, e from tile_expert (16 rows a tile share it)
 //                    or, for a batch of independent products (one weight per head, say), from the block's z.
 //                    bfloat16 operands on v_mfma_f32_16x16x32_bf16, float32 operands on v_mfma_f32_16x16x4_f32
-//                    (exact products); float32 sums in the order of k either way, whatever else is in the step.
+//                    (exact products); float32 sums, in the order of k, or in four parts of it where the weights are
+//                    streamed (the rows an expert has on average choose: a row's bits hang on the step by that rounding).
 //                    With two weights the epilogue forms silu(W0 a) * (W1 a), or another form of `GateAct`.
 //   combine          out[t] = sum_k weight[t][k] * rows[pair_row[t][k]] in the order of k, float32.
 //
@@ -649,9 +650,10 @@ __global__ void __launch_bounds__(256) grouped_stream_kernel(const T* __restrict
 // With a list the blocks are numbered so that an XCD gets a run of neighbours in the order (group of WIDE_GROUP row blocks,
 // columns, row block): the row blocks of an expert then share its weights in one L2, where dealing them to the XCDs in turn
 // has every XCD read every expert's weights.  `used` says how many tiles of the list are in use, so the runs are equally long.
-// 16 experts of 2,048 x 1,024, four a token, gate and up / down: 2,048 tokens 128 / 71 us (535 / 484 TFLOP/s; blocks that
-// staged both operands through LDS: 204 / 135 us), 4,096 tokens 215 / 117 us (370 / 240 us), 300 tokens 51 / 30 us (117 / 79
-// us straight from memory); the last round of blocks is nearly empty at some sizes, which costs up to a quarter.
+// 16 experts of 2,048 x 1,024, four a token, evenly loaded, gate and up / down: 2,048 tokens 128 / 71 us (535 / 484 TFLOP/s; blocks
+// that staged both operands through LDS: 204 / 135 us), 4,096 tokens 215 / 117 us (370 / 240 us), 300 tokens 51 / 30 us (117 / 79
+// us straight from memory).  With a router's uneven loads 2,048 tokens take 146 / 85 us; the last round of blocks is nearly empty at
+// some sizes, which costs up to a quarter.
 #define WIDE_GROUP 4
 
 template <int RT, int CT, bool GATED>
