@@ -163,21 +163,26 @@ gemm_f32_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lo
 // most 16 bits), a3 what is left (at most 8 bits).  a * w is then the sum of nine products of parts, exact in float32, of which
 // the six largest are added up on the bfloat16 matrix instruction (v_mfma_f32_16x16x32_bf16, float32 sums), 16 times the
 // rate of the float32 one: the three left out are below 2^-24 of the product together, and a sum takes 6 K / 32 roundings
-// instead of K / 2.  Against float64 (normal operands, K = 512, 4,096 and 14,336) a result is 3.4e-7, 1.0e-6 and 1.9e-6 off,
-// 4.1e-7, 1.15e-6 and 2.15e-6 with float32 operands; with positive operands 2.4e-7, 6.2e-7 and 1.2e-6 against 3.1e-7, 9.9e-7
+// instead of K / 2.  Against float64 (normal operands, K = 512, 4,096 and 14,336) a result is 3.3e-7, 9.7e-7 and 1.8e-6 off,
+// 4.0e-7, 1.15e-6 and 2.1e-6 with float32 operands; with positive operands 2.6e-7, 6.1e-7 and 1.1e-6 against 3.5e-7, 9.9e-7
 // and 1.8e-6.  Bound by the matrix cores and the vector instructions that make the parts (times that add).  743 rows, float32
-// operands and parts: 28,672 x 4,096 1,847 and 1,030 us (169 TFLOP/s of float32 products), 2,048 x 2,048 191 and 78 us; 64 rows
-// 6,144 x 4,096 361 and 139 us; 32 rows 168 and 91 us.
+// operands and parts: 28,672 x 4,096 1,847 and 1,034 us (169 TFLOP/s of float32 products), 2,048 x 2,048 191 and 74 us; 64 rows
+// 6,144 x 4,096 361 and 136 us; 32 rows 168 and 91 us.
 // The parts are made on the way into LDS, so memory holds float32 as before.  Both operands are multiplied by 2^23 first, and
 // the sums by 2^-46 at the end, which rounds nothing: the last bit of the smallest float32 is then a normal bfloat16, so that the parts
 // of small values are exact too (without it the third part is lost below 2^-110 and the second below 2^-118).  Rows of A and W with a
 // value of 2^32 or more, or an infinity, are left to float32 operands, element by element of the result: with smaller ones the sums of
 // up to 65,536 scaled products stay below 2^126.  So an element's order of k and of the parts depends on its own row and column alone.
+// The bfloat16 instruction rounds its sums down, not to the nearest: left alone, every result is low by the same amount (2.5e-8, 1.0e-7
+// and 4.1e-7 of the results' size at K = 512, 2,048 and 8,192), which adds up over a model's layers (16 layers of width 2,048: logits
+// 2.9e-6 off float64 where float32 operands are 2.4e-6).  So the 8 steps in the middle of every 16 go into the sum with its sign turned,
+// where rounding down is up: logits 2.0e-6 off, at the same times.
 #define SPLIT_STEP 32
 #define SPLIT_LD (SPLIT_STEP + 8)      // a row of a part in LDS: 80 bytes, so that 16 rows' pieces lie in different banks
 #define SPLIT_MOST_K 65536
 #define SPLIT_SCALE 8388608.0f               // 2^23
 #define SPLIT_UNSCALE 1.4210854715202004e-14f  // 2^-46
+#define SPLIT_TURN 4                         // steps after which the sum's sign turns, and 8 later again, of every 16
 #define SPLIT_LIMIT 3.602879701896397e16f    // 2^55: 2^32 once scaled
 
 typedef __bf16 bf16_pair __attribute__((ext_vector_type(2)));
@@ -226,8 +231,9 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
   uint32_t less_first = 0x0000bf80u, less_second = 0xbf800000u;
   asm("" : "+v"(less_first), "+v"(less_second));
   float largest_a[A_LOADS] = {}, largest_w[W_LOADS] = {};  // of a thread's pieces, which are the same rows' in every step
-  auto stage = [&](float4v v, bf16_t* parts, int plane, int f, float& largest) {
-    v *= SPLIT_SCALE;
+  float sign = 1.f;  // of the sums, and so of A's parts
+  auto stage = [&](float4v v, float scale, bf16_t* parts, int plane, int f, float& largest) {
+    v *= scale;
     if constexpr (TM * TN > 8)  // two instructions, or three in a shorter chain
       largest = fmaxf(fmaxf(fmaxf(fmaxf(largest, fabsf(v[0])), fabsf(v[1])), fabsf(v[2])), fabsf(v[3]));
     else
@@ -254,9 +260,9 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
     for (int b = 0; b < TN; ++b) acc[a][b] = (float4v){0.f, 0.f, 0.f, 0.f};
   auto step = [&](int set, int next) {
 #pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) stage(ra[set][i], a_parts, BM * SPLIT_LD, tid + i * THREADS, largest_a[i]);
+    for (int i = 0; i < A_LOADS; ++i) stage(ra[set][i], sign * SPLIT_SCALE, a_parts, BM * SPLIT_LD, tid + i * THREADS, largest_a[i]);
 #pragma unroll
-    for (int i = 0; i < W_LOADS; ++i) stage(rw[set][i], w_parts, BN * SPLIT_LD, tid + i * THREADS, largest_w[i]);
+    for (int i = 0; i < W_LOADS; ++i) stage(rw[set][i], SPLIT_SCALE, w_parts, BN * SPLIT_LD, tid + i * THREADS, largest_w[i]);
     __syncthreads();
     fetch(set, next);
     Frag8 fa[3][TM];
@@ -281,6 +287,13 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
   fetch(1, SPLIT_STEP);
   int k0 = 0;
   for (; k0 + 2 * SPLIT_STEP <= K; k0 += 2 * SPLIT_STEP) {
+    if (k0 / SPLIT_STEP % (2 * SPLIT_TURN) == SPLIT_TURN) {
+      sign = -sign;
+#pragma unroll
+      for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) acc[a][b] = -acc[a][b];
+    }
     step(0, k0 + 2 * SPLIT_STEP);
     step(1, k0 + 3 * SPLIT_STEP);
   }
@@ -312,7 +325,7 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
       for (int a = 0; a < TM; ++a) {
         const int m = m0 + (wm * TM + a) * 16 + r;
         if (any && (marked_rows[m - m0] | marked_columns[n - n0])) continue;
-        if (m < M) Elem<TC>::store(C + (size_t)m * ldc + n, acc[a][b][i] * SPLIT_UNSCALE + add);
+        if (m < M) Elem<TC>::store(C + (size_t)m * ldc + n, acc[a][b][i] * (sign * SPLIT_UNSCALE) + add);
       }
     }
   if (any) {

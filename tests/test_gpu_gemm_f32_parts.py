@@ -101,3 +101,15 @@ def test_a_value_beyond_the_parts_changes_no_other_row():
     # and the odd rows and columns are the same in any company
     assert torch.equal(ops.gemm_f32(odd[60:62].contiguous(), odd_w, b), got[60:62])
     assert torch.equal(ops.gemm_f32(odd, odd_w[8:9].contiguous(), b[8:9].contiguous())[:, 0][rows], got[:, 8][rows])
+
+
+@pytest.mark.parametrize("m,n", [(20, 2048), (227, 3072), (700, 9000)])
+@pytest.mark.parametrize("k", [512, 2048, 2080, 8192, 14336])
+def test_results_are_not_all_low_or_high(m, n, k):
+    """Roundings of an instruction that rounds down add up to the same amount in every result, and over a model's layers."""
+    from cwm_amd import ops
+
+    a, w = _normal((m, k), k), _normal((n, k), k + 1)
+    off = ops.gemm_f32(a, w).double() - a.double() @ w.double().T
+    # unbiased errors have a mean of their size over the root of their number, here at most 1 / 200 (five deviations: 0.025)
+    assert abs(float(off.mean())) <= 0.025 * float(off.square().mean().sqrt())
