@@ -695,7 +695,7 @@ __global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __re
     const int list_row = tile0 * TILE_ROWS + (id >> 3);
     long src;
     if (tile_expert)
-      src = list_row < n_tiles * TILE_ROWS ? max(row_token[list_row], 0) : 0;
+      src = list_row >= n_tiles * TILE_ROWS ? 0 : row_token ? max(row_token[list_row], 0) : min(list_row, n_rows - 1);
     else
       src = min(list_row, n_rows - 1);
     src_a[i] = a + (size_t)blockIdx.z * a_batch + (size_t)src * a_ld + (id & 7) * 8;
@@ -803,7 +803,7 @@ static void launch_grouped(bool vec, int tiles, int n_batch, hipStream_t stream,
                        w_stride, tile_expert, n_tiles, out, out_dtype, out_ld, out_batch, n_rows, N, K, act);
 }
 
-// a: rows of K values, `a_ld` apart (row `row_token[row]` for list row `row` if a list is given; batch z starts
+// a: rows of K values, `a_ld` apart (row `row_token[row]` for list row `row` if it is given, else row `row`; batch z starts
 // `a_batch` further).  w0 (and w1 for the gated form): [experts or batches][N][K], `w_stride` apart.  With
 // `tile_expert` the rows are the list's n_tiles * 16 and out is [rows][out_ld]; without, every batch z < n_batch
 // multiplies the same n_rows rows by its own weight into out + z * out_batch.  tiles_a_block: 1, 2, 4 or 8 row tiles
@@ -818,7 +818,7 @@ extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int d
   CWM_REQUIRE(act_kind >= 0 && act_kind <= 2, "grouped_product: unknown gated activation %d", act_kind);
   const GateAct act = {act_kind, act_alpha, act_limit};
   CWM_REQUIRE(N > 0 && K > 0 && a_ld >= K && out_ld >= 0, "grouped_product: bad sizes");
-  CWM_REQUIRE(tile_expert ? (n_tiles >= 0 && n_batch == 1 && row_token) : (n_batch >= 1 && n_batch <= 65535), "grouped_product: give a tile list or a number of batches");
+  CWM_REQUIRE(tile_expert ? (n_tiles >= 0 && n_batch == 1 && (row_token || n_rows >= n_tiles * TILE_ROWS)) : (n_batch >= 1 && n_batch <= 65535), "grouped_product: give a tile list or a number of batches");
   const int tiles = tile_expert ? n_tiles : (n_rows + TILE_ROWS - 1) / TILE_ROWS;
   if (tiles <= 0) return 0;
   const int esize = dtype == CWM_BF16 ? 2 : 4;

@@ -125,8 +125,9 @@ def group_by_expert(chosen: torch.Tensor, n_experts: int) -> ExpertGroups:
 def _grouped(
     a: torch.Tensor, a_ld: int, a_batch: int, groups: Optional[ExpertGroups], w0: torch.Tensor, w1: Optional[torch.Tensor],
     out: torch.Tensor, out_ld: int, out_batch: int, n_rows: int, n_batch: int,
-    activation: Optional["GatedActivation"] = None,
+    activation: Optional["GatedActivation"] = None, gather: bool = True,
 ) -> None:
+    """`gather`: `a` has the tokens' rows, which the list picks; else it has the list's own rows."""
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
     _need_gpu(a, w0, w1, out)
     if w0.dim() != 3 or not w0.is_contiguous() or w0.dtype != a.dtype or (w1 is not None and (w1.shape != w0.shape or not w1.is_contiguous() or w1.dtype != a.dtype)):
@@ -143,7 +144,7 @@ def _grouped(
         lib,
         lib.cwm_grouped_product(
             _ptr(a), ctypes.c_long(a_ld), ctypes.c_long(a_batch), ctypes.c_int(_code(a.dtype)),
-            _ptr(groups.row_token if groups is not None else None), _ptr(w0), _ptr(w1), ctypes.c_long(n * k),
+            _ptr(groups.row_token if groups is not None and gather else None), _ptr(w0), _ptr(w1), ctypes.c_long(n * k),
             _ptr(groups.tile_expert if groups is not None else None), _ptr(groups.used if groups is not None else None), ctypes.c_int(groups.n_tiles if groups is not None else 0),
             ctypes.c_int(n_batch), _ptr(out), ctypes.c_int(_code(out.dtype)), ctypes.c_long(out_ld), ctypes.c_long(out_batch),
             ctypes.c_int(n_rows), ctypes.c_int(n), ctypes.c_int(k), ctypes.c_int(tiles_a_block),
@@ -193,23 +194,8 @@ def grouped_linear(rows: torch.Tensor, groups: ExpertGroups, weight: torch.Tenso
     if rows.dim() != 2 or not rows.is_contiguous() or weight.shape[2] != rows.shape[1] or rows.shape[0] != groups.n_tiles * TILE_ROWS:
         raise KernelError("the rows do not fit the list or the experts' weights")
     out = torch.empty((rows.shape[0], weight.shape[1]), dtype=torch.float32, device=rows.device)
-    identity = ExpertGroups(_identity_rows(rows.shape[0], rows.device), groups.pair_row, groups.tile_expert, groups.n_tiles, groups.tiles_a_block, groups.top, groups.used)
-    _grouped(rows, rows.shape[1], 0, identity, weight, None, out, weight.shape[1], 0, rows.shape[0], 1)
+    _grouped(rows, rows.shape[1], 0, groups, weight, None, out, weight.shape[1], 0, rows.shape[0], 1, gather=False)
     return out
-
-
-_identity: dict = {}
-
-
-def _identity_rows(n: int, device: torch.device) -> torch.Tensor:
-    """0..n-1 as int32 on the device (kept: the same list serves every step of that many rows)."""
-    key = (device, n)
-    t = _identity.get(key)
-    if t is None:
-        if len(_identity) > 64:
-            _identity.clear()
-        t = _identity[key] = torch.arange(n, dtype=torch.int32, device=device)
-    return t
 
 
 def combine_routed(rows: torch.Tensor, groups: ExpertGroups, weights: torch.Tensor) -> torch.Tensor:

@@ -84,3 +84,36 @@ def test_lists_that_lie_elsewhere(n_tokens):
         assert torch.equal(ops.grouped_gate_up(x, lists, gate, up)[groups.pair_row.long()], want)
     with pytest.raises(ops.KernelError):
         ops.grouped_gate_up(x, dataclasses.replace(groups, tile_expert=groups.tile_expert[:-1]), gate, up)
+
+
+@pytest.mark.parametrize("dtype,n_tokens", [(torch.bfloat16, 8), (torch.bfloat16, 96), (torch.float32, 8)])
+def test_a_captured_product_reads_nothing_that_other_sizes_replace(dtype, n_tokens):
+    """Lists of many other sizes come between a capture and its replays, as prompts do between decode steps."""
+    from cwm_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(n_tokens)
+    normal = lambda *shape: torch.randn(shape, generator=g, device=DEV)  # noqa: E731
+    x, chosen = normal(n_tokens, 64).to(dtype), normal(n_tokens, 8).topk(2).indices.int().contiguous()
+    gate, up, down = (normal(8, *s).mul(0.1).to(dtype) for s in ((96, 64), (96, 64), (64, 96)))
+
+    def step(tokens, picks):
+        groups = ops.group_by_expert(picks, 8)
+        return ops.grouped_linear(ops.grouped_gate_up(tokens, groups, gate, up), groups, down)[groups.pair_row.long()]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(x, chosen)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step(x, chosen)
+    for turn in range(3):
+        for n in range(40 * turn + 9, 40 * turn + 49):  # 80 and more different lists
+            more = normal(4 * n, 64).to(dtype)
+            step(more, normal(4 * n, 8).topk(2).indices.int().contiguous())
+        taken = [torch.full((size,), 1 << 20, dtype=torch.int32, device=DEV) for size in range(128, 4096, 16)]  # what was freed, if anything was
+        x.copy_(normal(n_tokens, 64))
+        graph.replay()
+        assert torch.equal(out, step(x, chosen)), turn
+        del taken
