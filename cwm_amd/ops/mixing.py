@@ -6,6 +6,7 @@ Shapes, types and devices are checked on the host; there is no CPU path."""
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Any, Optional, Sequence, Tuple
 
 import torch
@@ -22,6 +23,7 @@ MAX_SIDE_ADDENDS = 4  # csrc/token_side.hip: SIDE_MAX_ADDENDS
 SIDE_TILE_FROM = 256  # csrc/token_side.hip: SIDE_TILE_FROM
 
 
+@functools.cache  # an import statement costs a launch-bound step a microsecond and more a call
 def _base():
     from . import KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream  # the shared helpers of this package
 

@@ -5,6 +5,7 @@ devices are checked on the host; there is no CPU path."""
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Any, Optional, Tuple
 
 import torch
@@ -15,6 +16,7 @@ MAX_CONV_QK_TAPS = 16  # csrc/conv_qk.hip: CONVQK_MAX_TAPS
 MAX_CONV_QK_CHANNELS = 60 * 1024 // 4  # csrc/conv_qk.hip: CONVQK_MAX_LDS
 
 
+@functools.cache  # an import statement costs a launch-bound step a microsecond and more a call
 def _base():
     from . import KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream  # the shared helpers of this package
 

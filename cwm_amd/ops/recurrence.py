@@ -7,6 +7,7 @@ no CPU path."""
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Any, Optional, Sequence, Tuple
 
 import torch
@@ -22,6 +23,7 @@ MIN_GRU_SEGMENT = 16  # tokens of a segment at least
 MIN_GRU_SEGMENTS = 128  # and segments of a portion at most
 
 
+@functools.cache  # an import statement costs a launch-bound step a microsecond and more a call
 def _base():
     from . import KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream  # the shared helpers of this package
 

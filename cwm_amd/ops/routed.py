@@ -4,6 +4,7 @@ in which every head has a weight matrix of its own."""
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 from typing import Optional, Tuple
 
@@ -23,6 +24,7 @@ STREAM_ROWS = 3  # up to so many rows an expert, gate and up go to the kernel th
 # of 2,048 x 1,024), 102 instead of 115 us (3,072 x 1,536, 32 experts); at 4 rows 35 and 33 us, 134 and 124 us
 
 
+@functools.cache  # an import statement costs a launch-bound step a microsecond and more a call
 def _base():
     from . import KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream
 

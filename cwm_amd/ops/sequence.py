@@ -5,6 +5,7 @@ the host; there is no CPU path."""
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Any, Optional
 
 import torch
@@ -15,6 +16,7 @@ MAX_CONV_TAPS = 8  # csrc/state_space.hip: CONV_MAX_TAPS
 MAX_SSM_STATE = 256  # csrc/state_space.hip: SCAN_ROWS * 16
 
 
+@functools.cache  # an import statement costs a launch-bound step a microsecond and more a call
 def _base():
     from . import KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream  # the shared helpers of this package
 

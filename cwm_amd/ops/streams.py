@@ -6,6 +6,7 @@ the host; there is no CPU path."""
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 from typing import Any, Optional, Tuple, Union
 
@@ -17,6 +18,7 @@ MAX_STREAMS = 8  # csrc/streams.hip: STREAMS_MAX
 ACTIVATIONS = {"relu2": 0, "relu": 1, "gelu_tanh": 2, "silu": 3, "gelu_erf": 4, "tanh": 5}  # csrc/rowwise.hip: act_value
 
 
+@functools.cache  # an import statement costs a launch-bound step a microsecond and more a call
 def _base():
     from . import KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream  # the shared helpers of this package
 
