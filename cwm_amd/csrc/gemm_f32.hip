@@ -298,20 +298,25 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
     step(1, k0 + 3 * SPLIT_STEP);
   }
   if (k0 < K) step(0, K);
-  // eight neighbouring threads have a row's pieces
-  bool any = false;
-  auto mark = [&](float largest, unsigned char* marks, int f) {
+  float largest = 0.f;
 #pragma unroll
-    for (int off = 1; off < 8; off <<= 1) largest = fmaxf(largest, __shfl_xor(largest, off, CWM_WAVE));
-    const bool beyond = !(largest < SPLIT_LIMIT);
-    any |= beyond;
-    if ((f & 7) == 0) marks[f / 8] = beyond;
-  };
+  for (int i = 0; i < A_LOADS; ++i) largest = fmaxf(largest, largest_a[i]);
 #pragma unroll
-  for (int i = 0; i < A_LOADS; ++i) mark(largest_a[i], marked_rows, tid + i * THREADS);
+  for (int i = 0; i < W_LOADS; ++i) largest = fmaxf(largest, largest_w[i]);
+  const bool any = __syncthreads_or(!(largest < SPLIT_LIMIT));
+  if (any) {
+    // eight neighbouring threads have a row's pieces
+    auto mark = [&](float largest, unsigned char* marks, int f) {
 #pragma unroll
-  for (int i = 0; i < W_LOADS; ++i) mark(largest_w[i], marked_columns, tid + i * THREADS);
-  any = __syncthreads_or(any);
+      for (int off = 1; off < 8; off <<= 1) largest = fmaxf(largest, __shfl_xor(largest, off, CWM_WAVE));
+      if ((f & 7) == 0) marks[f / 8] = !(largest < SPLIT_LIMIT);
+    };
+#pragma unroll
+    for (int i = 0; i < A_LOADS; ++i) mark(largest_a[i], marked_rows, tid + i * THREADS);
+#pragma unroll
+    for (int i = 0; i < W_LOADS; ++i) mark(largest_w[i], marked_columns, tid + i * THREADS);
+    __syncthreads();
+  }
   // lane 16 j + r of a tile holds row r, columns 4 j + i
 #pragma unroll
   for (int b = 0; b < TN; ++b)
