@@ -82,14 +82,14 @@ template <> struct SideVec<float> {
 // TOK tokens a block: the two matrices are read once for all of them.  The gate's rows are dealt to the block's
 // wavefronts, which read them 16 bytes a lane; every sum runs in one order whatever TOK is.
 template <typename TW, int TOK>
-__global__ void __launch_bounds__(SIDE_THREADS)
-token_side_kernel(float* __restrict__ h, const int* __restrict__ tokens, const TW* __restrict__ table, long table_ld,
+__device__ __forceinline__ void
+token_side_rows(const int block, float* __restrict__ h, const int* __restrict__ tokens, const TW* __restrict__ table, long table_ld,
                   int column0, const TW* __restrict__ w_gate, const TW* __restrict__ w_proj_t, const float* __restrict__ weight,
                   int n_tokens, int dim, int side_dim, int vocab, float eps, bool round_inputs, SideAddends addends, SidePortions portions) {
   extern __shared__ __attribute__((aligned(16))) float rows[];  // [TOK][dim], then the gated values [TOK][side_dim]
   __shared__ float scratch[16];
   float* gated = rows + (size_t)TOK * dim;
-  const int t0 = blockIdx.x * TOK;
+  const int t0 = block * TOK;
   bool mine[TOK], any = false;
 #pragma unroll
   for (int tok = 0; tok < TOK; ++tok) any |= mine[tok] = portions.serves(t0 + tok, n_tokens, false);
@@ -205,6 +205,15 @@ token_side_kernel(float* __restrict__ h, const int* __restrict__ tokens, const T
   }
 }
 
+template <typename TW, int TOK>
+__global__ void __launch_bounds__(SIDE_THREADS)
+token_side_kernel(float* __restrict__ h, const int* __restrict__ tokens, const TW* __restrict__ table, long table_ld,
+                  int column0, const TW* __restrict__ w_gate, const TW* __restrict__ w_proj_t, const float* __restrict__ weight,
+                  int n_tokens, int dim, int side_dim, int vocab, float eps, bool round_inputs, SideAddends addends, SidePortions portions) {
+  token_side_rows<TW, TOK>(blockIdx.x, h, tokens, table, table_ld, column0, w_gate, w_proj_t, weight, n_tokens, dim, side_dim, vocab, eps, round_inputs,
+                           addends, portions);
+}
+
 // The same for bfloat16 weights whose inputs are rounded, on the matrix cores: TOK tokens a block of sixteen wavefronts.  The
 // gate's product (16 tokens x side_dim, K = dim) is split over the wavefronts by columns and K, whose parts meet in LDS; the
 // projection's (16 x dim, K = side_dim) by columns.  Both weights are read as they lie, 16 bytes a lane, once a block: w_proj
@@ -217,8 +226,8 @@ token_side_kernel(float* __restrict__ h, const int* __restrict__ tokens, const T
 #define SIDE_TILE_MAX 128
 
 template <int TOK, int MAXT>
-__global__ void __launch_bounds__(SIDE_THREADS)
-token_side_tile_kernel(float* __restrict__ h, const int* __restrict__ tokens, const bf16_t* __restrict__ table, long table_ld, int column0,
+__device__ __forceinline__ void
+token_side_tile(const int block, float* __restrict__ h, const int* __restrict__ tokens, const bf16_t* __restrict__ table, long table_ld, int column0,
                        const bf16_t* __restrict__ w_gate, const bf16_t* __restrict__ w_proj, const float* __restrict__ weight, int n_tokens,
                        int dim, int side_dim, int vocab, float eps, SideAddends addends, SidePortions portions) {
   extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
@@ -229,7 +238,7 @@ token_side_tile_kernel(float* __restrict__ h, const int* __restrict__ tokens, co
   bf16_t* gated = (bf16_t*)(parts + WAVES * 16 * TOK);           // [TOK][SIDE_TILE_MAX + 8]
   float* squares = (float*)(gated + TOK * (SIDE_TILE_MAX + 8));  // [WAVES][TOK]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, j = lane >> 4;
-  const int t0 = blockIdx.x * TOK;
+  const int t0 = block * TOK;
   bool any = false;
 #pragma unroll
   for (int tok = 0; tok < TOK; ++tok) any |= portions.serves(t0 + tok, n_tokens, true);
@@ -337,18 +346,43 @@ token_side_tile_kernel(float* __restrict__ h, const int* __restrict__ tokens, co
   }
 }
 
+template <int TOK, int MAXT>
+__global__ void __launch_bounds__(SIDE_THREADS)
+token_side_tile_kernel(float* __restrict__ h, const int* __restrict__ tokens, const bf16_t* __restrict__ table, long table_ld, int column0,
+                       const bf16_t* __restrict__ w_gate, const bf16_t* __restrict__ w_proj, const float* __restrict__ weight, int n_tokens,
+                       int dim, int side_dim, int vocab, float eps, SideAddends addends, SidePortions portions) {
+  token_side_tile<TOK, MAXT>(blockIdx.x, h, tokens, table, table_ld, column0, w_gate, w_proj, weight, n_tokens, dim, side_dim, vocab, eps, addends, portions);
+}
+
+// Both in one launch, for a step whose short portions hold few tokens: the first `tile_blocks` blocks take the long portions' tokens,
+// then a block a token the short ones', beside them and not behind them.  1,006 and 48 tokens of width 3,072: 52 us, as the
+// tiles alone; a second launch of four tokens a block took 63 more.
+#define SIDE_FEW 128
+template <int TOK, int MAXT>
+__global__ void __launch_bounds__(SIDE_THREADS)
+token_side_both_kernel(float* __restrict__ h, const int* __restrict__ tokens, const bf16_t* __restrict__ table, long table_ld, int column0,
+                       const bf16_t* __restrict__ w_gate, const bf16_t* __restrict__ w_proj, const bf16_t* __restrict__ w_proj_t,
+                       const float* __restrict__ weight, int n_tokens, int dim, int side_dim, int vocab, float eps, SideAddends addends,
+                       SidePortions portions, int tile_blocks) {
+  if ((int)blockIdx.x < tile_blocks)
+    token_side_tile<TOK, MAXT>(blockIdx.x, h, tokens, table, table_ld, column0, w_gate, w_proj, weight, n_tokens, dim, side_dim, vocab, eps, addends, portions);
+  else
+    token_side_rows<bf16_t, 1>(blockIdx.x - tile_blocks, h, tokens, table, table_ld, column0, w_gate, w_proj_t, weight, n_tokens, dim, side_dim, vocab, eps,
+                               true, addends, portions);
+}
+
 // h: float32 [T, dim], changed in place.  Addend a (n_addends of them, or none): ptrs[a] of dtypes[a], rows lds[a]
 // elements apart, n_partials[a] slabs partial_strides[a] elements apart, times scales[a]; they are added to h first.
 // tokens: int32 [T].  table: [vocab, >= column0 + side_dim] of `w_dtype`, rows
 // table_ld apart; w_gate [side_dim, dim] and w_proj_t [side_dim, dim] (the projection transposed) of `w_dtype`, contiguous;
 // w_proj: the projection as [dim, side_dim], or null (then the matrix cores are not used);
 // weight: float32 [dim].  seq_of_token, cu_q: the step's portions where some have SIDE_TILE_FROM tokens and more and some fewer,
-// null where all tokens are one kind (then n_tokens stands for the portion).
+// null where all tokens are one kind (then n_tokens stands for the portion); n_few: the tokens of the shorter ones.
 extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, long table_ld, int column0, const void* w_gate,
                               const void* w_proj_t, const void* w_proj, int w_dtype, const float* weight, int n_tokens, int dim, int side_dim, int vocab,
                               float eps, int round_inputs, int n_addends, const void* const* ptrs, const int* dtypes,
                               const long* lds_, const int* n_partials, const long* partial_strides, const float* scales,
-                              const int* seq_of_token, const int* cu_q, hipStream_t stream) {
+                              const int* seq_of_token, const int* cu_q, int n_few, hipStream_t stream) {
   CWM_REQUIRE(n_tokens >= 0 && vocab >= 1 && column0 >= 0, "token_side: bad sizes");
   CWM_REQUIRE(dim >= 1 && dim <= SIDE_MAX_WIDTH, "token_side: rows of %d elements are outside 1..%d", dim, SIDE_MAX_WIDTH);
   CWM_REQUIRE(side_dim >= 1 && side_dim <= SIDE_MAX_DIM, "token_side: %d side values are outside 1..%d", side_dim, SIDE_MAX_DIM);
@@ -374,13 +408,22 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
   if (tiled) {
     // sixteen tokens a block where that leaves no compute unit without one, else eight
     const int tok = n_tokens >= 16 * 256 ? 16 : 8;
-    const size_t lds = (size_t)tok * (dim + 8) * 2 + 16 * 16 * tok * sizeof(float) + (size_t)tok * (SIDE_TILE_MAX + 8) * 2 + 16 * tok * sizeof(float);
+    const size_t lds_tile = (size_t)tok * (dim + 8) * 2 + 16 * 16 * tok * sizeof(float) + (size_t)tok * (SIDE_TILE_MAX + 8) * 2 + 16 * tok * sizeof(float);
+    const bool both = seq_of_token && n_few < SIDE_FEW;
+    const size_t lds_row = sizeof(float) * ((size_t)dim + side_dim), lds = both && lds_row > lds_tile ? lds_row : lds_tile;
+    const int tile_blocks = (n_tokens + tok - 1) / tok;
 #define CWM_SIDE_TILE(TOK, MAXT)                                                                                                           \
   do {                                                                                                                                     \
-    if (lds > 65536) (void)hipFuncSetAttribute((const void*)token_side_tile_kernel<TOK, MAXT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-    hipLaunchKernelGGL((token_side_tile_kernel<TOK, MAXT>), dim3((n_tokens + TOK - 1) / TOK), dim3(SIDE_THREADS), lds, stream, h, tokens,   \
-                       (const bf16_t*)table, table_ld, column0, (const bf16_t*)w_gate, (const bf16_t*)w_proj, weight, n_tokens, dim,        \
-                       side_dim, vocab, eps, ad, portions);                                                                                \
+    const void* kernel = both ? (const void*)token_side_both_kernel<TOK, MAXT> : (const void*)token_side_tile_kernel<TOK, MAXT>;           \
+    if (lds > 65536) (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                              \
+    if (both)                                                                                                                              \
+      hipLaunchKernelGGL((token_side_both_kernel<TOK, MAXT>), dim3(tile_blocks + n_tokens), dim3(SIDE_THREADS), lds, stream, h, tokens,     \
+                         (const bf16_t*)table, table_ld, column0, (const bf16_t*)w_gate, (const bf16_t*)w_proj, (const bf16_t*)w_proj_t,    \
+                         weight, n_tokens, dim, side_dim, vocab, eps, ad, portions, tile_blocks);                                          \
+    else                                                                                                                                   \
+      hipLaunchKernelGGL((token_side_tile_kernel<TOK, MAXT>), dim3(tile_blocks), dim3(SIDE_THREADS), lds, stream, h, tokens,                \
+                         (const bf16_t*)table, table_ld, column0, (const bf16_t*)w_gate, (const bf16_t*)w_proj, weight, n_tokens, dim,      \
+                         side_dim, vocab, eps, ad, portions);                                                                              \
   } while (0)
     if (tok == 16) {
       if (dim <= 2048) CWM_SIDE_TILE(16, 8); else CWM_SIDE_TILE(16, 16);
@@ -388,11 +431,12 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
       if (dim <= 2048) CWM_SIDE_TILE(8, 8); else CWM_SIDE_TILE(8, 16);
     }
 #undef CWM_SIDE_TILE
-    if (!seq_of_token) return cwm_launch_status("token_side");
+    if (!seq_of_token || both) return cwm_launch_status("token_side");
   }
   // tokens a block: as many (4, 2, 1) as fit the LDS and still leave the chip a block a few tokens
+  const int served = tiled ? n_few : n_tokens;
   int tok = 4;
-  while (tok > 1 && (sizeof(float) * (size_t)tok * (dim + side_dim) > SIDE_LDS_LIMIT || n_tokens < 64 * tok)) tok /= 2;
+  while (tok > 1 && (sizeof(float) * (size_t)tok * (dim + side_dim) > SIDE_LDS_LIMIT || served < 64 * tok)) tok /= 2;
   CWM_REQUIRE(sizeof(float) * ((size_t)dim + side_dim) <= SIDE_LDS_LIMIT, "token_side: a row of %d and %d side values do not fit the LDS", dim, side_dim);
   const size_t lds = sizeof(float) * (size_t)tok * (dim + side_dim);
   const int blocks = (n_tokens + tok - 1) / tok;

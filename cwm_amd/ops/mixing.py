@@ -440,12 +440,12 @@ def token_side(
                 raise KernelError(f"an addend {tuple(t.shape)} does not match the residual stream {tuple(h.shape)}")
             partials[i], strides[i], lds[i] = 1, 0, (t.stride(0) if n_tokens > 1 else dim)
         ptrs[i], dtypes[i], scales[i] = t.data_ptr(), _code(t.dtype), c
-    seq_of_token = cu_q = None
+    seq_of_token, cu_q, n_few = None, None, 0
     if w_proj is not None and batch is not None:
         if max(batch.q_lens, default=0) < SIDE_TILE_FROM:
             w_proj = None
         elif any(0 < q < SIDE_TILE_FROM for q in batch.q_lens):  # both kinds
-            seq_of_token, cu_q = batch.seq_of_token, batch.cu_q
+            seq_of_token, cu_q, n_few = batch.seq_of_token, batch.cu_q, sum(q for q in batch.q_lens if q < SIDE_TILE_FROM)
             _i32(seq_of_token, "seq_of_token")
             _i32(cu_q, "cu_q")
             if seq_of_token.numel() != n_tokens:
@@ -457,7 +457,7 @@ def token_side(
             _ptr(h), _ptr(tokens), _ptr(table), ctypes.c_long(table.stride(0)), ctypes.c_int(column0), _ptr(w_gate), _ptr(w_proj_t),
             _ptr(w_proj), ctypes.c_int(_code(table.dtype)), _ptr(weight), ctypes.c_int(n_tokens), ctypes.c_int(dim), ctypes.c_int(side_dim),
             ctypes.c_int(table.shape[0]), ctypes.c_float(eps), ctypes.c_int(int(round_inputs)), ctypes.c_int(len(terms)), ptrs, dtypes, lds,
-            partials, strides, scales, _ptr(seq_of_token), _ptr(cu_q), _stream(),
+            partials, strides, scales, _ptr(seq_of_token), _ptr(cu_q), ctypes.c_int(n_few), _stream(),
         ),
     )
 

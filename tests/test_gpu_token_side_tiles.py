@@ -44,13 +44,14 @@ def test_against_float64(n_tokens, dim, side):
         assert float(off.square().mean().sqrt()) <= 2e-3
 
 
-@pytest.mark.parametrize("q_lens", [[3, 300, 1], [1] * 260 + [256], [257, 255], [1] * 300, [400, 260], [17, 4100, 0, 2]])
-def test_a_portions_bits_do_not_depend_on_the_step(q_lens):
+@pytest.mark.parametrize("q_lens", [[3, 300, 1], [1] * 260 + [256], [127, 256], [128, 256], [257, 255], [1] * 300, [400, 260], [17, 4100, 0, 2]])
+@pytest.mark.parametrize("dim", [192, 2112])
+def test_a_portions_bits_do_not_depend_on_the_step(q_lens, dim):
     from cwm_amd import ops
 
     g = torch.Generator(device=DEV).manual_seed(sum(q_lens))
     normal = lambda *shape: torch.randn(shape, generator=g, device=DEV)  # noqa: E731
-    dim, side, vocab, n = 192, 64, 61, sum(q_lens)
+    side, vocab, n = 64, 61, sum(q_lens)
     h, tokens = normal(n, dim), torch.randint(vocab, (n,), generator=g, device=DEV, dtype=torch.int32)
     gate, proj, table = normal(side, dim).mul(dim ** -0.5).bfloat16(), normal(dim, side).bfloat16(), normal(vocab, side).bfloat16()
     args = (table, 0, gate, proj.t().contiguous(), normal(dim).abs() + 0.3, 1e-6, True)
