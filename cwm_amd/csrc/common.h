@@ -59,6 +59,33 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// Four adjacent elements (or one) of a row kept as n partial sums `stride` elements apart, added in their order to v.  Four
+// loads are under way at a time: each takes about a microsecond where another XCD has just written the sums, and a loop of a
+// load and its addition waits for every one of them.  What lies past the last is the last again and not added.
+__device__ __forceinline__ void add_slabs4(const float* __restrict__ p, int n, long stride, float (&v)[4]) {
+  for (int s = 0; s < n; s += 4) {
+    float4 z[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) z[u] = *(const float4*)(p + (size_t)min(s + u, n - 1) * stride);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const bool have = s + u < n;
+      v[0] += have ? z[u].x : 0.f, v[1] += have ? z[u].y : 0.f, v[2] += have ? z[u].z : 0.f, v[3] += have ? z[u].w : 0.f;
+    }
+  }
+}
+__device__ __forceinline__ float add_slabs(const float* __restrict__ p, int n, long stride) {
+  float v = 0.f;
+  for (int s = 0; s < n; s += 4) {
+    float z[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) z[u] = p[(size_t)min(s + u, n - 1) * stride];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v += s + u < n ? z[u] : 0.f;
+  }
+  return v;
+}
+
 // Sine and cosine of position * freq.  The product is exact (float64) and its whole turns are taken off before it is
 // rounded, so a far position is as exact as a near one (a float32 product of some hundred radians is off by up to 3e-5).
 __device__ __forceinline__ void sincos_turn(int position, float freq, float* s, float* c) {

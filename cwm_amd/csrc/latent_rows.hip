@@ -41,9 +41,8 @@ latent_rows_kernel(const TS* __restrict__ q_src, long q_stride, int q_partials, 
   if (kv_src && blockIdx.y == 0) {
     const TS* src = kv_src + (size_t)t * kv_stride;
     auto value = [&](int e) {
-      float v = 0.f;
-      for (int p = 0; p < kv_partials; ++p) v += Elem<TS>::load(src + (size_t)p * kv_partial_stride + e);
-      return v;
+      if constexpr (sizeof(TS) == 4) return add_slabs((const float*)src + e, kv_partials, kv_partial_stride);
+      else return Elem<TS>::load(src + e);  // partial sums are float32
     };
     float ss = 0.f;
     for (int e = threadIdx.x; e < rank; e += blockDim.x) {
@@ -77,9 +76,8 @@ latent_rows_kernel(const TS* __restrict__ q_src, long q_stride, int q_partials, 
   const TS* src = q_src + (size_t)t * q_stride;
   const int width = lead + n_rest;
   auto value = [&](int e) {
-    float v = 0.f;
-    for (int p = 0; p < q_partials; ++p) v += Elem<TS>::load(src + (size_t)p * q_partial_stride + e);
-    return v;
+    if constexpr (sizeof(TS) == 4) return add_slabs((const float*)src + e, q_partials, q_partial_stride);
+    else return Elem<TS>::load(src + e);
   };
   const int first = blockIdx.y * blockDim.x + threadIdx.x, step = gridDim.y * blockDim.x;
   const int half = lead / 2;

@@ -62,7 +62,7 @@ template <> struct LnStore<bf16_t> {
 
 // VEC: D is a multiple of 4 and every pointer and row start is 16-byte aligned (8 for bfloat16 rows).
 template <typename TO, bool VEC>
-__global__ void __launch_bounds__(LN_THREADS)
+__global__ void __launch_bounds__(1024)
 add_layernorm_kernel(float* __restrict__ h, LnAddends addends, const float* __restrict__ w1, const float* __restrict__ b1,
                      TO* __restrict__ out1, const float* __restrict__ w2, const float* __restrict__ b2, TO* __restrict__ out2,
                      const int* __restrict__ rows, int dim, float eps) {
@@ -73,7 +73,7 @@ add_layernorm_kernel(float* __restrict__ h, LnAddends addends, const float* __re
   float* hrow = h + t * dim;
   float sum = 0.f;
   if constexpr (VEC) {
-    for (int e = 4 * threadIdx.x; e < dim; e += 4 * LN_THREADS) {
+    for (int e = 4 * threadIdx.x; e < dim; e += 4 * blockDim.x) {
       float x[4];
       ln_load4(hrow, CWM_F32, e, x);
       for (int a = 0; a < addends.n; ++a) {
@@ -82,27 +82,23 @@ add_layernorm_kernel(float* __restrict__ h, LnAddends addends, const float* __re
         if (ad.n_partials == 1) {
           ln_load4(ad.ptr, ad.dtype, t * ad.ld + e, y);
         } else {
-          // four partial sums in flight at a time, added in their order; what lies beyond the last is the last again, times zero
-          for (int p = 0; p < ad.n_partials; p += 4) {
-            float z[4][4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) ln_load4(ad.ptr, ad.dtype, (size_t)min(p + u, ad.n_partials - 1) * ad.partial_stride + t * ad.ld + e, z[u]);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const float keep = p + u < ad.n_partials ? 1.0f : 0.0f;
-              y[0] = fmaf(keep, z[u][0], y[0]), y[1] = fmaf(keep, z[u][1], y[1]), y[2] = fmaf(keep, z[u][2], y[2]), y[3] = fmaf(keep, z[u][3], y[3]);
-            }
-          }
+          add_slabs4((const float*)ad.ptr + t * ad.ld + e, ad.n_partials, ad.partial_stride, y);
         }
         x[0] = fmaf(ad.scale, y[0], x[0]), x[1] = fmaf(ad.scale, y[1], x[1]);
         x[2] = fmaf(ad.scale, y[2], x[2]), x[3] = fmaf(ad.scale, y[3], x[3]);
       }
       if (!rows && addends.n > 0) *(float4*)(hrow + e) = make_float4(x[0], x[1], x[2], x[3]);
       *(float4*)(row + e) = make_float4(x[0], x[1], x[2], x[3]);
-      sum += (x[0] + x[1]) + (x[2] + x[3]);
     }
+    // the sums are LN_THREADS threads' whatever the block has, each of the elements 4 thread, 4 (thread + LN_THREADS), ...
+    __syncthreads();
+    if (threadIdx.x < LN_THREADS)
+      for (int e = 4 * threadIdx.x; e < dim; e += 4 * LN_THREADS) {
+        const float4 x = *(const float4*)(row + e);
+        sum += (x.x + x.y) + (x.z + x.w);
+      }
   } else {
-    for (int e = threadIdx.x; e < dim; e += LN_THREADS) {
+    for (int e = threadIdx.x; e < dim; e += blockDim.x) {
       float x = hrow[e];
       for (int a = 0; a < addends.n; ++a) {
         const LnAddend& ad = addends.a[a];
@@ -117,23 +113,23 @@ add_layernorm_kernel(float* __restrict__ h, LnAddends addends, const float* __re
   }
   if (!out1 && !out2) return;  // only the sum was wanted
   const float mean = block_sum(sum, scratch) / (float)dim;
-  // every thread reads back what it wrote itself: no barrier is needed before this pass
   float sq = 0.f;
   if constexpr (VEC) {
-    for (int e = 4 * threadIdx.x; e < dim; e += 4 * LN_THREADS) {
-      const float4 x = *(const float4*)(row + e);
-      const float d0 = x.x - mean, d1 = x.y - mean, d2 = x.z - mean, d3 = x.w - mean;
-      sq += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
-    }
+    if (threadIdx.x < LN_THREADS)
+      for (int e = 4 * threadIdx.x; e < dim; e += 4 * LN_THREADS) {
+        const float4 x = *(const float4*)(row + e);
+        const float d0 = x.x - mean, d1 = x.y - mean, d2 = x.z - mean, d3 = x.w - mean;
+        sq += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
+      }
   } else {
-    for (int e = threadIdx.x; e < dim; e += LN_THREADS) {
+    for (int e = threadIdx.x; e < dim; e += blockDim.x) {
       const float d = row[e] - mean;
       sq += d * d;
     }
   }
   const float rstd = 1.0f / sqrtf(block_sum(sq, scratch) / (float)dim + eps);
   if constexpr (VEC) {
-    for (int e = 4 * threadIdx.x; e < dim; e += 4 * LN_THREADS) {
+    for (int e = 4 * threadIdx.x; e < dim; e += 4 * blockDim.x) {
       const float4 x = *(const float4*)(row + e);
       const float n[4] = {(x.x - mean) * rstd, (x.y - mean) * rstd, (x.z - mean) * rstd, (x.w - mean) * rstd};
       if (out1) {
@@ -148,7 +144,7 @@ add_layernorm_kernel(float* __restrict__ h, LnAddends addends, const float* __re
       }
     }
   } else {
-    for (int e = threadIdx.x; e < dim; e += LN_THREADS) {
+    for (int e = threadIdx.x; e < dim; e += blockDim.x) {
       const float n = (row[e] - mean) * rstd;
       if (out1) Elem<TO>::store(out1 + (size_t)r * dim + e, fmaf(n, w1[e], b1[e]));
       if (out2) Elem<TO>::store(out2 + (size_t)r * dim + e, fmaf(n, w2[e], b2[e]));
@@ -183,8 +179,11 @@ extern "C" int cwm_add_layernorm(float* h, int n_addends, const void* const* ptr
   vec = vec && ((uintptr_t)out1 % (4 * out_bytes)) == 0 && ((uintptr_t)out2 % (4 * out_bytes)) == 0;
   vec = vec && ((uintptr_t)w1 % 16) == 0 && ((uintptr_t)b1 % 16) == 0 && ((uintptr_t)w2 % 16) == 0 && ((uintptr_t)b2 % 16) == 0;
   const size_t lds_bytes = (size_t)dim * sizeof(float);
+  // few rows of up to 4,096 elements: four a thread, so that all loads of a row are under way at once; many rows overlap one
+  // another's loads anyway, and narrow blocks fill a compute unit better.  The sums are the same threads' either way.
+  const int threads = vec && n_out < 512 && dim > 1024 && dim <= 4096 ? (dim / 4 + 63) / 64 * 64 : LN_THREADS;
 #define CWM_LN(TO, VEC)                                                                                                    \
-  hipLaunchKernelGGL((add_layernorm_kernel<TO, VEC>), dim3(n_out), dim3(LN_THREADS), lds_bytes, stream, h, ad, w1, b1,       \
+  hipLaunchKernelGGL((add_layernorm_kernel<TO, VEC>), dim3(n_out), dim3(threads), lds_bytes, stream, h, ad, w1, b1,       \
                      (TO*)out1, w2, b2, (TO*)out2, rows, dim, eps)
   if (out_dtype == CWM_F32) {
     if (vec) CWM_LN(float, true); else CWM_LN(float, false);

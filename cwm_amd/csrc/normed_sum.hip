@@ -253,8 +253,9 @@ extern "C" int cwm_normed_sum(float* h, int n_addends, const void* const* ptrs, 
     vec = vec && lds[a] % 4 == 0 && partial_strides[a] % 4 == 0 && ((uintptr_t)ptrs[a] % (4 * bytes)) == 0 && ((uintptr_t)weights[a] % 16) == 0;
   }
   const int n_chunks = dim / 4;
-  int threads = 64;
-  while (threads < 512 && threads * 2 < n_chunks) threads *= 2;
+  // rows of up to 4,096 elements: four a thread, so that all loads of a row are under way at once (the loops over the partial
+  // sums and the chosen rows keep a thread's next chunk waiting)
+  const int threads = n_chunks <= 1024 ? (n_chunks > 64 ? (n_chunks + 63) / 64 * 64 : 64) : 512;
   const int chunks = (n_chunks + threads - 1) / threads;
 #define CWM_NSUM_REGS(TO, N, C) \
   hipLaunchKernelGGL((normed_sum_regs_kernel<TO, N, C>), dim3(n_out), dim3(threads), 0, stream, h, ad, weight, (TO*)out, rows, dim, eps)

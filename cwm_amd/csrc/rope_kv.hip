@@ -315,7 +315,7 @@ template <> struct Four<bf16_t> {
 // VEC: every size is a multiple of 4 and every row starts at a multiple of 16 bytes (8 for bfloat16): a thread
 // takes four consecutive elements, two pairs, at a time.
 template <typename TS, typename TO, bool VEC>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(1024)
 qk_norm_rope_write_kernel(const TS* __restrict__ src, long src_stride, int n_partials, long partial_stride,
                           TO* __restrict__ q_out, const float* __restrict__ q_weight, const float* __restrict__ k_weight,
                           float eps, const int* __restrict__ positions, const int* __restrict__ seq_of_token,
@@ -336,7 +336,10 @@ qk_norm_rope_write_kernel(const TS* __restrict__ src, long src_stride, int n_par
   };
   auto value4 = [&](int e, float (&v)[4]) {
     v[0] = v[1] = v[2] = v[3] = 0.f;
-    for (int p = 0; p < n_partials; ++p) Four<TS>::add(srow + (size_t)p * partial_stride + e, v);
+    if constexpr (sizeof(TS) == 4)
+      add_slabs4((const float*)srow + e, n_partials, partial_stride, v);
+    else
+      Four<TS>::add(srow + e, v);  // partial sums are float32
   };
   TO* kdst = nullptr;
   TO* vdst = nullptr;
@@ -366,17 +369,27 @@ qk_norm_rope_write_kernel(const TS* __restrict__ src, long src_stride, int n_par
     float sq = 0.f, sk = 0.f;
     const int first = q_weight ? 0 : q_width, last = norm_k ? q_width + k_width : q_width;
     if constexpr (VEC) {
-      for (int e = first + 4 * threadIdx.x; e < last; e += 4 * blockDim.x) {
-        float v[4];
-        value4(e, v);
-        const float ss = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
-        if (e < q_width) sq += ss; else sk += ss;
+      // the pieces' sums in LDS, then added by 256 threads, each those of the pieces thread, thread + 256, ...
+      __shared__ float piece[1024];
+      for (int base = first; base < last; base += 4 * 1024) {
+        const int here = min(1024, (last - base) / 4);
+        __syncthreads();
+        for (int i = threadIdx.x; i < here; i += blockDim.x) {
+          float v[4];
+          value4(base + 4 * i, v);
+          piece[i] = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+        }
+        __syncthreads();
+        if (threadIdx.x < 256)
+          for (int i = threadIdx.x; i < here; i += 256)
+            if (base + 4 * i < q_width) sq += piece[i]; else sk += piece[i];
       }
     } else {
-      for (int e = first + threadIdx.x; e < last; e += blockDim.x) {
-        const float v = value(e);
-        if (e < q_width) sq += v * v; else sk += v * v;
-      }
+      if (threadIdx.x < 256)
+        for (int e = first + threadIdx.x; e < last; e += 256) {
+          const float v = value(e);
+          if (e < q_width) sq += v * v; else sk += v * v;
+        }
     }
     if (q_weight) q_rstd = 1.0f / sqrtf(block_sum(sq, scratch) / (float)q_width + eps);
     if (norm_k) k_rstd = 1.0f / sqrtf(block_sum(sk, scratch) / (float)k_width + eps);
@@ -487,8 +500,11 @@ extern "C" int cwm_qk_norm_rope_write(const void* src, int src_dtype, long src_s
   // few tokens: several blocks a token, so that a decode step's rows are not left to as many blocks
   const int heads = n_q_heads + n_kv_heads;
   const int gy = n_tokens >= 512 ? 1 : (heads < 8 ? heads : 8);
+  // few tokens: four elements of queries and keys a thread where that many fit, so that the sums of squares are one round of
+  // loads; the sums themselves are the same threads' either way
+  const int pieces = (heads * qk_dim + 3) / 4, threads = n_tokens >= 512 || pieces <= 256 ? 256 : pieces >= 1024 ? 1024 : (pieces + 63) / 64 * 64;
 #define CWM_NORM_ROPE_V(TS, TO, VEC)                                                                                       \
-  hipLaunchKernelGGL((qk_norm_rope_write_kernel<TS, TO, VEC>), dim3(n_tokens, gy), dim3(256), 0, stream, (const TS*)src,    \
+  hipLaunchKernelGGL((qk_norm_rope_write_kernel<TS, TO, VEC>), dim3(n_tokens, gy), dim3(threads), 0, stream, (const TS*)src, \
                      src_stride, n_partials, partial_stride, (TO*)q_out, q_weight, k_weight, eps, positions, seq_of_token, \
                      inv_freq, (TO*)cache, block_table, table_width, page_size, num_pages, n_q_heads, n_kv_heads, qk_dim,  \
                      v_dim, head_dim)
@@ -553,7 +569,10 @@ head_norm_rope_write_kernel(const TS* __restrict__ src, long src_stride, int n_p
   };
   auto value4 = [&](int e, float (&v)[4]) {
     v[0] = v[1] = v[2] = v[3] = 0.f;
-    for (int p = 0; p < n_partials; ++p) Four<TS>::add(srow + (size_t)p * partial_stride + e, v);
+    if constexpr (sizeof(TS) == 4)
+      add_slabs4((const float*)srow + e, n_partials, partial_stride, v);
+    else
+      Four<TS>::add(srow + e, v);  // partial sums are float32
     if (bias) {
       const float4 b = *(const float4*)(bias + e);
       v[0] += b.x, v[1] += b.y, v[2] += b.z, v[3] += b.w;

@@ -139,7 +139,7 @@ template <> struct Vec4<bf16_t> {
 };
 
 template <typename TD, typename TW, typename TO, int CHUNKS>
-__global__ void add_rmsnorm_regs_kernel(float* __restrict__ h, const TD* __restrict__ delta, int n_partials,
+__global__ void __launch_bounds__(1024) add_rmsnorm_regs_kernel(float* __restrict__ h, const TD* __restrict__ delta, int n_partials,
                                         long partial_stride, const TW* __restrict__ weight, TO* __restrict__ out,
                                         const int* __restrict__ rows, int dim, float eps) {
   __shared__ float scratch[16];
@@ -211,15 +211,18 @@ static void launch_add_rmsnorm(void* h, const void* delta, int n_partials, long 
   const int n_chunks = dim / 4;
   if (dim % 4 == 0 && n_chunks <= 4 * 512) {
     // all pointers are rows of contiguous tensors whose row length is a multiple of 4: 16-byte aligned loads
-    int threads = 64;
-    while (threads < 512 && threads * 4 < n_chunks) threads *= 2;
+    // Rows of up to 4,096 elements: four elements a thread.  A thread's further chunks would be asked for one after the other
+    // (the loop over the partial sums stands between them), each at the latency of memory that another XCD wrote: 24 rows of
+    // 2,048 with one / four / eight partial sums 2.5 / 2.6 / 2.9 us, with four chunks a thread 3.7 / 4.2 / 5.0; 4,096 rows 16.5 both.
+    // Longer rows: 512 threads, since wider blocks gain little there at few rows (6,144: 3.9 both with four partial sums) and fill
+    // a compute unit worse at many (1,024 rows 13.9 instead of 11.8 us).
+    const int threads = n_chunks <= 1024 ? (n_chunks + 63) / 64 * 64 : 512;
     const int chunks = (n_chunks + threads - 1) / threads;
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(n_out), dim3(threads), 0, stream, (float*)h, (const TD*)delta, n_partials,
                          partial_stride, (const TW*)w, (TO*)out, rows, dim, eps);
     };
     if (chunks <= 1) go(add_rmsnorm_regs_kernel<TD, TW, TO, 1>);
-    else if (chunks <= 2) go(add_rmsnorm_regs_kernel<TD, TW, TO, 2>);
     else if (chunks <= 3) go(add_rmsnorm_regs_kernel<TD, TW, TO, 3>);
     else go(add_rmsnorm_regs_kernel<TD, TW, TO, 4>);
     return;
