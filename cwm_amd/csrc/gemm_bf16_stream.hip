@@ -19,9 +19,10 @@
 //     B operand = A^T    (lane 16*j + r: row r of A, same k)
 //     result lane 16*j + r holds C[r][n0 + 4*j + i], i = 0..3
 //
-// Two shapes of block are built, both of 16 wavefronts: one 16-row tile of A with 12
-// steps of K per wavefront in registers (M <= 16, K up to 6144 without a split), and
-// four tiles of A with 4 steps of K per wavefront (M <= 64, K up to 2048 per split).
+// Three shapes of block are built, all of 16 wavefronts: one 16-row tile of A with 12
+// steps of K per wavefront in registers (M <= 16, K up to 6144 without a split), two
+// tiles with 6 steps (M <= 32, K up to 3072 per split), and four tiles of A with 4 steps
+// of K per wavefront (M <= 64, K up to 2048 per split).
 //
 // Several inputs: the rows of W may belong to several A's of one size, `tiles_per_input` tiles of 16 rows each (the last
 // may have fewer): blocks are dealt out by input, so a block still holds one slice of one A.
@@ -40,6 +41,12 @@ CWM_DEFINE_ERROR_API
 #ifndef ST1_HALF
 #define ST1_HALF 6
 #endif
+#ifndef ST2_WAVES
+#define ST2_WAVES 16
+#endif
+#ifndef ST2_HALF
+#define ST2_HALF 3
+#endif
 #ifndef ST4_WAVES
 #define ST4_WAVES 16
 #endif
@@ -47,8 +54,8 @@ CWM_DEFINE_ERROR_API
 #define ST4_HALF 2
 #endif
 
-extern "C" int cwm_gemm_bf16_stream_steps_per_wave(int m) { return m <= 16 ? 2 * ST1_HALF : 2 * ST4_HALF; }
-extern "C" int cwm_gemm_bf16_stream_waves(int m) { return m <= 16 ? ST1_WAVES : ST4_WAVES; }
+extern "C" int cwm_gemm_bf16_stream_steps_per_wave(int m) { return m <= 16 ? 2 * ST1_HALF : m <= 32 ? 2 * ST2_HALF : 2 * ST4_HALF; }
+extern "C" int cwm_gemm_bf16_stream_waves(int m) { return m <= 16 ? ST1_WAVES : m <= 32 ? ST2_WAVES : ST4_WAVES; }
 
 // What the joined q/k/v projection's epilogue needs to rotate queries and keys and to
 // put the new keys and values into the paged cache (the work of rope_kv.hip, same
@@ -163,7 +170,7 @@ gemm_stream_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restr
     for (int mt = 0; mt < MT; ++mt) *(float4v*)(mine + mt * 256 + r * 16 + 4 * j) = acc[mt];  // [row][column]
     __syncthreads();
     if (ROPE) {
-      if (threadIdx.x < 128) {
+      if (threadIdx.x < MT * 128) {
         // a pair of adjacent columns (2i, 2i + 1) of one row
         const int idx = threadIdx.x * 2;
         float s0 = 0.f, s1 = 0.f;
@@ -281,7 +288,7 @@ extern "C" int cwm_gemm_bf16_stream(const void* A, long lda, const void* W, long
                rope_page_size, rope_num_pages, rope_n_q_heads, rope_n_kv_heads, rope_head_dim};
   const bool rope = rope_positions != nullptr;
   if (rope) {
-    CWM_REQUIRE(k_split == 1 && c_dtype == CWM_BF16 && M <= 16, "gemm_bf16_stream: the q/k/v epilogue needs bfloat16 output and no split");
+    CWM_REQUIRE(k_split == 1 && c_dtype == CWM_BF16 && M <= 32, "gemm_bf16_stream: the q/k/v epilogue needs at most 32 rows, bfloat16 output and no split");
     CWM_REQUIRE(rope_seq_of_token && rope_cache && rope_block_table, "gemm_bf16_stream: cache arguments missing");
     CWM_REQUIRE(rope_head_dim > 0 && rope_head_dim % 2 == 0 && rope_n_q_heads > 0 && rope_n_kv_heads > 0 &&
                     N == (rope_n_q_heads + 2 * rope_n_kv_heads) * rope_head_dim,
@@ -289,14 +296,14 @@ extern "C" int cwm_gemm_bf16_stream(const void* A, long lda, const void* W, long
     CWM_REQUIRE(rope_page_size > 0 && rope_num_pages > 0 && rope_table_width > 0, "gemm_bf16_stream: bad cache geometry");
   }
   if (glu) {
-    CWM_REQUIRE(!rope && k_split == 1 && c_dtype == CWM_BF16 && M <= 16 && N % 16 == 0,
-                "gemm_bf16_stream: the gated epilogue needs at most 16 rows, no split, bfloat16 output and N a multiple of 16");
+    CWM_REQUIRE(!rope && k_split == 1 && c_dtype == CWM_BF16 && M <= 32 && N % 16 == 0,
+                "gemm_bf16_stream: the gated epilogue needs at most 32 rows, no split, bfloat16 output and N a multiple of 16");
     CWM_REQUIRE(2 * ldc >= N, "gemm_bf16_stream: row stride of the gated result shorter than its rows");
   }
   CWM_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_bf16_stream: bad sizes M=%d N=%d K=%d", M, N, K);
   CWM_REQUIRE(M <= 64, "gemm_bf16_stream: M=%d is more than 64 rows", M);
-  const int ST_WAVES = M <= 16 ? ST1_WAVES : ST4_WAVES;
-  const int ST_HALF = M <= 16 ? ST1_HALF : ST4_HALF;
+  const int ST_WAVES = cwm_gemm_bf16_stream_waves(M);
+  const int ST_HALF = cwm_gemm_bf16_stream_steps_per_wave(M) / 2;
   CWM_REQUIRE(K % 8 == 0, "gemm_bf16_stream: K=%d must be a multiple of 8", K);
   CWM_REQUIRE(lda % 8 == 0 && ldw % 8 == 0, "gemm_bf16_stream: row strides must be multiples of 8 elements");
   CWM_REQUIRE(((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0, "gemm_bf16_stream: operands must be 16-byte aligned");
@@ -335,14 +342,22 @@ extern "C" int cwm_gemm_bf16_stream(const void* A, long lda, const void* W, long
     else                                                            \
       CWM_LAUNCH_STREAM_AS(TC, ROPE, GLU, MT, WAVES, HALF, false);  \
   } while (0)
-  if (rope)
+  if (rope && M <= 16)
     CWM_LAUNCH_STREAM(bf16_t, true, false, 1, ST1_WAVES, ST1_HALF);
-  else if (glu)
+  else if (rope)
+    CWM_LAUNCH_STREAM(bf16_t, true, false, 2, ST2_WAVES, ST2_HALF);
+  else if (glu && M <= 16)
     CWM_LAUNCH_STREAM(bf16_t, false, true, 1, ST1_WAVES, ST1_HALF);
+  else if (glu)
+    CWM_LAUNCH_STREAM(bf16_t, false, true, 2, ST2_WAVES, ST2_HALF);
   else if (M <= 16 && c_dtype == CWM_F32)
     CWM_LAUNCH_STREAM(float, false, false, 1, ST1_WAVES, ST1_HALF);
   else if (M <= 16)
     CWM_LAUNCH_STREAM(bf16_t, false, false, 1, ST1_WAVES, ST1_HALF);
+  else if (M <= 32 && c_dtype == CWM_F32)
+    CWM_LAUNCH_STREAM(float, false, false, 2, ST2_WAVES, ST2_HALF);
+  else if (M <= 32)
+    CWM_LAUNCH_STREAM(bf16_t, false, false, 2, ST2_WAVES, ST2_HALF);
   else if (c_dtype == CWM_F32)
     CWM_LAUNCH_STREAM(float, false, false, 4, ST4_WAVES, ST4_HALF);
   else

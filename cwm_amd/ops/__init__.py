@@ -415,13 +415,14 @@ def gemm_bf16_stream(
         raise KernelError(f"gemm: bias {tuple(bias.shape)} does not fit {n} outputs")
     out_dtype = out_dtype or torch.bfloat16
     lib = _build.load("gemm_bf16_stream")
-    waves, regs = _stream_block_shape(m)
+    # from 17 rows on K is split as for 64, so that a row's bits are the same; the fused epilogues take the longer K that 32 rows' registers hold
+    waves, regs = _stream_block_shape(m if m <= 16 or rope is not None or glu else STREAM_MAX_ROWS)
     steps = (k + 31) // 32
     n_tiles = (n + 15) // 16
     cus = _compute_units(x.device)
     k_split = -(-steps // (waves * regs))  # K longer than one group of wavefronts' registers is split
-    if (rope is not None or glu) and (k_split != 1 or m > 16):
-        raise KernelError("the fused epilogues need at most 16 rows and a K that one group of wavefronts holds")
+    if (rope is not None or glu) and (k_split != 1 or m > STREAM_EPILOGUE_ROWS):
+        raise KernelError("the fused epilogues need at most 32 rows and a K that one group of wavefronts holds")
     if glu:
         partials_ok = False
     if partials_ok:
@@ -467,7 +468,7 @@ def gemm_bf16_stream(
 def linear_inputs_takes(x: torch.Tensor, weight: torch.Tensor, rows_per_input: int) -> bool:
     """Whether the product of a few rows of several inputs is one launch (`linear_inputs`)."""
     return (
-        x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 3 and x.shape[1] <= STREAM_EPILOGUE_ROWS
+        x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 3 and x.shape[1] <= 16
         and rows_per_input % 16 == 0 and x.is_contiguous() and x.shape[1] * x.shape[2] % 8 == 0 and _stream_takes(x[0], weight)
     )
 
@@ -689,11 +690,20 @@ def gemm_bf16_tile(
     return out if out.dim() == 3 or out.dtype == out_dtype else out.to(out_dtype)
 
 
-# rows up to which the streaming product (x in registers, every epilogue in the kernel) is preferred; its epilogues take
-# up to 16, but from 9 on the tiled product is as fast or faster where it takes the sizes (a decode step of the 32B shape at
-# batch 16: 15.3 against 15.6 ms)
+# rows up to which the streaming product (x in registers, every epilogue in the kernel) is preferred whatever the matrix
 STREAM_FUSED_ROWS = 8
-STREAM_EPILOGUE_ROWS = 16
+STREAM_EPILOGUE_ROWS = 32  # rows up to which its epilogues go
+# From 9 to 32 rows the streaming product is ahead for matrices of fewer entries than these, where there is a streaming copy: it
+# rotates, writes the cache and applies the gate in its epilogue, and leaves one to four partial sums where the tiled one, whose
+# blocks share tiles of a small matrix, leaves up to 16.  Measured with the kernels that then follow, streamed / tiled, us: q/k/v of
+# 3,072 x 2,048 6.5 / 13.1 at 12 rows and 7.9 / 13.5 at 24, of 6,144 x 4,096 14.8 / 20.5 at 12, of 8,192 x 6,144 21.0 / 24.2; gate/up
+# of 16,384 x 2,048 14.2 / 16.6 and 15.0 / 17.1, of 28,672 x 4,096 39.1 / 42.0, but of 43,008 x 6,144 83.1 / 80.8; K split over blocks:
+# 2,048 x 8,192 11.3 / 13.0 and 12.6 / 14.0, 3,072 x 9,216 15.4 / 17.4 and 16.9 / 18.3, but 4,096 x 14,336 26.6 / 24.8 and 28.1 / 25.9.
+STREAM_WHOLE_ENTRIES = 1 << 27
+STREAM_SPLIT_ENTRIES = 1 << 25
+# Matrices of fewer entries than this (half a megabyte, which reading does not bound) stay with the tiled product from 9 rows on
+# whether they have a copy or not, so that the bits of a small model do not depend on its copies.
+STREAM_LEAST_ENTRIES = 1 << 18
 TILE_ROWS = 128  # rows up to which the tiled product is the fastest whatever the shape
 TILE_TALL_ROWS = 256  # rows of its tallest block: up to there it reads W once
 TILE_COLUMNS = 128  # columns of a tall block's tile
@@ -704,15 +714,20 @@ TILE_FEW_ROWS_ENTRIES = 1 << 24
 
 
 def _prefers_tile(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], streamed: Optional[torch.Tensor] = None) -> bool:
-    """Whether this product goes to the tiled kernel (which has no bias of its own): from 9 rows on; and for
+    """Whether this product goes to the tiled kernel (which has no bias of its own): from 33 rows on, from 9 on where
+    the matrix has no streaming copy or is not among those of `STREAM_LEAST_ENTRIES` to `STREAM_WHOLE_ENTRIES`; and for
     fewer rows where the matrix is large and has no streaming copy, since the tiled kernel reads the row-major
     matrix in whole cache lines past the caches, which the streaming kernel can only do with that copy (a
     layer's four products of the 32B shape at 8 rows: 159 us tiled, 187 us streamed from the row-major
     matrices, 159 us streamed from the copies; at 1 row 163, 178 and 154 us)."""
     if bias is not None:
         return False
-    if x.shape[0] <= STREAM_FUSED_ROWS and (streamed is not None or weight.numel() < TILE_FEW_ROWS_ENTRIES):
+    m = x.shape[0]
+    if m <= STREAM_FUSED_ROWS and (streamed is not None or weight.numel() < TILE_FEW_ROWS_ENTRIES):
         return False
+    if m <= STREAM_EPILOGUE_ROWS and streamed is not None and weight.numel() >= STREAM_LEAST_ENTRIES:
+        if weight.numel() < (STREAM_WHOLE_ENTRIES if weight.shape[1] <= stream_unsplit_k(m) else STREAM_SPLIT_ENTRIES):
+            return False
     return _tile_wins(x, weight)
 
 
@@ -754,7 +769,8 @@ def gemm_bf16(
 ) -> torch.Tensor:
     """bfloat16 x [M, K] @ bfloat16 weight[N, K]^T, float32 accumulation.
 
-    Up to 8 rows: the hand-written persistent weight-streaming kernel, x in registers.
+    Up to 8 rows, and up to 32 for all but the largest matrices that have a streaming copy: the hand-written persistent
+    weight-streaming kernel, x in registers.
     Up to 128 rows (256 for a result of at most 16,384 columns): the hand-written tiled kernel, x and W
     through LDS (it needs K % 64 == 0 and N % 16 == 0; other sizes of up to 64 rows stream).
     More rows: the library product (hipBLASLt through torch), as the reference calls a
