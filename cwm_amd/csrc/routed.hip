@@ -22,6 +22,8 @@
 // 16 j + r holds out[r][n0 + 4 j + i], i = 0..3.
 #include "common.h"
 
+#include <type_traits>
+
 CWM_DEFINE_ERROR_API
 
 #define ROUTE_MAX_TOP 16
@@ -392,6 +394,7 @@ template <> struct Frag<bf16_t> {
   Frag8 f;
   __device__ __forceinline__ void zero() { f.u = make_uint4(0, 0, 0, 0); }
   __device__ __forceinline__ void load16(const bf16_t* p) { f.u = *(const uint4*)p; }
+  __device__ __forceinline__ void load16_once(const bf16_t* p) { f.w = __builtin_nontemporal_load((const decltype(f.w)*)p); }
   __device__ __forceinline__ void load_some(const bf16_t* p, int n) {
     zero();
     for (int i = 0; i < PER_LANE; ++i)
@@ -548,10 +551,12 @@ __global__ void __launch_bounds__(256) grouped_product_kernel(const T* __restric
 // Few rows an expert (a decode step): the product is bound by streaming the chosen experts' weights once.  A block
 // takes one row tile and 16 columns; its four wavefronts split K (wavefront w the steps w, w + 4, ...: together they
 // read whole lines of a weight row), each with STREAM_DEPTH steps of operands in flight while the ones before are
-// multiplied, and add their sums through LDS in the order of w.  Rows of a and W start at multiples of 16 bytes.
+// multiplied, and add their sums through LDS in the order of w.  Rows of a and W start at multiples of 16 bytes.  TILED: weights in
+// operand tiles, whose lines are read once and past the caches (eight tokens, 14 of 16 experts of 2,048 x 1,024: gate and up 24 us,
+// row-major 27).
 #define STREAM_DEPTH 4
 
-template <typename T, bool GATED>
+template <typename T, bool GATED, bool TILED>
 __global__ void __launch_bounds__(256) grouped_stream_kernel(const T* __restrict__ a, long a_ld, long a_batch, const int* __restrict__ row_token,
                                                              const T* __restrict__ w0, const T* __restrict__ w1, long w_stride,
                                                              const int* __restrict__ tile_expert, int n_tiles, void* __restrict__ out,
@@ -575,7 +580,7 @@ __global__ void __launch_bounds__(256) grouped_stream_kernel(const T* __restrict
   }
   const int n0 = blockIdx.y * 16;
   const int col = n0 + r;
-  const size_t at = (size_t)expert * w_stride + (size_t)(col < N ? col : N - 1) * K;
+  const size_t at = (size_t)expert * w_stride + (TILED ? ((size_t)blockIdx.y * (K / 32) * 64 + lane) * 8 : (size_t)(col < N ? col : N - 1) * K);
   const T* wrow0 = w0 + at;
   const T* wrow1 = GATED ? w1 + at : nullptr;
   const int row = tile * TILE_ROWS + r;
@@ -590,8 +595,13 @@ __global__ void __launch_bounds__(256) grouped_stream_kernel(const T* __restrict
       const int step = wave + 4 * (first + d);
       const int k = step * STEP + j * PIECE;
       if (step < steps && k < K) {
-        fw0[d].load16(wrow0 + k);
-        if (GATED) fw1[d].load16(wrow1 + k);
+        if constexpr (TILED) {
+          fw0[d].load16_once(wrow0 + (size_t)step * 512);
+          if (GATED) fw1[d].load16_once(wrow1 + (size_t)step * 512);
+        } else {
+          fw0[d].load16(wrow0 + k);
+          if (GATED) fw1[d].load16(wrow1 + k);
+        }
         if (arow) fa[d].load16(arow + k); else fa[d].zero();
       } else {
         fw0[d].zero();
@@ -650,79 +660,70 @@ __global__ void __launch_bounds__(256) grouped_stream_kernel(const T* __restrict
 // With a list the blocks are numbered so that an XCD gets a run of neighbours in the order (group of WIDE_GROUP row blocks,
 // columns, row block): the row blocks of an expert then share its weights in one L2, where dealing them to the XCDs in turn
 // has every XCD read every expert's weights.  `used` says how many tiles of the list are in use, so the runs are equally long.
-// 16 experts of 2,048 x 1,024, four a token, evenly loaded, gate and up / down: 2,048 tokens 128 / 71 us (535 / 484 TFLOP/s; blocks
-// that staged both operands through LDS: 204 / 135 us), 4,096 tokens 215 / 117 us (370 / 240 us), 300 tokens 51 / 30 us (117 / 79
-// us straight from memory).  With a router's uneven loads 2,048 tokens take 146 / 85 us; the last round of blocks is nearly empty at
-// some sizes, which costs up to a quarter.
+// TILED: the weights lie in operand tiles (an expert's [N / 16][K / 32][64 lanes][8 values]), 1 KB of consecutive memory a load.
+// Read from row-major weights, a load is 16 rows' pieces of 64 bytes, four neighbouring lanes in four rows, which costs the
+// vector memory path a lookup a lane: with half or all of a block's products left out the kernel took as long.  An expert's
+// last block multiplies as many row tiles as it has (2, 4 or 8).
+// 16 experts of 2,048 x 1,024, four a token, gate and up / down, operand tiles and row-major: 2,048 tokens evenly loaded 74 / 46 us
+// (924 / 743 TFLOP/s) and 105 / 58; with a router's uneven loads 100 / 58 and 135 / 76 (a CU that gets three blocks where others
+// get two decides), 1,500 tokens 72 / 42 and 97 / 53, 4,096 tokens 159 / 99 and 204 / 121, 300 tokens 38 / 20 and 42 / 21.
 #define WIDE_GROUP 4
+#define WIDE_MAX_ROWS 128
 
-template <int RT, int CT, bool GATED>
-__global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __restrict__ a, long a_ld, long a_batch, const int* __restrict__ row_token,
-                                                              const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, long w_stride,
-                                                              const int* __restrict__ tile_expert, const int* __restrict__ used, int n_tiles,
-                                                              int row_blocks, int col_blocks,
-                                                              void* __restrict__ out, int out_dtype, long out_ld, long out_batch, int vec_out,
-                                                              int n_rows, int N, int K, GateAct act) {
+// A wavefront's and a block's place in a wide product, and what its loop needs of the kernel's arguments.
+struct WideBlock {
+  const bf16_t* a;
+  long a_ld;
+  const int* row_token;  // with a list: the token of each of its rows, or null
+  const bf16_t *w0, *w1;  // the block's expert's
+  const int* tile_expert;
+  int n_tiles, expert, tile0, n0, n_rows, N, K;
+};
+
+// A barrier that waits for the wavefront's LDS accesses only, not for the global loads on their way.
+__device__ __forceinline__ void wide_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); }
+
+template <int RT, int CT, bool GATED, bool TILED, int BLOCK_ROWS>
+__device__ __forceinline__ void wide_rows(const WideBlock& wb, uint4 (*lds_rows)[BLOCK_ROWS * 8], void* __restrict__ out, int out_dtype,
+                                          size_t out_base, long out_ld, int vec_out, GateAct act) {
   constexpr int ROWS = RT * TILE_ROWS, FETCH = ROWS * 8 / 256;  // 16-byte pieces of the rows that a thread fetches a step
   constexpr int WT = GATED ? CT / 2 : CT;                       // column tiles of the result a wavefront makes
-  __shared__ uint4 lds_rows[2][ROWS * 8];
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
   const int r = lane & 15, j = lane >> 4;
-  int bx, by, expert;
-  if (tile_expert) {
-    const int live = ((used ? min(*used, n_tiles) : n_tiles) + RT - 1) / RT, total = live * col_blocks;
-    const int run = (total + 7) >> 3, at = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= run || at >= total) return;
-    const int first = at / (WIDE_GROUP * col_blocks) * WIDE_GROUP, rest = at - first * col_blocks;
-    const int together = min(WIDE_GROUP, live - first);
-    bx = first + rest % together;
-    by = rest / together;
-    expert = tile_expert[bx * RT];
-    if (expert < 0) return;
-  } else {
-    bx = blockIdx.x % row_blocks;
-    by = blockIdx.x / row_blocks;
-    expert = blockIdx.z;
-  }
-  const int tile0 = bx * RT;
-  const int n0 = by * (64 * WT) + wave * (16 * WT);
+  const int tile0 = wb.tile0, n0 = wb.n0, N = wb.N, K = wb.K;
   // rows that do not exist, and those of tiles that are another expert's, are read from a row that does; nothing uses the results
-  const bf16_t* src_a[FETCH];
+  uint32_t src_a[FETCH];  // in pieces: rows are whole pieces long
 #pragma unroll
   for (int i = 0; i < FETCH; ++i) {
-    const int id = threadIdx.x + 256 * i;
-    const int list_row = tile0 * TILE_ROWS + (id >> 3);
-    long src;
-    if (tile_expert)
-      src = list_row >= n_tiles * TILE_ROWS ? 0 : row_token ? max(row_token[list_row], 0) : min(list_row, n_rows - 1);
+    const int list_row = tile0 * TILE_ROWS + (threadIdx.x >> 3) + 32 * i;
+    int src;
+    if (wb.tile_expert)
+      src = list_row >= wb.n_tiles * TILE_ROWS ? 0 : wb.row_token ? max(wb.row_token[list_row], 0) : min(list_row, wb.n_rows - 1);
     else
-      src = min(list_row, n_rows - 1);
-    src_a[i] = a + (size_t)blockIdx.z * a_batch + (size_t)src * a_ld + (id & 7) * 8;
+      src = min(list_row, wb.n_rows - 1);
+    src_a[i] = (uint32_t)src * (uint32_t)(wb.a_ld / 8) + (threadIdx.x & 7);
   }
-  const bf16_t* we0 = w0 + (size_t)expert * w_stride;
-  const bf16_t* we1 = GATED ? w1 + (size_t)expert * w_stride : nullptr;
   uint32_t src_w[CT];  // N * K < 2^31
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct) src_w[ct] = (uint32_t)min(n0 + (ct % WT) * 16 + r, N - 1) * (uint32_t)K + j * 8;
+  for (int ct = 0; ct < CT; ++ct) {
+    const int n = n0 + (ct % WT) * 16;
+    src_w[ct] = TILED ? (uint32_t)min(n, N - 16) * (uint32_t)K + lane * 8 : (uint32_t)min(n + r, N - 1) * (uint32_t)K + j * 8;
+  }
   typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
   Words4 ra[FETCH];
   auto fetch = [&](int k0) {
 #pragma unroll
-    for (int i = 0; i < FETCH; ++i) ra[i] = *(const Words4*)(src_a[i] + k0);
+    for (int i = 0; i < FETCH; ++i) ra[i] = *((const Words4*)wb.a + src_a[i] + (uint32_t)k0 / 8);
   };
+  const int staged = (threadIdx.x & ~7) + ((threadIdx.x & 7) ^ ((threadIdx.x >> 3) & 7));
   auto stage = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < FETCH; ++i) {
-      const int id = threadIdx.x + 256 * i;
-      const int row = id >> 3, piece = id & 7;
-      *(Words4*)&lds_rows[buf][row * 8 + (piece ^ (row & 7))] = ra[i];
-    }
+    for (int i = 0; i < FETCH; ++i) *(Words4*)&lds_rows[buf][staged + 256 * i] = ra[i];
   };
   Frag8 fw[2][CT];
   auto load_weights = [&](int half, int k0) {
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) fw[half][ct].u = *(const uint4*)((ct < WT ? we0 : we1) + (src_w[ct] + (uint32_t)(k0 + 32 * half)));
+    for (int ct = 0; ct < CT; ++ct) fw[half][ct].u = *(const uint4*)((ct < WT ? wb.w0 : wb.w1) + (src_w[ct] + (TILED ? (uint32_t)(k0 * 16 + 512 * half) : (uint32_t)(k0 + 32 * half))));
   };
   float4v acc[RT][CT];
 #pragma unroll
@@ -730,17 +731,18 @@ __global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __re
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = (float4v){0.f, 0.f, 0.f, 0.f};
   const int steps = K / 64;
+  auto place = [&](int step) { return min(step, steps - 1) * 64; };
   fetch(0);
   load_weights(0, 0);
   load_weights(1, 0);
   stage(0);
-  fetch(min(1, steps - 1) * 64);
-  __syncthreads();
+  fetch(place(1));
+  wide_barrier();
   // No branch in the loop (the last steps load again what they have): with one around a load the compiler waits for the
   // load where the paths meet.  The scheduling barriers keep the loads where they are, ahead of the other half's products.
   for (int step = 0; step < steps; ++step) {
     const uint4* rows = lds_rows[step & 1];
-    const int next = min(step + 1, steps - 1) * 64;
+    const int next = place(step + 1);
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int piece = half * 4 + j;
@@ -748,22 +750,22 @@ __global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __re
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) fa[rt].u = rows[(rt * 16 + r) * 8 + (piece ^ (r & 7))];
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
+      for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[half][ct].v, fa[rt].v, acc[rt][ct], 0, 0, 0);
+        for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[half][ct].v, fa[rt].v, acc[rt][ct], 0, 0, 0);
       load_weights(half, next);
       __builtin_amdgcn_sched_barrier(0);
     }
     stage((step + 1) & 1);
     __builtin_amdgcn_sched_barrier(0);
-    fetch(min(step + 2, steps - 1) * 64);
-    __syncthreads();
+    fetch(place(step + 2));
+    wide_barrier();
   }
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int tile = tile0 + rt, row = tile * TILE_ROWS + r;
-    if (tile_expert ? !(tile < n_tiles && tile_expert[tile] == expert) : row >= n_rows) continue;
-    const size_t base = (size_t)blockIdx.z * out_batch + (size_t)row * out_ld;
+    if (wb.tile_expert ? !(tile < wb.n_tiles && wb.tile_expert[tile] == wb.expert) : row >= wb.n_rows) continue;
+    const size_t base = out_base + (size_t)row * out_ld;
 #pragma unroll
     for (int ct = 0; ct < WT; ++ct) {
       const int c = n0 + ct * 16 + 4 * j;  // four adjacent columns
@@ -789,6 +791,52 @@ __global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __re
   }
 }
 
+template <int RT, int CT, bool GATED, bool TILED>
+__global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __restrict__ a, long a_ld, long a_batch, const int* __restrict__ row_token,
+                                                              const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, long w_stride,
+                                                              const int* __restrict__ tile_expert, const int* __restrict__ used, int n_tiles,
+                                                              int row_blocks, int col_blocks,
+                                                              void* __restrict__ out, int out_dtype, long out_ld, long out_batch, int vec_out,
+                                                              int n_rows, int N, int K, GateAct act) {
+  constexpr int WT = GATED ? CT / 2 : CT;
+  __shared__ uint4 lds_rows[2][RT * TILE_ROWS * 8];
+  const int wave = threadIdx.x >> 6;
+  int bx, by, expert, live_tiles;
+  if (tile_expert) {
+    const int live = ((used ? min(*used, n_tiles) : n_tiles) + RT - 1) / RT, total = live * col_blocks;
+    const int run = (total + 7) >> 3, at = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= run || at >= total) return;
+    const int first = at / (WIDE_GROUP * col_blocks) * WIDE_GROUP, rest = at - first * col_blocks;
+    const int together = min(WIDE_GROUP, live - first);
+    bx = first + rest % together;
+    by = rest / together;
+    expert = tile_expert[bx * RT];
+    if (expert < 0) return;
+    live_tiles = 1;
+#pragma unroll
+    for (int t = 1; t < RT; ++t) live_tiles += bx * RT + t < n_tiles && tile_expert[min(bx * RT + t, n_tiles - 1)] == expert;
+  } else {
+    bx = blockIdx.x % row_blocks;
+    by = blockIdx.x / row_blocks;
+    expert = blockIdx.z;
+    live_tiles = (n_rows + TILE_ROWS - 1) / TILE_ROWS - bx * RT;
+  }
+  const WideBlock wb = {a + (size_t)blockIdx.z * a_batch, a_ld, row_token, w0 + (size_t)expert * w_stride, GATED ? w1 + (size_t)expert * w_stride : nullptr,
+                        tile_expert, n_tiles, expert, bx * RT, by * (64 * WT) + wave * (16 * WT), n_rows, N, K};
+  const size_t out_base = (size_t)blockIdx.z * out_batch;
+  // an expert's last block takes as many row tiles as it has, rounded up to 2, 4 or 8: the others' products would be for padding
+  auto go = [&](auto tiles) {
+    if constexpr (decltype(tiles)::value <= RT)
+      wide_rows<decltype(tiles)::value, CT, GATED, TILED, RT * TILE_ROWS>(wb, lds_rows, out, out_dtype, out_base, out_ld, vec_out, act);
+  };
+  if (RT >= 8 && live_tiles > 4)
+    go(std::integral_constant<int, 8>());
+  else if (RT >= 4 && live_tiles > 2)
+    go(std::integral_constant<int, 4>());
+  else
+    go(std::integral_constant<int, 2>());
+}
+
 template <typename T, int RT, int CT, int WR, bool GATED>
 static void launch_grouped(bool vec, int tiles, int n_batch, hipStream_t stream, const T* a, long a_ld, long a_batch, const int* row_token,
                            const T* w0, const T* w1, long w_stride, const int* tile_expert, int n_tiles, void* out, int out_dtype,
@@ -809,12 +857,14 @@ static void launch_grouped(bool vec, int tiles, int n_batch, hipStream_t stream,
 // multiplies the same n_rows rows by its own weight into out + z * out_batch.  tiles_a_block: 1, 2, 4 or 8 row tiles
 // a block; with a list, an expert's tiles start at a multiple of `tile_align`, itself a multiple of tiles_a_block.  used: how many
 // of the list's tiles may have rows (`cwm_group_by_expert` leaves the number), or null: any of them.  act_kind, act_alpha, act_limit: the gated
-// form's activation (`GateAct`).
+// form's activation (`GateAct`).  tiled: the weights are in operand tiles (bfloat16, [experts][N / 16][K / 32][64][8]).
 extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int dtype, const int* row_token, const void* w0, const void* w1,
                                    long w_stride, const int* tile_expert, const int* used, int n_tiles, int n_batch, void* out, int out_dtype, long out_ld,
                                    long out_batch, int n_rows, int N, int K, int tiles_a_block, int tile_align, int act_kind,
-                                   float act_alpha, float act_limit, hipStream_t stream) {
+                                   float act_alpha, float act_limit, int tiled, hipStream_t stream) {
   CWM_REQUIRE(a && w0 && out, "grouped_product: arguments missing");
+  CWM_REQUIRE(!tiled || (dtype == CWM_BF16 && N % 16 == 0 && K % 64 == 0 && (long)N * K < (1l << 31)),
+              "grouped_product: weights in operand tiles are bfloat16, N a multiple of 16 and K of 64");
   CWM_REQUIRE(act_kind >= 0 && act_kind <= 2, "grouped_product: unknown gated activation %d", act_kind);
   const GateAct act = {act_kind, act_alpha, act_limit};
   CWM_REQUIRE(N > 0 && K > 0 && a_ld >= K && out_ld >= 0, "grouped_product: bad sizes");
@@ -845,17 +895,17 @@ extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int d
       else CWM_GROUPED(T, 1, 1, 1, false);                                      \
     }                                                                           \
   } while (0)
-  if (tiles_a_block > 1 && vec && dtype == CWM_BF16 && K % 64 == 0 && (long)N * K < (1l << 31)) {
+  if (tiles_a_block > 1 && vec && dtype == CWM_BF16 && K % 64 == 0 && (long)N * K < (1l << 31) && (long)n_rows * (a_ld / 8) < (1l << 32)) {
     // the shape whose rows go through LDS
     const int osize = out_dtype == CWM_F32 ? 4 : 2;
     const int vec_out = (out_ld * osize) % (4 * osize) == 0 && (out_batch * osize) % (4 * osize) == 0 && ((uintptr_t)out % (4 * osize)) == 0;
     const int row_blocks = (tiles + tiles_a_block - 1) / tiles_a_block;
-#define CWM_WIDE(RT, CT, GATED)                                                                                                            \
+#define CWM_WIDE_AS(RT, CT, GATED, TILED)                                                                                                            \
   do {                                                                                                                                     \
     const int cols = (GATED ? 32 : 64) * CT, col_blocks = (N + cols - 1) / cols;                                                           \
     dim3 grid((row_blocks * col_blocks + 7) / 8 * 8, 1, nb);                                                                               \
     if (!tile_expert) grid.x = row_blocks * col_blocks;                                                                                    \
-    hipLaunchKernelGGL((grouped_wide_kernel<RT, CT, GATED>), grid, dim3(256), 0, stream, (const bf16_t*)a, a_ld, a_batch, row_token,        \
+    hipLaunchKernelGGL((grouped_wide_kernel<RT, CT, GATED, TILED>), grid, dim3(256), 0, stream, (const bf16_t*)a, a_ld, a_batch, row_token,        \
                        (const bf16_t*)w0, (const bf16_t*)w1, w_stride, tile_expert, used, n_tiles, row_blocks, col_blocks, out, out_dtype,       \
                        out_ld, out_batch, vec_out, n_rows, N, K, act);                                                                     \
   } while (0)
@@ -864,6 +914,13 @@ extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int d
     // 220 us; 32 of 3,072 x 1,536: 256 rows 320 and 363 us).  Blocks of two row tiles stream the weights: always two.
     const int blocks4 = row_blocks * ((N + (w1 ? 127 : 255)) / (w1 ? 128 : 256));
     const bool many = tiles_a_block == 8 ? blocks4 >= 500 : tiles_a_block == 4 && blocks4 >= 560;
+#define CWM_WIDE(RT, CT, GATED)            \
+  do {                                     \
+    if (tiled)                             \
+      CWM_WIDE_AS(RT, CT, GATED, true);    \
+    else                                   \
+      CWM_WIDE_AS(RT, CT, GATED, false);   \
+  } while (0)
 #define CWM_WIDE_COLS(RT, GATED)   \
   do {                             \
     if (many)                      \
@@ -882,22 +939,28 @@ extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int d
     }
 #undef CWM_WIDE_COLS
 #undef CWM_WIDE
+#undef CWM_WIDE_AS
     return cwm_launch_status("grouped_product");
   }
   if (tiles_a_block <= 2 && vec && (dtype == CWM_BF16 || dtype == CWM_F32)) {
     // the weight-streaming shape
     dim3 grid(tiles, (N + 15) / 16, nb);
-#define CWM_STREAMED(T, GATED)                                                                                                             \
-  hipLaunchKernelGGL((grouped_stream_kernel<T, GATED>), grid, dim3(256), 0, stream, (const T*)a, a_ld, a_batch, row_token, (const T*)w0,     \
+#define CWM_STREAMED(T, GATED, TILED)                                                                                                             \
+  hipLaunchKernelGGL((grouped_stream_kernel<T, GATED, TILED>), grid, dim3(256), 0, stream, (const T*)a, a_ld, a_batch, row_token, (const T*)w0,     \
                      (const T*)w1, w_stride, tile_expert, n_tiles, out, out_dtype, out_ld, out_batch, n_rows, N, K, act, tile_align)
     if (dtype == CWM_BF16) {
-      if (w1) CWM_STREAMED(bf16_t, true); else CWM_STREAMED(bf16_t, false);
+      if (tiled) {
+        if (w1) CWM_STREAMED(bf16_t, true, true); else CWM_STREAMED(bf16_t, false, true);
+      } else {
+        if (w1) CWM_STREAMED(bf16_t, true, false); else CWM_STREAMED(bf16_t, false, false);
+      }
     } else {
-      if (w1) CWM_STREAMED(float, true); else CWM_STREAMED(float, false);
+      if (w1) CWM_STREAMED(float, true, false); else CWM_STREAMED(float, false, false);
     }
 #undef CWM_STREAMED
     return cwm_launch_status("grouped_product");
   }
+  CWM_REQUIRE(!tiled, "grouped_product: weights in operand tiles need rows at multiples of 16 bytes");
   if (dtype == CWM_BF16)
     CWM_GROUPED_SHAPES(bf16_t);
   else if (dtype == CWM_F32)

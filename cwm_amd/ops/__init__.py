@@ -1337,7 +1337,7 @@ from .sequence import (  # noqa: E402
     scan_state_unpack, selective_scan, sigmoid_mul, step_segments, token_shift,
 )
 from .routed import (  # noqa: E402
-    MAX_EXPERTS, MAX_ROUTE_TOP, ExpertGroups, GatedActivation, absorb_queries, combine_routed, expand_values, group_by_expert,
+    MAX_EXPERTS, MAX_ROUTE_TOP, ExpertGroups, GatedActivation, absorb_queries, combine_routed, expand_values, expert_tiles, group_by_expert,
     grouped_gate_up, grouped_linear, route_top,
 )
 from .streams import (  # noqa: E402

@@ -124,6 +124,25 @@ def group_by_expert(chosen: torch.Tensor, n_experts: int) -> ExpertGroups:
     return groups
 
 
+def expert_tiles(weights: torch.Tensor) -> torch.Tensor:
+    """The experts' matrices [E, N, K] (bfloat16, N a multiple of 16, K of 64) in operand tiles [E, N / 16, K / 32, 64, 8]: lane
+    16 j + r of a step of 32 columns holds row r's columns 8 j .. 8 j + 7, as in `stream_layout`, so that a wavefront's load of an
+    operand is 1 KB of consecutive memory instead of 16 rows' pieces of 64 bytes.  The grouped products take either form and
+    give the same bits."""
+    from . import stream_layout
+
+    KernelError = _base()[0]
+    if weights.dim() != 3 or weights.dtype != torch.bfloat16 or not weights.is_contiguous() or weights.shape[1] % 16 or weights.shape[2] % 64:
+        raise KernelError(f"operand tiles are made of contiguous bfloat16 [E, N, K] with N a multiple of 16 and K of 64, not {tuple(weights.shape)} {weights.dtype}")
+    e, n, k = weights.shape
+    return stream_layout(weights.view(e * n, k)).view(e, n // 16, k // 32, 64, 8)
+
+
+def _weight_shape(w: torch.Tensor) -> Tuple[int, int, int]:
+    """(experts, N, K) of grouped weights in either form."""
+    return (w.shape[0], 16 * w.shape[1], 32 * w.shape[2]) if w.dim() == 5 else tuple(w.shape)
+
+
 def _grouped(
     a: torch.Tensor, a_ld: int, a_batch: int, groups: Optional[ExpertGroups], w0: torch.Tensor, w1: Optional[torch.Tensor],
     out: torch.Tensor, out_ld: int, out_batch: int, n_rows: int, n_batch: int,
@@ -132,9 +151,15 @@ def _grouped(
     """`gather`: `a` has the tokens' rows, which the list picks; else it has the list's own rows."""
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
     _need_gpu(a, w0, w1, out)
-    if w0.dim() != 3 or not w0.is_contiguous() or w0.dtype != a.dtype or (w1 is not None and (w1.shape != w0.shape or not w1.is_contiguous() or w1.dtype != a.dtype)):
-        raise KernelError("grouped weights must be contiguous [experts, N, K] tensors of the rows' type")
-    e, n, k = w0.shape
+    tiled = w0.dim() == 5
+    if (
+        not (w0.dim() == 3 or (tiled and tuple(w0.shape[3:]) == (64, 8) and w0.shape[2] % 2 == 0 and w0.dtype == torch.bfloat16))
+        or not w0.is_contiguous() or w0.dtype != a.dtype or (w1 is not None and (w1.shape != w0.shape or not w1.is_contiguous() or w1.dtype != a.dtype))
+    ):
+        raise KernelError("grouped weights must be contiguous [experts, N, K] tensors of the rows' type, or bfloat16 in operand tiles (`expert_tiles`)")
+    e, n, k = _weight_shape(w0)
+    if tiled and a.data_ptr() % 16 != 0:
+        a = a.clone()  # the kernels that read operand tiles take rows at multiples of 16 bytes
     if groups is not None:
         if groups.tile_expert.numel() < groups.n_tiles or groups.row_token.numel() < groups.n_tiles * TILE_ROWS:
             raise KernelError(f"lists of {groups.tile_expert.numel()} tiles and {groups.row_token.numel()} rows do not hold {groups.n_tiles} tiles")
@@ -152,7 +177,7 @@ def _grouped(
             ctypes.c_int(n_rows), ctypes.c_int(n), ctypes.c_int(k), ctypes.c_int(tiles_a_block),
             ctypes.c_int(groups.tiles_a_block if groups is not None else 1),
             ctypes.c_int(activation.code() if activation is not None else 0), ctypes.c_float(activation.alpha if activation is not None else 1.0),
-            ctypes.c_float(activation.limit if activation is not None else 0.0), _stream(),
+            ctypes.c_float(activation.limit if activation is not None else 0.0), ctypes.c_int(int(tiled)), _stream(),
         ),
     )
 
@@ -182,10 +207,11 @@ def grouped_gate_up(
     `x` [T, D] contiguous, weights [E, F, D]; returns [rows, F] in the type of `x` (rows of the padding are not
     written)."""
     KernelError = _base()[0]
-    if x.dim() != 2 or not x.is_contiguous() or gate.shape[2] != x.shape[1]:
+    _, hidden, dim = _weight_shape(gate)
+    if x.dim() != 2 or not x.is_contiguous() or dim != x.shape[1]:
         raise KernelError("x must be a contiguous [T, D] tensor that fits the experts' weights")
-    out = torch.empty((groups.n_tiles * TILE_ROWS, gate.shape[1]), dtype=x.dtype, device=x.device)
-    _grouped(x, x.shape[1], 0, groups, gate, up, out, gate.shape[1], 0, groups.n_tiles * TILE_ROWS, 1, activation)
+    out = torch.empty((groups.n_tiles * TILE_ROWS, hidden), dtype=x.dtype, device=x.device)
+    _grouped(x, x.shape[1], 0, groups, gate, up, out, hidden, 0, groups.n_tiles * TILE_ROWS, 1, activation)
     return out
 
 
@@ -193,10 +219,11 @@ def grouped_linear(rows: torch.Tensor, groups: ExpertGroups, weight: torch.Tenso
     """W_e row for every row of the list (`rows` [rows, F] as `grouped_gate_up` leaves them, `weight` [E, D, F]):
     float32 [rows, D]."""
     KernelError = _base()[0]
-    if rows.dim() != 2 or not rows.is_contiguous() or weight.shape[2] != rows.shape[1] or rows.shape[0] != groups.n_tiles * TILE_ROWS:
+    _, dim, hidden = _weight_shape(weight)
+    if rows.dim() != 2 or not rows.is_contiguous() or hidden != rows.shape[1] or rows.shape[0] != groups.n_tiles * TILE_ROWS:
         raise KernelError("the rows do not fit the list or the experts' weights")
-    out = torch.empty((rows.shape[0], weight.shape[1]), dtype=torch.float32, device=rows.device)
-    _grouped(rows, rows.shape[1], 0, groups, weight, None, out, weight.shape[1], 0, rows.shape[0], 1, gather=False)
+    out = torch.empty((rows.shape[0], dim), dtype=torch.float32, device=rows.device)
+    _grouped(rows, rows.shape[1], 0, groups, weight, None, out, dim, 0, rows.shape[0], 1, gather=False)
     return out
 
 

@@ -83,8 +83,15 @@ class RoutedExperts(FeedForward):
             n = len(self.shared_prefix)
             self.shared.bind({name[n:]: t for name, t in tensors.items() if name.startswith(self.shared_prefix)}, runtime)
         self.choice_correction = tensors["correction"].float().contiguous() if self.correction else None
-        stack = lambda name: torch.stack([tensors[f"e{e}.{name}"] for e in range(self.n_experts)]).contiguous()  # noqa: E731
-        self.gate, self.up, self.down = stack("gate"), stack("up"), stack("down")  # [experts, out, in]
+        # [experts, out, in], or, where the matrix cores read them as they lie in memory, in operand tiles (a layout; the same size)
+        tiles = (
+            runtime.device.type == "cuda" and runtime.act_dtype == torch.bfloat16 and self.dim % 64 == 0 and self.hidden_dim % 64 == 0
+            and self.dim * self.hidden_dim < 2 ** 31
+        )
+        def stack(name: str) -> torch.Tensor:
+            whole = torch.stack([tensors[f"e{e}.{name}"] for e in range(self.n_experts)])
+            return ops.expert_tiles(whole) if tiles and whole.dtype == torch.bfloat16 else whole
+        self.gate, self.up, self.down = stack("gate"), stack("up"), stack("down")
 
     def forward(self, x: torch.Tensor, batch: Any) -> Any:
         routed = self.forward_deferred(x, batch).combine()  # float32 [T, dim]
