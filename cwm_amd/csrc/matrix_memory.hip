@@ -19,10 +19,10 @@
 // and g_t = m_t - b_t, the recurrence unrolls to
 //     S_t = exp(g_c - g_t) S_c + sum_(c < s <= t) exp(a_s - g_t) k_s v_s^T        (c: the token before the block)
 // with no exponent above zero, so a block's results are (Q K^T, weighted and masked) V + (weighted Q) S_c, and the state
-// moves once a block.  `memory_maxima_kernel` walks m (a thread block a (head, sequence), the same float32 operations as the
-// walk above, so both give the same m) and sums f in float64, since differences of long sums are taken;
+// moves once a block.  `memory_maxima_kernel` walks m (one thread a (head, sequence), the same float32 operations as the
+// walk above, so both give the same m: 29 us for 1,531 tokens, 39 where a wavefront passed every gate through a scalar register) and sums f in float64, since differences of long sums are taken;
 // `memory_scores_kernel` works out every block's weighted scores and weights side by side, and `memory_chunk_kernel` (a thread
-// block a (tile of value columns, head, sequence)) walks the blocks with the remaining products on the float32 matrix
+// block a (tile of value columns, head, sequence or segment of one)) walks the blocks with the remaining products on the float32 matrix
 // instruction.  The normaliser n
 // is the column after the last value column, with ones for values, so n_t . q_t falls out as that column's result and the
 // division moves into `memory_out_kernel`.  This differs from the walk by rounding only.
@@ -207,6 +207,10 @@ memory_scan_kernel(const T* __restrict__ src, long src_stride, int q_off, int k_
 #define MEMX_THREADS 256
 static_assert(MEMC_COLS == MEMC_L, "a block's scores are staged like its values");
 #define MEMX_SPAN 1024    // tokens whose gates are worked out side by side before the maximum walks them
+#define MEMX_AHEAD 8      // of them walked between two reads of gates
+static_assert(MEMX_SPAN % MEMX_AHEAD == 0, "whole reads of gates");
+#define MEMS_L 256        // tokens of a segment (whole blocks)
+static_assert(MEMS_L % MEMC_L == 0, "a segment is whole blocks");
 
 // coef: float32 [T][heads][4]: {i_t, m_t, b_t as a float64 in two words}; b counts from the portion's start.
 // start: float64 [n_seqs][heads]: m before the portion.
@@ -214,10 +218,11 @@ __global__ void __launch_bounds__(MEMX_THREADS)
 memory_maxima_kernel(const float* __restrict__ gates, long gates_stride, float cap, float* __restrict__ state, long state_stride,
                      long head_elems, const int* __restrict__ cu_q, const int* __restrict__ state_slots, float* __restrict__ coef,
                      double* __restrict__ start, int heads, int e, int d_pad) {
-  __shared__ float gi_s[MEMX_SPAN], gf_s[MEMX_SPAN];
+  __shared__ __attribute__((aligned(16))) float2 gate_s[MEMX_SPAN + MEMX_AHEAD];  // {i, f}
+  __shared__ __attribute__((aligned(16))) float m_s[MEMX_SPAN];
+  __shared__ double sum_s[MEMX_SPAN];
   const int h = blockIdx.x, b = blockIdx.y;
   const int lane = threadIdx.x & (CWM_WAVE - 1);
-  const bool walker = threadIdx.x < CWM_WAVE;  // the first wavefront walks; all work out gates
   const int t0 = cu_q[b], t1 = cu_q[b + 1];
   float* st_m = state + (size_t)state_slots[b] * state_stride + (size_t)h * head_elems + (size_t)e * d_pad + d_pad;
   float m = *st_m;
@@ -225,55 +230,70 @@ memory_maxima_kernel(const float* __restrict__ gates, long gates_stride, float c
   const float inv_cap = 1.0f / cap;
   double before = 0.0;
   for (int span = t0; span < t1; span += MEMX_SPAN) {
-    const int n = min(MEMX_SPAN, t1 - span);
-    __syncthreads();  // the span before has been walked
-    for (int x = threadIdx.x; x < n; x += MEMX_THREADS) {
-      const float* g = gates + (size_t)(span + x) * gates_stride;
-      gi_s[x] = cap * tanhf(g[h] * inv_cap);
-      gf_s[x] = log_sigmoid(cap * tanhf(g[heads + h] * inv_cap));
+    const int n = min(MEMX_SPAN, t1 - span), whole = (n + MEMX_AHEAD - 1) / MEMX_AHEAD * MEMX_AHEAD;
+    // beyond the portion's end: gates that leave m and the sum as they are, so the walk below needs no branch
+    for (int x = threadIdx.x; x < whole + MEMX_AHEAD; x += MEMX_THREADS) {
+      float2 g = make_float2(-INFINITY, 0.f);
+      if (x < n) {
+        const float* at = gates + (size_t)(span + x) * gates_stride;
+        g = make_float2(cap * tanhf(at[h] * inv_cap), log_sigmoid(cap * tanhf(at[heads + h] * inv_cap)));
+      }
+      gate_s[x] = g;
     }
     __syncthreads();
-    if (!walker) continue;
-    for (int base = 0; base < n; base += CWM_WAVE) {
-      const int count = min(CWM_WAVE, n - base);
-      // beyond the portion's end: gates that leave m as it is, so the walk below needs no branch
-      const float gi = lane < count ? gi_s[base + lane] : -INFINITY, gf = lane < count ? gf_s[base + lane] : 0.f;
-      double sum = (double)gf;  // zero beyond the portion's end
+    if (threadIdx.x == 0) {
+      // the walk, a chain of an addition and a maximum a token: the next gates are read while these are walked
+      float4 now[MEMX_AHEAD / 2], then[MEMX_AHEAD / 2];
 #pragma unroll
-      for (int off = 1; off < CWM_WAVE; off <<= 1) {
-        const double o = __shfl_up(sum, off, CWM_WAVE);
-        if (lane >= off) sum += o;
-      }
-      float mine = 0.f;
+      for (int u = 0; u < MEMX_AHEAD / 2; ++u) now[u] = *(const float4*)&gate_s[2 * u];
+      for (int x = 0; x < whole; x += MEMX_AHEAD) {
+        float mine[MEMX_AHEAD];
 #pragma unroll
-      for (int j = 0; j < CWM_WAVE; ++j) {
-        // (a lane known when compiling: read through a scalar register, not through LDS)
-        const float fj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gf), j));
-        const float ij = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gi), j));
-        m = fmaxf(fj + m, ij);
-        mine = lane == j ? m : mine;
+        for (int u = 0; u < MEMX_AHEAD / 2; ++u) then[u] = *(const float4*)&gate_s[x + MEMX_AHEAD + 2 * u];
+#pragma unroll
+        for (int u = 0; u < MEMX_AHEAD / 2; ++u) {
+          mine[2 * u] = m = fmaxf(now[u].y + m, now[u].x);
+          mine[2 * u + 1] = m = fmaxf(now[u].w + m, now[u].z);
+        }
+#pragma unroll
+        for (int u = 0; u < MEMX_AHEAD / 4; ++u) *(float4*)&m_s[x + 4 * u] = make_float4(mine[4 * u], mine[4 * u + 1], mine[4 * u + 2], mine[4 * u + 3]);
+#pragma unroll
+        for (int u = 0; u < MEMX_AHEAD / 2; ++u) now[u] = then[u];
       }
-      if (lane < count) {
-        float* c = coef + ((size_t)(span + base + lane) * heads + h) * 4;
-        c[0] = gi, c[1] = mine;
-        *(double*)(c + 2) = before + sum;
+    } else if (threadIdx.x >= CWM_WAVE && threadIdx.x < 2 * CWM_WAVE) {
+      for (int base = 0; base < n; base += CWM_WAVE) {
+        double sum = base + lane < n ? (double)gate_s[base + lane].y : 0.0;
+#pragma unroll
+        for (int off = 1; off < CWM_WAVE; off <<= 1) {
+          const double o = __shfl_up(sum, off, CWM_WAVE);
+          if (lane >= off) sum += o;
+        }
+        if (base + lane < n) sum_s[base + lane] = before + sum;
+        before += __shfl(sum, CWM_WAVE - 1, CWM_WAVE);
       }
-      before += __shfl(sum, CWM_WAVE - 1, CWM_WAVE);
     }
+    __syncthreads();
+    for (int x = threadIdx.x; x < n; x += MEMX_THREADS) {
+      float* c = coef + ((size_t)(span + x) * heads + h) * 4;
+      c[0] = gate_s[x].x, c[1] = m_s[x];
+      *(double*)(c + 2) = sum_s[x];
+    }
+    __syncthreads();  // the next span's gates take this one's place
   }
   if (threadIdx.x == 0) *st_m = m;
 }
 
-// The blocks of a step, numbered so that no two share a number: block j of sequence b is cu_q[b] / MEMC_L + b + j.
-// Returns the sequence of number x and sets the block's first token, or -1 if x is no block's number.
+// The blocks (or segments) of a step, L tokens each, numbered so that no two share a number: block j of sequence b is
+// cu_q[b] / L + b + j.  Returns the sequence of number x and sets the block's first token, or -1 if x is no block's number.
+template <int L>
 __device__ __forceinline__ int memory_block_of(int x, const int* __restrict__ cu_q, int n_seqs, int* base) {
-  int lo = 0, hi = n_seqs - 1;  // the last b with cu_q[b] / MEMC_L + b <= x
-  if (cu_q[0] / MEMC_L > x) return -1;
+  int lo = 0, hi = n_seqs - 1;  // the last b with cu_q[b] / L + b <= x
+  if (cu_q[0] / L > x) return -1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) / 2;
-    if (cu_q[mid] / MEMC_L + mid <= x) lo = mid; else hi = mid - 1;
+    if (cu_q[mid] / L + mid <= x) lo = mid; else hi = mid - 1;
   }
-  *base = cu_q[lo] + MEMC_L * (x - (cu_q[lo] / MEMC_L + lo));
+  *base = cu_q[lo] + L * (x - (cu_q[lo] / L + lo));
   return *base < cu_q[lo + 1] ? lo : -1;
 }
 
@@ -292,7 +312,7 @@ memory_scores_kernel(const T* __restrict__ src, long src_stride, int q_off, int 
   __shared__ double ga_s[MEMC_L], gg_s[MEMC_L];  // a and g of the block's tokens
   const int h = blockIdx.y;
   int base;
-  const int b = memory_block_of(blockIdx.x, cu_q, n_seqs, &base);
+  const int b = memory_block_of<MEMC_L>(blockIdx.x, cu_q, n_seqs, &base);
   if (b < 0) return;
   const int t0 = cu_q[b], t1 = cu_q[b + 1];
   const int count = min(MEMC_L, t1 - base);
@@ -358,34 +378,53 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // instructions a wavefront: (weighted Q) S over its rows and its share of (scores) V into one result, which the wavefronts
 // add up through LDS, then K^T (weighted V) into S.  A block's q, k, v, scores and weights are fetched into registers
 // while the block before is worked on.
-template <typename T, int TILES>
+//
+// PART: 0, a thread block walks a whole portion.  A long portion is a chain of blocks of tokens at 3.9 us each with few thread
+// blocks under way, so it is cut into segments of MEMS_L tokens that are walked side by side: 1, what a segment (all but a
+// portion's last) adds to the state, from zero and without results, into its place in `saved`; `memory_join_kernel` then makes
+// of these the states before the segments; 2, the segments' results from there, and the portion's last state.
+// saved: float32 [segments][heads][32 gridDim.x columns][32 TILES rows].
+template <typename T, int TILES, int PART>
 __global__ void __launch_bounds__(CWM_WAVE * TILES)
 memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k_off, int v_off, float q_scale,
                     const float* __restrict__ scores, const float* __restrict__ wd, float* __restrict__ state, long state_stride,
                     long head_elems, const int* __restrict__ cu_q, const int* __restrict__ state_slots, float* __restrict__ y,
-                    float* __restrict__ nq, int heads, int d, int e, int d_pad) {
+                    float* __restrict__ nq, float* __restrict__ saved, int n_seqs, int heads, int d, int e, int d_pad) {
+  constexpr bool RESULTS = PART != 1;
   constexpr int THREADS = CWM_WAVE * TILES, DP = 32 * TILES;
   constexpr int ROWQ = DP + 1, ROWK = DP + 4;  // a column of q across tokens, a row of k along its elements: no bank twice
   constexpr int QK_REGS = MEMC_L * DP / THREADS, V_REGS = MEMC_L * MEMC_COLS / THREADS;
   constexpr int SHARE = (MEMC_L / 2) / TILES;  // instructions of (scores) V that a wavefront issues
-  __shared__ float q_s[MEMC_L][ROWQ];
+  __shared__ float q_s[RESULTS ? MEMC_L : 1][ROWQ];
   __shared__ float k_s[MEMC_L][ROWK];
-  __shared__ float red[TILES][MEMC_L][MEMC_COLS];  // every wavefront's part of the block's results
-  __shared__ float a_s[MEMC_L][MEMC_L + 1];        // weighted and masked scores
+  __shared__ float red[RESULTS ? TILES : 1][MEMC_L][MEMC_COLS];  // every wavefront's part of the block's results
+  __shared__ float a_s[RESULTS ? MEMC_L : 1][MEMC_L + 1];        // weighted and masked scores
   __shared__ float v_s[MEMC_L][MEMC_COLS];
   __shared__ float w_s[MEMC_L], dec_s[MEMC_L];     // exp(a_s - g_last), exp(g_c - g_t)
-  const int h = blockIdx.y, b = blockIdx.z;
+  const int h = blockIdx.y;
   const int lane = threadIdx.x & (CWM_WAVE - 1), wave = threadIdx.x / CWM_WAVE;
   const int c = lane & 31, half = lane >> 5;
   const int col = blockIdx.x * MEMC_COLS + c;  // column e is the normaliser
   const int tile_row = 32 * wave;
-  const int t0 = cu_q[b], t1 = cu_q[b + 1];
+  int b = blockIdx.z, t0, t1;
+  bool last = true;  // of its portion
+  if constexpr (PART == 0) {
+    t0 = cu_q[b], t1 = cu_q[b + 1];
+  } else {
+    b = memory_block_of<MEMS_L>(blockIdx.z, cu_q, n_seqs, &t0);
+    if (b < 0) return;
+    t1 = cu_q[b + 1];
+    last = t0 + MEMS_L >= t1;
+    if (PART == 1 && last) return;
+    t1 = min(t1, t0 + MEMS_L);
+  }
   float* st = state + (size_t)state_slots[b] * state_stride + (size_t)h * head_elems + (size_t)col * d_pad;
+  float* kept = PART == 0 ? nullptr : saved + (((size_t)blockIdx.z * heads + h) * (gridDim.x * MEMC_COLS) + col) * DP;
   memc_acc S;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int row = tile_row + 8 * (r / 4) + 4 * half + (r % 4);
-    S[r] = (col <= e && row < d_pad) ? st[row] : 0.f;
+    S[r] = PART == 1 ? 0.f : PART == 2 ? kept[row] : (col <= e && row < d_pad) ? st[row] : 0.f;
   }
   // What a fetch leaves in registers is what the loads return and nothing made of it: an operation on a loaded value would
   // wait for the load where the fetch is issued, not where the value is staged.  Every load is issued, from an address that
@@ -399,14 +438,15 @@ memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k
     for (int u = 0; u < QK_REGS; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x / DP, r = x - tok * DP;
       const T* row = src + (size_t)(base + min(tok, count - 1)) * src_stride + (size_t)h * d + min(r, d - 1);
-      q_r[u] = row[q_off], k_r[u] = row[k_off];
+      if constexpr (RESULTS) q_r[u] = row[q_off];
+      k_r[u] = row[k_off];
     }
 #pragma unroll
     for (int u = 0; u < V_REGS; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x / MEMC_COLS, cc = blockIdx.x * MEMC_COLS + (x - tok * MEMC_COLS);
       const size_t at = (size_t)(base + min(tok, count - 1));
       v_r[u] = src[at * src_stride + v_off + (size_t)h * e + min(cc, e - 1)];
-      a_r[u] = scores[(at * heads + h) * MEMC_L + (x - tok * MEMC_COLS)];
+      if constexpr (RESULTS) a_r[u] = scores[(at * heads + h) * MEMC_L + (x - tok * MEMC_COLS)];
     }
     wd_r = *(const float2*)(wd + ((size_t)(base + min((int)threadIdx.x, count - 1)) * heads + h) * 2);
   };
@@ -418,13 +458,14 @@ memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k
     for (int u = 0; u < QK_REGS; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x / DP, r = x - tok * DP;
       const bool live = tok < count && r < d;
-      q_s[tok][r] = live ? raw_to_f32(q_r[u]) * q_scale : 0.f, k_s[tok][r] = live ? raw_to_f32(k_r[u]) : 0.f;
+      if constexpr (RESULTS) q_s[tok][r] = live ? raw_to_f32(q_r[u]) * q_scale : 0.f;
+      k_s[tok][r] = live ? raw_to_f32(k_r[u]) : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < V_REGS; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x / MEMC_COLS, cl = x - tok * MEMC_COLS, cc = blockIdx.x * MEMC_COLS + cl;
       v_s[tok][cl] = tok < count ? (cc < e ? raw_to_f32(v_r[u]) : (cc == e ? 1.f : 0.f)) : 0.f;
-      a_s[tok][cl] = tok < count ? a_r[u] : 0.f;
+      if constexpr (RESULTS) a_s[tok][cl] = tok < count ? a_r[u] : 0.f;
     }
     if (threadIdx.x < MEMC_L) {
       const bool live = (int)threadIdx.x < count;
@@ -433,10 +474,10 @@ memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k
     if (base + MEMC_L < t1) fetch(base + MEMC_L);  // on its way during this block's products
     lds_barrier();
     // what lies beyond the portion's end was staged as zeros, so every chain runs over the whole block
-    memc_acc part;
+    if constexpr (RESULTS) {
+      memc_acc part;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) part[r] = 0.f;
-    {
+      for (int r = 0; r < 16; ++r) part[r] = 0.f;
       // token c of the block, as this lane's row of the left operand: the state before the block, weighted
       const float dec = dec_s[c];
 #pragma unroll
@@ -462,6 +503,7 @@ memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k
         S = __builtin_amdgcn_mfma_f32_32x32x2f32(k_s[s][tile_row + c], w_s[s] * v_s[s][c], S, 0, 0, 0);
       }
     }
+    if constexpr (!RESULTS) continue;
     lds_barrier();
 
     for (int x = threadIdx.x; x < MEMC_L * MEMC_COLS; x += THREADS) {
@@ -480,7 +522,54 @@ memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int row = tile_row + 8 * (r / 4) + 4 * half + (r % 4);
-    if (col <= e && row < d_pad) st[row] = S[r];
+    if (PART == 1)
+      kept[row] = S[r];
+    else if (last && col <= e && row < d_pad)
+      st[row] = S[r];
+  }
+}
+
+// The states before a portion's segments from what each adds: S_(j+1) = exp(g_(c of j) - g_(end of j)) S_j + added_j, S_j in the
+// place of added_j.  A thread four adjacent rows of a column at a time; gridDim as the chunk kernel's, a portion in z.
+template <int TILES>
+__global__ void __launch_bounds__(CWM_WAVE * TILES)
+memory_join_kernel(const float* __restrict__ coef, const double* __restrict__ start, const float* __restrict__ state, long state_stride,
+                   long head_elems, const int* __restrict__ cu_q, const int* __restrict__ state_slots, float* __restrict__ saved, int heads,
+                   int e, int d_pad) {
+  constexpr int DP = 32 * TILES, QUADS = MEMC_COLS * DP / 4, EACH = QUADS / (CWM_WAVE * TILES);
+  const int h = blockIdx.y, b = blockIdx.z, t0 = cu_q[b], t1 = cu_q[b + 1];
+  if (t0 >= t1) return;
+  const int segments = (t1 - t0 + MEMS_L - 1) / MEMS_L;
+  const float* st = state + (size_t)state_slots[b] * state_stride + (size_t)h * head_elems;
+  const size_t head_size = (size_t)gridDim.x * MEMC_COLS * DP, step = head_size * heads;
+  float4* at = (float4*)(saved + ((size_t)(t0 / MEMS_L + b) * heads + h) * head_size + (size_t)blockIdx.x * MEMC_COLS * DP);
+  float4 now[EACH];
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    const int x = threadIdx.x + i * CWM_WAVE * TILES, col = blockIdx.x * MEMC_COLS + x / (DP / 4), row = 4 * (x % (DP / 4));
+    now[i] = col <= e && row < d_pad ? *(const float4*)(st + (size_t)col * d_pad + row) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  double g = start[(size_t)b * heads + h];
+  for (int j = 0; j < segments; ++j) {
+    float4 added[EACH];
+    float keep = 0.f;
+    if (j + 1 < segments) {
+#pragma unroll
+      for (int i = 0; i < EACH; ++i) added[i] = at[threadIdx.x + i * CWM_WAVE * TILES];
+      const float* cf = coef + ((size_t)(t0 + (j + 1) * MEMS_L - 1) * heads + h) * 4;
+      const double g_end = (double)cf[1] - *(const double*)(cf + 2);
+      keep = expf((float)(g - g_end));
+      g = g_end;
+    }
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) {
+      at[threadIdx.x + i * CWM_WAVE * TILES] = now[i];
+      if (j + 1 < segments) {
+        now[i].x = fmaf(keep, now[i].x, added[i].x), now[i].y = fmaf(keep, now[i].y, added[i].y);
+        now[i].z = fmaf(keep, now[i].z, added[i].z), now[i].w = fmaf(keep, now[i].w, added[i].w);
+      }
+    }
+    at += step / 4;
   }
 }
 
@@ -513,6 +602,13 @@ memory_out_kernel(const float* __restrict__ y, const float* __restrict__ nq, con
 }
 
 extern "C" int cwm_matrix_memory_block_tokens() { return MEMC_L; }
+extern "C" int cwm_matrix_memory_segment_tokens() { return MEMS_L; }
+
+static inline int memc_tiles(int d) { return d <= 32 ? 1 : d <= 64 ? 2 : d <= 128 ? 4 : 8; }
+
+extern "C" long cwm_matrix_memory_saved_floats(int n_tokens, int n_seqs, int heads, int d, int e) {
+  return (long)(n_tokens / MEMS_L + n_seqs) * heads * ((e + 1 + MEMC_COLS - 1) / MEMC_COLS * MEMC_COLS) * 32 * memc_tiles(d);
+}
 
 // src: the joined projection [n_tokens][src_stride] of dtype: q at column q_off (heads * d), k at k_off (heads * d), v at
 // v_off (heads * e), the output gate at g_off (heads * e).  gates: float32 [n_tokens][gates_stride], the input gates'
@@ -520,11 +616,12 @@ extern "C" int cwm_matrix_memory_block_tokens() { return MEMC_L; }
 // [slots][state_stride].  coef: float32 scratch [n_tokens][heads][4]; y: float32 scratch [n_tokens][heads * e].
 // out: [n_tokens][heads * e] of dtype.  With `start` (float64 scratch [n_seqs][heads]), `nq` (float32 scratch
 // [n_tokens][heads]) and `scores` (float32 scratch [n_tokens][heads][block tokens + 2]) the portions are taken in blocks of
-// tokens; without them they are walked token by token.
+// tokens; without them they are walked token by token.  With `saved` as well (float32 scratch, 16-byte aligned, of
+// `cwm_matrix_memory_saved_floats` floats) the blocks of long portions are walked in segments side by side.
 extern "C" int cwm_matrix_memory(const void* src, int dtype, long src_stride, int q_off, int k_off, int v_off, int g_off,
                                  const float* gates, long gates_stride, float cap, float q_scale, float* state, long state_stride,
                                  int n_slots, const int* cu_q, const int* state_slots, int n_seqs, int n_tokens,
-                                 float* coef, float* y, double* start, float* nq, float* scores, const float* weight, float eps,
+                                 float* coef, float* y, double* start, float* nq, float* scores, float* saved, const float* weight, float eps,
                                  void* out, int heads, int d, int e, hipStream_t stream) {
   CWM_REQUIRE(heads >= 1 && d >= 1 && e >= 1 && d <= MEM_MAX_DIM, "matrix_memory: heads of %d x %d: d must lie in 1..%d", d, e, MEM_MAX_DIM);
   CWM_REQUIRE(n_seqs >= 0 && n_tokens >= 0 && n_slots >= 1, "matrix_memory: bad counts");
@@ -538,6 +635,7 @@ extern "C" int cwm_matrix_memory(const void* src, int dtype, long src_stride, in
   CWM_REQUIRE((start == nullptr) == (nq == nullptr) && (start == nullptr) == (scores == nullptr) && ((uintptr_t)start % 8) == 0 &&
                   ((uintptr_t)scores % 8) == 0,
               "matrix_memory: all scratch arrays of the blocked form, or none");
+  CWM_REQUIRE(!saved || (start && ((uintptr_t)saved % 16) == 0), "matrix_memory: segments belong to the blocked form, their scratch is 16-byte aligned");
   if (n_seqs == 0 || n_tokens == 0) return 0;
   CWM_REQUIRE(n_seqs <= 65535, "matrix_memory: too many sequences for one launch");
   const int d_pad = MEM_ROWS * split;
@@ -548,14 +646,26 @@ extern "C" int cwm_matrix_memory(const void* src, int dtype, long src_stride, in
   const unsigned out_blocks = (unsigned)((n_pairs + MEM_THREADS / CWM_WAVE - 1) / (MEM_THREADS / CWM_WAVE));
   float* wd = scores ? scores + (size_t)n_tokens * heads * MEMC_L : nullptr;  // [n_tokens][heads][2] behind the scores
   const unsigned numbered = (unsigned)(n_tokens / MEMC_L + n_seqs);  // more than the largest number of a block of tokens
+  const unsigned segments = (unsigned)(n_tokens / MEMS_L + n_seqs);  // likewise
+  CWM_REQUIRE(!saved || segments <= 65535, "matrix_memory: too many segments for one launch");
+#define CWM_MEMORY_CHUNK(T, TILES, PART, Z)                                                                                 \
+  hipLaunchKernelGGL((memory_chunk_kernel<T, TILES, PART>), dim3(block_tiles, heads, Z), dim3(CWM_WAVE * TILES), 0, stream,  \
+                     (const T*)src, src_stride, q_off, k_off, v_off, q_scale, (const float*)scores, (const float*)wd,       \
+                     state, state_stride, head_elems, cu_q, state_slots, y, nq, saved, n_seqs, heads, d, e, d_pad)
 #define CWM_MEMORY_BLOCKS(T, RPT, TILES)                                                                                    \
   do {                                                                                                                      \
     hipLaunchKernelGGL((memory_scores_kernel<T, RPT>), dim3(numbered, heads), dim3(MEMC_THREADS), 0, stream, (const T*)src,  \
                        src_stride, q_off, k_off, q_scale, (const float*)coef, (const double*)start, cu_q, n_seqs, scores,   \
                        wd, heads, d);                                                                                       \
-    hipLaunchKernelGGL((memory_chunk_kernel<T, TILES>), dim3(block_tiles, heads, n_seqs), dim3(CWM_WAVE * TILES), 0, stream, \
-                       (const T*)src, src_stride, q_off, k_off, v_off, q_scale, (const float*)scores, (const float*)wd,     \
-                       state, state_stride, head_elems, cu_q, state_slots, y, nq, heads, d, e, d_pad);                      \
+    if (saved) {                                                                                                            \
+      CWM_MEMORY_CHUNK(T, TILES, 1, segments);                                                                              \
+      hipLaunchKernelGGL((memory_join_kernel<TILES>), dim3(block_tiles, heads, n_seqs), dim3(CWM_WAVE * TILES), 0, stream,   \
+                         (const float*)coef, (const double*)start, (const float*)state, state_stride, head_elems, cu_q,     \
+                         state_slots, saved, heads, e, d_pad);                                                              \
+      CWM_MEMORY_CHUNK(T, TILES, 2, segments);                                                                              \
+    } else {                                                                                                                \
+      CWM_MEMORY_CHUNK(T, TILES, 0, n_seqs);                                                                                \
+    }                                                                                                                       \
   } while (0)
 #define CWM_MEMORY(T)                                                                                                       \
   do {                                                                                                                      \
@@ -590,5 +700,6 @@ extern "C" int cwm_matrix_memory(const void* src, int dtype, long src_stride, in
     return cwm_fail("matrix_memory: unknown type %d", dtype);
 #undef CWM_MEMORY
 #undef CWM_MEMORY_BLOCKS
+#undef CWM_MEMORY_CHUNK
   return cwm_launch_status("matrix_memory");
 }
