@@ -456,20 +456,17 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __res
 }
 #undef TEAM
 
-// ---- prompt portions: 64 * LDS_RT rows per block, keys and values shared through LDS ------- //
+// ---- prompt portions: 64 * RT rows per block, keys and values shared through LDS ------- //
 // work item: {sequence, first row, first key, end key (exclusive), partial slot or -1, chunks of
 // the item}; one block per (item, key/value head); an item whose keys cross multiples of 8,192 is
-// cut there into several such blocks, which leave partial results for the merge kernel; wavefront w takes the LDS_RT tiles of 16 rows from first_row +
-// 16 * LDS_RT * w, and every operand it reads from LDS serves all of them.  Every 32-key tile of
+// cut there into several such blocks, which leave partial results for the merge kernel; wavefront w takes the RT tiles of 16 rows from first_row +
+// 16 * RT * w, and every operand it reads from LDS serves all of them.  Every 32-key tile of
 // keys and values is fetched once per block into LDS (two buffers) and read from there as
 // matrix-core operands:
 //   keys   [tile t][row m][HEAD_DIM + 8]: row m of 16-key tile t is key 8*(m/4) + 4*t + m%4, so
 //          the 16 lanes of one read take 16 consecutive padded rows (no bank conflicts);
 //   values [8-key block][dim][8]: as in the cache, 16 lanes read 256 contiguous bytes.
 // Keys outside the block's span of keys are stored as zeros, so nothing stale is multiplied.
-#ifndef LDS_RT
-#define LDS_RT 2  // 16-row tiles per wavefront: a block takes 64 * LDS_RT rows
-#endif
 #define LDS_K_STRIDE (HEAD_DIM + 8)
 #define LDS_K_CHUNKS (32 * HEAD_DIM / 8)
 #define LDS_V_CHUNKS (4 * HEAD_DIM)
@@ -507,7 +504,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __res
 // MIN_BLOCKS blocks share a compute unit.  With two (at most 256 registers a wavefront) or three
 // (168) the compiler keeps the matrix-core accumulators in ordinary vector registers; from the
 // accumulation registers every rescaling would cost a copy out and a copy back.
-template <int MODE, int DMA_BUFFERS, int MIN_BLOCKS>
+template <int RT, int MODE, int DMA_BUFFERS, int MIN_BLOCKS>
 __global__ void __launch_bounds__(256, MIN_BLOCKS)
 attention_lds_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __restrict__ out, long out_stride,
                      const bf16_t* __restrict__ cache, const int* __restrict__ block_table, int table_width,
@@ -543,21 +540,21 @@ attention_lds_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __rest
 
   const int n = lane & 15;
   const int j = lane >> 4;
-  // this wavefront's LDS_RT tiles of 16 rows; every key and value it reads from LDS serves all of them
-  bool row_valid[LDS_RT];
-  int ti[LDS_RT], hq[LDS_RT], row_end[LDS_RT], row_start[LDS_RT];
-  Frag8 qf[LDS_RT][K32_STEPS];
-  float4v acc[LDS_RT][D_TILES];
-  float m_run[LDS_RT], neg_mc_run[LDS_RT], l_run[LDS_RT];
+  // this wavefront's RT tiles of 16 rows; every key and value it reads from LDS serves all of them
+  bool row_valid[RT];
+  int ti[RT], hq[RT], row_end[RT], row_start[RT];
+  Frag8 qf[RT][K32_STEPS];
+  float4v acc[RT][D_TILES];
+  float m_run[RT], neg_mc_run[RT], l_run[RT];
 #ifdef DISTANCE_BIAS
-  float slope_raw[LDS_RT], rate[LDS_RT];
+  float slope_raw[RT], rate[RT];
 #endif
   const float neg_inf = -__builtin_inff();
   const float lazy_raw = 8.0f / scale_log2e;  // 8 binary orders, in units of the raw scores
   const float inv_cap_raw = cap_raw > 0.f ? 1.0f / cap_raw : 0.f;
 #pragma unroll
-  for (int rt = 0; rt < LDS_RT; ++rt) {
-    const int r = w[1] + 16 * (LDS_RT * wave + rt) + n;
+  for (int rt = 0; rt < RT; ++rt) {
+    const int r = w[1] + 16 * (RT * wave + rt) + n;
     row_valid[rt] = r < n_rows;
     ti[rt] = row_valid[rt] ? r / group : 0;
     hq[rt] = g * group + (row_valid[rt] ? r - ti[rt] * group : 0);
@@ -713,7 +710,7 @@ attention_lds_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __rest
   // the span of keys that any row of this wavefront reads, and the span that all of them read
   int lo_w = 0x7fffffff, hi_w = -1, lo_all = 0x7fffffff, hi_all = -1;
 #pragma unroll
-  for (int rt = 0; rt < LDS_RT; ++rt) {
+  for (int rt = 0; rt < RT; ++rt) {
     int lo = row_valid[rt] ? row_start[rt] : 0x7fffffff;
     int hi = row_valid[rt] ? row_end[rt] : -1;
     int lo_a = lo, hi_a = hi;
@@ -740,11 +737,11 @@ attention_lds_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __rest
     // a wavefront whose rows all end before this tile, or start after it, has nothing to add
     if (!(kt <= hi_w && (kt + 31 >= lo_w || IS_KEPT(kt)))) return;
     // ---- S^T = K Q^T ------------------------------------------------------------------ //
-    float4v st[LDS_RT][2];
+    float4v st[RT][2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
-      for (int rt = 0; rt < LDS_RT; ++rt) st[rt][t] = (float4v){0.f, 0.f, 0.f, 0.f};
+      for (int rt = 0; rt < RT; ++rt) st[rt][t] = (float4v){0.f, 0.f, 0.f, 0.f};
       const bf16_t* krow = kbuf + (t * 16 + n) * (MODE == LDS_DMA ? HEAD_DIM : LDS_K_STRIDE);
 #pragma unroll
       for (int s = 0; s < K32_STEPS; ++s) {
@@ -755,17 +752,17 @@ attention_lds_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __rest
         else
           kf.u = filled ? *(const uint4*)(krow + 8 * j + 32 * s) : make_uint4(0, 0, 0, 0);
 #pragma unroll
-        for (int rt = 0; rt < LDS_RT; ++rt)
+        for (int rt = 0; rt < RT; ++rt)
           st[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf.v, qf[rt][s].v, st[rt][t], 0, 0, 0);
       }
     }
     // ---- mask, running maximum, probabilities ------------------------------------------------ //
     const bool need_mask = kept || kt < lo_all || kt + 31 > hi_all;
-    float alpha[LDS_RT];
-    Frag8 pf[LDS_RT];
+    float alpha[RT];
+    Frag8 pf[RT];
     bool moved = false;
 #pragma unroll
-    for (int rt = 0; rt < LDS_RT; ++rt) {
+    for (int rt = 0; rt < RT; ++rt) {
       SOFTMAX_TILE(true, st[rt][0], st[rt][1], need_mask,
                    row_valid[rt] && key <= row_end[rt] && (kept ? key < kept_end : key >= row_start[rt] || (IS_KEPT(key) && key >= key_begin)), m_run[rt],
                    neg_mc_run[rt], l_run[rt], alpha[rt], pf[rt], slope_raw[rt], rate[rt], row_end[rt] - (kt + 8 * j))
@@ -774,7 +771,7 @@ attention_lds_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __rest
     if (__any(moved)) {  // seldom after the first tiles
       asm volatile("" ::: "memory");  // keeps this a branch: unconditional, it is 4 multiplications per output tile
 #pragma unroll
-      for (int rt = 0; rt < LDS_RT; ++rt)
+      for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int dt = 0; dt < D_TILES; ++dt) {
           acc[rt][dt][0] *= alpha[rt];
@@ -790,7 +787,7 @@ attention_lds_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __rest
       Frag8 vf;
       vf.u = *(const uint4*)(vrow + dt * 16 * 8);
 #pragma unroll
-      for (int rt = 0; rt < LDS_RT; ++rt) {
+      for (int rt = 0; rt < RT; ++rt) {
         acc[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf[rt].v, acc[rt][dt], 0, 0, 0);
       }
     }
@@ -805,7 +802,7 @@ attention_lds_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __rest
     // the queries arrive before the first of these loads: the compiler, which does not see them,
     // would otherwise wait for "everything" at the queries' first use inside the loop
 #pragma unroll
-    for (int rt = 0; rt < LDS_RT; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int s = 0; s < K32_STEPS; ++s)
         asm volatile("" : : "v"(qf[rt][s].u.x), "v"(qf[rt][s].u.y), "v"(qf[rt][s].u.z), "v"(qf[rt][s].u.w));
@@ -947,7 +944,7 @@ attention_lds_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __rest
   }
 
 #pragma unroll
-  for (int rt = 0; rt < LDS_RT; ++rt) {
+  for (int rt = 0; rt < RT; ++rt) {
     float l_row = l_run[rt];
     l_row += __shfl_xor(l_row, 16, 64);
     l_row += __shfl_xor(l_row, 32, 64);
@@ -955,7 +952,7 @@ attention_lds_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __rest
     if (w[4] >= 0) {
       // the item's keys are cut into w[5] chunks and this block had one of them: its row tile t
       // leaves what it has at slot w[4] + t * w[5], in the form of the split kernel's partial results
-      const int slot = w[4] + (LDS_RT * wave + rt) * w[5];
+      const int slot = w[4] + (RT * wave + rt) * w[5];
       float* prow = partial + (((size_t)slot * n_kv_heads + g) * 16 + n) * PARTIAL_STRIDE;
 #pragma unroll
       for (int dt = 0; dt < D_TILES; ++dt) *(float4v*)(prow + 16 * dt + 4 * j) = acc[rt][dt];
@@ -1094,7 +1091,7 @@ extern "C" int cwm_attention_mfma(const void* q, long q_stride, void* out, long 
   CWM_REQUIRE(chunk >= 0 && softcap >= 0.f && scale > 0.f, "attention_mfma: a block of keys and a cap cannot be negative, the scale is positive");
   const float cap_raw = softcap > 0.f ? softcap / scale : 0.f;
   // `work`: items of one 16-row tile (may be split over chunks of keys), one wavefront each;
-  // `work_wide`: items of 4 * LDS_RT row tiles, one block each with keys and values in LDS
+  // `work_wide`: items of `wide_tiles` row tiles (8, or 4 where the loads write LDS themselves), one block each with keys and values in LDS
   CWM_REQUIRE(head_dim == HEAD_DIM, "attention_mfma: this library is built for head_dim %d, not %d", HEAD_DIM, head_dim);
   CWM_REQUIRE(n_q_heads > 0 && n_kv_heads > 0 && n_q_heads % n_kv_heads == 0,
               "attention_mfma: %d query heads do not divide into %d key/value heads", n_q_heads, n_kv_heads);
@@ -1102,8 +1099,7 @@ extern "C" int cwm_attention_mfma(const void* q, long q_stride, void* out, long 
   CWM_REQUIRE(num_pages > 0 && table_width > 0, "attention_mfma: bad cache geometry");
   CWM_REQUIRE(q_stride % 8 == 0 && out_stride % 4 == 0, "attention_mfma: token strides must keep 16-byte alignment");
   CWM_REQUIRE(n_work >= 0 && n_work_wide >= 0 && n_merge >= 0, "attention_mfma: negative work counts");
-  CWM_REQUIRE(n_work_wide == 0 || wide_tiles == 4 * LDS_RT, "attention_mfma: wide items must have %d row tiles, not %d",
-              4 * LDS_RT, wide_tiles);
+  CWM_REQUIRE(n_work_wide == 0 || wide_tiles == 8 || wide_tiles == 4, "attention_mfma: wide items have 4 or 8 row tiles, not %d", wide_tiles);
   CWM_REQUIRE(n_merge == 0 || partial != nullptr, "attention_mfma: partial buffer missing");
   const float scale_log2e = scale * 1.4426950408889634f;
   int page_shift = -1;
@@ -1133,31 +1129,41 @@ extern "C" int cwm_attention_mfma(const void* q, long q_stride, void* out, long 
   if (n_work_wide > 0) {
     const long long blocks = (long long)n_work_wide * n_kv_heads;
     CWM_REQUIRE(blocks <= 0x7fffffffLL, "attention_mfma: too many work items");
-#define CWM_LAUNCH_LDS(MODE, BUFFERS, MIN_BLOCKS)                                                                        \
-  hipLaunchKernelGGL((attention_lds_kernel<MODE, BUFFERS, MIN_BLOCKS>), dim3((unsigned)blocks), dim3(256), 0, stream,     \
+#define CWM_LAUNCH_LDS(RT, MODE, BUFFERS, MIN_BLOCKS)                                                                        \
+  hipLaunchKernelGGL((attention_lds_kernel<RT, MODE, BUFFERS, MIN_BLOCKS>), dim3((unsigned)blocks), dim3(256), 0, stream,     \
                      (const bf16_t*)q, q_stride,                                                                          \
                      (bf16_t*)out, out_stride, (const bf16_t*)cache, block_table, table_width, cu_q, kv_len, work_wide,   \
                      partial, n_kv_heads, n_q_heads, n_kv_heads, page_size, page_shift, num_pages, window_left, chunk, scale_log2e, cap_raw, sink, out_scale BIAS_ARGS KEPT_ARGS)
+    if (wide_tiles == 4) {
+#if DMA_HEAD_DIM_OK
+      CWM_REQUIRE(page_size % 32 == 0 && (unsigned long long)n_kv_heads * page_size * HEAD_DIM * 2 < (1ull << 31),
+                  "attention_mfma: wide items of 4 row tiles need pages of a multiple of 32 keys, of less than 2 GiB");
+      constexpr int HALF_BLOCKS = HEAD_DIM > 128 ? 2 : 3;  // a compute unit's, and the buffers of each
+      CWM_LAUNCH_LDS(1, LDS_DMA, HALF_BLOCKS, HALF_BLOCKS);
+#else
+      return cwm_fail("attention_mfma: wide items of 4 row tiles are not built for head_dim %d", HEAD_DIM);
+#endif
+    } else
     // tiles of 32 keys that never straddle a page, and shares of a tile that divide evenly over the block
     if (page_size % 32 == 0 && LDS_K_CHUNKS % 256 == 0 && LDS_V_CHUNKS % 256 == 0) {
 #if DMA_HEAD_DIM_OK
       // the values' offset from the keys of a page must fit the loads' 32-bit offsets
       if ((unsigned long long)n_kv_heads * page_size * HEAD_DIM * 2 >= (1ull << 31))
-        CWM_LAUNCH_LDS(LDS_STAGED, 2, LDS_BLOCKS_A_UNIT);
+        CWM_LAUNCH_LDS(2, LDS_STAGED, 2, LDS_BLOCKS_A_UNIT);
 #if HEAD_DIM > 128
       else  // one block a compute unit, whose buffers fill 128 KB of its LDS
-        CWM_LAUNCH_LDS(LDS_DMA, 4, LDS_BLOCKS_A_UNIT);
+        CWM_LAUNCH_LDS(2, LDS_DMA, 4, LDS_BLOCKS_A_UNIT);
 #else
       else if (wide_three_blocks)  // the caller's choice: three blocks a compute unit
-        CWM_LAUNCH_LDS(LDS_DMA, 3, 3);
+        CWM_LAUNCH_LDS(2, LDS_DMA, 3, 3);
       else
-        CWM_LAUNCH_LDS(LDS_DMA, 4, 2);
+        CWM_LAUNCH_LDS(2, LDS_DMA, 4, 2);
 #endif
 #else
-      CWM_LAUNCH_LDS(LDS_STAGED, 2, LDS_BLOCKS_A_UNIT);
+      CWM_LAUNCH_LDS(2, LDS_STAGED, 2, LDS_BLOCKS_A_UNIT);
 #endif
     } else {
-      CWM_LAUNCH_LDS(LDS_PLAIN, 2, LDS_BLOCKS_A_UNIT);
+      CWM_LAUNCH_LDS(2, LDS_PLAIN, 2, LDS_BLOCKS_A_UNIT);
     }
 #undef CWM_LAUNCH_LDS
     status = cwm_launch_status("attention_lds");

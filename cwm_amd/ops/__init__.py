@@ -965,7 +965,7 @@ class _UploadedPlan:
     """A step's attention work lists on the device, and what the launch needs to know of them."""
 
     work: torch.Tensor  # items of one row tile
-    wide: torch.Tensor  # items of WIDE_TILES row tiles
+    wide: torch.Tensor  # items of `item_tiles` row tiles
     merge: torch.Tensor
     n_work: int
     n_wide: int
@@ -975,6 +975,7 @@ class _UploadedPlan:
     n_partials: int
     work_keys: int  # keys of an average item of one row tile
     wide_shape: Tuple[int, float]  # key tiles of the longest wide item, and the mean
+    item_tiles: int = WIDE_TILES  # row tiles of a wide item
 
 
 class StaticPlans:
@@ -1026,20 +1027,25 @@ class StaticPlans:
         return True
 
 
-def _attention_plan(batch, group: int, n_kv: int, head_dim: int, window: Optional[int], device: torch.device, chunk: Optional[int] = None) -> _UploadedPlan:
+def _attention_plan(
+    batch, group: int, n_kv: int, head_dim: int, window: Optional[int], device: torch.device, chunk: Optional[int] = None, halves: bool = False,
+) -> _UploadedPlan:
     """The step's work list for this (group size, key/value heads and their size, window or block of keys), uploaded once per step."""
-    from .attention_plan import build_plan, cuts_finer
+    from .attention_plan import build_plan, cuts_finer, wide_item_tiles
 
     finer = cuts_finer(n_kv, head_dim)
     static = getattr(batch, "static", None)
     if static is not None:
         return static.plan(batch, group, n_kv, window, chunk, finer)
-    key = ("attention_plan", group, n_kv, window, chunk, finer)
+    key = ("attention_plan", group, n_kv, window, chunk, finer, halves)
     cached = batch.scratch.get(key)
     if cached is None:
         # a sequence whose blocks of 128 rows, over all key/value heads, would not give every compute unit two
         wide_cut_below = -(-2 * _compute_units(device) // n_kv) if device.type == "cuda" else 0
-        plan = build_plan(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, chunk, finer)
+        item_tiles = WIDE_TILES
+        if device.type == "cuda" and halves:
+            item_tiles = wide_item_tiles(batch.q_lens, batch.kv_lens, group, n_kv, head_dim, wide_cut_below, _compute_units(device))
+        plan = build_plan(batch.q_lens, batch.kv_lens, group, window, wide_cut_below, chunk, finer, item_tiles)
         flat = np.concatenate([plan.work.reshape(-1), plan.work_wide.reshape(-1), plan.merge.reshape(-1)]).astype(np.int32)
         host = torch.from_numpy(flat)
         if device.type == "cuda":
@@ -1052,7 +1058,7 @@ def _attention_plan(batch, group: int, n_kv: int, head_dim: int, window: Optiona
             work=dev[:a], wide=dev[a:b], merge=dev[b:], n_work=n_work, n_wide=n_wide, n_merge=n_merge,
             n_merge_mid=plan.n_merge_mid, n_merge_wide=plan.n_merge_wide, n_partials=plan.n_partials,
             work_keys=int((plan.work[:, 3] - plan.work[:, 2]).mean()) if n_work else 0,
-            wide_shape=(int(wide_tiles.max()), float(wide_tiles.mean())) if n_wide else (0, 0.0),
+            wide_shape=(int(wide_tiles.max()), float(wide_tiles.mean())) if n_wide else (0, 0.0), item_tiles=item_tiles,
         )
         batch.scratch[key] = cached
     return cached
@@ -1125,7 +1131,9 @@ def paged_attention_mfma(
     _i32(block_table, "block_table")
     if block_table.dim() != 2 or block_table.shape[0] != batch.n_seqs or n_tokens != batch.n_tokens:
         raise KernelError("block_table must be [B, W] for the batch's sequences, q [T, ...] for its tokens")
-    plan = _attention_plan(batch, n_q // n_kv, n_kv, hd, window, q.device, chunk)
+    # whether blocks of 64 rows are built for these sizes: keys and values that the loads write to LDS themselves
+    halves = page_size % 32 == 0 and n_kv * page_size * hd * 2 < 2 ** 31
+    plan = _attention_plan(batch, n_q // n_kv, n_kv, hd, window, q.device, chunk, halves)
     out = torch.empty((n_tokens, n_q * hd), dtype=q.dtype, device=q.device)
     partial = None
     if plan.n_partials:
@@ -1142,7 +1150,7 @@ def paged_attention_mfma(
             _ptr(q), ctypes.c_long(q.stride(0)), _ptr(out), ctypes.c_long(n_q * hd), _ptr(cache),
             _ptr(block_table), ctypes.c_int(block_table.shape[1]), _ptr(batch.cu_q), _ptr(batch.kv_len),
             _ptr(plan.work), ctypes.c_int(plan.n_work), ctypes.c_int(plan.work_keys),
-            _ptr(plan.wide), ctypes.c_int(plan.n_wide), ctypes.c_int(WIDE_TILES),
+            _ptr(plan.wide), ctypes.c_int(plan.n_wide), ctypes.c_int(plan.item_tiles),
             ctypes.c_int(_three_blocks_a_unit(plan.n_wide * n_kv, plan.wide_shape, q.device)),
             _ptr(plan.merge), ctypes.c_int(plan.n_merge), ctypes.c_int(plan.n_merge_mid), ctypes.c_int(plan.n_merge_wide), _ptr(partial),
             ctypes.c_int(n_q), ctypes.c_int(n_kv), ctypes.c_int(hd), ctypes.c_int(page_size),

@@ -20,6 +20,12 @@ SPLIT_MAX_TILES = 8  # sequences with more row tiles than this are not split
 WIDE_TILES = 8  # row tiles (128 rows) of one block of the kernel that shares keys and values through LDS
 WIDE_CHUNK = 8192  # keys after which such a block's range is cut (at fixed absolute positions, like the others)
 WIDE_CHUNK_FINE = 2048  # the same for a sequence with very few such blocks
+# Most blocks of WIDE_TILES row tiles a compute unit, by the head size, of a launch that takes half as high ones instead.  Such a
+# block walks its keys alone, so with few blocks the longest one's walk is the launch: a tile of 32 keys costs it 1.4 us with 128
+# rows and 0.9 with 64, and twice as many blocks read keys from LDS.  Blocks of 128 rows, us with them and with 64 rows: heads of
+# 128 256 blocks 44 / 30, 512 66 / 54, 656 61 / 46, 672 27 / 26, 752 92 / 97, 1,024 155 / 169; of 64 920 38 / 28, 1,024 108 / 112, 2,048 173 /
+# 186; of 256 (two such blocks share a compute unit, of 128 rows one has it to itself) 256 128 / 73, 2,048 1,009 / 626.
+WIDE_HALF_BLOCKS = {64: 3.75, 128: 2.7, 256: float("inf")}
 
 
 def chunk_keys(n_keys, few_heads: bool = False):
@@ -76,12 +82,13 @@ def first_keys(last_key, window: Optional[int], chunk: Optional[int]):
 
 def build_plan(
     q_lens: Sequence[int], kv_lens: Sequence[int], group: int, window: Optional[int], wide_cut_below: int = 0,
-    chunk: Optional[int] = None, few_heads: bool = False,
+    chunk: Optional[int] = None, few_heads: bool = False, wide_tiles: int = WIDE_TILES,
 ) -> AttentionPlan:
     """`window` or `chunk` (at most one): which keys a query reads, see `first_keys`.  `wide_cut_below`: a sequence with fewer wide items than this has their keys cut at multiples of
     WIDE_CHUNK (its blocks alone would leave compute units idle), with fewer than an eighth of it at
     multiples of WIDE_CHUNK_FINE; the caller derives the number from the model's heads and the chip,
-    so that it is the same whatever else the batch holds.  `few_heads`: see `chunk_keys`."""
+    so that it is the same whatever else the batch holds.  `few_heads`: see `chunk_keys`.  `wide_tiles`: row tiles of a wide
+    item, WIDE_TILES or what `wide_item_tiles` answers (a sequence's items are counted in the former where that decides on a cut)."""
     q = np.asarray(q_lens, dtype=np.int64)
     kv = np.asarray(kv_lens, dtype=np.int64)
     n_rows = q * group
@@ -93,14 +100,15 @@ def build_plan(
     for b in np.nonzero(is_wide)[0]:
         lo, hi, row0 = _tile_ranges(int(q[b]), int(kv[b]), int(n_tiles[b]), group, window, chunk)
         n_wide = (int(n_tiles[b]) + WIDE_TILES - 1) // WIDE_TILES
-        first = np.arange(n_wide) * WIDE_TILES
-        last = np.minimum(first + WIDE_TILES - 1, int(n_tiles[b]) - 1)
-        wide_seq.append(np.full(n_wide, b, dtype=np.int64))
+        n_items = (int(n_tiles[b]) + wide_tiles - 1) // wide_tiles
+        first = np.arange(n_items) * wide_tiles
+        last = np.minimum(first + wide_tiles - 1, int(n_tiles[b]) - 1)
+        wide_seq.append(np.full(n_items, b, dtype=np.int64))
         wide_row0.append(row0[first])
         wide_lo.append(lo[first])
         wide_hi.append(hi[last])
         wide_n_tiles.append(last - first + 1)
-        wide_cut.append(np.full(n_wide, 0 if n_wide >= wide_cut_below else (WIDE_CHUNK if 8 * n_wide >= wide_cut_below else WIDE_CHUNK_FINE)))
+        wide_cut.append(np.full(n_items, 0 if n_wide >= wide_cut_below else (WIDE_CHUNK if 8 * n_wide >= wide_cut_below else WIDE_CHUNK_FINE)))
 
     # ---- all tiles of the other sequences at once, in the order (sequence, tile, chunk)
     small = np.nonzero(~is_wide)[0]
@@ -187,6 +195,22 @@ def build_plan(
         n_merge_wide=n_merge_wide,
         n_merge_mid=n_merge_mid,
     )
+
+
+def wide_item_tiles(q_lens: Sequence[int], kv_lens: Sequence[int], group: int, n_kv: int, head_dim: int, wide_cut_below: int, units: int) -> int:
+    """Row tiles of a wide item for a step of these lengths on `units` compute units: half of WIDE_TILES where blocks of
+    WIDE_TILES are few (`WIDE_HALF_BLOCKS`; other head sizes have no such blocks).  A row's bits are the same either way unless
+    its keys are cut, so a step with a cut sequence keeps the whole size."""
+    blocks, most = 0, WIDE_HALF_BLOCKS.get(head_dim, 0) * units
+    for q, kv in zip(q_lens, kv_lens):
+        n_tiles = -(-q * group // ROWS_PER_TILE)
+        if n_tiles <= SPLIT_MAX_TILES:
+            continue
+        n_wide = -(-n_tiles // WIDE_TILES)
+        if n_wide < wide_cut_below and kv > (WIDE_CHUNK if 8 * n_wide >= wide_cut_below else WIDE_CHUNK_FINE):
+            return WIDE_TILES
+        blocks += n_wide * n_kv
+    return WIDE_TILES // 2 if 0 < blocks <= most else WIDE_TILES
 
 
 def _tile_ranges(n_new: int, kv: int, n_tiles: int, group: int, window: Optional[int], chunk: Optional[int] = None):
