@@ -353,6 +353,90 @@ __global__ void __launch_bounds__(1024) group_by_expert_kernel(const int* __rest
   group_pairs(chosen, n_pairs, n_experts, row_token, pair_row, tile_expert, used, n_tiles, top, tile_align, count, start);
 }
 
+// Few tokens (a decode step): the router's product, the choice and the grouping in one launch of one block, each of which is a few
+// microseconds of latency as a launch of its own (eight tokens, 16 experts, K = 2,048: 4.8 + 4.4 + 4.3 us).  The
+// product is that of gemm_bf16_stream.hip on one tile of columns after the other, its sums in the same order: the 16 wavefronts
+// share K, and add their parts through LDS.  w: the router's streaming copy [tiles of 16 experts][K / 32][64][8].
+#define ROUTE_GROUP_TOKENS 16
+#define ROUTE_GROUP_STEPS 16  // of 32 along K, at most, a wavefront
+
+__global__ void __launch_bounds__(1024) route_group_kernel(const bf16_t* __restrict__ x, long x_ld, const bf16_t* __restrict__ w,
+                                                           const float* __restrict__ bias, int K, int n_tokens, int n_experts, int top, int mode,
+                                                           const float* __restrict__ correction, float scale, int renormalize, int n_groups,
+                                                           int keep_groups, int* __restrict__ chosen, float* __restrict__ weights,
+                                                           int* __restrict__ row_token, int* __restrict__ pair_row, int* __restrict__ tile_expert,
+                                                           int* __restrict__ used, int n_tiles, int tile_align) {
+  __shared__ __attribute__((aligned(16))) float parts[16][256];
+  __shared__ float logits[ROUTE_GROUP_TOKENS][CWM_WAVE];
+  __shared__ int picks[ROUTE_GROUP_TOKENS * ROUTE_MAX_TOP];
+  __shared__ int count[ROUTE_MAX_EXPERTS], start[ROUTE_MAX_EXPERTS];
+  const int lane = threadIdx.x & (CWM_WAVE - 1), wave = threadIdx.x / CWM_WAVE;
+  const int r = lane & 15, j = lane >> 4;
+  const int steps = K / 32, each = (steps + 15) / 16, first = wave * each, last = min(steps, first + each);
+  const bf16_t* row = x + (size_t)min(r, n_tokens - 1) * x_ld + 8 * j;
+  for (int n0 = 0; n0 < n_experts; n0 += 16) {
+    const bf16_t* tile = w + ((size_t)(n0 / 16) * steps * 64 + lane) * 8;
+    float4v acc = (float4v){0.f, 0.f, 0.f, 0.f};
+    for (int s = first; s < last; s += 4) {
+      Frag8 fx[4], fw[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int at = min(s + u, last - 1);
+        fx[u].u = *(const uint4*)(row + 32 * at);
+        fw[u].u = *(const uint4*)(tile + (size_t)at * 512);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (s + u < last) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[u].v, fx[u].v, acc, 0, 0, 0);
+    }
+    __syncthreads();
+    *(float4v*)&parts[wave][r * 16 + 4 * j] = acc;  // [token][expert]
+    __syncthreads();
+    if (threadIdx.x < 256) {
+      float sum = 0.f;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) sum += parts[v][threadIdx.x];
+      const int e = n0 + (threadIdx.x & 15);
+      if (bias && e < n_experts) sum += bias[e];
+      logits[threadIdx.x >> 4][e] = sum;
+    }
+  }
+  __syncthreads();
+  if (wave < n_tokens)
+    route_few(lane < n_experts ? logits[wave][lane] : -__builtin_inff(), lane, n_experts, top, mode, correction, scale, renormalize, n_groups,
+              keep_groups, picks + wave * top, weights + (size_t)wave * top);
+  __syncthreads();
+  for (int i = threadIdx.x; i < n_tokens * top; i += blockDim.x) chosen[i] = picks[i];
+  group_pairs(picks, n_tokens * top, n_experts, row_token, pair_row, tile_expert, used, n_tiles, top, tile_align, count, start);
+}
+
+extern "C" int cwm_route_group_tokens() { return ROUTE_GROUP_TOKENS; }
+extern "C" int cwm_route_group_max_k() { return 16 * 32 * ROUTE_GROUP_STEPS; }
+
+// x: bfloat16 [n_tokens][x_ld]; w: the router's streaming copy; bias: float32 [n_experts] or null; the choice as in
+// `cwm_route_top` for at most 64 experts, the lists as in `cwm_group_by_expert`.
+extern "C" int cwm_route_group(const void* x, long x_ld, const void* w, const float* bias, int K, int n_tokens, int n_experts, int top, int mode,
+                               const float* correction, float scale, int renormalize, int n_groups, int keep_groups, int* chosen,
+                               float* weights, int* row_token, int* pair_row, int* tile_expert, int* used, int n_tiles, int tile_align,
+                               hipStream_t stream) {
+  CWM_REQUIRE(x && w && chosen && weights && row_token && pair_row && tile_expert && used, "route_group: arguments missing");
+  CWM_REQUIRE(n_tokens >= 0 && n_tokens <= ROUTE_GROUP_TOKENS, "route_group: %d tokens, the kernel takes up to %d", n_tokens, ROUTE_GROUP_TOKENS);
+  CWM_REQUIRE(n_experts >= 1 && n_experts <= CWM_WAVE && top >= 1 && top <= ROUTE_MAX_TOP && top <= n_experts, "route_group: %d of %d experts, the kernel takes up to %d of %d",
+              top, n_experts, ROUTE_MAX_TOP, CWM_WAVE);
+  CWM_REQUIRE(K >= 32 && K % 32 == 0 && K <= 16 * 32 * ROUTE_GROUP_STEPS && x_ld >= K && x_ld % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0,
+              "route_group: rows of %d elements must be a multiple of 32, up to %d, at multiples of 16 bytes", K, 16 * 32 * ROUTE_GROUP_STEPS);
+  CWM_REQUIRE(mode == 0 || mode == 1, "route_group: unknown mode %d", mode);
+  CWM_REQUIRE(n_groups >= 1 && n_experts % n_groups == 0 && keep_groups >= 1 && keep_groups <= n_groups && top <= keep_groups * (n_experts / n_groups),
+              "route_group: %d of %d groups of %d experts do not hold %d choices", keep_groups, n_groups, n_experts, top);
+  CWM_REQUIRE(tile_align >= 1 && (long)n_tiles >= ((long)n_tokens * top + TILE_ROWS - 1) / TILE_ROWS + (long)n_experts * tile_align,
+              "route_group: %d tiles do not hold %d pairs of %d experts", n_tiles, n_tokens * top, n_experts);
+  if (n_tokens == 0) return 0;
+  hipLaunchKernelGGL(route_group_kernel, dim3(1), dim3(1024), 0, stream, (const bf16_t*)x, x_ld, (const bf16_t*)w, bias, K, n_tokens, n_experts, top,
+                     mode, correction, scale, renormalize, n_groups, keep_groups, chosen, weights, row_token, pair_row, tile_expert, used, n_tiles,
+                     tile_align);
+  return cwm_launch_status("route_group");
+}
+
 // used: one number, the tiles up to the last one that has rows, rounded up to tile_align.  tile_align: an expert's first tile lies at a multiple of so many tiles (the tiles that one block of the product takes).
 extern "C" int cwm_group_by_expert(const int* chosen, int n_tokens, int top, int n_experts, int* row_token, int* pair_row,
                                    int* tile_expert, int* used, int n_tiles, int tile_align, hipStream_t stream) {

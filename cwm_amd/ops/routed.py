@@ -31,6 +31,23 @@ def _base():
     return KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream
 
 
+def _check_scores(scores: str, correction: Optional[torch.Tensor], scale: float, renormalize: bool, n_experts: int) -> None:
+    KernelError = _base()[0]
+    if scores not in ("softmax_chosen", "softmax_all"):
+        raise KernelError(f"router scores {scores!r}: 'softmax_chosen' and 'softmax_all' are known")
+    if scores == "softmax_chosen" and (correction is not None or scale != 1.0 or renormalize):
+        raise KernelError("a correction, a scale and renormalised weights belong to router scores over all experts")
+    if correction is not None and (correction.dtype != torch.float32 or correction.shape != (n_experts,) or not correction.is_contiguous()):
+        raise KernelError("the router's correction must be a contiguous float32 tensor, one value an expert")
+
+
+def _open_groups(groups: Optional[Tuple[int, int]], n_experts: int, top: int) -> Tuple[int, int]:
+    count, keep = groups if groups is not None else (1, 1)
+    if count < 1 or n_experts % count != 0 or not 1 <= keep <= count or top > keep * (n_experts // count):
+        raise _base()[0](f"{keep} of {count} groups of {n_experts} experts do not hold {top} choices")
+    return count, keep
+
+
 def route_top(
     logits: torch.Tensor, top: int, scores: str = "softmax_chosen", correction: Optional[torch.Tensor] = None, scale: float = 1.0,
     renormalize: bool = False, groups: Optional[Tuple[int, int]] = None,
@@ -44,20 +61,13 @@ def route_top(
     only those of the `keep` groups with the best members can be chosen."""
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
     _need_gpu(logits, correction)
-    if scores not in ("softmax_chosen", "softmax_all"):
-        raise KernelError(f"router scores {scores!r}: 'softmax_chosen' and 'softmax_all' are known")
-    if scores == "softmax_chosen" and (correction is not None or scale != 1.0 or renormalize):
-        raise KernelError("a correction, a scale and renormalised weights belong to router scores over all experts")
-    if correction is not None and (correction.dtype != torch.float32 or correction.shape != (logits.shape[-1],) or not correction.is_contiguous()):
-        raise KernelError("the router's correction must be a contiguous float32 tensor, one value an expert")
+    _check_scores(scores, correction, scale, renormalize, logits.shape[-1])
     if logits.dtype != torch.float32 or logits.dim() != 2 or not logits.is_contiguous():
         raise KernelError("router logits must be a contiguous float32 [T, E] tensor")
     n, e = logits.shape
     if not 1 <= top <= min(e, MAX_ROUTE_TOP):
         raise KernelError(f"{top} of {e} experts: the kernel takes 1..{min(e, MAX_ROUTE_TOP)}")
-    count, keep = groups if groups is not None else (1, 1)
-    if count < 1 or e % count != 0 or not 1 <= keep <= count or top > keep * (e // count):
-        raise KernelError(f"{keep} of {count} groups of {e} experts do not hold {top} choices")
+    count, keep = _open_groups(groups, e, top)
     chosen = torch.empty((n, top), dtype=torch.int32, device=logits.device)
     weights = torch.empty((n, top), dtype=torch.float32, device=logits.device)
     lib = _build.load("routed")
@@ -96,6 +106,58 @@ def _product_tiles(dtype: torch.dtype, k: int, rows: float, gated: bool) -> int:
     return 1 if gated and rows < STREAM_ROWS else _tiles_a_block(rows)
 
 
+def _empty_groups(n: int, top: int, n_experts: int, device: torch.device) -> ExpertGroups:
+    pairs = n * top
+    align = _tiles_a_block(pairs / n_experts)
+    n_tiles = -(-pairs // TILE_ROWS) + n_experts * align
+    lists = torch.empty(n_tiles * TILE_ROWS + pairs + n_tiles + 1, dtype=torch.int32, device=device)
+    row_token, pair_row, tile_expert, used = lists.split_with_sizes((n_tiles * TILE_ROWS, pairs, n_tiles, 1))
+    return ExpertGroups(row_token, pair_row, tile_expert, n_tiles, align, top, used)
+
+
+ROUTE_GROUP_TOKENS = 16  # csrc/routed.hip: ROUTE_GROUP_TOKENS
+ROUTE_GROUP_EXPERTS = 64
+ROUTE_GROUP_MAX_K = 8192  # csrc/routed.hip: 16 * 32 * ROUTE_GROUP_STEPS
+
+
+def route_and_group(
+    x: torch.Tensor, router_copy: torch.Tensor, bias: Optional[torch.Tensor], n_experts: int, top: int, scores: str = "softmax_chosen",
+    correction: Optional[torch.Tensor] = None, scale: float = 1.0, renormalize: bool = False, groups: Optional[Tuple[int, int]] = None,
+) -> Tuple[torch.Tensor, torch.Tensor, ExpertGroups]:
+    """(chosen, weights, lists): what `route_top` and `group_by_expert` make of the logits W x + bias, in one launch, the same bits.
+    `x` bfloat16 [T <= 16, K] (K a multiple of 32, up to 8,192), `router_copy` the streaming copy (`stream_layout`) of the
+    bfloat16 router [E <= 64, K], `bias` float32 [E] or None; the rest as in `route_top`."""
+    KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
+    _need_gpu(x, router_copy, bias, correction)
+    _check_scores(scores, correction, scale, renormalize, n_experts)
+    if x.dim() != 2 or x.dtype != torch.bfloat16 or x.stride(1) != 1 or x.shape[0] > ROUTE_GROUP_TOKENS:
+        raise KernelError(f"x must be bfloat16 [T <= {ROUTE_GROUP_TOKENS}, K] with contiguous rows")
+    n, k = x.shape
+    if not 1 <= n_experts <= ROUTE_GROUP_EXPERTS or k % 32 != 0 or k > ROUTE_GROUP_MAX_K:
+        raise KernelError(f"{n_experts} experts of rows of {k}: the kernel takes up to {ROUTE_GROUP_EXPERTS}, rows of a multiple of 32 up to {ROUTE_GROUP_MAX_K}")
+    if router_copy.dtype != torch.bfloat16 or tuple(router_copy.shape) != (-(-n_experts // 16), k // 32, 64, 8) or not router_copy.is_contiguous():
+        raise KernelError(f"the router's streaming copy {tuple(router_copy.shape)} does not fit {n_experts} experts of rows of {k}")
+    if bias is not None and (bias.dtype != torch.float32 or bias.shape != (n_experts,) or not bias.is_contiguous()):
+        raise KernelError("the router's bias must be a contiguous float32 tensor, one value an expert")
+    if not 1 <= top <= min(n_experts, MAX_ROUTE_TOP):
+        raise KernelError(f"{top} of {n_experts} experts: the kernel takes 1..{min(n_experts, MAX_ROUTE_TOP)}")
+    count, keep = _open_groups(groups, n_experts, top)
+    chosen = torch.empty((n, top), dtype=torch.int32, device=x.device)
+    weights = torch.empty((n, top), dtype=torch.float32, device=x.device)
+    lists = _empty_groups(n, top, n_experts, x.device)
+    lib = _build.load("routed")
+    _check(
+        lib,
+        lib.cwm_route_group(
+            _ptr(x), ctypes.c_long(x.stride(0) if n > 1 else k), _ptr(router_copy), _ptr(bias), ctypes.c_int(k), ctypes.c_int(n), ctypes.c_int(n_experts),
+            ctypes.c_int(top), ctypes.c_int(int(scores == "softmax_all")), _ptr(correction), ctypes.c_float(scale), ctypes.c_int(int(renormalize)),
+            ctypes.c_int(count), ctypes.c_int(keep), _ptr(chosen), _ptr(weights), _ptr(lists.row_token), _ptr(lists.pair_row), _ptr(lists.tile_expert),
+            _ptr(lists.used), ctypes.c_int(lists.n_tiles), ctypes.c_int(lists.tiles_a_block), _stream(),
+        ),
+    )
+    return chosen, weights, lists
+
+
 def group_by_expert(chosen: torch.Tensor, n_experts: int) -> ExpertGroups:
     """Group the pairs of `chosen` (int32 [T, top]) by expert.  The lists have a size that depends on T, top and
     the number of experts alone, so no count has to come to the host."""
@@ -107,12 +169,8 @@ def group_by_expert(chosen: torch.Tensor, n_experts: int) -> ExpertGroups:
     if not 1 <= n_experts <= MAX_EXPERTS:
         raise KernelError(f"{n_experts} experts: the kernel takes up to {MAX_EXPERTS}")
     n, top = chosen.shape
-    pairs = n * top
-    align = _tiles_a_block(pairs / n_experts)
-    n_tiles = -(-pairs // TILE_ROWS) + n_experts * align
-    lists = torch.empty(n_tiles * TILE_ROWS + pairs + n_tiles + 1, dtype=torch.int32, device=chosen.device)
-    row_token, pair_row, tile_expert, used = lists.split_with_sizes((n_tiles * TILE_ROWS, pairs, n_tiles, 1))
-    groups = ExpertGroups(row_token, pair_row, tile_expert, n_tiles, align, top, used)
+    groups = _empty_groups(n, top, n_experts, chosen.device)
+    n_tiles, align = groups.n_tiles, groups.tiles_a_block
     lib = _build.load("routed")
     _check(
         lib,

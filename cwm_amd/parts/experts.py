@@ -82,6 +82,13 @@ class RoutedExperts(FeedForward):
         if self.shared is not None:
             n = len(self.shared_prefix)
             self.shared.bind({name[n:]: t for name, t in tensors.items() if name.startswith(self.shared_prefix)}, runtime)
+        # the streaming copy of a small router: a step of few tokens makes its logits, choices and lists in one launch from it
+        self.router_copy: Optional[torch.Tensor] = None
+        if (
+            runtime.device.type == "cuda" and runtime.act_dtype == torch.bfloat16 and self.router.dtype == torch.bfloat16
+            and self.n_experts <= ops.ROUTE_GROUP_EXPERTS and self.dim % 32 == 0 and self.dim <= ops.ROUTE_GROUP_MAX_K
+        ):
+            self.router_copy = ops.stream_layout(self.router)
         self.choice_correction = tensors["correction"].float().contiguous() if self.correction else None
         # [experts, out, in], or, where the matrix cores read them as they lie in memory, in operand tiles (a layout; the same size)
         tiles = (
@@ -102,9 +109,12 @@ class RoutedExperts(FeedForward):
     def forward_deferred(self, x: torch.Tensor, batch: Any) -> "ops.RoutedSum":
         """The same without the last kernel: every pair's row and the weights, for a consumer that adds a token's
         rows up itself (a norm that takes a `RoutedSum` as the pending result)."""
-        logits = ops.linear(x, self.router, self.router_b, torch.float32)
-        chosen, weights = ops.route_top(logits, self.top, self.scores, self.choice_correction, self.weight_scale, self.renormalize, self.groups)
-        groups = ops.group_by_expert(chosen, self.n_experts)
+        router = (self.top, self.scores, self.choice_correction, self.weight_scale, self.renormalize, self.groups)
+        if self.router_copy is not None and x.shape[0] <= ops.ROUTE_GROUP_TOKENS and x.data_ptr() % 16 == 0:
+            _, weights, groups = ops.route_and_group(x, self.router_copy, self.router_b, self.n_experts, *router)
+        else:
+            chosen, weights = ops.route_top(ops.linear(x, self.router, self.router_b, torch.float32), *router)
+            groups = ops.group_by_expert(chosen, self.n_experts)
         if self.activation.kind == "silu":
             hidden = ops.grouped_gate_up(x, groups, self.gate, self.up)
         else:
