@@ -487,21 +487,53 @@ __global__ void __launch_bounds__(256) selective_scan_single_kernel(const T* __r
 // token t, S the state before the block, and everything per head:
 //       y_t = e^(L_t) S^T C_t + sum_(s <= t) (C_t . B_s) dt_s e^(L_t - L_s) x_s + D x_t
 //       S  <- e^(L_end) S + sum_s B_s (e^(L_end - L_s) dt_s x_s)^T
-// C_t . B_s are products of bfloat16 values (exact, float32 sums); the other products have float32 operands
-// (v_mfma_f32_16x16x4_f32) and so no value is rounded that the walk keeps.  The L are summed in float64: a difference of two
+// C_t . B_s are products of bfloat16 values (exact, float32 sums).  The other products have one float32 operand each (S, the
+// weighted x, the scores), which goes in as three bfloat16 parts that hold all its bits, so that every single product is exact
+// and no value is rounded that the walk keeps: three v_mfma_f32_16x16x32_bf16 of 16 cycles for eight v_mfma_f32_16x16x4_f32 of
+// 32 (2,048 tokens 154 us with those, 3.8e-7 off float64 instead of 2.4e-7).  The L are summed in float64: a difference of two
 // of them is as exact as the decays between them.  A wavefront has 16 columns of the head: its part of the state stays in
-// registers as the matrix instruction leaves it (lane 16 j + r: column r, rows 16 q + 4 j + i), which is also the operand that
-// C needs; a score's lane (query r, keys 4 j + i) is likewise the operand that x needs.
+// registers as the matrix instruction leaves it (lane 16 j + r: column r, rows 16 q + 4 j + i), and two such tiles are also the
+// operand that C needs, with its values of k in the order 4 j + i, 16 + 4 j + i; likewise two tiles of x.  The other operand is
+// read from LDS in that order.
 // MODE 1 leaves the state that every segment but a sequence's last makes from zero, and the segment's decay; then
 // `scan_carry_kernel` turns those into the states at the segments' starts; MODE 2 walks every segment from there and writes y.
 // Portions of one segment, decoded tokens among them, are left to the walk: their bits and their cost are what they are without a
 // long portion beside them (in blocks a decoded token pays for 64).
-// Bound by the float32 matrix instructions (110k of a compute unit's cycles at 2,048 tokens of 64 heads, 64 columns, 128 rows)
-// and by the waits between a block's stages, two blocks a compute unit; the walk was bound by its reads of B and C from LDS.
+// Bound by the waits between a block's stages, two blocks a compute unit (three in MODE 1; asked for, since the registers beyond
+// the first 256 would leave one), and by splitting values on the vector units; the walk was bound by its reads of B and C from LDS.
 #define BLOCK_TOKENS 64
 
-template <int NT, int MODE>  // NT: tiles of 16 rows of the state
-__global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ dt_raw, long dt_ld,
+// Eight float32 values as the operands of three bfloat16 matrix products whose sum is the product of the values: each part is
+// the leading eight bits of what the parts before leave, so three hold all 24, and with a bfloat16 second operand every single
+// product is exact.  An infinity or a NaN is its first part alone.
+__device__ __forceinline__ void three_parts(const float (&v)[8], Frag8 (&part)[3]) {
+  uint32_t w[3][8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t bits = __float_as_uint(v[e]);
+    w[0][e] = bits;
+    float rest = v[e] - __uint_as_float(bits & 0xffff0000u);
+    rest = (bits & 0x7f800000u) == 0x7f800000u ? 0.f : rest;
+    w[1][e] = __float_as_uint(rest);
+    w[2][e] = __float_as_uint(rest - __uint_as_float(w[1][e] & 0xffff0000u));
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    part[k].u = make_uint4(__builtin_amdgcn_perm(w[k][1], w[k][0], 0x07060302u), __builtin_amdgcn_perm(w[k][3], w[k][2], 0x07060302u),
+                           __builtin_amdgcn_perm(w[k][5], w[k][4], 0x07060302u), __builtin_amdgcn_perm(w[k][7], w[k][6], 0x07060302u));
+}
+
+// Sixteen bytes of an operand whose eight values of k are 4 j .. + 3 and 16 + 4 j .. + 3 of 32: the order in which two tiles of a
+// matrix instruction's result hold them.
+__device__ __forceinline__ Frag8 two_fours(const bf16_t* at) {
+  const uint2 low = *(const uint2*)at, high = *(const uint2*)(at + 16);
+  Frag8 f;
+  f.u = make_uint4(low.x, low.y, high.x, high.y);
+  return f;
+}
+
+template <int NT, int MODE>  // NT: tiles of 16 rows of the state (even)
+__global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ dt_raw, long dt_ld,
                                                          const float* __restrict__ dt_bias, const float* __restrict__ a_log,
                                                          const float* __restrict__ d_skip, float* __restrict__ state, long state_ld,
                                                          const int* __restrict__ slots, float* __restrict__ y, int heads, int P, int N, int groups,
@@ -509,11 +541,12 @@ __global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restric
                                                          float* __restrict__ seg_decay) {
   constexpr int ROWS = 16 * NT, PIECES = ROWS / 8, LOADS = BLOCK_TOKENS * PIECES / 256;
   constexpr int ROW_LD = ROWS + 8, COL_LD = BLOCK_TOKENS + 8, SCORE_LD = BLOCK_TOKENS + 4;
+  static_assert(NT % 2 == 0, "the state's rows go into products of 32");
   typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(16))) bf16_t b_rows[MODE == 2 ? BLOCK_TOKENS : 1][ROW_LD];
   __shared__ __attribute__((aligned(16))) bf16_t c_rows[MODE == 2 ? BLOCK_TOKENS : 1][ROW_LD];
   __shared__ __attribute__((aligned(16))) bf16_t b_cols[ROWS][COL_LD];
-  __shared__ __attribute__((aligned(16))) float scores[MODE == 2 ? BLOCK_TOKENS : 1][SCORE_LD];
+  __shared__ __attribute__((aligned(16))) bf16_t scores[MODE == 2 ? 3 : 1][MODE == 2 ? BLOCK_TOKENS : 1][SCORE_LD];  // in three parts
   __shared__ double sum_log[BLOCK_TOKENS];
   __shared__ __attribute__((aligned(16))) float step_size[BLOCK_TOKENS], from_start[BLOCK_TOKENS], to_end[BLOCK_TOKENS];
   const int* entry = segments + 6 * blockIdx.z;
@@ -579,7 +612,9 @@ __global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restric
       for (int e = 0; e < 8; ++e) b_cols[n + e][lane] = (bf16_t)(rb[k][e >> 1] >> (16 * (e & 1)));
     }
     float x[16];
-    uint32_t largest = 0;
+    uint32_t rx_now[8], largest = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) rx_now[k] = rx[k];  // (the next block's come into rx meanwhile)
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       x[k] = __uint_as_float(k & 1 ? rx[k >> 1] & 0xffff0000u : rx[k >> 1] << 16);
@@ -625,21 +660,38 @@ __global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restric
           const int key = 16 * b + 4 * j + i;
           acc[i] = key <= t ? acc[i] * dts[i] * expf((float)(mine - sum_log[key])) : 0.f;
         }
-        *(float4v*)&scores[t][16 * b + 4 * j] = acc;
+        uint32_t w[3][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          w[0][i] = __float_as_uint(acc[i]);
+          float rest = acc[i] - __uint_as_float(w[0][i] & 0xffff0000u);
+          rest = (w[0][i] & 0x7f800000u) == 0x7f800000u ? 0.f : rest;
+          w[1][i] = __float_as_uint(rest);
+          w[2][i] = __float_as_uint(rest - __uint_as_float(w[1][i] & 0xffff0000u));
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          *(uint2*)&scores[k][t][16 * b + 4 * j] =
+              make_uint2(__builtin_amdgcn_perm(w[k][1], w[k][0], 0x07060302u), __builtin_amdgcn_perm(w[k][3], w[k][2], 0x07060302u));
       }
+      if (wave % 2 == 0)  // keys go in pairs of tiles
+#pragma unroll
+        for (int k = 0; k < 3; ++k) *(uint2*)&scores[k][t][16 * (wave + 1) + 4 * j] = make_uint2(0u, 0u);
       __syncthreads();
       if (live) {
         float4v out[4];
 #pragma unroll
         for (int a = 0; a < 4; ++a) out[a] = (float4v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int q = 0; q < NT; ++q) {
+        for (int q = 0; q < NT; q += 2) {
+          const float v[8] = {S[q][0], S[q][1], S[q][2], S[q][3], S[q + 1][0], S[q + 1][1], S[q + 1][2], S[q + 1][3]};
+          Frag8 part[3];
+          three_parts(v, part);
 #pragma unroll
           for (int a = 0; a < 4; ++a) {
-            const uint2 w = *(const uint2*)&c_rows[16 * a + r][16 * q + 4 * j];
-            const float c[4] = {__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u)};
+            const Frag8 c = two_fours(&c_rows[16 * a + r][16 * q + 4 * j]);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) out[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(c[i], S[q][i], out[a], 0, 0, 0);
+            for (int k = 2; k >= 0; --k) out[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c.v, part[k].v, out[a], 0, 0, 0);
           }
         }
 #pragma unroll
@@ -648,15 +700,29 @@ __global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restric
 #pragma unroll
           for (int i = 0; i < 4; ++i) out[a][i] *= f[i];
         }
+        auto score = [&](int row, int key) {
+          return (bf16_to_f32(scores[0][row][key]) + bf16_to_f32(scores[1][row][key])) + bf16_to_f32(scores[2][row][key]);
+        };
+        if (all_finite) {
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+          for (int b = 0; b < 4; b += 2) {
+            Frag8 xs;  // x is bfloat16
+            xs.u = make_uint4(rx_now[2 * b], rx_now[2 * b + 1], rx_now[2 * b + 2], rx_now[2 * b + 3]);
 #pragma unroll
-          for (int a = b; a < 4; ++a) {
-            if (a == b && !all_finite) continue;
-            const float4v m = *(const float4v*)&scores[16 * a + r][16 * b + 4 * j];
+            for (int a = b; a < 4; ++a)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) out[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[i], x[4 * b + i], out[a], 0, 0, 0);
+              for (int k = 2; k >= 0; --k)
+                out[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(two_fours(&scores[k][16 * a + r][16 * b + 4 * j]).v, xs.v, out[a], 0, 0, 0);
           }
+        } else {
+#pragma unroll
+          for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int a = b + 1; a < 4; ++a)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                out[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(score(16 * a + r, 16 * b + 4 * j + i), x[4 * b + i], out[a], 0, 0, 0);
+        }
         if (!all_finite) {
           // a later key's score of 0 does not leave an infinity or a NaN out: the tiles on the diagonal key by key
 #pragma unroll
@@ -667,7 +733,7 @@ __global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restric
               const float value = __shfl(x[k], 16 * from + r, CWM_WAVE);
 #pragma unroll
               for (int i = 0; i < 4; ++i)
-                if (4 * j + i >= key) out[b][i] = fmaf(scores[16 * b + 4 * j + i][16 * b + key], value, out[b][i]);
+                if (4 * j + i >= key) out[b][i] = fmaf(score(16 * b + 4 * j + i, 16 * b + key), value, out[b][i]);
             }
           }
         }
@@ -690,14 +756,17 @@ __global__ void __launch_bounds__(256) scan_block_kernel(const bf16_t* __restric
       for (int i = 0; i < 4; ++i) S[q][i] *= whole;
     }
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < 4; b += 2) {
+      const float v[8] = {x[4 * b], x[4 * b + 1], x[4 * b + 2], x[4 * b + 3], x[4 * b + 4], x[4 * b + 5], x[4 * b + 6], x[4 * b + 7]};
+      Frag8 part[3];
+      three_parts(v, part);
 #pragma unroll
       for (int q = 0; q < NT; ++q) {
-        const uint2 w = *(const uint2*)&b_cols[16 * q + r][16 * b + 4 * j];
-        const float c[4] = {__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u)};
+        const Frag8 c = two_fours(&b_cols[16 * q + r][16 * b + 4 * j]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(c[i], x[4 * b + i], S[q], 0, 0, 0);
+        for (int k = 2; k >= 0; --k) S[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c.v, part[k].v, S[q], 0, 0, 0);
       }
+    }
   }
   float* home = nullptr;
   if (MODE == 1) {
@@ -801,8 +870,8 @@ extern "C" int cwm_selective_scan(const void* xbc, long xbc_ld, const void* dt_r
   const int unit = dtype == CWM_BF16 ? 8 : 4;
   const bool vec = N % unit == 0 && P % unit == 0 && xbc_ld % unit == 0 && ((uintptr_t)xbc % 16) == 0 && 16 * row / unit <= SCAN_PFV * 256;
   if (segments && dtype == CWM_BF16 && vec && N <= 128 && P % 16 == 0 && ((uintptr_t)seg_state % 16) == 0) {
-    // on the matrix cores: 2,048 tokens of 64 heads, 64 columns and 128 rows in 156 us instead of
-    // 565 (launches included), 300 tokens in 97 instead of 170, 4,096 in 289 instead of 1,126; of float64 it is 2.4e-7 off, the walk
+    // on the matrix cores: 2,048 tokens of 64 heads, 64 columns and 128 rows in 113 us instead of
+    // 565 (launches included), 300 tokens in 74 instead of 170, 4,096 in 209 instead of 1,126; of float64 it is 2.4e-7 off, the walk
     // of segments token by token 3.7e-7
     const dim3 blocks((P + 63) / 64, heads, n_segments);
     const long head_elems = (long)SCAN_ROWS * split * P;
