@@ -257,8 +257,11 @@ __device__ __forceinline__ void unpack4_bf16(uint2 x, float (&v)[4]) {
 // Matrix-core layout (v_mfma_f32_16x16x4_f32, lane = 16 g + m): A holds element [m][k = g], B [k = g][m], the result
 // rows 4 g + i (i = 0 .. 3) of column m.  Which four of the summed-over indices an instruction takes as its k is free as
 // long as A and B agree: with k = 4 g + i the accumulator register i of a tile of S is B as it stands.
+// The kernel waits for LDS and for sums over lanes most of the time, so it wants company on its compute unit: two blocks (three in
+// MODE 1) are asked for, since left alone the compiler takes more than 256 registers for heads of 128 rows and 128 columns and one
+// block has the unit to itself (16 heads, 1,500 tokens in 24 segments: MODE 2 137 us, 90 with two).
 template <int MODE, int KIND, int CS, int EC>
-__global__ void __launch_bounds__(GLA_THREADS)
+__global__ void __launch_bounds__(GLA_THREADS, MODE == 1 ? 3 : 2)
 gla_block_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
                  const bf16_t* __restrict__ gate, long proj_ld, const float* __restrict__ bonus, const float* __restrict__ z,
                  long z_ld, const float* __restrict__ weight, int weight_stride, float eps, float* __restrict__ o_raw,
