@@ -19,8 +19,8 @@
 // Entries exactly equal to the threshold are all kept.  Without a nucleus (top_p = 1)
 // nothing is stored: the draw recomputes e_i where it walks.  A row of 128k logits done so
 // takes about 22 us greedy, 44 us at a temperature and 170 us with a nucleus; rows of more than
-// 8,192 entries are cut into segments instead (below): 16, 21 and 27 us, 49 us with a nucleus of
-// thousands of entries, launches included; 743 such rows 200 us instead of 1,220.
+// 8,192 entries are cut into segments instead (below): 6, 11 and 21 us, 34 us with a nucleus of
+// thousands of entries, replayed from a graph; 300 such rows 41, 54, 87 and 109 us.
 #include "common.h"
 #include "no_alloc.h"
 
@@ -349,6 +349,7 @@ sample_kernel(const float* __restrict__ logits, long row_stride, int vocab, cons
 #define SEGMENTS_FROM 8192  // longer rows are cut: the second launch costs 4 us, and a nucleus in a row of 8,192 takes 37 us as a whole, 20 to 28 in segments
 #define SEG_LIST 4096    // entries of the decisive bin that are kept in LDS
 #define SEG_SORT 1024    // and those of its decisive part that are put in order
+#define SEG_RANK 256     // so few of them by counting: 2 entries 0.6 instead of 2.2 us by exchanges, 224 3.9 instead of 4.3 (the comparisons grow with the square)
 #define SEG_FIXED 4503599627370496.0f  // 2^52
 #define ROW_FIXED 17592186044416.0f    // 2^44
 
@@ -449,24 +450,47 @@ sample_segment_kernel(const float* __restrict__ logits, long row_stride, int voc
   if (tid == 0) seg_records(row_workspace)[seg] = SegRecord{best.v, best.i, ws[0] + ws[1] + ws[2] + ws[3], wz[0] + wz[1] + wz[2] + wz[3]};
 }
 
-// Inclusive sums over the block's threads in a fixed order; `scratch` holds 16 floats.
-__device__ __forceinline__ float block_scan(float v, float* scratch) {
+// Inclusive sums over the block's threads in a fixed order, of values that are not negative; `scratch` holds 32 floats.
+// With `total` the sum over the block as join_sum forms it.
+__device__ __forceinline__ float block_scan(float v, float* scratch, float* total = nullptr) {
   const int lane = threadIdx.x & (CWM_WAVE - 1), wave = threadIdx.x / CWM_WAVE;
+  const float wave_total = total ? wave_sum(v) : 0.f;
 #pragma unroll
   for (int off = 1; off < CWM_WAVE; off <<= 1) {
     const float o = __shfl_up(v, off, CWM_WAVE);
     if (lane >= off) v += o;
   }
   __syncthreads();
-  if (lane == CWM_WAVE - 1) scratch[wave] = v;
+  if (lane == CWM_WAVE - 1) {
+    scratch[wave] = v;
+    if (total) scratch[SAMPLE_THREADS / CWM_WAVE + wave] = wave_total;
+  }
   __syncthreads();
+  if (total) {
+    *total = 0.f;
+#pragma unroll
+    for (int w = 0; w < SAMPLE_THREADS / CWM_WAVE; ++w) *total += scratch[SAMPLE_THREADS / CWM_WAVE + w];
+  }
   float before = 0.f;
-  for (int w = 0; w < wave; ++w) before += scratch[w];
+#pragma unroll
+  for (int w = 0; w < SAMPLE_THREADS / CWM_WAVE - 1; ++w) before += w < wave ? scratch[w] : 0.f;  // read together
   return before + v;
 }
 
+// block_sum of SAMPLE_THREADS threads: its bits, with the wavefronts' sums read together.
+__device__ __forceinline__ float join_sum(float v, float* scratch) {
+  v = wave_sum(v);
+  __syncthreads();
+  if ((threadIdx.x & (CWM_WAVE - 1)) == 0) scratch[threadIdx.x / CWM_WAVE] = v;
+  __syncthreads();
+  float total = 0.f;
+#pragma unroll
+  for (int w = 0; w < SAMPLE_THREADS / CWM_WAVE; ++w) total += scratch[w];
+  return total;
+}
+
 struct JoinShared {
-  float scratch[16];
+  float scratch[32];
   int first, last, count, smallest;
   int argmax[SEG_MOST];
   float max[SEG_MOST], scale[SEG_MOST], mass[SEG_MOST];
@@ -487,9 +511,11 @@ struct JoinShared {
 __device__ __forceinline__ int first_past(JoinShared& sh, float mass, float cum, float target, float& before) {
   if (threadIdx.x == 0) sh.first = 0x7fffffff, sh.last = -1;
   __syncthreads();
-  if (mass > 0.f) {
-    if (cum > target) atomicMin(&sh.first, (int)threadIdx.x);
-    atomicMax(&sh.last, (int)threadIdx.x);
+  const int lane = threadIdx.x & (CWM_WAVE - 1), wave_first = threadIdx.x - lane;
+  const unsigned long long with = __ballot(mass > 0.f), past = __ballot(mass > 0.f && cum > target);
+  if (lane == 0) {
+    if (past) atomicMin(&sh.first, wave_first + __ffsll(past) - 1);
+    if (with) atomicMax(&sh.last, wave_first + CWM_WAVE - 1 - __clzll((long long)with));
   }
   __syncthreads();
   const int pick = sh.first != 0x7fffffff ? sh.first : sh.last;
@@ -521,7 +547,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
 #pragma unroll
   for (int w = 1; w < SEG_MOST / CWM_WAVE; ++w) best = better(best, MaxIdx{sh.max[w], sh.argmax[w]});
   const float xmax = best.v;
-  const float sum = block_sum(tid < n_segs ? (rec.max == -__builtin_inff() ? rec.sum : rec.sum * expf(rec.max - xmax)) : 0.f, sh.scratch);
+  const float sum = join_sum(tid < n_segs ? (rec.max == -__builtin_inff() ? rec.sum : rec.sum * expf(rec.max - xmax)) : 0.f, sh.scratch);
   const float lse = xmax + logf(sum);
   // NaN among the logits, infinities, temperatures at which a bin's number would not be exact: one block, pass by pass
   const float inv_t = 1.0f / temp, inv_w = inv_t * 11.541560327f;
@@ -548,7 +574,7 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
     sh.below[tid] = scale > 0.f ? bins_below(top_floor, rec.max * inv_w) : SEG_BINS;
     sh.kept[tid] = 0;
   }
-  const float z = block_sum(seg_mass, sh.scratch);
+  const float z = join_sum(seg_mass, sh.scratch);
   const bool nucleus = row_top_p < 1.0f;
   int bin = SEG_BINS, sub = SEG_BINS;  // kept whole: the bins before `bin`, and of that one the parts before `sub`
   float least = 0.f;                   // kept of part `sub` (of the whole bin if it is not divided): the entries from here on
@@ -572,9 +598,17 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
     const float target = row_top_p * z;
     const int g = tid & (SEG_BINS - 1);
     float m = 0.f;
-    for (int s = tid / SEG_BINS; s < n_segs; s += SAMPLE_THREADS / SEG_BINS) {
-      const int k = g - sh.below[s];
-      if (k >= 0 && k < SEG_BINS - 1) m += seg_histogram(row_workspace, n_segs, s)[k] * sh.scale[s];
+    constexpr int APART = SAMPLE_THREADS / SEG_BINS, TOGETHER = 4;  // histograms whose loads are in flight at once
+    for (int s0 = tid / SEG_BINS; s0 < n_segs; s0 += APART * TOGETHER) {
+      float h[TOGETHER];
+#pragma unroll
+      for (int q = 0; q < TOGETHER; ++q) {
+        const int s = min(s0 + q * APART, n_segs - 1), k = g - sh.below[s];
+        h[q] = 0.f;
+        if (s0 + q * APART < n_segs && k >= 0 && k < SEG_BINS - 1) h[q] = seg_histogram(row_workspace, n_segs, s)[k];
+      }
+#pragma unroll
+      for (int q = 0; q < TOGETHER; ++q) m = fmaf(h[q], sh.scale[min(s0 + q * APART, n_segs - 1)], m);
     }
     sh.part[tid / SEG_BINS][g] = m;
     __syncthreads();
@@ -582,7 +616,8 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
     const float cum = block_scan(m, sh.scratch);
     if (tid == 0) sh.first = SEG_BINS, sh.count = 0, sh.smallest = 0x7f800000;
     __syncthreads();
-    if (m > 0.f && cum > target) atomicMin(&sh.first, tid);
+    const unsigned long long past = __ballot(m > 0.f && cum > target);
+    if (lane == 0 && past) atomicMin(&sh.first, tid + __ffsll(past) - 1);
     __syncthreads();
     bin = sh.first;
     if (bin >= SEG_BINS - 1) {  // the passing point lies below 32 octaves
@@ -593,13 +628,48 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
     __syncthreads();
     float above = sh.before;
 
+    // of every segment the bins before it, a wavefront a segment: used at the end, read with the loads that follow
+    constexpr int WAVES = SAMPLE_THREADS / CWM_WAVE, SEGS = 4;  // segments of a wavefront at once
+    const int first_seg = __builtin_amdgcn_readfirstlane(wave);
+    for (int s0 = first_seg; s0 < n_segs; s0 += WAVES * SEGS) {
+      float h[SEGS][SEG_BINS / CWM_WAVE] = {};
+#pragma unroll
+      for (int g = 0; g < SEGS; ++g) {
+        const int s = s0 + g * WAVES;
+        if (s < n_segs) {
+          const int below = sh.below[s];
+          const float* hist = seg_histogram(row_workspace, n_segs, s);
+#pragma unroll
+          for (int q = 0; q < SEG_BINS / CWM_WAVE; ++q) {
+            const int k = q * CWM_WAVE + lane;
+            if (k < SEG_BINS - 1 && k + below < bin) h[g][q] = hist[k];
+          }
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < SEGS; ++g) {
+        const int s = s0 + g * WAVES;
+        if (s < n_segs) {
+          float whole = 0.f;
+#pragma unroll
+          for (int q = 0; q < SEG_BINS / CWM_WAVE; ++q) whole += h[g][q];
+          whole = wave_sum(whole);
+          if (lane == 0) sh.mass[s] = whole;
+        }
+      }
+    }
+
     // 4. that bin's entries, a segment a wavefront, where the segment has mass in it: take(segment, its first entry,
     //    the lane's entries that lie in the bin)
     const float edge = top_floor - bin;  // x lies in the bin if edge <= x * inv_w < edge + 1
+    static_assert(SEG_MOST <= SAMPLE_THREADS, "a lane looks at one of its wavefront's segments");
+    const int looked = wave + lane * (SAMPLE_THREADS / CWM_WAVE);
+    const int looked_bin = looked < n_segs ? bin - sh.below[looked] : -1;
+    const unsigned long long with_mass =
+        __ballot(looked_bin >= 0 && seg_histogram(row_workspace, n_segs, looked)[min(looked_bin, SEG_BINS - 1)] > 0.f);
     auto scan_bin = [&](auto&& take) {
-      for (int s = wave; s < n_segs; s += SAMPLE_THREADS / CWM_WAVE) {
-        const int k = bin - sh.below[s];
-        if (k < 0 || !(seg_histogram(row_workspace, n_segs, s)[min(k, SEG_BINS - 1)] > 0.f)) continue;
+      for (unsigned long long left = with_mass; left; left &= left - 1) {
+        const int s = wave + (__ffsll(left) - 1) * (SAMPLE_THREADS / CWM_WAVE);
         const int begin = s * seg_len, end = min(vocab, begin + seg_len);
         constexpr int LOADS = SEG_ENTRIES / (4 * CWM_WAVE);
         uint32_t marked = 0;
@@ -719,8 +789,23 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
     const float own = tid < n ? e_of(sh.list_x[tid]) : 0.f;
     const int owner = tid < n ? sh.list_i[tid] / seg_len : 0;
     float key = own;
-    int size = CWM_WAVE;
-    while (size < n) size <<= 1;
+    if (n <= SEG_RANK) {
+      // an entry's place is the number of larger ones and of equal ones before it, counted by RANKERS threads
+      constexpr int RANKERS = SAMPLE_THREADS / SEG_RANK;
+      if (tid < SEG_RANK) sh.part[0][tid] = own;
+      __syncthreads();
+      const int entry = tid / RANKERS, at = tid % RANKERS;
+      const float mine = sh.part[0][entry];
+      int place = 0;
+      for (int j = at; j < n; j += RANKERS) place += sh.part[0][j] > mine || (sh.part[0][j] == mine && j < entry);
+#pragma unroll
+      for (int off = 1; off < RANKERS; off <<= 1) place += __shfl_xor(place, off, CWM_WAVE);
+      if (at == 0 && entry < n) sh.part[1][place] = mine;
+      __syncthreads();
+      key = tid < n ? sh.part[1][tid] : 0.f;
+    }
+    int size = n <= SEG_RANK ? 1 : CWM_WAVE;
+    while (size > 1 && size < n) size <<= 1;
     for (int k = 2; k <= size; k <<= 1)
       for (int j = k >> 1; j > 0; j >>= 1) {
         float other;
@@ -735,32 +820,20 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
         key = ((tid & k) == 0) == ((tid & j) == 0) ? fmaxf(key, other) : fminf(key, other);
       }
     const float through = block_scan(key, sh.scratch);
-    if (tid < n && above + (through - key) <= target) atomicMin(&sh.smallest, __float_as_int(key));
+    const unsigned long long fits = __ballot(tid < n && above + (through - key) <= target);
+    if (fits && lane == CWM_WAVE - 1 - __clzll((long long)fits)) atomicMin(&sh.smallest, __float_as_int(key));  // the wavefront's smallest: keys descend
     __syncthreads();
     least = __int_as_float(sh.smallest);
     if (tid < n && own >= least) atomicAdd(&sh.kept[owner], __float2ull_rn(own * ROW_FIXED));
     __syncthreads();
-    // the kept mass of every segment: its bins before `bin`, a wavefront a segment, and what the list gave
-    seg_mass = 0.f;
-    for (int s = wave; s < n_segs; s += SAMPLE_THREADS / CWM_WAVE) {
-      const float* hist = seg_histogram(row_workspace, n_segs, s);
-      float h = 0.f;
-#pragma unroll
-      for (int q = 0; q < SEG_BINS / CWM_WAVE; ++q) {
-        const int k = q * CWM_WAVE + lane;
-        if (k < SEG_BINS - 1 && k + sh.below[s] < bin) h += hist[k];
-      }
-      h = wave_sum(h);
-      if (lane == 0) sh.mass[s] = h * sh.scale[s] + (float)sh.kept[s] * (1.0f / ROW_FIXED);
-    }
-    __syncthreads();
-    seg_mass = tid < n_segs ? sh.mass[tid] : 0.f;
+    // the kept mass of every segment: its bins before `bin` and what the list gave
+    seg_mass = tid < n_segs ? sh.mass[tid] * sh.scale[tid] + (float)sh.kept[tid] * (1.0f / ROW_FIXED) : 0.f;
   }
 
   // 7. inverse CDF: the segment in which the running mass passes u * (kept mass), then the entry.  The two levels' sums are
   //    rounded differently, so a level may find the point beyond its last mass: it then takes its last entry with mass.
-  const float run = block_scan(seg_mass, sh.scratch);
-  const float total = block_sum(seg_mass, sh.scratch);
+  float total;
+  const float run = block_scan(seg_mass, sh.scratch, &total);
   const float target = u * total;
   float before;
   const int seg = first_past(sh, seg_mass, run, target, before);
@@ -786,6 +859,12 @@ __device__ __forceinline__ bool join_segments(JoinShared& sh, const int row, con
   return true;
 }
 
+// One block a row, so it is bound by its own chain: records, histograms, the bin's entries, the kept segments' masses and the
+// segment with the draw are read one after the other, with barriers and sums over the block between them.  So that a link costs
+// one trip to memory, loads of one kind are issued together: four histograms (only where they count: the rows of all 63 without
+// condition were 7 instead of 3 us), the segments that hold the bin by one look, the masses before the bin with the first of
+// these; the wavefronts' sums are read as a block, and a wavefront sends one atomic, not one a lane.  A row of 128,256 with a
+// nucleus of few entries 16.2 instead of 22.7 us, of 32,768 14.6 instead of 19.8; at top_p = 1 the choice as a whole 11 instead of 19.
 template <bool VEC>
 __global__ void __launch_bounds__(SAMPLE_THREADS, 8)
 sample_join_kernel(const float* __restrict__ logits, long row_stride, int vocab, int seg_len, int n_segs, const float* __restrict__ temperature,

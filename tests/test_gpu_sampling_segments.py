@@ -138,3 +138,34 @@ def test_ties_that_a_rounded_product_leaves_at_a_bins_edge(value, temp, ties):
         assert kept[tok] > 0, (r, tok)
         assert float(cdf[tok] - kept[tok] / kept.sum()) <= float(us[r]) + 2e-5 and float(cdf[tok]) >= float(us[r]) - 2e-5, (r, tok)
         np.testing.assert_allclose(float(slp[r]), math.log(float(kept[tok] / kept.sum())), atol=2e-5)
+
+
+@pytest.mark.parametrize("levels", [None, 6])
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 255, 256, 257, 511, 513, 1024])
+def test_the_nucleus_ends_in_a_bin_of_so_many_entries(count, levels):
+    """At the numbers of entries where the way of putting them in order changes, all different and with ties."""
+    from cwm_amd import ops
+
+    vocab, n = 32768, 64
+    g = torch.Generator().manual_seed(count)
+    within = torch.rand(count, generator=g)
+    if levels:
+        within = torch.floor(within * levels) / levels
+    logits = torch.full((vocab,), -20.0)  # all others together: 32768 exp(-29.9), below 1e-8 of the mass
+    where = torch.randperm(vocab, generator=g)[:count]
+    logits[where] = (115.05 + 0.9 * within) * (math.log(2.0) / 8.0)  # one eighth of an octave, away from its edges
+    us = (torch.arange(n) + 0.5) / n
+    args = [logits.expand(n, vocab).contiguous(), torch.ones(n), torch.full((n,), 0.6), us]
+    toks, _, slp = (t.cpu() for t in ops.unpack_sampled(ops.sample_packed(*(t.to(DEV) for t in args))))
+    probs = torch.softmax(logits.double(), -1)
+    values = torch.sort(probs, descending=True).values
+    above = torch.cumsum(values, 0) - values
+    # 2^-24 for each of the at most 12 additions that a mass goes through and for the exponential: 1e-6 of the target
+    kept = [probs >= float(values[above <= 0.6 + off][-1]) * (1 - 1e-6) for off in (-1e-6, 1e-6)]
+    least, most = (float((probs * k).sum()) for k in kept)
+    for u, tok, s in zip(us.tolist(), toks.tolist(), slp.tolist()):
+        assert bool(kept[1][tok])
+        assert math.log(float(probs[tok]) / most) - 1e-5 <= s <= math.log(float(probs[tok]) / least) + 1e-5
+        upto = torch.cumsum(probs * kept[1], 0)
+        slack = 1e-5 + (most - least) / least  # an entry at the threshold may be in or out
+        assert float(upto[tok] - probs[tok]) / most <= u + slack and float(upto[tok]) / most >= u - slack
