@@ -1030,14 +1030,16 @@ class StaticPlans:
 def _attention_plan(
     batch, group: int, n_kv: int, head_dim: int, window: Optional[int], device: torch.device, chunk: Optional[int] = None, halves: bool = False,
 ) -> _UploadedPlan:
-    """The step's work list for this (group size, key/value heads and their size, window or block of keys), uploaded once per step."""
+    """The step's work list for this (group size, key/value heads and their size, window or block of keys), uploaded once per step.
+    `halves`: whether blocks of 64 rows are built for what the layer has (`_half_blocks_built`)."""
     from .attention_plan import build_plan, cuts_finer, wide_item_tiles
 
     finer = cuts_finer(n_kv, head_dim)
     static = getattr(batch, "static", None)
     if static is not None:
         return static.plan(batch, group, n_kv, window, chunk, finer)
-    key = ("attention_plan", group, n_kv, window, chunk, finer, halves)
+    # with such blocks the list depends on the head size, by which they are chosen; layers of other sizes have lists of their own
+    key = ("attention_plan", group, n_kv, window, chunk, finer, head_dim if halves else None)
     cached = batch.scratch.get(key)
     if cached is None:
         # a sequence whose blocks of 128 rows, over all key/value heads, would not give every compute unit two
@@ -1082,6 +1084,14 @@ def _three_blocks_a_unit(n_blocks: int, shape: Tuple[int, float], device: torch.
     two = max(longest, mean * -(-n_blocks // (2 * units)))
     three = _THREE_BLOCKS_TILE_TIME * max(longest, mean * -(-n_blocks // (3 * units)))
     return int(three < two)
+
+
+def _half_blocks_built(n_kv: int, head_dim: int, page_size: int) -> bool:
+    """Whether the matrix-core attention kernel has blocks of 64 rows for these sizes: the head sizes and pages whose keys and
+    values the loads write to LDS themselves."""
+    from .attention_plan import WIDE_HALF_BLOCKS
+
+    return head_dim in WIDE_HALF_BLOCKS and page_size % 32 == 0 and n_kv * page_size * head_dim * 2 < 2 ** 31
 
 
 def mfma_attention_takes(dtype: torch.dtype, head_dim: int, page_size: int) -> bool:
@@ -1131,9 +1141,7 @@ def paged_attention_mfma(
     _i32(block_table, "block_table")
     if block_table.dim() != 2 or block_table.shape[0] != batch.n_seqs or n_tokens != batch.n_tokens:
         raise KernelError("block_table must be [B, W] for the batch's sequences, q [T, ...] for its tokens")
-    # whether blocks of 64 rows are built for these sizes: keys and values that the loads write to LDS themselves
-    halves = page_size % 32 == 0 and n_kv * page_size * hd * 2 < 2 ** 31
-    plan = _attention_plan(batch, n_q // n_kv, n_kv, hd, window, q.device, chunk, halves)
+    plan = _attention_plan(batch, n_q // n_kv, n_kv, hd, window, q.device, chunk, _half_blocks_built(n_kv, hd, page_size))
     out = torch.empty((n_tokens, n_q * hd), dtype=q.dtype, device=q.device)
     partial = None
     if plan.n_partials:
