@@ -1086,12 +1086,14 @@ def _three_blocks_a_unit(n_blocks: int, shape: Tuple[int, float], device: torch.
     return int(three < two)
 
 
-def _half_blocks_built(n_kv: int, head_dim: int, page_size: int) -> bool:
+def _half_blocks_built(n_kv: int, head_dim: int, page_size: int, keep_first: int = 0) -> bool:
     """Whether the matrix-core attention kernel has blocks of 64 rows for these sizes: the head sizes and pages whose keys and
-    values the loads write to LDS themselves."""
+    values the loads write to LDS themselves.  Not with kept first keys: a block takes those before its rows' windows ahead
+    of them, so a tile that holds both is one pass or two by where the block's first row stands, and a row's bits would
+    depend on the block's height, that is on what else is in the step."""
     from .attention_plan import WIDE_HALF_BLOCKS
 
-    return head_dim in WIDE_HALF_BLOCKS and page_size % 32 == 0 and n_kv * page_size * head_dim * 2 < 2 ** 31
+    return head_dim in WIDE_HALF_BLOCKS and page_size % 32 == 0 and n_kv * page_size * head_dim * 2 < 2 ** 31 and keep_first == 0
 
 
 def mfma_attention_takes(dtype: torch.dtype, head_dim: int, page_size: int) -> bool:
@@ -1141,7 +1143,7 @@ def paged_attention_mfma(
     _i32(block_table, "block_table")
     if block_table.dim() != 2 or block_table.shape[0] != batch.n_seqs or n_tokens != batch.n_tokens:
         raise KernelError("block_table must be [B, W] for the batch's sequences, q [T, ...] for its tokens")
-    plan = _attention_plan(batch, n_q // n_kv, n_kv, hd, window, q.device, chunk, _half_blocks_built(n_kv, hd, page_size))
+    plan = _attention_plan(batch, n_q // n_kv, n_kv, hd, window, q.device, chunk, _half_blocks_built(n_kv, hd, page_size, keep_first))
     out = torch.empty((n_tokens, n_q * hd), dtype=q.dtype, device=q.device)
     partial = None
     if plan.n_partials:

@@ -200,7 +200,8 @@ def build_plan(
 def wide_item_tiles(q_lens: Sequence[int], kv_lens: Sequence[int], group: int, n_kv: int, head_dim: int, wide_cut_below: int, units: int) -> int:
     """Row tiles of a wide item for a step of these lengths on `units` compute units: half of WIDE_TILES where blocks of
     WIDE_TILES are few (`WIDE_HALF_BLOCKS`; other head sizes have no such blocks).  A row's bits are the same either way unless
-    its keys are cut, so a step with a cut sequence keeps the whole size."""
+    its keys are cut, so a step with a cut sequence keeps the whole size, or first keys are kept beside a window, for which the
+    caller does not ask."""
     blocks, most = 0, WIDE_HALF_BLOCKS.get(head_dim, 0) * units
     for q, kv in zip(q_lens, kv_lens):
         n_tiles = -(-q * group // ROWS_PER_TILE)
