@@ -22,7 +22,7 @@
 // moves once a block.  `memory_maxima_kernel` walks m (one thread a (head, sequence), the same float32 operations as the
 // walk above, so both give the same m: 29 us for 1,531 tokens, 39 where a wavefront passed every gate through a scalar register) and sums f in float64, since differences of long sums are taken;
 // `memory_scores_kernel` works out every block's weighted scores and weights side by side, and `memory_chunk_kernel` (a thread
-// block a (tile of value columns, head, sequence or segment of one)) walks the blocks with the remaining products on the float32 matrix
+// block a (tile of value columns, head, sequence or segment of a long one)) walks the blocks with the remaining products on the float32 matrix
 // instruction.  The normaliser n
 // is the column after the last value column, with ones for values, so n_t . q_t falls out as that column's result and the
 // division moves into `memory_out_kernel`.  This differs from the walk by rounding only.
@@ -211,6 +211,11 @@ static_assert(MEMC_COLS == MEMC_L, "a block's scores are staged like its values"
 static_assert(MEMX_SPAN % MEMX_AHEAD == 0, "whole reads of gates");
 #define MEMS_L 256        // tokens of a segment (whole blocks)
 static_assert(MEMS_L % MEMC_L == 0, "a segment is whole blocks");
+// From so many tokens a portion's blocks are walked in segments side by side: a chain of 48 blocks (1,531 tokens, 16 heads of 128)
+// takes 189 us in one piece and 25 + 6 + 50 us in segments, which do half as much again; a portion of one segment gains nothing.
+// A portion is cut by its own length alone, whatever lies beside it, so that its results and its state have the same bits.
+#define MEMS_FROM 512
+static_assert(MEMS_FROM >= 2 * MEMS_L, "segment_place counts on two segments");
 
 // coef: float32 [T][heads][4]: {i_t, m_t, b_t as a float64 in two words}; b counts from the portion's start.
 // start: float64 [n_seqs][heads]: m before the portion.
@@ -283,17 +288,32 @@ memory_maxima_kernel(const float* __restrict__ gates, long gates_stride, float c
   if (threadIdx.x == 0) *st_m = m;
 }
 
-// The blocks (or segments) of a step, L tokens each, numbered so that no two share a number: block j of sequence b is
-// cu_q[b] / L + b + j.  Returns the sequence of number x and sets the block's first token, or -1 if x is no block's number.
-template <int L>
+// The blocks of a step, numbered so that no two share a number: block j of sequence b is cu_q[b] / MEMC_L + b + j.
+// Returns the sequence of number x and sets the block's first token, or -1 if x is no block's number.
 __device__ __forceinline__ int memory_block_of(int x, const int* __restrict__ cu_q, int n_seqs, int* base) {
-  int lo = 0, hi = n_seqs - 1;  // the last b with cu_q[b] / L + b <= x
-  if (cu_q[0] / L > x) return -1;
+  int lo = 0, hi = n_seqs - 1;  // the last b with cu_q[b] / MEMC_L + b <= x
+  if (cu_q[0] / MEMC_L > x) return -1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) / 2;
-    if (cu_q[mid] / L + mid <= x) lo = mid; else hi = mid - 1;
+    if (cu_q[mid] / MEMC_L + mid <= x) lo = mid; else hi = mid - 1;
   }
-  *base = cu_q[lo] + L * (x - (cu_q[lo] / L + lo));
+  *base = cu_q[lo] + MEMC_L * (x - (cu_q[lo] / MEMC_L + lo));
+  return *base < cu_q[lo + 1] ? lo : -1;
+}
+
+// Likewise the segments of the portions that are cut, without numbers for the others: segment j of a portion that starts at
+// token t is segment_place(t) + j.  A portion of n >= 2 MEMS_L tokens has ceil(n / MEMS_L) <= floor(3 n / (2 MEMS_L)) segments,
+// and so ends before the place of what follows it.
+__host__ __device__ __forceinline__ int segment_place(int t) { return (int)(3l * t / (2 * MEMS_L)); }
+__device__ __forceinline__ int memory_segment_of(int x, const int* __restrict__ cu_q, int n_seqs, int* base) {
+  int lo = 0, hi = n_seqs - 1;  // the last b whose place is at most x
+  if (segment_place(cu_q[0]) > x) return -1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) / 2;
+    if (segment_place(cu_q[mid]) <= x) lo = mid; else hi = mid - 1;
+  }
+  if (cu_q[lo + 1] - cu_q[lo] < MEMS_FROM) return -1;
+  *base = cu_q[lo] + MEMS_L * (x - segment_place(cu_q[lo]));
   return *base < cu_q[lo + 1] ? lo : -1;
 }
 
@@ -312,7 +332,7 @@ memory_scores_kernel(const T* __restrict__ src, long src_stride, int q_off, int 
   __shared__ double ga_s[MEMC_L], gg_s[MEMC_L];  // a and g of the block's tokens
   const int h = blockIdx.y;
   int base;
-  const int b = memory_block_of<MEMC_L>(blockIdx.x, cu_q, n_seqs, &base);
+  const int b = memory_block_of(blockIdx.x, cu_q, n_seqs, &base);
   if (b < 0) return;
   const int t0 = cu_q[b], t1 = cu_q[b + 1];
   const int count = min(MEMC_L, t1 - base);
@@ -379,18 +399,22 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // add up through LDS, then K^T (weighted V) into S.  A block's q, k, v, scores and weights are fetched into registers
 // while the block before is worked on.
 //
-// PART: 0, a thread block walks a whole portion.  A long portion is a chain of blocks of tokens at 3.9 us each with few thread
-// blocks under way, so it is cut into segments of MEMS_L tokens that are walked side by side: 1, what a segment (all but a
-// portion's last) adds to the state, from zero and without results, into its place in `saved`; `memory_join_kernel` then makes
-// of these the states before the segments; 2, the segments' results from there, and the portion's last state.
-// saved: float32 [segments][heads][32 gridDim.x columns][32 TILES rows].
-template <typename T, int TILES, int PART>
+// A long portion (MEMS_FROM) is a chain of blocks of tokens at 3.9 us each with few thread blocks under way, so it is cut into
+// segments of MEMS_L tokens that are walked side by side.  Without RESULTS: what a segment (all but a portion's last) adds to the
+// state, from zero, into its place in `saved`; `memory_join_kernel` then makes of these the states before the segments.  With
+// RESULTS: the segments from their states, the last one of a portion leaving the portion's; then, behind the places, the portions
+// that are not cut (all if there are no places), from theirs: 1,000 tokens with 40 decoded ones 146 us, with 256 458 (160 and 565
+// where those were copied into segments of their own; 180 and 538 with a launch of their own).
+// saved: float32 [segment_place(tokens)][heads][32 gridDim.x columns][32 TILES rows].
+// v or zero, without a branch around what v is made of, which would wait for v's load alone.
+__device__ __forceinline__ float only(bool have, float v) { return __uint_as_float(__float_as_uint(v) & (have ? 0xffffffffu : 0u)); }
+
+template <typename T, int TILES, bool RESULTS>
 __global__ void __launch_bounds__(CWM_WAVE * TILES)
 memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k_off, int v_off, float q_scale,
                     const float* __restrict__ scores, const float* __restrict__ wd, float* __restrict__ state, long state_stride,
                     long head_elems, const int* __restrict__ cu_q, const int* __restrict__ state_slots, float* __restrict__ y,
-                    float* __restrict__ nq, float* __restrict__ saved, int n_seqs, int heads, int d, int e, int d_pad) {
-  constexpr bool RESULTS = PART != 1;
+                    float* __restrict__ nq, float* __restrict__ saved, int places, int n_seqs, int heads, int d, int e, int d_pad) {
   constexpr int THREADS = CWM_WAVE * TILES, DP = 32 * TILES;
   constexpr int ROWQ = DP + 1, ROWK = DP + 4;  // a column of q across tokens, a row of k along its elements: no bank twice
   constexpr int QK_REGS = MEMC_L * DP / THREADS, V_REGS = MEMC_L * MEMC_COLS / THREADS;
@@ -406,25 +430,33 @@ memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k
   const int c = lane & 31, half = lane >> 5;
   const int col = blockIdx.x * MEMC_COLS + c;  // column e is the normaliser
   const int tile_row = 32 * wave;
-  int b = blockIdx.z, t0, t1;
+  const bool whole = RESULTS && (int)blockIdx.z >= places;  // a portion in one piece
+  int b = (int)blockIdx.z - places, t0, t1;
   bool last = true;  // of its portion
-  if constexpr (PART == 0) {
+  if (whole) {
     t0 = cu_q[b], t1 = cu_q[b + 1];
+    if (places > 0 && t1 - t0 >= MEMS_FROM) return;
   } else {
-    b = memory_block_of<MEMS_L>(blockIdx.z, cu_q, n_seqs, &t0);
+    b = memory_segment_of(blockIdx.z, cu_q, n_seqs, &t0);
     if (b < 0) return;
     t1 = cu_q[b + 1];
     last = t0 + MEMS_L >= t1;
-    if (PART == 1 && last) return;
+    if (!RESULTS && last) return;
     t1 = min(t1, t0 + MEMS_L);
   }
   float* st = state + (size_t)state_slots[b] * state_stride + (size_t)h * head_elems + (size_t)col * d_pad;
-  float* kept = PART == 0 ? nullptr : saved + (((size_t)blockIdx.z * heads + h) * (gridDim.x * MEMC_COLS) + col) * DP;
+  float* kept = saved + (((size_t)blockIdx.z * heads + h) * (gridDim.x * MEMC_COLS) + col) * DP;
+  // where the state comes from; of a column or rows that do not exist, what does is read, and zero taken
+  const float* from = whole ? st - (size_t)max(col - e, 0) * d_pad : kept;
+  const int rows = !whole ? DP : col <= e ? d_pad : 0, last_four = (whole ? d_pad : DP) - 4;
   memc_acc S;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int row = tile_row + 8 * (r / 4) + 4 * half + (r % 4);
-    S[r] = PART == 1 ? 0.f : PART == 2 ? kept[row] : (col <= e && row < d_pad) ? st[row] : 0.f;
+  for (int r = 0; r < 16; r += 4) {  // four adjacent rows; d_pad is a multiple of 16
+    const int row = tile_row + 2 * r + 4 * half;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (RESULTS) v = *(const float4*)(from + min(row, last_four));
+    const bool have = row < rows;
+    S[r] = have ? v.x : 0.f, S[r + 1] = have ? v.y : 0.f, S[r + 2] = have ? v.z : 0.f, S[r + 3] = have ? v.w : 0.f;
   }
   // What a fetch leaves in registers is what the loads return and nothing made of it: an operation on a loaded value would
   // wait for the load where the fetch is issued, not where the value is staged.  Every load is issued, from an address that
@@ -458,14 +490,14 @@ memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k
     for (int u = 0; u < QK_REGS; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x / DP, r = x - tok * DP;
       const bool live = tok < count && r < d;
-      if constexpr (RESULTS) q_s[tok][r] = live ? raw_to_f32(q_r[u]) * q_scale : 0.f;
-      k_s[tok][r] = live ? raw_to_f32(k_r[u]) : 0.f;
+      if constexpr (RESULTS) q_s[tok][r] = only(live, raw_to_f32(q_r[u]) * q_scale);
+      k_s[tok][r] = only(live, raw_to_f32(k_r[u]));
     }
 #pragma unroll
     for (int u = 0; u < V_REGS; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x / MEMC_COLS, cl = x - tok * MEMC_COLS, cc = blockIdx.x * MEMC_COLS + cl;
-      v_s[tok][cl] = tok < count ? (cc < e ? raw_to_f32(v_r[u]) : (cc == e ? 1.f : 0.f)) : 0.f;
-      if constexpr (RESULTS) a_s[tok][cl] = tok < count ? a_r[u] : 0.f;
+      v_s[tok][cl] = only(tok < count && cc <= e, cc == e ? 1.f : raw_to_f32(v_r[u]));
+      if constexpr (RESULTS) a_s[tok][cl] = only(tok < count, a_r[u]);
     }
     if (threadIdx.x < MEMC_L) {
       const bool live = (int)threadIdx.x < count;
@@ -522,7 +554,7 @@ memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int row = tile_row + 8 * (r / 4) + 4 * half + (r % 4);
-    if (PART == 1)
+    if (!RESULTS)
       kept[row] = S[r];
     else if (last && col <= e && row < d_pad)
       st[row] = S[r];
@@ -538,11 +570,11 @@ memory_join_kernel(const float* __restrict__ coef, const double* __restrict__ st
                    int e, int d_pad) {
   constexpr int DP = 32 * TILES, QUADS = MEMC_COLS * DP / 4, EACH = QUADS / (CWM_WAVE * TILES);
   const int h = blockIdx.y, b = blockIdx.z, t0 = cu_q[b], t1 = cu_q[b + 1];
-  if (t0 >= t1) return;
+  if (t1 - t0 < MEMS_FROM) return;
   const int segments = (t1 - t0 + MEMS_L - 1) / MEMS_L;
   const float* st = state + (size_t)state_slots[b] * state_stride + (size_t)h * head_elems;
   const size_t head_size = (size_t)gridDim.x * MEMC_COLS * DP, step = head_size * heads;
-  float4* at = (float4*)(saved + ((size_t)(t0 / MEMS_L + b) * heads + h) * head_size + (size_t)blockIdx.x * MEMC_COLS * DP);
+  float4* at = (float4*)(saved + ((size_t)segment_place(t0) * heads + h) * head_size + (size_t)blockIdx.x * MEMC_COLS * DP);
   float4 now[EACH];
 #pragma unroll
   for (int i = 0; i < EACH; ++i) {
@@ -602,12 +634,12 @@ memory_out_kernel(const float* __restrict__ y, const float* __restrict__ nq, con
 }
 
 extern "C" int cwm_matrix_memory_block_tokens() { return MEMC_L; }
-extern "C" int cwm_matrix_memory_segment_tokens() { return MEMS_L; }
+extern "C" int cwm_matrix_memory_segments_from() { return MEMS_FROM; }
 
 static inline int memc_tiles(int d) { return d <= 32 ? 1 : d <= 64 ? 2 : d <= 128 ? 4 : 8; }
 
-extern "C" long cwm_matrix_memory_saved_floats(int n_tokens, int n_seqs, int heads, int d, int e) {
-  return (long)(n_tokens / MEMS_L + n_seqs) * heads * ((e + 1 + MEMC_COLS - 1) / MEMC_COLS * MEMC_COLS) * 32 * memc_tiles(d);
+extern "C" long cwm_matrix_memory_saved_floats(int n_tokens, int heads, int d, int e) {
+  return (long)segment_place(n_tokens) * heads * ((e + 1 + MEMC_COLS - 1) / MEMC_COLS * MEMC_COLS) * 32 * memc_tiles(d);
 }
 
 // src: the joined projection [n_tokens][src_stride] of dtype: q at column q_off (heads * d), k at k_off (heads * d), v at
@@ -617,7 +649,7 @@ extern "C" long cwm_matrix_memory_saved_floats(int n_tokens, int n_seqs, int hea
 // out: [n_tokens][heads * e] of dtype.  With `start` (float64 scratch [n_seqs][heads]), `nq` (float32 scratch
 // [n_tokens][heads]) and `scores` (float32 scratch [n_tokens][heads][block tokens + 2]) the portions are taken in blocks of
 // tokens; without them they are walked token by token.  With `saved` as well (float32 scratch, 16-byte aligned, of
-// `cwm_matrix_memory_saved_floats` floats) the blocks of long portions are walked in segments side by side.
+// `cwm_matrix_memory_saved_floats` floats) the blocks of portions of MEMS_FROM tokens and more are walked in segments side by side.
 extern "C" int cwm_matrix_memory(const void* src, int dtype, long src_stride, int q_off, int k_off, int v_off, int g_off,
                                  const float* gates, long gates_stride, float cap, float q_scale, float* state, long state_stride,
                                  int n_slots, const int* cu_q, const int* state_slots, int n_seqs, int n_tokens,
@@ -646,26 +678,24 @@ extern "C" int cwm_matrix_memory(const void* src, int dtype, long src_stride, in
   const unsigned out_blocks = (unsigned)((n_pairs + MEM_THREADS / CWM_WAVE - 1) / (MEM_THREADS / CWM_WAVE));
   float* wd = scores ? scores + (size_t)n_tokens * heads * MEMC_L : nullptr;  // [n_tokens][heads][2] behind the scores
   const unsigned numbered = (unsigned)(n_tokens / MEMC_L + n_seqs);  // more than the largest number of a block of tokens
-  const unsigned segments = (unsigned)(n_tokens / MEMS_L + n_seqs);  // likewise
-  CWM_REQUIRE(!saved || segments <= 65535, "matrix_memory: too many segments for one launch");
-#define CWM_MEMORY_CHUNK(T, TILES, PART, Z)                                                                                 \
-  hipLaunchKernelGGL((memory_chunk_kernel<T, TILES, PART>), dim3(block_tiles, heads, Z), dim3(CWM_WAVE * TILES), 0, stream,  \
+  int places = saved ? segment_place(n_tokens) : 0;  // more than the largest of a segment
+  if (places + n_seqs > 65535) places = 0;           // more than a launch numbers: every portion in one piece
+#define CWM_MEMORY_CHUNK(T, TILES, RESULTS, Z)                                                                              \
+  hipLaunchKernelGGL((memory_chunk_kernel<T, TILES, RESULTS>), dim3(block_tiles, heads, Z), dim3(CWM_WAVE * TILES), 0, stream, \
                      (const T*)src, src_stride, q_off, k_off, v_off, q_scale, (const float*)scores, (const float*)wd,       \
-                     state, state_stride, head_elems, cu_q, state_slots, y, nq, saved, n_seqs, heads, d, e, d_pad)
+                     state, state_stride, head_elems, cu_q, state_slots, y, nq, saved, places, n_seqs, heads, d, e, d_pad)
 #define CWM_MEMORY_BLOCKS(T, RPT, TILES)                                                                                    \
   do {                                                                                                                      \
     hipLaunchKernelGGL((memory_scores_kernel<T, RPT>), dim3(numbered, heads), dim3(MEMC_THREADS), 0, stream, (const T*)src,  \
                        src_stride, q_off, k_off, q_scale, (const float*)coef, (const double*)start, cu_q, n_seqs, scores,   \
                        wd, heads, d);                                                                                       \
-    if (saved) {                                                                                                            \
-      CWM_MEMORY_CHUNK(T, TILES, 1, segments);                                                                              \
+    if (places > 0) {                                                                                                       \
+      CWM_MEMORY_CHUNK(T, TILES, false, places);                                                                            \
       hipLaunchKernelGGL((memory_join_kernel<TILES>), dim3(block_tiles, heads, n_seqs), dim3(CWM_WAVE * TILES), 0, stream,   \
                          (const float*)coef, (const double*)start, (const float*)state, state_stride, head_elems, cu_q,     \
                          state_slots, saved, heads, e, d_pad);                                                              \
-      CWM_MEMORY_CHUNK(T, TILES, 2, segments);                                                                              \
-    } else {                                                                                                                \
-      CWM_MEMORY_CHUNK(T, TILES, 0, n_seqs);                                                                                \
     }                                                                                                                       \
+    CWM_MEMORY_CHUNK(T, TILES, true, places + n_seqs);                                                                      \
   } while (0)
 #define CWM_MEMORY(T)                                                                                                       \
   do {                                                                                                                      \

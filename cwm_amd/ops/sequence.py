@@ -6,7 +6,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
-from typing import Any, Optional
+from typing import Any, Optional, Tuple
 
 import torch
 
@@ -429,20 +429,20 @@ def add_layernorm(
 
 # --------------------------------------------------------------------------- #
 MAX_MEMORY_DIM = 256  # csrc/matrix_memory.hip: MEM_MAX_DIM
-# From so many tokens a portion's blocks are walked in segments of 256 side by side: a chain of 48 blocks (1,531 tokens, 16 heads of 128)
-# takes 189 us in one piece and 32 + 7 + 77 us in segments, which do half as much again; a portion of one segment gains nothing.
-MEMORY_SEGMENTS_FROM = 512
 MEMORY_WALK = 8  # tokens of the longest portion that a step still walks one by one; longer ones go in blocks of tokens
 
 
-_MEMORY_BLOCK_TOKENS = None
+_MEMORY_SIZES = None
 
 
-def _memory_block_tokens() -> int:
-    global _MEMORY_BLOCK_TOKENS
-    if _MEMORY_BLOCK_TOKENS is None:
-        _MEMORY_BLOCK_TOKENS = int(_build.load("matrix_memory").cwm_matrix_memory_block_tokens())
-    return _MEMORY_BLOCK_TOKENS
+def _memory_sizes() -> Tuple[int, int]:
+    """(tokens of a block, tokens from which on a portion is walked in segments), as the library has them."""
+    global _MEMORY_SIZES
+    if _MEMORY_SIZES is None:
+        lib = _build.load("matrix_memory")
+        lib.cwm_matrix_memory_saved_floats.restype = ctypes.c_long
+        _MEMORY_SIZES = int(lib.cwm_matrix_memory_block_tokens()), int(lib.cwm_matrix_memory_segments_from())
+    return _MEMORY_SIZES
 
 
 def matrix_memory_state_elems(heads: int, dim: int, vdim: int) -> int:
@@ -502,10 +502,10 @@ def matrix_memory(
     if q_lens and max(q_lens) > MEMORY_WALK:
         start = torch.empty((batch.n_seqs, heads), dtype=torch.float64, device=proj.device)
         nq = torch.empty((n_tokens, heads), dtype=torch.float32, device=proj.device)
-        scores = torch.empty((n_tokens, heads, _memory_block_tokens() + 2), dtype=torch.float32, device=proj.device)
-        if max(q_lens) >= MEMORY_SEGMENTS_FROM:
-            lib.cwm_matrix_memory_saved_floats.restype = ctypes.c_long
-            floats = lib.cwm_matrix_memory_saved_floats(ctypes.c_int(n_tokens), ctypes.c_int(batch.n_seqs), ctypes.c_int(heads), ctypes.c_int(dim), ctypes.c_int(vdim))
+        block_tokens, segments_from = _memory_sizes()
+        scores = torch.empty((n_tokens, heads, block_tokens + 2), dtype=torch.float32, device=proj.device)
+        if max(q_lens) >= segments_from:
+            floats = lib.cwm_matrix_memory_saved_floats(ctypes.c_int(n_tokens), ctypes.c_int(heads), ctypes.c_int(dim), ctypes.c_int(vdim))
             saved = torch.empty(floats, dtype=torch.float32, device=proj.device)
     _check(
         lib,
@@ -515,8 +515,7 @@ def matrix_memory(
             _ptr(gates), ctypes.c_long(gates.stride(0) if n_tokens > 1 else 2 * heads), ctypes.c_float(cap),
             ctypes.c_float(dim ** -0.5 if q_scale is None else q_scale), _ptr(state), ctypes.c_long(state.shape[1]), ctypes.c_int(state.shape[0]),
             _ptr(batch.cu_q), _ptr(batch.state_slots), ctypes.c_int(batch.n_seqs), ctypes.c_int(n_tokens),
-            _ptr(coef), _ptr(y), _ptr(start), _ptr(nq), _ptr(scores), _ptr(saved), _ptr(weight), ctypes.c_float(eps), _ptr(out), ctypes.c_int(heads), ctypes.c_int(dim),
-            ctypes.c_int(vdim), _stream(),
+            _ptr(coef), _ptr(y), _ptr(start), _ptr(nq), _ptr(scores), _ptr(saved), _ptr(weight), ctypes.c_float(eps), _ptr(out), ctypes.c_int(heads), ctypes.c_int(dim), ctypes.c_int(vdim), _stream(),
         ),
     )
     return out
