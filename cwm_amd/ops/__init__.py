@@ -379,13 +379,15 @@ def gemm_bf16_stream(
     glu: bool = False,
     streamed: Optional[torch.Tensor] = None,
     rows_per_input: Optional[int] = None,
+    keep_sums: bool = False,
 ) -> torch.Tensor:
     """bfloat16 x [M <= 64, K] @ weight[N, K]^T with persistent blocks that keep x in
     registers and stream the weight once.  `streamed` is the matrix's streaming copy
     (`stream_layout(weight)`); with it the kernel reads that copy, in whole cache lines and past the
     caches, instead of `weight`.  Returns [M, N]; with `partials_ok` it may
     return float32 partial sums [P, M, N] of a split K for the caller to add (the
-    residual-add + RMSNorm kernel takes them).  `rope`
+    residual-add + RMSNorm kernel takes them); with `keep_sums` it then does so (P = 1) for a K that is not
+    split too, instead of a result of a shorter type, so that nothing is rounded between the product and what follows.  `rope`
     (positions, seq_of_token, inv_freq, cache, block_table, n_q_heads, n_kv_heads,
     head_dim) makes the epilogue rotate the q and k columns and write k and v into the
     paged cache (see `qkv_rope_write`).  `glu`: the weight's rows are gate and up rows in
@@ -440,7 +442,9 @@ def gemm_bf16_stream(
             tiles_a_block += 1
         blocks = k_split * ((inputs - 1) * a_input + rest)
         input_args = (ctypes.c_long(input_stride), ctypes.c_int(per), ctypes.c_int(a_input))
-    if k_split == 1:
+    if k_split == 1 and partials_ok and keep_sums and out_dtype != torch.float32:
+        out = torch.empty((1, m, n), dtype=torch.float32, device=x.device)  # the consumer adds float32 sums, here one
+    elif k_split == 1:
         out = torch.empty((m, n // 2 if glu else n), dtype=out_dtype, device=x.device)
     else:
         out = torch.empty((k_split, m, n), dtype=torch.float32, device=x.device)
@@ -785,7 +789,9 @@ def gemm_bf16(
     if _prefers_tile(x, weight, bias, streamed):
         return gemm_bf16_tile(x, weight, None, out_dtype, partials_ok)
     if m <= STREAM_MAX_ROWS:
-        return gemm_bf16_stream(x, weight, bias, out_dtype, partials_ok, streamed=streamed)
+        # where the tiled kernel would leave partial sums, the sums of an unsplit K are not rounded either
+        keep_sums = partials_ok and bias is None and m > STREAM_FUSED_ROWS and _tile_wins(x, weight)
+        return gemm_bf16_stream(x, weight, bias, out_dtype, partials_ok, streamed=streamed, keep_sums=keep_sums)
     if out_dtype == torch.float32:
         y = torch.mm(x, weight.t(), out_dtype=torch.float32)  # bfloat16 operands, float32 sums written as they are
         return y if bias is None else y + bias.float()

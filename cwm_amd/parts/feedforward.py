@@ -54,8 +54,8 @@ register_part("feed_forward", "swiglu", SwiGLU)
 
 class ActivatedMLP(FeedForward):
     """W_down act(W_up x), no gate and no biases; `activation` is one of `ops.ACTIVATIONS` ("relu2": the square of
-    relu).  The activation is computed in float32 on the product's sums and rounded once.  `up` and `down` are
-    the tensors' local names."""
+    relu).  The activation is computed in float32 on the product's sums (rounded before as `GatedMLP` says) and
+    rounded once.  `up` and `down` are the tensors' local names."""
 
     replayable = True
 
@@ -87,7 +87,8 @@ class GatedMLP(FeedForward):
     u' = clamp(u, -act_limit, act_limit);  "gelu_tanh": gelu(g) * u, the tanh form.  With `row_gate` (a tensor's local name, [1, dim]) the whole result is
     multiplied by sigmoid(w . x), one number a token: the gate's row rides as one more output of the joined gate/up
     product and scales the activation's rows, which the linear down product carries through.  The activation is
-    computed in float32 on the product's sums and rounded once.  `gate`, `up`, `down`: the tensors' local names."""
+    computed in float32 on the product's sums and rounded once (sums that one block finishes are rounded before, to the
+    activations' type, for up to 8 rows, in the tiled kernel and where that does not take the sizes, and so are the library's).  `gate`, `up`, `down`: the tensors' local names."""
 
     replayable = True
 
