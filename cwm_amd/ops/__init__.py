@@ -192,7 +192,7 @@ def gate_up_silu(
         and x.shape[0] <= STREAM_EPILOGUE_ROWS and _stream_takes(x, weight)
         and x.shape[1] <= stream_unsplit_k(x.shape[0])  # K fits one group of wavefronts: no split
     )
-    tiled = x.is_cuda and x.dim() == 2 and _prefers_tile(x, weight, bias, streamed)
+    tiled = x.is_cuda and x.dim() == 2 and _prefers_tile(x, weight, bias, streamed, fused)
     if fused and not tiled:
         return gemm_bf16_stream(x, weight, bias, torch.bfloat16, glu=True, streamed=streamed)
     if tiled and grouped and x.shape[0] <= TILE_ROWS:
@@ -348,10 +348,11 @@ def _stream_block_shape(m: int) -> Tuple[int, int]:
     return shape
 
 
-def stream_unsplit_k(m: int) -> int:
+def stream_unsplit_k(m: int, fused: bool = True) -> int:
     """The longest K that one group of wavefronts of the streaming product holds for `m` rows, so that K is not
-    split over blocks: the fused epilogues (rotation + cache write, gated activation) need that."""
-    waves, regs = _stream_block_shape(m)
+    split over blocks: the fused epilogues (rotation + cache write, gated activation) need that.  Products without an
+    epilogue are split from 17 rows on as for 64, so that a row's bits are the same."""
+    waves, regs = _stream_block_shape(m if m <= 16 or fused else STREAM_MAX_ROWS)
     return 32 * waves * regs
 
 
@@ -417,12 +418,11 @@ def gemm_bf16_stream(
         raise KernelError(f"gemm: bias {tuple(bias.shape)} does not fit {n} outputs")
     out_dtype = out_dtype or torch.bfloat16
     lib = _build.load("gemm_bf16_stream")
-    # from 17 rows on K is split as for 64, so that a row's bits are the same; the fused epilogues take the longer K that 32 rows' registers hold
-    waves, regs = _stream_block_shape(m if m <= 16 or rope is not None or glu else STREAM_MAX_ROWS)
+    waves = _stream_block_shape(m)[0]
     steps = (k + 31) // 32
     n_tiles = (n + 15) // 16
     cus = _compute_units(x.device)
-    k_split = -(-steps // (waves * regs))  # K longer than one group of wavefronts' registers is split
+    k_split = -(-steps * 32 // stream_unsplit_k(m, rope is not None or glu))  # K longer than one group of wavefronts' registers is split
     if (rope is not None or glu) and (k_split != 1 or m > STREAM_EPILOGUE_ROWS):
         raise KernelError("the fused epilogues need at most 32 rows and a K that one group of wavefronts holds")
     if glu:
@@ -529,7 +529,7 @@ def qkv_rope_write(
         and head_dim <= 256
         and _stream_takes(x, weight)
         and x.shape[1] <= stream_unsplit_k(x.shape[0])  # K fits one group of wavefronts: no split
-        and not _prefers_tile(x, weight, bias, streamed)
+        and not _prefers_tile(x, weight, bias, streamed, True)
     )
     if fused:
         _i32(positions, "positions")
@@ -717,20 +717,23 @@ TILE_COLUMNS = 128  # columns of a tall block's tile
 TILE_FEW_ROWS_ENTRIES = 1 << 24
 
 
-def _prefers_tile(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], streamed: Optional[torch.Tensor] = None) -> bool:
+def _prefers_tile(
+    x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], streamed: Optional[torch.Tensor] = None, fused: bool = False,
+) -> bool:
     """Whether this product goes to the tiled kernel (which has no bias of its own): from 33 rows on, from 9 on where
     the matrix has no streaming copy or is not among those of `STREAM_LEAST_ENTRIES` to `STREAM_WHOLE_ENTRIES`; and for
     fewer rows where the matrix is large and has no streaming copy, since the tiled kernel reads the row-major
     matrix in whole cache lines past the caches, which the streaming kernel can only do with that copy (a
     layer's four products of the 32B shape at 8 rows: 159 us tiled, 187 us streamed from the row-major
-    matrices, 159 us streamed from the copies; at 1 row 163, 178 and 154 us)."""
+    matrices, 159 us streamed from the copies; at 1 row 163, 178 and 154 us).  `fused`: whether the streaming product
+    would have an epilogue, which takes a longer K without a split."""
     if bias is not None:
         return False
     m = x.shape[0]
     if m <= STREAM_FUSED_ROWS and (streamed is not None or weight.numel() < TILE_FEW_ROWS_ENTRIES):
         return False
     if m <= STREAM_EPILOGUE_ROWS and streamed is not None and weight.numel() >= STREAM_LEAST_ENTRIES:
-        if weight.numel() < (STREAM_WHOLE_ENTRIES if weight.shape[1] <= stream_unsplit_k(m) else STREAM_SPLIT_ENTRIES):
+        if weight.numel() < (STREAM_WHOLE_ENTRIES if weight.shape[1] <= stream_unsplit_k(m, fused) else STREAM_SPLIT_ENTRIES):
             return False
     return _tile_wins(x, weight)
 

@@ -1,0 +1,31 @@
+"""Which kernel a product of few rows goes to: the rule and the kernel agree on where K is split (host arithmetic only)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from cwm_amd import ops
+
+
+def matrices(m, n, k):
+    """Operands that nothing reads, and a stand-in for the streaming copy."""
+    return torch.empty((m, k), dtype=torch.bfloat16), torch.empty((n, k), dtype=torch.bfloat16), torch.empty(0)
+
+
+@pytest.mark.parametrize("m", [9, 16, 17, 24, 32])
+@pytest.mark.parametrize("k", [2048, 2112, 3072, 3136, 6144, 6208])
+def test_the_limit_is_that_of_a_split_k(m, k):
+    """2^25 entries for products that split K, 2^27 for those that do not: the plain product of 17 to 32 rows splits from a K
+    of 2,048, with an epilogue from 3,072, of up to 16 rows both from 6,144."""
+    x, w, copy = matrices(m, (1 << 25) // k + 16 & -16, k)
+    for fused, most in ((False, 6144 if m <= 16 else 2048), (True, 6144 if m <= 16 else 3072)):
+        assert ops.stream_unsplit_k(m, fused) == most
+        assert ops._prefers_tile(x, w, None, copy, fused) == (k > most)
+    x, w, copy = matrices(m, (1 << 27) // k + 16 & -16, k)
+    assert ops._prefers_tile(x, w, None, copy, False) and ops._prefers_tile(x, w, None, copy, True)
+
+
+def test_a_head_of_24_rows_is_one_launch_of_whole_tiles():
+    x, w, copy = matrices(24, 32768, 3072)
+    assert ops._prefers_tile(x, w, None, copy)
