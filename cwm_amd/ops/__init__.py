@@ -705,6 +705,13 @@ STREAM_EPILOGUE_ROWS = 32  # rows up to which its epilogues go
 # 2,048 x 8,192 11.3 / 13.0 and 12.6 / 14.0, 3,072 x 9,216 15.4 / 17.4 and 16.9 / 18.3, but 4,096 x 14,336 26.6 / 24.8 and 28.1 / 25.9.
 STREAM_WHOLE_ENTRIES = 1 << 27
 STREAM_SPLIT_ENTRIES = 1 << 25
+# Wide results of a short K are the tiled kernel's: its blocks own whole tiles there, while a streaming block pays its sum over
+# the wavefronts for one 16-column tile after the other.  Streamed / tiled, us, at 9 rows and at 17: 24,576 x 512 11.0 / 8.7 and
+# 9.1 / 8.9, 32,768 x 512 14.3 / 9.6 and 11.0 / 9.2, 32,768 x 768 13.6 / 11.6 and 11.3 / 11.8, 128,256 x 512 46 / 25 and 35 / 26; but 16,384 x
+# 256 7.6 / 8.8 and 6.7 / 8.9, 20,480 x 1,024 11.4 / 14.1 and 9.6 / 14.7.  At a K of 1,024, 32,768 columns 16.3 / 15.1 and 12.9 / 14.1,
+# 128,256 50 / 44 and 46 / 48.
+STREAM_WIDE, STREAM_WIDE_K = 20480, 1024
+STREAM_WIDER = 32768  # up to 16 rows the K of 1,024 itself is short from here on
 # Matrices of fewer entries than this (half a megabyte, which reading does not bound) stay with the tiled product from 9 rows on
 # whether they have a copy or not, so that the bits of a small model do not depend on its copies.
 STREAM_LEAST_ENTRIES = 1 << 18
@@ -717,11 +724,15 @@ TILE_COLUMNS = 128  # columns of a tall block's tile
 TILE_FEW_ROWS_ENTRIES = 1 << 24
 
 
+def _wide_and_short(m: int, n: int, k: int) -> bool:
+    return k < STREAM_WIDE_K and n >= STREAM_WIDE or k == STREAM_WIDE_K and n >= STREAM_WIDER and m <= 16
+
+
 def _prefers_tile(
     x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], streamed: Optional[torch.Tensor] = None, fused: bool = False,
 ) -> bool:
     """Whether this product goes to the tiled kernel (which has no bias of its own): from 33 rows on, from 9 on where
-    the matrix has no streaming copy or is not among those of `STREAM_LEAST_ENTRIES` to `STREAM_WHOLE_ENTRIES`; and for
+    the matrix has no streaming copy, is not among those of `STREAM_LEAST_ENTRIES` to `STREAM_WHOLE_ENTRIES` or wide and short; and for
     fewer rows where the matrix is large and has no streaming copy, since the tiled kernel reads the row-major
     matrix in whole cache lines past the caches, which the streaming kernel can only do with that copy (a
     layer's four products of the 32B shape at 8 rows: 159 us tiled, 187 us streamed from the row-major
@@ -732,7 +743,7 @@ def _prefers_tile(
     m = x.shape[0]
     if m <= STREAM_FUSED_ROWS and (streamed is not None or weight.numel() < TILE_FEW_ROWS_ENTRIES):
         return False
-    if m <= STREAM_EPILOGUE_ROWS and streamed is not None and weight.numel() >= STREAM_LEAST_ENTRIES:
+    if m <= STREAM_EPILOGUE_ROWS and streamed is not None and weight.numel() >= STREAM_LEAST_ENTRIES and not _wide_and_short(m, *weight.shape):
         if weight.numel() < (STREAM_WHOLE_ENTRIES if weight.shape[1] <= stream_unsplit_k(m, fused) else STREAM_SPLIT_ENTRIES):
             return False
     return _tile_wins(x, weight)

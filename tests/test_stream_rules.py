@@ -29,3 +29,13 @@ def test_the_limit_is_that_of_a_split_k(m, k):
 def test_a_head_of_24_rows_is_one_launch_of_whole_tiles():
     x, w, copy = matrices(24, 32768, 3072)
     assert ops._prefers_tile(x, w, None, copy)
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("m,n,k,tiled", [
+    (9, 32768, 512, True), (32, 32768, 512, True), (16, 128256, 512, True), (17, 20480, 960, True), (9, 20464, 960, False), (9, 16384, 256, False),
+    (16, 32768, 1024, True), (17, 32768, 1024, False), (16, 32752, 1024, False), (16, 32768, 1088, False), (8, 32768, 512, False), (9, 20480, 1024, False),
+])
+def test_wide_results_of_a_short_k_are_tiled(m, n, k, tiled, fused):
+    x, w, copy = matrices(m, n, k)
+    assert ops._prefers_tile(x, w, None, copy, fused) == tiled
