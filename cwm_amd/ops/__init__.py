@@ -697,7 +697,7 @@ def gemm_bf16_tile(
 # rows up to which the streaming product (x in registers, every epilogue in the kernel) is preferred whatever the matrix
 STREAM_FUSED_ROWS = 8
 STREAM_EPILOGUE_ROWS = 32  # rows up to which its epilogues go
-# From 9 to 32 rows the streaming product is ahead for matrices of fewer entries than these, where there is a streaming copy: it
+# From 9 to 32 rows the streaming product from a copy is ahead for matrices of fewer entries than these: it
 # rotates, writes the cache and applies the gate in its epilogue, and leaves one to four partial sums where the tiled one, whose
 # blocks share tiles of a small matrix, leaves up to 16.  Measured with the kernels that then follow, streamed / tiled, us: q/k/v of
 # 3,072 x 2,048 6.5 / 13.1 at 12 rows and 7.9 / 13.5 at 24, of 6,144 x 4,096 14.8 / 20.5 at 12, of 8,192 x 6,144 21.0 / 24.2; gate/up
@@ -712,9 +712,14 @@ STREAM_SPLIT_ENTRIES = 1 << 25
 # 128,256 50 / 44 and 46 / 48.
 STREAM_WIDE, STREAM_WIDE_K = 20480, 1024
 STREAM_WIDER = 32768  # up to 16 rows the K of 1,024 itself is short from here on
-# Matrices of fewer entries than this (half a megabyte, which reading does not bound) stay with the tiled product from 9 rows on
-# whether they have a copy or not, so that the bits of a small model do not depend on its copies.
-STREAM_LEAST_ENTRIES = 1 << 18
+# Matrices of fewer entries than this are streamed from 9 to 32 rows whether they have a copy or not, so that a copy does not
+# decide on bits there (as below `TILE_FEW_ROWS_ENTRIES` up to 8 rows).  Streamed row-major / tiled, us, with the norm that follows, at 9 and
+# 32 rows: 256 x 512 5.8 / 9.5 and 5.7 / 9.9, 1,024 x 2,048 7.0 / 9.6 and 7.1 / 10.1, 2,048 x 2,048 8.0 / 9.8 and 8.9 / 10.5, 512 x 8,064 7.7 / 12.4 and
+# 9.3 / 13.1; above, the copy is what makes it worth while: 1,536 x 4,608 10.4 / 10.9 and 13.0 / 12.0, 2,048 x 6,144 11.2 / 11.5 and 15.1 / 12.9.
+STREAM_ANY_ENTRIES = 1 << 22
+# The smallest matrices (64 KB, a test model's) stay with the tiled kernel from 9 rows on, with a copy or without: some 2 us a product
+# (208 x 128 8.3 instead of 5.9 us) are not worth other bits for what such models give.
+STREAM_LEAST_ENTRIES = 1 << 15
 TILE_ROWS = 128  # rows up to which the tiled product is the fastest whatever the shape
 TILE_TALL_ROWS = 256  # rows of its tallest block: up to there it reads W once
 TILE_COLUMNS = 128  # columns of a tall block's tile
@@ -731,20 +736,22 @@ def _wide_and_short(m: int, n: int, k: int) -> bool:
 def _prefers_tile(
     x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], streamed: Optional[torch.Tensor] = None, fused: bool = False,
 ) -> bool:
-    """Whether this product goes to the tiled kernel (which has no bias of its own): from 33 rows on, from 9 on where
-    the matrix has no streaming copy, is not among those of `STREAM_LEAST_ENTRIES` to `STREAM_WHOLE_ENTRIES` or wide and short; and for
-    fewer rows where the matrix is large and has no streaming copy, since the tiled kernel reads the row-major
-    matrix in whole cache lines past the caches, which the streaming kernel can only do with that copy (a
-    layer's four products of the 32B shape at 8 rows: 159 us tiled, 187 us streamed from the row-major
-    matrices, 159 us streamed from the copies; at 1 row 163, 178 and 154 us).  `fused`: whether the streaming product
-    would have an epilogue, which takes a longer K without a split."""
+    """Whether this product goes to the tiled kernel (which has no bias of its own): from 33 rows on; from 9 on where
+    the matrix is among the smallest (`STREAM_LEAST_ENTRIES`), wide and short, or so large that it pays to read it
+    row-major in whole cache lines past the caches, which the streaming kernel can only do with a copy
+    (`STREAM_WHOLE_ENTRIES` and `STREAM_SPLIT_ENTRIES` with one, `STREAM_ANY_ENTRIES` without); and for fewer rows
+    where the matrix is large and has no streaming copy (a layer's four products of the 32B shape at 8 rows: 159 us tiled,
+    187 us streamed from the row-major matrices, 159 us streamed from the copies; at 1 row 163, 178 and 154 us).
+    `fused`: whether the streaming product would have an epilogue, which takes a longer K without a split."""
     if bias is not None:
         return False
     m = x.shape[0]
     if m <= STREAM_FUSED_ROWS and (streamed is not None or weight.numel() < TILE_FEW_ROWS_ENTRIES):
         return False
-    if m <= STREAM_EPILOGUE_ROWS and streamed is not None and weight.numel() >= STREAM_LEAST_ENTRIES and not _wide_and_short(m, *weight.shape):
-        if weight.numel() < (STREAM_WHOLE_ENTRIES if weight.shape[1] <= stream_unsplit_k(m, fused) else STREAM_SPLIT_ENTRIES):
+    n, k = weight.shape
+    if STREAM_FUSED_ROWS < m <= STREAM_EPILOGUE_ROWS and n * k >= STREAM_LEAST_ENTRIES and not _wide_and_short(m, n, k):
+        with_copy = STREAM_WHOLE_ENTRIES if k <= stream_unsplit_k(m, fused) else STREAM_SPLIT_ENTRIES
+        if n * k < (STREAM_ANY_ENTRIES if streamed is None else with_copy):
             return False
     return _tile_wins(x, weight)
 
@@ -787,8 +794,8 @@ def gemm_bf16(
 ) -> torch.Tensor:
     """bfloat16 x [M, K] @ bfloat16 weight[N, K]^T, float32 accumulation.
 
-    Up to 8 rows, and up to 32 for all but the largest matrices that have a streaming copy: the hand-written persistent
-    weight-streaming kernel, x in registers.
+    Up to 8 rows, and up to 32 for all but the smallest and the largest matrices (`_prefers_tile`): the hand-written
+    persistent weight-streaming kernel, x in registers.
     Up to 128 rows (256 for a result of at most 16,384 columns): the hand-written tiled kernel, x and W
     through LDS (it needs K % 64 == 0 and N % 16 == 0; other sizes of up to 64 rows stream).
     More rows: the library product (hipBLASLt through torch), as the reference calls a

@@ -57,11 +57,33 @@ def test_fused_epilogues(m, k):
 def test_which_products_stream(m):
     from cwm_amd import ops
 
-    for n, k, streams in ((256, 512, False), (1024, 512, True), (1 << 12, (1 << 13) + 64, False), ((1 << 15) - 16, 1 << 12, m <= 16)):
+    for n, k, streams in ((208, 128, False), (256, 512, True), (1024, 512, True), (1 << 12, (1 << 13) + 64, False), ((1 << 15) - 16, 1 << 12, m <= 16)):
         x, w = drawn(m, n, k)
         copy = ops.stream_layout(w)
         got = ops.linear(x, w, None, torch.float32, partials_ok=True, streamed=copy)
         tiled = ops.gemm_bf16_tile(x, w, None, torch.float32, partials_ok=True)
         chosen = ops.gemm_bf16_stream(x, w, None, torch.float32, partials_ok=True, streamed=copy) if m <= 32 and streams else tiled
         assert torch.equal(got, chosen)
-        assert torch.equal(ops.linear(x, w, None, torch.float32, partials_ok=True), tiled)  # without a copy
+        without = ops.linear(x, w, None, torch.float32, partials_ok=True)
+        assert torch.equal(without, chosen if n * k < 1 << 22 else tiled)
+
+
+@pytest.mark.parametrize("m", [9, 16, 17, 32])
+@pytest.mark.parametrize("n,k", [(512, 64), (320, 512), (768, 1088), (1024, 4032), (256, 8192)])
+def test_a_copy_changes_no_bit_below_its_limit(m, n, k):
+    """Every way a product of these sizes is called: plain, as partial sums, with the gate, with the rotation and cache write."""
+    from cwm_amd import ops
+
+    x, w = drawn(m, n, k)
+    copy = ops.stream_layout(w)
+    assert torch.equal(ops.linear(x, w), ops.linear(x, w, streamed=copy))
+    assert torch.equal(ops.linear(x, w, None, partials_ok=True), ops.linear(x, w, None, partials_ok=True, streamed=copy))
+    assert torch.equal(ops.gate_up_silu(x, w, None, True), ops.gate_up_silu(x, w, None, True, streamed=copy))
+    hd, n_kv = 32, n // 128
+    positions = torch.arange(m, device=DEV, dtype=torch.int32) % 16
+    seq = torch.arange(m, device=DEV, dtype=torch.int32)
+    caches = [torch.zeros((m, 2, n_kv, 16 * hd), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    wq = w[: 4 * n_kv * hd].contiguous()
+    got = [ops.qkv_rope_write(x, wq, None, 2 * n_kv, n_kv, hd, positions, torch.rand(hd // 2, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1)),
+                              cache, seq[:, None].contiguous(), seq, streamed=s) for cache, s in zip(caches, (None, ops.stream_layout(wq)))]
+    assert torch.equal(*got) and torch.equal(*caches)
