@@ -356,7 +356,9 @@ __global__ void __launch_bounds__(1024) group_by_expert_kernel(const int* __rest
 // Few tokens (a decode step): the router's product, the choice and the grouping in one launch of one block, each of which is a few
 // microseconds of latency as a launch of its own (eight tokens, 16 experts, K = 2,048: 4.8 + 4.4 + 4.3 us).  The
 // product is that of gemm_bf16_stream.hip on one tile of columns after the other, its sums in the same order: the 16 wavefronts
-// share K, and add their parts through LDS.  w: the router's streaming copy [tiles of 16 experts][K / 32][64][8].
+// share K, and add their parts through LDS.  Bound by its rounds of loads, four steps of 32 a wavefront at a time and one tile of 16
+// experts after the other: `route_group_pays` says up to where that is less than three launches.  w: the router's streaming copy
+// [tiles of 16 experts][K / 32][64][8].
 #define ROUTE_GROUP_TOKENS 16
 #define ROUTE_GROUP_STEPS 16  // of 32 along K, at most, a wavefront
 

@@ -118,13 +118,25 @@ def _empty_groups(n: int, top: int, n_experts: int, device: torch.device) -> Exp
 ROUTE_GROUP_TOKENS = 16  # csrc/routed.hip: ROUTE_GROUP_TOKENS
 ROUTE_GROUP_EXPERTS = 64
 ROUTE_GROUP_MAX_K = 8192  # csrc/routed.hip: 16 * 32 * ROUTE_GROUP_STEPS
+# Its one block reads the router 16 experts after the other, so it is ahead of the three launches for so many and a K of up to
+# 4,096 only.  One launch / three, us, weights not in a cache, at 1, 8 and 16 tokens: 16 experts, K = 1,024 7.8 / 9.5, 8.5 / 10.3, 9.1 / 10.1;
+# 2,048 8.7 / 10.9, 9.5 / 11.7, 10.7 / 12.6; 4,096 10.3 / 13.2, 11.8 / 14.9, 13.7 / 16.0; 8,192 13.1 / 14.6, 16.5 / 16.2, 20.7 / 17.8; 8 experts, 4,096 9.6 /
+# 11.5, 10.9 / 12.9, 13.4 / 14.4; 32 experts, 1,024 10.3 / 10.5, 11.5 / 11.3, 14.1 / 11.3; 2,048 11.3 / 11.6, 13.6 / 12.1, 15.5 / 13.4; 4,096 14.8 /
+# 14.0, 17.4 / 15.3, 21.9 / 17.0; 64 experts, 2,048 18.0 / 13.0, 20.7 / 13.6, 24.9 / 14.7; 8,192 35 / 17, 48 / 19, 61 / 20.
+ROUTE_GROUP_PAYS_EXPERTS, ROUTE_GROUP_PAYS_K = 16, 4096
+
+
+def route_group_pays(n_experts: int, k: int) -> bool:
+    """Whether a step of few tokens makes logits, choices and lists of such a router faster in one launch than in three."""
+    return n_experts <= ROUTE_GROUP_PAYS_EXPERTS and k % 32 == 0 and k <= ROUTE_GROUP_PAYS_K
 
 
 def route_and_group(
     x: torch.Tensor, router_copy: torch.Tensor, bias: Optional[torch.Tensor], n_experts: int, top: int, scores: str = "softmax_chosen",
     correction: Optional[torch.Tensor] = None, scale: float = 1.0, renormalize: bool = False, groups: Optional[Tuple[int, int]] = None,
 ) -> Tuple[torch.Tensor, torch.Tensor, ExpertGroups]:
-    """(chosen, weights, lists): what `route_top` and `group_by_expert` make of the logits W x + bias, in one launch, the same bits.
+    """(chosen, weights, lists): what `route_top` and `group_by_expert` make of the logits W x + bias, in one launch; the logits are added in the
+    streaming product's order, so the bits are the same where that does not split K (up to 6,144).
     `x` bfloat16 [T <= 16, K] (K a multiple of 32, up to 8,192), `router_copy` the streaming copy (`stream_layout`) of the
     bfloat16 router [E <= 64, K], `bias` float32 [E] or None; the rest as in `route_top`."""
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()

@@ -86,7 +86,7 @@ class RoutedExperts(FeedForward):
         self.router_copy: Optional[torch.Tensor] = None
         if (
             runtime.device.type == "cuda" and runtime.act_dtype == torch.bfloat16 and self.router.dtype == torch.bfloat16
-            and self.n_experts <= ops.ROUTE_GROUP_EXPERTS and self.dim % 32 == 0 and self.dim <= ops.ROUTE_GROUP_MAX_K
+            and ops.route_group_pays(self.n_experts, self.dim)
         ):
             self.router_copy = ops.stream_layout(self.router)
         self.choice_correction = tensors["correction"].float().contiguous() if self.correction else None
