@@ -490,7 +490,7 @@ __global__ void __launch_bounds__(256) selective_scan_single_kernel(const T* __r
 // C_t . B_s are products of bfloat16 values (exact, float32 sums).  The other products have one float32 operand each (S, the
 // weighted x, the scores), which goes in as three bfloat16 parts that hold all its bits, so that every single product is exact
 // and no value is rounded that the walk keeps: three v_mfma_f32_16x16x32_bf16 of 16 cycles for eight v_mfma_f32_16x16x4_f32 of
-// 32 (2,048 tokens 154 us with those, 3.8e-7 off float64 instead of 2.4e-7).  The L are summed in float64: a difference of two
+// 32 (2,048 tokens 154 us with those; off float64, on the same 1,025 tokens of 8 heads of 64 x 128, 3.9e-7 instead of 2.4e-7).  The L are summed in float64: a difference of two
 // of them is as exact as the decays between them.  A wavefront has 16 columns of the head: its part of the state stays in
 // registers as the matrix instruction leaves it (lane 16 j + r: column r, rows 16 q + 4 j + i), and two such tiles are also the
 // operand that C needs, with its values of k in the order 4 j + i, 16 + 4 j + i; likewise two tiles of x.  The other operand is
@@ -500,12 +500,13 @@ __global__ void __launch_bounds__(256) selective_scan_single_kernel(const T* __r
 // Portions of one segment, decoded tokens among them, are left to the walk: their bits and their cost are what they are without a
 // long portion beside them (in blocks a decoded token pays for 64).
 // Bound by the waits between a block's stages, two blocks a compute unit (three in MODE 1; asked for, since the registers beyond
-// the first 256 would leave one), and by splitting values on the vector units; the walk was bound by its reads of B and C from LDS.
+// the first 256 would leave one), and by splitting values on the vector units (looking for infinities among B and C costs 2 of 115 us); the walk was bound by its reads of B and C from LDS.
 #define BLOCK_TOKENS 64
 
 // Eight float32 values as the operands of three bfloat16 matrix products whose sum is the product of the values: each part is
-// the leading eight bits of what the parts before leave, so three hold all 24, and with a bfloat16 second operand every single
-// product is exact.  An infinity or a NaN is its first part alone.
+// the leading eight bits of what the parts before leave, so three hold all 24 (of values below 2^-110 the last lie among bfloat16's
+// subnormals and may be lost: less than 2^-125), and with a bfloat16 second operand every single product is exact.  An infinity or
+// a NaN is its first part alone; the other operand has to be finite, since a part may be zero.
 __device__ __forceinline__ void three_parts(const float (&v)[8], Frag8 (&part)[3]) {
   uint32_t w[3][8];
 #pragma unroll
@@ -521,6 +522,27 @@ __device__ __forceinline__ void three_parts(const float (&v)[8], Frag8 (&part)[3
   for (int k = 0; k < 3; ++k)
     part[k].u = make_uint4(__builtin_amdgcn_perm(w[k][1], w[k][0], 0x07060302u), __builtin_amdgcn_perm(w[k][3], w[k][2], 0x07060302u),
                            __builtin_amdgcn_perm(w[k][5], w[k][4], 0x07060302u), __builtin_amdgcn_perm(w[k][7], w[k][6], 0x07060302u));
+}
+
+typedef unsigned short Halves __attribute__((ext_vector_type(2)));
+
+// The larger magnitudes, halves apart, of two bfloat16 values a word; from 0x7f80 on an infinity or a NaN.
+__device__ __forceinline__ Halves larger_magnitudes(Halves so_far, uint32_t w) {
+  return __builtin_elementwise_max(so_far, __builtin_bit_cast(Halves, w & 0x7fff7fffu));
+}
+
+// What is made of this value is made after this place: the compiler would move what both ways of a branch have in common
+// before it, and hold all of it in registers.
+__device__ __forceinline__ int keep_apart(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// Four bfloat16 values of an operand as float32.
+__device__ __forceinline__ void four_floats(const bf16_t* at, float (&c)[4]) {
+  const uint2 w = *(const uint2*)at;
+  c[0] = __uint_as_float(w.x << 16), c[1] = __uint_as_float(w.x & 0xffff0000u);
+  c[2] = __uint_as_float(w.y << 16), c[3] = __uint_as_float(w.y & 0xffff0000u);
 }
 
 // Sixteen bytes of an operand whose eight values of k are 4 j .. + 3 and 16 + 4 j .. + 3 of 32: the order in which two tiles of a
@@ -549,6 +571,7 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
   __shared__ __attribute__((aligned(16))) bf16_t scores[MODE == 2 ? 3 : 1][MODE == 2 ? BLOCK_TOKENS : 1][SCORE_LD];  // in three parts
   __shared__ double sum_log[BLOCK_TOKENS];
   __shared__ __attribute__((aligned(16))) float step_size[BLOCK_TOKENS], from_start[BLOCK_TOKENS], to_end[BLOCK_TOKENS];
+  __shared__ int spoilt;  // whether a B or C of the segment so far was not finite: from there on its products are the float32 instruction's
   const int* entry = segments + 6 * blockIdx.z;
   const int t0 = entry[1], t1 = entry[2], seg = entry[3], seg_base = entry[4], n_segs = entry[5];
   if (n_segs == 1) return;                     // a short portion is walked
@@ -598,12 +621,19 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
   };
   double segment_log = 0.0;  // MODE 1, the first wavefront: of the segment's decay
 
+  if (tid == 0) spoilt = 0;
   fetch(t0);
   for (int c0 = t0; c0 < t1; c0 += BLOCK_TOKENS) {
     __syncthreads();  // the block of tokens before is done with
+    Halves most = {0, 0};
 #pragma unroll
     for (int k = 0; k < LOADS; ++k) {
       const int n = 8 * (4 * k + wave);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        most = larger_magnitudes(most, rb[k][e]);
+        if constexpr (MODE == 2) most = larger_magnitudes(most, rc[k][e]);
+      }
       if constexpr (MODE == 2) {
         *(Words4*)&b_rows[lane][n] = rb[k];
         *(Words4*)&c_rows[lane][n] = rc[k];
@@ -611,6 +641,7 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
 #pragma unroll
       for (int e = 0; e < 8; ++e) b_cols[n + e][lane] = (bf16_t)(rb[k][e >> 1] >> (16 * (e & 1)));
     }
+    if (max(most.x, most.y) >= 0x7f80) spoilt = 1;
     float x[16];
     uint32_t rx_now[8], largest = 0;
 #pragma unroll
@@ -640,6 +671,7 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
       if constexpr (MODE == 1) segment_log += all;
     }
     __syncthreads();
+    const bool all_plain = __builtin_amdgcn_readfirstlane(spoilt) == 0;
     if (c0 + BLOCK_TOKENS < t1) fetch(c0 + BLOCK_TOKENS);  // in flight while this block of tokens is worked on
     if constexpr (MODE == 2) {
       // scores of the wavefront's 16 queries and the keys up to them
@@ -682,17 +714,31 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
         float4v out[4];
 #pragma unroll
         for (int a = 0; a < 4; ++a) out[a] = (float4v){0.f, 0.f, 0.f, 0.f};
+        if (__builtin_expect(all_plain, 1)) {
 #pragma unroll
-        for (int q = 0; q < NT; q += 2) {
-          const float v[8] = {S[q][0], S[q][1], S[q][2], S[q][3], S[q + 1][0], S[q + 1][1], S[q + 1][2], S[q + 1][3]};
-          Frag8 part[3];
-          three_parts(v, part);
+          for (int q = 0; q < NT; q += 2) {
+            const float v[8] = {S[q][0], S[q][1], S[q][2], S[q][3], S[q + 1][0], S[q + 1][1], S[q + 1][2], S[q + 1][3]};
+            Frag8 part[3];
+            three_parts(v, part);
 #pragma unroll
-          for (int a = 0; a < 4; ++a) {
-            const Frag8 c = two_fours(&c_rows[16 * a + r][16 * q + 4 * j]);
+            for (int a = 0; a < 4; ++a) {
+              const Frag8 c = two_fours(&c_rows[16 * a + r][16 * q + 4 * j]);
 #pragma unroll
-            for (int k = 2; k >= 0; --k) out[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c.v, part[k].v, out[a], 0, 0, 0);
+              for (int k = 2; k >= 0; --k) out[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c.v, part[k].v, out[a], 0, 0, 0);
+            }
           }
+        } else {
+          const int row = keep_apart(r);
+#pragma unroll
+          for (int q = 0; q < NT; ++q)
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+              float c[4];
+              four_floats(&c_rows[16 * a + row][16 * q + 4 * j], c);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) out[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(c[i], S[q][i], out[a], 0, 0, 0);
+              __builtin_amdgcn_sched_barrier(0);
+            }
         }
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
@@ -748,23 +794,46 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
     }
     // the state after the block of tokens
     const float whole = from_start[BLOCK_TOKENS - 1];
+    if (__builtin_expect(all_plain, 1)) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) x[k] *= to_end[16 * (k >> 2) + 4 * j + (k & 3)];
-#pragma unroll
-    for (int q = 0; q < NT; ++q) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) S[q][i] *= whole;
-    }
-#pragma unroll
-    for (int b = 0; b < 4; b += 2) {
-      const float v[8] = {x[4 * b], x[4 * b + 1], x[4 * b + 2], x[4 * b + 3], x[4 * b + 4], x[4 * b + 5], x[4 * b + 6], x[4 * b + 7]};
-      Frag8 part[3];
-      three_parts(v, part);
+      for (int k = 0; k < 16; ++k) x[k] *= to_end[16 * (k >> 2) + 4 * j + (k & 3)];
 #pragma unroll
       for (int q = 0; q < NT; ++q) {
-        const Frag8 c = two_fours(&b_cols[16 * q + r][16 * b + 4 * j]);
 #pragma unroll
-        for (int k = 2; k >= 0; --k) S[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c.v, part[k].v, S[q], 0, 0, 0);
+        for (int i = 0; i < 4; ++i) S[q][i] *= whole;
+      }
+#pragma unroll
+      for (int b = 0; b < 4; b += 2) {
+        const float v[8] = {x[4 * b], x[4 * b + 1], x[4 * b + 2], x[4 * b + 3], x[4 * b + 4], x[4 * b + 5], x[4 * b + 6], x[4 * b + 7]};
+        Frag8 part[3];
+        three_parts(v, part);
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          const Frag8 c = two_fours(&b_cols[16 * q + r][16 * b + 4 * j]);
+#pragma unroll
+          for (int k = 2; k >= 0; --k) S[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c.v, part[k].v, S[q], 0, 0, 0);
+        }
+      }
+    } else {
+      const int row = keep_apart(r), group = keep_apart(4 * j);
+#pragma unroll
+      for (int q = 0; q < NT; ++q) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[q][i] *= whole;
+      }
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        float xs[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xs[i] = x[4 * b + i] * to_end[16 * b + group + i];
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          float c[4];
+          four_floats(&b_cols[16 * q + row][16 * b + group], c);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) S[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(c[i], xs[i], S[q], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);  // few values at a time: this seldom walked way must not cost the other one registers
+        }
       }
     }
   }
@@ -870,9 +939,9 @@ extern "C" int cwm_selective_scan(const void* xbc, long xbc_ld, const void* dt_r
   const int unit = dtype == CWM_BF16 ? 8 : 4;
   const bool vec = N % unit == 0 && P % unit == 0 && xbc_ld % unit == 0 && ((uintptr_t)xbc % 16) == 0 && 16 * row / unit <= SCAN_PFV * 256;
   if (segments && dtype == CWM_BF16 && vec && N <= 128 && P % 16 == 0 && ((uintptr_t)seg_state % 16) == 0) {
-    // on the matrix cores: 2,048 tokens of 64 heads, 64 columns and 128 rows in 113 us instead of
-    // 565 (launches included), 300 tokens in 74 instead of 170, 4,096 in 209 instead of 1,126; of float64 it is 2.4e-7 off, the walk
-    // of segments token by token 3.7e-7
+    // on the matrix cores: 2,048 tokens of 64 heads, 64 columns and 128 rows in 115 us instead of
+    // 565 (launches included), 300 tokens in 77 instead of 170, 4,096 in 213 instead of 1,126; off float64, on the same 1,025 tokens
+    // of 8 heads, 2.4e-7, the walk of segments token by token 2.4e-6
     const dim3 blocks((P + 63) / 64, heads, n_segments);
     const long head_elems = (long)SCAN_ROWS * split * P;
 #define CWM_SCAN_BLOCK(NT, MODE)                                                                                                           \
