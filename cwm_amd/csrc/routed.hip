@@ -413,6 +413,7 @@ __global__ void __launch_bounds__(1024) route_group_kernel(const bf16_t* __restr
 }
 
 extern "C" int cwm_route_group_tokens() { return ROUTE_GROUP_TOKENS; }
+extern "C" int cwm_route_group_experts() { return CWM_WAVE; }
 extern "C" int cwm_route_group_max_k() { return 16 * 32 * ROUTE_GROUP_STEPS; }
 
 // x: bfloat16 [n_tokens][x_ld]; w: the router's streaming copy; bias: float32 [n_experts] or null; the choice as in
@@ -754,7 +755,6 @@ __global__ void __launch_bounds__(256) grouped_stream_kernel(const T* __restrict
 // (924 / 743 TFLOP/s) and 105 / 58; with a router's uneven loads 100 / 58 and 135 / 76 (a CU that gets three blocks where others
 // get two decides), 1,500 tokens 72 / 42 and 97 / 53, 4,096 tokens 159 / 99 and 204 / 121, 300 tokens 38 / 20 and 42 / 21.
 #define WIDE_GROUP 4
-#define WIDE_MAX_ROWS 128
 
 // A wavefront's and a block's place in a wide product, and what its loop needs of the kernel's arguments.
 struct WideBlock {

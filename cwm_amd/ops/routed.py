@@ -115,10 +115,19 @@ def _empty_groups(n: int, top: int, n_experts: int, device: torch.device) -> Exp
     return ExpertGroups(row_token, pair_row, tile_expert, n_tiles, align, top, used)
 
 
-ROUTE_GROUP_TOKENS = 16  # csrc/routed.hip: ROUTE_GROUP_TOKENS
-ROUTE_GROUP_EXPERTS = 64
-ROUTE_GROUP_MAX_K = 8192  # csrc/routed.hip: 16 * 32 * ROUTE_GROUP_STEPS
-# Its one block reads the router 16 experts after the other, so it is ahead of the three launches for so many and a K of up to
+_ROUTE_GROUP_LIMITS: Optional[Tuple[int, int, int]] = None
+
+
+def route_group_limits() -> Tuple[int, int, int]:
+    """(tokens, experts, K) up to which `route_and_group` goes, asked of the library."""
+    global _ROUTE_GROUP_LIMITS
+    if _ROUTE_GROUP_LIMITS is None:
+        lib = _build.load("routed")
+        _ROUTE_GROUP_LIMITS = int(lib.cwm_route_group_tokens()), int(lib.cwm_route_group_experts()), int(lib.cwm_route_group_max_k())
+    return _ROUTE_GROUP_LIMITS
+
+
+# The one block of `route_and_group` reads the router 16 experts after the other, so it is ahead of the three launches for so many and a K of up to
 # 4,096 only.  One launch / three, us, weights not in a cache, at 1, 8 and 16 tokens: 16 experts, K = 1,024 7.8 / 9.5, 8.5 / 10.3, 9.1 / 10.1;
 # 2,048 8.7 / 10.9, 9.5 / 11.7, 10.7 / 12.6; 4,096 10.3 / 13.2, 11.8 / 14.9, 13.7 / 16.0; 8,192 13.1 / 14.6, 16.5 / 16.2, 20.7 / 17.8; 8 experts, 4,096 9.6 /
 # 11.5, 10.9 / 12.9, 13.4 / 14.4; 32 experts, 1,024 10.3 / 10.5, 11.5 / 11.3, 14.1 / 11.3; 2,048 11.3 / 11.6, 13.6 / 12.1, 15.5 / 13.4; 4,096 14.8 /
@@ -142,11 +151,12 @@ def route_and_group(
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
     _need_gpu(x, router_copy, bias, correction)
     _check_scores(scores, correction, scale, renormalize, n_experts)
-    if x.dim() != 2 or x.dtype != torch.bfloat16 or x.stride(1) != 1 or x.shape[0] > ROUTE_GROUP_TOKENS:
-        raise KernelError(f"x must be bfloat16 [T <= {ROUTE_GROUP_TOKENS}, K] with contiguous rows")
+    most_tokens, most_experts, most_k = route_group_limits()
+    if x.dim() != 2 or x.dtype != torch.bfloat16 or x.stride(1) != 1 or x.shape[0] > most_tokens:
+        raise KernelError(f"x must be bfloat16 [T <= {most_tokens}, K] with contiguous rows")
     n, k = x.shape
-    if not 1 <= n_experts <= ROUTE_GROUP_EXPERTS or k % 32 != 0 or k > ROUTE_GROUP_MAX_K:
-        raise KernelError(f"{n_experts} experts of rows of {k}: the kernel takes up to {ROUTE_GROUP_EXPERTS}, rows of a multiple of 32 up to {ROUTE_GROUP_MAX_K}")
+    if not 1 <= n_experts <= most_experts or k % 32 != 0 or k > most_k:
+        raise KernelError(f"{n_experts} experts of rows of {k}: the kernel takes up to {most_experts}, rows of a multiple of 32 up to {most_k}")
     if router_copy.dtype != torch.bfloat16 or tuple(router_copy.shape) != (-(-n_experts // 16), k // 32, 64, 8) or not router_copy.is_contiguous():
         raise KernelError(f"the router's streaming copy {tuple(router_copy.shape)} does not fit {n_experts} experts of rows of {k}")
     if bias is not None and (bias.dtype != torch.float32 or bias.shape != (n_experts,) or not bias.is_contiguous()):

@@ -89,6 +89,7 @@ class RoutedExperts(FeedForward):
             and ops.route_group_pays(self.n_experts, self.dim)
         ):
             self.router_copy = ops.stream_layout(self.router)
+            self.few_tokens = ops.route_group_limits()[0]
         self.choice_correction = tensors["correction"].float().contiguous() if self.correction else None
         # [experts, out, in], or, where the matrix cores read them as they lie in memory, in operand tiles (a layout; the same size)
         tiles = (
@@ -110,7 +111,7 @@ class RoutedExperts(FeedForward):
         """The same without the last kernel: every pair's row and the weights, for a consumer that adds a token's
         rows up itself (a norm that takes a `RoutedSum` as the pending result)."""
         router = (self.top, self.scores, self.choice_correction, self.weight_scale, self.renormalize, self.groups)
-        if self.router_copy is not None and x.shape[0] <= ops.ROUTE_GROUP_TOKENS and x.data_ptr() % 16 == 0:
+        if self.router_copy is not None and x.shape[0] <= self.few_tokens and x.data_ptr() % 16 == 0:
             _, weights, groups = ops.route_and_group(x, self.router_copy, self.router_b, self.n_experts, *router)
         else:
             chosen, weights = ops.route_top(ops.linear(x, self.router, self.router_b, torch.float32), *router)
