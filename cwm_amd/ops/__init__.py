@@ -21,6 +21,7 @@ import numpy as np
 import torch
 
 from . import build as _build
+from . import attention_plan as _work_lists
 from .attention_plan import WIDE_TILES
 from .build import KernelBuildError
 
@@ -388,7 +389,8 @@ def gemm_bf16_stream(
     caches, instead of `weight`.  Returns [M, N]; with `partials_ok` it may
     return float32 partial sums [P, M, N] of a split K for the caller to add (the
     residual-add + RMSNorm kernel takes them); with `keep_sums` it then does so (P = 1) for a K that is not
-    split too, instead of a result of a shorter type, so that nothing is rounded between the product and what follows.  `rope`
+    split too, instead of a result of a shorter type, so that nothing is rounded between the product and what follows
+    (for products that the tiled kernel, which leaves such sums, takes as well).  `rope`
     (positions, seq_of_token, inv_freq, cache, block_table, n_q_heads, n_kv_heads,
     head_dim) makes the epilogue rotate the q and k columns and write k and v into the
     paged cache (see `qkv_rope_write`).  `glu`: the weight's rows are gate and up rows in
@@ -442,7 +444,7 @@ def gemm_bf16_stream(
             tiles_a_block += 1
         blocks = k_split * ((inputs - 1) * a_input + rest)
         input_args = (ctypes.c_long(input_stride), ctypes.c_int(per), ctypes.c_int(a_input))
-    if k_split == 1 and partials_ok and keep_sums and out_dtype != torch.float32:
+    if k_split == 1 and partials_ok and keep_sums and out_dtype != torch.float32 and _tile_wins(x, weight):
         out = torch.empty((1, m, n), dtype=torch.float32, device=x.device)  # the consumer adds float32 sums, here one
     elif k_split == 1:
         out = torch.empty((m, n // 2 if glu else n), dtype=out_dtype, device=x.device)
@@ -748,11 +750,12 @@ def _prefers_tile(
     m = x.shape[0]
     if m <= STREAM_FUSED_ROWS and (streamed is not None or weight.numel() < TILE_FEW_ROWS_ENTRIES):
         return False
-    n, k = weight.shape
-    if STREAM_FUSED_ROWS < m <= STREAM_EPILOGUE_ROWS and n * k >= STREAM_LEAST_ENTRIES and not _wide_and_short(m, n, k):
-        with_copy = STREAM_WHOLE_ENTRIES if k <= stream_unsplit_k(m, fused) else STREAM_SPLIT_ENTRIES
-        if n * k < (STREAM_ANY_ENTRIES if streamed is None else with_copy):
-            return False
+    if STREAM_FUSED_ROWS < m <= STREAM_EPILOGUE_ROWS:
+        n, k = weight.shape
+        if n * k >= STREAM_LEAST_ENTRIES and not _wide_and_short(m, n, k):
+            with_copy = STREAM_WHOLE_ENTRIES if k <= stream_unsplit_k(m, fused) else STREAM_SPLIT_ENTRIES
+            if n * k < (STREAM_ANY_ENTRIES if streamed is None else with_copy):
+                return False
     return _tile_wins(x, weight)
 
 
@@ -810,9 +813,7 @@ def gemm_bf16(
     if _prefers_tile(x, weight, bias, streamed):
         return gemm_bf16_tile(x, weight, None, out_dtype, partials_ok)
     if m <= STREAM_MAX_ROWS:
-        # where the tiled kernel would leave partial sums, the sums of an unsplit K are not rounded either
-        keep_sums = partials_ok and bias is None and m > STREAM_FUSED_ROWS and _tile_wins(x, weight)
-        return gemm_bf16_stream(x, weight, bias, out_dtype, partials_ok, streamed=streamed, keep_sums=keep_sums)
+        return gemm_bf16_stream(x, weight, bias, out_dtype, partials_ok, streamed=streamed, keep_sums=bias is None and m > STREAM_FUSED_ROWS)
     if out_dtype == torch.float32:
         y = torch.mm(x, weight.t(), out_dtype=torch.float32)  # bfloat16 operands, float32 sums written as they are
         return y if bias is None else y + bias.float()
@@ -1118,9 +1119,7 @@ def _half_blocks_built(n_kv: int, head_dim: int, page_size: int, keep_first: int
     values the loads write to LDS themselves.  Not with kept first keys: a block takes those before its rows' windows ahead
     of them, so a tile that holds both is one pass or two by where the block's first row stands, and a row's bits would
     depend on the block's height, that is on what else is in the step."""
-    from .attention_plan import WIDE_HALF_BLOCKS
-
-    return head_dim in WIDE_HALF_BLOCKS and page_size % 32 == 0 and n_kv * page_size * head_dim * 2 < 2 ** 31 and keep_first == 0
+    return head_dim in _work_lists.WIDE_HALF_BLOCKS and page_size % 32 == 0 and n_kv * page_size * head_dim * 2 < 2 ** 31 and keep_first == 0
 
 
 def mfma_attention_takes(dtype: torch.dtype, head_dim: int, page_size: int) -> bool:
