@@ -19,8 +19,8 @@
 // Entries exactly equal to the threshold are all kept.  Without a nucleus (top_p = 1)
 // nothing is stored: the draw recomputes e_i where it walks.  A row of 128k logits done so
 // takes about 22 us greedy, 44 us at a temperature and 170 us with a nucleus; rows of more than
-// 8,192 entries are cut into segments instead (below): 6, 11 and 21 us, 34 us with a nucleus of
-// thousands of entries, replayed from a graph; 300 such rows 41, 54, 87 and 109 us.
+// 8,192 entries are cut into segments instead (below): 6, 11 and, by the logits' spread, 21 to 62 us replayed
+// from a graph (launched one by one 15, 16 and 21 to 62); 743 such rows 97, 129 and 205 to 396 us.
 #include "common.h"
 #include "no_alloc.h"
 
