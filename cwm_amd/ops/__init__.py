@@ -5,8 +5,8 @@ torch's current HIP stream through the C entry points of `cwm_amd/csrc`.  There 
 no CPU path and no library substitute: tensors that are not on a HIP device, or a
 missing kernel library, raise an error.
 
-The only library routine on the model's path is the bfloat16 matrix product for
-more rows than the hand-written kernels take (`torch.mm`, i.e. hipBLASLt), where
+The only library routine on the model's path is the bfloat16 matrix product of many
+rows where its tiles fill the chip (`torch.mm`, i.e. hipBLASLt), where
 the reference also calls a library
 (cwm/fastgen/forward.py:593-606).
 """
@@ -198,6 +198,8 @@ def gate_up_silu(
         return gemm_bf16_stream(x, weight, bias, torch.bfloat16, glu=True, streamed=streamed)
     if tiled and grouped and x.shape[0] <= TILE_ROWS:
         return gemm_bf16_tile(x, weight, None, torch.bfloat16, glu=True)
+    if grouped and not tiled and bias is None and x.is_cuda and x.dim() == 2 and x.shape[0] > STREAM_MAX_ROWS and _prefers_wide(x, weight, glu=True):
+        return gemm_bf16_wide(x, weight, glu=True)
     return silu_mul(linear(x, weight, bias, partials_ok=True, streamed=streamed), out_dtype=x.dtype, grouped=grouped)
 
 
@@ -776,6 +778,55 @@ def _tile_wins(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return 2 * -(-weight.shape[0] // TILE_COLUMNS) <= _compute_units(x.device)
 
 
+def _wide_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    k, n = x.shape[1], weight.shape[0]
+    return (
+        x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+        and k % 64 == 0 and n % 16 == 0 and x.shape[0] > 0
+        and x.stride(-1) == 1 and weight.stride(-1) == 1
+        and (x.shape[0] <= 1 or x.stride(0) % 8 == 0) and (n <= 1 or weight.stride(0) % 8 == 0)
+        and max(x.stride(0), weight.stride(0)) < (1 << 22)
+        and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+    )
+
+
+def _prefers_wide(x: torch.Tensor, weight: torch.Tensor, glu: bool = False) -> bool:
+    """Whether a product of more rows than the tiled kernel takes goes to the wide kernel instead of the library: where it is
+    expected to be faster, by the costs of both kernels' tiles (csrc/gemm_bf16_wide.hip)."""
+    if not _wide_takes(x, weight):
+        return False
+    return bool(_build.load("gemm_bf16_wide").cwm_gemm_bf16_wide_pays(x.shape[0], weight.shape[0], x.shape[1], _compute_units(x.device), int(glu)))
+
+
+def gemm_bf16_wide(
+    x: torch.Tensor, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None, glu: bool = False, units: Optional[int] = None,
+    tile: Optional[int] = None,
+) -> torch.Tensor:
+    """bfloat16 x [M, K] @ weight[N, K]^T with float32 sums, [M, N] in bfloat16 or float32: persistent blocks whose tiles of
+    64 to 256 rows and 128 or 256 columns reach LDS by direct loads.  `glu`: the weight's rows are gate and up rows in
+    alternating groups of 8 and the result is silu(gate) * up, [M, N / 2] in bfloat16.  `units` (tests) stands in for the
+    number of compute units, `tile` (tests) names one of the kernel's tiles."""
+    _need_gpu(x, weight)
+    if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] or not _wide_takes(x, weight):
+        raise KernelError(
+            "the wide product takes bfloat16 x [M, K] and weight [N, K] with K a multiple of 64, N of 16 and 16-byte aligned "
+            f"rows; got {tuple(x.shape)} {x.dtype} and {tuple(weight.shape)} {weight.dtype}"
+        )
+    m, k = x.shape
+    n = weight.shape[0]
+    out = torch.empty((m, n // 2 if glu else n), dtype=torch.bfloat16 if glu else out_dtype or torch.bfloat16, device=x.device)
+    lib = _build.load("gemm_bf16_wide")
+    _check(
+        lib,
+        lib.cwm_gemm_bf16_wide(
+            _ptr(x), ctypes.c_long(x.stride(0) if m > 1 else k), _ptr(weight), ctypes.c_long(weight.stride(0)), _ptr(out),
+            ctypes.c_int(_code(out.dtype)), ctypes.c_long(out.shape[1]), ctypes.c_int(m), ctypes.c_int(n), ctypes.c_int(k),
+            ctypes.c_int(units or _compute_units(x.device)), ctypes.c_int(int(glu)), ctypes.c_int(-1 if tile is None else tile), _stream(),
+        ),
+    )
+    return out
+
+
 def _stream_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
     k = x.shape[1]
     return (
@@ -801,7 +852,8 @@ def gemm_bf16(
     persistent weight-streaming kernel, x in registers.
     Up to 128 rows (256 for a result of at most 16,384 columns): the hand-written tiled kernel, x and W
     through LDS (it needs K % 64 == 0 and N % 16 == 0; other sizes of up to 64 rows stream).
-    More rows: the library product (hipBLASLt through torch), as the reference calls a
+    More rows: the hand-written wide kernel where it is ahead of the library, mostly where the library's tiles would leave much
+    of the chip idle (`_prefers_wide`; it needs the same sizes and no bias), else the library product (hipBLASLt through torch), as the reference calls a
     library here, with a bfloat16 or a float32 result.  Row lengths that are no multiple
     of 8 go to the float32 kernel, which takes any size.
     """
@@ -814,6 +866,8 @@ def gemm_bf16(
         return gemm_bf16_tile(x, weight, None, out_dtype, partials_ok)
     if m <= STREAM_MAX_ROWS:
         return gemm_bf16_stream(x, weight, bias, out_dtype, partials_ok, streamed=streamed, keep_sums=bias is None and m > STREAM_FUSED_ROWS)
+    if bias is None and _prefers_wide(x, weight):
+        return gemm_bf16_wide(x, weight, out_dtype)
     if out_dtype == torch.float32:
         y = torch.mm(x, weight.t(), out_dtype=torch.float32)  # bfloat16 operands, float32 sums written as they are
         return y if bias is None else y + bias.float()

@@ -54,6 +54,7 @@ SOURCES: Dict[str, Tuple[Mapping[str, int], ...]] = {
     "sampling": ({},),
     "gemm_bf16_stream": ({},),
     "gemm_bf16_tile": ({},),
+    "gemm_bf16_wide": ({},),
     "ceilings": ({},),
     "groupnorm": ({},),
     "state_space": ({},),
