@@ -1,6 +1,6 @@
 // C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in float32 on the matrix cores
 // (v_mfma_f32_32x32x2_f32: float32 operands, exact products, float32 sums; float32 operands with
-// K a multiple of 32 and up to 65,536 in exact bfloat16 parts instead, see below): the matrix
+// K a multiple of 32 and up to 65,536 in exact bfloat16 parts instead, with an entry of their own, see below): the matrix
 // product of the 32-bit path.  Operands may be stored as float32 or bfloat16 (converted
 // exactly on load).  Every output
 // element is the sum over k = 0, 1, ... in one fixed grouping (eight values at a time, as the
@@ -165,10 +165,8 @@ gemm_f32_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lo
 // rate of the float32 one: the three left out are below 2^-24 of the product together, and a sum takes 6 K / 32 roundings
 // instead of K / 2.  Against float64 (normal operands, K = 512, 4,096 and 14,336) a result is 3.3e-7, 9.7e-7 and 1.8e-6 off,
 // 4.0e-7, 1.15e-6 and 2.1e-6 with float32 operands; with positive operands 2.6e-7, 6.1e-7 and 1.1e-6 against 3.5e-7, 9.9e-7
-// and 1.8e-6.  Bound by the matrix cores and the vector instructions that make the parts (times that add).  743 rows, float32
-// operands and parts: 28,672 x 4,096 1,847 and 1,034 us (169 TFLOP/s of float32 products), 2,048 x 2,048 191 and 74 us; 64 rows
-// 6,144 x 4,096 361 and 136 us; 32 rows 168 and 91 us.
-// The parts are made on the way into LDS, so memory holds float32 as before.  Both operands are multiplied by 2^23 first, and
+// and 1.8e-6.  743 rows, float32 operands and parts: 28,672 x 4,096 1,847 and 828 us, 2,048 x 2,048 191 and 61 us.
+// Memory holds float32: W's parts are made in registers.  Both operands are multiplied by 2^23 first, and
 // the sums by 2^-46 at the end, which rounds nothing: the last bit of the smallest float32 is then a normal bfloat16, so that the parts
 // of small values are exact too (without it the third part is lost below 2^-110 and the second below 2^-118).  Rows of A and W with a
 // value of 2^32 or more, or an infinity, are left to float32 operands, element by element of the result: with smaller ones the sums of
@@ -178,185 +176,255 @@ gemm_f32_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lo
 // 2.9e-6 off float64 where float32 operands are 2.4e-6).  So the 8 steps in the middle of every 16 go into the sum with its sign turned,
 // where rounding down is up: logits 2.0e-6 off, at the same times.
 #define SPLIT_STEP 32
-#define SPLIT_LD (SPLIT_STEP + 8)      // a row of a part in LDS: 80 bytes, so that 16 rows' pieces lie in different banks
 #define SPLIT_MOST_K 65536
 #define SPLIT_SCALE 8388608.0f               // 2^23
 #define SPLIT_UNSCALE 1.4210854715202004e-14f  // 2^-46
 #define SPLIT_TURN 4                         // steps after which the sum's sign turns, and 8 later again, of every 16
 #define SPLIT_LIMIT 3.602879701896397e16f    // 2^55: 2^32 once scaled
 
-typedef __bf16 bf16_pair __attribute__((ext_vector_type(2)));
-// c plus the product of two pairs of bfloat16 values (v_dot2_f32_bf16); with (-1, 0) or (0, -1) for `by`: c less one of the pair
-__device__ __forceinline__ float plus_pairs(uint32_t pair, uint32_t by, float c) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16_pair, pair), __builtin_bit_cast(bf16_pair, by), c, false);
+//
+// What bounded a kernel whose blocks made both operands' parts on their way into LDS was the making: vector instructions, which add to the
+// matrix cores' time, two thirds as many cycles in a block of 128 x 128, and again in every block that read the row (28,672 x 4,096 986 us,
+// 128,256 x 4,096 4,290, 6,144 x 4,096 283, 4,096 x 14,336 693, 2,048 x 2,048 72).  So A's parts are made once, by a kernel that writes them as operands of the
+// matrix instruction, [tile of 16 rows][step of 32 k][part][64 lanes][8 values], signs turned with their steps; and a block takes up to 256
+// rows, so that few blocks take a row of W apart, and the one wavefront that multiplies it does: the wavefronts lie side by side along the
+// columns, 16 each, with all WM tiles of 16 rows.  Operands of A and raw rows of W reach LDS by direct loads, W two steps further ahead; a
+// wavefront takes the next step's W apart while it multiplies; one barrier a step.  Now 828, 3,440 (1.36 PFLOP/s of bfloat16 products, of
+// which the chip's power allows 1.5 to 1.7), 198, 495 and 61 us, and the same bits.
+#define PARTS_STEPS 8  // of K whose parts a wavefront of the first kernel makes
+
+struct PartRows {  // a row's marks: bit r of [row tile][group of PARTS_STEPS steps]
+  const uint32_t* flags;
+  int groups;
+};
+
+__global__ void __launch_bounds__(256) f32_parts_kernel(const float* __restrict__ A, long lda, int M, int steps, uint4* __restrict__ parts, uint32_t* __restrict__ flags,
+                                                        int groups) {
+  const int lane = threadIdx.x & 63, r = lane & 15, j = lane >> 4;
+  const int tile = blockIdx.x, group = blockIdx.y * 4 + (threadIdx.x >> 6);
+  if (group >= groups) return;
+  const int m = tile * 16 + r;
+  const float* src = A + (size_t)min(m, M - 1) * lda + 8 * j;
+  float largest = 0.f;
+  const int first = group * PARTS_STEPS, end = min(first + PARTS_STEPS, steps);
+  for (int s = first; s < end; ++s) {
+    const float4v x = *(const float4v*)(src + 32 * s), y = *(const float4v*)(src + 32 * s + 4);
+    float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+    const float scale = ((s + SPLIT_TURN) / (2 * SPLIT_TURN)) & 1 ? -SPLIT_SCALE : SPLIT_SCALE;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[e] = m < M ? v[e] * scale : 0.f;
+      largest = fmaxf(largest, fabsf(v[e]));
+    }
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+      uint32_t w[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        w[e] = pack2_bf16(v[2 * e], v[2 * e + 1]);
+        v[2 * e] -= __uint_as_float(w[e] << 16), v[2 * e + 1] -= __uint_as_float(w[e] & 0xffff0000u);
+      }
+      parts[(((size_t)tile * steps + s) * 3 + part) * 64 + lane] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  }
+  const unsigned long long over = __ballot(!(largest < SPLIT_LIMIT));
+  if (lane == 0) flags[(size_t)tile * groups + group] = (uint32_t)((over | over >> 16 | over >> 32 | over >> 48) & 0xffffu);
 }
 
-// WAVES_M x WAVES_N wavefronts, each with TM x TN tiles of 16 x 16.  PAIRS: a value less its part in one instruction instead of two.
-// It has the shorter chain and the lower rate, so it pays where blocks wait for themselves: with 64 x 128 blocks and 300 rows of 4,096 x
-// 14,336 (160 blocks) 487 us and 504, 743 rows of 2,048 x 2,048 (192) 76 and 87, but 743 rows of 6,144 x 4,096 (576) 306 and 295.
-template <typename TC, int WAVES_M, int WAVES_N, int TM, int TN, bool PAIRS>
-__global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, TM * TN <= 8 ? 3 : 2)
-gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, TC* __restrict__ C, long ldc,
-                      const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int row_blocks, int total) {
-  constexpr int BM = 16 * TM * WAVES_M, BN = 16 * TN * WAVES_N, THREADS = 64 * WAVES_M * WAVES_N;
-  constexpr int A_LOADS = BM * (SPLIT_STEP / 4) / THREADS, W_LOADS = BN * (SPLIT_STEP / 4) / THREADS;
-  constexpr int PARTS_BYTES = 3 * (BM + BN) * SPLIT_LD * 2, WHOLE_BYTES = (BM + BN) * (16 + 4) * 4;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[PARTS_BYTES > WHOLE_BYTES ? PARTS_BYTES : WHOLE_BYTES];
-  __shared__ unsigned char marked_rows[BM], marked_columns[BN];
-  bf16_t* a_parts = (bf16_t*)lds;                  // [3][BM][SPLIT_LD]
-  bf16_t* w_parts = a_parts + 3 * BM * SPLIT_LD;   // [3][BN][SPLIT_LD]
-  // an XCD gets a run of neighbours, the row blocks of a panel of W one after the other: its L2 reads the panel once
+template <typename TC, int WM, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, 2)
+gemm_f32_parts_kernel(const unsigned char* __restrict__ parts, PartRows marks, const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw,
+                      TC* __restrict__ C, long ldc, const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int row_blocks, int total) {
+  constexpr int BM = 16 * WM, BN = 16 * WAVES;
+  constexpr int A_STAGE = WM * 3 * 1024, W_STAGE = BN * 128;
+  // steps of A under way or in use, and of W
+  constexpr int SA = 4 * A_STAGE + 6 * W_STAGE <= 160 * 1024 ? 4 : 3 * A_STAGE + 5 * W_STAGE <= 160 * 1024 ? 3 : 2, SW = SA + 2;
+  constexpr int NA = (WM * 3 + WAVES - 1) / WAVES, NW = W_STAGE / 1024 / WAVES;  // a wavefront's loads a step
+  static_assert(SA * A_STAGE + SW * W_STAGE <= 160 * 1024, "the steps fit the LDS");
+  static_assert(WM % 2 == 0, "row tiles go in pairs");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[SA * A_STAGE + SW * W_STAGE];
   const int run = (total + 7) >> 3, at = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= run || at >= total) return;
   const int m0 = at % row_blocks * BM, n0 = at / row_blocks * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, j = lane >> 4;
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  // piece f of a step: row f / 8, values 4 (f % 8) .. + 3; rows past the last are read from the last, their results not written
-  const float* src_a[A_LOADS];
-  const float* src_w[W_LOADS];
+  const int lane = threadIdx.x & 63, r = lane & 15, j = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int steps = K / SPLIT_STEP, last = steps - 1, row_tiles = (M + 15) / 16;
+  const uint32_t lds_a = (uint32_t)(uintptr_t)(&lds[0]), lds_w = lds_a + SA * A_STAGE;
+
+  // this wavefront's loads: 1 KB pieces of A's operands (tiles past the last are the last again), eight rows of W each
+  const unsigned char* a_src[NA];
+  uint32_t a_dst[NA], w_off[NW];
 #pragma unroll
-  for (int i = 0; i < A_LOADS; ++i) src_a[i] = A + (size_t)min(m0 + (tid + i * THREADS) / 8, M - 1) * lda + 4 * (tid & 7);
+  for (int i = 0; i < NA; ++i) {
+    const int p = min(wave + WAVES * i, WM * 3 - 1), tile = min(m0 / 16 + p / 3, row_tiles - 1);
+    a_src[i] = parts + ((size_t)tile * steps * 3 + p % 3) * 1024;
+    a_dst[i] = p * 1024;
+  }
 #pragma unroll
-  for (int i = 0; i < W_LOADS; ++i) src_w[i] = W + (size_t)min(n0 + (tid + i * THREADS) / 8, N - 1) * ldw + 4 * (tid & 7);
-  // two steps of operands on their way: what is fetched while step k is multiplied goes into LDS before step k + 2
-  float4v ra[2][A_LOADS], rw[2][W_LOADS];
-  auto fetch = [&](int set, int k) {
-    const int k0 = min(k, K - SPLIT_STEP);
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) ra[set][i] = *(const float4v*)(src_a[i] + k0);
-#pragma unroll
-    for (int i = 0; i < W_LOADS; ++i) rw[set][i] = *(const float4v*)(src_w[i] + k0);
+  for (int i = 0; i < NW; ++i) {
+    const int row = 8 * (NW * wave + i) + (lane >> 3);
+    w_off[i] = (uint32_t)((size_t)min(row, N - 1 - n0) * ldw * 4) + 16 * ((lane & 7) ^ ((row >> 1) & 7));
+  }
+  const float* w_src = W + (size_t)n0 * ldw;
+  auto load_a = [&](int i, int step, int buf) { dma16((const bf16_t*)(a_src[i] + (size_t)step * 3072), lane * 16, lds_a + buf * A_STAGE + a_dst[i]); };
+  auto load_w = [&](int i, int step, int buf) { dma16((const bf16_t*)(w_src + (size_t)step * 32), w_off[i], lds_w + buf * W_STAGE + (NW * wave + i) * 1024); };
+
+  float largest = 0.f;
+  // the wavefront's 16 rows of W of a step, taken apart
+  const int w_row = (wave * 16 + r) * 128, w_key = (r >> 1) & 7;
+  auto raw = [&](int buf, float4v& x, float4v& y) {
+    const unsigned char* row = lds + SA * A_STAGE + buf * W_STAGE + w_row;
+    x = *(const float4v*)(row + ((2 * j) ^ w_key) * 16);
+    y = *(const float4v*)(row + ((2 * j + 1) ^ w_key) * 16);
   };
-  // (-1, 0) and (0, -1), in registers: as an inline constant the instruction reads -1.0 as something else
-  uint32_t less_first = 0x0000bf80u, less_second = 0xbf800000u;
-  asm("" : "+v"(less_first), "+v"(less_second));
-  float largest_a[A_LOADS] = {}, largest_w[W_LOADS] = {};  // of a thread's pieces, which are the same rows' in every step
-  float sign = 1.f;  // of the sums, and so of A's parts
-  auto stage = [&](float4v v, float scale, bf16_t* parts, int plane, int f, float& largest) {
-    v *= scale;
-    if constexpr (TM * TN > 8)  // two instructions, or three in a shorter chain
-      largest = fmaxf(fmaxf(fmaxf(fmaxf(largest, fabsf(v[0])), fabsf(v[1])), fabsf(v[2])), fabsf(v[3]));
-    else
-      largest = fmaxf(largest, fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
-    bf16_t* to = parts + (f / 8) * SPLIT_LD + 4 * (f % 8);
+  auto take_apart = [&](float4v x, float4v y, Frag8 (&fw)[3]) {
+    x *= SPLIT_SCALE, y *= SPLIT_SCALE;
+    largest = fmaxf(fmaxf(fmaxf(fmaxf(largest, fabsf(x[0])), fabsf(x[1])), fabsf(x[2])), fabsf(x[3]));
+    largest = fmaxf(fmaxf(fmaxf(fmaxf(largest, fabsf(y[0])), fabsf(y[1])), fabsf(y[2])), fabsf(y[3]));
 #pragma unroll
     for (int part = 0; part < 3; ++part) {
-      const uint32_t lo = pack2_bf16(v[0], v[1]), hi = pack2_bf16(v[2], v[3]);
-      *(uint2*)(to + part * plane) = make_uint2(lo, hi);
-      // what is left, exactly
-      if constexpr (PAIRS) {
-        v[0] = plus_pairs(lo, less_first, v[0]), v[1] = plus_pairs(lo, less_second, v[1]);
-        v[2] = plus_pairs(hi, less_first, v[2]), v[3] = plus_pairs(hi, less_second, v[3]);
-      } else {
-        v[0] -= __uint_as_float(lo << 16), v[1] -= __uint_as_float(lo & 0xffff0000u);
-        v[2] -= __uint_as_float(hi << 16), v[3] -= __uint_as_float(hi & 0xffff0000u);
+      const uint32_t w0 = pack2_bf16(x[0], x[1]), w1 = pack2_bf16(x[2], x[3]), w2 = pack2_bf16(y[0], y[1]), w3 = pack2_bf16(y[2], y[3]);
+      fw[part].u = make_uint4(w0, w1, w2, w3);
+      if (part < 2) {
+        x[0] -= __uint_as_float(w0 << 16), x[1] -= __uint_as_float(w0 & 0xffff0000u), x[2] -= __uint_as_float(w1 << 16), x[3] -= __uint_as_float(w1 & 0xffff0000u);
+        y[0] -= __uint_as_float(w2 << 16), y[1] -= __uint_as_float(w2 & 0xffff0000u), y[2] -= __uint_as_float(w3 << 16), y[3] -= __uint_as_float(w3 & 0xffff0000u);
       }
     }
   };
-  float4v acc[TM][TN];
+
+  float4v acc[WM];
 #pragma unroll
-  for (int a = 0; a < TM; ++a)
+  for (int a = 0; a < WM; ++a) acc[a] = (float4v){0.f, 0.f, 0.f, 0.f};
+  // the loads in the order in which the waits below count them: step s of A with step s + 2 of W
 #pragma unroll
-    for (int b = 0; b < TN; ++b) acc[a][b] = (float4v){0.f, 0.f, 0.f, 0.f};
-  auto step = [&](int set, int next) {
+  for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) stage(ra[set][i], sign * SPLIT_SCALE, a_parts, BM * SPLIT_LD, tid + i * THREADS, largest_a[i]);
+    for (int i = 0; i < NW; ++i) load_w(i, min(s, last), s);
 #pragma unroll
-    for (int i = 0; i < W_LOADS; ++i) stage(rw[set][i], SPLIT_SCALE, w_parts, BN * SPLIT_LD, tid + i * THREADS, largest_w[i]);
-    __syncthreads();
-    fetch(set, next);
-    Frag8 fa[3][TM];
+  for (int s = 0; s < SA - 1; ++s) {
 #pragma unroll
-    for (int part = 0; part < 3; ++part)
+    for (int i = 0; i < NA; ++i) load_a(i, min(s, last), s);
 #pragma unroll
-      for (int a = 0; a < TM; ++a) fa[part][a].u = *(const uint4*)(a_parts + (part * BM + (wm * TM + a) * 16 + r) * SPLIT_LD + 8 * j);
+    for (int i = 0; i < NW; ++i) load_w(i, min(s + 2, last), s + 2);
+  }
+  Frag8 fw[3], fn[3];
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(NW + (SA - 2) * (NA + NW)) : "memory");
+  {
+    float4v x, y;
+    raw(0, x, y);
+    take_apart(x, y, fw);
+  }
+  float sign = 1.f;
+  int a_buf = 0, w_buf = 0;  // of the step that is multiplied
+  for (int k = 0; k < steps; ++k) {
+    // this wavefront's loads of this step of A and the next of W have landed and it has left the step before; after the barrier
+    // so has everyone
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(NW + (SA - 2) * (NA + NW)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    const int a_free = a_buf == 0 ? SA - 1 : a_buf - 1, w_free = w_buf == 0 ? SW - 1 : w_buf - 1, w_next = w_buf + 1 == SW ? 0 : w_buf + 1;
+    if (k % (2 * SPLIT_TURN) == SPLIT_TURN) {
+      sign = -sign;
 #pragma unroll
-    for (int b = 0; b < TN; ++b) {
-      Frag8 fw[3];
+      for (int a = 0; a < WM; ++a) acc[a] = -acc[a];
+    }
+    const unsigned char* st = lds + a_buf * A_STAGE + lane * 16;
+    float4v x, y;
+    raw(w_next, x, y);
+    Frag8 fa[2][2][3];
 #pragma unroll
-      for (int part = 0; part < 3; ++part) fw[part].u = *(const uint4*)(w_parts + (part * BN + (wn * TN + b) * 16 + r) * SPLIT_LD + 8 * j);
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int part = 0; part < 3; ++part) fa[0][u][part].u = *(const uint4*)(st + (u * 3 + part) * 1024);
+#pragma unroll
+    for (int p = 0; p < WM / 2; ++p) {
+      if (p + 1 < WM / 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int part = 0; part < 3; ++part) fa[(p + 1) & 1][u][part].u = *(const uint4*)(st + ((2 * (p + 1) + u) * 3 + part) * 1024);
+      }
+      __builtin_amdgcn_sched_barrier(0);
       constexpr int PART_A[6] = {2, 0, 1, 1, 0, 0}, PART_W[6] = {0, 2, 1, 0, 1, 0};  // the smaller products first
 #pragma unroll
       for (int q = 0; q < 6; ++q)
 #pragma unroll
-        for (int a = 0; a < TM; ++a) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[PART_W[q]].v, fa[PART_A[q]][a].v, acc[a][b], 0, 0, 0);
-    }
-    __syncthreads();
-  };
-  fetch(0, 0);
-  fetch(1, SPLIT_STEP);
-  int k0 = 0;
-  for (; k0 + 2 * SPLIT_STEP <= K; k0 += 2 * SPLIT_STEP) {
-    if (k0 / SPLIT_STEP % (2 * SPLIT_TURN) == SPLIT_TURN) {
-      sign = -sign;
+        for (int u = 0; u < 2; ++u)
+          acc[2 * p + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[PART_W[q]].v, fa[p & 1][u][PART_A[q]].v, acc[2 * p + u], 0, 0, 0);
+      if (p == 0) take_apart(x, y, fn);
+      // the loads of a step to come, a few after each pair
 #pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b) acc[a][b] = -acc[a][b];
-    }
-    step(0, k0 + 2 * SPLIT_STEP);
-    step(1, k0 + 3 * SPLIT_STEP);
-  }
-  if (k0 < K) step(0, K);
-  float largest = 0.f;
-#pragma unroll
-  for (int i = 0; i < A_LOADS; ++i) largest = fmaxf(largest, largest_a[i]);
-#pragma unroll
-  for (int i = 0; i < W_LOADS; ++i) largest = fmaxf(largest, largest_w[i]);
-  const bool any = __syncthreads_or(!(largest < SPLIT_LIMIT));
-  if (any) {
-    // eight neighbouring threads have a row's pieces
-    auto mark = [&](float largest, unsigned char* marks, int f) {
-#pragma unroll
-      for (int off = 1; off < 8; off <<= 1) largest = fmaxf(largest, __shfl_xor(largest, off, CWM_WAVE));
-      if ((f & 7) == 0) marks[f / 8] = !(largest < SPLIT_LIMIT);
-    };
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) mark(largest_a[i], marked_rows, tid + i * THREADS);
-#pragma unroll
-    for (int i = 0; i < W_LOADS; ++i) mark(largest_w[i], marked_columns, tid + i * THREADS);
-    __syncthreads();
-  }
-  // lane 16 j + r of a tile holds row r, columns 4 j + i
-#pragma unroll
-  for (int b = 0; b < TN; ++b)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int n = n0 + (wn * TN + b) * 16 + 4 * j + i;
-      if (n >= N) continue;
-      float add = 0.f;
-      if (bias) add = bias_dtype == CWM_BF16 ? bf16_to_f32(((const bf16_t*)bias)[n]) : ((const float*)bias)[n];
-#pragma unroll
-      for (int a = 0; a < TM; ++a) {
-        const int m = m0 + (wm * TM + a) * 16 + r;
-        if (any && (marked_rows[m - m0] | marked_columns[n - n0])) continue;
-        if (m < M) Elem<TC>::store(C + (size_t)m * ldc + n, acc[a][b][i] * (sign * SPLIT_UNSCALE) + add);
+      for (int i = 0; i < NA + NW; ++i) {
+        if (i * (WM / 2) / (NA + NW) != p) continue;
+        if (i < NA)
+          load_a(i, min(k + SA - 1, last), a_free);
+        else
+          load_w(i - NA, min(k + SW - 1, last), w_free);
       }
     }
-  if (any) {
-    constexpr int WHOLE_M = BM / 32, WHOLE_N = BN / 32;
-    gemm_f32_tile<float, float, TC, WAVES_M, WAVES_N, WHOLE_M / WAVES_M, WHOLE_N / WAVES_N, 16, true>(
-        A, lda, W, ldw, C, ldc, bias, bias_dtype, M, N, K, 1, 1, m0, n0, (float*)lds, (float*)lds + BM * 20, marked_rows, marked_columns);
+#pragma unroll
+    for (int part = 0; part < 3; ++part) fw[part] = fn[part];
+    a_buf = a_buf + 1 == SA ? 0 : a_buf + 1;
+    w_buf = w_next;
   }
-}
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // the loads past the last step; everyone has left the buffers
 
-template <typename TC>
-static void launch_split(const float* A, long lda, const float* W, long ldw, TC* C, long ldc, const void* bias, int bias_dtype, int M, int N, int K,
-                         hipStream_t stream) {
-#define CWM_SPLIT(WAVES_M, WAVES_N, TM, TN, PAIRS)                                                                                          \
-  do {                                                                                                                                     \
-    const int row_blocks = (M + 16 * TM * WAVES_M - 1) / (16 * TM * WAVES_M), total = row_blocks * ((N + 16 * TN * WAVES_N - 1) / (16 * TN * WAVES_N)); \
-    hipLaunchKernelGGL((gemm_f32_split_kernel<TC, WAVES_M, WAVES_N, TM, TN, PAIRS>), dim3((total + 7) / 8 * 8), dim3(64 * WAVES_M * WAVES_N), 0, stream, A,   \
-                       lda, W, ldw, C, ldc, bias, bias_dtype, M, N, K, row_blocks, total);                                                \
-  } while (0)
-  const long wide = (long)((M + 127) / 128) * ((N + 127) / 128);
-  if (M <= 32)
-    CWM_SPLIT(1, 2, 2, 2, true);
-  else if (M <= 64 || wide < 512)  // too few blocks of 128 x 128 for two a compute unit
-    if ((long)((M + 63) / 64) * ((N + 127) / 128) <= 256) CWM_SPLIT(2, 2, 2, 4, true); else CWM_SPLIT(2, 2, 2, 4, false);
-  else
-    CWM_SPLIT(2, 2, 4, 4, false);
-#undef CWM_SPLIT
+  // rows and columns with a value beyond the parts
+  constexpr int WHOLE = 64 * 20 + BN * 20;  // floats of the tile of whole operands
+  unsigned char* marked_rows = lds + WHOLE * 4;
+  unsigned char* marked_columns = marked_rows + (BM + 63) / 64 * 64;
+  uint32_t* any_of = (uint32_t*)(marked_columns + BN);
+  largest = fmaxf(largest, __shfl_xor(largest, 16, CWM_WAVE));
+  largest = fmaxf(largest, __shfl_xor(largest, 32, CWM_WAVE));
+  const bool column = !(largest < SPLIT_LIMIT);
+  if (j == 0) marked_columns[wave * 16 + r] = column;
+  uint32_t rows = 0;  // of the row tiles wave, wave + WAVES, ...
+#pragma unroll
+  for (int t = 0; t < (WM + WAVES - 1) / WAVES; ++t) {
+    const int tile = wave + WAVES * t;
+    uint32_t f = 0;
+    if (tile < WM && m0 / 16 + tile < row_tiles)
+      for (int g = lane; g < marks.groups; g += 64) f |= marks.flags[(size_t)(m0 / 16 + tile) * marks.groups + g];
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) f |= __shfl_xor(f, off, CWM_WAVE);
+    if (tile < WM && lane < 16) marked_rows[tile * 16 + lane] = (f >> lane) & 1;
+    rows |= f;
+  }
+  if (lane == 0) any_of[wave] = rows;
+  if (__any(column) && lane == 0) any_of[wave] = 1;
+  __syncthreads();
+  uint32_t any = 0;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) any |= any_of[w];
+
+  // lane 16 j + r of a tile holds row r, columns 4 j + i
+  const int n = n0 + wave * 16 + 4 * j;
+  float add[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    add[i] = 0.f;
+    if (bias && n + i < N) add[i] = bias_dtype == CWM_BF16 ? bf16_to_f32(((const bf16_t*)bias)[n + i]) : ((const float*)bias)[n + i];
+  }
+  const bool whole = sizeof(TC) == 4 && any == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0 && n + 3 < N;
+#pragma unroll
+  for (int a = 0; a < WM; ++a) {
+    const int m = m0 + a * 16 + r;
+    if (m >= M) continue;
+    const float4v v = acc[a] * (sign * SPLIT_UNSCALE);
+    if (whole) {
+      *(float4*)((float*)C + (size_t)m * ldc + n) = make_float4(v[0] + add[0], v[1] + add[1], v[2] + add[2], v[3] + add[3]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (n + i < N && !(any && (marked_rows[m - m0] | marked_columns[n + i - n0]))) Elem<TC>::store(C + (size_t)m * ldc + n + i, v[i] + add[i]);
+    }
+  }
+  if (any) {
+    for (int sub = 0; sub < BM && m0 + sub < M; sub += 64) {
+      gemm_f32_tile<float, float, TC, 2, WAVES / 2, 1, 1, 16, true>(A, lda, W, ldw, C, ldc, bias, bias_dtype, min(M, m0 + BM), N, K, 1, 1, m0 + sub, n0, (float*)lds,
+                                                            (float*)lds + 64 * 20, marked_rows + sub, marked_columns);
+      __syncthreads();
+    }
+  }
 }
 
 template <typename TA, typename TW, typename TC>
@@ -365,12 +433,6 @@ static void launch(const void* A, long lda, const void* W, long ldw, void* C, lo
   // 16-byte loads of four values where every row allows them
   const int vec_a = lda % 4 == 0 && ((uintptr_t)A % 16) == 0;
   const int vec_w = ldw % 4 == 0 && ((uintptr_t)W % 16) == 0;
-  if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4) {
-    if (vec_a && vec_w && K % SPLIT_STEP == 0 && K <= SPLIT_MOST_K) {  // whatever M is: a row's result does not depend on the others
-      launch_split<TC>((const float*)A, lda, (const float*)W, ldw, (TC*)C, ldc, bias, bias_dtype, M, N, K, stream);
-      return;
-    }
-  }
   if (M > 32) {
     dim3 grid((N + 127) / 128, (M + 127) / 128);
     hipLaunchKernelGGL((gemm_f32_kernel<TA, TW, TC, 2, 2, 2, 2, 16>), grid, dim3(256), 0, stream, (const TA*)A, lda, (const TW*)W,
@@ -404,4 +466,63 @@ extern "C" int cwm_gemm_f32(const void* A, int a_dtype, long lda, const void* W,
     default: return cwm_fail("gemm_f32: unknown dtypes a=%d w=%d c=%d", a_dtype, w_dtype, c_dtype);
   }
   return cwm_launch_status("gemm_f32");
+}
+
+// The blocks of the product in parts, (row tiles, wavefronts), and what a step of one costs, us, with most of the chip busy: 743 rows,
+// 128 steps.  Blocks of 64 columns and four wavefronts share a compute unit by two, and a step of both takes 0.64; taller ones of four
+// wavefronts or short ones of eight were nowhere ahead.  30 and 60 rows of 4,096 x 4,096: 32 rows and 64 columns 55 and 57 us, 64 x 128 101 and 102.
+struct PartsBlock {
+  int row_tiles, waves;
+  float step;
+};
+static const PartsBlock parts_blocks[] = {{16, 8, 2.05f}, {12, 8, 1.62f}, {10, 8, 1.44f}, {8, 8, 1.19f}, {6, 8, 1.03f}, {4, 8, 0.80f}, {2, 4, 0.44f}};
+#define PARTS_BLOCKS 7
+static int parts_block(int M, int N) {
+  int best = 0;
+  float least = 0.f;
+  for (int i = 0; i < PARTS_BLOCKS; ++i) {
+    const PartsBlock& b = parts_blocks[i];
+    const long blocks = (long)((M + 16 * b.row_tiles - 1) / (16 * b.row_tiles)) * ((N + 16 * b.waves - 1) / (16 * b.waves));
+    const float us = b.waves == 4 && blocks > 256 ? (float)((blocks + 511) / 512) * 0.64f : (float)((blocks + 255) / 256) * b.step;
+    if (i == 0 || us < least) best = i, least = us;
+  }
+  return best;
+}
+// float32 A and W, K a multiple of 32.  `scratch`: for every started 16 rows 3,072 bytes a step of 32 k and 4 every 256 k, 16-byte
+// aligned.  `block`: -1, or the number of one of the list above (tests).
+extern "C" int cwm_gemm_f32_parts(const void* A, long lda, const void* W, long ldw, void* C, int c_dtype, long ldc, const void* bias, int bias_dtype, int M, int N,
+                                  int K, void* scratch, int block, hipStream_t stream) {
+  CWM_REQUIRE(M > 0 && N > 0 && K > 0 && K % SPLIT_STEP == 0 && K <= SPLIT_MOST_K, "gemm_f32_parts: bad sizes M=%d N=%d K=%d", M, N, K);
+  CWM_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_f32_parts: row strides shorter than rows");
+  CWM_REQUIRE(lda % 4 == 0 && ldw % 4 == 0 && ldw < (1L << 23) && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)scratch % 16) == 0,
+              "gemm_f32_parts: rows must be 16-byte aligned");
+  CWM_REQUIRE(c_dtype == CWM_F32 || c_dtype == CWM_BF16, "gemm_f32_parts: unknown output dtype %d", c_dtype);
+  const int row_tiles = (M + 15) / 16, steps = K / SPLIT_STEP, groups = (steps + PARTS_STEPS - 1) / PARTS_STEPS;
+  unsigned char* parts = (unsigned char*)scratch;
+  uint32_t* flags = (uint32_t*)(parts + (size_t)row_tiles * steps * 3072);
+  hipLaunchKernelGGL(f32_parts_kernel, dim3((unsigned)row_tiles, (unsigned)((groups + 3) / 4)), dim3(256), 0, stream, (const float*)A, lda, M, steps, (uint4*)parts, flags, groups);
+  const PartRows marks = {flags, groups};
+  if (block < 0) block = parts_block(M, N);
+#define CWM_PARTS(AT, WM, WAVES)                                                                                                          \
+  case AT: {                                                                                                                             \
+    const int row_blocks = (M + 16 * WM - 1) / (16 * WM), total = row_blocks * ((N + 16 * WAVES - 1) / (16 * WAVES));                     \
+    if (c_dtype == CWM_F32)                                                                                                              \
+      hipLaunchKernelGGL((gemm_f32_parts_kernel<float, WM, WAVES>), dim3((total + 7) / 8 * 8), dim3(64 * WAVES), 0, stream, parts, marks,  \
+                         (const float*)A, lda, (const float*)W, ldw, (float*)C, ldc, bias, bias_dtype, M, N, K, row_blocks, total);        \
+    else                                                                                                                                 \
+      hipLaunchKernelGGL((gemm_f32_parts_kernel<bf16_t, WM, WAVES>), dim3((total + 7) / 8 * 8), dim3(64 * WAVES), 0, stream, parts, marks, \
+                         (const float*)A, lda, (const float*)W, ldw, (bf16_t*)C, ldc, bias, bias_dtype, M, N, K, row_blocks, total);       \
+  } break;
+  switch (block) {
+    CWM_PARTS(0, 16, 8)
+    CWM_PARTS(1, 12, 8)
+    CWM_PARTS(2, 10, 8)
+    CWM_PARTS(3, 8, 8)
+    CWM_PARTS(4, 6, 8)
+    CWM_PARTS(5, 4, 8)
+    CWM_PARTS(6, 2, 4)
+    default: return cwm_fail("gemm_f32_parts: no block %d", block);
+  }
+#undef CWM_PARTS
+  return cwm_launch_status("gemm_f32_parts");
 }

@@ -215,6 +215,8 @@ def gemm_f32(
     _need_gpu(x, weight, bias)
     if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
         raise KernelError(f"gemm: x {tuple(x.shape)} and weight {tuple(weight.shape)} do not fit")
+    if _f32_parts_takes(x, weight):  # whatever the number of rows: a row's result does not depend on the others
+        return gemm_f32_parts(x, weight, bias, out_dtype)
     _rows_contiguous(x, "gemm x")
     _rows_contiguous(weight, "gemm weight")
     m, k = x.shape
@@ -235,6 +237,45 @@ def gemm_f32(
         ),
     )
     return out
+
+
+def gemm_f32_parts(
+    x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None, block: Optional[int] = None,
+) -> torch.Tensor:
+    """The product of `gemm_f32` where both operands are float32, K is a multiple of 32 up to 65,536 and rows are 16-byte aligned:
+    every value in three exact bfloat16 parts, six of their nine products on the matrix cores.  x's parts are made by a kernel of
+    their own, into scratch memory of 6 bytes a value.  `block` (tests): the number of a block of the kernel's list."""
+    _need_gpu(x, weight, bias)
+    if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] or not _f32_parts_takes(x, weight):
+        raise KernelError(
+            "the float32 product in parts takes float32 x [M, K] and weight [N, K] with K a multiple of 32 and 16-byte aligned rows; "
+            f"got {tuple(x.shape)} {x.dtype} and {tuple(weight.shape)} {weight.dtype}"
+        )
+    m, k = x.shape
+    n = weight.shape[0]
+    if bias is not None and (bias.shape != (n,) or not bias.is_contiguous()):
+        raise KernelError(f"gemm: bias {tuple(bias.shape)} does not fit {n} outputs")
+    lib = _build.load("gemm_f32")
+    out = torch.empty((m, n), dtype=out_dtype or x.dtype, device=x.device)
+    scratch = torch.empty(-(-m // 16) * (k // 32 * 3072 + -(-k // 256) * 4), dtype=torch.uint8, device=x.device)
+    _check(
+        lib,
+        lib.cwm_gemm_f32_parts(
+            _ptr(x), ctypes.c_long(x.stride(0) if m > 1 else k), _ptr(weight), ctypes.c_long(weight.stride(0) if n > 1 else k), _ptr(out),
+            ctypes.c_int(_code(out.dtype)), ctypes.c_long(n), _ptr(bias), ctypes.c_int(_code(bias.dtype) if bias is not None else F32),
+            ctypes.c_int(m), ctypes.c_int(n), ctypes.c_int(k), _ptr(scratch), ctypes.c_int(-1 if block is None else block), _stream(),
+        ),
+    )
+    return out
+
+
+def _f32_parts_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    return (
+        x.dtype == torch.float32 and weight.dtype == torch.float32
+        and x.shape[0] > 0 and x.shape[1] % 32 == 0 and 0 < x.shape[1] <= 65536 and x.stride(-1) == 1 and weight.stride(-1) == 1
+        and (x.shape[0] <= 1 or x.stride(0) % 4 == 0) and (weight.shape[0] <= 1 or weight.stride(0) % 4 == 0)
+        and weight.stride(0) < (1 << 23) and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+    )
 
 
 F32_STREAM_MAX_ROWS = 16
