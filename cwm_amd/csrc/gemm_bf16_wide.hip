@@ -39,6 +39,8 @@ struct PlainSource {
   WideOrder order;
   const bf16_t *a, *w;
   uint32_t off[WideShape<WM, WN>::ND];
+  static constexpr bool W_TILES = false;
+  __device__ __forceinline__ const bf16_t* base(int p) const { return p < WideShape<WM, WN>::BM / 8 ? a : w; }
   __device__ __forceinline__ void enter(int tile) {
     constexpr int BM = WideShape<WM, WN>::BM, BN = WideShape<WM, WN>::BN;
     int tm, tn;

@@ -22,6 +22,9 @@
 //
 // In LDS the 16-byte piece p of a row lies at p ^ key(row); the keys spread the 16 rows of one operand read over all
 // banks: rows of A follow one another, (row / 2) % 8; rows of W come in fours 4 WN apart.
+//
+// A SOURCE with W_TILES has W in operand tiles, [16 rows][32 k][64 lanes][8 values]: 1 KB is an operand, in memory as in LDS, row r of
+// tile b is the column 16 b + r, and a lane's sums are 4 consecutive columns of each tile.
 #pragma once
 
 #include "common.h"
@@ -44,8 +47,8 @@ __device__ __forceinline__ int wide_w_key(int row) {  // of a row of W within th
   return ((row >> 1) & 1) | (((row / (4 * WN)) & 3) << 1);
 }
 
-// SOURCE: enter(tile) sets `a` and `w`, the first rows of the tile's operands, and `off[ND]`, this lane's byte offsets of its
-// loads from them (uniform pointers: loads p < BM / 8 read A's rows 8 p .., the others W's).  SINK: store(tile, acc) writes
+// SOURCE: enter(tile) sets what base(p) answers, where piece p of a step lies (a uniform pointer; pieces p < BM / 8 are A's rows
+// 8 p .., the others eight rows of W, or an operand of half a step), and `off[ND]`, this lane's byte offsets of its loads from there.  SINK: store(tile, acc) writes
 // the sums, with exactly STORES store instructions if it answers true.
 template <int WM, int WN, int STORES, typename SOURCE, typename SINK>
 __device__ __forceinline__ void wide_loop(unsigned char* lds, SOURCE& src, SINK& sink, int tile, int tile_stride, int n_tiles, int steps) {
@@ -61,11 +64,11 @@ __device__ __forceinline__ void wide_loop(unsigned char* lds, SOURCE& src, SINK&
   const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
   int i_tile = tile, i_step = 0, i_left = n_tiles * steps;
   src.enter(i_tile);
-  auto issue_one = [&](int i, uint32_t stage) {
+  auto issue_one = [&](int i, uint32_t stage) __attribute__((always_inline)) {
     const int p = min(wave + 8 * i, PIECES - 1);
-    dma16((p < BM / 8 ? src.a : src.w) + (size_t)i_step * WIDE_BK, src.off[i], lds0 + stage + p * 1024);
+    dma16(src.base(p) + (size_t)i_step * (SOURCE::W_TILES && p >= BM / 8 ? 1024 : WIDE_BK), src.off[i], lds0 + stage + p * 1024);
   };
-  auto advance = [&]() {  // past the last step: that step again, into a buffer nobody reads
+  auto advance = [&]() __attribute__((always_inline)) {  // past the last step: that step again, into a buffer nobody reads
     if (i_left > 1) {
       --i_left;
       if (++i_step == steps) {
@@ -79,16 +82,16 @@ __device__ __forceinline__ void wide_loop(unsigned char* lds, SOURCE& src, SINK&
   const int a_key = (r >> 1) & 7;
   const int w_row = 4 * WN * (r >> 2) + (r & 3);  // of tile b: + 4 b, the key's row bits of which follow from b alone
   const unsigned char* const a_base = lds + (wm * WM * 16 + r) * 128;
-  const unsigned char* const w_base = lds + BM * 128 + (wn * WN * 16 + w_row) * 128;
-  int w_piece[WN];  // of the first half; the second half's is ^ 64 bytes
+  const unsigned char* const w_base = lds + BM * 128 + (SOURCE::W_TILES ? wn * WN * 2048 + lane * 16 : (wn * WN * 16 + w_row) * 128);
+  int w_piece[WN];  // of the first half; the second half's is ^ 64 bytes, or 1 KB further
 #pragma unroll
-  for (int b = 0; b < WN; ++b) w_piece[b] = b * 512 + ((j ^ wide_w_key<WN>(wn * WN * 16 + w_row + 4 * b)) * 16);
+  for (int b = 0; b < WN; ++b) w_piece[b] = SOURCE::W_TILES ? b * 2048 : b * 512 + ((j ^ wide_w_key<WN>(wn * WN * 16 + w_row + 4 * b)) * 16);
   const int a_piece = (j ^ a_key) * 16;
 
   float4v acc[WM][WN];
   Frag8 a0[WM], b0[WN], a1[WM], b1[WN];
 #define WIDE_READ_A(FA, ST, HALF, i) FA[i].u = *(const uint4*)(a_base + (ST) + (i) * 2048 + (a_piece ^ ((HALF) * 64)))
-#define WIDE_READ_W(FB, ST, HALF, i) FB[i].u = *(const uint4*)(w_base + (ST) + (w_piece[i] ^ ((HALF) * 64)))
+#define WIDE_READ_W(FB, ST, HALF, i) FB[i].u = *(const uint4*)(w_base + (ST) + (w_piece[i] ^ ((HALF) * (SOURCE::W_TILES ? 1024 : 64))))
 #define WIDE_ROW(FA, FB, i) \
   _Pragma("unroll") for (int b = 0; b < WN; ++b) acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(FB[b].v, FA[i].v, acc[i][b], 0, 0, 0);
   constexpr int READS = (WN + WM + WM - 2) / (WM - 1);  // after a row of matrix instructions, so that none follow the last
@@ -98,7 +101,7 @@ __device__ __forceinline__ void wide_loop(unsigned char* lds, SOURCE& src, SINK&
     else if (q < WN + WM) { WIDE_READ_A(FA, ST, HALF, q - WN); }                  \
   }
 
-#pragma unroll
+#pragma unroll 1  // entering a tile is much code
   for (int s = 0; s < S; ++s) {
 #pragma unroll
     for (int i = 0; i < ND; ++i) issue_one(i, s * STAGE);
@@ -146,7 +149,7 @@ __device__ __forceinline__ void wide_loop(unsigned char* lds, SOURCE& src, SINK&
     }
     stored = sink.store(tile, acc);
   }
-  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // the loads past the last step
+  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // the loads past the last step, and the last stores
 #undef WIDE_READ_A
 #undef WIDE_READ_W
 #undef WIDE_ROW

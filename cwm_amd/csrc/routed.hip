@@ -20,7 +20,7 @@
 // Matrix-core layout as in the other products of this package: operand A = the weight tile (lane 16 j + r: row
 // n0 + r, 8 values of k from 32 s + 8 j), operand B = the rows (lane 16 j + r: row r, the same k), result lane
 // 16 j + r holds out[r][n0 + 4 j + i], i = 0..3.
-#include "common.h"
+#include "gemm_wide.h"
 
 #include <type_traits>
 
@@ -923,6 +923,173 @@ __global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __re
     go(std::integral_constant<int, 2>());
 }
 
+// ---- many rows an expert, weights in operand tiles: the loop of gemm_wide.h ---------------------------------------------- //
+// What bounded the kernel above was its last round of blocks (two a compute unit; 576 on 512 places take 100 us where 512 take 74) and
+// the weights' way through registers, a step ahead.  Here 256 blocks stay, one a compute unit, and rows and weights are on their way two steps
+// ahead by direct loads, the rows gathered by the loads' own addresses.  A tile is a list's block of 128 rows of one expert and 256 columns
+// of its weights (gated: 128 gates and the same ups).  What whole rounds of such tiles leave over, where it would fill less than half of a
+// round, goes in quarters, 64 rows by 128 columns, over all blocks.  The sums' order is that of the kernel above, and so are the bits.
+// 16 experts of 2,048 x 1,024, four a token, uneven loads, the kernel above / this, gate and up, then down, us: 2,048 tokens 111 / 92 and 59 / 51,
+// 700 50 / 43 and 25 / 25, 4,096 161 / 153 and 101 / 95; 32 of 3,072 x 1,536, 1,000 tokens 174 / 156 and 105 / 90; 8 of 512 x 320, 300 tokens
+// 14.0 / 8.6 and 8.3 / 6.5; but 1,500 tokens, whose second round is two thirds full, 72 / 75 and 40 / 41: the caller's rule leaves such to it.
+#define GROUPED_BLOCKS 256
+typedef const __attribute__((address_space(4))) int* list_ints;  // read by scalar loads, which do not wait for the loads under way
+
+struct GroupedWide {
+  const bf16_t* a;
+  long a_ld;
+  list_ints row_token;  // or null: the list's own rows
+  const bf16_t *w0, *w1;
+  long w_stride;
+  list_ints tile_expert;
+  int n_tiles, n_rows, N, K;
+  int row_blocks, col_blocks;  // of whole tiles: 8 row tiles, 256 columns of weights
+  void* out;
+  long out_ld;
+  GateAct act;
+  // tile t in the order (group of WIDE_GROUP row blocks, column block, row block of the group); quarters of a tile follow one another
+  __device__ __forceinline__ void place(int t, bool quarters, int& tile0, int& col) const {
+    const int whole = quarters ? t >> 2 : t;
+    const int first = whole / (WIDE_GROUP * col_blocks) * WIDE_GROUP, rest = whole - first * col_blocks;
+    const int together = min(WIDE_GROUP, row_blocks - first);
+    tile0 = (first + rest % together) * 8 + (quarters ? (t & 1) * 4 : 0);
+    col = rest / together * 2 + (quarters ? (t >> 1) & 1 : 0);
+    if (!quarters) col >>= 1;
+  }
+};
+
+// the same for all lanes, which the compiler cannot see behind a list's entry
+__device__ __forceinline__ const bf16_t* same_for_all(const bf16_t* p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t high = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)), low = __builtin_amdgcn_readfirstlane((uint32_t)v);  // unsigned: the builtin's int would extend its sign
+  return (const bf16_t*)((uint64_t)high << 32 | low);
+}
+
+template <int WM, int WN, bool GATED, bool QUARTERS>
+struct GroupedSource {
+  const GroupedWide g;
+  int lane, wave;
+  const bf16_t *a, *u0;
+  long up;  // from the gates' weights to the ups'
+  uint32_t off[WideShape<WM, WN>::ND];
+  static constexpr bool W_TILES = true;
+  static constexpr int BM = WideShape<WM, WN>::BM;
+  __device__ __forceinline__ const bf16_t* base(int p) const {
+    const int q = p - BM / 8;
+    return q < 0 ? a : u0 + (GATED && (q >> 1) % WN >= WN / 2 ? up : 0);
+  }
+  __device__ __forceinline__ void enter(int tile) {
+    int tile0, col;
+    g.place(tile, QUARTERS, tile0, col);
+    const int expert = __builtin_amdgcn_readfirstlane(max(0, g.tile_expert[tile0 / 8 * 8]));
+    a = g.row_token ? g.a : g.a + (size_t)tile0 * TILE_ROWS * g.a_ld;
+    u0 = g.w0 + (size_t)expert * g.w_stride;
+    a = same_for_all(a), u0 = same_for_all(u0);
+    const int last_row = g.n_tiles * TILE_ROWS - 1;
+#pragma unroll
+    for (int i = 0; i < WideShape<WM, WN>::ND; ++i) {
+      const int p = min(wave + 8 * i, WideShape<WM, WN>::PIECES - 1);
+      if (p < BM / 8) {
+        const int row = 8 * p + (lane >> 3);
+        int from = min(row, last_row - tile0 * TILE_ROWS);
+        if (g.row_token) {  // eight rows, eight scalars; padding reads token 0
+          const int at = min(tile0 * TILE_ROWS + 8 * p, last_row - 7);
+          int token[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            token[e] = g.row_token[at + e];
+            asm volatile("" : "+s"(token[e]));  // or the compiler makes it a load of each lane's own, behind all that are under way
+          }
+          from = token[0];
+#pragma unroll
+          for (int e = 1; e < 8; ++e) from = (lane >> 3) == e ? token[e] : from;
+          from = max(0, from);
+        }
+        off[i] = (uint32_t)(from * (int)(g.a_ld / 8) + ((lane & 7) ^ ((row >> 1) & 7))) * 16u;
+      } else {
+        const int q = p - BM / 8, wn = q / (2 * WN), b = (q >> 1) % WN, half = q & 1;
+        constexpr int WT = GATED ? WN / 2 : WN;  // column tiles of a wavefront
+        const int n_tile = min((col * 4 + wn) * WT + b % WT, g.N / 16 - 1);  // columns past the last: theirs are not stored
+        off[i] = (uint32_t)(n_tile * (g.K / 32) + half) * 1024u + 16u * lane;
+      }
+    }
+  }
+};
+
+template <int WM, int WN, typename TC, bool GATED, bool QUARTERS>
+struct GroupedSink {
+  const GroupedWide g;
+  int lane, wave;
+  static constexpr int WT = GATED ? WN / 2 : WN, STORES = WM * WT;
+  __device__ __forceinline__ bool store(int tile, float4v (&acc)[WM][WN]) const {
+    int tile0, col;
+    g.place(tile, QUARTERS, tile0, col);
+    const int expert = g.tile_expert[tile0 / 8 * 8];
+    const int r = lane & 15, j = lane >> 4, wm = wave >> 2, wn = wave & 3;
+    const int n0 = (col * 4 + wn) * WT * 16 + 4 * j;
+    bool whole = (col + 1) * 4 * WT * 16 <= g.N;
+#pragma unroll
+    for (int a = 0; a < WM; ++a) {
+      const int t = tile0 + wm * WM + a;
+      const bool live = t < g.n_tiles && expert >= 0 && g.tile_expert[t] == expert;
+      whole = whole && live;
+      if (!live) continue;
+      TC* row = (TC*)g.out + (size_t)(t * TILE_ROWS + r) * g.out_ld + n0;
+#pragma unroll
+      for (int b = 0; b < WT; ++b) {
+        if (n0 + 16 * b >= g.N) continue;  // N is a multiple of 16: four columns lie before or past the end together
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = GATED ? gated_value(acc[a][b][i], acc[a][b + (GATED ? WT : 0)][i], g.act) : acc[a][b][i];
+        if constexpr (sizeof(TC) == 4)
+          *(float4*)(row + 16 * b) = make_float4(v[0], v[1], v[2], v[3]);
+        else
+          *(uint2*)(row + 16 * b) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+      }
+    }
+    return whole;
+  }
+};
+
+template <typename TC, bool GATED>
+__global__ void __launch_bounds__(512, 2) grouped_loop_kernel(const GroupedWide args, const int* __restrict__ used) {
+  constexpr int WM = 4, WN = 4, QM = 2, QN = 2;
+  typedef WideShape<WM, WN> Whole;
+  typedef WideShape<QM, QN> Quarter;
+  constexpr int BYTES = Whole::S * Whole::STAGE > Quarter::S * Quarter::STAGE ? Whole::S * Whole::STAGE : Quarter::S * Quarter::STAGE;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[BYTES];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  GroupedWide g = args;
+  g.row_blocks = __builtin_amdgcn_readfirstlane(((used ? min(*used, g.n_tiles) : g.n_tiles) + 7) / 8);
+  const int total = g.row_blocks * g.col_blocks, blocks = (int)gridDim.x;
+  // whole rounds of whole tiles, and one more where what is left fills more than half of it
+  int whole = total / blocks * blocks;
+  if (2 * (total - whole) > blocks) whole = total;
+  // the XCDs (block number modulo 8) take consecutive runs, their blocks in turn
+  const int groups = min(8, blocks), xcd = blockIdx.x % groups, idx = blockIdx.x / groups, peers = (blocks + groups - 1 - xcd) / groups;
+  auto share = [&](int n, int& first, int& mine) {
+    const int per = n / groups, rest = n % groups;
+    first = xcd * per + min(xcd, rest) + idx;
+    mine = (per + (xcd < rest ? 1 : 0) - idx + peers - 1) / peers;
+  };
+  const int steps = g.K / WIDE_BK;
+  int first, mine;
+  share(whole, first, mine);
+  if (mine > 0) {
+    GroupedSource<WM, WN, GATED, false> src = {g, lane, wave, nullptr, nullptr, GATED ? g.w1 - g.w0 : 0};
+    GroupedSink<WM, WN, TC, GATED, false> sink = {g, lane, wave};
+    wide_loop<WM, WN, GroupedSink<WM, WN, TC, GATED, false>::STORES>(lds, src, sink, first, peers, mine, steps);
+    asm volatile("s_barrier" ::: "memory");  // everyone has left the buffers
+  }
+  share(4 * (total - whole), first, mine);
+  if (mine > 0) {
+    GroupedSource<QM, QN, GATED, true> src = {g, lane, wave, nullptr, nullptr, GATED ? g.w1 - g.w0 : 0};
+    GroupedSink<QM, QN, TC, GATED, true> sink = {g, lane, wave};
+    wide_loop<QM, QN, GroupedSink<QM, QN, TC, GATED, true>::STORES>(lds, src, sink, 4 * whole + first, peers, mine, steps);
+  }
+}
+
 template <typename T, int RT, int CT, int WR, bool GATED>
 static void launch_grouped(bool vec, int tiles, int n_batch, hipStream_t stream, const T* a, long a_ld, long a_batch, const int* row_token,
                            const T* w0, const T* w1, long w_stride, const int* tile_expert, int n_tiles, void* out, int out_dtype,
@@ -943,11 +1110,12 @@ static void launch_grouped(bool vec, int tiles, int n_batch, hipStream_t stream,
 // multiplies the same n_rows rows by its own weight into out + z * out_batch.  tiles_a_block: 1, 2, 4 or 8 row tiles
 // a block; with a list, an expert's tiles start at a multiple of `tile_align`, itself a multiple of tiles_a_block.  used: how many
 // of the list's tiles may have rows (`cwm_group_by_expert` leaves the number), or null: any of them.  act_kind, act_alpha, act_limit: the gated
-// form's activation (`GateAct`).  tiled: the weights are in operand tiles (bfloat16, [experts][N / 16][K / 32][64][8]).
+// form's activation (`GateAct`).  tiled: the weights are in operand tiles (bfloat16, [experts][N / 16][K / 32][64][8]).  loop: products of
+// eight row tiles a block with such weights go to persistent blocks, where the rows' offsets fit 32 bits.
 extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int dtype, const int* row_token, const void* w0, const void* w1,
                                    long w_stride, const int* tile_expert, const int* used, int n_tiles, int n_batch, void* out, int out_dtype, long out_ld,
                                    long out_batch, int n_rows, int N, int K, int tiles_a_block, int tile_align, int act_kind,
-                                   float act_alpha, float act_limit, int tiled, hipStream_t stream) {
+                                   float act_alpha, float act_limit, int tiled, int loop, hipStream_t stream) {
   CWM_REQUIRE(a && w0 && out, "grouped_product: arguments missing");
   CWM_REQUIRE(!tiled || (dtype == CWM_BF16 && N % 16 == 0 && K % 64 == 0 && (long)N * K < (1l << 31)),
               "grouped_product: weights in operand tiles are bfloat16, N a multiple of 16 and K of 64");
@@ -985,6 +1153,16 @@ extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int d
     // the shape whose rows go through LDS
     const int osize = out_dtype == CWM_F32 ? 4 : 2;
     const int vec_out = (out_ld * osize) % (4 * osize) == 0 && (out_batch * osize) % (4 * osize) == 0 && ((uintptr_t)out % (4 * osize)) == 0;
+    if (loop && tiled && tiles_a_block == 8 && tile_expert && tile_align == 8 && vec_out && (unsigned long long)n_rows * a_ld * 2 < (1ull << 32) &&
+        out_dtype == (w1 ? CWM_BF16 : CWM_F32)) {
+      GroupedWide g = {(const bf16_t*)a, a_ld, (list_ints)row_token, (const bf16_t*)w0, (const bf16_t*)w1, w_stride, (list_ints)tile_expert, n_tiles, n_rows, N, K,
+                       0, (N + (w1 ? 127 : 255)) / (w1 ? 128 : 256), out, out_ld, act};
+      if (w1)
+        hipLaunchKernelGGL((grouped_loop_kernel<bf16_t, true>), dim3(GROUPED_BLOCKS), dim3(512), 0, stream, g, used);
+      else
+        hipLaunchKernelGGL((grouped_loop_kernel<float, false>), dim3(GROUPED_BLOCKS), dim3(512), 0, stream, g, used);
+      return cwm_launch_status("grouped_product");
+    }
     const int row_blocks = (tiles + tiles_a_block - 1) / tiles_a_block;
 #define CWM_WIDE_AS(RT, CT, GATED, TILED)                                                                                                            \
   do {                                                                                                                                     \

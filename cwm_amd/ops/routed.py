@@ -106,6 +106,17 @@ def _product_tiles(dtype: torch.dtype, k: int, rows: float, gated: bool) -> int:
     return 1 if gated and rows < STREAM_ROWS else _tiles_a_block(rows)
 
 
+LOOP_BLOCKS = 256  # csrc/routed.hip: GROUPED_BLOCKS
+
+
+def _loop_pays(pairs: int, n_experts: int, columns: int, gated: bool) -> bool:
+    """Whether a product of many rows an expert goes to the persistent blocks, which take tiles of 128 rows and 256 columns of
+    weights in rounds: not where the second round would be between a third and five sixths full, as the rows and half a tile of
+    padding an expert make expect (us, 1.5 and 1.7 rounds 74 and 75, the other kernel 73 and 72; 1.2 56 and 63; 2.0 77 and 97; 2.2 92 and 111)."""
+    rounds = (pairs / 128 + n_experts / 2) * -(-columns // (128 if gated else 256)) / LOOP_BLOCKS
+    return not 1.35 < rounds < 1.85
+
+
 def _empty_groups(n: int, top: int, n_experts: int, device: torch.device) -> ExpertGroups:
     pairs = n * top
     align = _tiles_a_block(pairs / n_experts)
@@ -257,7 +268,8 @@ def _grouped(
             ctypes.c_int(n_rows), ctypes.c_int(n), ctypes.c_int(k), ctypes.c_int(tiles_a_block),
             ctypes.c_int(groups.tiles_a_block if groups is not None else 1),
             ctypes.c_int(activation.code() if activation is not None else 0), ctypes.c_float(activation.alpha if activation is not None else 1.0),
-            ctypes.c_float(activation.limit if activation is not None else 0.0), ctypes.c_int(int(tiled)), _stream(),
+            ctypes.c_float(activation.limit if activation is not None else 0.0), ctypes.c_int(int(tiled)),
+            ctypes.c_int(int(groups is not None and _loop_pays(groups.pair_row.numel(), e, n, w1 is not None))), _stream(),
         ),
     )
 

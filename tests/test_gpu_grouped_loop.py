@@ -1,0 +1,36 @@
+"""Routed experts' products of many rows with weights in operand tiles (persistent blocks) beside the row-major ones: the same bits."""
+
+import pytest
+import torch
+
+from cwm_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# fewer tiles of 128 rows and 256 columns than half a round of 256 blocks (quarters alone), more than half of one (one round), rounds with a
+# rest in quarters and with one more round; a lone step of K and columns that end inside a tile; experts without rows, or with nearly all of them
+@pytest.mark.parametrize("n_tokens,n_experts,top", [(200, 4, 2), (1500, 8, 4), (3000, 8, 4), (2100, 32, 4)])
+@pytest.mark.parametrize("dim,hidden", [(64, 1088), (192, 272), (1024, 64)])
+@pytest.mark.parametrize("crowded", [False, True])
+def test_the_same_bits(n_tokens, n_experts, top, dim, hidden, crowded, monkeypatch):
+    monkeypatch.setattr("cwm_amd.ops.routed._loop_pays", lambda *sizes: True)
+    g = torch.Generator(device=DEV).manual_seed(n_tokens + dim + hidden)
+    normal = lambda *shape: torch.randn(shape, generator=g, device=DEV)  # noqa: E731
+    x = normal(n_tokens, dim).bfloat16()
+    gate, up = (normal(n_experts, hidden, dim).mul(dim**-0.5).bfloat16() for _ in range(2))
+    down = normal(n_experts, dim, hidden).mul(hidden**-0.5).bfloat16()
+    scores = normal(n_tokens, n_experts)
+    if crowded:
+        scores[:, -top:] += 5.0
+        scores[:, 0] -= 30.0
+    groups = ops.group_by_expert(scores.topk(top).indices.int().contiguous(), n_experts)
+    assert groups.tiles_a_block == 8
+    mine = groups.pair_row.long()
+    for activation in (None, ops.GatedActivation("clamped_swish", 1.7, 2.0)):
+        want = ops.grouped_gate_up(x, groups, gate, up, activation)
+        got = ops.grouped_gate_up(x, groups, ops.expert_tiles(gate), ops.expert_tiles(up), activation)
+        assert torch.equal(got[mine], want[mine])
+    if hidden % 64 == 0:
+        assert torch.equal(ops.grouped_linear(want, groups, ops.expert_tiles(down))[mine], ops.grouped_linear(want, groups, down)[mine])
