@@ -115,7 +115,10 @@ class GatedMLP(FeedForward):
         super().bind(tensors, runtime)
         matrices = [tensors[self.gate_name], tensors[self.up_name]]
         if self.row_gate is not None:
-            matrices.append(tensors[self.row_gate])
+            # with zeros up to whole groups of 16 rows: the products that share x and W through LDS take no others (2,049 columns of
+            # 2,048 at 1,500 rows: the library 23.2 us, 2,064 columns 19.0)
+            row = tensors[self.row_gate]
+            matrices += [row, row.new_zeros((-(2 * self.hidden_dim + 1) % 16, self.dim))]
         self.gate_up = LinearWeights.joined(matrices, [None] * len(matrices), stream_copy=runtime.stream_copies)
         self.down = LinearWeights(tensors[self.down_name], stream_copy=runtime.stream_copies)
 
