@@ -362,6 +362,9 @@ __global__ void __launch_bounds__(1024) group_by_expert_kernel(const int* __rest
 #define ROUTE_GROUP_TOKENS 16
 #define ROUTE_GROUP_STEPS 16  // of 32 along K, at most, a wavefront
 
+// Without GROUP a block for every 16 tokens makes logits and choices alone: any number of tokens.  Logits as a product and then the choice /
+// this, us, 16 experts: K = 2,048 17 tokens 8.6 / 6.0, 128 12.1 / 6.3, 2,048 8.3 / 6.4, 4,096 9.1 / 7.0; K = 1,024 7.1 to 12.2 / 6.0 to 6.5, 4,096 9.0 to 13.2 / 8.1 to 9.3.
+template <bool GROUP>
 __global__ void __launch_bounds__(1024) route_group_kernel(const bf16_t* __restrict__ x, long x_ld, const bf16_t* __restrict__ w,
                                                            const float* __restrict__ bias, int K, int n_tokens, int n_experts, int top, int mode,
                                                            const float* __restrict__ correction, float scale, int renormalize, int n_groups,
@@ -375,6 +378,13 @@ __global__ void __launch_bounds__(1024) route_group_kernel(const bf16_t* __restr
   const int lane = threadIdx.x & (CWM_WAVE - 1), wave = threadIdx.x / CWM_WAVE;
   const int r = lane & 15, j = lane >> 4;
   const int steps = K / 32, each = (steps + 15) / 16, first = wave * each, last = min(steps, first + each);
+  if constexpr (!GROUP) {
+    const int done = blockIdx.x * ROUTE_GROUP_TOKENS;
+    x += (size_t)done * x_ld;
+    chosen += (size_t)done * top;
+    weights += (size_t)done * top;
+    n_tokens = min(ROUTE_GROUP_TOKENS, n_tokens - done);
+  }
   const bf16_t* row = x + (size_t)min(r, n_tokens - 1) * x_ld + 8 * j;
   for (int n0 = 0; n0 < n_experts; n0 += 16) {
     const bf16_t* tile = w + ((size_t)(n0 / 16) * steps * 64 + lane) * 8;
@@ -406,7 +416,8 @@ __global__ void __launch_bounds__(1024) route_group_kernel(const bf16_t* __restr
   __syncthreads();
   if (wave < n_tokens)
     route_few(lane < n_experts ? logits[wave][lane] : -__builtin_inff(), lane, n_experts, top, mode, correction, scale, renormalize, n_groups,
-              keep_groups, picks + wave * top, weights + (size_t)wave * top);
+              keep_groups, GROUP ? picks + wave * top : chosen + (size_t)wave * top, weights + (size_t)wave * top);
+  if constexpr (!GROUP) return;
   __syncthreads();
   for (int i = threadIdx.x; i < n_tokens * top; i += blockDim.x) chosen[i] = picks[i];
   group_pairs(picks, n_tokens * top, n_experts, row_token, pair_row, tile_expert, used, n_tiles, top, tile_align, count, start);
@@ -434,10 +445,29 @@ extern "C" int cwm_route_group(const void* x, long x_ld, const void* w, const fl
   CWM_REQUIRE(tile_align >= 1 && (long)n_tiles >= ((long)n_tokens * top + TILE_ROWS - 1) / TILE_ROWS + (long)n_experts * tile_align,
               "route_group: %d tiles do not hold %d pairs of %d experts", n_tiles, n_tokens * top, n_experts);
   if (n_tokens == 0) return 0;
-  hipLaunchKernelGGL(route_group_kernel, dim3(1), dim3(1024), 0, stream, (const bf16_t*)x, x_ld, (const bf16_t*)w, bias, K, n_tokens, n_experts, top,
+  hipLaunchKernelGGL(route_group_kernel<true>, dim3(1), dim3(1024), 0, stream, (const bf16_t*)x, x_ld, (const bf16_t*)w, bias, K, n_tokens, n_experts, top,
                      mode, correction, scale, renormalize, n_groups, keep_groups, chosen, weights, row_token, pair_row, tile_expert, used, n_tiles,
                      tile_align);
   return cwm_launch_status("route_group");
+}
+
+// The same without the lists, for any number of tokens.
+extern "C" int cwm_route_rows(const void* x, long x_ld, const void* w, const float* bias, int K, int n_tokens, int n_experts, int top, int mode,
+                              const float* correction, float scale, int renormalize, int n_groups, int keep_groups, int* chosen, float* weights,
+                              hipStream_t stream) {
+  CWM_REQUIRE(x && w && chosen && weights && n_tokens >= 0, "route_rows: arguments missing");
+  CWM_REQUIRE(n_experts >= 1 && n_experts <= CWM_WAVE && top >= 1 && top <= ROUTE_MAX_TOP && top <= n_experts, "route_rows: %d of %d experts, the kernel takes up to %d of %d",
+              top, n_experts, ROUTE_MAX_TOP, CWM_WAVE);
+  CWM_REQUIRE(K >= 32 && K % 32 == 0 && K <= 16 * 32 * ROUTE_GROUP_STEPS && x_ld >= K && x_ld % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0,
+              "route_rows: rows of %d elements must be a multiple of 32, up to %d, at multiples of 16 bytes", K, 16 * 32 * ROUTE_GROUP_STEPS);
+  CWM_REQUIRE(mode == 0 || mode == 1, "route_rows: unknown mode %d", mode);
+  CWM_REQUIRE(n_groups >= 1 && n_experts % n_groups == 0 && keep_groups >= 1 && keep_groups <= n_groups && top <= keep_groups * (n_experts / n_groups),
+              "route_rows: %d of %d groups of %d experts do not hold %d choices", keep_groups, n_groups, n_experts, top);
+  if (n_tokens == 0) return 0;
+  hipLaunchKernelGGL(route_group_kernel<false>, dim3((n_tokens + ROUTE_GROUP_TOKENS - 1) / ROUTE_GROUP_TOKENS), dim3(1024), 0, stream, (const bf16_t*)x, x_ld,
+                     (const bf16_t*)w, bias, K, n_tokens, n_experts, top, mode, correction, scale, renormalize, n_groups, keep_groups, chosen, weights,
+                     nullptr, nullptr, nullptr, nullptr, 0, 1);
+  return cwm_launch_status("route_rows");
 }
 
 // used: one number, the tiles up to the last one that has rows, rounded up to tile_align.  tile_align: an expert's first tile lies at a multiple of so many tiles (the tiles that one block of the product takes).

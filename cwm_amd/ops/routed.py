@@ -151,20 +151,14 @@ def route_group_pays(n_experts: int, k: int) -> bool:
     return n_experts <= ROUTE_GROUP_PAYS_EXPERTS and k % 32 == 0 and k <= ROUTE_GROUP_PAYS_K
 
 
-def route_and_group(
-    x: torch.Tensor, router_copy: torch.Tensor, bias: Optional[torch.Tensor], n_experts: int, top: int, scores: str = "softmax_chosen",
-    correction: Optional[torch.Tensor] = None, scale: float = 1.0, renormalize: bool = False, groups: Optional[Tuple[int, int]] = None,
-) -> Tuple[torch.Tensor, torch.Tensor, ExpertGroups]:
-    """(chosen, weights, lists): what `route_top` and `group_by_expert` make of the logits W x + bias, in one launch; the logits are added in the
-    streaming product's order, so the bits are the same where that does not split K (up to 6,144).
-    `x` bfloat16 [T <= 16, K] (K a multiple of 32, up to 8,192), `router_copy` the streaming copy (`stream_layout`) of the
-    bfloat16 router [E <= 64, K], `bias` float32 [E] or None; the rest as in `route_top`."""
-    KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
+def _route_checks(x, router_copy, bias, n_experts, top, scores, correction, scale, renormalize, groups) -> Tuple[int, int, int, int]:
+    """(tokens, K, groups of experts, groups that stay open) of a router's launch after checking its arguments."""
+    KernelError, _, _, _, _need_gpu, *_ = _base()
     _need_gpu(x, router_copy, bias, correction)
     _check_scores(scores, correction, scale, renormalize, n_experts)
-    most_tokens, most_experts, most_k = route_group_limits()
-    if x.dim() != 2 or x.dtype != torch.bfloat16 or x.stride(1) != 1 or x.shape[0] > most_tokens:
-        raise KernelError(f"x must be bfloat16 [T <= {most_tokens}, K] with contiguous rows")
+    _, most_experts, most_k = route_group_limits()
+    if x.dim() != 2 or x.dtype != torch.bfloat16 or x.stride(1) != 1:
+        raise KernelError("x must be bfloat16 [T, K] with contiguous rows")
     n, k = x.shape
     if not 1 <= n_experts <= most_experts or k % 32 != 0 or k > most_k:
         raise KernelError(f"{n_experts} experts of rows of {k}: the kernel takes up to {most_experts}, rows of a multiple of 32 up to {most_k}")
@@ -175,6 +169,43 @@ def route_and_group(
     if not 1 <= top <= min(n_experts, MAX_ROUTE_TOP):
         raise KernelError(f"{top} of {n_experts} experts: the kernel takes 1..{min(n_experts, MAX_ROUTE_TOP)}")
     count, keep = _open_groups(groups, n_experts, top)
+    return n, k, count, keep
+
+
+def route_rows(
+    x: torch.Tensor, router_copy: torch.Tensor, bias: Optional[torch.Tensor], n_experts: int, top: int, scores: str = "softmax_chosen",
+    correction: Optional[torch.Tensor] = None, scale: float = 1.0, renormalize: bool = False, groups: Optional[Tuple[int, int]] = None,
+) -> Tuple[torch.Tensor, torch.Tensor]:
+    """A router's logits (bfloat16 x [T, K], its streaming copy, `bias` float32 [E] or None) and the choice of `route_top` in one launch, a
+    block for every 16 tokens: (chosen, weights).  The logits' sums are those of `route_and_group`."""
+    KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
+    n, k, count, keep = _route_checks(x, router_copy, bias, n_experts, top, scores, correction, scale, renormalize, groups)
+    chosen = torch.empty((n, top), dtype=torch.int32, device=x.device)
+    weights = torch.empty((n, top), dtype=torch.float32, device=x.device)
+    lib = _build.load("routed")
+    _check(
+        lib,
+        lib.cwm_route_rows(
+            _ptr(x), ctypes.c_long(x.stride(0) if n > 1 else k), _ptr(router_copy), _ptr(bias), ctypes.c_int(k), ctypes.c_int(n), ctypes.c_int(n_experts),
+            ctypes.c_int(top), ctypes.c_int(int(scores == "softmax_all")), _ptr(correction), ctypes.c_float(scale), ctypes.c_int(int(renormalize)),
+            ctypes.c_int(count), ctypes.c_int(keep), _ptr(chosen), _ptr(weights), _stream(),
+        ),
+    )
+    return chosen, weights
+
+
+def route_and_group(
+    x: torch.Tensor, router_copy: torch.Tensor, bias: Optional[torch.Tensor], n_experts: int, top: int, scores: str = "softmax_chosen",
+    correction: Optional[torch.Tensor] = None, scale: float = 1.0, renormalize: bool = False, groups: Optional[Tuple[int, int]] = None,
+) -> Tuple[torch.Tensor, torch.Tensor, ExpertGroups]:
+    """(chosen, weights, lists): what `route_top` and `group_by_expert` make of the logits W x + bias, in one launch; the logits are added in the
+    streaming product's order, so the bits are the same where that does not split K (up to 6,144).
+    `x` bfloat16 [T <= 16, K] (K a multiple of 32, up to 8,192), `router_copy` the streaming copy (`stream_layout`) of the
+    bfloat16 router [E <= 64, K], `bias` float32 [E] or None; the rest as in `route_top`."""
+    KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
+    if x.dim() == 2 and x.shape[0] > route_group_limits()[0]:
+        raise KernelError(f"x must be bfloat16 [T <= {route_group_limits()[0]}, K] with contiguous rows")
+    n, k, count, keep = _route_checks(x, router_copy, bias, n_experts, top, scores, correction, scale, renormalize, groups)
     chosen = torch.empty((n, top), dtype=torch.int32, device=x.device)
     weights = torch.empty((n, top), dtype=torch.float32, device=x.device)
     lists = _empty_groups(n, top, n_experts, x.device)

@@ -82,7 +82,7 @@ class RoutedExperts(FeedForward):
         if self.shared is not None:
             n = len(self.shared_prefix)
             self.shared.bind({name[n:]: t for name, t in tensors.items() if name.startswith(self.shared_prefix)}, runtime)
-        # the streaming copy of a small router: a step of few tokens makes its logits, choices and lists in one launch from it
+        # the streaming copy of a small router: logits and choices (a step of few tokens: the lists too) come from it in one launch
         self.router_copy: Optional[torch.Tensor] = None
         if (
             runtime.device.type == "cuda" and runtime.act_dtype == torch.bfloat16 and self.router.dtype == torch.bfloat16
@@ -111,8 +111,12 @@ class RoutedExperts(FeedForward):
         """The same without the last kernel: every pair's row and the weights, for a consumer that adds a token's
         rows up itself (a norm that takes a `RoutedSum` as the pending result)."""
         router = (self.top, self.scores, self.choice_correction, self.weight_scale, self.renormalize, self.groups)
-        if self.router_copy is not None and x.shape[0] <= self.few_tokens and x.data_ptr() % 16 == 0:
-            _, weights, groups = ops.route_and_group(x, self.router_copy, self.router_b, self.n_experts, *router)
+        if self.router_copy is not None and x.data_ptr() % 16 == 0 and x.stride(0) % 8 == 0:
+            if x.shape[0] <= self.few_tokens:
+                _, weights, groups = ops.route_and_group(x, self.router_copy, self.router_b, self.n_experts, *router)
+            else:
+                chosen, weights = ops.route_rows(x, self.router_copy, self.router_b, self.n_experts, *router)
+                groups = ops.group_by_expert(chosen, self.n_experts)
         else:
             chosen, weights = ops.route_top(ops.linear(x, self.router, self.router_b, torch.float32), *router)
             groups = ops.group_by_expert(chosen, self.n_experts)
