@@ -526,6 +526,40 @@ extern "C" int cwm_qk_norm_rope_write(const void* src, int src_dtype, long src_s
   return cwm_launch_status("qk_norm_rope_write");
 }
 
+// Whole value blocks of a step's tokens.  A value block is eight keys of a page, 16 bytes of bfloat16 for each dimension; a block of
+// threads a token writes two bytes of each.  The eight blocks of a window of tokens [8 b, 8 b + 8) therefore share the eight tokens
+// in a row, first one in the window, whose places are a value block from its first key to its last (one at most begins in a
+// window, since two in a row begin eight tokens apart): each block writes an eighth of the dimensions, 16 bytes at a time.
+// One wavefront calls `find` with the window's first token; the others read the result behind a barrier.
+struct ValueRuns {
+  enum { SPAN = 24 };  // tokens 8 b - 8 .. 8 b + 15: runs that begin in the window or reach into it
+  int page[SPAN], slot[SPAN];
+  unsigned starts;  // bit i: a run begins at token 8 b - 8 + i
+
+  __device__ __forceinline__ void find(int window, int n_tokens, const int* positions, const int* seq_of_token, const int* block_table,
+                                       int table_width, int page_size, int num_pages) {
+    const int lane = threadIdx.x & (CWM_WAVE - 1), u = window - 8 + lane;
+    int p = -1, s = 0;
+    if (lane < SPAN && u >= 0 && u < n_tokens) {
+      const int pos = positions[u], lp = pos / page_size;
+      s = pos - lp * page_size;
+      if (lp >= 0 && lp < table_width) p = block_table[(size_t)seq_of_token[u] * table_width + lp];
+      if (p >= num_pages) p = -1;
+    }
+    const int next_p = __shfl_down(p, 1, CWM_WAVE), next_s = __shfl_down(s, 1, CWM_WAVE);
+    const unsigned follows = (unsigned)__ballot(lane < SPAN - 1 && p >= 0 && next_p == p && next_s == s + 1);
+    const unsigned first = (unsigned)__ballot(lane < SPAN && p >= 0 && s % 8 == 0);
+    if (lane < SPAN) page[lane] = p, slot[lane] = s;
+    const unsigned two = follows & (follows >> 1), four = two & (two >> 2);  // that many tokens follow on from here
+    if (lane == 0) starts = first & four & (two >> 4) & (follows >> 6);
+  }
+  // whether token `u` of the window is written with a run
+  __device__ __forceinline__ bool covers(int u) const {
+    const int i = 8 + (u & 7);
+    return page[i] >= 0 && slot[i] >= 0 && (starts >> (i - slot[i] % 8)) & 1;
+  }
+};
+
 // ---- projection rows -> bias -> norm of every head -> rotation -> (values mixed with another layer's) -> cache -- //
 // A token's row of the joined projection is [q: Hq * qk_dim | k: Hkv * qk_dim | v: Hkv * v_dim | ...] (type TS, or
 // float32 partial sums of a split K, added in order), to which `bias` (float32, one value a column of q, k and v) is
@@ -540,10 +574,14 @@ extern "C" int cwm_qk_norm_rope_write(const void* src, int src_dtype, long src_s
 // reduction over the lanes; the blocks of a token (gridDim.y of them) share its heads.
 // VEC: head_dim / 4 is a power of two up to a wavefront, every size is a multiple of 4 and every row starts at a multiple of 16
 // bytes (8 for bfloat16): head_dim / 4 lanes take a head, four elements each.  An XCD takes a run of neighbouring tokens: eight
-// of them write the eight values of each 16 bytes of a value block, which meet in its L2.  Bound by the values' narrow writes:
-// 2,296 tokens with 16 and 4 heads of 128 take 15.6 us where a wavefront a head, one element a load and neighbouring tokens on
-// different XCDs took 27.7; with 32 and 8 heads 27.6 against 47.8; one token of 32 and 8 heads 4.2 against 5.1.
-template <typename TS, typename TO, bool VEC>
+// of them write the eight values of each 16 bytes of a value block, which meet in its L2.  Against a wavefront a head, one element a
+// load and neighbouring tokens on different XCDs: 2,296 tokens with 16 and 4 heads of 128 15.6 and 27.7 us; with 32 and 8 heads 27.6
+// and 47.8; one token of 32 and 8 heads 4.2 and 5.1.
+// RUNS: whole value blocks (`ValueRuns`) instead of the two-byte writes that bounded it, us at 512, 2,296 and 8,192 tokens: 16 and 4
+// heads of 128 7.1, 14.4, 38.6 to 6.0, 12.4, 34.2; 32 and 8 10.4, 26.0, 65.7 to 8.8, 20.9, 52.5; 16 and 16 of 64 7.9, 19.3, 53.4 to 5.9,
+// 11.7, 32.1; 8 and 1 of 256 6.7, 12.5, 31.4 to 6.1, 12.2, 33.5, so an eighth of the queries' heads stays with narrow writes.  (A head's
+// elements asked for a head ahead: 32 and 8 heads 21.6 and 57.4.)
+template <typename TS, typename TO, bool VEC, bool RUNS>
 __global__ void __launch_bounds__(256)
 head_norm_rope_write_kernel(const TS* __restrict__ src, long src_stride, int n_partials, long partial_stride,
                             const float* __restrict__ bias, TO* __restrict__ q_out, const float* __restrict__ q_weight,
@@ -599,6 +637,9 @@ head_norm_rope_write_kernel(const TS* __restrict__ src, long src_stride, int n_p
     cs[2 * i] = c;
     cs[2 * i + 1] = s;
   }
+  __shared__ ValueRuns runs;  // only where RUNS reads it
+  if constexpr (RUNS)
+    if (wave == 3) runs.find(t & ~7, n_tokens, positions, seq_of_token, block_table, table_width, page_size, num_pages);
   __syncthreads();
   const int n_heads = n_q_heads + (cache ? n_kv_heads : 0);
   const int waves = blockDim.x / CWM_WAVE;
@@ -667,6 +708,43 @@ head_norm_rope_write_kernel(const TS* __restrict__ src, long src_stride, int n_p
         Elem<TO>::store(dst + 2 * i + 1, b * c + a * s);
       }
     }
+  }
+  if constexpr (RUNS) {
+    const unsigned begins = (runs.starts >> 8) & 0xff;
+    if (begins) {
+      const int i = 8 + __builtin_ctz(begins), first = (t & ~7) - 8 + i;  // the run's first token
+      const int v_base = q_width + k_width;
+      const float mix = (v_other && v_mix) ? *v_mix : 0.f;
+      TO* to = cache + ((size_t)runs.page[i] * 2 + 1) * n_kv_heads * page_size * head_dim + (size_t)(runs.slot[i] / 8) * head_dim * 8;
+      const int share = (n_kv_heads * head_dim + 7) / 8, last = min(n_kv_heads * head_dim, ((t & 7) + 1) * share);
+      // the last wavefronts first: they have the fewest heads
+      for (int e = (t & 7) * share + (threadIdx.x ^ 192); e < last; e += 256) {
+        const int head = e / head_dim, d = e - head * head_dim;
+        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (d < v_dim) {
+          const int at = v_base + head * v_dim + d;
+          const TS* from = src + (size_t)first * src_stride + at;
+          for (int p = 0; p < n_partials; ++p)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] += Elem<TS>::load(from + j * src_stride + (size_t)p * partial_stride);
+          const float b = bias ? bias[at] : 0.f;
+          if (bias)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] += b;
+          if (v_other) {
+            const TO* other = v_other + (size_t)first * v_other_stride + head * v_dim + d;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = (1.0f - mix) * v[j] + mix * Elem<TO>::load(other + j * v_other_stride);
+          }
+          if (v_keep)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) Elem<TO>::store(v_keep + ((size_t)(first + j) * n_kv_heads + head) * v_dim + d, v[j]);
+        }
+        *(uint4*)(to + (size_t)head * head_dim * page_size + d * 8) =
+            make_uint4(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]), pack2_bf16(v[4], v[5]), pack2_bf16(v[6], v[7]));
+      }
+    }
+    if (runs.covers(t)) return;
   }
   if (vdst || v_keep) {
     const int v_block = (page_size % 8 == 0) ? 8 : page_size;
@@ -746,12 +824,16 @@ extern "C" int cwm_head_norm_rope_write(const void* src, int src_dtype, long src
   const bool vec = head_dim % 4 == 0 && quarter <= CWM_WAVE && (quarter & (quarter - 1)) == 0 && qk_dim % 4 == 0 && v_dim % 4 == 0 && src_stride % 4 == 0 &&
                    partial_stride % 4 == 0 && v_other_stride % 4 == 0 && aligned(src, src_dtype) && aligned(q_out, out_dtype) && aligned(cache, out_dtype) &&
                    aligned(v_other, out_dtype) && aligned(v_keep, out_dtype) && (((uintptr_t)bias | (uintptr_t)q_weight | (uintptr_t)k_weight) % 16) == 0;
+  // whole value blocks where a block takes a token and the values are enough of the work (times above)
+  const bool runs = vec && gy == 1 && cache && 8 * n_kv_heads > n_q_heads && out_dtype == CWM_BF16 && page_size % 8 == 0 && (uintptr_t)cache % 16 == 0;
 #define CWM_HEAD_NORM_ROPE(TS, TO)                                                                                         \
   do {                                                                                                                     \
-    if (vec) CWM_HEAD_NORM_ROPE_V(TS, TO, true); else CWM_HEAD_NORM_ROPE_V(TS, TO, false);                                 \
+    if (runs) CWM_HEAD_NORM_ROPE_V(TS, TO, true, sizeof(TO) == 2);                                                         \
+    else if (vec) CWM_HEAD_NORM_ROPE_V(TS, TO, true, false);                                                               \
+    else CWM_HEAD_NORM_ROPE_V(TS, TO, false, false);                                                                       \
   } while (0)
-#define CWM_HEAD_NORM_ROPE_V(TS, TO, V)                                                                                    \
-  hipLaunchKernelGGL((head_norm_rope_write_kernel<TS, TO, V>), grid, dim3(256), 0, stream, (const TS*)src,                  \
+#define CWM_HEAD_NORM_ROPE_V(TS, TO, V, RUNS)                                                                              \
+  hipLaunchKernelGGL((head_norm_rope_write_kernel<TS, TO, V, RUNS>), grid, dim3(256), 0, stream, (const TS*)src,                  \
                      src_stride, n_partials, partial_stride, bias, (TO*)q_out, q_weight, k_weight, eps, positions,         \
                      seq_of_token, inv_freq, (TO*)cache, block_table, table_width, page_size, num_pages, n_q_heads,        \
                      n_kv_heads, qk_dim, v_dim, head_dim, (const TO*)v_other, v_other_stride, v_mix, (TO*)v_keep, temp_coef, temp_every, n_tokens)
