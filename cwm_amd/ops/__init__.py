@@ -810,7 +810,7 @@ def _tile_wins(x: torch.Tensor, weight: torch.Tensor) -> bool:
     (up to 16,384 columns: 41 against 67 us for the 32B shape's q/k/v product at 256 rows, 89 against 234 us
     for its feed-forward's second product).  With two blocks of rows (up to 512) it was ahead on that second
     product alone (144 against 195 us at 384 rows), which the float32 partial sums that the next kernel then
-    reads cost again in a decode step, so more than 256 rows go to the library."""
+    reads cost again in a decode step, so more than 256 rows go to the wide kernel or the library (`_prefers_wide`)."""
     m = x.shape[0]
     if m > TILE_TALL_ROWS or not _tile_takes(x, weight):
         return False
