@@ -978,7 +978,7 @@ struct GroupedWide {
   long out_ld;
   GateAct act;
   // tile t in the order (group of WIDE_GROUP row blocks, column block, row block of the group); quarters of a tile follow one another
-  __device__ __forceinline__ void place(int t, bool quarters, int& tile0, int& col) const {
+  __host__ __device__ __forceinline__ void place(int t, bool quarters, int& tile0, int& col) const {
     const int whole = quarters ? t >> 2 : t;
     const int first = whole / (WIDE_GROUP * col_blocks) * WIDE_GROUP, rest = whole - first * col_blocks;
     const int together = min(WIDE_GROUP, row_blocks - first);
@@ -986,7 +986,21 @@ struct GroupedWide {
     col = rest / together * 2 + (quarters ? (t >> 1) & 1 : 0);
     if (!quarters) col >>= 1;
   }
+  // the row that a tile's loads start from, and how far past it its row `row` is read: rows past the list are its last one again.  A list whose
+  // tiles in use are not counted may end inside a block, and the lower quarters of that block begin past it
+  __host__ __device__ __forceinline__ int first_row(int tile0) const { return min(tile0, n_tiles - 1) * TILE_ROWS; }
+  __host__ __device__ __forceinline__ int from_first(int tile0, int row) const { return min(row, n_tiles * TILE_ROWS - 1 - first_row(tile0)); }
 };
+
+// for tests: what `from_first` gives for tile `t` of a list of `n_tiles`, and the row it counts from
+extern "C" int cwm_grouped_loop_rows(int n_tiles, int col_blocks, int t, int quarters, int row, int* first) {
+  GroupedWide g = {};
+  g.n_tiles = n_tiles, g.row_blocks = (n_tiles + 7) / 8, g.col_blocks = col_blocks;
+  int tile0, col;
+  g.place(t, quarters != 0, tile0, col);
+  *first = g.first_row(tile0);
+  return g.from_first(tile0, row);
+}
 
 // the same for all lanes, which the compiler cannot see behind a list's entry
 __device__ __forceinline__ const bf16_t* same_for_all(const bf16_t* p) {
@@ -1012,7 +1026,7 @@ struct GroupedSource {
     int tile0, col;
     g.place(tile, QUARTERS, tile0, col);
     const int expert = __builtin_amdgcn_readfirstlane(max(0, g.tile_expert[tile0 / 8 * 8]));
-    a = g.row_token ? g.a : g.a + (size_t)tile0 * TILE_ROWS * g.a_ld;
+    a = g.row_token ? g.a : g.a + (size_t)g.first_row(tile0) * g.a_ld;
     u0 = g.w0 + (size_t)expert * g.w_stride;
     a = same_for_all(a), u0 = same_for_all(u0);
     const int last_row = g.n_tiles * TILE_ROWS - 1;
@@ -1021,7 +1035,7 @@ struct GroupedSource {
       const int p = min(wave + 8 * i, WideShape<WM, WN>::PIECES - 1);
       if (p < BM / 8) {
         const int row = 8 * p + (lane >> 3);
-        int from = min(row, last_row - tile0 * TILE_ROWS);
+        int from = g.from_first(tile0, row);
         if (g.row_token) {  // eight rows, eight scalars; padding reads token 0
           const int at = min(tile0 * TILE_ROWS + 8 * p, last_row - 7);
           int token[8];

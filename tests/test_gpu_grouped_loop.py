@@ -1,5 +1,7 @@
 """Routed experts' products of many rows with weights in operand tiles (persistent blocks) beside the row-major ones: the same bits."""
 
+import dataclasses
+
 import pytest
 import torch
 
@@ -34,3 +36,23 @@ def test_the_same_bits(n_tokens, n_experts, top, dim, hidden, crowded, monkeypat
         assert torch.equal(got[mine], want[mine])
     if hidden % 64 == 0:
         assert torch.equal(ops.grouped_linear(want, groups, ops.expert_tiles(down))[mine], ops.grouped_linear(want, groups, down)[mine])
+
+
+# lists of one to eight tiles past a whole block, which end in each of a block's tiles
+@pytest.mark.parametrize("past", range(1, 9))
+def test_lists_whose_tiles_are_not_counted(past, monkeypatch):
+    """Without the number of tiles in use the blocks walk the whole list, whose last one may end inside its rows."""
+    monkeypatch.setattr("cwm_amd.ops.routed._loop_pays", lambda *sizes: True)
+    n_experts, top, dim, hidden = 4, 2, 192, 320
+    n_tokens = 8 * (64 + past) - 3
+    g = torch.Generator(device=DEV).manual_seed(past)
+    normal = lambda *shape: torch.randn(shape, generator=g, device=DEV)  # noqa: E731
+    x, gate, up = normal(n_tokens, dim).bfloat16(), *(normal(n_experts, hidden, dim).mul(dim**-0.5).bfloat16() for _ in range(2))
+    down = normal(n_experts, dim, hidden).mul(hidden**-0.5).bfloat16()
+    groups = ops.group_by_expert(normal(n_tokens, n_experts).topk(top).indices.int().contiguous(), n_experts)
+    assert groups.tiles_a_block == 8 and groups.n_tiles % 8 == past % 8
+    mine = groups.pair_row.long()
+    want = ops.grouped_gate_up(x, groups, gate, up)
+    lists = dataclasses.replace(groups, used=None)
+    assert torch.equal(ops.grouped_gate_up(x, lists, ops.expert_tiles(gate), ops.expert_tiles(up))[mine], want[mine])
+    assert torch.equal(ops.grouped_linear(want, lists, ops.expert_tiles(down))[mine], ops.grouped_linear(want, groups, down)[mine])
