@@ -1,0 +1,41 @@
+"""Which products of many rows the wide kernel takes: what it refuses goes to the library, as any operand did before there was such a kernel."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from cwm_amd import ops
+
+M, N, K = 300, 1024, 512
+
+
+def _operands(device):
+    gen = torch.Generator().manual_seed(1)
+    x, w = torch.randn(M, K + 8, generator=gen).bfloat16().to(device), (torch.randn(N, K + 8, generator=gen) * K**-0.5).bfloat16().to(device)
+    return x, w
+
+
+def _overlapping(x, w):
+    """Pairs with rows that repeat or overlap: one row for all, and windows that move on by eight elements."""
+    flat_x, flat_w = x.reshape(-1), w.reshape(-1)
+    yield x[:1, :K].expand(M, K), w[:, :K]
+    yield x[:, :K], w[:1, :K].expand(N, K)
+    yield flat_x.as_strided((M, K), (8, 1)), w[:, :K]
+    yield x[:, :K], flat_w.as_strided((N, K), (K - 8, 1))
+
+
+def test_rows_that_overlap_are_not_taken():
+    x, w = _operands("cpu")
+    assert ops._wide_takes(x[:, :K], w[:, :K])
+    assert ops._wide_takes(x[:1, :K], w[:, :K])  # of a lone row the stride says nothing
+    assert not any(ops._wide_takes(*pair) for pair in _overlapping(x, w))
+
+
+@pytest.mark.gpu
+def test_rows_that_overlap_go_to_the_library():
+    x, w = _operands("cuda:0")
+    assert ops._prefers_wide(x[:, :K], w[:, :K])
+    for a, b in _overlapping(x, w):
+        assert torch.equal(ops.gemm_bf16(a, b), torch.mm(a, b.t()))
+        assert torch.equal(ops.gate_up_silu(a, b, None, True), ops.silu_mul(torch.mm(a, b.t()), grouped=True))
