@@ -671,7 +671,6 @@ def _tile_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
         and k % 64 == 0 and n % 16 == 0 and 0 < x.shape[0] <= TILE_MAX_ROWS
         and x.stride(-1) == 1 and weight.stride(-1) == 1
         and (x.shape[0] <= 1 or x.stride(0) % 8 == 0) and (n <= 1 or weight.stride(0) % 8 == 0)
-        and (x.shape[0] <= 1 or x.stride(0) >= k) and (n <= 1 or weight.stride(0) >= k)  # rows that overlap are the library's
         and max(x.stride(0), weight.stride(0)) < (1 << 22)
         and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
     )

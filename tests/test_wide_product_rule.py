@@ -39,3 +39,18 @@ def test_rows_that_overlap_go_to_the_library():
     for a, b in _overlapping(x, w):
         assert torch.equal(ops.gemm_bf16(a, b), torch.mm(a, b.t()))
         assert torch.equal(ops.gate_up_silu(a, b, None, True), ops.silu_mul(torch.mm(a, b.t()), grouped=True))
+
+
+def test_rows_that_overlap_stay_with_the_tiled_kernels_check():
+    """Up to its number of rows the tiled kernel has always been asked first, and refuses such operands."""
+    x, w = _operands("cpu")
+    assert all(ops._tile_takes(a[:100], b) for a, b in _overlapping(x, w))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [40, 100, 200])
+def test_few_rows_that_overlap_are_refused(rows):
+    x, w = _operands("cuda:0")
+    for a, b in _overlapping(x, w):
+        with pytest.raises(ops.KernelError):
+            ops.gemm_bf16(a[:rows], b)
