@@ -239,6 +239,9 @@ def gemm_f32(
     return out
 
 
+F32_PARTS_STRIDE = 1 << 23  # csrc/gemm_f32.hip: a block's byte offsets from its first row of W fit 32 bits; rows further apart are copied
+
+
 def gemm_f32_parts(
     x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None, block: Optional[int] = None,
 ) -> torch.Tensor:
@@ -255,6 +258,8 @@ def gemm_f32_parts(
     n = weight.shape[0]
     if bias is not None and (bias.shape != (n,) or not bias.is_contiguous()):
         raise KernelError(f"gemm: bias {tuple(bias.shape)} does not fit {n} outputs")
+    if n > 1 and weight.stride(0) >= F32_PARTS_STRIDE:
+        weight = weight.contiguous()
     lib = _build.load("gemm_f32")
     out = torch.empty((m, n), dtype=out_dtype or x.dtype, device=x.device)
     scratch = torch.empty(-(-m // 16) * (k // 32 * 3072 + -(-k // 256) * 4), dtype=torch.uint8, device=x.device)
@@ -274,7 +279,7 @@ def _f32_parts_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
         x.dtype == torch.float32 and weight.dtype == torch.float32
         and x.shape[0] > 0 and x.shape[1] % 32 == 0 and 0 < x.shape[1] <= 65536 and x.stride(-1) == 1 and weight.stride(-1) == 1
         and (x.shape[0] <= 1 or x.stride(0) % 4 == 0) and (weight.shape[0] <= 1 or weight.stride(0) % 4 == 0)
-        and weight.stride(0) < (1 << 23) and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+        and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
     )
 
 

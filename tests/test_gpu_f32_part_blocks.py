@@ -44,3 +44,13 @@ def test_what_it_refuses():
             ops.gemm_f32_parts(*bad)
     with pytest.raises(ops.KernelError):
         ops.gemm_f32_parts(x, w, block=BLOCKS)
+
+
+@pytest.mark.parametrize("rows", [1, 5])
+def test_weights_whose_rows_lie_far_apart(rows):
+    """Rows 32 MB apart and more are no other product: the bits of the same rows side by side."""
+    apart = 1 << 23
+    x, far = torch.randn(40, 96, device=DEV), torch.empty((rows - 1) * apart + 96, device=DEV).as_strided((rows, 96), (apart, 1))
+    far.copy_(torch.randn(rows, 96, device=DEV))
+    assert ops._f32_parts_takes(x, far)
+    assert torch.equal(ops.gemm_f32(x, far), ops.gemm_f32(x, far.contiguous()))
