@@ -191,57 +191,89 @@ gemm_f32_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lo
 // columns, 16 each, with all WM tiles of 16 rows.  Operands of A and raw rows of W reach LDS by direct loads, W two steps further ahead; a
 // wavefront takes the next step's W apart while it multiplies; one barrier a step.  Now 828, 3,440 (1.36 PFLOP/s of bfloat16 products, of
 // which the chip's power allows 1.5 to 1.7), 198, 495 and 61 us, and the same bits.
-#define PARTS_STEPS 8  // of K whose parts a wavefront of the first kernel makes
+#define PARTS_STEPS 8  // of K whose parts a block of the first kernel makes
 
 struct PartRows {  // a row's marks: bit r of [row tile][group of PARTS_STEPS steps]
   const uint32_t* flags;
   int groups;
 };
 
-__global__ void __launch_bounds__(256) f32_parts_kernel(const float* __restrict__ A, long lda, int M, int steps, uint4* __restrict__ parts, uint32_t* __restrict__ flags,
-                                                        int groups) {
-  const int lane = threadIdx.x & 63, r = lane & 15, j = lane >> 4;
-  const int tile = blockIdx.x, group = blockIdx.y * 4 + (threadIdx.x >> 6);
-  if (group >= groups) return;
-  const int m = tile * 16 + r;
-  const float* src = A + (size_t)min(m, M - 1) * lda + 8 * j;
-  float largest = 0.f;
-  const int first = group * PARTS_STEPS, end = min(first + PARTS_STEPS, steps);
-  for (int s = first; s < end; ++s) {
-    const float4v x = *(const float4v*)(src + 32 * s), y = *(const float4v*)(src + 32 * s + 4);
-    float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
-    const float scale = ((s + SPLIT_TURN) / (2 * SPLIT_TURN)) & 1 ? -SPLIT_SCALE : SPLIT_SCALE;
+// Eight values of a row at step `s`, turned with it, as their three parts in the matrix instruction's order; the largest of them, once scaled.
+__device__ __forceinline__ float take_eight_apart(const float4v& x, const float4v& y, int s, bool live, uint4 (&part)[3]) {
+  float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]}, largest = 0.f;
+  const float scale = ((s + SPLIT_TURN) / (2 * SPLIT_TURN)) & 1 ? -SPLIT_SCALE : SPLIT_SCALE;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      v[e] = m < M ? v[e] * scale : 0.f;
-      largest = fmaxf(largest, fabsf(v[e]));
-    }
-#pragma unroll
-    for (int part = 0; part < 3; ++part) {
-      uint32_t w[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        w[e] = pack2_bf16(v[2 * e], v[2 * e + 1]);
-        v[2 * e] -= __uint_as_float(w[e] << 16), v[2 * e + 1] -= __uint_as_float(w[e] & 0xffff0000u);
-      }
-      parts[(((size_t)tile * steps + s) * 3 + part) * 64 + lane] = make_uint4(w[0], w[1], w[2], w[3]);
-    }
+  for (int e = 0; e < 8; ++e) {
+    v[e] = live ? v[e] * scale : 0.f;
+    largest = fmaxf(largest, fabsf(v[e]));
   }
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      w[e] = pack2_bf16(v[2 * e], v[2 * e + 1]);
+      v[2 * e] -= __uint_as_float(w[e] << 16), v[2 * e + 1] -= __uint_as_float(w[e] & 0xffff0000u);
+    }
+    part[p] = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+  return largest;
+}
+// Bit r: the wavefront's lanes 16 j + r saw a value beyond the parts.
+__device__ __forceinline__ uint32_t rows_beyond(float largest) {
   const unsigned long long over = __ballot(!(largest < SPLIT_LIMIT));
-  if (lane == 0) flags[(size_t)tile * groups + group] = (uint32_t)((over | over >> 16 | over >> 32 | over >> 48) & 0xffffu);
+  return (uint32_t)((over | over >> 16 | over >> 32 | over >> 48) & 0xffffu);
 }
 
-template <typename TC, int WM, int WAVES>
+// A block makes the parts of PARTS_STEPS steps of a row tile, each of its four wavefronts of two.  (A wavefront that took eight steps one after the
+// other waited for its loads eight times: 4,096 x 256 10.7 us.)
+__global__ void __launch_bounds__(256) f32_parts_kernel(const float* __restrict__ A, long lda, int M, int steps, uint4* __restrict__ parts, uint32_t* __restrict__ flags,
+                                                        int groups) {
+  constexpr int EACH = PARTS_STEPS / 4;
+  __shared__ uint32_t beyond[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, j = lane >> 4;
+  const int tile = blockIdx.x, first = blockIdx.y * PARTS_STEPS + wave * EACH;
+  const int m = tile * 16 + r;
+  const float* src = A + (size_t)min(m, M - 1) * lda + 8 * j;
+  float4v x[EACH], y[EACH];
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    const float* from = src + 32 * min(first + i, steps - 1);
+    x[i] = *(const float4v*)from, y[i] = *(const float4v*)(from + 4);
+  }
+  float largest = 0.f;
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    const int s = first + i;
+    if (s >= steps) break;
+    uint4 part[3];
+    largest = fmaxf(largest, take_eight_apart(x[i], y[i], s, m < M, part));
+#pragma unroll
+    for (int p = 0; p < 3; ++p) parts[(((size_t)tile * steps + s) * 3 + p) * 64 + lane] = part[p];
+  }
+  const uint32_t over = rows_beyond(largest);
+  if (lane == 0) beyond[wave] = over;
+  __syncthreads();
+  if (threadIdx.x == 0) flags[(size_t)tile * groups + blockIdx.y] = beyond[0] | beyond[1] | beyond[2] | beyond[3];
+}
+
+// ALONE: not 0: a K of up to so many steps, all of which fit the LDS, in one launch: a block makes the parts of its rows of A itself.  Bound by a
+// launch and one trip to memory.  A kernel that took both operands apart, two launches, this, us: 4 rows of 1,024 x 32 4.6, 5.7, 3.7; of 2,048 x
+// 64 5.3, 6.2, 4.0; of 512 x 256 9.1, 8.6, 7.0; 300 rows of 2,048 x 64 10.9, 8.2, 5.6.  And no scratch memory, and less of the host's time a call.
+#define ALONE_STEPS 8
+template <typename TC, int WM, int WAVES, int ALONE>
 __global__ void __launch_bounds__(64 * WAVES, 2)
 gemm_f32_parts_kernel(const unsigned char* __restrict__ parts, PartRows marks, const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw,
                       TC* __restrict__ C, long ldc, const void* __restrict__ bias, int bias_dtype, int M, int N, int K, int row_blocks, int total) {
   constexpr int BM = 16 * WM, BN = 16 * WAVES;
   constexpr int A_STAGE = WM * 3 * 1024, W_STAGE = BN * 128;
   // steps of A under way or in use, and of W
-  constexpr int SA = 4 * A_STAGE + 6 * W_STAGE <= 160 * 1024 ? 4 : 3 * A_STAGE + 5 * W_STAGE <= 160 * 1024 ? 3 : 2, SW = SA + 2;
+  constexpr int SA = ALONE ? ALONE : 4 * A_STAGE + 6 * W_STAGE <= 160 * 1024 ? 4 : 3 * A_STAGE + 5 * W_STAGE <= 160 * 1024 ? 3 : 2;
+  constexpr int SW = ALONE ? SA : SA + 2;
   constexpr int NA = (WM * 3 + WAVES - 1) / WAVES, NW = W_STAGE / 1024 / WAVES;  // a wavefront's loads a step
   static_assert(SA * A_STAGE + SW * W_STAGE <= 160 * 1024, "the steps fit the LDS");
   static_assert(WM % 2 == 0, "row tiles go in pairs");
+  static_assert(!ALONE || WAVES % WM == 0, "a wavefront makes the parts of one row tile");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[SA * A_STAGE + SW * W_STAGE];
   const int run = (total + 7) >> 3, at = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= run || at >= total) return;
@@ -295,20 +327,39 @@ gemm_f32_parts_kernel(const unsigned char* __restrict__ parts, PartRows marks, c
   float4v acc[WM];
 #pragma unroll
   for (int a = 0; a < WM; ++a) acc[a] = (float4v){0.f, 0.f, 0.f, 0.f};
-  // the loads in the order in which the waits below count them: step s of A with step s + 2 of W
+  __shared__ uint32_t beyond[ALONE ? WAVES : 1];  // of the row tile whose parts a wavefront made
+  if constexpr (ALONE) {
+    for (int s = 0; s < steps; ++s)
 #pragma unroll
-  for (int s = 0; s < 2; ++s)
+      for (int i = 0; i < NW; ++i) load_w(i, s, s);
+    const int tile = wave % WM, m = m0 + tile * 16 + r;
+    const float* src = A + (size_t)min(m, M - 1) * lda + 8 * j;
+    float most = 0.f;
+    for (int s = wave / WM; s < steps; s += WAVES / WM) {
+      uint4 part[3];
+      most = fmaxf(most, take_eight_apart(*(const float4v*)(src + 32 * s), *(const float4v*)(src + 32 * s + 4), s, m < M, part));
 #pragma unroll
-    for (int i = 0; i < NW; ++i) load_w(i, min(s, last), s);
+      for (int p = 0; p < 3; ++p) *(uint4*)(lds + s * A_STAGE + (tile * 3 + p) * 1024 + lane * 16) = part[p];
+    }
+    const uint32_t over = rows_beyond(most);
+    if (lane == 0) beyond[wave] = over;
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+  } else {
+    // the loads in the order in which the waits below count them: step s of A with step s + 2 of W
 #pragma unroll
-  for (int s = 0; s < SA - 1; ++s) {
+    for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int i = 0; i < NA; ++i) load_a(i, min(s, last), s);
+      for (int i = 0; i < NW; ++i) load_w(i, min(s, last), s);
 #pragma unroll
-    for (int i = 0; i < NW; ++i) load_w(i, min(s + 2, last), s + 2);
+    for (int s = 0; s < SA - 1; ++s) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) load_a(i, min(s, last), s);
+#pragma unroll
+      for (int i = 0; i < NW; ++i) load_w(i, min(s + 2, last), s + 2);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(NW + (SA - 2) * (NA + NW)) : "memory");
   }
   Frag8 fw[3], fn[3];
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(NW + (SA - 2) * (NA + NW)) : "memory");
   {
     float4v x, y;
     raw(0, x, y);
@@ -319,9 +370,10 @@ gemm_f32_parts_kernel(const unsigned char* __restrict__ parts, PartRows marks, c
   for (int k = 0; k < steps; ++k) {
     // this wavefront's loads of this step of A and the next of W have landed and it has left the step before; after the barrier
     // so has everyone
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(NW + (SA - 2) * (NA + NW)) : "memory");
+    if constexpr (!ALONE) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(NW + (SA - 2) * (NA + NW)) : "memory");
     __builtin_amdgcn_sched_barrier(0);
-    const int a_free = a_buf == 0 ? SA - 1 : a_buf - 1, w_free = w_buf == 0 ? SW - 1 : w_buf - 1, w_next = w_buf + 1 == SW ? 0 : w_buf + 1;
+    const int a_free = a_buf == 0 ? SA - 1 : a_buf - 1, w_free = w_buf == 0 ? SW - 1 : w_buf - 1;
+    const int w_next = ALONE ? min(k + 1, last) : w_buf + 1 == SW ? 0 : w_buf + 1;
     if (k % (2 * SPLIT_TURN) == SPLIT_TURN) {
       sign = -sign;
 #pragma unroll
@@ -354,7 +406,7 @@ gemm_f32_parts_kernel(const unsigned char* __restrict__ parts, PartRows marks, c
       // the loads of a step to come, a few after each pair
 #pragma unroll
       for (int i = 0; i < NA + NW; ++i) {
-        if (i * (WM / 2) / (NA + NW) != p) continue;
+        if (ALONE || i * (WM / 2) / (NA + NW) != p) continue;
         if (i < NA)
           load_a(i, min(k + SA - 1, last), a_free);
         else
@@ -382,7 +434,10 @@ gemm_f32_parts_kernel(const unsigned char* __restrict__ parts, PartRows marks, c
   for (int t = 0; t < (WM + WAVES - 1) / WAVES; ++t) {
     const int tile = wave + WAVES * t;
     uint32_t f = 0;
-    if (tile < WM && m0 / 16 + tile < row_tiles)
+    if constexpr (ALONE) {
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) f |= w % WM == tile ? beyond[w] : 0u;
+    } else if (tile < WM && m0 / 16 + tile < row_tiles)
       for (int g = lane; g < marks.groups; g += 64) f |= marks.flags[(size_t)(m0 / 16 + tile) * marks.groups + g];
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) f |= __shfl_xor(f, off, CWM_WAVE);
@@ -477,6 +532,8 @@ struct PartsBlock {
 };
 static const PartsBlock parts_blocks[] = {{16, 8, 2.05f}, {12, 8, 1.62f}, {10, 8, 1.44f}, {8, 8, 1.19f}, {6, 8, 1.03f}, {4, 8, 0.80f}, {2, 4, 0.44f}};
 #define PARTS_BLOCKS 7
+#define PARTS_ALONE -2  // the number that asks for the product in one launch (32 rows and 64 columns a block)
+#define PARTS_ALONE_SHORT -3
 static int parts_block(int M, int N) {
   int best = 0;
   float least = 0.f;
@@ -489,7 +546,7 @@ static int parts_block(int M, int N) {
   return best;
 }
 // float32 A and W, K a multiple of 32.  `scratch`: for every started 16 rows 3,072 bytes a step of 32 k and 4 every 256 k, 16-byte
-// aligned.  `block`: -1, or the number of one of the list above (tests).
+// aligned; none with PARTS_ALONE.  `block`: -1, PARTS_ALONE, or the number of one of the list above (tests).
 extern "C" int cwm_gemm_f32_parts(const void* A, long lda, const void* W, long ldw, void* C, int c_dtype, long ldc, const void* bias, int bias_dtype, int M, int N,
                                   int K, void* scratch, int block, hipStream_t stream) {
   CWM_REQUIRE(M > 0 && N > 0 && K > 0 && K % SPLIT_STEP == 0 && K <= SPLIT_MOST_K, "gemm_f32_parts: bad sizes M=%d N=%d K=%d", M, N, K);
@@ -500,27 +557,32 @@ extern "C" int cwm_gemm_f32_parts(const void* A, long lda, const void* W, long l
   const int row_tiles = (M + 15) / 16, steps = K / SPLIT_STEP, groups = (steps + PARTS_STEPS - 1) / PARTS_STEPS;
   unsigned char* parts = (unsigned char*)scratch;
   uint32_t* flags = (uint32_t*)(parts + (size_t)row_tiles * steps * 3072);
-  hipLaunchKernelGGL(f32_parts_kernel, dim3((unsigned)row_tiles, (unsigned)((groups + 3) / 4)), dim3(256), 0, stream, (const float*)A, lda, M, steps, (uint4*)parts, flags, groups);
+  CWM_REQUIRE(block == PARTS_ALONE ? steps <= ALONE_STEPS : scratch != nullptr && block >= -1, "gemm_f32_parts: K=%d takes two launches and scratch memory", K);
+  if (block != PARTS_ALONE)
+    hipLaunchKernelGGL(f32_parts_kernel, dim3((unsigned)row_tiles, (unsigned)groups), dim3(256), 0, stream, (const float*)A, lda, M, steps, (uint4*)parts, flags, groups);
   const PartRows marks = {flags, groups};
-  if (block < 0) block = parts_block(M, N);
-#define CWM_PARTS(AT, WM, WAVES)                                                                                                          \
-  case AT: {                                                                                                                             \
-    const int row_blocks = (M + 16 * WM - 1) / (16 * WM), total = row_blocks * ((N + 16 * WAVES - 1) / (16 * WAVES));                     \
-    if (c_dtype == CWM_F32)                                                                                                              \
-      hipLaunchKernelGGL((gemm_f32_parts_kernel<float, WM, WAVES>), dim3((total + 7) / 8 * 8), dim3(64 * WAVES), 0, stream, parts, marks,  \
-                         (const float*)A, lda, (const float*)W, ldw, (float*)C, ldc, bias, bias_dtype, M, N, K, row_blocks, total);        \
-    else                                                                                                                                 \
-      hipLaunchKernelGGL((gemm_f32_parts_kernel<bf16_t, WM, WAVES>), dim3((total + 7) / 8 * 8), dim3(64 * WAVES), 0, stream, parts, marks, \
-                         (const float*)A, lda, (const float*)W, ldw, (bf16_t*)C, ldc, bias, bias_dtype, M, N, K, row_blocks, total);       \
+  if (block == -1) block = parts_block(M, N);
+  if (block == PARTS_ALONE && steps <= ALONE_STEPS / 2) block = PARTS_ALONE_SHORT;  // two blocks a compute unit
+#define CWM_PARTS(AT, WM, WAVES, ALONE)                                                                                                           \
+  case AT: {                                                                                                                                      \
+    const int row_blocks = (M + 16 * WM - 1) / (16 * WM), total = row_blocks * ((N + 16 * WAVES - 1) / (16 * WAVES));                             \
+    if (c_dtype == CWM_F32)                                                                                                                       \
+      hipLaunchKernelGGL((gemm_f32_parts_kernel<float, WM, WAVES, ALONE>), dim3((total + 7) / 8 * 8), dim3(64 * WAVES), 0, stream, parts, marks,  \
+                         (const float*)A, lda, (const float*)W, ldw, (float*)C, ldc, bias, bias_dtype, M, N, K, row_blocks, total);               \
+    else                                                                                                                                          \
+      hipLaunchKernelGGL((gemm_f32_parts_kernel<bf16_t, WM, WAVES, ALONE>), dim3((total + 7) / 8 * 8), dim3(64 * WAVES), 0, stream, parts, marks, \
+                         (const float*)A, lda, (const float*)W, ldw, (bf16_t*)C, ldc, bias, bias_dtype, M, N, K, row_blocks, total);              \
   } break;
   switch (block) {
-    CWM_PARTS(0, 16, 8)
-    CWM_PARTS(1, 12, 8)
-    CWM_PARTS(2, 10, 8)
-    CWM_PARTS(3, 8, 8)
-    CWM_PARTS(4, 6, 8)
-    CWM_PARTS(5, 4, 8)
-    CWM_PARTS(6, 2, 4)
+    CWM_PARTS(0, 16, 8, 0)
+    CWM_PARTS(1, 12, 8, 0)
+    CWM_PARTS(2, 10, 8, 0)
+    CWM_PARTS(3, 8, 8, 0)
+    CWM_PARTS(4, 6, 8, 0)
+    CWM_PARTS(5, 4, 8, 0)
+    CWM_PARTS(6, 2, 4, 0)
+    CWM_PARTS(PARTS_ALONE, 2, 4, ALONE_STEPS)
+    CWM_PARTS(PARTS_ALONE_SHORT, 2, 4, ALONE_STEPS / 2)
     default: return cwm_fail("gemm_f32_parts: no block %d", block);
   }
 #undef CWM_PARTS

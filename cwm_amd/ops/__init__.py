@@ -216,7 +216,7 @@ def gemm_f32(
     if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
         raise KernelError(f"gemm: x {tuple(x.shape)} and weight {tuple(weight.shape)} do not fit")
     if _f32_parts_takes(x, weight):  # whatever the number of rows: a row's result does not depend on the others
-        return gemm_f32_parts(x, weight, bias, out_dtype)
+        return _f32_parts(x, weight, bias, out_dtype, -2 if _f32_parts_alone(x.shape[0], weight.shape[0], x.shape[1]) else -1)
     _rows_contiguous(x, "gemm x")
     _rows_contiguous(weight, "gemm weight")
     m, k = x.shape
@@ -247,13 +247,18 @@ def gemm_f32_parts(
 ) -> torch.Tensor:
     """The product of `gemm_f32` where both operands are float32, K is a multiple of 32 up to 65,536 and rows are 16-byte aligned:
     every value in three exact bfloat16 parts, six of their nine products on the matrix cores.  x's parts are made by a kernel of
-    their own, into scratch memory of 6 bytes a value.  `block` (tests): the number of a block of the kernel's list."""
+    their own, into scratch memory of 6 bytes a value.  `block` (tests): the number of a block of the kernel's list, or -2 for one
+    launch without scratch memory (K up to 256)."""
     _need_gpu(x, weight, bias)
     if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] or not _f32_parts_takes(x, weight):
         raise KernelError(
             "the float32 product in parts takes float32 x [M, K] and weight [N, K] with K a multiple of 32 and 16-byte aligned rows; "
             f"got {tuple(x.shape)} {x.dtype} and {tuple(weight.shape)} {weight.dtype}"
         )
+    return _f32_parts(x, weight, bias, out_dtype, -1 if block is None else block)
+
+
+def _f32_parts(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out_dtype: Optional[torch.dtype], block: int) -> torch.Tensor:
     m, k = x.shape
     n = weight.shape[0]
     if bias is not None and (bias.shape != (n,) or not bias.is_contiguous()):
@@ -262,24 +267,37 @@ def gemm_f32_parts(
         weight = weight.contiguous()
     lib = _build.load("gemm_f32")
     out = torch.empty((m, n), dtype=out_dtype or x.dtype, device=x.device)
-    scratch = torch.empty(-(-m // 16) * (k // 32 * 3072 + -(-k // 256) * 4), dtype=torch.uint8, device=x.device)
+    scratch = None if block == -2 else torch.empty(-(-m // 16) * (k // 32 * 3072 + -(-k // 256) * 4), dtype=torch.uint8, device=x.device)
     _check(
         lib,
         lib.cwm_gemm_f32_parts(
             _ptr(x), ctypes.c_long(x.stride(0) if m > 1 else k), _ptr(weight), ctypes.c_long(weight.stride(0) if n > 1 else k), _ptr(out),
             ctypes.c_int(_code(out.dtype)), ctypes.c_long(n), _ptr(bias), ctypes.c_int(_code(bias.dtype) if bias is not None else F32),
-            ctypes.c_int(m), ctypes.c_int(n), ctypes.c_int(k), _ptr(scratch), ctypes.c_int(-1 if block is None else block), _stream(),
+            ctypes.c_int(m), ctypes.c_int(n), ctypes.c_int(k), _ptr(scratch), ctypes.c_int(block), _stream(),
         ),
     )
     return out
 
 
+F32_ALONE_K = 256  # csrc/gemm_f32.hip: ALONE_STEPS
+# Blocks of 32 rows and 64 columns up to which it pays that each makes its rows' parts again; of a K above half of that, whose blocks do not
+# share a compute unit, a quarter.  Two launches / one, us: K = 64, 1,024 blocks 11.0 / 10.2, 2,048 17.6 / 17.7; K = 128, 512 blocks 11.3 / 8.0, 1,024
+# 12.2 to 15.5 / 13.1 to 13.5, 2,048 23.1 / 22.9; K = 256, 256 blocks 13.0 / 9.1, 384 12.6 / 14.7, 512 15.7 / 16.1, 1,024 16.4 / 28.2.
+F32_ALONE_BLOCKS = 1024
+
+
+def _f32_parts_alone(m: int, n: int, k: int) -> bool:
+    """Whether a product in parts is one launch, whose blocks make the parts of their rows of x themselves."""
+    return k <= F32_ALONE_K and -(-m // 32) * -(-n // 64) <= (F32_ALONE_BLOCKS if 2 * k <= F32_ALONE_K else F32_ALONE_BLOCKS // 4)
+
+
 def _f32_parts_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    if x.dtype != torch.float32 or weight.dtype != torch.float32:
+        return False
+    (m, k), (x_row, x_one), (w_row, w_one) = x.shape, x.stride(), weight.stride()
     return (
-        x.dtype == torch.float32 and weight.dtype == torch.float32
-        and x.shape[0] > 0 and x.shape[1] % 32 == 0 and 0 < x.shape[1] <= 65536 and x.stride(-1) == 1 and weight.stride(-1) == 1
-        and (x.shape[0] <= 1 or x.stride(0) % 4 == 0) and (weight.shape[0] <= 1 or weight.stride(0) % 4 == 0)
-        and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+        m > 0 and k % 32 == 0 and 0 < k <= 65536 and x_one == 1 and w_one == 1
+        and (m <= 1 or x_row % 4 == 0) and (weight.shape[0] <= 1 or w_row % 4 == 0) and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
     )
 
 

@@ -54,3 +54,28 @@ def test_weights_whose_rows_lie_far_apart(rows):
     far.copy_(torch.randn(rows, 96, device=DEV))
     assert ops._f32_parts_takes(x, far)
     assert torch.equal(ops.gemm_f32(x, far), ops.gemm_f32(x, far.contiguous()))
+
+
+# one to eight steps of K, of which half fit the shorter of two forms; rows at the edges of the 32 of a block and of a tile of 16, columns at the edges of 64; operands whose rows lie apart
+@pytest.mark.parametrize("m", [1, 15, 17, 32, 33, 100])
+@pytest.mark.parametrize("n,k,pad", [(1, 32, 0), (64, 64, 4), (70, 96, 0), (200, 128, 8), (64, 160, 0), (130, 256, 4)])
+def test_one_launch_gives_the_same_bits(m, n, k, pad):
+    gen = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k + pad, generator=gen).to(DEV)[:, :k]
+    w = torch.randn(n, k + pad, generator=gen).to(DEV)[:, :k]
+    b = torch.randn(n, generator=gen).to(DEV)
+    assert torch.equal(ops.gemm_f32_parts(x, w, b, block=-2), ops.gemm_f32_parts(x, w, b))
+    assert torch.equal(ops.gemm_f32_parts(x, w, None, torch.bfloat16, block=-2), ops.gemm_f32_parts(x, w, None, torch.bfloat16))
+    # values beyond the parts, in rows and steps that different wavefronts take apart; a NaN, which stays in its row and column
+    for row, column, value in ((m - 1, k - 1, 1e20), (m // 2, 3, float("inf")), (0, k // 2, float("nan"))):
+        far_x, far_w = x.clone(), w.clone()
+        far_x[row, column] = far_w[n // 3, k - 1 - column] = value
+        got, want = (ops.gemm_f32_parts(far_x, far_w, b, block=block) for block in (-2, 0))
+        assert torch.equal(got.nan_to_num(3.0), want.nan_to_num(3.0)) and torch.equal(got.isnan(), want.isnan())
+
+
+def test_what_one_launch_refuses():
+    x, w = torch.randn(40, 288, device=DEV), torch.randn(50, 288, device=DEV)
+    for block in (-2, -3, -4):
+        with pytest.raises(ops.KernelError):
+            ops.gemm_f32_parts(x, w, block=block)
