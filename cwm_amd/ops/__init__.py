@@ -863,6 +863,14 @@ def _prefers_wide(x: torch.Tensor, weight: torch.Tensor, glu: bool = False) -> b
     return bool(_build.load("gemm_bf16_wide").cwm_gemm_bf16_wide_pays(x.shape[0], weight.shape[0], x.shape[1], _compute_units(x.device), int(glu)))
 
 
+def _wide_keeps_sums(m: int, n: int, k: int) -> bool:
+    """Whether the wide kernel's float32 sums are no further from the exact ones than the library's.  Both add K in its order, with the same bits, but
+    where few or very many tiles make the library cut K, and its sums are then shorter: float32 results off float64, library / wide, 130 x 512 x 2,048
+    1.3e-7 / 2.7e-7, 2,048 x 10,304 x 6,144 4.3e-7 / 4.9e-7, 600 x 1,024 x 21,504 5.9e-7 / 9.4e-7.  Of 2,162 sizes with a K of 512 to 28,672 none in these
+    bounds is.  A bfloat16 result does not show it: rounded, the errors differ by a millionth of themselves."""
+    return k <= 1024 or (k <= 2048 and (1 << 17) < m * n <= (1 << 26))
+
+
 def gemm_bf16_wide(
     x: torch.Tensor, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None, glu: bool = False, units: Optional[int] = None,
     tile: Optional[int] = None,
@@ -931,7 +939,7 @@ def gemm_bf16(
         return gemm_bf16_tile(x, weight, None, out_dtype, partials_ok)
     if m <= STREAM_MAX_ROWS:
         return gemm_bf16_stream(x, weight, bias, out_dtype, partials_ok, streamed=streamed, keep_sums=bias is None and m > STREAM_FUSED_ROWS)
-    if bias is None and _prefers_wide(x, weight):
+    if bias is None and (out_dtype != torch.float32 or _wide_keeps_sums(m, *weight.shape)) and _prefers_wide(x, weight):
         return gemm_bf16_wide(x, weight, out_dtype)
     if out_dtype == torch.float32:
         y = torch.mm(x, weight.t(), out_dtype=torch.float32)  # bfloat16 operands, float32 sums written as they are

@@ -54,3 +54,21 @@ def test_few_rows_that_overlap_are_refused(rows):
     for a, b in _overlapping(x, w):
         with pytest.raises(ops.KernelError):
             ops.gemm_bf16(a[:rows], b)
+
+
+def test_float32_results_of_a_long_k_are_not_the_wide_kernels():
+    assert ops._wide_keeps_sums(1500, 4096, 1024) and ops._wide_keeps_sums(1500, 4096, 2048)
+    for m, n, k in ((130, 512, 2048), (2652, 28672, 2048), (1500, 4096, 2112), (600, 1024, 21504)):
+        assert not ops._wide_keeps_sums(m, n, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(600, 1024, 21504), (777, 4096, 6144), (1040, 2048, 512)])
+def test_float32_results_are_as_near_as_the_librarys(m, n, k):
+    gen = torch.Generator().manual_seed(m)
+    x, w = torch.randn(m, k, generator=gen).bfloat16().to("cuda:0"), (torch.randn(n, k, generator=gen) * k**-0.5).bfloat16().to("cuda:0")
+    assert ops._prefers_wide(x, w)
+    exact = x.double() @ w.double().t()
+    off = lambda y: ((y.double() - exact).norm() / exact.norm()).item()  # noqa: E731
+    # the same sums, or the library's own; a different order of terms of equal length would differ by about a fiftieth
+    assert off(ops.gemm_bf16(x, w, out_dtype=torch.float32)) <= 1.02 * off(torch.mm(x, w.t(), out_dtype=torch.float32))
