@@ -866,7 +866,7 @@ def _prefers_wide(x: torch.Tensor, weight: torch.Tensor, glu: bool = False) -> b
 def _wide_keeps_sums(m: int, n: int, k: int) -> bool:
     """Whether the wide kernel's float32 sums are no further from the exact ones than the library's.  Both add K in its order, with the same bits, but
     where few or very many tiles make the library cut K, and its sums are then shorter: float32 results off float64, library / wide, 130 x 512 x 2,048
-    1.3e-7 / 2.7e-7, 2,048 x 10,304 x 6,144 4.3e-7 / 4.9e-7, 600 x 1,024 x 21,504 5.9e-7 / 9.4e-7.  Of 2,162 sizes with a K of 512 to 28,672 none in these
+    1.3e-7 / 2.7e-7, 2,048 x 10,304 x 6,144 4.4e-7 / 5.0e-7, 600 x 1,024 x 21,504 5.9e-7 / 9.4e-7.  Of 2,162 sizes with a K of 512 to 28,672 none in these
     bounds is.  A bfloat16 result does not show it: rounded, the errors differ by a millionth of themselves."""
     return k <= 1024 or (k <= 2048 and (1 << 17) < m * n <= (1 << 26))
 
