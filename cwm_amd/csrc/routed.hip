@@ -961,7 +961,8 @@ __global__ void __launch_bounds__(256, 2) grouped_wide_kernel(const bf16_t* __re
 // round, goes in quarters, 64 rows by 128 columns, over all blocks.  The sums' order is that of the kernel above, and so are the bits.
 // 16 experts of 2,048 x 1,024, four a token, uneven loads, the kernel above / this, gate and up, then down, us: 2,048 tokens 111 / 92 and 59 / 51,
 // 700 50 / 43 and 25 / 25, 4,096 161 / 153 and 101 / 95; 32 of 3,072 x 1,536, 1,000 tokens 174 / 156 and 105 / 90; 8 of 512 x 320, 300 tokens
-// 14.0 / 8.6 and 8.3 / 6.5; but 1,500 tokens, whose second round is two thirds full, 72 / 75 and 40 / 41: the caller's rule leaves such to it.
+// 14.0 / 8.6 and 8.3 / 6.5; but 1,500 tokens, whose second round is two thirds full, 72 / 75 and 40 / 41:
+// the caller's rule (`_loop_pays`) leaves such, and others that were not ahead, to it.
 #define GROUPED_BLOCKS 256
 typedef const __attribute__((address_space(4))) int* list_ints;  // read by scalar loads, which do not wait for the loads under way
 

@@ -109,12 +109,20 @@ def _product_tiles(dtype: torch.dtype, k: int, rows: float, gated: bool) -> int:
 LOOP_BLOCKS = 256  # csrc/routed.hip: GROUPED_BLOCKS
 
 
-def _loop_pays(pairs: int, n_experts: int, columns: int, gated: bool) -> bool:
+def _loop_pays(pairs: int, n_experts: int, columns: int, k: int, gated: bool) -> bool:
     """Whether a product of many rows an expert goes to the persistent blocks, which take tiles of 128 rows and 256 columns of
-    weights in rounds: not where the second round would be between a third and five sixths full, as the rows and half a tile of
-    padding an expert make expect (us, 1.5 and 1.7 rounds 74 and 75, the other kernel 73 and 72; 1.2 56 and 63; 2.0 77 and 97; 2.2 92 and 111)."""
+    weights in rounds, and what is left below half a round in quarters.  The rounds are those that the rows and half a tile of padding an
+    expert make expect.  One round of quarters is always ahead (the other kernel / this, us, weights not in a cache: 4 experts of
+    2,048 x 2,048, 203 tokens, gates and ups then without, 34 / 22 and 29 / 19).  Two of them are ahead with gates and ups, and not without (16 of
+    2,048 x 1,024, 262 tokens, evenly spread 36 / 36 and 20 / 24, unevenly 48 / 41 and 27 / 26; 8 of 1,024 x 1,024, 0.4 rounds, 18.2 / 19.6).  Whole
+    tiles take a round to its end: ahead from two thirds of one up to 1.25 and from 1.9 on, in between or not (4 of 2,048 x 2,048, 1.4
+    rounds 59 / 66, 1.6 68 / 67).  A short K has too little to do between a tile's sums (8 of 512 x 320, 1.1 rounds 18 / 24), and
+    after four rounds the other kernel's last one weighs no more (64 of 2,048 x 768 with gates and ups, 2,600 tokens 168 / 169, 8,195 408 / 435).  Of 1,300 products of 13 shapes and 48 to 4,096 rows an expert, evenly and unevenly spread, this
+    takes 556, 1.12 times as fast in the mean and 33 slower by more than 3% (evenly spread rows that end with their tiles, mostly)."""
     rounds = (pairs / 128 + n_experts / 2) * -(-columns // (128 if gated else 256)) / LOOP_BLOCKS
-    return not 1.35 < rounds < 1.85
+    if rounds <= 0.25:
+        return True
+    return k >= (1536 if gated else 640) and ((gated or rounds > 0.65) and rounds <= 1.25 or 1.9 < rounds <= 4.2)
 
 
 def _empty_groups(n: int, top: int, n_experts: int, device: torch.device) -> ExpertGroups:
@@ -300,7 +308,7 @@ def _grouped(
             ctypes.c_int(groups.tiles_a_block if groups is not None else 1),
             ctypes.c_int(activation.code() if activation is not None else 0), ctypes.c_float(activation.alpha if activation is not None else 1.0),
             ctypes.c_float(activation.limit if activation is not None else 0.0), ctypes.c_int(int(tiled)),
-            ctypes.c_int(int(groups is not None and _loop_pays(groups.pair_row.numel(), e, n, w1 is not None))), _stream(),
+            ctypes.c_int(int(groups is not None and _loop_pays(groups.pair_row.numel(), e, n, k, w1 is not None))), _stream(),
         ),
     )
 
