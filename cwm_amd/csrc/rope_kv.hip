@@ -579,8 +579,7 @@ struct ValueRuns {
 // and 47.8; one token of 32 and 8 heads 4.2 and 5.1.
 // RUNS: whole value blocks (`ValueRuns`) instead of the two-byte writes that bounded it, us at 512, 2,296 and 8,192 tokens: 16 and 4
 // heads of 128 7.1, 14.4, 38.6 to 6.0, 12.4, 34.2; 32 and 8 10.4, 26.0, 65.7 to 8.8, 20.9, 52.5; 16 and 16 of 64 7.9, 19.3, 53.4 to 5.9,
-// 11.7, 32.1; 8 and 1 of 256 6.7, 12.5, 31.4 to 6.1, 12.2, 33.5, so an eighth of the queries' heads stays with narrow writes.  (A head's
-// elements asked for a head ahead: 32 and 8 heads 21.6 and 57.4.)
+// 11.7, 32.1 (`cwm_value_runs_pay`: where not).  (A head's elements asked for a head ahead: 32 and 8 heads 21.6 and 57.4.)
 template <typename TS, typename TO, bool VEC, bool RUNS>
 __global__ void __launch_bounds__(256)
 head_norm_rope_write_kernel(const TS* __restrict__ src, long src_stride, int n_partials, long partial_stride,
@@ -785,6 +784,15 @@ head_norm_rope_write_kernel(const TS* __restrict__ src, long src_stride, int n_p
   }
 }
 
+// Whether a step of `n_seqs` sequences writes whole value blocks: finding them costs every block a little (up to a fifth of the time of a step
+// that has none), so only where one block takes a token, sequences have tokens in a row, and values are enough of the work.  Narrow writes /
+// whole blocks, us, 16 and 4 heads of 128: 2,048 tokens of 2,048 sequences 17.3 / 20.1, of 186 14.1 / 15.5, of 43 13.8 / 13.4, of one 13.4 / 12.3;
+// 32 and 8: 26.9 / 29.5, 23.0 / 24.2, 22.8 / 20.5, 23.8 / 20.2.  Heads, one sequence of 8,192: 8 and 2 of 128 25.1 / 27.0, 2 and 1 of 64 16.3 / 17.6,
+// 12 and 3 of 128 29.8 / 31.0, 28 and 4 44.1 / 45.0, but 40 and 8 69.7 / 59.2, 8 and 8 of 64 31.0 / 23.9.
+extern "C" int cwm_value_runs_pay(int n_tokens, int n_seqs, int n_q_heads, int n_kv_heads, int head_dim) {
+  return n_tokens >= 512 && n_tokens >= 64l * n_seqs && n_kv_heads * head_dim >= 512 && n_q_heads <= 5 * n_kv_heads;
+}
+
 // src: [n_tokens][src_stride] of src_dtype (the row may go on beyond q, k and v), or n_partials float32 slabs
 // partial_stride apart.  bias: float32 [(Hq + Hkv) * qk_dim + Hkv * v_dim] or null.  q_weight, k_weight: float32
 // [qk_dim] or null.  inv_freq: float32 [head_dim / 2] or null.  v_other ([n_tokens][v_other_stride], the cache's type)
@@ -793,7 +801,7 @@ head_norm_rope_write_kernel(const TS* __restrict__ src, long src_stride, int n_p
 extern "C" int cwm_head_norm_rope_write(const void* src, int src_dtype, long src_stride, int n_partials, long partial_stride,
                                         const float* bias, void* q_out, int out_dtype, const float* q_weight, const float* k_weight,
                                         float eps, const int* positions, const int* seq_of_token, const float* inv_freq, void* cache,
-                                        const int* block_table, int table_width, int page_size, int num_pages, int n_tokens,
+                                        const int* block_table, int table_width, int n_seqs, int page_size, int num_pages, int n_tokens,
                                         int n_q_heads, int n_kv_heads, int qk_dim, int v_dim, int head_dim, const void* v_other,
                                         long v_other_stride, const float* v_mix, void* v_keep, float temp_coef, int temp_every,
                                         hipStream_t stream) {
@@ -824,8 +832,8 @@ extern "C" int cwm_head_norm_rope_write(const void* src, int src_dtype, long src
   const bool vec = head_dim % 4 == 0 && quarter <= CWM_WAVE && (quarter & (quarter - 1)) == 0 && qk_dim % 4 == 0 && v_dim % 4 == 0 && src_stride % 4 == 0 &&
                    partial_stride % 4 == 0 && v_other_stride % 4 == 0 && aligned(src, src_dtype) && aligned(q_out, out_dtype) && aligned(cache, out_dtype) &&
                    aligned(v_other, out_dtype) && aligned(v_keep, out_dtype) && (((uintptr_t)bias | (uintptr_t)q_weight | (uintptr_t)k_weight) % 16) == 0;
-  // whole value blocks where a block takes a token and the values are enough of the work (times above)
-  const bool runs = vec && gy == 1 && cache && 8 * n_kv_heads > n_q_heads && out_dtype == CWM_BF16 && page_size % 8 == 0 && (uintptr_t)cache % 16 == 0;
+  const bool runs = vec && cache && cwm_value_runs_pay(n_tokens, n_seqs, n_q_heads, n_kv_heads, head_dim) && out_dtype == CWM_BF16 &&
+                    page_size % 8 == 0 && (uintptr_t)cache % 16 == 0;
 #define CWM_HEAD_NORM_ROPE(TS, TO)                                                                                         \
   do {                                                                                                                     \
     if (runs) CWM_HEAD_NORM_ROPE_V(TS, TO, true, sizeof(TO) == 2);                                                         \

@@ -288,7 +288,7 @@ def head_norm_rope_write(
     _i32(positions, "positions")
     if positions.numel() != n_tokens:
         raise KernelError("one position per token is needed")
-    page_size = num_pages = table_width = 0
+    page_size = num_pages = table_width = n_seqs = 0
     if cache is not None:
         if block_table is None or seq_of_token is None:
             raise KernelError("a cache write needs a block table and the sequence of each token")
@@ -300,7 +300,8 @@ def head_norm_rope_write(
         _i32(seq_of_token, "seq_of_token")
         if block_table.dim() != 2 or seq_of_token.numel() != n_tokens:
             raise KernelError("block_table must be [B, W] and seq_of_token [T]")
-        num_pages, page_size, table_width = cache.shape[0], cache.shape[3] // head_dim, block_table.shape[1]
+        num_pages, page_size = cache.shape[0], cache.shape[3] // head_dim
+        n_seqs, table_width = block_table.shape
     if temperature is not None and temperature[1] < 1:
         raise KernelError("the queries' temperature rises every so many positions, at least one")
     if (v_other is None) != (v_mix is None):
@@ -321,7 +322,7 @@ def head_norm_rope_write(
             _ptr(qkv), ctypes.c_int(_code(qkv.dtype)), ctypes.c_long(stride), ctypes.c_int(n_partials), ctypes.c_long(partial_stride),
             _ptr(bias), _ptr(q), ctypes.c_int(_code(out_dtype)), _ptr(q_weight), _ptr(k_weight), ctypes.c_float(eps),
             _ptr(positions), _ptr(seq_of_token), _ptr(inv_freq), _ptr(cache), _ptr(block_table),
-            ctypes.c_int(table_width), ctypes.c_int(page_size), ctypes.c_int(num_pages), ctypes.c_int(n_tokens),
+            ctypes.c_int(table_width), ctypes.c_int(n_seqs), ctypes.c_int(page_size), ctypes.c_int(num_pages), ctypes.c_int(n_tokens),
             ctypes.c_int(n_q_heads), ctypes.c_int(n_kv_heads), ctypes.c_int(qk_dim), ctypes.c_int(v_dim), ctypes.c_int(head_dim),
             _ptr(v_other), ctypes.c_long(other_stride), _ptr(v_mix), _ptr(kept), ctypes.c_float(temperature[0] if temperature else 0.0),
             ctypes.c_int(temperature[1] if temperature else 0), _stream(),

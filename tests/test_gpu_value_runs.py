@@ -1,4 +1,5 @@
-"""Values of many tokens written a value block at a time: the bits of calls of few tokens, which write each token's own."""
+"""Values of many tokens written a value block at a time, where the heads are many enough: the bits of calls of few tokens, which write
+each token's own."""
 
 import pytest
 import torch
@@ -15,7 +16,8 @@ STEPS = [[(0, 512)], [(5, 523)], [(7, 1), (30, 1), (0, 300), (11, 1), (3, 221)],
 
 @pytest.mark.parametrize("step", STEPS)
 @pytest.mark.parametrize("page", [8, 24, 12])
-@pytest.mark.parametrize("n_kv,qk,vd,hd,kind", [(4, 128, 128, 128, "rows"), (1, 20, 12, 32, "mixed"), (3, 64, 64, 64, "partials"), (2, 4, 4, 4, "rows")])
+@pytest.mark.parametrize("n_kv,qk,vd,hd,kind", [(4, 128, 128, 128, "rows"), (1, 20, 12, 32, "mixed"), (3, 64, 64, 64, "partials"), (2, 4, 4, 4, "rows"),
+                                                  (16, 20, 12, 32, "mixed"), (8, 64, 64, 64, "partials"), (128, 4, 4, 4, "rows")])
 def test_the_bits_of_few_tokens(step, page, n_kv, qk, vd, hd, kind):
     n_q, total = 2, sum(n for _, n in step)
     g = torch.Generator(device=DEV).manual_seed(total + page + hd)
@@ -36,6 +38,8 @@ def test_the_bits_of_few_tokens(step, page, n_kv, qk, vd, hd, kind):
         return ops.head_norm_rope_write(rows, n_q, n_kv, qk, vd, hd, bias, weight, weight, 1e-5, positions[lo:hi], inv_freq, torch.bfloat16, cache, table, seq[lo:hi],
                                         v_other=None if other is None else other[lo:hi], v_mix=mix, keep_values=True)
 
+    lib = ops._build.load("rope_kv")
+    assert not lib.cwm_value_runs_pay(100, 1, n_q, n_kv, hd) and bool(lib.cwm_value_runs_pay(total, len(step), n_q, n_kv, hd)) == (n_kv * hd >= 512)
     caches = [torch.full((table.numel(), 2, n_kv, hd * page), 9.0, device=DEV, dtype=torch.bfloat16) for _ in range(2)]
     q, kept = run(caches[0], 0, total)
     parts = [run(caches[1], lo, min(lo + 100, total)) for lo in range(0, total, 100)]
