@@ -115,15 +115,21 @@ class GatedMLP(FeedForward):
         super().bind(tensors, runtime)
         matrices = [tensors[self.gate_name], tensors[self.up_name]]
         if self.row_gate is not None:
-            # with zeros up to whole groups of 16 rows: the products that share x and W through LDS take no others (2,049 columns of
+            # with zeros up to whole groups of 16 rows, which the wide product takes and no other number of columns (2,049 columns of
             # 2,048 at 1,500 rows: the library 23.2 us, 2,064 columns 19.0)
             row = tensors[self.row_gate]
             matrices += [row, row.new_zeros((-(2 * self.hidden_dim + 1) % 16, self.dim))]
-        self.gate_up = LinearWeights.joined(matrices, [None] * len(matrices), stream_copy=runtime.stream_copies)
+        self.gate_up = self.gate_up_wide = LinearWeights.joined(matrices, [None] * len(matrices), stream_copy=runtime.stream_copies)
+        if self.row_gate is not None:
+            # Up to as many rows as the tiled product takes, the columns there are: it would take 2,064 too, in more time than the streaming product
+            # or the library 2,049 (us, 2,049 / 2,064 columns: 129 rows 14.8 / 17.7, 256 16.1 / 21.3; 513 / 528 of 256: 33 rows 7.0 / 10.6).
+            streamed = self.gate_up.streamed
+            self.gate_up = self.gate_up.rows(0, 2 * self.hidden_dim + 1)
+            self.gate_up.streamed = streamed  # its tiles of 16 rows end in the same zeros
         self.down = LinearWeights(tensors[self.down_name], stream_copy=runtime.stream_copies)
 
     def forward(self, x: torch.Tensor, batch: Any) -> torch.Tensor:
-        joined = self.gate_up(x, partials_ok=True)
+        joined = (self.gate_up if x.shape[0] <= ops.TILE_TALL_ROWS else self.gate_up_wide)(x, partials_ok=True)
         hidden = ops.gated_act_rows(joined, self.hidden_dim, self.activation, x.dtype, 2 * self.hidden_dim if self.row_gate is not None else None)
         return self.down(hidden, partials_ok=True)
 
