@@ -1509,7 +1509,7 @@ from .sequence import (  # noqa: E402
 )
 from .routed import (  # noqa: E402
     MAX_EXPERTS, MAX_ROUTE_TOP, ExpertGroups, GatedActivation, absorb_queries, combine_routed, expand_values, expert_tiles, group_by_expert,
-    grouped_gate_up, grouped_linear, route_and_group, route_group_limits, route_group_pays, route_rows, route_top,
+    grouped_gate_up, grouped_linear, route_and_group, route_group_limits, route_group_pays, route_rows, route_rows_pays, route_top,
 )
 from .streams import (  # noqa: E402
     ACTIVATIONS, MAX_STREAMS, RoutedSum, act_rows, embedding_streams, head_norm_rope_write, qk_norm_rope_write, stream_mix_norm,

@@ -180,6 +180,14 @@ def _route_checks(x, router_copy, bias, n_experts, top, scores, correction, scal
     return n, k, count, keep
 
 
+def route_rows_pays(n_tokens: int, k: int) -> bool:
+    """Whether so many tokens' logits and choices are made faster in one launch than as a product and its choice.  The product reads x once
+    whatever the number of tokens; the one launch is ahead by what a launch costs, for 2 to 16 experts up to 4,096 tokens (us, product / one launch, 16
+    experts of 2,048: 17 tokens 8.6 / 6.0, 2,048 8.3 / 6.4) and with rows of up to 1,536 to 8,192; of 2,048 and more 6,000 tokens take 9.2 / 9.9 (2
+    experts) to 13.0 / 13.6 (16 of 3,072), 16,384 17 to 18.5 / 19 to 20 and 65,536 of 3,072 84 to 98 / 115 to 119."""
+    return n_tokens <= (8192 if k <= 1536 else 4096)
+
+
 def route_rows(
     x: torch.Tensor, router_copy: torch.Tensor, bias: Optional[torch.Tensor], n_experts: int, top: int, scores: str = "softmax_chosen",
     correction: Optional[torch.Tensor] = None, scale: float = 1.0, renormalize: bool = False, groups: Optional[Tuple[int, int]] = None,

@@ -111,9 +111,7 @@ class RoutedExperts(FeedForward):
         """The same without the last kernel: every pair's row and the weights, for a consumer that adds a token's
         rows up itself (a norm that takes a `RoutedSum` as the pending result)."""
         router = (self.top, self.scores, self.choice_correction, self.weight_scale, self.renormalize, self.groups)
-        # Short rows of very many tokens go as a product: 16 experts of 1,024, 8,192 tokens 9.4 us as a product and 9.0 in one
-        # launch, 16,384 13.8 and 15.5, 32,768 25.0 and 28.0; of 2,048, 16,384 tokens 19.9 and 18.1 (8 experts of 1,536 16.9 and 14.5).
-        one_launch = x.shape[0] <= 8192 or x.shape[1] >= 1536
+        one_launch = ops.route_rows_pays(*x.shape)
         if self.router_copy is not None and one_launch and x.data_ptr() % 16 == 0 and x.stride(0) % 8 == 0:
             if x.shape[0] <= self.few_tokens:
                 _, weights, groups = ops.route_and_group(x, self.router_copy, self.router_b, self.n_experts, *router)

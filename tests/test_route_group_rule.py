@@ -15,6 +15,11 @@ def test_one_launch_where_it_pays(experts, k, pays):
     assert ops.route_group_pays(experts, k) == pays
 
 
+@pytest.mark.parametrize("tokens,k,pays", [(17, 4096, True), (4096, 2048, True), (4097, 2048, False), (8192, 1024, True), (8192, 1536, True), (8193, 1024, False), (65536, 3072, False)])
+def test_many_tokens_of_long_rows_stay_a_product(tokens, k, pays):
+    assert ops.route_rows_pays(tokens, k) == pays
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("experts,pays", [(16, True), (32, False)])
 def test_a_layer_asks_the_rule(experts, pays):
