@@ -26,6 +26,8 @@ from cwm_amd.ops import build
     (2048, 3072, 28672, 0, False),  # (276 / 362)
     (3538, 10304, 14336, 0, False),  # many full rounds (807 / 931)
     (3538, 10304, 8192, 0, False),  # (457 / 505)
+    (1040, 4096, 14336, 0, True),  # too many small tiles to cut K, and large ones that fill little (148 / 135)
+    (1040, 28672, 4096, 1, True),  # (255 / 238)
     (900, 5120, 21504, 1, True),  # (283 / 213)
     (8192, 10304, 512, 1, True),  # a short K (194 / 115)
     (2048, 16, 2048, 0, False),  # fewer columns than a tile (11.5 / 12.2)
