@@ -206,9 +206,9 @@ static float library_fill(const TileCost& t, int M, int N, int units) {
 // meets library tiles (the first three) that leave a quarter of the chip idle.  A small result leaves the chip idle whatever the tile, and there the
 // library cuts K and this kernel does not (library / this, us: 384 x 128 x 1,536 7.0 / 10.6, 450 x 512 x 3,072 9.5 / 18.0, 600 x 1,024 x 3,072 17 / 20); from a
 // K of 16,384 on its cuts cost it more than they give (300 x 6,144 x 21,504 178 / 136), until they fill the chip.
-// Of 11,686 products timed, 3,467 of them of sizes drawn at random, with weights from memory, it takes 9,097, 1.29 times as fast in the mean and 107
-// slower by more than 5%, which is twice what repeated times differ by (1,500 x 4,096 x 28,672 by 8%, 512 x 2,048 x 1,536 by 18%); of those drawn 2,842,
-// 1.35 times as fast, 25 slower.  Taken wherever a quarter of the chip was idle, whatever K, 987 of those products were slower by more than 5%
+// Of 11,686 products timed, 3,467 of them of sizes drawn at random, with weights from memory, it takes 9,275, 1.28 times as fast in the mean and 130
+// slower by more than 5%, which is twice what repeated times differ by (1,500 x 4,096 x 28,672 by 8%, 512 x 2,048 x 1,536 by 18%); of those drawn 2,872,
+// 1.35 times as fast, 31 slower.  Taken wherever a quarter of the chip was idle, whatever K, 987 of those products were slower by more than 5%
 // (3,000 x 512 x 14,336 73 / 85, 3,538 x 10,304 x 14,336 by 13%).  Results of fewer columns than a tile (a router's 16: 2,048 x 16 x 2,048 11.5 / 12.2) stay too.
 extern "C" int cwm_gemm_bf16_wide_pays(int M, int N, int K, int units, int glu) {
   if (M <= 0 || N < 128 || K <= 0 || K % WIDE_BK || N % 16 || units <= 0) return 0;
@@ -230,8 +230,8 @@ extern "C" int cwm_gemm_bf16_wide_pays(int M, int N, int K, int units, int glu) 
   // many full rounds: the chip's power bounds both, which the costs do not know (3,538 x 10,304 x 8,192 457 / 505)
   if (share > 2.f) return us < 0.89f * library;
   // The costs of the library are too low where its large tiles leave most of the chip idle, and too many small ones for it to cut K fill the rest
-  // (1,040 x 4,096 x 14,336 148 / 135); a little where they leave much of a round idle (1,040 x 28,672 x 4,096 gated 255 / 238).
-  return us < (share > 0.19f && fill < 0.4f ? 1.05f : fill < 0.6f ? 0.96f : 0.92f) * library;
+  // (1,040 x 4,096 x 14,336 148 / 135); a little where they leave much of a round idle, and where a gate follows (1,040 x 28,672 x 4,096 255 / 238).
+  return us < (share > 0.19f && fill < 0.4f ? 1.05f : fill < 0.6f || glu ? 0.96f : 0.92f) * library;
 }
 
 // C [M][ldc] of c_dtype; glu: W holds gate and up rows in alternating groups of 8 and C [M, N / 2] receives silu(gate) * up in
