@@ -202,19 +202,20 @@ static float library_fill(const TileCost& t, int M, int N, int units) {
 }
 
 // Whether this kernel is expected to be faster than the library's product, with `glu` followed by the kernel that gates its
-// result (3 us and three passes that mostly stay in the memory-side cache): by the costs above, with room for their errors, and wherever a short K
-// meets library tiles (the first three) that leave a quarter of the chip idle.  A small result leaves the chip idle whatever the tile, and there the
-// library cuts K and this kernel does not (library / this, us: 384 x 128 x 1,536 7.0 / 10.6, 450 x 512 x 3,072 9.5 / 18.0, 600 x 1,024 x 3,072 17 / 20); from a
-// K of 16,384 on its cuts cost it more than they give (300 x 6,144 x 21,504 178 / 136), until they fill the chip.
-// Of 11,686 products timed, 3,467 of them of sizes drawn at random, with weights from memory, it takes 9,275, 1.28 times as fast in the mean and 130
-// slower by more than 5%, which is twice what repeated times differ by (1,500 x 4,096 x 28,672 by 8%, 512 x 2,048 x 1,536 by 18%); of those drawn 2,872,
-// 1.35 times as fast, 31 slower.  Taken wherever a quarter of the chip was idle, whatever K, 987 of those products were slower by more than 5%
-// (3,000 x 512 x 14,336 73 / 85, 3,538 x 10,304 x 14,336 by 13%).  Results of fewer columns than a tile (a router's 16: 2,048 x 16 x 2,048 11.5 / 12.2) stay too.
+// result (3 us and three passes that mostly stay in the memory-side cache): by the costs above, with room for their errors, and wherever a
+// short K, one of up to 4,096 of a large result, or a very long one meets library tiles (the first three) that leave a quarter of the chip
+// idle.  A small result leaves the chip idle whatever the tile, and there the library cuts K and this kernel does not (library / this, us:
+// 384 x 128 x 1,536 7.0 / 10.6, 450 x 512 x 3,072 9.5 / 18.0, 600 x 1,024 x 3,072 17 / 20); from a K of 16,384 on its cuts cost it more
+// than they give (300 x 6,144 x 21,504 178 / 136).
+// Of 11,686 products timed, 3,467 of them of sizes drawn at random, with weights from memory, it takes 9,460, 1.28 times as fast in the mean
+// and 143 slower by more than 5%, which is twice what repeated times differ by (512 x 2,048 x 1,536 by 18%); of those drawn 2,939, 1.34
+// times as fast, 36 slower.  Taken wherever a quarter of the chip was idle, whatever K, 987 of those products were slower by more than 5%
+// (3,000 x 512 x 14,336 73 / 85, 3,538 x 10,304 x 14,336 by 13%).  Results of fewer columns than a tile (a router's 16: 2,048 x 16 x 2,048
+// 11.5 / 12.2) stay too.
 extern "C" int cwm_gemm_bf16_wide_pays(int M, int N, int K, int units, int glu) {
   if (M <= 0 || N < 128 || K <= 0 || K % WIDE_BK || N % 16 || units <= 0) return 0;
   const float share = (float)M * (float)N / (65536.f * (float)units);
   if (share < 0.03f ? K > 1024 : share < 0.06f ? K >= 1536 : share < 0.08f && K >= 2048) return 0;
-  if (K >= 16384 && K < 24576 && share < 0.35f) return 1;
   float us = 0.f, library = 0.f, fill = 0.f;
   wide_tile(M, N, K, units, glu != 0, &us);
   for (int i = 0; i < (int)(sizeof(library_tiles) / sizeof(library_tiles[0])); ++i) {
@@ -226,8 +227,8 @@ extern "C" int cwm_gemm_bf16_wide_pays(int M, int N, int K, int units, int glu) 
   // 4,096, 6,144, 8,192, 10,240 and 12,288 columns, 1.15 at 4,128, 6,208, 8,224, 10,304 and 12,352 (2,048 x 10,304 x 2,048 97 / 87)
   if (N % 128) library *= 1.1f;
   if (glu) library += 3.f + 3e-7f * (float)M * (float)N;
-  if (K < 1536) return fill < 0.75f || us < 0.96f * library;
-  // many full rounds: the chip's power bounds both, which the costs do not know (3,538 x 10,304 x 8,192 457 / 505)
+  if (K < 1536 || (K <= 4096 && share > 1.2f) || (K >= 16384 && K < 24576 && share < 2.f)) return fill < 0.75f || us < 0.96f * library;
+  // many full rounds of a long K: the chip's power bounds both, which the costs do not know (3,538 x 10,304 x 8,192 457 / 505)
   if (share > 2.f) return us < 0.89f * library;
   // The costs of the library are too low where its large tiles leave most of the chip idle, and too many small ones for it to cut K fill the rest
   // (1,040 x 4,096 x 14,336 148 / 135); a little where they leave much of a round idle, and where a gate follows (1,040 x 28,672 x 4,096 255 / 238).
