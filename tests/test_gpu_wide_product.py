@@ -63,3 +63,42 @@ def test_what_it_refuses():
         ops.gemm_bf16_wide(x, w, tile=TILES)
     with pytest.raises(ops.KernelError):
         ops.gemm_bf16_wide(x, w, glu=True, tile=TILES - 1)
+
+
+# thousands of rows: several bands of row tiles, blocks that walk several tiles each, with and without ragged ends
+@pytest.mark.parametrize("m,n,k", [(2296, 2048, 2048), (2652, 10304, 576), (8193, 2064, 192)])
+def test_thousands_of_rows(m, n, k):
+    x, w = _operands(m, n, k, 0)
+    got = ops.gemm_bf16_wide(x, w, torch.float32)
+    assert torch.equal(ops.gemm_bf16_wide(x, w), got.bfloat16())
+    assert torch.equal(ops.gemm_bf16_wide(x, w, glu=True), ops.silu_mul(got.bfloat16(), grouped=True))
+    for lo in range(0, m, 1024):
+        exact = x[lo : lo + 1024].double() @ w.double().t()
+        # a float32 sum of K products is off by at most K * 2^-24 of the sum of their sizes
+        bound = k * 2.0**-24 * (x[lo : lo + 1024].double().abs() @ w.double().abs().t())
+        assert ((got[lo : lo + 1024].double() - exact).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("tile", range(TILES))
+def test_infinities_and_nan(tile):
+    """A row or column of W with one gives what float64 gives there, and the bits of all others stay."""
+    m, n, k = 300, 288, 192
+    x, w = _operands(m, n, k, 0)
+    clean = ops.gemm_bf16_wide(x, w, torch.float32, tile=tile)
+    x[3, 7], x[130, 0], x[299, k - 1], w[40, 5], w[287, 100] = float("inf"), float("nan"), -float("inf"), float("inf"), float("nan")
+    got = ops.gemm_bf16_wide(x, w, torch.float32, tile=tile)
+    exact = x.double() @ w.double().t()
+    rows, columns = torch.ones(m, dtype=torch.bool, device=DEV), torch.ones(n, dtype=torch.bool, device=DEV)
+    rows[[3, 130, 299]], columns[[40, 287]] = False, False
+    assert torch.equal(got[rows][:, columns], clean[rows][:, columns])
+    rest = ~(rows[:, None] & columns[None, :])
+    assert not exact[rest].isfinite().any()
+    assert torch.equal(got[rest].double().nan_to_num(2.0, 1.0, -1.0), exact[rest].nan_to_num(2.0, 1.0, -1.0))
+    if tile < TILES - 3:
+        gate, up = (got.bfloat16().float().view(m, n // 16, 2, 8)[:, :, i].reshape(m, n // 2).double() for i in range(2))
+        want = gate / (1.0 + torch.exp(-gate)) * up
+        gated = ops.gemm_bf16_wide(x, w, glu=True, tile=tile).double()
+        finite = want.isfinite()
+        assert torch.equal(gated[~finite].nan_to_num(2.0, 1.0, -1.0), want[~finite].nan_to_num(2.0, 1.0, -1.0))
+        # expf, the quotient and the product in float32 are off by far less than the rounding to bfloat16, 2^-9 of the value
+        assert ((gated[finite] - want[finite]).abs() <= 2.0**-8 * want[finite].abs() + 1e-30).all()
