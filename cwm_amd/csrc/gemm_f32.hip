@@ -189,8 +189,8 @@ gemm_f32_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lo
 // matrix instruction, [tile of 16 rows][step of 32 k][part][64 lanes][8 values], signs turned with their steps; and a block takes up to 256
 // rows, so that few blocks take a row of W apart, and the one wavefront that multiplies it does: the wavefronts lie side by side along the
 // columns, 16 each, with all WM tiles of 16 rows.  Operands of A and raw rows of W reach LDS by direct loads, W two steps further ahead; a
-// wavefront takes the next step's W apart while it multiplies; one barrier a step.  Now 828, 3,440 (1.36 PFLOP/s of bfloat16 products, of
-// which the chip's power allows 1.5 to 1.7), 198, 495 and 61 us, and the same bits.
+// wavefront takes the next step's W apart while it multiplies; one barrier a step.  Now 828, 3,440 (1.36 PFLOP/s of bfloat16 products; a
+// loop of nothing but these instructions reaches 1.45, ceilings.hip), 198, 495 and 60 us, and the same bits.
 #define PARTS_STEPS 8  // of K whose parts a block of the first kernel makes
 
 struct PartRows {  // a row's marks: bit r of [row tile][group of PARTS_STEPS steps]

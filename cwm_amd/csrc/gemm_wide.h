@@ -9,10 +9,10 @@
 // of registers and issues the loads of a step to come, a few of each after every row of matrix instructions: issued in one
 // go they queue up before the memory pipe while the matrix cores wait.  One barrier a step.
 //
-// What bounds it: with random operands on all 256 compute units the chip's power, at 1.7 to 1.8 PFLOP/s for matrix
-// instructions that do nothing else (2.4 with zeros); below that a step's loads (64 KB in flight a compute unit against
-// 1.3 to 1.6 us of latency), which is why smaller tiles with three to five buffers are used and no tile of 256 x 256 with
-// two.  A load of 64-byte instead of 128-byte rows is slower by a third, two groups of wavefronts that take turns between
+// What bounds it: on all 256 compute units the chip's power (a loop of nothing but these instructions on varied operands,
+// ceilings.hip, reaches 1.45 PFLOP/s; the library's best product 1.58); below that a step's loads (64 KB in flight a compute
+// unit against 1.3 to 1.6 us of latency), which is why smaller tiles with three to five buffers are used and no tile of
+// 256 x 256 with two.  A load of 64-byte instead of 128-byte rows is slower by a third, two groups of wavefronts that take turns between
 // reading and multiplying by 5 to 15%.
 //
 //   v_mfma_f32_16x16x32_bf16:  C^T[n, m] += W[n, k] * A[m, k]

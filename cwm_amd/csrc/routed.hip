@@ -973,7 +973,7 @@ struct GroupedWide {
   const bf16_t *w0, *w1;
   long w_stride;
   list_ints tile_expert;
-  int n_tiles, n_rows, N, K;
+  int n_tiles, N, K;
   int row_blocks, col_blocks;  // of whole tiles: 8 row tiles, 256 columns of weights
   void* out;
   long out_ld;
@@ -1200,7 +1200,7 @@ extern "C" int cwm_grouped_product(const void* a, long a_ld, long a_batch, int d
     const int vec_out = (out_ld * osize) % (4 * osize) == 0 && (out_batch * osize) % (4 * osize) == 0 && ((uintptr_t)out % (4 * osize)) == 0;
     if (loop && tiled && tiles_a_block == 8 && tile_expert && tile_align == 8 && vec_out && (unsigned long long)n_rows * a_ld * 2 < (1ull << 32) &&
         out_dtype == (w1 ? CWM_BF16 : CWM_F32)) {
-      GroupedWide g = {(const bf16_t*)a, a_ld, (list_ints)row_token, (const bf16_t*)w0, (const bf16_t*)w1, w_stride, (list_ints)tile_expert, n_tiles, n_rows, N, K,
+      GroupedWide g = {(const bf16_t*)a, a_ld, (list_ints)row_token, (const bf16_t*)w0, (const bf16_t*)w1, w_stride, (list_ints)tile_expert, n_tiles, N, K,
                        0, (N + (w1 ? 127 : 255)) / (w1 ? 128 : 256), out, out_ld, act};
       if (w1)
         hipLaunchKernelGGL((grouped_loop_kernel<bf16_t, true>), dim3(GROUPED_BLOCKS), dim3(512), 0, stream, g, used);
