@@ -5,7 +5,7 @@
 //
 // Measured, library / this, us: 1,040 x 4,096 x 4,096 46 / 39, 1,040 x 4,096 x 14,336 147 / 130, 2,296 x 2,048 x 2,048 27.5 / 21.7,
 // 1,500 x 2,048 x 2,048 21.4 / 17.0, 2,048 x 10,304 x 2,048 95 / 87, 600 x 4,096 x 4,096 37 / 29; but 4,096 x 8,192 x 6,144, two full rounds of
-// 256 x 256, 284 / 338, and 3,000 x 512 x 14,336, where the library cuts K, 73 / 85.
+// 256 x 256, 284 / 338, and 3,000 x 512 x 14,336, where the library cuts K, 62 / 79.
 //
 // Every sum adds its 64-wide steps of K in their order whatever the tile, so a row's bits depend on its own values alone.
 //
@@ -169,9 +169,9 @@ static float tile_us(const TileCost& t, int M, int N, int K, int units, float mo
   const float rounds = ceilf(tiles / (float)units), steps = (float)K / WIDE_BK;
   return t.start + rounds * (t.round + more_a_round + steps * t.step) + tiles / (float)units * steps * t.fill;
 }
-// This kernel's tiles.  Fitted to 1,100 products of 130 to 4,096 rows, 512 to 28,672 columns and a K of 512 to 14,336, within 8% (a K below
-// 512 takes up to a fifth longer); the tile it picks is on average 1% slower than the best one.  Tiles of 192 columns are not among them: at 42 of those
-// sizes one was ahead of all of these by more than 3%, by 17% at the most (3,538 x 3,072 x 6,144 112 / 131, 1,040 x 28,672 x 6,144 317 / 351).
+// This kernel's tiles.  Fitted to 1,100 products of 130 to 4,096 rows, 512 to 28,672 columns and a K of 512 to 14,336, within 8%;
+// the tile it picks is on average 1% slower than the best one.  Tiles of 192 columns were built too: among the best nowhere by
+// more than 3%.
 static const TileCost wide_tiles[] = {
     {256, 128, 2.18f, 2.96f, 0.54f, 0.30f}, {192, 128, 2.64f, 2.31f, 0.43f, 0.24f}, {128, 128, 3.18f, 1.29f, 0.35f, 0.18f},
     {64, 128, 2.94f, 0.61f, 0.26f, 0.10f},  {128, 256, 2.37f, 2.70f, 0.58f, 0.28f}, {160, 256, 2.39f, 3.40f, 0.69f, 0.31f},
@@ -189,8 +189,7 @@ static int wide_tile(int M, int N, int K, int units, bool glu, float* us) {
   return best;
 }
 // The library's product, as if it picked the best of these tiles: fitted to its times for the same sizes, within 14%.  It wins
-// where its large tiles fill whole rounds (4,096 x 8,192 x 6,144).  Small results and a K outside that range it misses by more (short ones take
-// up to 1.5 times as long), which the rule below knows.
+// where its large tiles fill whole rounds (4,096 x 8,192 x 6,144).
 static const TileCost library_tiles[] = {
     {256, 256, 6.9f, 6.4f, 0.97f, 0.43f}, {256, 192, 3.2f, 5.3f, 1.25f, 0.f},  {192, 256, 0.f, 10.3f, 0.72f, 0.42f},  {256, 128, 0.f, 12.7f, 0.38f, 0.58f},
     {128, 256, 9.4f, 0.f, 0.31f, 0.58f},  {128, 128, 12.f, 1.3f, 0.f, 0.49f}, {160, 128, 0.f, 13.5f, 0.64f, 0.f}};
@@ -202,20 +201,16 @@ static float library_fill(const TileCost& t, int M, int N, int units) {
 }
 
 // Whether this kernel is expected to be faster than the library's product, with `glu` followed by the kernel that gates its
-// result (3 us and three passes that mostly stay in the memory-side cache): by the costs above, with room for their errors, and wherever a
-// short K, one of up to 4,096 of a large result, or a very long one meets library tiles (the first three) that leave a quarter of the chip
-// idle.  A small result leaves the chip idle whatever the tile, and there the library cuts K and this kernel does not (library / this, us:
-// 384 x 128 x 1,536 7.0 / 10.6, 450 x 512 x 3,072 9.5 / 18.0, 600 x 1,024 x 3,072 17 / 20); from a K of 16,384 on its cuts cost it more
-// than they give (300 x 6,144 x 21,504 178 / 136).
-// Of 11,686 products timed, 3,467 of them of sizes drawn at random, with weights from memory, it takes 9,460, 1.28 times as fast in the mean
-// and 143 slower by more than 5%, which is twice what repeated times differ by (512 x 2,048 x 1,536 by 18%); of those drawn 2,939, 1.34
-// times as fast, 36 slower.  Taken wherever a quarter of the chip was idle, whatever K, 987 of those products were slower by more than 5%
-// (3,000 x 512 x 14,336 73 / 85, 3,538 x 10,304 x 14,336 by 13%).  Results of fewer columns than a tile (a router's 16: 2,048 x 16 x 2,048
-// 11.5 / 12.2) stay too.
+// result (3 us and three passes that mostly stay in the memory-side cache): where its largest tiles (the first three) leave a
+// quarter of the chip idle, or by the costs above, by 4% at least.  Of those 1,100 products it takes 693, 1.38 times as fast in the
+// mean and 8 of them slower by more than 3% (3,000 x 512 x 14,336 by 15%); with the gate 294 of 455, 1.23 times as fast, 5 slower
+// (1,040 x 28,672 x 4,096 249 / 227, but 2,048 x 28,672 x 4,096, which stays, 382 / 395).  A result that covers a few hundredths of the
+// chip leaves it idle whatever the tile, and there the library cuts a long K and this kernel does not: 130 x 512, K of 3,072
+// 24 / 19, 6,144 25 / 35.  Results of fewer columns than a tile (a router's 16: 2,048 x 16 x 2,048 11.5 / 12.2) stay too.
 extern "C" int cwm_gemm_bf16_wide_pays(int M, int N, int K, int units, int glu) {
   if (M <= 0 || N < 128 || K <= 0 || K % WIDE_BK || N % 16 || units <= 0) return 0;
   const float share = (float)M * (float)N / (65536.f * (float)units);
-  if (share < 0.03f ? K > 1024 : share < 0.06f ? K >= 1536 : share < 0.08f && K >= 2048) return 0;
+  if (K > (share < 0.04f ? 3072 : share < 0.08f ? 4096 : K)) return 0;
   float us = 0.f, library = 0.f, fill = 0.f;
   wide_tile(M, N, K, units, glu != 0, &us);
   for (int i = 0; i < (int)(sizeof(library_tiles) / sizeof(library_tiles[0])); ++i) {
@@ -227,12 +222,7 @@ extern "C" int cwm_gemm_bf16_wide_pays(int M, int N, int K, int units, int glu) 
   // 4,096, 6,144, 8,192, 10,240 and 12,288 columns, 1.15 at 4,128, 6,208, 8,224, 10,304 and 12,352 (2,048 x 10,304 x 2,048 97 / 87)
   if (N % 128) library *= 1.1f;
   if (glu) library += 3.f + 3e-7f * (float)M * (float)N;
-  if (K < 1536 || (K <= 4096 && share > 1.2f) || (K >= 16384 && K < 24576 && share < 2.f)) return fill < 0.75f || us < 0.96f * library;
-  // many full rounds of a long K: the chip's power bounds both, which the costs do not know (3,538 x 10,304 x 8,192 457 / 505)
-  if (share > 2.f) return us < 0.89f * library;
-  // The costs of the library are too low where its large tiles leave most of the chip idle, and too many small ones for it to cut K fill the rest
-  // (1,040 x 4,096 x 14,336 148 / 135); a little where they leave much of a round idle, and where a gate follows (1,040 x 28,672 x 4,096 255 / 238).
-  return us < (share > 0.19f && fill < 0.4f ? 1.05f : fill < 0.6f || glu ? 0.96f : 0.92f) * library;
+  return fill < 0.75f || us < 0.96f * library;
 }
 
 // C [M][ldc] of c_dtype; glu: W holds gate and up rows in alternating groups of 8 and C [M, N / 2] receives silu(gate) * up in
