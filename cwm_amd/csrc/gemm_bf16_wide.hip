@@ -5,7 +5,7 @@
 //
 // Measured, library / this, us: 1,040 x 4,096 x 4,096 46 / 39, 1,040 x 4,096 x 14,336 147 / 130, 2,296 x 2,048 x 2,048 27.5 / 21.7,
 // 1,500 x 2,048 x 2,048 21.4 / 17.0, 2,048 x 10,304 x 2,048 95 / 87, 600 x 4,096 x 4,096 37 / 29; but 4,096 x 8,192 x 6,144, two full rounds of
-// 256 x 256, 284 / 338, and 3,000 x 512 x 14,336, where the library cuts K, 62 / 79.
+// 256 x 256, 284 / 338, and 3,000 x 512 x 14,336, where the library cuts K, 73 / 85.
 //
 // Every sum adds its 64-wide steps of K in their order whatever the tile, so a row's bits depend on its own values alone.
 //
@@ -169,9 +169,9 @@ static float tile_us(const TileCost& t, int M, int N, int K, int units, float mo
   const float rounds = ceilf(tiles / (float)units), steps = (float)K / WIDE_BK;
   return t.start + rounds * (t.round + more_a_round + steps * t.step) + tiles / (float)units * steps * t.fill;
 }
-// This kernel's tiles.  Fitted to 1,100 products of 130 to 4,096 rows, 512 to 28,672 columns and a K of 512 to 14,336, within 8%;
-// the tile it picks is on average 1% slower than the best one.  Tiles of 192 columns were built too: among the best nowhere by
-// more than 3%.
+// This kernel's tiles.  Fitted to 1,100 products of 130 to 4,096 rows, 512 to 28,672 columns and a K of 512 to 14,336, within 8% (a K below
+// 512 takes up to a fifth longer); the tile it picks is on average 1% slower than the best one.  Tiles of 192 columns are not among them: at 42 of those
+// sizes one was ahead of all of these by more than 3%, by 17% at the most (3,538 x 3,072 x 6,144 112 / 131, 1,040 x 28,672 x 6,144 317 / 351).
 static const TileCost wide_tiles[] = {
     {256, 128, 2.18f, 2.96f, 0.54f, 0.30f}, {192, 128, 2.64f, 2.31f, 0.43f, 0.24f}, {128, 128, 3.18f, 1.29f, 0.35f, 0.18f},
     {64, 128, 2.94f, 0.61f, 0.26f, 0.10f},  {128, 256, 2.37f, 2.70f, 0.58f, 0.28f}, {160, 256, 2.39f, 3.40f, 0.69f, 0.31f},
@@ -200,13 +200,14 @@ static float library_fill(const TileCost& t, int M, int N, int units) {
   return (float)M * (float)N / (ceilf(tiles / (float)units) * (float)units * (float)(t.rows * t.columns));
 }
 
-// Whether this kernel is expected to be faster than the library's product, with `glu` followed by the kernel that gates its
-// result (3 us and three passes that mostly stay in the memory-side cache): where its largest tiles (the first three) leave a
-// quarter of the chip idle, or by the costs above, by 4% at least.  Of those 1,100 products it takes 693, 1.38 times as fast in the
-// mean and 8 of them slower by more than 3% (3,000 x 512 x 14,336 by 15%); with the gate 294 of 455, 1.23 times as fast, 5 slower
-// (1,040 x 28,672 x 4,096 249 / 227, but 2,048 x 28,672 x 4,096, which stays, 382 / 395).  A result that covers a few hundredths of the
-// chip leaves it idle whatever the tile, and there the library cuts a long K and this kernel does not: 130 x 512, K of 3,072
-// 24 / 19, 6,144 25 / 35.  Results of fewer columns than a tile (a router's 16: 2,048 x 16 x 2,048 11.5 / 12.2) stay too.
+// Whether this kernel takes a product from the library, with `glu` also the kernel that gates its result (3 us and three passes that mostly
+// stay in the memory-side cache): where the library's largest tiles (the first three) leave a quarter of the chip idle, or by the costs above, by
+// 4% at least.  Of 2,127 products that drawn steps of all designs bring it, timed on the GPU with weights from memory, it is 1.09 times as fast in
+// the mean, and 338 times slower by more than 5%, 20 times by more than 10 us: small results, where the library cuts a K of 1,536 and more and this
+// kernel does not (library / this, us: 450 x 512 x 3,072 9.5 / 18.0, 384 x 2,048 x 2,048 12.4 / 14.9).  They stay all the same, down to a few
+// hundredths of the chip: a call of the library takes the host 20 us more in a step, and steps of such products wait for the host (60 drawn steps with the
+// library for most of those 338 took 3.2% longer, up to 10%; 380 tokens with three of them 1,614 us and 1,485).  Results of fewer columns than a
+// tile (a router's 16: 2,048 x 16 x 2,048 11.5 / 12.2) stay with the library.
 extern "C" int cwm_gemm_bf16_wide_pays(int M, int N, int K, int units, int glu) {
   if (M <= 0 || N < 128 || K <= 0 || K % WIDE_BK || N % 16 || units <= 0) return 0;
   const float share = (float)M * (float)N / (65536.f * (float)units);
