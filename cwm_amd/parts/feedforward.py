@@ -121,15 +121,17 @@ class GatedMLP(FeedForward):
             matrices += [row, row.new_zeros((-(2 * self.hidden_dim + 1) % 16, self.dim))]
         self.gate_up = self.gate_up_wide = LinearWeights.joined(matrices, [None] * len(matrices), stream_copy=runtime.stream_copies)
         if self.row_gate is not None:
-            # Up to as many rows as the tiled product takes, the columns there are: it would take 2,064 too, in more time than the streaming product
-            # or the library 2,049 (us, 2,049 / 2,064 columns: 129 rows 14.8 / 17.7, 256 16.1 / 21.3; 513 / 528 of 256: 33 rows 7.0 / 10.6).
+            # Up to as many rows as the streaming product takes, the columns there are: the tiled product would take 2,064, in more time than that
+            # one 2,049 (us, 2,049 / 2,064 columns without a copy: 16 rows 9.1 / 11.1; 513 / 528 of 512: 33 rows 7.4 / 10.6).  Of 65 to 256 rows
+            # the library takes 2,049, in 3 to 5 us less than the tiled product 2,064, but its call costs the host 20 us more: a step of
+            # four layers and 128 rows 1,548 us with 2,049 columns, 1,505 with 2,064.
             streamed = self.gate_up.streamed
             self.gate_up = self.gate_up.rows(0, 2 * self.hidden_dim + 1)
             self.gate_up.streamed = streamed  # its tiles of 16 rows end in the same zeros
         self.down = LinearWeights(tensors[self.down_name], stream_copy=runtime.stream_copies)
 
     def forward(self, x: torch.Tensor, batch: Any) -> torch.Tensor:
-        joined = (self.gate_up if x.shape[0] <= ops.TILE_TALL_ROWS else self.gate_up_wide)(x, partials_ok=True)
+        joined = (self.gate_up if x.shape[0] <= ops.STREAM_MAX_ROWS else self.gate_up_wide)(x, partials_ok=True)
         hidden = ops.gated_act_rows(joined, self.hidden_dim, self.activation, x.dtype, 2 * self.hidden_dim if self.row_gate is not None else None)
         return self.down(hidden, partials_ok=True)
 
