@@ -63,6 +63,7 @@ SOURCES: Dict[str, Tuple[Mapping[str, int], ...]] = {
     "layernorm": ({},),
     "matrix_memory": ({},),
     "attention_talk": ({},),
+    "attention_talk_tile": ({},),
     "linear_attention": ({},),
     "short_conv": ({},),
     "token_side": ({},),

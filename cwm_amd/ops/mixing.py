@@ -1,6 +1,6 @@
 """Entry points of the kernels of layers whose attention heads exchange their weights, of gated linear attention, of
 short input convolutions, of a layer's own token input and of gated activations on rows
-(`csrc/attention_talk.hip`, `csrc/linear_attention.hip`, `csrc/short_conv.hip`, `csrc/token_side.hip`, `csrc/rowwise.hip`).
+(`csrc/attention_talk.hip`, `csrc/attention_talk_tile.hip`, `csrc/linear_attention.hip`, `csrc/short_conv.hip`, `csrc/token_side.hip`, `csrc/rowwise.hip`).
 Shapes, types and devices are checked on the host; there is no CPU path."""
 
 from __future__ import annotations
@@ -73,6 +73,58 @@ def _talking_long(q_rows, out_rows, cache, table_row, pos0, window, scale, sink,
         out_rows[r0:r1] = mixed.reshape(n_kv, m, per, hd).permute(1, 0, 2, 3).reshape(m, n_q * hd)
 
 
+# Tokens of a portion from which, where `csrc/attention_talk_tile.hip` has kernels for the model's heads, no table of scores is made (16
+# heads of 128, us through the table and without: 16 tokens after 2,000 84 and 53, after none 33 and 24, after 30,000 731 and 415; 8 tokens
+# after 2,000 63 and 50, 2 of them 47 and 49; portions of 128 and more, whose scores were a library's products: 1,500 214 and 81,
+# 130 100 and 31, 4,096 after 4,096 2,000 and 1,160; 24 heads, 1,500 tokens 333 and 129).
+TALK_TILE_FROM = 16
+TALK_TILE_KEYS = 32  # csrc/attention_talk_tile.hip: TILE_KEYS, of which a page holds a multiple, and rows of a tile
+TALK_TABLE_BYTES = 1 << 28  # most of a launch's table of mixed weights, where a tile of rows needs no more
+
+
+@functools.cache
+def _talk_tiles_built(n_q: int, n_kv: int, hd: int) -> bool:
+    return _build.load("attention_talk_tile").cwm_talking_tile_heads(ctypes.c_int(n_q), ctypes.c_int(n_kv), ctypes.c_int(hd)) > 0
+
+
+def _talking_tiles(q, out, cache, block_table, portions, window, scale, sink, talk) -> None:
+    """Portions of a prompt (sequence, first token, tokens, position of the first) with the mixed weights alone in memory, a table of
+    at most TALK_TABLE_BYTES at a time."""
+    KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
+    _n, n_q, hd = q.shape
+    n_kv = cache.shape[2]
+    lib = _build.load("attention_talk_tile")
+    launches, room = [[]], TALK_TABLE_BYTES // 2
+    for b, t0, n, pos0 in portions:
+        r0 = 0
+        while r0 < n:
+            # a tile of 32 rows reads its window and its own positions, from anywhere in a step of keys to anywhere in another
+            reach = pos0 + n if window is None else min(pos0 + n, window - 1 + 2 * TALK_TILE_KEYS)
+            columns = (reach // TALK_TILE_KEYS + 2) * TALK_TILE_KEYS
+            fits = room // (n_q * columns)
+            if launches[-1] and (fits < min(n - r0, TALK_TILE_KEYS) or len(launches[-1]) == lib.cwm_talking_tile_portions()):
+                launches.append([])
+                room = TALK_TABLE_BYTES // 2
+                continue
+            r1 = min(n, r0 + max(fits // TALK_TILE_KEYS, 1) * TALK_TILE_KEYS)
+            launches[-1].append((b, t0, n, pos0, r0, r1, columns))
+            room -= n_q * (r1 - r0) * columns
+            r0 = r1
+    stats = torch.empty((q.shape[0], n_q, 2), dtype=torch.float32, device=q.device)
+    weights = torch.empty(max(sum(n_q * (p[5] - p[4]) * p[6] for p in some) for some in launches), dtype=q.dtype, device=q.device)
+    for some in launches:
+        flat = [x for p in some for x in p]
+        _check(
+            lib,
+            lib.cwm_talking_tiles(
+                _ptr(q), ctypes.c_long(q.stride(0) if q.shape[0] > 1 else n_q * hd), _ptr(cache), _ptr(block_table), ctypes.c_int(block_table.shape[1]),
+                (ctypes.c_int * len(flat))(*flat), ctypes.c_int(len(some)), ctypes.c_int(n_q), ctypes.c_int(n_kv), ctypes.c_int(hd),
+                ctypes.c_int(cache.shape[3] // hd), ctypes.c_int(cache.shape[0]), ctypes.c_int(-1 if window is None else window - 1), ctypes.c_float(scale),
+                _ptr(sink), _ptr(talk), _ptr(stats), _ptr(weights), _ptr(out), _stream(),
+            ),
+        )
+
+
 def talking_attention(
     q: torch.Tensor,
     cache: torch.Tensor,
@@ -89,7 +141,8 @@ def talking_attention(
     None; `talk`: float32 [Hq, Hq] or None (no mixing).  `batch`: the step's descriptor (positions, sequence of each
     token, `cu_q`, `kv_len` and the host's `q_lens`, `kv_lens`).  Scores and weights of the step go through a table in
     float32 (`csrc/attention_talk.hip`); portions of `TALK_LONG_ROWS` tokens and more in bfloat16 take the scores and the
-    weighted values as matrix products instead.  Returns [T, Hq * hd] in the type of `q`."""
+    weighted values as matrix products instead, portions of `TALK_TILE_FROM` and more of most heads' sizes have no table of scores at all
+    (`csrc/attention_talk_tile.hip`).  Returns [T, Hq * hd] in the type of `q`."""
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
     _need_gpu(q, cache, block_table, sink, talk)
     if q.dim() != 3 or q.stride(2) != 1 or q.stride(1) != q.shape[2]:
@@ -120,13 +173,20 @@ def talking_attention(
         columns = reach(static.max_keys - 1) + 1
     else:
         q_lens, kv_lens = batch.q_lens, batch.kv_lens
-        long = [b for b, n in enumerate(q_lens) if n >= TALK_LONG_ROWS] if q.dtype == torch.bfloat16 else []
+        tiled = (
+            q.dtype == torch.bfloat16 and talk is not None and cache.shape[3] // hd % TALK_TILE_KEYS == 0 and q.data_ptr() % 16 == 0
+            and cache.data_ptr() % 16 == 0 and (q.stride(0) % 8 == 0 or n_tokens == 1) and _talk_tiles_built(n_q, n_kv, hd)
+        )
+        from_tokens = TALK_TILE_FROM if tiled else TALK_LONG_ROWS
+        long = [b for b, n in enumerate(q_lens) if n >= from_tokens] if q.dtype == torch.bfloat16 else []
         if long:
             out = torch.empty((n_tokens, width), dtype=q.dtype, device=q.device)
             starts = [0]
             for n in q_lens:
                 starts.append(starts[-1] + n)
-            for b in long:
+            if tiled:
+                _talking_tiles(q, out, cache, block_table, [(b, starts[b], q_lens[b], kv_lens[b] - q_lens[b]) for b in long], window, scale, sink, talk)
+            for b in () if tiled else long:
                 t0, t1 = starts[b], starts[b + 1]
                 _talking_long(q[t0:t1], out[t0:t1], cache, block_table[b], kv_lens[b] - q_lens[b], window, scale, sink, talk, lib)
             rest = [t for b, n in enumerate(q_lens) if b not in long for t in range(starts[b], starts[b] + n)]
