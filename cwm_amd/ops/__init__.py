@@ -538,15 +538,18 @@ def gemm_bf16_stream(
 
 
 def linear_inputs_takes(x: torch.Tensor, weight: torch.Tensor, rows_per_input: int) -> bool:
-    """Whether the product of a few rows of several inputs is one launch (`linear_inputs`)."""
+    """Whether the product of a few rows of several inputs is one launch (`linear_inputs`): as many as the streaming product takes.  A decode
+    step of two layers whose four products of 2,048 x 2,048 and their low rank meet five inputs, apart (five launches, and four more up to the
+    gated result) and so (two), us: 17 rows 377 and 316, 32 rows 416 and 367, 33 rows 496 and 392, 64 rows 557 and 478; at a width of 1,024 32 rows
+    375 and 366, 64 rows 476 and 447; of 3,072 24 rows 504 and 429."""
     return (
-        x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 3 and x.shape[1] <= 16
+        x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 3 and x.shape[1] <= STREAM_MAX_ROWS
         and rows_per_input % 16 == 0 and x.is_contiguous() and x.shape[1] * x.shape[2] % 8 == 0 and _stream_takes(x[0], weight)
     )
 
 
 def linear_inputs(x: torch.Tensor, weight: torch.Tensor, rows_per_input: int, streamed: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Several inputs x [G, M <= 16, K] times the rows of one joined weight that belong to each (`rows_per_input` rows an
+    """Several inputs x [G, M <= 64, K] times the rows of one joined weight that belong to each (`rows_per_input` rows an
     input, the last one's may be fewer), side by side: float32 partial sums [P, M, N] for the caller to add."""
     out = gemm_bf16_stream(x, weight, None, torch.float32, partials_ok=True, streamed=streamed, rows_per_input=rows_per_input)
     return out if out.dim() == 3 else out.unsqueeze(0)
