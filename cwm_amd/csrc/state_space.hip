@@ -39,13 +39,10 @@ __global__ void __launch_bounds__(256) conv_silu_kernel(const T* __restrict__ in
                                                         const float* __restrict__ bias, float* state, long state_ld, long state_off,
                                                         const int* __restrict__ slots, const int* __restrict__ cu_q,
                                                         const int* __restrict__ seq_of_token, T* __restrict__ out, int channels,
-                                                        int taps, int n_slots, int by_sequence) {
+                                                        int taps, int n_slots) {
   const int c = blockIdx.y * blockDim.x + threadIdx.x;
   if (c >= channels) return;
-  // a block a token; or (by_sequence) a block a sequence, for its first tokens and its state alone, the other
-  // tokens being the other kernel's
-  const int b = by_sequence ? blockIdx.x : seq_of_token[blockIdx.x];
-  const int t = by_sequence ? cu_q[b] : blockIdx.x;
+  const int t = blockIdx.x, b = seq_of_token[t];
   const int first = cu_q[b];
   const int j = t - first;
   const int q = cu_q[b + 1] - first;
@@ -95,40 +92,117 @@ __global__ void __launch_bounds__(256) conv_silu_kernel(const T* __restrict__ in
   }
 }
 
-// The tokens that read no state (place >= taps - 1 in their portion), bfloat16, eight channels a thread: a tap's eight
-// inputs are one load of 16 bytes.  The sums run in the order of the kernel above.
-__global__ void __launch_bounds__(256) conv_silu_body_kernel(const bf16_t* __restrict__ in, long in_ld, const float* __restrict__ w_by_tap,
-                                                             const float* __restrict__ bias, const int* __restrict__ cu_q,
-                                                             const int* __restrict__ seq_of_token, bf16_t* __restrict__ out, int channels,
-                                                             int taps) {
-  const int c = 8 * (blockIdx.y * blockDim.x + threadIdx.x);
-  if (c >= channels) return;
-  const int t = blockIdx.x;
-  const int hist = taps - 1;
-  if (t - cu_q[seq_of_token[t]] < hist) return;
-  float acc[8];
-  {
-    const float4 b0 = *(const float4*)(bias + c), b1 = *(const float4*)(bias + c + 4);
-    acc[0] = b0.x, acc[1] = b0.y, acc[2] = b0.z, acc[3] = b0.w, acc[4] = b1.x, acc[5] = b1.y, acc[6] = b1.z, acc[7] = b1.w;
-  }
+// Portions of a prompt in bfloat16, eight channels a thread: a unit of threads has CONV_RUN consecutive tokens, whose rows and the TAPS - 1
+// before them it reads once, all in flight, and makes those that read no state (place >= TAPS - 1 in their portion); a further unit a sequence
+// makes the first TAPS - 1 tokens, which do, and then leaves the new state.  The sums run in the order of the kernel above.  A thread a (token, eight channels)
+// for the former, which read every row TAPS times, and a launch of the kernel above for the latter took 21.7 and 5.3 us (2,048 tokens, 6,144
+// channels, four taps); this takes 20.9, most of it the activation's exponential and division, 300 tokens 6.4 instead of 9.5.
+// w_by_tap: the weights tap by tap ([taps][channels]): a thread's eight are 32 bytes, the threads' side by side.
+#define CONV_RUN 4
+template <int TAPS>
+__global__ void __launch_bounds__(256) conv_silu_runs_kernel(const bf16_t* __restrict__ in, long in_ld, const float* __restrict__ w_by_tap,
+                                                             const float* __restrict__ bias, float* __restrict__ state, long state_ld, long state_off,
+                                                             const int* __restrict__ slots, const int* __restrict__ cu_q,
+                                                             const int* __restrict__ seq_of_token, bf16_t* __restrict__ out, int n_tokens, int n_seqs,
+                                                             int channels, int n_slots) {
+  constexpr int HIST = TAPS - 1;
+  const int per = channels / 8, at = blockIdx.x * 256 + threadIdx.x, runs = (n_tokens + CONV_RUN - 1) / CONV_RUN;
+  int unit = at / per;
+  const int c = 8 * (at - unit * per);
+  if (unit >= runs + (HIST > 0 ? n_seqs : 0)) return;
+  auto eight = [](const float* p, float (&v)[8]) {
+    const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
+    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+  };
+  float wk[TAPS][8], bc[8];
+  eight(bias + c, bc);
 #pragma unroll
-  for (int k = 0; k < CONV_MAX_TAPS; ++k) {
-    if (k < taps) {
-      Frag8 x;
-      x.u = *(const uint4*)(in + (size_t)(t - (hist - k)) * in_ld + c);
-      // the weights tap by tap ([taps][channels]): a thread's eight are 32 bytes, the threads' side by side
-      const float4 w0 = *(const float4*)(w_by_tap + (size_t)k * channels + c), w1 = *(const float4*)(w_by_tap + (size_t)k * channels + c + 4);
-      const float wv[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+  for (int k = 0; k < TAPS; ++k) eight(w_by_tap + (size_t)k * channels + c, wk[k]);
+  auto leave = [&](int t, const float (&x)[TAPS][8]) {  // x: the oldest input first
+    float acc[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = fmaf(wv[e], bf16_to_f32(x.h[e]), acc[e]);
+    for (int e = 0; e < 8; ++e) acc[e] = bc[e];
+#pragma unroll
+    for (int k = 0; k < TAPS; ++k)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = fmaf(wk[k][e], x[k][e], acc[e]);
+    uint4 o;
+    o.x = pack2_bf16(silu_f32(acc[0]), silu_f32(acc[1]));
+    o.y = pack2_bf16(silu_f32(acc[2]), silu_f32(acc[3]));
+    o.z = pack2_bf16(silu_f32(acc[4]), silu_f32(acc[5]));
+    o.w = pack2_bf16(silu_f32(acc[6]), silu_f32(acc[7]));
+    *(uint4*)(out + (size_t)t * channels + c) = o;
+  };
+  auto widen = [](const Frag8& f, float (&v)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = bf16_to_f32(f.h[e]);
+  };
+  if (unit < runs) {
+    const int t0 = unit * CONV_RUN;
+    Frag8 rows[CONV_RUN + HIST];
+    int place[CONV_RUN];
+#pragma unroll
+    for (int i = 0; i < CONV_RUN + HIST; ++i) rows[i].u = *(const uint4*)(in + (size_t)max(0, min(t0 + i - HIST, n_tokens - 1)) * in_ld + c);
+#pragma unroll
+    for (int i = 0; i < CONV_RUN; ++i) {
+      const int t = min(t0 + i, n_tokens - 1);
+      place[i] = t - cu_q[seq_of_token[t]];
     }
+#pragma unroll
+    for (int i = 0; i < CONV_RUN; ++i) {
+      if (t0 + i >= n_tokens || place[i] < HIST) continue;
+      float x[TAPS][8];
+#pragma unroll
+      for (int k = 0; k < TAPS; ++k) widen(rows[i + k], x[k]);
+      leave(t0 + i, x);
+    }
+    return;
   }
-  uint4 o;
-  o.x = pack2_bf16(silu_f32(acc[0]), silu_f32(acc[1]));
-  o.y = pack2_bf16(silu_f32(acc[2]), silu_f32(acc[3]));
-  o.z = pack2_bf16(silu_f32(acc[4]), silu_f32(acc[5]));
-  o.w = pack2_bf16(silu_f32(acc[6]), silu_f32(acc[7]));
-  *(uint4*)(out + (size_t)t * channels + c) = o;
+  unit -= runs;
+  const int start = cu_q[unit], n = cu_q[unit + 1] - start, slot = slots[unit];
+  if (n == 0) return;
+  float* st = slot >= 0 && slot < n_slots ? state + (size_t)slot * state_ld + state_off + c : nullptr;
+  // the state, then the portion's first HIST inputs (the last again where it has fewer)
+  float x[HIST > 0 ? 2 * HIST : 1][8];
+#pragma unroll
+  for (int m = 0; m < HIST; ++m) {
+    Frag8 f;
+    f.u = *(const uint4*)(in + (size_t)(start + min(m, n - 1)) * in_ld + c);
+    widen(f, x[HIST + m]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[m][e] = 0.f;
+    if (st) eight(st + (size_t)m * channels, x[m]);
+  }
+#pragma unroll
+  for (int i = 0; i < HIST; ++i) {
+    if (i >= n) continue;
+    float taps[TAPS][8];
+#pragma unroll
+    for (int k = 0; k < TAPS; ++k)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) taps[k][e] = x[i + k][e];
+    leave(start + i, taps);
+  }
+  if (!st) return;
+#pragma unroll
+  for (int m = 0; m < HIST; ++m) {
+    float v[8];
+    if (n >= HIST) {
+      Frag8 f;
+      f.u = *(const uint4*)(in + (size_t)(start + n - HIST + m) * in_ld + c);
+      widen(f, v);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = 0.f;
+#pragma unroll
+      for (int k = 1; k < HIST; ++k)
+        if (n == k)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = x[m + k][e];
+    }
+    *(float4*)(st + (size_t)m * channels) = make_float4(v[0], v[1], v[2], v[3]);
+    *(float4*)(st + (size_t)m * channels + 4) = make_float4(v[4], v[5], v[6], v[7]);
+  }
 }
 
 // w_by_tap: the same weights as [taps][channels], or null (then every token goes through the kernel of a thread a channel)
@@ -141,19 +215,32 @@ extern "C" int cwm_conv_silu(const void* in, long in_ld, int dtype, const float*
   CWM_REQUIRE(state_off >= 0 && state_off + (long)(taps - 1) * channels <= state_ld, "conv_silu: the state row is too short");
   if (n_tokens == 0) return 0;
   dim3 grid(n_tokens, (channels + 255) / 256);
-  if (dtype == CWM_BF16 && w_by_tap && n_seqs > 0 && n_tokens > n_seqs && channels % 8 == 0 && in_ld % 8 == 0 && ((uintptr_t)in % 16) == 0 &&
-      ((uintptr_t)out % 16) == 0 && ((uintptr_t)w_by_tap % 16) == 0 && ((uintptr_t)bias % 16) == 0) {
-    // portions of a prompt: the tokens that read no state in pieces of 16 bytes, then a block a sequence for the rest
-    hipLaunchKernelGGL(conv_silu_body_kernel, dim3(n_tokens, (channels / 8 + 255) / 256), dim3(256), 0, stream, (const bf16_t*)in, in_ld, w_by_tap,
-                       bias, cu_q, seq_of_token, (bf16_t*)out, channels, taps);
-    hipLaunchKernelGGL(conv_silu_kernel<bf16_t>, dim3(n_seqs, (channels + 255) / 256), dim3(256), 0, stream, (const bf16_t*)in, in_ld, w, bias,
-                       state, state_ld, state_off, slots, cu_q, seq_of_token, (bf16_t*)out, channels, taps, n_slots, 1);
+  if (dtype == CWM_BF16 && w_by_tap && n_seqs > 0 && n_tokens > n_seqs && channels % 8 == 0 && in_ld % 8 == 0 && state_ld % 4 == 0 &&
+      state_off % 4 == 0 && ((uintptr_t)in % 16) == 0 && ((uintptr_t)out % 16) == 0 && ((uintptr_t)w_by_tap % 16) == 0 && ((uintptr_t)bias % 16) == 0 &&
+      ((uintptr_t)state % 16) == 0) {
+    const long threads = ((long)(n_tokens + CONV_RUN - 1) / CONV_RUN + n_seqs) * (channels / 8);
+    CWM_REQUIRE(threads < (1L << 31) - 256, "conv_silu: too many tokens");
+#define CWM_CONV_RUNS(TAPS)                                                                                                              \
+  hipLaunchKernelGGL(conv_silu_runs_kernel<TAPS>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, (const bf16_t*)in, in_ld, \
+                     w_by_tap, bias, state, state_ld, state_off, slots, cu_q, seq_of_token, (bf16_t*)out, n_tokens, n_seqs, channels, n_slots)
+    static_assert(CONV_MAX_TAPS == 8, "a build for every number of taps");
+    switch (taps) {
+      case 1: CWM_CONV_RUNS(1); break;
+      case 2: CWM_CONV_RUNS(2); break;
+      case 3: CWM_CONV_RUNS(3); break;
+      case 4: CWM_CONV_RUNS(4); break;
+      case 5: CWM_CONV_RUNS(5); break;
+      case 6: CWM_CONV_RUNS(6); break;
+      case 7: CWM_CONV_RUNS(7); break;
+      default: CWM_CONV_RUNS(8);
+    }
+#undef CWM_CONV_RUNS
   } else if (dtype == CWM_BF16)
     hipLaunchKernelGGL(conv_silu_kernel<bf16_t>, grid, dim3(256), 0, stream, (const bf16_t*)in, in_ld, w, bias, state, state_ld, state_off,
-                       slots, cu_q, seq_of_token, (bf16_t*)out, channels, taps, n_slots, 0);
+                       slots, cu_q, seq_of_token, (bf16_t*)out, channels, taps, n_slots);
   else if (dtype == CWM_F32)
     hipLaunchKernelGGL(conv_silu_kernel<float>, grid, dim3(256), 0, stream, (const float*)in, in_ld, w, bias, state, state_ld, state_off,
-                       slots, cu_q, seq_of_token, (float*)out, channels, taps, n_slots, 0);
+                       slots, cu_q, seq_of_token, (float*)out, channels, taps, n_slots);
   else
     return cwm_fail("conv_silu: unknown dtype %d", dtype);
   return cwm_launch_status("conv_silu");
