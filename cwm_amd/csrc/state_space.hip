@@ -586,8 +586,10 @@ __global__ void __launch_bounds__(256) selective_scan_single_kernel(const T* __r
 // `scan_carry_kernel` turns those into the states at the segments' starts; MODE 2 walks every segment from there and writes y.
 // Portions of one segment, decoded tokens among them, are left to the walk: their bits and their cost are what they are without a
 // long portion beside them (in blocks a decoded token pays for 64).
-// Bound by the waits between a block's stages, two blocks a compute unit (three in MODE 1; asked for, since the registers beyond
-// the first 256 would leave one), and by splitting values on the vector units (looking for infinities among B and C costs 2 of 115 us); the walk was bound by its reads of B and C from LDS.
+// A step of 64 tokens takes a block 9 us, 1.5 of them matrix instructions: scores 2 us (ten tiles of keys for four wavefronts, three at most),
+// S^T C and the state's update 1.4 each, y's stores 1.4, staging 1.2.  Step sizes and sums of logs are made a step ahead by the first
+// wavefront, which has one tile of scores, instead of while the others wait (58 to 55 us with the dealt tiles).  Two blocks a compute unit
+// (three in MODE 1; asked for, since the registers beyond the first 256 would leave one); bound by the vector units and by splitting values on them (looking for infinities among B and C costs 2 of 115 us); the walk was bound by its reads of B and C from LDS.
 #define BLOCK_TOKENS 64
 
 // Eight float32 values as the operands of three bfloat16 matrix products whose sum is the product of the values: each part is
@@ -649,15 +651,16 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
                                                          int split, int n_slots, const int* __restrict__ segments, float* __restrict__ seg_state,
                                                          float* __restrict__ seg_decay) {
   constexpr int ROWS = 16 * NT, PIECES = ROWS / 8, LOADS = BLOCK_TOKENS * PIECES / 256;
-  constexpr int ROW_LD = ROWS + 8, COL_LD = BLOCK_TOKENS + 8, SCORE_LD = BLOCK_TOKENS + 4;
+  constexpr int ROW_LD = ROWS + 8, COL_LD = BLOCK_TOKENS + 4, SCORE_LD = BLOCK_TOKENS + 4;
   static_assert(NT % 2 == 0, "the state's rows go into products of 32");
   typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(16))) bf16_t b_rows[MODE == 2 ? BLOCK_TOKENS : 1][ROW_LD];
   __shared__ __attribute__((aligned(16))) bf16_t c_rows[MODE == 2 ? BLOCK_TOKENS : 1][ROW_LD];
   __shared__ __attribute__((aligned(16))) bf16_t b_cols[ROWS][COL_LD];
   __shared__ __attribute__((aligned(16))) bf16_t scores[MODE == 2 ? 3 : 1][MODE == 2 ? BLOCK_TOKENS : 1][SCORE_LD];  // in three parts
-  __shared__ double sum_log[BLOCK_TOKENS];
-  __shared__ __attribute__((aligned(16))) float step_size[BLOCK_TOKENS], from_start[BLOCK_TOKENS], to_end[BLOCK_TOKENS];
+  // of this block of tokens and of the next, in turn
+  __shared__ double sum_log_of[2][BLOCK_TOKENS];
+  __shared__ __attribute__((aligned(16))) float step_size_of[2][BLOCK_TOKENS], from_start_of[2][BLOCK_TOKENS], to_end_of[2][BLOCK_TOKENS];
   __shared__ int spoilt;  // whether a B or C of the segment so far was not finite: from there on its products are the float32 instruction's
   const int* entry = segments + 6 * blockIdx.z;
   const int t0 = entry[1], t1 = entry[2], seg = entry[3], seg_base = entry[4], n_segs = entry[5];
@@ -671,100 +674,120 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
   const float bias = dt_bias[h], rate = -expf(a_log[h]), skip = d_skip[h];
 
   // rows 16 q + 4 j .. + 3 of column p as they lie in a head's state (rows past SCAN_ROWS * split do not exist)
-  auto state_at = [&](int q) -> long {
-    const int four = 4 * q + j;
+  auto state_at = [&](int q, int quarter) -> long {
+    const int four = 4 * q + quarter;
     return live && four < 4 * split ? (((long)(four / split) * P + p) * split + four % split) * 4 : -1;
   };
   float4v S[NT];
 #pragma unroll
   for (int q = 0; q < NT; ++q) {
-    const long at = state_at(q);
+    const long at = state_at(q, j);
     S[q] = MODE == 2 && at >= 0 ? *(const float4v*)(seg_state + ((size_t)(seg_base + seg) * heads + h) * head_elems + at) : (float4v){0.f, 0.f, 0.f, 0.f};
   }
 
   Words4 rb[LOADS], rc[MODE == 2 ? LOADS : 1];
-  uint32_t rx[8];
-  float r_dt = 0.f;
-  const bf16_t* b_src = xbc + inner + (size_t)g * N;
+  uint32_t rx[16];
+  uint32_t r_dt = 0;
+  const bf16_t* b_src = xbc + (size_t)t0 * xbc_ld + inner + (size_t)g * N;  // (a segment's offsets take 32 bits)
   const bf16_t* c_src = b_src + (size_t)groups * N;
-  // a thread fetches pieces of 16 bytes, the lanes of a wavefront those of its tokens at one place of the row
+  const bf16_t* x_src = xbc + (size_t)t0 * xbc_ld + (size_t)h * P;
+  const uint32_t x_col = live ? p : 0;
+  const uint32_t y_lane = 4 * j * inner + p;
+  // a thread fetches pieces of 16 bytes, the lanes of a wavefront those of its tokens at one place of the row (with a row's in neighbouring
+  // lanes the stores into b_cols meet in a bank four at a time: MODE 1 28 us instead of 24)
   auto fetch = [&](int c0) {
 #pragma unroll
     for (int k = 0; k < LOADS; ++k) {
       const int t = c0 + lane, n = 8 * (4 * k + wave);
-      const bool inside = t < t1 && n < N;  // N: a multiple of 8
-      const size_t at = (size_t)(inside ? t : t0) * xbc_ld + (inside ? n : 0);
-      const Words4 zero = {0, 0, 0, 0};
-      rb[k] = inside ? *(const Words4*)(b_src + at) : zero;
-      if constexpr (MODE == 2) rc[k] = inside ? *(const Words4*)(c_src + at) : zero;
+      // what lies past the end or beyond the state's rows (N: a multiple of 8) is read from a place that exists and left out when it is staged
+      const uint32_t at = (uint32_t)(min(t, t1 - 1) - t0) * (uint32_t)xbc_ld + min(n, N - 8);
+      rb[k] = *(const Words4*)(b_src + at);
+      if constexpr (MODE == 2) rc[k] = *(const Words4*)(c_src + at);
     }
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {  // tokens 16 (k / 4) + 4 j + k % 4 of the lane's column
-      const int t = c0 + 16 * (k >> 2) + 4 * j + (k & 3);
-      const uint32_t v = live && t < t1 ? xbc[(size_t)t * xbc_ld + (size_t)h * P + p] : 0;
-      rx[k >> 1] = k & 1 ? rx[k >> 1] | v << 16 : v;
-    }
-    if (wave == 0) r_dt = c0 + lane < t1 ? bf16_to_f32(dt_raw[(size_t)(c0 + lane) * dt_ld + h]) : 0.f;
+    // tokens 16 (k / 4) + 4 j + k % 4 of the lane's column; what lies past the end is the last token's and is left out when the
+    // values are used: a value put together or a branch taken here waits for its load (16 waits one after the other: 2,048 tokens of
+    // 64 heads 71 us instead of 58 in MODE 2, 38 instead of 24 in MODE 1)
+    for (int k = 0; k < 16; ++k) rx[k] = x_src[(uint32_t)(min(c0 + 16 * (k >> 2) + 4 * j + (k & 3), t1 - 1) - t0) * (uint32_t)xbc_ld + x_col];
+  };
+  auto fetch_dt = [&](int c0) {
+    if (wave == 0) r_dt = dt_raw[(size_t)min(c0 + lane, t1 - 1) * dt_ld + h];
   };
   double segment_log = 0.0;  // MODE 1, the first wavefront: of the segment's decay
 
+  // step sizes and sums of log decays of a block of tokens, by the first wavefront, which has the fewest scores to make
+  auto weigh = [&](int c0, int place, uint32_t raw) {
+    const bool inside = c0 + lane < t1;
+    const float zt = bf16_to_f32((bf16_t)raw) + bias, dt = inside ? (zt > 20.f ? zt : log1pf(expf(zt))) : 0.f;
+    // e^-128 is 0 in float32, as the decays of more are; bounded, they leave differences of sums finite and exact
+    const float log_decay = inside ? rate * dt : 0.f;
+    double through = (double)(log_decay < -128.f ? -128.f : log_decay);
+#pragma unroll
+    for (int off = 1; off < CWM_WAVE; off <<= 1) {
+      const double o = __shfl_up(through, off, CWM_WAVE);
+      if (lane >= off) through += o;
+    }
+    const double all = __shfl(through, CWM_WAVE - 1, CWM_WAVE);
+    sum_log_of[place][lane] = through;
+    step_size_of[place][lane] = dt;
+    from_start_of[place][lane] = expf((float)through);
+    to_end_of[place][lane] = expf((float)(all - through)) * dt;
+    if constexpr (MODE == 1) segment_log += all;
+  };
+
   if (tid == 0) spoilt = 0;
+  fetch_dt(t0);
   fetch(t0);
+  if (wave == 0) weigh(t0, 0, r_dt);
+  fetch_dt(t0 + BLOCK_TOKENS);
   for (int c0 = t0; c0 < t1; c0 += BLOCK_TOKENS) {
+    const int place = ((c0 - t0) / BLOCK_TOKENS) & 1;
+    const double* sum_log = sum_log_of[place];
+    const float *step_size = step_size_of[place], *from_start = from_start_of[place], *to_end = to_end_of[place];
     __syncthreads();  // the block of tokens before is done with
     Halves most = {0, 0};
 #pragma unroll
     for (int k = 0; k < LOADS; ++k) {
-      const int n = 8 * (4 * k + wave);
+      const int token = lane, n = 8 * (4 * k + wave);
+      const uint32_t inside = c0 + token < t1 && n < N ? 0xffffffffu : 0u;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
+        rb[k][e] &= inside;
+        if constexpr (MODE == 2) rc[k][e] &= inside;
         most = larger_magnitudes(most, rb[k][e]);
         if constexpr (MODE == 2) most = larger_magnitudes(most, rc[k][e]);
       }
       if constexpr (MODE == 2) {
-        *(Words4*)&b_rows[lane][n] = rb[k];
-        *(Words4*)&c_rows[lane][n] = rc[k];
+        *(Words4*)&b_rows[token][n] = rb[k];
+        *(Words4*)&c_rows[token][n] = rc[k];
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) b_cols[n + e][lane] = (bf16_t)(rb[k][e >> 1] >> (16 * (e & 1)));
+      for (int e = 0; e < 8; ++e) b_cols[n + e][token] = (bf16_t)(rb[k][e >> 1] >> (16 * (e & 1)));
     }
     if (max(most.x, most.y) >= 0x7f80) spoilt = 1;
-    float x[16];
-    uint32_t rx_now[8], largest = 0;
+    uint32_t rx_now[8];  // (the next block's come into rx meanwhile)
+    Halves largest = {0, 0};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) rx_now[k] = rx[k];  // (the next block's come into rx meanwhile)
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      x[k] = __uint_as_float(k & 1 ? rx[k >> 1] & 0xffff0000u : rx[k >> 1] << 16);
-      largest = max(largest, __float_as_uint(x[k]) & 0x7fffffffu);
+    for (int k = 0; k < 16; k += 2) {
+      const int t = c0 + 16 * (k >> 2) + 4 * j + (k & 3);
+      const uint32_t low = live && t < t1 ? rx[k] : 0, high = live && t + 1 < t1 ? rx[k + 1] : 0;
+      rx_now[k >> 1] = low | high << 16;
+      largest = larger_magnitudes(largest, rx_now[k >> 1]);
     }
-    const bool all_finite = __ballot(largest >= 0x7f800000u) == 0;  // of the wavefront's columns
-    if (wave == 0) {
-      const bool inside = c0 + lane < t1;
-      const float zt = r_dt + bias, dt = inside ? (zt > 20.f ? zt : log1pf(expf(zt))) : 0.f;
-      // e^-128 is 0 in float32, as the decays of more are; bounded, they leave differences of sums finite and exact
-      const float log_decay = inside ? rate * dt : 0.f;
-      double through = (double)(log_decay < -128.f ? -128.f : log_decay);
-#pragma unroll
-      for (int off = 1; off < CWM_WAVE; off <<= 1) {
-        const double o = __shfl_up(through, off, CWM_WAVE);
-        if (lane >= off) through += o;
-      }
-      const double all = __shfl(through, CWM_WAVE - 1, CWM_WAVE);
-      sum_log[lane] = through;
-      step_size[lane] = dt;
-      from_start[lane] = expf((float)through);
-      to_end[lane] = expf((float)(all - through)) * dt;
-      if constexpr (MODE == 1) segment_log += all;
-    }
+    auto x_of = [&](int k) { return __uint_as_float(k & 1 ? rx_now[k >> 1] & 0xffff0000u : rx_now[k >> 1] << 16); };
+    const uint32_t dt_next = keep_apart(r_dt);  // (taken here, where the loads are waited for)
+    const bool all_finite = __ballot(max(largest.x, largest.y) >= 0x7f80) == 0;  // of the wavefront's columns
     __syncthreads();
     const bool all_plain = __builtin_amdgcn_readfirstlane(spoilt) == 0;
+    fetch_dt(c0 + 2 * BLOCK_TOKENS);
     if (c0 + BLOCK_TOKENS < t1) fetch(c0 + BLOCK_TOKENS);  // in flight while this block of tokens is worked on
     if constexpr (MODE == 2) {
-      // scores of the wavefront's 16 queries and the keys up to them
-      const int t = 16 * wave + r;
-      const double mine = sum_log[t];
-      for (int b = 0; b <= wave; ++b) {
+      // scores of the wavefront's 16 queries and the keys up to them; of the last wavefront's four tiles of keys the second wavefront,
+      // which has two of its own, makes the first
+      for (int tile = wave == 3 ? 1 : 0; tile < (wave == 1 ? 3 : wave + 1); ++tile) {
+        const bool lent = wave == 1 && tile == 2;
+        const int b = lent ? 0 : tile, t = 16 * (lent ? 3 : wave) + r;
+        const double mine = sum_log[t];
         float4v acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q = 0; q < NT / 2; ++q) {
@@ -793,9 +816,10 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
           *(uint2*)&scores[k][t][16 * b + 4 * j] =
               make_uint2(__builtin_amdgcn_perm(w[k][1], w[k][0], 0x07060302u), __builtin_amdgcn_perm(w[k][3], w[k][2], 0x07060302u));
       }
+      if (wave == 0) weigh(c0 + BLOCK_TOKENS, place ^ 1, dt_next);
       if (wave % 2 == 0)  // keys go in pairs of tiles
 #pragma unroll
-        for (int k = 0; k < 3; ++k) *(uint2*)&scores[k][t][16 * (wave + 1) + 4 * j] = make_uint2(0u, 0u);
+        for (int k = 0; k < 3; ++k) *(uint2*)&scores[k][16 * wave + r][16 * (wave + 1) + 4 * j] = make_uint2(0u, 0u);
       __syncthreads();
       if (live) {
         float4v out[4];
@@ -854,7 +878,7 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
             for (int a = b + 1; a < 4; ++a)
 #pragma unroll
               for (int i = 0; i < 4; ++i)
-                out[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(score(16 * a + r, 16 * b + 4 * j + i), x[4 * b + i], out[a], 0, 0, 0);
+                out[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(score(16 * a + r, 16 * b + 4 * j + i), x_of(4 * b + i), out[a], 0, 0, 0);
         }
         if (!all_finite) {
           // a later key's score of 0 does not leave an infinity or a NaN out: the tiles on the diagonal key by key
@@ -863,7 +887,7 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
             const int b = k >> 2;
             for (int from = 0; from < 4; ++from) {
               const int key = 4 * from + (k & 3);
-              const float value = __shfl(x[k], 16 * from + r, CWM_WAVE);
+              const float value = __shfl(x_of(k), 16 * from + r, CWM_WAVE);
 #pragma unroll
               for (int i = 0; i < 4; ++i)
                 if (4 * j + i >= key) out[b][i] = fmaf(score(16 * b + 4 * j + i, 16 * b + key), value, out[b][i]);
@@ -874,16 +898,15 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
         for (int a = 0; a < 4; ++a)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int at = c0 + 16 * a + 4 * j + i;
-            if (at < t1) y[(size_t)at * inner + (size_t)h * P + p] = out[a][i] + skip * x[4 * a + i];
+            const int at = c0 + 16 * a + i;  // of the lane's quarter 0
+            if (at + 4 * j < t1) y[(size_t)at * inner + (size_t)h * P + y_lane] = out[a][i] + skip * x_of(4 * a + i);
           }
       }
     }
+    if (MODE == 1 && wave == 0 && c0 + BLOCK_TOKENS < t1) weigh(c0 + BLOCK_TOKENS, place ^ 1, dt_next);
     // the state after the block of tokens
     const float whole = from_start[BLOCK_TOKENS - 1];
     if (__builtin_expect(all_plain, 1)) {
-#pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] *= to_end[16 * (k >> 2) + 4 * j + (k & 3)];
 #pragma unroll
       for (int q = 0; q < NT; ++q) {
 #pragma unroll
@@ -891,7 +914,9 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
       }
 #pragma unroll
       for (int b = 0; b < 4; b += 2) {
-        const float v[8] = {x[4 * b], x[4 * b + 1], x[4 * b + 2], x[4 * b + 3], x[4 * b + 4], x[4 * b + 5], x[4 * b + 6], x[4 * b + 7]};
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = x_of(4 * b + k) * to_end[16 * (b + (k >> 2)) + 4 * j + (k & 3)];
         Frag8 part[3];
         three_parts(v, part);
 #pragma unroll
@@ -912,7 +937,7 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
       for (int b = 0; b < 4; ++b) {
         float xs[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) xs[i] = x[4 * b + i] * to_end[16 * b + group + i];
+        for (int i = 0; i < 4; ++i) xs[i] = x_of(4 * b + i) * to_end[16 * b + group + i];
 #pragma unroll
         for (int q = 0; q < NT; ++q) {
           float c[4];
@@ -933,9 +958,10 @@ __global__ void __launch_bounds__(256, MODE == 1 ? 3 : 2) scan_block_kernel(cons
     if (slot >= 0 && slot < n_slots) home = state + (size_t)slot * state_ld + (size_t)h * head_elems;
   }
   if (!home) return;
+  const int quarter = keep_apart(j);  // (the places are worked out again, not kept through the walk)
 #pragma unroll
   for (int q = 0; q < NT; ++q) {
-    const long at = state_at(q);
+    const long at = state_at(q, quarter);
     if (at >= 0) *(float4v*)(home + at) = S[q];
   }
 }
