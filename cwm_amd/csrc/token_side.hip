@@ -216,14 +216,25 @@ token_side_kernel(float* __restrict__ h, const int* __restrict__ tokens, const T
 
 // The same for bfloat16 weights whose inputs are rounded, on the matrix cores: TOK tokens a block of sixteen wavefronts.  The
 // gate's product (16 tokens x side_dim, K = dim) is split over the wavefronts by columns and K, whose parts meet in LDS; the
-// projection's (16 x dim, K = side_dim) by columns.  Both weights are read as they lie, 16 bytes a lane, once a block: w_proj
-// is [dim, side_dim] here.  A lane's results are four adjacent elements of one token's row.  The kernel above is bound by its
+// projection's (16 x dim, K = side_dim) by columns.  w_proj is [dim, side_dim] here.  The kernel above is bound by its
 // multiply-adds and by LDS (every product's x and gated value is a read of its own): of width 2,048 with 64 side values and two
-// addends, 1,500 tokens take it 88 us and 4,096 169; here 37 and 54, bound by the latency of a block's three stages.  All of a
-// row's loads in flight at once (24 more registers a load stage) measured slower, 38 to 68 us: they spill.
+// addends, 1,500 tokens take it 88 us; here 24.  A block's stages follow one another (rows 4 us, gate's product 6, projection 5, each bound
+// by its loads), so what can be asked for before a stage is: the tokens' values and the gate's first weights before the rows, the projection's
+// before the gate's sums, the norm's before the squares; a row's pieces four at a time; the rows stay in LDS in float32 and are
+// written once.  (38 us with a piece at a time, rows written and read again, and operands fetched a row a lane.)
 // dim: a multiple of 64 and at most 256 MAXT; side_dim: a multiple of 32, at most SIDE_TILE_MAX; rows of h, the addends and the
 // norm's weight start at multiples of 16 bytes (bfloat16 addends: of 8).
 #define SIDE_TILE_MAX 128
+#define SIDE_AHEAD 8  // steps of the gate's product whose weights are in flight
+#define SIDE_RUN 4    // pieces of a row that a thread has in flight
+#define SIDE_TURN_ROW 80  // bytes between a turned operand's rows of 64: no bank twice
+#define SIDE_TURN_BYTES (16 * SIDE_TURN_ROW)
+// bytes of LDS for TOK tokens a block
+static inline size_t side_tile_lds(int tok, int dim) {
+  const int waves = SIDE_THREADS / CWM_WAVE;
+  return (size_t)tok * (dim + 4) * sizeof(float) + (size_t)waves * 16 * tok * sizeof(float) + (size_t)tok * (SIDE_TILE_MAX + 8) * 2 + (size_t)waves * tok * sizeof(float) +
+         (size_t)waves * 2 * SIDE_TURN_BYTES;
+}
 
 template <int TOK, int MAXT>
 __device__ __forceinline__ void
@@ -232,118 +243,212 @@ token_side_tile(const int block, float* __restrict__ h, const int* __restrict__ 
                        int dim, int side_dim, int vocab, float eps, SideAddends addends, SidePortions portions) {
   extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
   constexpr int WAVES = SIDE_THREADS / CWM_WAVE, A_TOKEN = WAVES / TOK;  // wavefronts that load a token's row
-  const int x_ld = dim + 8;
-  bf16_t* xs = (bf16_t*)tile_lds;                                // [TOK][x_ld]
-  float* parts = (float*)(xs + (size_t)TOK * x_ld);              // [WAVES][16 side values][TOK]
+  constexpr int GATED = TOK * SIDE_TILE_MAX / SIDE_THREADS > 1 ? TOK * SIDE_TILE_MAX / SIDE_THREADS : 1;  // gated values a thread makes at most
+  const int x_ld = dim + 4;
+  float* xs = (float*)tile_lds;                                  // [TOK][x_ld]
+  float* parts = xs + (size_t)TOK * x_ld;                        // [WAVES][16 side values][TOK]
   bf16_t* gated = (bf16_t*)(parts + WAVES * 16 * TOK);           // [TOK][SIDE_TILE_MAX + 8]
   float* squares = (float*)(gated + TOK * (SIDE_TILE_MAX + 8));  // [WAVES][TOK]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, j = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, j = lane >> 4;
+  // A weight operand of 16 rows and 32 values is fetched four lanes a row (64 consecutive bytes) and turned to a lane's row through a place of
+  // the wavefront's own in LDS: fetched as the instruction takes it, neighbouring lanes lie in 16 rows, which costs a lookup a lane.
+  unsigned char* turn = (unsigned char*)(squares + WAVES * TOK) + wave * 2 * SIDE_TURN_BYTES;
+  const int turn_row = lane >> 2, turn_piece = lane & 3;
+  auto turned = [&](uint4 w, int slot) {
+    Frag8 f;
+    __builtin_amdgcn_wave_barrier();
+    *(uint4*)(turn + slot * SIDE_TURN_BYTES + turn_row * SIDE_TURN_ROW + turn_piece * 16) = w;
+    __builtin_amdgcn_wave_barrier();
+    f.u = *(const uint4*)(turn + slot * SIDE_TURN_BYTES + r * SIDE_TURN_ROW + j * 16);
+    __builtin_amdgcn_wave_barrier();
+    return f;
+  };
   const int t0 = block * TOK;
   bool any = false;
 #pragma unroll
   for (int tok = 0; tok < TOK; ++tok) any |= portions.serves(t0 + tok, n_tokens, true);
   if (!any) return;
-  // 1. the rows: pending addends into the residual, bfloat16 into LDS
+  // what does not hang on the rows is asked for before them: the tokens' own values and the gate's first steps
+  float own[GATED];
+  {
+    int token[GATED];
+#pragma unroll
+    for (int u = 0; u < GATED; ++u) token[u] = tokens[min(t0 + (int)(threadIdx.x + u * SIDE_THREADS) % TOK, n_tokens - 1)];
+#pragma unroll
+    for (int u = 0; u < GATED; ++u) {
+      const int k = (threadIdx.x + u * SIDE_THREADS) / TOK;
+      const bool known = token[u] >= 0 && token[u] < vocab;
+      const bf16_t e_k = table[(size_t)(known ? token[u] : 0) * table_ld + column0 + min(k, side_dim - 1)];
+      own[u] = known ? bf16_to_f32(e_k) : __uint_as_float(0x7fc00000u);
+    }
+  }
+  // the gate's product: wavefront w has the side values 16 (w % columns) .. + 15 and part w / columns of K.  The wavefronts' parts lie
+  // apart and each starts at a place of its own (of the column, not of the block, so that a sum has one order): rows lie a power of two
+  // apart, and in step they would all ask the same few channels of the caches
+  const int columns = side_dim / 16, k_parts = WAVES / columns, steps = dim / 32;
+  const int gate_column = wave % columns, gate_part = wave / columns, part_steps = (steps + k_parts - 1) / k_parts;
+  const int gate_from = min(gate_part * part_steps, steps - 1);
+  const int gate_count = gate_part < k_parts ? max(min(part_steps, steps - gate_part * part_steps), 0) : 0;  // wavefronts left over have no part
+  const int gate_start = gate_count > 0 ? 4 * gate_column % gate_count : 0;
+  auto gate_step = [&](int u) {  // the u-th of the wavefront's steps; past the last: the last once more
+    const int v = min(u, max(gate_count - 1, 0)) + gate_start;
+    return gate_from + (v >= gate_count ? max(v - gate_count, 0) : v);
+  };
+  const bf16_t* gate_row = w_gate + (size_t)(16 * gate_column + turn_row) * dim + 8 * turn_piece;
+  uint4 gate_w[SIDE_AHEAD];
+  auto fetch_gate = [&](int first) {
+#pragma unroll
+    for (int u = 0; u < SIDE_AHEAD; ++u) gate_w[u] = *(const uint4*)(gate_row + 32 * gate_step(first + u));
+  };
+  fetch_gate(0);
+  // 1. the rows: pending addends onto the residual, into LDS
   {
     const int tok = wave / A_TOKEN, t = t0 + tok;
     const bool serve = portions.serves(t, n_tokens, true);
-    for (int e = 4 * ((wave % A_TOKEN) * CWM_WAVE + lane); e < dim; e += 4 * CWM_WAVE * A_TOKEN) {
-      float4v x = {0.f, 0.f, 0.f, 0.f};
+    float* x_row = xs + (size_t)tok * x_ld;
+    const int e0 = 4 * ((wave % A_TOKEN) * CWM_WAVE + lane);
+    for (int at = e0; at < dim; at += SIDE_RUN * 4 * CWM_WAVE * A_TOKEN) {
+      float4v x[SIDE_RUN];
+      int e[SIDE_RUN];
+#pragma unroll
+      for (int u = 0; u < SIDE_RUN; ++u) {
+        e[u] = min(at + u * 4 * CWM_WAVE * A_TOKEN, dim - 4);  // a piece past the end: the row's last once more
+        x[u] = (float4v){0.f, 0.f, 0.f, 0.f};
+      }
       if (serve) {
-        x = *(const float4v*)(h + (size_t)t * dim + e);
+#pragma unroll
+        for (int u = 0; u < SIDE_RUN; ++u) x[u] = *(const float4v*)(h + (size_t)t * dim + e[u]);
         for (int a = 0; a < addends.n; ++a) {
           const SideAddend& ad = addends.a[a];
-          float4v y = {0.f, 0.f, 0.f, 0.f};
-          for (int p = 0; p < ad.n_partials; ++p) {
-            const size_t at = (size_t)p * ad.partial_stride + (size_t)t * ad.ld + e;
-            if (ad.dtype == CWM_F32) {
-              y += *(const float4v*)((const float*)ad.ptr + at);
-            } else {
-              const uint2 w = *(const uint2*)((const bf16_t*)ad.ptr + at);
-              y += (float4v){__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u)};
+          float4v y[SIDE_RUN];
+#pragma unroll
+          for (int u = 0; u < SIDE_RUN; ++u) y[u] = (float4v){0.f, 0.f, 0.f, 0.f};
+          if (ad.dtype == CWM_F32) {
+            for (int p = 0; p < ad.n_partials; ++p) {
+              const float* from = (const float*)ad.ptr + (size_t)p * ad.partial_stride + (size_t)t * ad.ld;
+#pragma unroll
+              for (int u = 0; u < SIDE_RUN; ++u) y[u] += *(const float4v*)(from + e[u]);
             }
+          } else {
+            const bf16_t* from = (const bf16_t*)ad.ptr + (size_t)t * ad.ld;
+            uint2 w[SIDE_RUN];
+#pragma unroll
+            for (int u = 0; u < SIDE_RUN; ++u) w[u] = *(const uint2*)(from + e[u]);
+#pragma unroll
+            for (int u = 0; u < SIDE_RUN; ++u)
+              y[u] += (float4v){__uint_as_float(w[u].x << 16), __uint_as_float(w[u].x & 0xffff0000u), __uint_as_float(w[u].y << 16), __uint_as_float(w[u].y & 0xffff0000u)};
           }
 #pragma unroll
-          for (int i = 0; i < 4; ++i) x[i] = fmaf(ad.scale, y[i], x[i]);
+          for (int u = 0; u < SIDE_RUN; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[u][i] = fmaf(ad.scale, y[u][i], x[u][i]);
         }
-        if (addends.n > 0) *(float4v*)(h + (size_t)t * dim + e) = x;  // read again at the end, after the block's barriers
       }
-      *(uint2*)(xs + (size_t)tok * x_ld + e) = make_uint2(pack2_bf16(x[0], x[1]), pack2_bf16(x[2], x[3]));
+#pragma unroll
+      for (int u = 0; u < SIDE_RUN; ++u) *(float4v*)(x_row + e[u]) = x[u];
     }
   }
   __syncthreads();
-  // 2. the gate's product: wavefront w has the side values 16 (w % columns) .. + 15 and every k_parts-th step of K from w / columns on
-  const int columns = side_dim / 16, k_parts = WAVES / columns;
+  // 2. the gate's product
   {
-    const int c = wave % columns, first = wave / columns;
     float4v acc = {0.f, 0.f, 0.f, 0.f};
-    if (first < k_parts) {
-      const bf16_t* w = w_gate + (size_t)(16 * c + r) * dim + 8 * j;
-      const bf16_t* x = xs + (size_t)min(r, TOK - 1) * x_ld + 8 * j;
-#pragma unroll 4
-      for (int step = first; step < dim / 32; step += k_parts) {
-        Frag8 fw, fx;
-        fw.u = *(const uint4*)(w + 32 * step);
-        fx.u = *(const uint4*)(x + 32 * step);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw.v, fx.v, acc, 0, 0, 0);
+    const float* x_row = xs + (size_t)min(r, TOK - 1) * x_ld + 8 * j;
+    for (int first = 0; first < gate_count; first += SIDE_AHEAD) {
+      uint4 now[SIDE_AHEAD];
+#pragma unroll
+      for (int u = 0; u < SIDE_AHEAD; ++u) now[u] = gate_w[u];
+      fetch_gate(first + SIDE_AHEAD);
+#pragma unroll
+      for (int u = 0; u < SIDE_AHEAD; ++u) {
+        const int s = gate_step(first + u);
+        if (first + u < gate_count) {
+          const float4v a = *(const float4v*)(x_row + 32 * s), b = *(const float4v*)(x_row + 32 * s + 4);
+          Frag8 fx;
+          fx.u = make_uint4(pack2_bf16(a[0], a[1]), pack2_bf16(a[2], a[3]), pack2_bf16(b[0], b[1]), pack2_bf16(b[2], b[3]));
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(turned(now[u], u & 1).v, fx.v, acc, 0, 0, 0);
+        }
       }
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (r < TOK) parts[(wave * 16 + 4 * j + i) * TOK + r] = acc[i];
   }
+  // the projection: wavefront w has the tiles w, w + 16, ... of 16 elements; its first weights are on their way past the barriers
+  // (eight tiles at a time: with sixteen tiles' weights and results both in registers they spill)
+  constexpr int GROUP = MAXT < 8 ? MAXT : 8;
+  static_assert(MAXT % GROUP == 0, "whole groups of tiles");
+  uint4 proj_w[GROUP];
+  auto fetch_proj = [&](int q0, int k) {
+#pragma unroll
+    for (int q = 0; q < GROUP; ++q)
+      proj_w[q] = *(const uint4*)(w_proj + (size_t)(min(16 * ((q0 + q) * WAVES + wave), dim - 16) + turn_row) * side_dim + k + 8 * turn_piece);
+  };
+  fetch_proj(0, 0);
   __syncthreads();
-  for (int id = threadIdx.x; id < TOK * side_dim; id += SIDE_THREADS) {
-    const int tok = id % TOK, k = id / TOK, t = t0 + tok;
-    float sum = 0.f;
-    for (int part = 0; part < k_parts; ++part) sum += parts[((part * columns + k / 16) * 16 + k % 16) * TOK + tok];
-    const float z = side_round(sum, true);
-    const float gelu = 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-    const int token = t < n_tokens ? tokens[t] : 0;
-    const bool known = token >= 0 && token < vocab;
-    const float e_k = known ? bf16_to_f32(table[(size_t)token * table_ld + column0 + k]) : __uint_as_float(0x7fc00000u);
-    gated[tok * (SIDE_TILE_MAX + 8) + k] = f32_to_bf16(gelu * e_k);
+#pragma unroll
+  for (int u = 0; u < GATED; ++u) {
+    const int id = threadIdx.x + u * SIDE_THREADS;
+    if (id < TOK * side_dim) {
+      const int tok = id % TOK, k = id / TOK;
+      float sum = 0.f;
+      for (int part = 0; part < k_parts; ++part) sum += parts[((part * columns + k / 16) * 16 + k % 16) * TOK + tok];
+      const float z = side_round(sum, true);
+      const float gelu = 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+      gated[tok * (SIDE_TILE_MAX + 8) + k] = f32_to_bf16(gelu * own[u]);
+    }
   }
   __syncthreads();
-  // 3. the projection: wavefront w has the tiles w, w + 16, ... of 16 elements; its squares; the scaled row into the residual
+  // 3. the projection; its squares; the scaled row into the residual
   float4v y[MAXT];
+#pragma unroll
+  for (int q = 0; q < MAXT; ++q) y[q] = (float4v){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q0 = 0; q0 < MAXT; q0 += GROUP)
+    for (int k = 0; k < side_dim; k += 32) {
+      Frag8 fg;
+      fg.u = *(const uint4*)(gated + min(r, TOK - 1) * (SIDE_TILE_MAX + 8) + k + 8 * j);
+#pragma unroll
+      for (int q = 0; q < GROUP; ++q)
+        if (16 * ((q0 + q) * WAVES + wave) < dim) y[q0 + q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(turned(proj_w[q], q & 1).v, fg.v, y[q0 + q], 0, 0, 0);
+      const bool more = k + 32 < side_dim;
+      fetch_proj(more ? q0 : min(q0 + GROUP, MAXT - GROUP), more ? k + 32 : 0);
+    }
   float sq = 0.f;
 #pragma unroll
-  for (int q = 0; q < MAXT; ++q) {
-    y[q] = (float4v){0.f, 0.f, 0.f, 0.f};
-    const int e = 16 * (q * WAVES + wave);
-    if (e < dim) {
-      for (int k = 0; k < side_dim; k += 32) {
-        Frag8 fw, fg;
-        fw.u = *(const uint4*)(w_proj + (size_t)(e + r) * side_dim + k + 8 * j);
-        fg.u = *(const uint4*)(gated + min(r, TOK - 1) * (SIDE_TILE_MAX + 8) + k + 8 * j);
-        y[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw.v, fg.v, y[q], 0, 0, 0);
-      }
-    }
+  for (int q = 0; q < MAXT; ++q)
 #pragma unroll
     for (int i = 0; i < 4; ++i) sq = fmaf(y[q][i], y[q][i], sq);
-  }
   sq += __shfl_xor(sq, 16, CWM_WAVE);
   sq += __shfl_xor(sq, 32, CWM_WAVE);
   if (j == 0 && r < TOK) squares[wave * TOK + r] = sq;
+  float4v norm[GROUP];  // of the first group; the others' behind the barrier
+#pragma unroll
+  for (int q = 0; q < GROUP; ++q) norm[q] = *(const float4v*)(weight + min(16 * (q * WAVES + wave), dim - 16) + 4 * j);
   __syncthreads();
-  if (r >= TOK || !portions.serves(t0 + r, n_tokens, true)) return;
-  float total = 0.f;
+  if (r < TOK) {
+    float total = 0.f;
 #pragma unroll
-  for (int w = 0; w < WAVES; ++w) total += squares[w * TOK + r];
-  const float rstd = 1.0f / sqrtf(total / (float)dim + eps);
-  float* row = h + (size_t)(t0 + r) * dim;
+    for (int w = 0; w < WAVES; ++w) total += squares[w * TOK + r];
+    const float rstd = 1.0f / sqrtf(total / (float)dim + eps);
+    float* x_row = xs + (size_t)r * x_ld;
 #pragma unroll
-  for (int q = 0; q < MAXT; ++q) {
-    const int e = 16 * (q * WAVES + wave) + 4 * j;
-    if (e < dim) {
-      const float4v n = *(const float4v*)(weight + e);
-      float4v x = *(const float4v*)(row + e);
+    for (int q = 0; q < MAXT; ++q) {
+      const int e = 16 * (q * WAVES + wave) + 4 * j;
+      if (e < dim) {
+        const float4v n = q < GROUP ? norm[q % GROUP] : *(const float4v*)(weight + e);
+        float4v x = *(const float4v*)(x_row + e);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] += y[q][i] * rstd * n[i];
-      *(float4v*)(row + e) = x;
+        for (int i = 0; i < 4; ++i) x[i] += y[q][i] * rstd * n[i];
+        *(float4v*)(x_row + e) = x;
+      }
     }
   }
+  __syncthreads();
+  // whole rows, a wavefront 1 KB at a time
+  const int tok = wave / A_TOKEN, t = t0 + tok;
+  if (!portions.serves(t, n_tokens, true)) return;
+  for (int e = 4 * ((wave % A_TOKEN) * CWM_WAVE + lane); e < dim; e += 4 * CWM_WAVE * A_TOKEN)
+    *(float4v*)(h + (size_t)t * dim + e) = *(const float4v*)(xs + (size_t)tok * x_ld + e);
 }
 
 template <int TOK, int MAXT>
@@ -406,9 +511,9 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
     tiled = tiled && lds_[a] % 4 == 0 && partial_strides[a] % 4 == 0 && ((uintptr_t)ptrs[a] % (dtypes[a] == CWM_F32 ? 16 : 8)) == 0;
   const SidePortions portions = {tiled ? seq_of_token : nullptr, cu_q};
   if (tiled) {
-    // sixteen tokens a block where that leaves no compute unit without one, else eight
-    const int tok = n_tokens >= 16 * 256 ? 16 : 8;
-    const size_t lds_tile = (size_t)tok * (dim + 8) * 2 + 16 * 16 * tok * sizeof(float) + (size_t)tok * (SIDE_TILE_MAX + 8) * 2 + 16 * tok * sizeof(float);
+    // eight tokens a block where their rows fit the LDS (up to 3,456 elements), else four
+    const int tok = side_tile_lds(8, dim) <= 163840 ? 8 : 4;
+    const size_t lds_tile = side_tile_lds(tok, dim);
     const bool both = seq_of_token && n_few < SIDE_FEW;
     const size_t lds_row = sizeof(float) * ((size_t)dim + side_dim), lds = both && lds_row > lds_tile ? lds_row : lds_tile;
     const int tile_blocks = (n_tokens + tok - 1) / tok;
@@ -425,11 +530,9 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
                          (const bf16_t*)table, table_ld, column0, (const bf16_t*)w_gate, (const bf16_t*)w_proj, weight, n_tokens, dim,      \
                          side_dim, vocab, eps, ad, portions);                                                                              \
   } while (0)
-    if (tok == 16) {
-      if (dim <= 2048) CWM_SIDE_TILE(16, 8); else CWM_SIDE_TILE(16, 16);
-    } else {
-      if (dim <= 2048) CWM_SIDE_TILE(8, 8); else CWM_SIDE_TILE(8, 16);
-    }
+    if (tok == 4) CWM_SIDE_TILE(4, 16);
+    else if (dim <= 2048) CWM_SIDE_TILE(8, 8);
+    else CWM_SIDE_TILE(8, 16);
 #undef CWM_SIDE_TILE
     if (!seq_of_token || both) return cwm_launch_status("token_side");
   }
