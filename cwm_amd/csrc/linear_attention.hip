@@ -259,7 +259,8 @@ __device__ __forceinline__ void unpack4_bf16(uint2 x, float (&v)[4]) {
 // long as A and B agree: with k = 4 g + i the accumulator register i of a tile of S is B as it stands.
 // The kernel waits for LDS and for sums over lanes most of the time, so it wants company on its compute unit: two blocks (three in
 // MODE 1) are asked for, since left alone the compiler takes more than 256 registers for heads of 128 rows and 128 columns and one
-// block has the unit to itself (16 heads, 1,500 tokens in 24 segments: MODE 2 137 us, 90 with two).
+// block has the unit to itself (16 heads, 1,500 tokens in 24 segments: MODE 2 137 us, 90 with two).  70 and MODE 1 41 us instead of 88 and 50 since
+// the norm's weight is read once and not behind every store, results are stored a block of tokens later, and the state's places cost a division for four rows.
 template <int MODE, int KIND, int CS, int EC>
 __global__ void __launch_bounds__(GLA_THREADS, MODE == 1 ? 3 : 2)
 gla_block_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
@@ -286,25 +287,28 @@ gla_block_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, con
 
   // the state's place in memory (the walking kernel's order)
   const int cols = GLA_THREADS / split, rows = gla_rows(dim, split), n_vt = (vdim + cols - 1) / cols;
-  auto state_at = [&](int d, int e) -> long {  // -1: a row or column that the state does not have
+  auto state_at = [&](int d, int e) -> long {  // of row d, a multiple of 4; the rows after it are GLA_THREADS apart.  -1: the state does not have them
     if (d >= split * rows || e >= n_vt * cols) return -1;
     const int vt = e / cols, col = e - vt * cols, part = d / rows, r = d - part * rows;
     return (((long)h * n_vt + vt) * rows + r) * GLA_THREADS + col * split + part;
   };
   float* home = state + (size_t)slot * state_ld;
+  const float* from = alone ? home : seg_start + (size_t)seg * seg_ld;
   float4v S[DT][EC];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int ec = 0; ec < EC; ++ec)
+    for (int ec = 0; ec < EC; ++ec) {
+      S[dt][ec] = (float4v){0.f, 0.f, 0.f, 0.f};
+      if constexpr (MODE == 2) {  // every load is issued, from an address that exists
+        const long at = state_at(16 * dt + 4 * g, e0 + 16 * (EC * wave + ec) + m);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        S[dt][ec][i] = 0.f;
-        if constexpr (MODE == 2) {
-          const long at = state_at(16 * dt + 4 * g + i, e0 + 16 * (EC * wave + ec) + m);
-          if (at >= 0) S[dt][ec][i] = alone ? home[at] : seg_start[(size_t)seg * seg_ld + at];
+        for (int i = 0; i < 4; ++i) {
+          const float x = from[(at >= 0 ? at : 0) + i * GLA_THREADS];
+          S[dt][ec][i] = at >= 0 ? x : 0.f;
         }
       }
+    }
   // the upper triangle of the block's scores is zero and stays so
   if constexpr (MODE == 2) As[tid >> 4][tid & 15] = 0.f;
 
@@ -329,6 +333,27 @@ gla_block_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, con
     }
 #pragma unroll
     for (int i = 0; i < EC; ++i) rv[i] = load4_bf16(v + row + h * vdim, e0 + 4 * (EC * sl + i), there ? vdim : 0, vec);
+  };
+  float scale[EC];  // the norm's weight of the lane's columns
+#pragma unroll
+  for (int ec = 0; ec < EC; ++ec)
+    scale[ec] = MODE == 2 && whole_head ? weight[h * weight_stride + min(e0 + 16 * (EC * wave + ec) + m, vdim - 1)] : 0.f;
+  // results of the block of tokens before: they are stored once the next one is staged, since waiting for what is staged waits for
+  // the stores before it too
+  uint32_t done[4][EC];
+  int done_at = -1;
+  auto store_done = [&]() {
+    if (MODE != 2 || done_at < 0) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int ec = 0; ec < EC; ++ec) {
+        const int t = done_at + 4 * g + i, e = e0 + 16 * (EC * wave + ec) + m;
+        if (t < t1 && e < vdim) {
+          const size_t at = ((size_t)t * heads + h) * vdim + e;
+          if (whole_head) out[at] = (bf16_t)done[i][ec]; else o_raw[at] = __uint_as_float(done[i][ec]);
+        }
+      }
   };
   float product = 1.f;  // MODE 1: of the segment's decays, in the thread that forms a channel's products
   fetch(t0);
@@ -357,16 +382,17 @@ gla_block_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, con
       *(float4*)&Vs[ts][4 * (EC * sl + i)] = make_float4(vv[0], vv[1], vv[2], vv[3]);
     }
     __syncthreads();
+    store_done();
     if (c0 + 16 < t1) fetch(c0 + 16);  // in flight while this block of tokens is worked on
     bf16_t gt[4][EC];
     if constexpr (MODE == 2) {
+      if (whole_head) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int ec = 0; ec < EC; ++ec) {
-          const int t = 4 * g + i, e = e0 + 16 * (EC * wave + ec) + m;
-          gt[i][ec] = (whole_head && t < n && e < vdim) ? gate[(size_t)(c0 + t) * proj_ld + h * vdim + e] : (bf16_t)0;
-        }
+          for (int ec = 0; ec < EC; ++ec)
+            gt[i][ec] = gate[(size_t)min(c0 + 4 * g + i, t1 - 1) * proj_ld + h * vdim + min(e0 + 16 * (EC * wave + ec) + m, vdim - 1)];
+      }
     }
     // ---- products of decays: queries from the block's start (threads of the last wavefronts), keys to its end ------- //
     for (int job = GLA_THREADS - 1 - tid; job < 2 * DP; job += GLA_THREADS) {
@@ -481,34 +507,29 @@ gla_block_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, con
         const float rstd = 1.0f / sqrtf(sq / (float)vdim + eps);
 #pragma unroll
         for (int ec = 0; ec < EC; ++ec) {
-          const int e = e0 + 16 * (EC * wave + ec) + m;
-          if (t < n && e < vdim) {
-            const size_t at = ((size_t)(c0 + t) * heads + h) * vdim + e;
-            if (whole_head) {
-              const float gv = bf16_to_f32(gt[i][ec]);
-              out[at] = f32_to_bf16(o[ec][i] * rstd * weight[h * weight_stride + e] * (gv / (1.0f + expf(-gv))));
-            } else {
-              o_raw[at] = o[ec][i];
-            }
+          if (whole_head) {
+            const float gv = bf16_to_f32(gt[i][ec]);
+            done[i][ec] = f32_to_bf16(o[ec][i] * rstd * scale[ec] * (gv / (1.0f + expf(-gv))));
+          } else {
+            done[i][ec] = __float_as_uint(o[ec][i]);
           }
         }
       }
+      done_at = c0;
     }
   }
+  store_done();
   if (MODE == 1 || last) {
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int ec = 0; ec < EC; ++ec)
+      for (int ec = 0; ec < EC; ++ec) {
+        const long at = state_at(16 * dt + 4 * g, e0 + 16 * (EC * wave + ec) + m);
+        if (at < 0) continue;
+        float* to = MODE == 1 ? seg_local + (size_t)seg * seg_ld : home;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const long at = state_at(16 * dt + 4 * g + i, e0 + 16 * (EC * wave + ec) + m);
-          if (at < 0) continue;
-          if constexpr (MODE == 1)
-            seg_local[(size_t)seg * seg_ld + at] = S[dt][ec][i];
-          else
-            home[at] = S[dt][ec][i];
-        }
+        for (int i = 0; i < 4; ++i) to[at + i * GLA_THREADS] = S[dt][ec][i];
+      }
   }
   if constexpr (MODE == 1) {
     const int c = GLA_THREADS - 1 - tid;
