@@ -12,7 +12,7 @@
 //
 // Both are exact under any cut of a sequence into portions: a portion starts from the state as the previous one
 // left it and performs the same operations in the same order as the whole sequence would.
-#include "common.h"
+#include "three_parts.h"
 #include <type_traits>
 
 CWM_DEFINE_ERROR_API
@@ -591,34 +591,6 @@ __global__ void __launch_bounds__(256) selective_scan_single_kernel(const T* __r
 // wavefront, which has one tile of scores, instead of while the others wait (58 to 55 us with the dealt tiles).  Two blocks a compute unit
 // (three in MODE 1; asked for, since the registers beyond the first 256 would leave one); bound by the vector units and by splitting values on them (looking for infinities among B and C costs 2 of 115 us); the walk was bound by its reads of B and C from LDS.
 #define BLOCK_TOKENS 64
-
-// Eight float32 values as the operands of three bfloat16 matrix products whose sum is the product of the values: each part is
-// the leading eight bits of what the parts before leave, so three hold all 24 (of values below 2^-110 the last lie among bfloat16's
-// subnormals and may be lost: less than 2^-125), and with a bfloat16 second operand every single product is exact.  An infinity or
-// a NaN is its first part alone; the other operand has to be finite, since a part may be zero.
-__device__ __forceinline__ void three_parts(const float (&v)[8], Frag8 (&part)[3]) {
-  uint32_t w[3][8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const uint32_t bits = __float_as_uint(v[e]);
-    w[0][e] = bits;
-    float rest = v[e] - __uint_as_float(bits & 0xffff0000u);
-    rest = (bits & 0x7f800000u) == 0x7f800000u ? 0.f : rest;
-    w[1][e] = __float_as_uint(rest);
-    w[2][e] = __float_as_uint(rest - __uint_as_float(w[1][e] & 0xffff0000u));
-  }
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-    part[k].u = make_uint4(__builtin_amdgcn_perm(w[k][1], w[k][0], 0x07060302u), __builtin_amdgcn_perm(w[k][3], w[k][2], 0x07060302u),
-                           __builtin_amdgcn_perm(w[k][5], w[k][4], 0x07060302u), __builtin_amdgcn_perm(w[k][7], w[k][6], 0x07060302u));
-}
-
-typedef unsigned short Halves __attribute__((ext_vector_type(2)));
-
-// The larger magnitudes, halves apart, of two bfloat16 values a word; from 0x7f80 on an infinity or a NaN.
-__device__ __forceinline__ Halves larger_magnitudes(Halves so_far, uint32_t w) {
-  return __builtin_elementwise_max(so_far, __builtin_bit_cast(Halves, w & 0x7fff7fffu));
-}
 
 // What is made of this value is made after this place: the compiler would move what both ways of a branch have in common
 // before it, and hold all of it in registers.
