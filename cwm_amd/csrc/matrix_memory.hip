@@ -780,16 +780,18 @@ memory_tile_kernel(const bf16_t* __restrict__ src, long src_stride, int q_off, i
 #pragma unroll
       for (int r = 0; r < 16; ++r) part[r] = 0.f;
       if (__builtin_expect(plain, 1)) {
+        Frag8 s[2][3], q[2];  // the small parts first, so that the sum is rounded at its full size twice only
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const float v[8] = {S[8 * u], S[8 * u + 1], S[8 * u + 2], S[8 * u + 3], S[8 * u + 4], S[8 * u + 5], S[8 * u + 6], S[8 * u + 7]};
-          Frag8 s[3], q;
-          three_parts(v, s);
+          three_parts(v, s[u]);
           const uint2 low = *(const uint2*)&q_rows[c][tile_row + 16 * u + 4 * half], high = *(const uint2*)&q_rows[c][tile_row + 16 * u + 8 + 4 * half];
-          q.u = make_uint4(low.x, low.y, high.x, high.y);
-#pragma unroll
-          for (int k = 2; k >= 0; --k) part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q.v, s[k].v, part, 0, 0, 0);
+          q[u].u = make_uint4(low.x, low.y, high.x, high.y);
         }
+#pragma unroll
+        for (int k = 2; k >= 0; --k)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q[u].v, s[u][k].v, part, 0, 0, 0);
       } else {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -825,9 +827,11 @@ memory_tile_kernel(const bf16_t* __restrict__ src, long src_stride, int q_off, i
     }
     {
       const float keep = dec_s[count - 1];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) S[r] *= keep;
       if (__builtin_expect(plain, 1)) {
+        memc_acc more;  // summed by itself, so that the state is rounded once a block of tokens
+#pragma unroll
+        for (int r = 0; r < 16; ++r) more[r] = 0.f;
+        Frag8 s[2][3], k[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const uint4 w = *(const uint4*)&v_cols[c][16 * u + 8 * half];
@@ -835,13 +839,18 @@ memory_tile_kernel(const bf16_t* __restrict__ src, long src_stride, int q_off, i
           const float v[8] = {__uint_as_float(w.x << 16) * f0.x, __uint_as_float(w.x & 0xffff0000u) * f0.y, __uint_as_float(w.y << 16) * f0.z,
                               __uint_as_float(w.y & 0xffff0000u) * f0.w, __uint_as_float(w.z << 16) * f1.x, __uint_as_float(w.z & 0xffff0000u) * f1.y,
                               __uint_as_float(w.w << 16) * f1.z, __uint_as_float(w.w & 0xffff0000u) * f1.w};
-          Frag8 s[3], k;
-          three_parts(v, s);
-          k.u = *(const uint4*)&k_cols[tile_row + c][16 * u + 8 * half];
-#pragma unroll
-          for (int x = 2; x >= 0; --x) S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k.v, s[x].v, S, 0, 0, 0);
+          three_parts(v, s[u]);
+          k[u].u = *(const uint4*)&k_cols[tile_row + c][16 * u + 8 * half];
         }
+#pragma unroll
+        for (int x = 2; x >= 0; --x)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) more = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k[u].v, s[u][x].v, more, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) S[r] = fmaf(keep, S[r], more[r]);
       } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) S[r] *= keep;
 #pragma unroll
         for (int i = 0; i < MEMC_L / 2; ++i) {
           const int s = 2 * i + half;
