@@ -68,7 +68,13 @@ __device__ __forceinline__ int tile_page(const int* table, const TalkTileArgs& A
   const int page = lp < A.table_width ? table[lp] : -1;
   return (unsigned)page < (unsigned)A.num_pages ? page : 0;
 }
-// whether a key of [first, last] lies in a page that is not there
+// the same of one thread's own range
+__device__ __forceinline__ bool row_lacks_page(const int* table, const TalkTileArgs& A, int first, int last) {
+  for (int lp = page_number(A, first); lp <= page_number(A, last); ++lp)
+    if (lp >= A.table_width || (unsigned)table[lp] >= (unsigned)A.num_pages) return true;
+  return false;
+}
+// whether a key of [first, last] lies in a page that is not there, of a wavefront's range
 __device__ __forceinline__ bool lacks_page(const int* table, const TalkTileArgs& A, int first, int last) {
   bool bad = false;
   for (int lp = page_number(A, first) + (int)(threadIdx.x & 63); lp <= page_number(A, last); lp += 64) {
@@ -349,6 +355,28 @@ talk_tile_mix_kernel(TalkTileArgs A, TalkPortions P, const float* __restrict__ s
 }
 
 // ---- values ------------------------------------------------------------------------------------------------------------ //
+// A row of a tile has weight zero for the tile's keys that it does not read, and zero times an infinity or a NaN is a NaN.  So a result
+// that is not finite, and all of a tile that reads a missing page, is made again from the row's own keys alone, sums of 128 keys one after the
+// other (an infinite or NaN value reaches its readers only, whatever rows lie beside them); rows that read a missing page are NaN, the others are not.
+#define VALUE_RANGE 128
+__device__ __forceinline__ float4 values_of_own_keys(const TalkTileArgs& A, const int* table, const bf16_t* weights, const bf16_t* values, size_t page_stride,
+                                                  int head_dim, int d, int first, int last) {
+  float total[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int from = first; from <= last; from += VALUE_RANGE) {
+    float part[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int key = from; key <= min(last, from + VALUE_RANGE - 1); ++key) {
+      const int lp = page_number(A, key), slot = key - lp * A.page_size;
+      const bf16_t* v = values + (size_t)table[lp] * page_stride + ((size_t)(slot / 8) * head_dim + d) * 8 + slot % 8;
+      const float w = bf16_to_f32(weights[key]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[i] = fmaf(w, bf16_to_f32(v[8 * i]), part[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) total[i] += part[i];
+  }
+  return make_float4(total[0], total[1], total[2], total[3]);
+}
+
 // HEADS: heads of a block, which share the values' operands.
 template <int HD, int HEADS, int RT>
 __global__ void __launch_bounds__(64 * VALUE_WAVES, 2)
@@ -364,7 +392,6 @@ talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int* table = A.block_table + (size_t)po.seq * A.table_width;
   const int p_last = po.pos0 + min(row0 + ROWS, po.r1) - 1, lo = first_key(A, po.pos0 + row0), base = table_base(A, po, row0);
-  const bool missing = lacks_page(table, A, lo, p_last);
 
   const bf16_t* from_w[RT][HEADS];
 #pragma unroll
@@ -414,7 +441,18 @@ talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict
         for (int g = 0; g < HEADS; ++g) acc[u][g][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt].v, wf[u][g].v, acc[u][g][dt], 0, 0, 0);
   }
   // lane 16 j + n holds row n, dims 16 dt + 4 j + i
-  const float nan = __uint_as_float(0x7fc00000u);
+  constexpr int ITEMS = HEADS * 16 * (HD / 4) / (64 * VALUE_WAVES);  // four dims of a row and head each, of a thread for 16 rows
+  static_assert(RT * ITEMS <= 32 && ITEMS * 64 * VALUE_WAVES == HEADS * 16 * (HD / 4), "a bit an item");
+  const bool missing = lacks_page(table, A, lo, p_last);
+  uint32_t again = missing ? 0xffffffffu : 0u;
+  auto item = [&](int u, int i, int& g, int& r, int& d) {
+    const int e = threadIdx.x + 64 * VALUE_WAVES * i;
+    d = e % (HD / 4) * 4, g = e / (HD / 4) % HEADS, r = e / (HD / 4) / HEADS;
+    return g0 + g < per && row0 + 16 * u + r < po.r1;
+  };
+  auto leave = [&](int row, int g, int d, float4v v) {
+    *(uint2*)(out + (size_t)(po.t0 + row) * A.n_q_heads * HD + (size_t)(c * per + g0 + g) * HD + d) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+  };
 #pragma unroll
   for (int u = 0; u < RT; ++u) {
     if (u > 0) __syncthreads();
@@ -423,15 +461,31 @@ talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) *(float4v*)&sums[wave][g][n][16 * dt + 4 * j] = acc[u][g][dt];
     __syncthreads();
-    for (int e = threadIdx.x; e < HEADS * 16 * (HD / 4); e += 64 * VALUE_WAVES) {
-      const int d = e % (HD / 4) * 4, g = e / (HD / 4) % HEADS, r = e / (HD / 4) / HEADS, row = row0 + 16 * u + r;
-      if (g0 + g >= per || row >= po.r1) continue;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      int g, r, d;
+      if (!item(u, i, g, r, d)) continue;
       float4v v = *(const float4v*)&sums[0][g][r][d];
 #pragma unroll
       for (int w = 1; w < VALUE_WAVES; ++w) v += *(const float4v*)&sums[w][g][r][d];
-      if (missing) v = (float4v){nan, nan, nan, nan};
-      *(uint2*)(out + (size_t)(po.t0 + row) * A.n_q_heads * HD + (size_t)(c * per + g0 + g) * HD + d) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+      if (!(fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < __builtin_inff())) again |= 1u << (u * ITEMS + i);
+      leave(row0 + 16 * u + r, g, d, v);
     }
+  }
+  if (__builtin_expect(again == 0, 1)) return;
+  const float nan = __uint_as_float(0x7fc00000u);
+  for (int x = 0; x < RT * ITEMS; ++x) {
+    int g, r, d;
+    const int u = x / ITEMS;
+    if (!(again >> x & 1) || !item(u, x % ITEMS, g, r, d)) continue;
+    const int row = row0 + 16 * u + r, p = po.pos0 + row, first = first_key(A, p);
+    if (missing && row_lacks_page(table, A, first, p)) {
+      leave(row, g, d, (float4v){nan, nan, nan, nan});
+      continue;
+    }
+    const bf16_t* w = weights + po.table + ((size_t)(c * per + g0 + g) * (po.r1 - po.r0) + row - po.r0) * po.columns - base;
+    const float4 own = values_of_own_keys(A, table, w, A.cache + plane + (size_t)c * A.page_size * HD, 2 * plane, HD, d, first, p);
+    leave(row, g, d, (float4v){own.x, own.y, own.z, own.w});
   }
 }
 

@@ -84,6 +84,61 @@ def test_a_missing_page_of_a_long_portion():
     gone[0, :9] = -1  # keys 0..287: before every row's window (301 on)
     got = ops.talking_attention(q, cache, gone, batch, 100, scale, sink=sink, talk=mix)
     assert torch.equal(got, ops.talking_attention(q, cache, table, batch, 100, scale, sink=sink, talk=mix))
-    gone[0, 15] = cache.shape[0]  # keys 480..511, out of range: rows 80 to 199 read one or more (and rows of their tile of 32 may answer so too)
+    gone[0, 15] = cache.shape[0]  # keys 480..511, out of range: rows 80 to 199 read one or more
     got = ops.talking_attention(q, cache, gone, batch, 100, scale, sink=sink, talk=mix)
-    assert torch.isnan(got[80:]).all() and torch.isfinite(got[:64]).all()
+    assert torch.isnan(got[80:]).all() and torch.isfinite(got[:80]).all()
+
+
+def _value_of(cache, table, b, key, n_kv, hd):
+    """The place of a key's values in the cache, [Hkv, hd]."""
+    page = cache.shape[3] // hd
+    slot = key % page
+    return cache[int(table[b, key // page]), 1].view(n_kv, page // 8, hd, 8)[:, slot // 8, :, slot % 8]
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("n_q,n_kv,hd,old,new,window", [(16, 8, 128, 5, 40, None), (8, 4, 64, 70, 100, 33), (24, 8, 128, 40, 130, 64), (9, 3, 128, 0, 16, None), (20, 4, 64, 300, 77, 1)])
+def test_a_value_that_is_not_finite_reaches_its_readers_only(bad, n_q, n_kv, hd, old, new, window):
+    """One element of one token's values: of the heads and elements that it lies in, the rows that read the token are not
+    finite, the others what they were up to another order of their sums; all else keeps its bits."""
+    from cwm_amd import ops
+
+    case = _talking_case(torch.bfloat16, n_q, n_kv, hd, 64, [old], [new], window, seed=n_q + new)
+    q, cache, table, batch, scale, sink, mix, want = case
+    clean = ops.talking_attention(q, cache, table, batch, window, scale, sink=sink, talk=mix).cpu()
+    bound = _bound(case, window)
+    key, head, d, per = old + new * 2 // 3, n_kv - 1, hd - 3, n_q // n_kv
+    _value_of(cache, table, 0, key, n_kv, hd)[head, d] = bad
+    got = ops.talking_attention(q, cache, table, batch, window, scale, sink=sink, talk=mix).cpu()
+    at = torch.arange(old, old + new)
+    reads = (at >= key) & (at - key < (window if window is not None else old + new))
+    assert reads.any() and not reads.all()
+    there = torch.zeros((n_q, hd), dtype=torch.bool)
+    there[head * per :, d] = True
+    there = there.flatten()
+    assert not torch.isfinite(got[reads][:, there]).any()
+    assert bool(((got.double() - want).abs() <= bound)[~reads].all())
+    assert torch.equal(got[:, ~there][reads], clean[:, ~there][reads])
+
+
+@pytest.mark.parametrize("place", ["q", "k"])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_queries_and_keys_that_are_not_finite(place, bad):
+    from cwm_amd import ops
+
+    n_q, n_kv, hd, old, new, window = 16, 8, 128, 20, 90, 48
+    q, cache, table, batch, scale, sink, mix, want = _talking_case(torch.bfloat16, n_q, n_kv, hd, 64, [old], [new], window, seed=4)
+    clean = ops.talking_attention(q, cache, table, batch, window, scale, sink=sink, talk=mix).cpu()
+    key = old + 50
+    if place == "q":
+        q[50, 3, 7] = bad
+    else:
+        cache[int(table[0, key // 64]), 0].view(n_kv, 64, hd)[2, key % 64, 7] = bad
+    got = ops.talking_attention(q, cache, table, batch, window, scale, sink=sink, talk=mix).cpu()
+    at = torch.arange(old, old + new)
+    reads = at == key if place == "q" else (at >= key) & (at - key < window)
+    assert torch.equal(got[~reads], clean[~reads])
+    if place == "q" or bad != bad:
+        assert torch.isnan(got[reads]).all()  # every head has a share of the bad one's weights
+    else:  # a score of an infinity either way: all weight or none
+        assert bool((~torch.isfinite(got[reads])).any())
