@@ -61,7 +61,7 @@ __device__ __forceinline__ int first_key(const TalkTileArgs& A, int p) { return 
 // the first key of a row's table: of its tile of 32 rows
 __device__ __forceinline__ int table_base(const TalkTileArgs& A, const TalkPortion& po, int row) { return first_key(A, po.pos0 + (row & ~31)) & ~(TILE_KEYS - 1); }
 
-// the page of the 32 keys from `kt` on (pages hold a multiple of 32 keys); a page that is not there: page 0
+// the page of the 32 keys from `kt` on (pages hold a multiple of 32 keys); a page that is not there, in the table or behind its end: page 0
 __device__ __forceinline__ int tile_page(const int* table, const TalkTileArgs& A, int kt, int& slot) {
   const int lp = page_number(A, kt);
   slot = kt - lp * A.page_size;
@@ -546,7 +546,6 @@ extern "C" int cwm_talking_tiles(const void* q, long q_stride, const void* cache
     TalkPortion& po = P.of[i];
     po.seq = d[0], po.t0 = d[1], po.n = d[2], po.pos0 = d[3], po.r0 = d[4], po.r1 = d[5], po.columns = d[6], po.table = at;
     CWM_REQUIRE(po.seq >= 0 && po.t0 >= 0 && po.pos0 >= 0 && po.r0 >= 0 && po.r0 % 32 == 0 && po.r1 > po.r0 && po.r1 <= po.n && po.columns % TILE_KEYS == 0, "talking_tiles: bad portion");
-    CWM_REQUIRE((po.pos0 + po.n - 1) / page_size < table_width, "talking_tiles: the block table ends before the last key");
     most_steps[i] = 0;
     for (int row0 = po.r0; row0 < po.r1; row0 += mix_rows) {
       const int tile = po.pos0 + row0 / 32 * 32, last = po.pos0 + (row0 + mix_rows < po.n ? row0 + mix_rows : po.n) - 1;

@@ -142,3 +142,15 @@ def test_queries_and_keys_that_are_not_finite(place, bad):
         assert torch.isnan(got[reads]).all()  # every head has a share of the bad one's weights
     else:  # a score of an infinity either way: all weight or none
         assert bool((~torch.isfinite(got[reads])).any())
+
+
+def test_a_block_table_that_ends_before_the_last_key():
+    """The rows whose keys the table does not reach have no result, the others theirs; nothing is refused."""
+    from cwm_amd import ops
+
+    for new in (40, 200):
+        q, cache, table, batch, scale, sink, mix, want = _talking_case(torch.bfloat16, 8, 4, 64, 32, [100], [new], None, seed=6)
+        whole = ops.talking_attention(q, cache, table, batch, None, scale, sink=sink, talk=mix)
+        pages = 4  # keys 0..127: rows 0..27
+        got = ops.talking_attention(q, cache, table[:, :pages].contiguous(), batch, None, scale, sink=sink, talk=mix)
+        assert torch.isnan(got[28:]).all() and torch.equal(got[:28], whole[:28])
