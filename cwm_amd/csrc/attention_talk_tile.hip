@@ -533,6 +533,7 @@ extern "C" int cwm_talking_tiles(const void* q, long q_stride, const void* cache
   CWM_REQUIRE(count >= 1 && count <= TILE_PORTIONS && portions, "talking_tiles: %d portions in a launch", count);
   CWM_REQUIRE(page_size > 0 && page_size % TILE_KEYS == 0 && num_pages > 0 && table_width > 0, "talking_tiles: bad cache sizes");
   CWM_REQUIRE(q && cache && block_table && talk && stats && weights && out, "talking_tiles: arguments missing");
+  CWM_REQUIRE(scale > 0.f, "talking_tiles: the maxima are those of unscaled scores, which takes a positive scale");
   CWM_REQUIRE(q_stride % 8 == 0 && ((uintptr_t)q % 16) == 0 && ((uintptr_t)cache % 16) == 0 && ((uintptr_t)out % 8) == 0 && ((uintptr_t)weights % 16) == 0,
               "talking_tiles: rows must be 16-byte aligned");
   const int per = n_q_heads / n_kv_heads, together = per <= 4 ? per : per % 3 == 0 ? 3 : 4;  // heads of a block of the first and the third kernel

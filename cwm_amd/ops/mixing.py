@@ -174,7 +174,7 @@ def talking_attention(
     else:
         q_lens, kv_lens = batch.q_lens, batch.kv_lens
         tiled = (
-            q.dtype == torch.bfloat16 and talk is not None and cache.shape[3] // hd % TALK_TILE_KEYS == 0 and q.data_ptr() % 16 == 0
+            q.dtype == torch.bfloat16 and talk is not None and scale > 0 and cache.shape[3] // hd % TALK_TILE_KEYS == 0 and q.data_ptr() % 16 == 0
             and cache.data_ptr() % 16 == 0 and (q.stride(0) % 8 == 0 or n_tokens == 1) and _talk_tiles_built(n_q, n_kv, hd)
         )
         from_tokens = TALK_TILE_FROM if tiled else TALK_LONG_ROWS

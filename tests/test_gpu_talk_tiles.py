@@ -154,3 +154,16 @@ def test_a_block_table_that_ends_before_the_last_key():
         pages = 4  # keys 0..127: rows 0..27
         got = ops.talking_attention(q, cache, table[:, :pages].contiguous(), batch, None, scale, sink=sink, talk=mix)
         assert torch.isnan(got[28:]).all() and torch.equal(got[:28], whole[:28])
+
+
+@pytest.mark.parametrize("new", [20, 150])
+def test_scales_that_are_not_positive(new):
+    """Scores of minus the scale are those of minus the queries; a scale of zero gives all keys the same score."""
+    from cwm_amd import ops
+
+    q, cache, table, batch, scale, sink, mix, want = _talking_case(torch.bfloat16, 8, 4, 64, 32, [100], [new], 60, seed=7)
+    got = ops.talking_attention(-q, cache, table, batch, 60, -scale, sink=sink, talk=mix).cpu().double()
+    torch.testing.assert_close(got, want, rtol=3e-2, atol=3e-2)
+    none = ops.talking_attention(q, cache, table, batch, 60, 0.0, sink=sink, talk=mix)
+    zero = ops.talking_attention(torch.zeros_like(q), cache, table, batch, 60, scale, sink=sink, talk=mix)
+    torch.testing.assert_close(none.float(), zero.float(), rtol=2 ** -6, atol=2 ** -6)  # bfloat16 weights and results
