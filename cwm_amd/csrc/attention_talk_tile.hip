@@ -502,6 +502,14 @@ static int tile_steps(const TalkPortion& po, int row0, int rows, int window_left
   const int first = po.pos0 + row0, last = po.pos0 + (row0 + rows < po.n ? row0 + rows : po.n) - 1;
   return last / TILE_KEYS - (window_left >= 0 && first > window_left ? first - window_left : 0) / TILE_KEYS + 1;
 }
+// heads of a block of the first and the third kernel
+static int tile_heads_together(int per) { return per <= 4 ? per : per % 3 == 0 ? 3 : 4; }
+// blocks of those kernels for a tile of rows; 0: sizes there are no kernels for
+extern "C" int cwm_talking_tile_groups(int n_q_heads, int n_kv_heads, int head_dim) {
+  if (cwm_talking_tile_heads(n_q_heads, n_kv_heads, head_dim) == 0) return 0;
+  const int per = n_q_heads / n_kv_heads, together = tile_heads_together(per);
+  return n_kv_heads * ((per + together - 1) / together);
+}
 extern "C" int cwm_talking_tile_portions() { return TILE_PORTIONS; }
 
 // Steps of a block of the second kernel.  No sum goes from one step to the next, so they may be cut anywhere: where rounds of 224
@@ -536,8 +544,8 @@ extern "C" int cwm_talking_tiles(const void* q, long q_stride, const void* cache
   CWM_REQUIRE(scale > 0.f, "talking_tiles: the maxima are those of unscaled scores, which takes a positive scale");
   CWM_REQUIRE(q_stride % 8 == 0 && ((uintptr_t)q % 16) == 0 && ((uintptr_t)cache % 16) == 0 && ((uintptr_t)out % 8) == 0 && ((uintptr_t)weights % 16) == 0,
               "talking_tiles: rows must be 16-byte aligned");
-  const int per = n_q_heads / n_kv_heads, together = per <= 4 ? per : per % 3 == 0 ? 3 : 4;  // heads of a block of the first and the third kernel
-  const int mix_rows = n_q_heads <= 16 ? 32 : 16, value_rows = together <= 2 ? 32 : 16, groups = n_kv_heads * ((per + together - 1) / together);
+  const int per = n_q_heads / n_kv_heads, together = tile_heads_together(per);
+  const int mix_rows = n_q_heads <= 16 ? 32 : 16, value_rows = together <= 2 ? 32 : 16, groups = cwm_talking_tile_groups(n_q_heads, n_kv_heads, head_dim);
   TalkPortions P;
   P.count = count;
   long blocks[3] = {0, 0, 0}, at = 0;

@@ -73,18 +73,43 @@ def _talking_long(q_rows, out_rows, cache, table_row, pos0, window, scale, sink,
         out_rows[r0:r1] = mixed.reshape(n_kv, m, per, hd).permute(1, 0, 2, 3).reshape(m, n_q * hd)
 
 
-# Tokens of a portion from which, where `csrc/attention_talk_tile.hip` has kernels for the model's heads, no table of scores is made (16
-# heads of 128, us through the table and without: 16 tokens after 2,000 84 and 53, after none 33 and 24, after 30,000 731 and 415; 8 tokens
-# after 2,000 63 and 50, 2 of them 47 and 49; portions of 128 and more, whose scores were a library's products: 1,500 214 and 81,
-# 130 100 and 31, 4,096 after 4,096 2,000 and 1,160; 24 heads, 1,500 tokens 333 and 129).
+# Tokens of a portion from which it may go without a table of scores, where `csrc/attention_talk_tile.hip` has kernels for the model's heads
 TALK_TILE_FROM = 16
 TALK_TILE_KEYS = 32  # csrc/attention_talk_tile.hip: TILE_KEYS, of which a page holds a multiple, and rows of a tile
 TALK_TABLE_BYTES = 1 << 28  # most of a launch's table of mixed weights, where a tile of rows needs no more
 
 
 @functools.cache
+def _talk_tile_groups(n_q: int, n_kv: int, hd: int) -> int:
+    """Blocks of the tiles' first and third kernel for a tile of rows (each walks its keys alone); 0: no kernels for these heads."""
+    return _build.load("attention_talk_tile").cwm_talking_tile_groups(ctypes.c_int(n_q), ctypes.c_int(n_kv), ctypes.c_int(hd))
+
+
 def _talk_tiles_built(n_q: int, n_kv: int, hd: int) -> bool:
-    return _build.load("attention_talk_tile").cwm_talking_tile_heads(ctypes.c_int(n_q), ctypes.c_int(n_kv), ctypes.c_int(hd)) > 0
+    return _talk_tile_groups(n_q, n_kv, hd) > 0
+
+
+def talk_tiles_take(tokens: int, keys: int, groups: int, n_q: int, n_kv: int, hd: int) -> bool:
+    """Whether a portion of `tokens` tokens, a row of which reads up to `keys` keys, makes no table of scores; its own sizes alone
+    decide, so that its bits do not hang on the rest of the step.  A block of the tiles' kernels walks all keys of its 32 rows, so the table
+    (whose ranges of keys are blocks of their own) and the library's products are ahead where few blocks walk many keys.
+
+    us through the table or the library and in tiles, tokens after a context, heads of 128: 16 heads on 8, 16 after 2,000 81 and 52, 1,500 after
+    none 207 and 78, 4,096 after none 824 and 455, 130 after none 40 and 29, but 1,024 after 30,000 2,295 and 2,670; 32 on 8, 1,500 after none 484 and 158;
+    16 on 4 (half the blocks), 16 after 4,000 13% more in tiles, 64 after 1,000 38% less, 128 after 4,000 24% more, 512 after 4,000 17% less;
+    8 on 1 (a quarter), 16 after 4,000 60% more, 64 after 4,000 12% less, 512 after none 27% more, 2,048 after 1,000 38% less; 8 on 8, 128 after
+    4,000 6% less, after 6,000 13% more."""
+    if groups == 0 or tokens < TALK_TILE_FROM:
+        return False
+    if tokens < TALK_LONG_ROWS:
+        return tokens * groups >= 128 and (groups >= 6 or (tokens >= 64 and keys >= 128))
+    if keys * hd > (1 << 21 if groups >= 8 and n_q >= 24 else 1 << 19 if n_q < 16 and tokens < 512 else 1 << 20):
+        return False
+    if groups >= 6:
+        return True
+    if groups >= 4 and n_kv > 1:
+        return tokens >= 512 or (hd == 64 and keys <= 4224)
+    return tokens >= 2048 and n_q > 1
 
 
 def _talking_tiles(q, out, cache, block_table, portions, window, scale, sink, talk) -> None:
@@ -141,7 +166,7 @@ def talking_attention(
     None; `talk`: float32 [Hq, Hq] or None (no mixing).  `batch`: the step's descriptor (positions, sequence of each
     token, `cu_q`, `kv_len` and the host's `q_lens`, `kv_lens`).  Scores and weights of the step go through a table in
     float32 (`csrc/attention_talk.hip`); portions of `TALK_LONG_ROWS` tokens and more in bfloat16 take the scores and the
-    weighted values as matrix products instead, portions of `TALK_TILE_FROM` and more of most heads' sizes have no table of scores at all
+    weighted values as matrix products instead, those that `talk_tiles_take` names have no table of scores at all
     (`csrc/attention_talk_tile.hip`).  Returns [T, Hq * hd] in the type of `q`."""
     KernelError, _check, _code, _i32, _need_gpu, _ptr, _stream = _base()
     _need_gpu(q, cache, block_table, sink, talk)
@@ -175,18 +200,24 @@ def talking_attention(
         q_lens, kv_lens = batch.q_lens, batch.kv_lens
         tiled = (
             q.dtype == torch.bfloat16 and talk is not None and scale > 0 and cache.shape[3] // hd % TALK_TILE_KEYS == 0 and q.data_ptr() % 16 == 0
-            and cache.data_ptr() % 16 == 0 and (q.stride(0) % 8 == 0 or n_tokens == 1) and _talk_tiles_built(n_q, n_kv, hd)
+            and cache.data_ptr() % 16 == 0 and (q.stride(0) % 8 == 0 or n_tokens == 1)
         )
-        from_tokens = TALK_TILE_FROM if tiled else TALK_LONG_ROWS
-        long = [b for b, n in enumerate(q_lens) if n >= from_tokens] if q.dtype == torch.bfloat16 else []
+        tiles = []
+        if tiled and max(q_lens, default=0) >= TALK_TILE_FROM:
+            groups = _talk_tile_groups(n_q, n_kv, hd)
+            most = max(kv_lens) if window is None else window - 1 + TALK_TILE_KEYS
+            tiles = [b for b, n in enumerate(q_lens) if talk_tiles_take(n, min(kv_lens[b], most), groups, n_q, n_kv, hd)]
+        long = [b for b, n in enumerate(q_lens) if n >= TALK_LONG_ROWS or b in tiles] if q.dtype == torch.bfloat16 else []
         if long:
             out = torch.empty((n_tokens, width), dtype=q.dtype, device=q.device)
             starts = [0]
             for n in q_lens:
                 starts.append(starts[-1] + n)
-            if tiled:
-                _talking_tiles(q, out, cache, block_table, [(b, starts[b], q_lens[b], kv_lens[b] - q_lens[b]) for b in long], window, scale, sink, talk)
-            for b in () if tiled else long:
+            if tiles:
+                _talking_tiles(q, out, cache, block_table, [(b, starts[b], q_lens[b], kv_lens[b] - q_lens[b]) for b in tiles], window, scale, sink, talk)
+            for b in long:
+                if b in tiles:
+                    continue
                 t0, t1 = starts[b], starts[b + 1]
                 _talking_long(q[t0:t1], out[t0:t1], cache, block_table[b], kv_lens[b] - q_lens[b], window, scale, sink, talk, lib)
             rest = [t for b, n in enumerate(q_lens) if b not in long for t in range(starts[b], starts[b] + n)]

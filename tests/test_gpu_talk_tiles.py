@@ -11,6 +11,14 @@ from test_gpu_digasun import DEV, _talking_case
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def every_portion_in_tiles(monkeypatch):
+    """Sizes that the rule leaves to the table of scores and the library's products as well."""
+    from cwm_amd.ops import mixing
+
+    monkeypatch.setattr(mixing, "talk_tiles_take", lambda tokens, keys, groups, n_q, n_kv, hd: groups > 0 and tokens >= mixing.TALK_TILE_FROM)
+
+
 def _bound(case, window):
     """What the kernels' roundings can add up to, float64 [T, H * hd]: the mixed weights and the result in bfloat16 (seven bits after
     the first: half of the last is at most 2^-8 of the value) and, far below them, float32 scores, exponentials and sums (2^-15 of the unmixed weights' size)."""
