@@ -10,6 +10,7 @@
 // `round_inputs`: x and g are rounded to bfloat16 before they enter their products, as a model does
 // that keeps its activations in bfloat16; the sums, the activation and the norm are float32 either way.
 #include "common.h"
+#include <type_traits>
 
 CWM_DEFINE_ERROR_API
 
@@ -218,23 +219,33 @@ token_side_kernel(float* __restrict__ h, const int* __restrict__ tokens, const T
 // gate's product (16 tokens x side_dim, K = dim) is split over the wavefronts by columns and K, whose parts meet in LDS; the
 // projection's (16 x dim, K = side_dim) by columns.  w_proj is [dim, side_dim] here.  The kernel above is bound by its
 // multiply-adds and by LDS (every product's x and gated value is a read of its own): of width 2,048 with 64 side values and two
-// addends, 1,500 tokens take it 88 us; here 24.  A block's stages follow one another (rows 4 us, gate's product 6, projection 5, each bound
+// addends, 1,500 tokens take it 88 us; here 21.  A block's stages follow one another (rows, gate's product, projection, each bound
 // by its loads), so what can be asked for before a stage is: the tokens' values and the gate's first weights before the rows, the projection's
 // before the gate's sums, the norm's before the squares; a row's pieces four at a time; the rows stay in LDS in float32 and are
-// written once.  (38 us with a piece at a time, rows written and read again, and operands fetched a row a lane.)
+// written once.  (38 us with a piece at a time, rows written and read again, and operands fetched a row a lane.)  Sixteen tokens a block, whose
+// rows are bfloat16 in LDS and lie in the residual meanwhile: a token's sums have one order whatever TOK is.  Builds for short rows have no more
+// loads than such a row has pieces and steps: a build for 2,048 took 256 tokens of width 512 12.1 us, of width 64 10.7, these 8.3 and 6.0.
 // dim: a multiple of 64 and at most 256 MAXT; side_dim: a multiple of 32, at most SIDE_TILE_MAX; rows of h, the addends and the
 // norm's weight start at multiples of 16 bytes (bfloat16 addends: of 8).
 #define SIDE_TILE_MAX 128
-#define SIDE_AHEAD 8  // steps of the gate's product whose weights are in flight
-#define SIDE_RUN 4    // pieces of a row that a thread has in flight
-#define SIDE_TURN_ROW 80  // bytes between a turned operand's rows of 64: no bank twice
-#define SIDE_TURN_BYTES (16 * SIDE_TURN_ROW)
-// bytes of LDS for TOK tokens a block
-static inline size_t side_tile_lds(int tok, int dim) {
-  const int waves = SIDE_THREADS / CWM_WAVE;
-  return (size_t)tok * (dim + 4) * sizeof(float) + (size_t)waves * 16 * tok * sizeof(float) + (size_t)tok * (SIDE_TILE_MAX + 8) * 2 + (size_t)waves * tok * sizeof(float) +
-         (size_t)waves * 2 * SIDE_TURN_BYTES;
+#define SIDE_TURN_BYTES 1024  // an operand of 16 rows of 64 bytes
+// bytes of LDS for `tok` tokens a block, whose rows stay there in float32 (`kept`) or, of bfloat16, for the gate's product alone
+static inline size_t side_tile_lds(int tok, int dim, bool kept) {
+  const int waves = SIDE_THREADS / CWM_WAVE, parts = 16 * tok * (int)sizeof(float);
+  return (size_t)tok * (kept ? (dim + 4) * sizeof(float) : (dim + 8) * sizeof(bf16_t)) + (size_t)waves * (parts > SIDE_TURN_BYTES ? parts : SIDE_TURN_BYTES) +
+         (size_t)tok * (SIDE_TILE_MAX + 8) * 2 + (size_t)waves * tok * sizeof(float);
 }
+
+// Tokens a block.  A block has a compute unit to itself beyond rows of 1,024 elements, so sixteen where eight would need a second round of blocks
+// (64 side values, us with eight and sixteen: 2,500 tokens of width 1,024 28 and 19, of 2,048 42 and 31, of 4,096 82 and 57; 8,192 of 2,048 94 and
+// 83), but not where three short rounds are less than two long ones (32 side values, 5,000 tokens of width 2,048 49 and 56); of the widest rows four
+// where eight would leave more than half the chip idle (256 tokens of width 4,096 24.4 and 26.9; 1,000 tokens 35.3 and 36).
+extern "C" int cwm_token_side_tile_tokens(int n_tokens, int dim, int side_dim) {
+  if (side_dim <= 32 && dim > 1024 && n_tokens > 16 * 256 && n_tokens <= 24 * 256) return 8;
+  if (n_tokens > 8 * 256) return 16;
+  return dim > 3456 && n_tokens <= 4 * 256 ? 4 : 8;
+}
+extern "C" long cwm_token_side_tile_lds(int tok, int dim) { return (long)side_tile_lds(tok, dim, tok < 16); }
 
 template <int TOK, int MAXT>
 __device__ __forceinline__ void
@@ -243,23 +254,30 @@ token_side_tile(const int block, float* __restrict__ h, const int* __restrict__ 
                        int dim, int side_dim, int vocab, float eps, SideAddends addends, SidePortions portions) {
   extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
   constexpr int WAVES = SIDE_THREADS / CWM_WAVE, A_TOKEN = WAVES / TOK;  // wavefronts that load a token's row
+  constexpr int AHEAD = MAXT <= 2 ? 2 * MAXT : MAXT == 4 && TOK == 16 ? 4 : 8;  // steps of the gate's product whose weights are in flight
+  constexpr int RUN = MAXT <= 2 ? (MAXT * TOK + 15) / 16 : MAXT == 4 && TOK == 16 ? 2 : 4;  // pieces of a row that a thread has in flight
   constexpr int GATED = TOK * SIDE_TILE_MAX / SIDE_THREADS > 1 ? TOK * SIDE_TILE_MAX / SIDE_THREADS : 1;  // gated values a thread makes at most
-  const int x_ld = dim + 4;
-  float* xs = (float*)tile_lds;                                  // [TOK][x_ld]
-  float* parts = xs + (size_t)TOK * x_ld;                        // [WAVES][16 side values][TOK]
-  bf16_t* gated = (bf16_t*)(parts + WAVES * 16 * TOK);           // [TOK][SIDE_TILE_MAX + 8]
+  constexpr bool KEPT = TOK < 16;  // sixteen rows of float32 are more than the LDS holds
+  typedef std::conditional_t<KEPT, float, bf16_t> Row;
+  const int x_ld = dim + (KEPT ? 4 : 8);
+  Row* xs = (Row*)tile_lds;                                      // [TOK][x_ld]
+  // a wavefront's part of the gate's product, [16 side values][TOK], where its operands are turned before and after
+  constexpr int PART = 16 * TOK * 4 > SIDE_TURN_BYTES ? 16 * TOK : SIDE_TURN_BYTES / 4;
+  float* parts = (float*)(xs + (size_t)TOK * x_ld);
+  bf16_t* gated = (bf16_t*)(parts + WAVES * PART);               // [TOK][SIDE_TILE_MAX + 8]
   float* squares = (float*)(gated + TOK * (SIDE_TILE_MAX + 8));  // [WAVES][TOK]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, j = lane >> 4;
   // A weight operand of 16 rows and 32 values is fetched four lanes a row (64 consecutive bytes) and turned to a lane's row through a place of
-  // the wavefront's own in LDS: fetched as the instruction takes it, neighbouring lanes lie in 16 rows, which costs a lookup a lane.
-  unsigned char* turn = (unsigned char*)(squares + WAVES * TOK) + wave * 2 * SIDE_TURN_BYTES;
+  // the wavefront's own in LDS: fetched as the instruction takes it, neighbouring lanes lie in 16 rows, which costs a lookup a lane.  A row's
+  // four pieces change places with the row, so that no bank is met twice.
+  unsigned char* turn = (unsigned char*)(parts + wave * PART);
   const int turn_row = lane >> 2, turn_piece = lane & 3;
-  auto turned = [&](uint4 w, int slot) {
+  auto turned = [&](uint4 w) {
     Frag8 f;
     __builtin_amdgcn_wave_barrier();
-    *(uint4*)(turn + slot * SIDE_TURN_BYTES + turn_row * SIDE_TURN_ROW + turn_piece * 16) = w;
+    *(uint4*)(turn + turn_row * 64 + (turn_piece ^ (turn_row >> 2)) * 16) = w;
     __builtin_amdgcn_wave_barrier();
-    f.u = *(const uint4*)(turn + slot * SIDE_TURN_BYTES + r * SIDE_TURN_ROW + j * 16);
+    f.u = *(const uint4*)(turn + r * 64 + (j ^ (r >> 2)) * 16);
     __builtin_amdgcn_wave_barrier();
     return f;
   };
@@ -290,88 +308,101 @@ token_side_tile(const int block, float* __restrict__ h, const int* __restrict__ 
   const int gate_from = min(gate_part * part_steps, steps - 1);
   const int gate_count = gate_part < k_parts ? max(min(part_steps, steps - gate_part * part_steps), 0) : 0;  // wavefronts left over have no part
   const int gate_start = gate_count > 0 ? 4 * gate_column % gate_count : 0;
-  auto gate_step = [&](int u) {  // the u-th of the wavefront's steps; past the last: the last once more
-    const int v = min(u, max(gate_count - 1, 0)) + gate_start;
-    return gate_from + (v >= gate_count ? max(v - gate_count, 0) : v);
+  auto gate_step = [&](int u) {  // the u-th of the wavefront's steps
+    const int v = u + gate_start;
+    return gate_from + (v >= gate_count ? v - gate_count : v);
   };
   const bf16_t* gate_row = w_gate + (size_t)(16 * gate_column + turn_row) * dim + 8 * turn_piece;
-  uint4 gate_w[SIDE_AHEAD];
+  uint4 gate_w[AHEAD];
   auto fetch_gate = [&](int first) {
 #pragma unroll
-    for (int u = 0; u < SIDE_AHEAD; ++u) gate_w[u] = *(const uint4*)(gate_row + 32 * gate_step(first + u));
+    for (int u = 0; u < AHEAD; ++u)
+      if (first + u < gate_count) gate_w[u] = *(const uint4*)(gate_row + 32 * gate_step(first + u));
   };
   fetch_gate(0);
   // 1. the rows: pending addends onto the residual, into LDS
   {
     const int tok = wave / A_TOKEN, t = t0 + tok;
     const bool serve = portions.serves(t, n_tokens, true);
-    float* x_row = xs + (size_t)tok * x_ld;
+    Row* x_row = xs + (size_t)tok * x_ld;
     const int e0 = 4 * ((wave % A_TOKEN) * CWM_WAVE + lane);
-    for (int at = e0; at < dim; at += SIDE_RUN * 4 * CWM_WAVE * A_TOKEN) {
-      float4v x[SIDE_RUN];
-      int e[SIDE_RUN];
+    for (int at = e0; at < dim; at += RUN * 4 * CWM_WAVE * A_TOKEN) {
+      float4v x[RUN];
+      int e[RUN];
 #pragma unroll
-      for (int u = 0; u < SIDE_RUN; ++u) {
+      for (int u = 0; u < RUN; ++u) {
         e[u] = min(at + u * 4 * CWM_WAVE * A_TOKEN, dim - 4);  // a piece past the end: the row's last once more
         x[u] = (float4v){0.f, 0.f, 0.f, 0.f};
       }
       if (serve) {
 #pragma unroll
-        for (int u = 0; u < SIDE_RUN; ++u) x[u] = *(const float4v*)(h + (size_t)t * dim + e[u]);
+        for (int u = 0; u < RUN; ++u) x[u] = *(const float4v*)(h + (size_t)t * dim + e[u]);
         for (int a = 0; a < addends.n; ++a) {
           const SideAddend& ad = addends.a[a];
-          float4v y[SIDE_RUN];
+          float4v y[RUN];
 #pragma unroll
-          for (int u = 0; u < SIDE_RUN; ++u) y[u] = (float4v){0.f, 0.f, 0.f, 0.f};
+          for (int u = 0; u < RUN; ++u) y[u] = (float4v){0.f, 0.f, 0.f, 0.f};
           if (ad.dtype == CWM_F32) {
             for (int p = 0; p < ad.n_partials; ++p) {
               const float* from = (const float*)ad.ptr + (size_t)p * ad.partial_stride + (size_t)t * ad.ld;
 #pragma unroll
-              for (int u = 0; u < SIDE_RUN; ++u) y[u] += *(const float4v*)(from + e[u]);
+              for (int u = 0; u < RUN; ++u) y[u] += *(const float4v*)(from + e[u]);
             }
           } else {
             const bf16_t* from = (const bf16_t*)ad.ptr + (size_t)t * ad.ld;
-            uint2 w[SIDE_RUN];
+            uint2 w[RUN];
 #pragma unroll
-            for (int u = 0; u < SIDE_RUN; ++u) w[u] = *(const uint2*)(from + e[u]);
+            for (int u = 0; u < RUN; ++u) w[u] = *(const uint2*)(from + e[u]);
 #pragma unroll
-            for (int u = 0; u < SIDE_RUN; ++u)
+            for (int u = 0; u < RUN; ++u)
               y[u] += (float4v){__uint_as_float(w[u].x << 16), __uint_as_float(w[u].x & 0xffff0000u), __uint_as_float(w[u].y << 16), __uint_as_float(w[u].y & 0xffff0000u)};
           }
 #pragma unroll
-          for (int u = 0; u < SIDE_RUN; ++u)
+          for (int u = 0; u < RUN; ++u)
 #pragma unroll
             for (int i = 0; i < 4; ++i) x[u][i] = fmaf(ad.scale, y[u][i], x[u][i]);
         }
       }
 #pragma unroll
-      for (int u = 0; u < SIDE_RUN; ++u) *(float4v*)(x_row + e[u]) = x[u];
+      for (int u = 0; u < RUN; ++u) {
+        if constexpr (KEPT) {
+          *(float4v*)(x_row + e[u]) = x[u];
+        } else {
+          if (at + u * 4 * CWM_WAVE * A_TOKEN >= dim) continue;  // (the row's last piece may have been written by its own thread before it was read here)
+          if (serve && addends.n > 0) *(float4v*)(h + (size_t)t * dim + e[u]) = x[u];  // read again at the end, after the block's barriers
+          *(uint2*)(x_row + e[u]) = make_uint2(pack2_bf16(x[u][0], x[u][1]), pack2_bf16(x[u][2], x[u][3]));
+        }
+      }
     }
   }
   __syncthreads();
   // 2. the gate's product
   {
     float4v acc = {0.f, 0.f, 0.f, 0.f};
-    const float* x_row = xs + (size_t)min(r, TOK - 1) * x_ld + 8 * j;
-    for (int first = 0; first < gate_count; first += SIDE_AHEAD) {
-      uint4 now[SIDE_AHEAD];
+    const Row* x_row = xs + (size_t)min(r, TOK - 1) * x_ld + 8 * j;
+    for (int first = 0; first < gate_count; first += AHEAD) {
+      uint4 now[AHEAD];
 #pragma unroll
-      for (int u = 0; u < SIDE_AHEAD; ++u) now[u] = gate_w[u];
-      fetch_gate(first + SIDE_AHEAD);
+      for (int u = 0; u < AHEAD; ++u) now[u] = gate_w[u];
+      fetch_gate(first + AHEAD);
 #pragma unroll
-      for (int u = 0; u < SIDE_AHEAD; ++u) {
+      for (int u = 0; u < AHEAD; ++u) {
         const int s = gate_step(first + u);
         if (first + u < gate_count) {
-          const float4v a = *(const float4v*)(x_row + 32 * s), b = *(const float4v*)(x_row + 32 * s + 4);
           Frag8 fx;
-          fx.u = make_uint4(pack2_bf16(a[0], a[1]), pack2_bf16(a[2], a[3]), pack2_bf16(b[0], b[1]), pack2_bf16(b[2], b[3]));
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(turned(now[u], u & 1).v, fx.v, acc, 0, 0, 0);
+          if constexpr (KEPT) {
+            const float4v a = *(const float4v*)(x_row + 32 * s), b = *(const float4v*)(x_row + 32 * s + 4);
+            fx.u = make_uint4(pack2_bf16(a[0], a[1]), pack2_bf16(a[2], a[3]), pack2_bf16(b[0], b[1]), pack2_bf16(b[2], b[3]));
+          } else {
+            fx.u = *(const uint4*)(x_row + 32 * s);
+          }
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(turned(now[u]).v, fx.v, acc, 0, 0, 0);
         }
       }
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (r < TOK) parts[(wave * 16 + 4 * j + i) * TOK + r] = acc[i];
+      if (r < TOK) parts[wave * PART + (4 * j + i) * TOK + r] = acc[i];
   }
   // the projection: wavefront w has the tiles w, w + 16, ... of 16 elements; its first weights are on their way past the barriers
   // (eight tiles at a time: with sixteen tiles' weights and results both in registers they spill)
@@ -391,7 +422,7 @@ token_side_tile(const int block, float* __restrict__ h, const int* __restrict__ 
     if (id < TOK * side_dim) {
       const int tok = id % TOK, k = id / TOK;
       float sum = 0.f;
-      for (int part = 0; part < k_parts; ++part) sum += parts[((part * columns + k / 16) * 16 + k % 16) * TOK + tok];
+      for (int part = 0; part < k_parts; ++part) sum += parts[(part * columns + k / 16) * PART + k % 16 * TOK + tok];
       const float z = side_round(sum, true);
       const float gelu = 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
       gated[tok * (SIDE_TILE_MAX + 8) + k] = f32_to_bf16(gelu * own[u]);
@@ -409,7 +440,7 @@ token_side_tile(const int block, float* __restrict__ h, const int* __restrict__ 
       fg.u = *(const uint4*)(gated + min(r, TOK - 1) * (SIDE_TILE_MAX + 8) + k + 8 * j);
 #pragma unroll
       for (int q = 0; q < GROUP; ++q)
-        if (16 * ((q0 + q) * WAVES + wave) < dim) y[q0 + q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(turned(proj_w[q], q & 1).v, fg.v, y[q0 + q], 0, 0, 0);
+        if (16 * ((q0 + q) * WAVES + wave) < dim) y[q0 + q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(turned(proj_w[q]).v, fg.v, y[q0 + q], 0, 0, 0);
       const bool more = k + 32 < side_dim;
       fetch_proj(more ? q0 : min(q0 + GROUP, MAXT - GROUP), more ? k + 32 : 0);
     }
@@ -425,12 +456,14 @@ token_side_tile(const int block, float* __restrict__ h, const int* __restrict__ 
 #pragma unroll
   for (int q = 0; q < GROUP; ++q) norm[q] = *(const float4v*)(weight + min(16 * (q * WAVES + wave), dim - 16) + 4 * j);
   __syncthreads();
-  if (r < TOK) {
+  if (r < TOK && (KEPT || portions.serves(t0 + r, n_tokens, true))) {
     float total = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) total += squares[w * TOK + r];
     const float rstd = 1.0f / sqrtf(total / (float)dim + eps);
-    float* x_row = xs + (size_t)r * x_ld;
+    float* x_row;  // the row before the input: in LDS, or where the first stage has left it
+    if constexpr (KEPT) x_row = xs + (size_t)r * x_ld;
+    else x_row = h + (size_t)(t0 + r) * dim;
 #pragma unroll
     for (int q = 0; q < MAXT; ++q) {
       const int e = 16 * (q * WAVES + wave) + 4 * j;
@@ -443,12 +476,13 @@ token_side_tile(const int block, float* __restrict__ h, const int* __restrict__ 
       }
     }
   }
+  if constexpr (!KEPT) return;
   __syncthreads();
   // whole rows, a wavefront 1 KB at a time
   const int tok = wave / A_TOKEN, t = t0 + tok;
   if (!portions.serves(t, n_tokens, true)) return;
   for (int e = 4 * ((wave % A_TOKEN) * CWM_WAVE + lane); e < dim; e += 4 * CWM_WAVE * A_TOKEN)
-    *(float4v*)(h + (size_t)t * dim + e) = *(const float4v*)(xs + (size_t)tok * x_ld + e);
+    *(float4v*)(h + (size_t)t * dim + e) = *(const float4v*)((const float*)xs + (size_t)tok * x_ld + e);
 }
 
 template <int TOK, int MAXT>
@@ -460,8 +494,8 @@ token_side_tile_kernel(float* __restrict__ h, const int* __restrict__ tokens, co
 }
 
 // Both in one launch, for a step whose short portions hold few tokens: the first `tile_blocks` blocks take the long portions' tokens,
-// then a block a token the short ones', beside them and not behind them.  1,006 and 48 tokens of width 3,072: 52 us, as the
-// tiles alone; a second launch of four tokens a block took 63 more.
+// then a block a token the short ones', beside them and not behind them.  1,006 and 48 tokens of width 3,072: 29.9 us,
+// 28.1 of them the tiles alone; two launches 51.7.
 #define SIDE_FEW 128
 template <int TOK, int MAXT>
 __global__ void __launch_bounds__(SIDE_THREADS)
@@ -503,21 +537,21 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
     CWM_REQUIRE(n_partials[a] == 1 || dtypes[a] == CWM_F32, "token_side: partial sums must be float32");
     ad.a[a] = SideAddend{ptrs[a], lds_[a], partial_strides[a], n_partials[a], dtypes[a], scales[a]};
   }
-  // portions from SIDE_TILE_FROM tokens on (32 blocks of eight): with fewer the other kernel's blocks of one or two tokens spread over more of the chip
-  // (8 to 48 tokens of width 2,048: 19 us against 30; 300 tokens 44 against 31)
+  // portions from SIDE_TILE_FROM tokens on (32 blocks of eight): with few the other kernel's blocks of one or two tokens spread over more of the chip (8 to
+  // 64 tokens of width 2,048: 14.2 to 14.6 us against 15.8 to 16.1 in tiles; 128 to 255 tokens 21.9 to 22.5 against 16.3 to 16.6, so the line could lie
+  // at 128; 300 tokens 40 against 16.7)
   bool tiled = n_tokens >= SIDE_TILE_FROM && w_proj && w_dtype == CWM_BF16 && round_inputs && dim % 64 == 0 && dim <= 4096 && side_dim % 32 == 0 && side_dim <= SIDE_TILE_MAX &&
                (((uintptr_t)h | (uintptr_t)w_gate | (uintptr_t)w_proj | (uintptr_t)weight) % 16) == 0;
   for (int a = 0; a < n_addends; ++a)
     tiled = tiled && lds_[a] % 4 == 0 && partial_strides[a] % 4 == 0 && ((uintptr_t)ptrs[a] % (dtypes[a] == CWM_F32 ? 16 : 8)) == 0;
   const SidePortions portions = {tiled ? seq_of_token : nullptr, cu_q};
   if (tiled) {
-    // eight tokens a block where their rows fit the LDS (up to 3,456 elements), else four
-    const int tok = side_tile_lds(8, dim) <= 163840 ? 8 : 4;
-    const size_t lds_tile = side_tile_lds(tok, dim);
+    const int tok = cwm_token_side_tile_tokens(n_tokens, dim, side_dim);
+    const size_t lds_tile = side_tile_lds(tok, dim, tok < 16);
     const bool both = seq_of_token && n_few < SIDE_FEW;
     const size_t lds_row = sizeof(float) * ((size_t)dim + side_dim), lds = both && lds_row > lds_tile ? lds_row : lds_tile;
     const int tile_blocks = (n_tokens + tok - 1) / tok;
-#define CWM_SIDE_TILE(TOK, MAXT)                                                                                                           \
+#define CWM_SIDE_TILE(TOK, MAXT)                                                                                                          \
   do {                                                                                                                                     \
     const void* kernel = both ? (const void*)token_side_both_kernel<TOK, MAXT> : (const void*)token_side_tile_kernel<TOK, MAXT>;           \
     if (lds > 65536) (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                              \
@@ -531,8 +565,16 @@ extern "C" int cwm_token_side(float* h, const int* tokens, const void* table, lo
                          side_dim, vocab, eps, ad, portions);                                                                              \
   } while (0)
     if (tok == 4) CWM_SIDE_TILE(4, 16);
-    else if (dim <= 2048) CWM_SIDE_TILE(8, 8);
-    else CWM_SIDE_TILE(8, 16);
+    else if (tok == 8 && dim <= 256) CWM_SIDE_TILE(8, 1);
+    else if (tok == 8 && dim <= 512) CWM_SIDE_TILE(8, 2);
+    else if (tok == 8 && dim <= 1024) CWM_SIDE_TILE(8, 4);
+    else if (tok == 8 && dim <= 2048) CWM_SIDE_TILE(8, 8);
+    else if (tok == 8) CWM_SIDE_TILE(8, 16);
+    else if (dim <= 256) CWM_SIDE_TILE(16, 1);
+    else if (dim <= 512) CWM_SIDE_TILE(16, 2);
+    else if (dim <= 1024) CWM_SIDE_TILE(16, 4);
+    else if (dim <= 2048) CWM_SIDE_TILE(16, 8);
+    else CWM_SIDE_TILE(16, 16);
 #undef CWM_SIDE_TILE
     if (!seq_of_token || both) return cwm_launch_status("token_side");
   }
