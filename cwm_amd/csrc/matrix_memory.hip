@@ -23,7 +23,7 @@
 // walk above, so both give the same m: 29 us for 1,531 tokens, 39 where a wavefront passed every gate through a scalar register) and sums f in float64, since differences of long sums are taken;
 // `memory_scores_kernel` works out every block's weighted scores and weights side by side, and `memory_chunk_kernel` (a thread
 // block a (tile of value columns, head, sequence or segment of a long one)) walks the blocks with the remaining products on the float32 matrix
-// instruction; bfloat16 rows have kernels of their own for both, on the bfloat16 instruction.  The normaliser n
+// instruction; bfloat16 rows of whole pieces of 16 bytes have kernels of their own for both, on the bfloat16 instruction.  The normaliser n
 // is the column after the last value column, with ones for values, so n_t . q_t falls out as that column's result and the
 // division moves into `memory_out_kernel`.  This differs from the walk by rounding only.
 //
@@ -321,9 +321,9 @@ __device__ __forceinline__ int memory_segment_of(int x, const int* __restrict__ 
 // scores: float32 [T][heads][MEMC_L], row t: (q_t . k_s) exp(a_s - g_t) for the sources s <= t of t's block, else 0;
 // wd: float32 [T][heads][2]: {exp(a_t - g_last), exp(g_c - g_t)}, the token's weight in the state after its block and
 // the weight of the state before its block in the token's result.
-template <int RPT>
+template <typename T, int RPT>
 __global__ void __launch_bounds__(MEMC_THREADS)
-memory_scores_kernel(const float* __restrict__ src, long src_stride, int q_off, int k_off, float q_scale, const float* __restrict__ coef,
+memory_scores_kernel(const T* __restrict__ src, long src_stride, int q_off, int k_off, float q_scale, const float* __restrict__ coef,
                      const double* __restrict__ start, const int* __restrict__ cu_q, int n_seqs, float* __restrict__ scores,
                      float* __restrict__ wd, int heads, int d) {
   constexpr int DP = MEMC_GROUPS * RPT, ROW = DP + 4;
@@ -340,8 +340,8 @@ memory_scores_kernel(const float* __restrict__ src, long src_stride, int q_off, 
     const int tok = x / DP, r = x - tok * DP;
     float qv = 0.f, kv = 0.f;
     if (tok < count && r < d) {
-      const float* row = src + (size_t)(base + tok) * src_stride + (size_t)h * d + r;
-      qv = row[q_off] * q_scale, kv = row[k_off];
+      const T* row = src + (size_t)(base + tok) * src_stride + (size_t)h * d + r;
+      qv = Elem<T>::load(row + q_off) * q_scale, kv = Elem<T>::load(row + k_off);
     }
     q_s[tok][r] = qv, k_s[tok][r] = kv;
   }
@@ -385,6 +385,9 @@ memory_scores_kernel(const float* __restrict__ src, long src_stride, int q_off, 
 
 typedef float memc_acc __attribute__((ext_vector_type(16)));
 
+__device__ __forceinline__ float raw_to_f32(float x) { return x; }
+__device__ __forceinline__ float raw_to_f32(bf16_t x) { return bf16_to_f32(x); }
+
 // A barrier that waits for the wavefront's LDS accesses only: __syncthreads() also waits for every global load on its
 // way, which here are the next block's rows, fetched early so that they arrive during this block's products.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); }
@@ -406,9 +409,9 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // v or zero, without a branch around what v is made of, which would wait for v's load alone.
 __device__ __forceinline__ float only(bool have, float v) { return __uint_as_float(__float_as_uint(v) & (have ? 0xffffffffu : 0u)); }
 
-template <int TILES, bool RESULTS>
+template <typename T, int TILES, bool RESULTS>
 __global__ void __launch_bounds__(CWM_WAVE * TILES)
-memory_chunk_kernel(const float* __restrict__ src, long src_stride, int q_off, int k_off, int v_off, float q_scale,
+memory_chunk_kernel(const T* __restrict__ src, long src_stride, int q_off, int k_off, int v_off, float q_scale,
                     const float* __restrict__ scores, const float* __restrict__ wd, float* __restrict__ state, long state_stride,
                     long head_elems, const int* __restrict__ cu_q, const int* __restrict__ state_slots, float* __restrict__ y,
                     float* __restrict__ nq, float* __restrict__ saved, int places, int n_seqs, int heads, int d, int e, int d_pad) {
@@ -458,7 +461,7 @@ memory_chunk_kernel(const float* __restrict__ src, long src_stride, int q_off, i
   // What a fetch leaves in registers is what the loads return and nothing made of it: an operation on a loaded value would
   // wait for the load where the fetch is issued, not where the value is staged.  Every load is issued, from an address that
   // exists; conversion, scale and the zeros beyond the portion's end or the head's size are applied when the block is staged.
-  float q_r[QK_REGS], k_r[QK_REGS], v_r[V_REGS];
+  T q_r[QK_REGS], k_r[QK_REGS], v_r[V_REGS];
   float a_r[V_REGS];
   float2 wd_r = make_float2(0.f, 0.f);
   auto fetch = [&](int base) {
@@ -466,7 +469,7 @@ memory_chunk_kernel(const float* __restrict__ src, long src_stride, int q_off, i
 #pragma unroll
     for (int u = 0; u < QK_REGS; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x / DP, r = x - tok * DP;
-      const float* row = src + (size_t)(base + min(tok, count - 1)) * src_stride + (size_t)h * d + min(r, d - 1);
+      const T* row = src + (size_t)(base + min(tok, count - 1)) * src_stride + (size_t)h * d + min(r, d - 1);
       if constexpr (RESULTS) q_r[u] = row[q_off];
       k_r[u] = row[k_off];
     }
@@ -487,13 +490,13 @@ memory_chunk_kernel(const float* __restrict__ src, long src_stride, int q_off, i
     for (int u = 0; u < QK_REGS; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x / DP, r = x - tok * DP;
       const bool live = tok < count && r < d;
-      if constexpr (RESULTS) q_s[tok][r] = only(live, q_r[u] * q_scale);
-      k_s[tok][r] = only(live, k_r[u]);
+      if constexpr (RESULTS) q_s[tok][r] = only(live, raw_to_f32(q_r[u]) * q_scale);
+      k_s[tok][r] = only(live, raw_to_f32(k_r[u]));
     }
 #pragma unroll
     for (int u = 0; u < V_REGS; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x / MEMC_COLS, cl = x - tok * MEMC_COLS, cc = blockIdx.x * MEMC_COLS + cl;
-      v_s[tok][cl] = only(tok < count && cc <= e, cc == e ? 1.f : v_r[u]);
+      v_s[tok][cl] = only(tok < count && cc <= e, cc == e ? 1.f : raw_to_f32(v_r[u]));
       if constexpr (RESULTS) a_s[tok][cl] = only(tok < count, a_r[u]);
     }
     if (threadIdx.x < MEMC_L) {
@@ -558,22 +561,16 @@ memory_chunk_kernel(const float* __restrict__ src, long src_stride, int q_off, i
   }
 }
 
-// ---- bfloat16 rows: the same blocks on the bfloat16 matrix instruction ------------------------------------------------ //
+// ---- bfloat16 rows of whole pieces: the same blocks on the bfloat16 matrix instruction ------------------------------------------------ //
 // q, k and v are bfloat16 to begin with; the other operand of each product (the state, the scores, the weighted values) is float32
 // and goes in as three bfloat16 parts (three_parts.h), so every single product is exact and nothing is rounded that the kernels above keep.
 // Three v_mfma_f32_32x32x16_bf16 of 32 cycles take the place of eight v_mfma_f32_32x32x2_f32 of 64; a block of tokens took a wavefront 36 of
 // those, with five wavefronts a SIMD 42 of the 77 us that 2,296 tokens of 16 heads of 128 took with results (without 32); now 47 and 24, bound by
 // the waits between a block's stages.
 
-// Eight values of a row from element `at` on, those from `limit` on zero.  vec: rows and limits are multiples of 16 bytes; then what
-// lies past the limit is what a place that exists holds, and `masked` clears it when the piece is used (nothing here waits for the load).
-__device__ __forceinline__ uint4 eight_of(const bf16_t* row, int at, int limit, bool vec) {
-  if (vec) return *(const uint4*)(row + min(at, limit - 8));
-  uint32_t v[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = at + e < limit ? row[at + e] : 0u;
-  return make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
-}
+// Eight values of a row from element `at` on; what lies past `limit` (a multiple of 8) is what a place that exists holds, and `masked`
+// clears it when the piece is used (nothing here waits for the load).
+__device__ __forceinline__ uint4 eight_of(const bf16_t* row, int at, int limit) { return *(const uint4*)(row + min(at, limit - 8)); }
 __device__ __forceinline__ uint4 masked(uint4 w, bool have) {
   const uint32_t keep = have ? 0xffffffffu : 0u;
   return make_uint4(w.x & keep, w.y & keep, w.z & keep, w.w & keep);
@@ -588,7 +585,7 @@ template <int STEPS>  // of 16 elements of a head
 __global__ void __launch_bounds__(256)
 memory_tile_scores_kernel(const bf16_t* __restrict__ src, long src_stride, int q_off, int k_off, float q_scale, const float* __restrict__ coef,
                           const double* __restrict__ start, const int* __restrict__ cu_q, int n_seqs, float* __restrict__ scores,
-                          float* __restrict__ wd, int heads, int d, bool vec) {
+                          float* __restrict__ wd, int heads, int d) {
   constexpr int AHEAD = STEPS < 8 ? STEPS : 8;
   const int lane = threadIdx.x & (CWM_WAVE - 1), c = lane & 31, half = lane >> 5;
   const int h = blockIdx.y * (256 / CWM_WAVE) + threadIdx.x / CWM_WAVE;
@@ -608,7 +605,7 @@ memory_tile_scores_kernel(const bf16_t* __restrict__ src, long src_stride, int q
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) {
       const int at = 16 * (u0 + u) + 8 * half;
-      fq[u] = eight_of(row + q_off, at, d, vec), fk[u] = eight_of(row + k_off, at, d, vec);
+      fq[u] = eight_of(row + q_off, at, d), fk[u] = eight_of(row + k_off, at, d);
     }
     if (u0 == 0 && c < count) {
       const float* cf = coef + ((size_t)(base + c) * heads + h) * 4;
@@ -647,7 +644,7 @@ __global__ void __launch_bounds__(CWM_WAVE * TILES, 3)
 memory_tile_kernel(const bf16_t* __restrict__ src, long src_stride, int q_off, int k_off, int v_off, float q_scale,
                    const float* __restrict__ scores, const float* __restrict__ wd, float* __restrict__ state, long state_stride,
                    long head_elems, const int* __restrict__ cu_q, const int* __restrict__ state_slots, float* __restrict__ y,
-                   float* __restrict__ nq, float* __restrict__ saved, int places, int n_seqs, int heads, int d, int e, int d_pad, bool vec) {
+                   float* __restrict__ nq, float* __restrict__ saved, int places, int n_seqs, int heads, int d, int e, int d_pad) {
   constexpr int THREADS = CWM_WAVE * TILES, DP = 32 * TILES;
   constexpr int ROW_LD = DP + 4, COL_LD = MEMC_L + 8;  // a column of rows 8 bytes a lane, a row of columns 16: no bank twice
   constexpr int QK_PIECES = MEMC_L * DP / 8 / THREADS, V_PIECES = THREADS < 128 ? 128 / THREADS : 1, S_PIECES = THREADS < 256 ? 256 / THREADS : 1;
@@ -700,13 +697,13 @@ memory_tile_kernel(const bf16_t* __restrict__ src, long src_stride, int q_off, i
     for (int u = 0; u < QK_PIECES; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x % MEMC_L, r0 = 8 * (x / MEMC_L);
       const bf16_t* row = src + (size_t)(base + min(tok, count - 1)) * src_stride + (size_t)h * d;
-      if constexpr (RESULTS) q_r[u] = eight_of(row + q_off, r0, d, vec);
-      k_r[u] = eight_of(row + k_off, r0, d, vec);
+      if constexpr (RESULTS) q_r[u] = eight_of(row + q_off, r0, d);
+      k_r[u] = eight_of(row + k_off, r0, d);
     }
 #pragma unroll
     for (int u = 0; u < V_PIECES; ++u) {
       const int x = threadIdx.x + u * THREADS, tok = x % MEMC_L, c0 = 8 * (x / MEMC_L);
-      v_r[u] = eight_of(src + (size_t)(base + min(tok, count - 1)) * src_stride + v_off + (size_t)h * e, blockIdx.x * MEMC_COLS + c0, e, vec);
+      v_r[u] = eight_of(src + (size_t)(base + min(tok, count - 1)) * src_stride + v_off + (size_t)h * e, blockIdx.x * MEMC_COLS + c0, e);
     }
     if constexpr (RESULTS) {
 #pragma unroll
@@ -993,6 +990,11 @@ memory_out_pairs_kernel(const float* __restrict__ y, const float* __restrict__ n
   }
 }
 
+// Whether bfloat16 rows of these sizes are whole pieces of 16 bytes, which the tiles read; element by element they wait for every load where it is
+// issued and take longer than the kernels on the float32 instruction (6 heads of 100 x 60, 700 tokens: 126 us against 75).
+extern "C" int cwm_matrix_memory_tiles(long src_stride, int q_off, int k_off, int v_off, int d, int e) {
+  return (src_stride | q_off | k_off | v_off | d | e) % 8 == 0;
+}
 extern "C" int cwm_matrix_memory_block_tokens() { return MEMC_L; }
 extern "C" int cwm_matrix_memory_segments_from() { return MEMS_FROM; }
 
@@ -1040,28 +1042,27 @@ extern "C" int cwm_matrix_memory(const void* src, int dtype, long src_stride, in
   const unsigned numbered = (unsigned)(n_tokens / MEMC_L + n_seqs);  // more than the largest number of a block of tokens
   int places = saved ? segment_place(n_tokens) : 0;  // more than the largest of a segment
   if (places + n_seqs > 65535) places = 0;           // more than a launch numbers: every portion in one piece
-  // rows, heads and offsets of whole pieces of 16 bytes, for the kernels on bfloat16 rows
-  const bool vec = (src_stride | q_off | k_off | v_off | d | e) % 8 == 0 && ((uintptr_t)src % 16) == 0;
+  const bool in_tiles = dtype == CWM_BF16 && cwm_matrix_memory_tiles(src_stride, q_off, k_off, v_off, d, e) && ((uintptr_t)src % 16) == 0;
   const bool pairs = e <= 256 && (src_stride | g_off | e) % 2 == 0 && (((uintptr_t)src | (uintptr_t)out) % 4) == 0 && (((uintptr_t)y | (uintptr_t)weight) % 8) == 0;
 #define CWM_MEMORY_CHUNK(T, TILES, RESULTS, Z)                                                                              \
   do {                                                                                                                      \
-    if constexpr (sizeof(T) == 2)                                                                                           \
+    if (in_tiles)                                                                                                           \
       hipLaunchKernelGGL((memory_tile_kernel<TILES, RESULTS>), dim3(block_tiles, heads, Z), dim3(CWM_WAVE * TILES), 0, stream, \
                          (const bf16_t*)src, src_stride, q_off, k_off, v_off, q_scale, (const float*)scores, (const float*)wd, \
-                         state, state_stride, head_elems, cu_q, state_slots, y, nq, saved, places, n_seqs, heads, d, e, d_pad, vec); \
+                         state, state_stride, head_elems, cu_q, state_slots, y, nq, saved, places, n_seqs, heads, d, e, d_pad); \
     else                                                                                                                    \
-      hipLaunchKernelGGL((memory_chunk_kernel<TILES, RESULTS>), dim3(block_tiles, heads, Z), dim3(CWM_WAVE * TILES), 0, stream, \
-                         (const float*)src, src_stride, q_off, k_off, v_off, q_scale, (const float*)scores, (const float*)wd, \
+      hipLaunchKernelGGL((memory_chunk_kernel<T, TILES, RESULTS>), dim3(block_tiles, heads, Z), dim3(CWM_WAVE * TILES), 0, stream, \
+                         (const T*)src, src_stride, q_off, k_off, v_off, q_scale, (const float*)scores, (const float*)wd,    \
                          state, state_stride, head_elems, cu_q, state_slots, y, nq, saved, places, n_seqs, heads, d, e, d_pad); \
   } while (0)
 #define CWM_MEMORY_BLOCKS(T, RPT, TILES)                                                                                    \
   do {                                                                                                                      \
-    if constexpr (sizeof(T) == 2)                                                                                           \
+    if (in_tiles)                                                                                                           \
       hipLaunchKernelGGL((memory_tile_scores_kernel<2 * TILES>), dim3(numbered, (heads + 3) / 4), dim3(256), 0, stream,      \
                          (const bf16_t*)src, src_stride, q_off, k_off, q_scale, (const float*)coef, (const double*)start, cu_q, n_seqs, \
-                         scores, wd, heads, d, vec);                                                                        \
+                         scores, wd, heads, d);                                                                             \
     else                                                                                                                    \
-      hipLaunchKernelGGL((memory_scores_kernel<RPT>), dim3(numbered, heads), dim3(MEMC_THREADS), 0, stream, (const float*)src, \
+      hipLaunchKernelGGL((memory_scores_kernel<T, RPT>), dim3(numbered, heads), dim3(MEMC_THREADS), 0, stream, (const T*)src, \
                          src_stride, q_off, k_off, q_scale, (const float*)coef, (const double*)start, cu_q, n_seqs, scores, \
                          wd, heads, d);                                                                                     \
     if (places > 0) {                                                                                                       \
