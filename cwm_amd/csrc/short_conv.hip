@@ -184,6 +184,12 @@ short_conv_runs_kernel(const bf16_t* __restrict__ x, long x_ld, const float* __r
   }
 }
 
+static long short_conv_runs_threads(int n_tokens, int n_seqs, int dim) { return (((long)n_tokens + SCONV_RUN - 1) / SCONV_RUN + n_seqs) * (dim / 8); }
+// Whether a step's sizes go through the kernel of runs, whose threads are numbered in 31 bits; larger ones keep the kernels above
+extern "C" int cwm_short_conv_in_runs(int n_tokens, int n_seqs, int taps, int dim) {
+  return n_tokens > n_seqs && taps >= 2 && taps <= 4 && dim % 8 == 0 && short_conv_runs_threads(n_tokens, n_seqs, dim) < (1L << 31) - SCONV_THREADS;
+}
+
 // x: [T, dim] of `dtype`, rows x_ld elements apart.  w1 (and w2, or null): float32 [taps, dim], a row a tap, the last
 // row the current token's.  out1 (and out2): contiguous [T, dim] of `dtype`.  state: float32 [n_slots, state_ld] with
 // (taps - 1) * dim <= state_ld (null where taps == 1); slots: int32 [n_seqs]; cu_q: int32 [n_seqs + 1]; seq_of_token:
@@ -199,11 +205,9 @@ extern "C" int cwm_short_conv(const void* x, long x_ld, int dtype, const float* 
   if (n_tokens == 0) return 0;
   const int gy = (dim + SCONV_THREADS - 1) / SCONV_THREADS;
   auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  if (dtype == CWM_BF16 && write_state != 2 && n_tokens > n_seqs && taps >= 2 && taps <= 4 && dim % 8 == 0 && x_ld % 8 == 0 && state_ld % 4 == 0 && aligned(x) &&
+  if (dtype == CWM_BF16 && write_state != 2 && cwm_short_conv_in_runs(n_tokens, n_seqs, taps, dim) && x_ld % 8 == 0 && state_ld % 4 == 0 && aligned(x) &&
       aligned(w1) && aligned(w2) && aligned(out1) && aligned(out2) && aligned(state)) {
-    const long threads = ((long)(n_tokens + SCONV_RUN - 1) / SCONV_RUN + n_seqs) * (dim / 8);
-    CWM_REQUIRE(threads < (1L << 31) - SCONV_THREADS, "short_conv: too many tokens");
-    const dim3 grid((unsigned)((threads + SCONV_THREADS - 1) / SCONV_THREADS));
+    const dim3 grid((unsigned)((short_conv_runs_threads(n_tokens, n_seqs, dim) + SCONV_THREADS - 1) / SCONV_THREADS));
 #define CWM_SCONV_RUNS(TAPS, TWO)                                                                                                             \
   hipLaunchKernelGGL((short_conv_runs_kernel<TAPS, TWO>), grid, dim3(SCONV_THREADS), 0, stream, (const bf16_t*)x, x_ld, w1, w2, (bf16_t*)out1, \
                      (bf16_t*)out2, state, state_ld, slots, cu_q, seq_of_token, n_slots, n_tokens, n_seqs, dim, write_state == 1)

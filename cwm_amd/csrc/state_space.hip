@@ -205,6 +205,12 @@ __global__ void __launch_bounds__(256) conv_silu_runs_kernel(const bf16_t* __res
   }
 }
 
+static long conv_runs_threads(int n_tokens, int n_seqs, int channels) { return (((long)n_tokens + CONV_RUN - 1) / CONV_RUN + n_seqs) * (channels / 8); }
+// Whether a step's sizes go through the kernel of runs, whose threads are numbered in 31 bits; larger ones keep the kernel of a thread a channel
+extern "C" int cwm_conv_silu_in_runs(int n_tokens, int n_seqs, int channels) {
+  return n_seqs > 0 && n_tokens > n_seqs && channels % 8 == 0 && conv_runs_threads(n_tokens, n_seqs, channels) < (1L << 31) - 256;
+}
+
 // w_by_tap: the same weights as [taps][channels], or null (then every token goes through the kernel of a thread a channel)
 extern "C" int cwm_conv_silu(const void* in, long in_ld, int dtype, const float* w, const float* w_by_tap, const float* bias, float* state, long state_ld,
                              long state_off, const int* slots, const int* cu_q, const int* seq_of_token, void* out, int n_tokens,
@@ -215,11 +221,10 @@ extern "C" int cwm_conv_silu(const void* in, long in_ld, int dtype, const float*
   CWM_REQUIRE(state_off >= 0 && state_off + (long)(taps - 1) * channels <= state_ld, "conv_silu: the state row is too short");
   if (n_tokens == 0) return 0;
   dim3 grid(n_tokens, (channels + 255) / 256);
-  if (dtype == CWM_BF16 && w_by_tap && n_seqs > 0 && n_tokens > n_seqs && channels % 8 == 0 && in_ld % 8 == 0 && state_ld % 4 == 0 &&
+  if (dtype == CWM_BF16 && w_by_tap && cwm_conv_silu_in_runs(n_tokens, n_seqs, channels) && in_ld % 8 == 0 && state_ld % 4 == 0 &&
       state_off % 4 == 0 && ((uintptr_t)in % 16) == 0 && ((uintptr_t)out % 16) == 0 && ((uintptr_t)w_by_tap % 16) == 0 && ((uintptr_t)bias % 16) == 0 &&
       ((uintptr_t)state % 16) == 0) {
-    const long threads = ((long)(n_tokens + CONV_RUN - 1) / CONV_RUN + n_seqs) * (channels / 8);
-    CWM_REQUIRE(threads < (1L << 31) - 256, "conv_silu: too many tokens");
+    const long threads = conv_runs_threads(n_tokens, n_seqs, channels);
 #define CWM_CONV_RUNS(TAPS)                                                                                                              \
   hipLaunchKernelGGL(conv_silu_runs_kernel<TAPS>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, (const bf16_t*)in, in_ld, \
                      w_by_tap, bias, state, state_ld, state_off, slots, cu_q, seq_of_token, (bf16_t*)out, n_tokens, n_seqs, channels, n_slots)
