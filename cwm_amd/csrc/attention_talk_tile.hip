@@ -19,7 +19,7 @@
 // 32 x 32; 16 of the mixing product's 128 cycles a pair tile would be bfloat16's, but weights stay float32 until they are mixed).  All in one
 // kernel, the outputs kept in registers, took 59 to 87 with 10 for the sum of cut ranges: with them there is room for 16 rows only, and a
 // compute unit then reads 128 KB of keys and values a step at about 50 GB/s.
-#include "common.h"
+#include "three_parts.h"
 
 CWM_DEFINE_ERROR_API
 
@@ -62,11 +62,13 @@ __device__ __forceinline__ int first_key(const TalkTileArgs& A, int p) { return 
 __device__ __forceinline__ int table_base(const TalkTileArgs& A, const TalkPortion& po, int row) { return first_key(A, po.pos0 + (row & ~31)) & ~(TILE_KEYS - 1); }
 
 // the page of the 32 keys from `kt` on (pages hold a multiple of 32 keys); a page that is not there, in the table or behind its end: page 0
-__device__ __forceinline__ int tile_page(const int* table, const TalkTileArgs& A, int kt, int& slot) {
+__device__ __forceinline__ int tile_page(const int* table, const TalkTileArgs& A, int kt, int& slot, bool* there = nullptr) {
   const int lp = page_number(A, kt);
   slot = kt - lp * A.page_size;
   const int page = lp < A.table_width ? table[lp] : -1;
-  return (unsigned)page < (unsigned)A.num_pages ? page : 0;
+  const bool known = (unsigned)page < (unsigned)A.num_pages;
+  if (there) *there = known;
+  return known ? page : 0;
 }
 // the same of one thread's own range
 __device__ __forceinline__ bool row_lacks_page(const int* table, const TalkTileArgs& A, int first, int last) {
@@ -355,26 +357,39 @@ talk_tile_mix_kernel(TalkTileArgs A, TalkPortions P, const float* __restrict__ s
 }
 
 // ---- values ------------------------------------------------------------------------------------------------------------ //
-// A row of a tile has weight zero for the tile's keys that it does not read, and zero times an infinity or a NaN is a NaN.  So a result
-// that is not finite, and all of a tile that reads a missing page, is made again from the row's own keys alone, sums of 128 keys one after the
-// other (an infinite or NaN value reaches its readers only, whatever rows lie beside them); rows that read a missing page are NaN, the others are not.
-#define VALUE_RANGE 128
-__device__ __forceinline__ float4 values_of_own_keys(const TalkTileArgs& A, const int* table, const bf16_t* weights, const bf16_t* values, size_t page_stride,
-                                                  int head_dim, int d, int first, int last) {
-  float total[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int from = first; from <= last; from += VALUE_RANGE) {
-    float part[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int key = from; key <= min(last, from + VALUE_RANGE - 1); ++key) {
-      const int lp = page_number(A, key), slot = key - lp * A.page_size;
-      const bf16_t* v = values + (size_t)table[lp] * page_stride + ((size_t)(slot / 8) * head_dim + d) * 8 + slot % 8;
-      const float w = bf16_to_f32(weights[key]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) part[i] = fmaf(w, bf16_to_f32(v[8 * i]), part[i]);
+// A row of a tile has weight zero for the tile's keys that it does not read, and zero times an infinity or a NaN is a NaN.  Such keys lie in
+// the steps at the tile's two ends alone (`TileEnds`): there values that are not finite, and all of a missing page, are zeros to the matrix
+// instruction, and a row's own products with the former are added to its sums.  So an infinite or NaN value reaches its readers only, whatever rows
+// lie beside them, and every other result has the bits that it has without; rows that read a missing page are NaN, the others are not.
+struct TileEnds {
+  int lo, lo_all, p_first, p_last;  // the first key that any row reads; from lo_all to p_first every row reads every key; the last key
+  __device__ __forceinline__ bool of(int kt) const { return kt < lo_all || kt + TILE_KEYS - 1 > p_first; }
+};
+__device__ __forceinline__ bool not_finite(uint32_t half) { return (half & 0x7f80u) == 0x7f80u; }
+__device__ __forceinline__ uint32_t finite_only(uint32_t two) {
+  return (not_finite(two) ? 0u : two & 0x0000ffffu) | (not_finite(two >> 16) ? 0u : two & 0xffff0000u);
+}
+// a row's products of the tile's ends with values that are not finite, onto `sum`, four dims from d on
+__device__ __forceinline__ float4v add_not_finite(const TalkTileArgs& A, const TileEnds& ends, const int* table, const bf16_t* weights, const bf16_t* values,
+                                                  size_t page_stride, int head_dim, int d, int first, int p, float4v sum) {
+  for (int kt = ends.lo & ~(TILE_KEYS - 1); kt <= p; kt += TILE_KEYS) {
+    if (!ends.of(kt)) {
+      kt = max(kt, (ends.p_first & ~(TILE_KEYS - 1)) - TILE_KEYS);
+      continue;
     }
+    int slot;
+    bool there;
+    const bf16_t* from = values + (size_t)tile_page(table, A, kt, slot, &there) * page_stride;
+    if (!there) continue;
+    for (int key = max(kt, first); key <= min(kt + TILE_KEYS - 1, p); ++key) {
+      const int s = slot + key - kt;
+      const bf16_t* v = from + ((size_t)(s / 8) * head_dim + d) * 8 + s % 8;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) total[i] += part[i];
+      for (int i = 0; i < 4; ++i)
+        if (not_finite(v[8 * i])) sum[i] = fmaf(bf16_to_f32(weights[key]), bf16_to_f32(v[8 * i]), sum[i]);
+    }
   }
-  return make_float4(total[0], total[1], total[2], total[3]);
+  return sum;
 }
 
 // HEADS: heads of a block, which share the values' operands.
@@ -383,6 +398,7 @@ __global__ void __launch_bounds__(64 * VALUE_WAVES, 2)
 talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict__ weights, bf16_t* __restrict__ out) {
   constexpr int DT = HD / 16, ROWS = 16 * RT;
   __shared__ __attribute__((aligned(16))) float sums[VALUE_WAVES][HEADS][16][HD + 4];
+  __shared__ int odd_of[VALUE_WAVES];
   const TalkPortion& po = portion_of(P, 2);
   const int per = A.n_q_heads / A.n_kv_heads, groups = A.n_kv_heads * ((per + HEADS - 1) / HEADS);
   const int block = blockIdx.x - po.at[2], tiles = (po.r1 - po.r0 + ROWS - 1) / ROWS;
@@ -392,6 +408,7 @@ talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int* table = A.block_table + (size_t)po.seq * A.table_width;
   const int p_last = po.pos0 + min(row0 + ROWS, po.r1) - 1, lo = first_key(A, po.pos0 + row0), base = table_base(A, po, row0);
+  const TileEnds ends = {lo, first_key(A, p_last), po.pos0 + row0, p_last};
 
   const bf16_t* from_w[RT][HEADS];
 #pragma unroll
@@ -410,9 +427,10 @@ talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) acc[u][g][dt] = (float4v){0.f, 0.f, 0.f, 0.f};
   Frag8 vf[DT], wf[RT][HEADS];
+  bool there;
   auto load = [&](int kt) {
     int slot;
-    const int page = tile_page(table, A, kt, slot);
+    const int page = tile_page(table, A, kt, slot, &there);
     const bf16_t* from = values + (size_t)page * 2 * plane + (size_t)(slot / 8 + j) * HD * 8;
 #pragma unroll
     for (int u = 0; u < RT; ++u)
@@ -421,17 +439,27 @@ talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) vf[dt].u = *(const uint4*)(from + dt * 16 * 8);
   };
+  int odd = 0;  // whether the wavefront has left values out that are not finite
   for (int kt = (lo & ~(TILE_KEYS - 1)) + TILE_KEYS * wave; kt <= p_last; kt += TILE_KEYS * VALUE_WAVES) {
     load(kt);
-    if (kt < lo || kt + TILE_KEYS - 1 > p_last) {  // values that no row reads may be anything
-      uint32_t keep[4] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu};
+    if (ends.of(kt)) {
+      uint32_t keep[4];  // values that no row reads may be anything
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int key = kt + 8 * j + e;
-        if (key < lo || key > p_last) keep[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
+      for (int e = 0; e < 4; ++e) {
+        const int key = kt + 8 * j + 2 * e;
+        keep[e] = there ? (key >= lo && key <= p_last ? 0x0000ffffu : 0u) | (key + 1 >= lo && key + 1 <= p_last ? 0xffff0000u : 0u) : 0u;
       }
+      Halves most = {0, 0};
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) vf[dt].u.x &= keep[0], vf[dt].u.y &= keep[1], vf[dt].u.z &= keep[2], vf[dt].u.w &= keep[3];
+      for (int dt = 0; dt < DT; ++dt) {
+        vf[dt].u.x &= keep[0], vf[dt].u.y &= keep[1], vf[dt].u.z &= keep[2], vf[dt].u.w &= keep[3];
+        most = larger_magnitudes(larger_magnitudes(larger_magnitudes(larger_magnitudes(most, vf[dt].u.x), vf[dt].u.y), vf[dt].u.z), vf[dt].u.w);
+      }
+      if (__any(max(most.x, most.y) >= 0x7f80)) {
+        odd = 1;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) vf[dt].u = make_uint4(finite_only(vf[dt].u.x), finite_only(vf[dt].u.y), finite_only(vf[dt].u.z), finite_only(vf[dt].u.w));
+      }
     }
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -441,18 +469,9 @@ talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict
         for (int g = 0; g < HEADS; ++g) acc[u][g][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt].v, wf[u][g].v, acc[u][g][dt], 0, 0, 0);
   }
   // lane 16 j + n holds row n, dims 16 dt + 4 j + i
-  constexpr int ITEMS = HEADS * 16 * (HD / 4) / (64 * VALUE_WAVES);  // four dims of a row and head each, of a thread for 16 rows
-  static_assert(RT * ITEMS <= 32 && ITEMS * 64 * VALUE_WAVES == HEADS * 16 * (HD / 4), "a bit an item");
   const bool missing = lacks_page(table, A, lo, p_last);
-  uint32_t again = missing ? 0xffffffffu : 0u;
-  auto item = [&](int u, int i, int& g, int& r, int& d) {
-    const int e = threadIdx.x + 64 * VALUE_WAVES * i;
-    d = e % (HD / 4) * 4, g = e / (HD / 4) % HEADS, r = e / (HD / 4) / HEADS;
-    return g0 + g < per && row0 + 16 * u + r < po.r1;
-  };
-  auto leave = [&](int row, int g, int d, float4v v) {
-    *(uint2*)(out + (size_t)(po.t0 + row) * A.n_q_heads * HD + (size_t)(c * per + g0 + g) * HD + d) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
-  };
+  const float nan = __uint_as_float(0x7fc00000u);
+  if (lane == 0) odd_of[wave] = odd;
 #pragma unroll
   for (int u = 0; u < RT; ++u) {
     if (u > 0) __syncthreads();
@@ -461,31 +480,24 @@ talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) *(float4v*)&sums[wave][g][n][16 * dt + 4 * j] = acc[u][g][dt];
     __syncthreads();
+    int any_odd = 0;
 #pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      int g, r, d;
-      if (!item(u, i, g, r, d)) continue;
+    for (int w = 0; w < VALUE_WAVES; ++w) any_odd |= odd_of[w];
+    const bool plain = __builtin_amdgcn_readfirstlane(any_odd) == 0 && !missing;
+    for (int e = threadIdx.x; e < HEADS * 16 * (HD / 4); e += 64 * VALUE_WAVES) {
+      const int d = e % (HD / 4) * 4, g = e / (HD / 4) % HEADS, r = e / (HD / 4) / HEADS, row = row0 + 16 * u + r;
+      if (g0 + g >= per || row >= po.r1) continue;
       float4v v = *(const float4v*)&sums[0][g][r][d];
 #pragma unroll
       for (int w = 1; w < VALUE_WAVES; ++w) v += *(const float4v*)&sums[w][g][r][d];
-      if (!(fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < __builtin_inff())) again |= 1u << (u * ITEMS + i);
-      leave(row0 + 16 * u + r, g, d, v);
+      if (__builtin_expect(!plain, 0)) {
+        const int p = po.pos0 + row, first = first_key(A, p);
+        const bf16_t* w = weights + po.table + ((size_t)(c * per + g0 + g) * (po.r1 - po.r0) + row - po.r0) * po.columns - base;
+        if (missing && row_lacks_page(table, A, first, p)) v = (float4v){nan, nan, nan, nan};
+        else v = add_not_finite(A, ends, table, w, A.cache + plane + (size_t)c * A.page_size * HD, 2 * plane, HD, d, first, p, v);
+      }
+      *(uint2*)(out + (size_t)(po.t0 + row) * A.n_q_heads * HD + (size_t)(c * per + g0 + g) * HD + d) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
     }
-  }
-  if (__builtin_expect(again == 0, 1)) return;
-  const float nan = __uint_as_float(0x7fc00000u);
-  for (int x = 0; x < RT * ITEMS; ++x) {
-    int g, r, d;
-    const int u = x / ITEMS;
-    if (!(again >> x & 1) || !item(u, x % ITEMS, g, r, d)) continue;
-    const int row = row0 + 16 * u + r, p = po.pos0 + row, first = first_key(A, p);
-    if (missing && row_lacks_page(table, A, first, p)) {
-      leave(row, g, d, (float4v){nan, nan, nan, nan});
-      continue;
-    }
-    const bf16_t* w = weights + po.table + ((size_t)(c * per + g0 + g) * (po.r1 - po.r0) + row - po.r0) * po.columns - base;
-    const float4 own = values_of_own_keys(A, table, w, A.cache + plane + (size_t)c * A.page_size * HD, 2 * plane, HD, d, first, p);
-    leave(row, g, d, (float4v){own.x, own.y, own.z, own.w});
   }
 }
 

@@ -108,13 +108,12 @@ def _value_of(cache, table, b, key, n_kv, hd):
 @pytest.mark.parametrize("n_q,n_kv,hd,old,new,window", [(16, 8, 128, 5, 40, None), (8, 4, 64, 70, 100, 33), (24, 8, 128, 40, 130, 64), (9, 3, 128, 0, 16, None), (20, 4, 64, 300, 77, 1)])
 def test_a_value_that_is_not_finite_reaches_its_readers_only(bad, n_q, n_kv, hd, old, new, window):
     """One element of one token's values: of the heads and elements that it lies in, the rows that read the token are not
-    finite, the others what they were up to another order of their sums; all else keeps its bits."""
+    finite; all else keeps its bits."""
     from cwm_amd import ops
 
     case = _talking_case(torch.bfloat16, n_q, n_kv, hd, 64, [old], [new], window, seed=n_q + new)
     q, cache, table, batch, scale, sink, mix, want = case
     clean = ops.talking_attention(q, cache, table, batch, window, scale, sink=sink, talk=mix).cpu()
-    bound = _bound(case, window)
     key, head, d, per = old + new * 2 // 3, n_kv - 1, hd - 3, n_q // n_kv
     _value_of(cache, table, 0, key, n_kv, hd)[head, d] = bad
     got = ops.talking_attention(q, cache, table, batch, window, scale, sink=sink, talk=mix).cpu()
@@ -125,7 +124,7 @@ def test_a_value_that_is_not_finite_reaches_its_readers_only(bad, n_q, n_kv, hd,
     there[head * per :, d] = True
     there = there.flatten()
     assert not torch.isfinite(got[reads][:, there]).any()
-    assert bool(((got.double() - want).abs() <= bound)[~reads].all())
+    assert torch.equal(got[~reads], clean[~reads])
     assert torch.equal(got[:, ~there][reads], clean[:, ~there][reads])
 
 
