@@ -174,3 +174,53 @@ def test_scales_that_are_not_positive(new):
     none = ops.talking_attention(q, cache, table, batch, 60, 0.0, sink=sink, talk=mix)
     zero = ops.talking_attention(torch.zeros_like(q), cache, table, batch, 60, scale, sink=sink, talk=mix)
     torch.testing.assert_close(none.float(), zero.float(), rtol=2 ** -6, atol=2 ** -6)  # bfloat16 weights and results
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,lens_old,lens_new,window", [
+    (16, 8, 128, [300, 31], [700, 143], None), (16, 8, 128, [300, 31], [143, 700], 64), (24, 8, 64, [0, 100], [333, 200], None), (24, 8, 128, [40, 5], [97, 260], 50),
+])
+def test_portions_over_several_launches(n_q, n_kv, hd, lens_old, lens_new, window, monkeypatch):
+    """A table of weights that holds a few tiles of rows: the portions go over many launches, with the bits of one."""
+    from cwm_amd import ops
+    from cwm_amd.ops import mixing
+
+    q, cache, table, batch, scale, sink, mix, want = _talking_case(torch.bfloat16, n_q, n_kv, hd, 64, lens_old, lens_new, window, seed=n_q + sum(lens_new))
+    lib, launches = mixing._build.load("attention_talk_tile"), []
+
+    class Counting:
+        def __getattr__(self, name):
+            return getattr(lib, name)
+
+        def cwm_talking_tiles(self, *args):
+            launches.append(args)
+            return lib.cwm_talking_tiles(*args)
+
+    mixing._build._loaded["attention_talk_tile"] = Counting()
+    try:
+        whole = ops.talking_attention(q, cache, table, batch, window, scale, sink=sink, talk=mix)
+        assert len(launches) == 1
+        for table_bytes in (1, 300_000, 1_000_000):
+            monkeypatch.setattr(mixing, "TALK_TABLE_BYTES", table_bytes)
+            del launches[:]
+            got = ops.talking_attention(q, cache, table, batch, window, scale, sink=sink, talk=mix)
+            assert len(launches) > 1, table_bytes
+            assert torch.equal(got, whole), table_bytes
+        monkeypatch.setattr(mixing, "TALK_TABLE_BYTES", 1)
+        del launches[:]
+        ops.talking_attention(q, cache, table, batch, window, scale, sink=sink, talk=mix)
+        assert len(launches) == sum(-(-n // 32) for n in lens_new)  # a tile of rows each
+    finally:
+        mixing._build._loaded["attention_talk_tile"] = lib
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,old,new,window", [(16, 8, 128, 77, 130, None), (24, 8, 64, 300, 45, 64), (9, 3, 128, 0, 16, None)])
+def test_without_a_sink(n_q, n_kv, hd, old, new, window):
+    """A sink far below every score adds nothing, so it gives the bits of none; a quiet one gives others."""
+    from cwm_amd import ops
+
+    case = _talking_case(torch.bfloat16, n_q, n_kv, hd, 64, [old], [new], window, seed=n_q)
+    q, cache, table, batch, scale, sink, mix, want = case
+    none = ops.talking_attention(q, cache, table, batch, window, scale, sink=None, talk=mix)
+    low = ops.talking_attention(q, cache, table, batch, window, scale, sink=torch.full_like(sink, -1e30), talk=mix)
+    assert torch.equal(none, low)
+    assert not torch.equal(none, ops.talking_attention(q, cache, table, batch, window, scale, sink=sink, talk=mix))
