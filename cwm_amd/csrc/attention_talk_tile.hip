@@ -19,7 +19,8 @@
 // 32 x 32; 16 of the mixing product's 128 cycles a pair tile would be bfloat16's, but weights stay float32 until they are mixed).  All in one
 // kernel, the outputs kept in registers, took 59 to 87 with 10 for the sum of cut ranges: with them there is room for 16 rows only, and a
 // compute unit then reads 128 KB of keys and values a step at about 50 GB/s.
-#include "three_parts.h"
+#include "common.h"
+#include <type_traits>
 
 CWM_DEFINE_ERROR_API
 
@@ -357,10 +358,11 @@ talk_tile_mix_kernel(TalkTileArgs A, TalkPortions P, const float* __restrict__ s
 }
 
 // ---- values ------------------------------------------------------------------------------------------------------------ //
-// A row of a tile has weight zero for the tile's keys that it does not read, and zero times an infinity or a NaN is a NaN.  Such keys lie in
-// the steps at the tile's two ends alone (`TileEnds`): there values that are not finite, and all of a missing page, are zeros to the matrix
-// instruction, and a row's own products with the former are added to its sums.  So an infinite or NaN value reaches its readers only, whatever rows
-// lie beside them, and every other result has the bits that it has without; rows that read a missing page are NaN, the others are not.
+// A row of a tile has weight zero for the tile's keys that it does not read, and zero times an infinity or a NaN is a NaN.  So a block with a
+// result that is not finite, or a missing page, goes over its keys once more.  Keys that a row does not read lie in the steps at the tile's two
+// ends alone (`TileEnds`): there values that are not finite, and all of a missing page, are zeros to the matrix instruction then, and a row's own
+// products with the former are added to its sums.  An infinite or NaN value reaches its readers only, whatever rows lie beside them, and every
+// other result has the bits that it has without; rows that read a missing page are NaN, the others are not.
 struct TileEnds {
   int lo, lo_all, p_first, p_last;  // the first key that any row reads; from lo_all to p_first every row reads every key; the last key
   __device__ __forceinline__ bool of(int kt) const { return kt < lo_all || kt + TILE_KEYS - 1 > p_first; }
@@ -398,7 +400,6 @@ __global__ void __launch_bounds__(64 * VALUE_WAVES, 2)
 talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict__ weights, bf16_t* __restrict__ out) {
   constexpr int DT = HD / 16, ROWS = 16 * RT;
   __shared__ __attribute__((aligned(16))) float sums[VALUE_WAVES][HEADS][16][HD + 4];
-  __shared__ int odd_of[VALUE_WAVES];
   const TalkPortion& po = portion_of(P, 2);
   const int per = A.n_q_heads / A.n_kv_heads, groups = A.n_kv_heads * ((per + HEADS - 1) / HEADS);
   const int block = blockIdx.x - po.at[2], tiles = (po.r1 - po.r0 + ROWS - 1) / ROWS;
@@ -419,13 +420,6 @@ talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict
   const size_t plane = (size_t)A.n_kv_heads * A.page_size * HD;
   const bf16_t* values = A.cache + plane + (size_t)c * A.page_size * HD + (size_t)n * 8;
 
-  float4v acc[RT][HEADS][DT];
-#pragma unroll
-  for (int u = 0; u < RT; ++u)
-#pragma unroll
-    for (int g = 0; g < HEADS; ++g)
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) acc[u][g][dt] = (float4v){0.f, 0.f, 0.f, 0.f};
   Frag8 vf[DT], wf[RT][HEADS];
   bool there;
   auto load = [&](int kt) {
@@ -439,66 +433,72 @@ talk_tile_values_kernel(TalkTileArgs A, TalkPortions P, const bf16_t* __restrict
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) vf[dt].u = *(const uint4*)(from + dt * 16 * 8);
   };
-  int odd = 0;  // whether the wavefront has left values out that are not finite
-  for (int kt = (lo & ~(TILE_KEYS - 1)) + TILE_KEYS * wave; kt <= p_last; kt += TILE_KEYS * VALUE_WAVES) {
-    load(kt);
-    if (ends.of(kt)) {
-      uint32_t keep[4];  // values that no row reads may be anything
+  // whether all is finite and no page missing
+  auto pass = [&](auto once_more) {
+    constexpr bool again = decltype(once_more)::value;
+    float4v acc[RT][HEADS][DT];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int key = kt + 8 * j + 2 * e;
-        keep[e] = there ? (key >= lo && key <= p_last ? 0x0000ffffu : 0u) | (key + 1 >= lo && key + 1 <= p_last ? 0xffff0000u : 0u) : 0u;
+    for (int u = 0; u < RT; ++u)
+#pragma unroll
+      for (int g = 0; g < HEADS; ++g)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) acc[u][g][dt] = (float4v){0.f, 0.f, 0.f, 0.f};
+    for (int kt = (lo & ~(TILE_KEYS - 1)) + TILE_KEYS * wave; kt <= p_last; kt += TILE_KEYS * VALUE_WAVES) {
+      load(kt);
+      if (kt < lo || kt + TILE_KEYS - 1 > p_last) {  // values that no row reads may be anything
+        uint32_t keep[4] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int key = kt + 8 * j + e;
+          if (key < lo || key > p_last) keep[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
+        }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) vf[dt].u.x &= keep[0], vf[dt].u.y &= keep[1], vf[dt].u.z &= keep[2], vf[dt].u.w &= keep[3];
       }
-      Halves most = {0, 0};
+      if (again && ends.of(kt)) {
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        vf[dt].u.x &= keep[0], vf[dt].u.y &= keep[1], vf[dt].u.z &= keep[2], vf[dt].u.w &= keep[3];
-        most = larger_magnitudes(larger_magnitudes(larger_magnitudes(larger_magnitudes(most, vf[dt].u.x), vf[dt].u.y), vf[dt].u.z), vf[dt].u.w);
+        for (int dt = 0; dt < DT; ++dt)
+          vf[dt].u = there ? make_uint4(finite_only(vf[dt].u.x), finite_only(vf[dt].u.y), finite_only(vf[dt].u.z), finite_only(vf[dt].u.w)) : make_uint4(0u, 0u, 0u, 0u);
       }
-      if (__any(max(most.x, most.y) >= 0x7f80)) {
-        odd = 1;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) vf[dt].u = make_uint4(finite_only(vf[dt].u.x), finite_only(vf[dt].u.y), finite_only(vf[dt].u.z), finite_only(vf[dt].u.w));
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int u = 0; u < RT; ++u)
+#pragma unroll
+          for (int g = 0; g < HEADS; ++g) acc[u][g][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt].v, wf[u][g].v, acc[u][g][dt], 0, 0, 0);
+    }
+    // lane 16 j + n holds row n, dims 16 dt + 4 j + i
+    const bool missing = lacks_page(table, A, lo, p_last);
+    bool plain = !missing;
+#pragma unroll
+    for (int u = 0; u < RT; ++u) {
+      if (u > 0) __syncthreads();
+#pragma unroll
+      for (int g = 0; g < HEADS; ++g)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) *(float4v*)&sums[wave][g][n][16 * dt + 4 * j] = acc[u][g][dt];
+      __syncthreads();
+      for (int e = threadIdx.x; e < HEADS * 16 * (HD / 4); e += 64 * VALUE_WAVES) {
+        const int d = e % (HD / 4) * 4, g = e / (HD / 4) % HEADS, r = e / (HD / 4) / HEADS, row = row0 + 16 * u + r;
+        if (g0 + g >= per || row >= po.r1) continue;
+        float4v v = *(const float4v*)&sums[0][g][r][d];
+#pragma unroll
+        for (int w = 1; w < VALUE_WAVES; ++w) v += *(const float4v*)&sums[w][g][r][d];
+        plain = plain && fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < __builtin_inff();
+        if constexpr (again) {
+          const int p = po.pos0 + row, first = first_key(A, p);
+          const float nan = __uint_as_float(0x7fc00000u);
+          const bf16_t* w = weights + po.table + ((size_t)(c * per + g0 + g) * (po.r1 - po.r0) + row - po.r0) * po.columns - base;
+          if (missing && row_lacks_page(table, A, first, p)) v = (float4v){nan, nan, nan, nan};
+          else v = add_not_finite(A, ends, table, w, A.cache + plane + (size_t)c * A.page_size * HD, 2 * plane, HD, d, first, p, v);
+        }
+        *(uint2*)(out + (size_t)(po.t0 + row) * A.n_q_heads * HD + (size_t)(c * per + g0 + g) * HD + d) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
       }
     }
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int u = 0; u < RT; ++u)
-#pragma unroll
-        for (int g = 0; g < HEADS; ++g) acc[u][g][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt].v, wf[u][g].v, acc[u][g][dt], 0, 0, 0);
-  }
-  // lane 16 j + n holds row n, dims 16 dt + 4 j + i
-  const bool missing = lacks_page(table, A, lo, p_last);
-  const float nan = __uint_as_float(0x7fc00000u);
-  if (lane == 0) odd_of[wave] = odd;
-#pragma unroll
-  for (int u = 0; u < RT; ++u) {
-    if (u > 0) __syncthreads();
-#pragma unroll
-    for (int g = 0; g < HEADS; ++g)
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) *(float4v*)&sums[wave][g][n][16 * dt + 4 * j] = acc[u][g][dt];
-    __syncthreads();
-    int any_odd = 0;
-#pragma unroll
-    for (int w = 0; w < VALUE_WAVES; ++w) any_odd |= odd_of[w];
-    const bool plain = __builtin_amdgcn_readfirstlane(any_odd) == 0 && !missing;
-    for (int e = threadIdx.x; e < HEADS * 16 * (HD / 4); e += 64 * VALUE_WAVES) {
-      const int d = e % (HD / 4) * 4, g = e / (HD / 4) % HEADS, r = e / (HD / 4) / HEADS, row = row0 + 16 * u + r;
-      if (g0 + g >= per || row >= po.r1) continue;
-      float4v v = *(const float4v*)&sums[0][g][r][d];
-#pragma unroll
-      for (int w = 1; w < VALUE_WAVES; ++w) v += *(const float4v*)&sums[w][g][r][d];
-      if (__builtin_expect(!plain, 0)) {
-        const int p = po.pos0 + row, first = first_key(A, p);
-        const bf16_t* w = weights + po.table + ((size_t)(c * per + g0 + g) * (po.r1 - po.r0) + row - po.r0) * po.columns - base;
-        if (missing && row_lacks_page(table, A, first, p)) v = (float4v){nan, nan, nan, nan};
-        else v = add_not_finite(A, ends, table, w, A.cache + plane + (size_t)c * A.page_size * HD, 2 * plane, HD, d, first, p, v);
-      }
-      *(uint2*)(out + (size_t)(po.t0 + row) * A.n_q_heads * HD + (size_t)(c * per + g0 + g) * HD + d) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
-    }
-  }
+    return plain;
+  };
+  if (__builtin_expect(__syncthreads_and(pass(std::false_type())), 1)) return;
+  pass(std::true_type());
 }
 
 // ---- entry points ---------------------------------------------------------------------------------------------------- //
