@@ -20,6 +20,7 @@
 // kernel, the outputs kept in registers, took 59 to 87 with 10 for the sum of cut ranges: with them there is room for 16 rows only, and a
 // compute unit then reads 128 KB of keys and values a step at about 50 GB/s.
 #include "common.h"
+#include <algorithm>
 #include <type_traits>
 
 CWM_DEFINE_ERROR_API
@@ -524,20 +525,48 @@ extern "C" int cwm_talking_tile_groups(int n_q_heads, int n_kv_heads, int head_d
 }
 extern "C" int cwm_talking_tile_portions() { return TILE_PORTIONS; }
 
-// Steps of a block of the second kernel.  No sum goes from one step to the next, so they may be cut anywhere: where rounds of 224
-// blocks take least (a compute unit has room for one, and the XCDs do not get equally many), a block costing 7 us and 3.7 a step (1,500 tokens, 16 heads of 128: blocks of 4, 5, 6, 8, 12 and all 47 steps
-// take 48, 55, 35, 42, 56 and 184 us).
-static int mix_steps(const TalkPortions& P, int count, int mix_rows, int window_left) {
-  int best = 1;
+// Steps of a block of the second kernel.  No sum goes from one step to the next, so they may be cut anywhere: where the rounds of blocks take
+// least, a block costing 7 us and 3.7 a step.  A compute unit has room for one block (148 KB of LDS).  A round is counted in two ways, and the
+// larger number holds: as 224 blocks, since not all of 256 units are had at once, and as the fullest of 32 lots of 8 units, which a launch's blocks are
+// dealt to in turn: tiles whose number is a multiple of 32 leave the rows with most keys in few lots.  Up to 8 heads (74 KB) two blocks share a
+// unit beyond 192 blocks, which makes a round of twice as many 1.6 times as long.  us by steps: 16 heads of 128, 1,500 tokens 91 (4), 78 (6), 85 (8),
+// 100 (12) and 174 (32); 2,048, whose 221 blocks of 11 steps leave 9 in a lot, 145 (11), 117 (13); 8 heads, 1,500 tokens 65 (3), 77 (6), 69 (8).  Over 88
+// portions of 8 to 32 heads of 64 and 128, 64 to 4,096 tokens, the choice is within 8% of the best of all steps, 1.1% in the mean; without the lots
+// and the second block within 30% and 3.4%.
+#define MIX_LOTS 32
+static int mix_steps(const TalkPortions& P, int count, int mix_rows, int n_q_heads, int window_left) {
+  const int room = n_q_heads <= 8 ? 2 : 1;
+  int best = 2;
   float least = 0.f;
   for (int steps = 2; steps <= 32; ++steps) {
-    long blocks = 0;
-    for (int i = 0; i < count; ++i)
-      for (int row0 = P.of[i].r0; row0 < P.of[i].r1; row0 += mix_rows) blocks += (tile_steps(P.of[i], row0, mix_rows, window_left) + steps - 1) / steps;
-    const float us = (float)((blocks + 223) / 224) * (7.f + 3.7f * steps);
+    long blocks = 0, at = 0;
+    int lots[MIX_LOTS] = {}, fullest = 0;
+    for (int i = 0; i < count; ++i) {
+      const TalkPortion& po = P.of[i];
+      const int tiles = (po.r1 - po.r0 + mix_rows - 1) / mix_rows;
+      int most = 0;
+      for (int tile = 0; tile < tiles; ++tile) {
+        const int cuts = (tile_steps(po, po.r0 + tile * mix_rows, mix_rows, window_left) + steps - 1) / steps;
+        blocks += cuts, most = cuts > most ? cuts : most;
+        if (blocks > 4 * 224 * room) continue;  // (many rounds even out, and are not worth the counting)
+        for (int cut = 0; cut < cuts; ++cut) fullest = std::max(fullest, ++lots[(at + (long)cut * tiles + tiles - 1 - tile) % MIX_LOTS]);
+      }
+      at += (long)tiles * most;
+    }
+    if (blocks > 4 * 224 * room) fullest = 0;
+    const bool alone = room == 1 || (blocks <= 192 && fullest <= 8);
+    const long rounds = std::max((blocks + 224 * room - 1) / (224 * room), (long)(fullest + 8 * room - 1) / (8 * room));
+    const float us = (float)rounds * (7.f + 3.7f * steps) * (alone ? 1.f : 1.6f);
     if (steps == 2 || us < least) best = steps, least = us;
   }
   return best;
+}
+static int tile_mix_rows(int n_q_heads) { return n_q_heads <= 16 ? 32 : 16; }
+// the steps of a launch that takes `n` tokens after `pos0` whole
+extern "C" int cwm_talking_tile_steps(int n, int pos0, int n_q_heads, int window_left) {
+  TalkPortions P = {};
+  P.count = 1, P.of[0].n = P.of[0].r1 = n, P.of[0].pos0 = pos0;
+  return mix_steps(P, 1, tile_mix_rows(n_q_heads), n_q_heads, window_left);
 }
 
 // `portions`: for every portion sequence, first token, tokens, position of the first, the rows that this launch takes (from a multiple
@@ -557,7 +586,7 @@ extern "C" int cwm_talking_tiles(const void* q, long q_stride, const void* cache
   CWM_REQUIRE(q_stride % 8 == 0 && ((uintptr_t)q % 16) == 0 && ((uintptr_t)cache % 16) == 0 && ((uintptr_t)out % 8) == 0 && ((uintptr_t)weights % 16) == 0,
               "talking_tiles: rows must be 16-byte aligned");
   const int per = n_q_heads / n_kv_heads, together = tile_heads_together(per);
-  const int mix_rows = n_q_heads <= 16 ? 32 : 16, value_rows = together <= 2 ? 32 : 16, groups = cwm_talking_tile_groups(n_q_heads, n_kv_heads, head_dim);
+  const int mix_rows = tile_mix_rows(n_q_heads), value_rows = together <= 2 ? 32 : 16, groups = cwm_talking_tile_groups(n_q_heads, n_kv_heads, head_dim);
   TalkPortions P;
   P.count = count;
   long blocks[3] = {0, 0, 0}, at = 0;
@@ -576,7 +605,7 @@ extern "C" int cwm_talking_tiles(const void* q, long q_stride, const void* cache
     }
     at += (long)n_q_heads * (po.r1 - po.r0) * po.columns;
   }
-  const int steps = mix_steps(P, count, mix_rows, window_left);
+  const int steps = mix_steps(P, count, mix_rows, n_q_heads, window_left);
   for (int i = 0; i < count; ++i) {
     TalkPortion& po = P.of[i];
     const int rows = po.r1 - po.r0;
