@@ -18,7 +18,8 @@
 //      written in the activation type; zero for a column the row does not read);
 //   3. `talk_values_kernel`: a block a (row, key/value head, range of columns) adds weight times value and leaves a
 //      partial sum a range, which the caller adds in their order (the weights are final, so the partial sums are plain).
-// Every block reads only its own head's keys or values, once.  A long portion of a prompt in bfloat16 takes stages 1
+// Every block reads only its own head's keys or values, once.  Portions of a prompt in bfloat16 go without the table where
+// `attention_talk_tile.hip` has kernels for the heads and is ahead (`talk_tiles_take` in ops/mixing.py); other long ones take stages 1
 // and 3 as matrix products on keys and values gathered from the pages (`talk_gather_kernel`), with the scores and
 // weights of a sequence as [key/value head][row][head of the group][column]; stage 2 takes either layout by its
 // strides.  Every sum's order depends only on the row's own position, its sequence's portion and the window.

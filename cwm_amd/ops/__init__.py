@@ -538,10 +538,11 @@ def gemm_bf16_stream(
 
 
 def linear_inputs_takes(x: torch.Tensor, weight: torch.Tensor, rows_per_input: int) -> bool:
-    """Whether the product of a few rows of several inputs is one launch (`linear_inputs`): as many as the streaming product takes.  A decode
-    step of two layers whose four products of 2,048 x 2,048 and their low rank meet five inputs, apart (five launches, and four more up to the
-    gated result) and so (two), us: 17 rows 377 and 316, 32 rows 416 and 367, 33 rows 496 and 392, 64 rows 557 and 478; at a width of 1,024 32 rows
-    375 and 366, 64 rows 476 and 447; of 3,072 24 rows 504 and 429."""
+    """Whether the product of a few rows of several inputs is one launch (`linear_inputs`): as many as the streaming product takes.  Linear
+    attention's layer of four products and their low rank of 64 on five inputs, apart (five launches, and four more up to the gated result) and so
+    (two), replayed, us by rows 17, 32, 33 and 64: width 512 42 and 19, 46 and 20, 74 and 25, 81 and 27; 2,048 65 and 34, 78 and 43, 108 and 49, 128 and
+    68; 3,072 81 and 44, 110 and 58, 125 and 67, 159 and 94; 5,120 122 and 78, 149 and 96, 166 and 111, 231 and 156; 8,192 196 and 149, 233 and 188, 245
+    and 203, 322 and 276.  Without the weights' streaming copies no size of these is slower either (8,192, 24 rows 211 and 201)."""
     return (
         x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 3 and x.shape[1] <= STREAM_MAX_ROWS
         and rows_per_input % 16 == 0 and x.is_contiguous() and x.shape[1] * x.shape[2] % 8 == 0 and _stream_takes(x[0], weight)
